@@ -152,11 +152,11 @@ def tolerance(case):
     """About four times what the path differs by from itself with its sums in another order (direct instead of Winograd
     convolutions, separate instead of fused epilogues and classifier tail; another batch around the same images).
 
-    fp32 inference: 1.2e-6, 5e-6 at the worst value.  bf16 inference: 7e-4 and 6e-3
-    against the same roundings with sums in 64 bits, where a sum a hair off now and then rounds to the next bf16 value.  Train steps: 2e-3 to 7e-3 in the deep networks and 3e-7
-    or as much in the shallow ones, because the gradients are discontinuous: a max-pool window or a ReLU on the edge
-    goes the other way in one sample of some millions, and moves that sample's whole share of a filter's gradient (0.1 to 0.4
-    of a typical value where few samples add up)."""
+    fp32 inference: 1.2e-6, 5e-6 at the worst value.  bf16 inference: 7e-4 and 6e-3 against the same roundings with sums
+    in 64 bits, where a sum a hair off now and then rounds to the next bf16 value.  Train steps: 2e-3 to 7e-3 in the
+    deep networks and 3e-7 or as much in the shallow ones, because the gradients are discontinuous: a max-pool window or
+    a ReLU on the edge goes the other way in one sample of some millions, and moves that sample's whole share of a
+    filter's gradient (0.1 to 0.4 of a typical value where few samples add up)."""
     if case["mode"] == "train":
         return {"rel": 0.025, "max": 0.99}
     return {"rel": 3e-3, "max": 2e-2} if case["mode"] == "infer_bf16" else {"rel": 1e-5, "max": 1e-4}
