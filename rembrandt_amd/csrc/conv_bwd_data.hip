@@ -182,6 +182,12 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
     }
     if (flags & RH_ALGO_WINOGRAD) return RH_E_UNSUPPORTED;
   }
+  if (!(flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET)) && d.x_elems > 0) {
+    const LdsConvPlan lp = plan_lds_bwd_data(d);
+    if (lds_pays(d, lp))
+      return launch_conv_lds(lp, true, d.N, d.K, d.P, d.Q, d.C, d.H, d.W, d.R, d.R - 1 - d.pad, dy, w, dx, alpha, beta, nullptr, 0,
+                             mask, ws, stream);
+  }
   const int KRS = d.K * d.R * d.S;
   const PhasePlan pp = plan_phase_bwd_data(d);
   if (pp.ok && !(flags & RH_ALGO_GATHER)) {

@@ -866,6 +866,8 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
         const WinoGeom wg = wino_shape5(d) ? wino_geom_fwd5(d) : wino_geom_fwd(d);
         if (wg.ok && wg.total() > need) need = wg.total();
       }
+      const size_t lp = lds_part_bytes(d.R, d.S, d.st, d.y_elems);
+      if (lp > need) need = lp;
       return need;
     }
     case RH_CONV_BWD_DATA: {
@@ -879,6 +881,8 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
         const WinoGeom wg = wino_geom_bwd_data(d);
         if (wg.ok && wg.total() > need) need = wg.total();
       }
+      const size_t lp = lds_part_bytes(d.R, d.S, d.st, d.x_elems);
+      if (lp > need) need = lp;
       return need;
     }
     case RH_CONV_BWD_FILTER: {

@@ -1,5 +1,6 @@
 // Host-side helpers shared by the three convolution passes.
 #pragma once
+#include <math.h>
 #include <stdlib.h>
 
 #include "gemm_core.h"
@@ -367,6 +368,44 @@ int launch_conv_wino_bwd_filter(const ConvDims& d, const WinoFilterPlan& p, cons
                                 float beta, void* ws, hipStream_t stream);
 int launch_conv_wino(const WinoGeom& g, bool bwd, const float* in, const float* w, float* out, float alpha, float beta,
                      const float* bias, int relu, const float* mask, void* ws, hipStream_t stream, const char* tag);
+
+// Stride-1 layers with both operands staged in LDS as they lie in memory (conv_lds.hip), forward and backward-data.
+constexpr int kLdsShapeCount = 6;
+// Partial sums of a sliced call are at most this large (more would take longer than the slices save: 16 MB are 8 us), so
+// that the workspace of a call is known without choosing its plan.
+constexpr size_t kLdsMaxPart = size_t(16) << 20;
+constexpr int kLdsMaxSlices = 32;
+inline size_t lds_part_bytes(int R, int S, int st, long long out_elems) {
+  if (R != S || (R != 3 && R != 5) || st != 1) return 0;
+  const size_t most = kLdsMaxSlices * sizeof(float) * (size_t)out_elems;
+  return align256(most < kLdsMaxPart ? most : kLdsMaxPart);
+}
+struct LdsConvPlan {
+  bool ok;
+  int shape, npos;       // tile shape; staged positions per channel
+  int qps, splits;       // channel quads per slice of the contraction; slices
+  double us;             // what a call is expected to take
+};
+// What the engine's forward and backward-data forms take on a stride-1 layer, with their operand copies and reductions, by
+// the direct form's FLOPs: a fit to the same layers (rms error 17 %; 14 us at 50 MFLOP, 34 at 1 GFLOP, 119 at 10, 363 at 50).
+// The staged form is taken where its own estimate is below this: at every batch of a small network's layers, up to
+// some 10 GFLOP on 128 rows and more, beyond 30 on the 64-row tiles the engine is weakest at.
+inline double conv_engine_us(const ConvDims& d) {
+  const double mflop = 2e-6 * (double)d.y_elems * d.C * d.R * d.S;
+  return 9.3 + mflop / 197.0 + 0.59 * sqrt(mflop);
+}
+// N images of Ci channels, `rows` result channels of P x Q.
+LdsConvPlan plan_conv_lds(int N, int Ci, int rows, int P, int Q, int R, int S, int st);
+inline LdsConvPlan plan_lds_fwd(const ConvDims& d) { return plan_conv_lds(d.N, d.C, d.K, d.P, d.Q, d.R, d.S, d.st); }
+inline LdsConvPlan plan_lds_bwd_data(const ConvDims& d) {   // (halo R - 1 - pad)
+  LdsConvPlan p = plan_conv_lds(d.N, d.K, d.C, d.H, d.W, d.R, d.S, d.st);
+  p.ok = p.ok && d.pad <= d.R - 1;
+  return p;
+}
+inline bool lds_pays(const ConvDims& d, const LdsConvPlan& p) { return p.ok && p.us < conv_engine_us(d); }
+int launch_conv_lds(const LdsConvPlan& pl, bool bwd, int N, int Ci, int H, int W, int rows, int P, int Q, int R, int halo,
+                    const float* in, const float* w, float* out, float alpha, float beta, const float* bias, int relu,
+                    const float* mask, void* ws, hipStream_t stream);
 
 // Forward with packed bf16 operands (RH_MATH_BF16_MFMA_FP32ACC, input channels a multiple of 8): the contraction runs
 // over k = (r, s, c) with c fastest, the image is copied once to bf16 as [n][hp][c/8][wp][8] with its zero border,

@@ -603,6 +603,12 @@ extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x,
                               (flags & RH_FUSE_RELU) ? 1 : 0, nullptr, ws, stream, "conv_fwd_wino");
     if (flags & RH_ALGO_WINOGRAD) return RH_E_UNSUPPORTED;
   }
+  if (!(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET))) {
+    const LdsConvPlan lp = plan_lds_fwd(d);
+    if (lds_pays(d, lp))
+      return launch_conv_lds(lp, false, d.N, d.C, d.H, d.W, d.K, d.P, d.Q, d.R, d.pad, x, w, y, alpha, beta,
+                             (flags & RH_FUSE_BIAS) ? bias : nullptr, (flags & RH_FUSE_RELU) ? 1 : 0, nullptr, ws, stream);
+  }
   const int CRS = d.C * d.R * d.S;
   if ((flags & RH_MATH_BF16_MFMA_FP32ACC) && !(flags & RH_ALGO_GATHER)) {
     const Bf16FwdPlan bpn = plan_bf16_fwd(d);

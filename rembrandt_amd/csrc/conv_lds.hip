@@ -1,0 +1,404 @@
+// Stride-1 convolution whose operands are staged in LDS as they lie in memory: forward and backward-data of small
+// grids, in one launch (plus a reduction where even these tiles do not fill the GPU).
+//
+//   out[n][row][p][q] = sum over (ch, r, s) of  wt(row, ch, r, s) * in[n][ch][p + r - halo][q + s - halo]
+//   forward:        in = x,  wt(ko, c, r, s) = w[ko][c][r][s],             halo = pad
+//   backward-data:  in = dy, wt(c, ko, r, s) = w[ko][c][R-1-r][S-1-s],     halo = R - 1 - pad
+//
+// What bounds it: the layers it is for (everything of a small network, the layers of a large one at a few images)
+// are chains of launches of a few microseconds, each waiting for memory once or twice.  The engine of gemm_core.h
+// needs a zero-bordered copy of the image, a transposed filter and an offset table in front of such a contraction
+// and often a reduction behind it: two dependent launches of which neither computes, and the products themselves read
+// their operands through L2 once per tile column.  Here a block stages what its tile needs itself:
+//  - the image rows its BN consecutive output pixels (n, p, q flattened) reach, four channels ("a quad") of them at a
+//    time (border and absent channels are out-of-range loads, which read zero).  Rows of consecutive images follow
+//    each other, so a tile may span images.
+//  - the filter of its BM rows for that quad: [tap][row].
+// Either lies in LDS as two planes of channel pairs.  An operand of v_mfma_f32_32x32x2_f32 is then one 8-byte LDS read
+// per two MFMAs: lanes 0-31 take channels 0, 1 of the quad and lanes 32-63 channels 2, 3 of the same position (or row), so
+// the first MFMA contracts channels {0, 2}, the second {1, 3}.  A tap is a displacement r Wp + s of the position: R
+// address registers and constant offsets, no arithmetic between the MFMAs.  Two stages of LDS, one barrier a stage, the next
+// stage in registers while this one is multiplied; two to four blocks a CU.
+//
+// Measured, one call (with whatever it launches) against the same call on the engine, fp32, stride 1:
+//   20 -> 50, 5x5, 14x14, batch 64: 15.3 us (29.8);  32 -> 32, 5x5, 16x16, batch 128: 21.1 (35.1);
+//   64 -> 64, 3x3, 56x56, batch 8: 29.6 (60.5), batch 32: 81 (94), batch 128: 256 (273);
+//   384 -> 384, 3x3, 13x13, batch 1: 18.3 (30.5), batch 4: 33.6 (41.8); 96 -> 256, 5x5, 27x27, batch 16: 123 (155).
+// Where the time goes on 64 channels, 56x56, batch 32 (47 us at the matrix peak, 54 with 6.1 blocks of work a CU as 7):
+// MFMAs, barriers, prologues and the epilogue 74, LDS traffic 4, loads 6.
+#include <string.h>
+
+#include <algorithm>
+
+#include "conv_common.h"
+
+namespace rh {
+
+typedef float f32x2_t __attribute__((ext_vector_type(2)));
+
+struct LdsConvParams {
+  const float* in; const float* w;
+  uint32_t in_bytes, w_bytes;
+  int Ci, HW, H, W;        // the image
+  int halo, Wp, Hp;        // zeros in front; staged row pitch Q + S - 1; staged rows per image P + R - 1
+  int npos;                // staged positions per channel, a multiple of 64
+  int row_str, ch_str;     // filter strides of a result row and of a contraction channel, in floats
+  int flip;                // taps in reverse order (backward-data)
+  int nq, qps;             // channel quads; quads per slice (a multiple of the quads of a stage)
+  int tiles_m;
+  FastDiv dQ, dP, dWp, dHp;
+};
+
+constexpr int kLdsMaxPos = 512;   // staged positions per channel and tile: two a thread
+
+// A tap's filter slab: [half][BM rows][2 channels], and a skew that spreads the writes over the banks (a wave writes the
+// taps of seven rows of a 3x3 filter, of two or three rows of a 5x5 one).
+template <int R> constexpr int lds_tap_stride(int bm) { return bm * 4 + (R == 3 ? 14 : 6); }
+
+// R: filter extent.  T: tile (BM x BN over WM x WN waves).  WK: waves that share a tile and split the quads of a stage
+// among them (their sums meet in LDS at the end).  QC: quads per stage.
+template <int R, class T, int WK, int QC>
+__global__ __launch_bounds__(256) void conv_lds_kernel(LdsConvParams p, EpiParams ep) {
+  constexpr int RS = R * R, BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN;
+  static_assert(T::NT * WK == 256 && QC % WK == 0, "four waves");
+  constexpr int WSTR = lds_tap_stride<R>(BM);   // floats from a tap's filter slab to the next
+  constexpr int WQ = RS * WSTR;                 // floats of a quad's filter slab
+  constexpr int WE = (BM * RS + 255) / 256;     // (row, tap) pairs a thread brings per quad
+  constexpr int ND = kLdsMaxPos / 256;          // positions a thread brings per quad, at most
+  extern __shared__ __attribute__((aligned(16))) float smem[];
+  const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wk = wave % WK, wmn = wave / WK, wm = wmn % T::WM, wn = wmn / T::WM;
+  const int half = lane >> 5, l32 = lane & 31;
+  const int tile = xcd_remap((int)blockIdx.x, (int)gridDim.x);
+  const int m0 = (tile % p.tiles_m) * BM, n0 = (tile / p.tiles_m) * BN;
+  const int XQ = p.npos * 4;                    // floats of a quad's image slab
+  float* const xs = smem;                       // [2][QC][half][npos][2]
+  float* const wsm = smem + 2 * QC * XQ;        // [2][QC][RS][WSTR]
+
+  // the tile's first output row (image nb, row pb); position 0 is that row's first staged image row
+  uint32_t t, q, nb, pb;
+  p.dQ.divmod((uint32_t)n0, t, q);
+  p.dP.divmod(t, nb, pb);
+  uint32_t xoff[ND];
+#pragma unroll
+  for (int i = 0; i < ND; ++i) {
+    const uint32_t pos = (uint32_t)(i * 256 + tid);
+    uint32_t row, col, n, hp;
+    p.dWp.divmod(pos, row, col);
+    p.dHp.divmod(row + pb, n, hp);
+    n += nb;
+    const int h = (int)hp - p.halo, wc = (int)col - p.halo;
+    const bool ok = (unsigned)h < (unsigned)p.H && (unsigned)wc < (unsigned)p.W && (int)(n * (uint32_t)p.dQ.div * p.dP.div) < ep.cols;
+    xoff[i] = ok ? (n * (uint32_t)p.Ci * (uint32_t)p.HW + (uint32_t)(h * p.W + wc)) * 4u : kInvalidByteOff;
+  }
+  // filter loads: pair e = tid + 256 i is row e / RS, tap e % RS (memory order within a row)
+  uint32_t woff[WE], wdst[WE];
+#pragma unroll
+  for (int i = 0; i < WE; ++i) {
+    const int e = tid + 256 * i, row = e / RS, rs = e - row * RS;
+    const bool ok = row < BM && m0 + row < ep.rows;
+    woff[i] = ok ? (uint32_t)((m0 + row) * p.row_str + rs) * 4u : kInvalidByteOff;
+    wdst[i] = row < BM ? (uint32_t)((p.flip ? RS - 1 - rs : rs) * WSTR + row * 2) : 0xffffffffu;
+  }
+  const __amdgpu_buffer_rsrc_t rin = make_rsrc(p.in, p.in_bytes), rw = make_rsrc(p.w, p.w_bytes);
+
+  float xreg[QC][ND][4], wreg[QC][WE][4];   // the next stage on its way to LDS
+  // (no branches between the loads: a channel past the last one sets the top bit of its offsets, which is out of range)
+  auto load = [&](int quad) {
+#pragma unroll
+    for (int c = 0; c < QC; ++c)
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int ch = (quad + c) * 4 + j;
+        const uint32_t none = (uint32_t)((p.Ci - 1 - ch) >> 31) & kInvalidByteOff;
+#pragma unroll
+        for (int i = 0; i < ND; ++i)
+          xreg[c][i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rin, (int)(xoff[i] | none), (int)((uint32_t)ch * (uint32_t)p.HW * 4u), 0));
+#pragma unroll
+        for (int i = 0; i < WE; ++i)
+          wreg[c][i][j] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rw, (int)(woff[i] | none), (int)((uint32_t)ch * (uint32_t)p.ch_str * 4u), 0));
+      }
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int c = 0; c < QC; ++c) {
+#pragma unroll
+      for (int i = 0; i < ND; ++i)
+        if (i * 256 + tid < p.npos) {
+          float* const d = xs + (buf * QC + c) * XQ + (i * 256 + tid) * 2;
+          *reinterpret_cast<float2*>(d) = make_float2(xreg[c][i][0], xreg[c][i][1]);
+          *reinterpret_cast<float2*>(d + p.npos * 2) = make_float2(xreg[c][i][2], xreg[c][i][3]);
+        }
+#pragma unroll
+      for (int i = 0; i < WE; ++i)
+        if (BM * RS % 256 == 0 || i < WE - 1 || wdst[i] != 0xffffffffu) {
+          float* const d = wsm + (buf * QC + c) * WQ + wdst[i];
+          *reinterpret_cast<float2*>(d) = make_float2(wreg[c][i][0], wreg[c][i][1]);
+          *reinterpret_cast<float2*>(d + BM * 2) = make_float2(wreg[c][i][2], wreg[c][i][3]);
+        }
+    }
+  };
+
+  // this lane's positions: column block j, filter row r
+  int xb[TN][R];
+#pragma unroll
+  for (int j = 0; j < TN; ++j) {
+    int m = n0 + wn * (TN * 32) + j * 32 + l32;
+    if (m >= ep.cols) m = n0;
+    uint32_t pq, qq, n, pp;
+    p.dQ.divmod((uint32_t)m, pq, qq);
+    p.dP.divmod(pq, n, pp);
+    const int pos = ((int)(n - nb) * p.Hp + (int)pp - (int)pb) * p.Wp + (int)qq;
+#pragma unroll
+    for (int r = 0; r < R; ++r) xb[j][r] = (pos + r * p.Wp) * 2 + half * (p.npos * 2);
+  }
+  const int wb = (wm * (TM * 32) + l32) * 2 + half * (BM * 2);
+
+  f32x16 acc[TM][TN];
+#pragma unroll
+  for (int i = 0; i < TM; ++i)
+#pragma unroll
+    for (int j = 0; j < TN; ++j)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+
+  // Operands of tap u of this wave's share of a stage (QC / WK quads of RS taps): read DIST taps ahead of their MFMAs.
+  constexpr int NU = QC / WK * RS, DIST = TM * TN == 1 ? 2 : 1;
+  f32x2_t a[DIST + 1][TM], b[DIST + 1][TN];
+  auto read = [&](int u, int slot, int buf) {
+    const int c = u / RS, rs = u % RS, r = rs / R, s = rs % R;
+    const float* const xq = xs + (buf * QC + wk * (QC / WK) + c) * XQ;
+    const float* const wq = wsm + (buf * QC + wk * (QC / WK) + c) * WQ + wb;
+#pragma unroll
+    for (int i = 0; i < TM; ++i) a[slot][i] = *reinterpret_cast<const f32x2_t*>(wq + rs * WSTR + i * 64);
+#pragma unroll
+    for (int j = 0; j < TN; ++j) b[slot][j] = *reinterpret_cast<const f32x2_t*>(xq + xb[j][r] + s * 2);
+  };
+  auto mul = [&](int slot) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[slot][i][e], b[slot][j][e], acc[i][j], 0, 0, 0);
+  };
+
+  const int q0 = (int)blockIdx.y * p.qps, q1 = min(q0 + p.qps, p.nq);
+  load(q0);
+  store(0);
+  __syncthreads();
+#pragma unroll
+  for (int u = 0; u < DIST; ++u) read(u, u, 0);
+  // Slots rotate through the taps of a stage; NU need be no multiple of DIST + 1, so a stage ends by moving the first
+  // operands of the next one to the slots it starts with.
+  int buf = 0;
+  for (int qd = q0;;) {
+    const bool more = qd + QC < q1;
+    if (more) load(qd + QC);
+#pragma unroll
+    for (int u = 0; u < NU - DIST; ++u) {
+      read(u + DIST, (u + DIST) % (DIST + 1), buf);
+      __builtin_amdgcn_sched_barrier(0);
+      mul(u % (DIST + 1));
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if (!more) break;
+    // every operand of this stage is in registers: the next one goes to the other buffer, and its first operands are
+    // read under the last MFMAs of this one
+    store(buf ^ 1);
+    __syncthreads();
+    buf ^= 1;
+    qd += QC;
+    f32x2_t a2[DIST][TM], b2[DIST][TN];
+#pragma unroll
+    for (int u = 0; u < DIST; ++u) {
+      constexpr int free_slot = NU % (DIST + 1);
+      read(u, free_slot, buf);
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a2[u][i] = a[free_slot][i];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b2[u][j] = b[free_slot][j];
+    }
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = NU - DIST; u < NU; ++u) mul(u % (DIST + 1));
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int u = 0; u < DIST; ++u) {
+#pragma unroll
+      for (int i = 0; i < TM; ++i) a[u][i] = a2[u][i];
+#pragma unroll
+      for (int j = 0; j < TN; ++j) b[u][j] = b2[u][j];
+    }
+  }
+#pragma unroll
+  for (int u = NU - DIST; u < NU; ++u) mul(u % (DIST + 1));
+  if constexpr (WK > 1) {
+    // the WK waves of a tile add their sums in LDS, in the order of their quads
+    static_assert(TM == 1 && TN == 1, "one block a wave");
+    __syncthreads();
+    float* const red = smem;   // [tile waves][WK - 1][16][64]
+    if (wk > 0)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) red[((wmn * (WK - 1) + wk - 1) * 16 + v) * 64 + lane] = acc[0][0][v];
+    __syncthreads();
+    if (wk > 0) return;
+#pragma unroll
+    for (int k = 1; k < WK; ++k)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) acc[0][0][v] += red[((wmn * (WK - 1) + k - 1) * 16 + v) * 64 + lane];
+  }
+  store_tile<T, true>(acc, ep, m0, n0, wm, wn, lane, ep.split_stride != 0 ? (int)blockIdx.y : -1);
+}
+
+typedef Tile<64, 128, 2, 1, 4> L64x128;
+typedef Tile<64, 64, 2, 2, 2> L64x64;
+typedef Tile<32, 128, 2, 1, 4> L32x128;
+typedef Tile<32, 64, 2, 1, 2> L32x64;    // two waves a column block
+typedef Tile<32, 32, 2, 1, 1> L32x32;    // four
+
+// mfmas: MFMAs of a wave per tap and stage
+struct LdsShape { int bm, bn, qc, mfmas; };
+static const LdsShape kLdsShapes[kLdsShapeCount] = {{64, 128, 1, 4}, {64, 64, 1, 2}, {32, 128, 1, 2}, {32, 64, 2, 2}, {32, 32, 4, 2}, {32, 128, 2, 4}};
+
+// Staged positions per channel that any tile of `bn` consecutive output pixels can need.
+static int lds_positions(int P, int Q, int R, int bn) {
+  const long long out_rows = cdiv(bn - 1, Q) + 1;                        // output rows such a run can touch
+  const long long crossings = cdiv<long long>(out_rows - 1, P);         // image boundaries among them
+  const long long n = (out_rows + (crossings + 1) * (R - 1)) * (Q + R - 1);
+  return n > (1 << 20) ? (1 << 20) : round_up((int)n, 64);
+}
+
+static size_t lds_conv_bytes(int R, int shape, int npos) {
+  const LdsShape& s = kLdsShapes[shape];
+  return 4 * (size_t)2 * s.qc * ((size_t)npos * 4 + (size_t)R * R * (R == 3 ? lds_tap_stride<3>(s.bm) : lds_tap_stride<5>(s.bm)));
+}
+
+// Time of a call in microseconds, as a function of shape and slices: rounds of the blocks a CU holds at a time, each block
+// taking its stages' MFMAs (times `mfma`, what barriers and the other blocks cost) or, with few blocks, its stages' MFMAs
+// one by one with `wait` in between; 1.2 us a round for prologue and epilogue; slices write and read their partial sums at
+// 4 TB/s in a launch of their own.  The constants are a fit to some 4000 timings (14 layers, both passes, batches 1 to 128,
+// all shapes and slice counts; rms error 8 %, the shape it picks is 3 % from the best on average).
+struct LdsCost { double wait, mfma; };
+static const LdsCost kLdsCost3[kLdsShapeCount] = {{0.70, 1.15}, {0.65, 1.47}, {0.55, 1.36}, {0.92, 1.89}, {0.26, 3.78}, {0.97, 1.40}};
+static const LdsCost kLdsCost5[kLdsShapeCount] = {{1.14, 1.15}, {0.87, 1.32}, {0.54, 1.15}, {0.35, 1.60}, {0.23, 2.43}, {0.87, 1.12}};
+
+static LdsConvPlan make_lds_plan(int N, int Ci, int rows, int P, int Q, int R) {
+  LdsConvPlan p;
+  p.ok = false;
+  p.us = 0.0;
+  const long long cols = (long long)N * P * Q;
+  const int nq = cdiv(Ci, 4);
+  const double out_bytes = 4.0 * (double)cols * rows;
+  static const int kSlices[] = {1, 2, 3, 4, 5, 6, 8, 10, 12, 16, 24, 32};
+  for (int shape = 0; shape < kLdsShapeCount; ++shape) {
+    const LdsShape& s = kLdsShapes[shape];
+    if (rows <= 32 && s.bm > 32) continue;
+    const int npos = lds_positions(P, Q, R, s.bn);
+    const size_t lds = lds_conv_bytes(R, shape, npos);
+    if (npos > kLdsMaxPos || lds > 160 * 1024) continue;
+    const int stages = cdiv(nq, s.qc);
+    const long long tiles = (long long)cdiv(rows, s.bm) * cdiv<long long>(cols, s.bn);
+    const LdsCost& c = (R == 3 ? kLdsCost3 : kLdsCost5)[shape];
+    const double mfma_us = s.mfmas * R * R * 64.0 / 2300.0;   // one stage of a wave at the clock it gets
+    const int held = min((int)(160 * 1024 / lds), shape == 0 || shape == 4 ? 4 : 6);
+    for (int want : kSlices) {
+      if (want > stages) break;
+      const int per = cdiv(stages, want), slices = cdiv(stages, per);
+      if (slices != want || (slices > 1 && (double)slices * out_bytes > (double)kLdsMaxPart)) continue;
+      const long long per_cu = cdiv<long long>(tiles * slices, 256);
+      auto round_us = [&](long long k) { return per * std::max((double)k * mfma_us * c.mfma, mfma_us + c.wait) + 1.2; };
+      const long long full = per_cu / held, rem = per_cu - full * held;
+      double us = 2.8 + (double)full * round_us(held) + (rem ? round_us(rem) : 0.0);
+      if (slices > 1) us += 2.5 + out_bytes * (2 * slices + 1) / 4.0e6;
+      if (!p.ok || us < p.us) {
+        p.ok = true;
+        p.us = us; p.shape = shape; p.npos = npos; p.splits = slices; p.qps = per * s.qc;
+      }
+    }
+  }
+  return p;
+}
+
+// Every step asks for the same plans again and choosing one costs as much host time as a launch: each thread keeps the last
+// plan of each of a few slots.  (A function of the six numbers alone.)
+LdsConvPlan plan_conv_lds(int N, int Ci, int rows, int P, int Q, int R, int S, int st) {
+  if (R != S || (R != 3 && R != 5) || st != 1 || P <= 0 || Q <= 0) {
+    LdsConvPlan none;
+    none.ok = false; none.us = 0.0;
+    return none;
+  }
+  struct Slot { int key[6]; LdsConvPlan plan; };
+  static thread_local Slot slots[64] = {};
+  const int key[6] = {N, Ci, rows, P, Q, R};
+  uint32_t h = 2166136261u;
+  for (int k : key) h = (h ^ (uint32_t)k) * 16777619u;
+  Slot& s = slots[(h >> 8) & 63];
+  if (memcmp(s.key, key, sizeof key) != 0) {
+    s.plan = make_lds_plan(N, Ci, rows, P, Q, R);
+    memcpy(s.key, key, sizeof key);
+  }
+  return s.plan;
+}
+
+template <int R, class T, int WK, int QC>
+static int launch_lds_shape(const LdsConvParams& p, const EpiParams& ep, int splits, hipStream_t stream) {
+  const size_t lds = 4 * (size_t)2 * QC * ((size_t)p.npos * 4 + (size_t)R * R * lds_tap_stride<R>(T::BM));
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&conv_lds_kernel<R, T, WK, QC>),
+                                                     hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024);
+  if (attr != hipSuccess) return (int)attr;
+  hipLaunchKernelGGL((conv_lds_kernel<R, T, WK, QC>), dim3((unsigned)(p.tiles_m * cdiv(ep.cols, T::BN)), (unsigned)splits),
+                     dim3(256), lds, stream, p, ep);
+  return launch_status();
+}
+
+template <int R>
+static int launch_lds_R(int shape, const LdsConvParams& p, const EpiParams& ep, int splits, hipStream_t stream) {
+  switch (shape) {
+    case 0: return launch_lds_shape<R, L64x128, 1, 1>(p, ep, splits, stream);
+    case 1: return launch_lds_shape<R, L64x64, 1, 1>(p, ep, splits, stream);
+    case 2: return launch_lds_shape<R, L32x128, 1, 1>(p, ep, splits, stream);
+    case 3: return launch_lds_shape<R, L32x64, 2, 2>(p, ep, splits, stream);
+    case 4: return launch_lds_shape<R, L32x32, 4, 4>(p, ep, splits, stream);
+    default: return launch_lds_shape<R, L32x128, 1, 2>(p, ep, splits, stream);
+  }
+}
+
+int launch_conv_lds(const LdsConvPlan& pl, bool bwd, int N, int Ci, int H, int W, int rows, int P, int Q, int R, int halo,
+                    const float* in, const float* w, float* out, float alpha, float beta, const float* bias, int relu,
+                    const float* mask, void* ws, hipStream_t stream) {
+  LdsConvParams p;
+  p.in = in; p.w = w;
+  p.in_bytes = (uint32_t)(sizeof(float) * (size_t)N * Ci * H * W);
+  p.w_bytes = (uint32_t)(sizeof(float) * (size_t)rows * Ci * R * R);
+  p.Ci = Ci; p.HW = H * W; p.H = H; p.W = W;
+  p.halo = halo; p.Wp = Q + R - 1; p.Hp = P + R - 1;
+  p.npos = pl.npos;
+  p.row_str = bwd ? R * R : Ci * R * R;
+  p.ch_str = bwd ? rows * R * R : R * R;
+  p.flip = bwd ? 1 : 0;
+  p.nq = cdiv(Ci, 4); p.qps = pl.qps;
+  p.tiles_m = cdiv(rows, kLdsShapes[pl.shape].bm);
+  p.dQ = FastDiv((uint32_t)Q); p.dP = FastDiv((uint32_t)P); p.dWp = FastDiv((uint32_t)p.Wp); p.dHp = FastDiv((uint32_t)p.Hp);
+  EpiParams ep;
+  ep.out = out; ep.bias = bias; ep.alpha = alpha; ep.beta = beta;
+  ep.rows = rows; ep.cols = N * P * Q; ep.inner = P * Q; ep.ld = 0; ep.relu = relu; ep.split_stride = 0; ep.mask = mask;
+  const long long total = (long long)rows * ep.cols;
+  const double flops = 2.0 * (double)total * Ci * R * R;
+  EpiParams kep = ep;
+  if (pl.splits > 1) {
+    kep.out = static_cast<float*>(ws); kep.split_stride = total; kep.bias = nullptr; kep.relu = 0; kep.mask = nullptr;
+  }
+  {
+    ProfScope prof(bwd ? "conv_bwd_data_lds" : "conv_fwd_lds", flops, stream);
+    if (int e = R == 3 ? launch_lds_R<3>(pl.shape, p, kep, pl.splits, stream) : launch_lds_R<5>(pl.shape, p, kep, pl.splits, stream))
+      return e;
+  }
+  if (pl.splits <= 1) return 0;
+  launch_split_reduce_nchw(static_cast<float*>(ws), pl.splits, total, out, total, ep.inner, rows, alpha, beta, bias, relu, stream, 0,
+                           mask);
+  return launch_status();
+}
+
+}  // namespace rh

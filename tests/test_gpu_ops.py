@@ -8,6 +8,7 @@ import torch
 import oracle as O
 from rembrandt_amd import _lib, ops, synth
 from conftest import assert_close, say
+from test_gpu_step_graph import profile_tags
 
 pytestmark = pytest.mark.gpu
 
@@ -149,6 +150,45 @@ def test_conv2d_all_passes(dev, case, algo):
     else:
         assert st > 1
     torch.cuda.synchronize()
+
+
+# Stride-1 layers with both operands staged in LDS: for each tile shape and filter extent, whole and in slices of the
+# channels, sizes with remainders everywhere (rows, pixels, channels; tiles that span images), the smallest there is, and
+# a 5x5 layer without padding
+STAGED_CASES = [
+    # N, C, H, W, K, R, pad
+    (1, 1, 1, 1, 1, 3, 1), (2, 5, 9, 7, 21, 5, 0), (3, 2, 4, 30, 33, 3, 2),
+    (16, 3, 56, 56, 33, 3, 1), (11, 66, 31, 32, 33, 3, 1), (25, 3, 28, 28, 130, 5, 2), (22, 33, 27, 28, 33, 5, 2),   # 64 x 128
+    (5, 3, 40, 41, 33, 5, 2), (19, 20, 13, 13, 33, 5, 2), (1, 132, 13, 13, 65, 3, 1),                               # 64 x 64
+    (1, 3, 5, 5, 20, 3, 1), (1, 20, 5, 6, 20, 5, 2), (20, 12, 27, 29, 96, 5, 2),                                     # 32 x 128
+    (1, 8, 5, 6, 20, 3, 1), (1, 33, 5, 5, 33, 5, 2), (9, 40, 20, 20, 70, 3, 1),                                      # 32 x 64
+    (1, 66, 5, 5, 20, 3, 1), (1, 13, 5, 5, 20, 5, 2), (32, 32, 16, 16, 32, 5, 2),                                    # 32 x 32
+    (27, 8, 17, 18, 33, 5, 2), (2, 33, 28, 29, 33, 5, 2),                                                            # 32 x 128, two quads
+]
+
+
+@pytest.mark.parametrize("case", STAGED_CASES, ids=str)
+def test_conv2d_staged_operands(dev, case):
+    """Forward and backward-data against the oracle at the edges of the staged form's tiles, with its epilogues."""
+    Nn, C, H, W, K, R, pad = case
+    say("staged case", case)
+    x, w, b = synth.normal(17, 1, (Nn, C, H, W)), synth.normal(17, 2, (K, C, R, R)), synth.normal(17, 3, (K,))
+    y_ref = O.conv2d_fwd(x, w, 1, pad)
+    dy = synth.normal(17, 4, y_ref.shape)
+    y0, dx0 = synth.normal(17, 5, y_ref.shape), synth.normal(17, 6, x.shape)
+    xd, wd, bd, dyd = T(x, dev), T(w, dev), T(b, dev), T(dy, dev)
+    (y, dx), tags = profile_tags(lambda: (ops.conv2d_fwd(xd, wd, 1, pad), ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad)))
+    assert "conv_fwd_lds" in tags, tags   # (the data gradient of a few channels may keep the engine)
+    assert_close(N(y), y_ref, "staged fwd")
+    assert_close(N(dx), O.conv2d_bwd_data(w, dy, x.shape, 1, pad), "staged bwd data")
+    yf = ops.conv2d_fwd(xd, wd, 1, pad, bias=bd, relu=True)
+    assert torch.equal(torch.clamp_min(y + bd.view(1, -1, 1, 1), 0.0), yf), "fused epilogue == conv, add_bias, rect"
+    yb = ops.conv2d_fwd(xd, wd, 1, pad, alpha=0.5, beta=2.0, y=T(y0, dev))
+    assert_close(N(yb), O.conv2d_fwd(x, w, 1, pad, alpha=0.5, beta=2.0, y=y0.copy()), "staged fwd alpha/beta")
+    one = ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, alpha=0.5, beta=2.0, dx=T(dx0, dev), relu_of=xd)
+    two = ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, alpha=0.5, beta=2.0, dx=T(dx0, dev))
+    ops.rect_backprop_inplace(xd, two)
+    assert torch.equal(one, two), "masked data gradient"
 
 
 # 3x3 stride-1 layers in the Winograd F(2x2, 3x3) form: odd and even extents (tiles that hang over the edge), every
