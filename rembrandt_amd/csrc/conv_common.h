@@ -315,7 +315,8 @@ struct WinoGeom {
   long long tiles, tiles_p;   // 2x2 output tiles; rounded up to whole column tiles
   size_t u_bytes, v_bytes;
   bool ok;
-  // Tail form (V made in the kernel only): the blocks past the last multiple of 256 are cut into tail_S slices of the
+  double us;                  // what a call is expected to take
+  // Tail form (V made in the kernel only): the blocks past the last multiple of 256 (all of them where there are fewer) are cut into tail_S slices of the
   // channel loop, tail_L stages each, whose untransformed-blend partial results go to slabs of scratch that hold the
   // result from element part_first on (the first image a tail block touches); tail_S == 1: not worth it.
   int full_tiles, tail_S, tail_L;
@@ -336,20 +337,6 @@ inline bool wino_shape5(const ConvDims& d) { return d.R == 5 && d.S == 5 && d.st
 inline WinoGeom wino_geom_fwd5(const ConvDims& d) { return wino_geom(d.N, d.C, d.H, d.W, d.K, d.pad, 1); }
 inline WinoGeom wino_geom_fwd(const ConvDims& d) { return wino_geom(d.N, d.C, d.H, d.W, d.K, d.pad); }
 inline WinoGeom wino_geom_bwd_data(const ConvDims& d) { return wino_geom(d.N, d.K, d.P, d.Q, d.C, 2 - d.pad); }
-// Where the library takes it by itself: enough channels on both sides for the 16 products to be worth their
-// transforms, and a grid that fills the GPU.
-inline bool wino_pays(const WinoGeom& g) {
-  // (rows: 128-row tiles at least three quarters full: 64 filters in one would execute as much as the direct form)
-  return g.ok && g.Ci >= 64 && g.Ko >= 64 && 4 * g.Ko >= 3 * g.rows_p &&
-         (long long)(g.rows_p / kWinoBM) * (g.tiles_p / kWinoBN) >= 192;
-}
-// The 5x5 forward form executes 64 % of the direct form's multiply-adds (a little more where the 2x2 tiles overhang
-// the result) at a lower rate than the direct kernels reach, 18 % less time on 96 -> 256 channels, 27 x 27, batch 256:
-// taken for full row tiles, a channel loop long next to a block's prologue and epilogue, and several rounds of blocks.
-inline bool wino_pays5(const WinoGeom& g) {
-  return g.ok && g.blk5 && g.C5 >= 64 && g.Ko >= 64 && 8 * g.Ko >= 7 * g.rows_p &&
-         (long long)(g.rows_p / kWinoBM) * (g.tiles_p / kWinoBN) >= 512;
-}
 // Filter gradient in the same form: zero-bordered copies of x and dy, S slices of the tiles, their partial sums.
 struct WinoFilterPlan {
   bool ok;
@@ -403,6 +390,33 @@ inline LdsConvPlan plan_lds_bwd_data(const ConvDims& d) {   // (halo R - 1 - pad
   return p;
 }
 inline bool lds_pays(const ConvDims& d, const LdsConvPlan& p) { return p.ok && p.us < conv_engine_us(d); }
+// Where the library takes the Winograd form by itself: enough channels on both sides for the 16 products to be worth their
+// transforms, and either a grid that fills the GPU, or (sliced, wino_geom) a call expected to take less time than both
+// direct forms: from batch 5 or so on for 128 channels and more (256 -> 384, 13 x 13: batch 3 33 us against 25 staged,
+// batch 8 36 against 46 on the engine and 41 staged, batch 32 79 against 97 and 111).
+// (Against the staged form by an eighth at least: its two or three launches count for more in a chain of layers than timed
+// back to back, ResNet-18 on 9 images 457 us with 1/8, 476 with the plain comparison.)
+inline bool wino_fastest(const ConvDims& d, const WinoGeom& g, const LdsConvPlan& lp) {
+  return g.Ci % 4 == 0 && g.us < conv_engine_us(d) && !(lp.ok && lp.us * 0.875 <= g.us);
+}
+inline bool wino_pays(const ConvDims& d, const WinoGeom& g, const LdsConvPlan& lp) {
+  if (!g.ok || g.Ci < 64 || g.Ko < 64) return false;
+  // (rows: 128-row tiles at least three quarters full: 64 filters in one would execute as much as the direct form)
+  if (4 * g.Ko >= 3 * g.rows_p && (long long)(g.rows_p / kWinoBM) * (g.tiles_p / kWinoBN) >= 192) return true;
+  return wino_fastest(d, g, lp);
+}
+// The 5x5 forward form executes 64 % of the direct form's multiply-adds (a little more where the 2x2 tiles overhang
+// the result) at a lower rate than the direct kernels reach, 18 % less time on 96 -> 256 channels, 27 x 27, batch 256:
+// taken for full row tiles, a channel loop long next to a block's prologue and epilogue, and several rounds of blocks, or
+// for several row tiles (which share the patches a block reads four times over) from one round on where it is expected to be
+// the fastest (the same layer at batch 24: 151 us against 204 on the engine and 200 staged; below one round, at batch
+// 16, 122 against 124 staged: not worth its scratch).
+inline bool wino_pays5(const ConvDims& d, const WinoGeom& g, const LdsConvPlan& lp) {
+  if (!g.ok || !g.blk5 || g.C5 < 64 || g.Ko < 64 || 8 * g.Ko < 7 * g.rows_p) return false;
+  const long long blocks = (long long)(g.rows_p / kWinoBM) * (g.tiles_p / kWinoBN);
+  return blocks >= 512 || (blocks >= 256 && g.rows_p > kWinoBM && wino_fastest(d, g, lp));
+}
+
 int launch_conv_lds(const LdsConvPlan& pl, bool bwd, int N, int Ci, int H, int W, int rows, int P, int Q, int R, int halo,
                     const float* in, const float* w, float* out, float alpha, float beta, const float* bias, int relu,
                     const float* mask, void* ws, hipStream_t stream);

@@ -73,21 +73,37 @@ WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int blk5) {
   g.full_tiles = 0; g.tail_S = 1; g.tail_L = g.Cg; g.part_first = 0; g.slab_elems = 0; g.part_bytes = 0;
   const long long tiles_m = g.rows_p / kWinoBM, T = tiles_m * (g.tiles_p / kWinoBN);
   const long long full = T / 256 * 256, tail = T - full;
-  if (g.ok && Ci % 4 == 0 && full > 0 && tail > 0) {
-    double best = (double)cdiv<long long>(T, 256) * 0.97;
+  const long long out_elems = (long long)N * Ko * g.P * g.Q;
+  // Time of a call in microseconds (a fit to 260 timings of nine layers, both passes, batches 1 to 128; rms error 6 %): a
+  // stage takes 0.98 us, a block's prologue and epilogue as long as 8.2 of them; the filter transform writes U at 1.6 TB/s,
+  // the slabs pass at 2.8 TB/s through a launch of 2 us; the 5x5 form's copy is a launch more.
+  const double fixed_us = 7.8 + (double)ub / 1.6e6 + (blk5 ? 4.0 + 2.0 * (double)g.img_bytes / 22.0e6 : 0.0);
+  auto stages_us = [](double rounds, int stages) { return rounds * (stages + 8.2) * 0.975; };
+  g.us = fixed_us + stages_us((double)cdiv<long long>(T, 256), g.Cg);
+  if (g.ok && Ci % 4 == 0 && tail > 0) {
+    double best = (double)cdiv<long long>(T, 256) * 0.97, best_us = g.us;
     for (int S = 2; S <= 16; ++S) {
       const int L = cdiv(g.Cg, S);
       if (L < 4 || cdiv(g.Cg, L) != S) continue;
-      const double cost = (double)(full / 256) + (double)cdiv<long long>(tail * S, 256) * (L + 8.0) / (g.Cg + 8.0) + 0.03;
-      if (cost < best) { best = cost; g.tail_S = S; g.tail_L = L; }
+      if (full > 0) {
+        const double cost = (double)(full / 256) + (double)cdiv<long long>(tail * S, 256) * (L + 8.0) / (g.Cg + 8.0) + 0.03;
+        if (cost < best) { best = cost; g.tail_S = S; g.tail_L = L; }
+      } else {
+        // Fewer blocks than CUs: all of them are cut, into as many slices as the whole call is shortest with (384 -> 384 on
+        // 13 x 13, batch 8: 39 blocks as 8 slices, 44 us; whole 116; the direct form 58).
+        const double us = fixed_us + stages_us((double)cdiv<long long>(T * S, 256), L) + 2.0 + 4.0 * (double)out_elems * (S + 1) / 2.84e6;
+        if (us < best_us) { best_us = us; g.tail_S = S; g.tail_L = L; }
+      }
     }
     if (g.tail_S > 1) {
       g.full_tiles = (int)full;
       const long long first_tile = (full / tiles_m) * kWinoBN;   // first image tile of the first column tile with a tail block
       const long long n0 = first_tile / ((long long)g.TP * g.TQ);
       g.part_first = n0 * g.Ko * g.P * g.Q;
-      g.slab_elems = (long long)N * g.Ko * g.P * g.Q - g.part_first;
+      g.slab_elems = out_elems - g.part_first;
       g.part_bytes = align256(sizeof(float) * (size_t)g.slab_elems * g.tail_S);
+      g.us = fixed_us + stages_us((double)(full / 256), g.Cg) + stages_us((double)cdiv<long long>(tail * g.tail_S, 256), g.tail_L) +
+             2.0 + 4.0 * (double)g.slab_elems * (g.tail_S + 1) / 2.84e6;
     }
   }
   return g;
@@ -1301,7 +1317,7 @@ extern "C" double rh_conv2d_winograd_flops(const rh_conv_geom* g, int pass, int 
   if (flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT)) return 0.0;
   if (wino_shape5(d) && pass == RH_CONV_FWD) {
     const WinoGeom wg = wino_geom_fwd5(d);
-    if (!(flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays5(wg))) return 0.0;
+    if (!(flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays5(d, wg, plan_lds_fwd(d)))) return 0.0;
     return 2.0 * 16.0 * (double)wg.Ko * wg.Ci * (double)wg.tiles;
   }
   if (!wino_shape(d)) return 0.0;
@@ -1312,7 +1328,7 @@ extern "C" double rh_conv2d_winograd_flops(const rh_conv_geom* g, int pass, int 
   }
   if (pass != RH_CONV_FWD && pass != RH_CONV_BWD_DATA) return 0.0;
   const WinoGeom wg = pass == RH_CONV_FWD ? wino_geom_fwd(d) : wino_geom_bwd_data(d);
-  if (!(flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays(wg))) return 0.0;
+  if (!(flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays(d, wg, pass == RH_CONV_FWD ? plan_lds_fwd(d) : plan_lds_bwd_data(d)))) return 0.0;
   return 2.0 * 16.0 * (double)wg.Ko * wg.Ci * (double)wg.tiles;
 }
 

@@ -210,6 +210,8 @@ WINO_CASES = [
     (70, 384, 13, 13, 64, 1),     # the same in the data gradient
     (16, 128, 28, 28, 64, 1),
     (90, 64, 13, 13, 128, 1),     # 4410 tiles: the filter gradient in the form too, its tiles in several slices
+    (1, 260, 7, 9, 130, 1),       # two blocks in sixteen slices of five stages (the last one of none)
+    (5, 132, 12, 14, 64, 1),      # seven blocks, half of their rows past the last filter, in eight slices
 ]
 
 
