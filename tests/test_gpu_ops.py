@@ -1074,6 +1074,27 @@ def test_bnorm(dev, shape):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("shape", [(1, 3, 16, 128), (9, 3, 4, 57), (4, 2, 32, 64), (3, 2, 4, 683), (5, 2, 64, 64), (1, 2, 4, 5121),
+                                   (512, 3, 1, 3), (29, 3, 1, 53), (2048, 3, 1, 3), (5, 2, 1, 1229), (4096, 2, 1, 5), (2, 2, 1, 10241)])
+def test_bnorm_at_the_bounds_of_its_forms(dev, shape):
+    """Values per channel at and just past what each block size of the one-launch form holds (2048 / 8192 / 20480 in
+    16-byte units, 1536 / 6144 / 20480 single), where the last is the bound to the two-launch form; results written over
+    their own input are those written elsewhere."""
+    test_bnorm(dev, shape)
+    C = shape[1]
+    x = synth.normal(18, 1, shape) * np.float32(2.0) + np.float32(3.0)
+    scale, bias = T(synth.normal(18, 4, (C,)), dev), T(synth.normal(18, 5, (C,)), dev)
+    stats = [T(np.zeros(C, np.float32), dev) for _ in range(4)]
+    apart, cm, ci = ops.bnorm_fwd_train(T(x, dev), scale, bias, stats[0], stats[1], 0.1, 1e-5)
+    over = T(x, dev)
+    ops.bnorm_fwd_train(over, scale, bias, stats[2], stats[3], 0.1, 1e-5, y=over)
+    assert np.array_equal(N(over), N(apart))
+    dy = T(synth.normal(18, 2, shape), dev)
+    dx = N(ops.bnorm_bwd(T(x, dev), dy, scale, cm, ci, 1e-5)[0])
+    ops.bnorm_bwd(T(x, dev), dy, scale, cm, ci, 1e-5, dx=dy)
+    assert np.array_equal(N(dy), dx)
+
+
 @pytest.mark.parametrize("case", [(2, 3, 9, 3, 2, 0), (2, 3, 9, 3, 2, 1), (3, 4, 8, 2, 2, 0), (2, 5, 27, 3, 2, 0), (2, 2, 13, 3, 3, 1)])
 @pytest.mark.parametrize("rounding", [_lib.RH_ROUND_FLOOR, _lib.RH_ROUND_CEIL])
 def test_pool2d_bwd_with_folded_relu_mask(dev, case, rounding):
