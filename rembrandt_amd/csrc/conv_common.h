@@ -88,11 +88,10 @@ inline int launch_mfma_gemm(const typename AL::Params& ap, const typename BL::Pa
 }
 
 // Same grid and split logic for the bf16-operand kernel.  FLOPs are counted as for fp32.
-template <class T, class AL, class BL, bool NCHW, class PASS, bool PK = false>
+template <class T, class AL, class BL, bool NCHW, class PASS>
 inline int launch_mfma_gemm_bf16(const typename AL::Params& ap, const typename BL::Params& bp,
                                  const EpiParams& ep, int K, int splits, int* splits_used,
-                                 hipStream_t stream, const char* tag, int k_algorithmic = 0,
-                                 const PackedOut& pk = PackedOut()) {
+                                 hipStream_t stream, const char* tag, int k_algorithmic = 0) {
   const int tiles_m = cdiv(ep.rows, T::BM), tiles_n = cdiv(ep.cols, T::BN);
   const int k_chunks = cdiv(K, T::BK);
   if (splits < 1) splits = 1;
@@ -104,36 +103,35 @@ inline int launch_mfma_gemm_bf16(const typename AL::Params& ap, const typename B
   static_assert(lds_bytes <= 160 * 1024, "tile does not fit the 160 KB LDS of a CU");
   if (lds_bytes > 48 * 1024) {
     static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&mfma_gemm_bf16_kernel<T, AL, BL, NCHW, PASS, PK>),
+        reinterpret_cast<const void*>(&mfma_gemm_bf16_kernel<T, AL, BL, NCHW, PASS>),
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
     if (attr != hipSuccess) return (int)attr;
   }
   ProfScope prof(tag, 2.0 * (double)ep.rows * (double)ep.cols * (double)(k_algorithmic > 0 ? k_algorithmic : K), stream);
-  if (PK && (splits != 1 || !pk.ptr)) return RH_E_INVALID;
-  hipLaunchKernelGGL((mfma_gemm_bf16_kernel<T, AL, BL, NCHW, PASS, PK>), grid, dim3(T::NT), lds_bytes, stream, ap, bp, ep,
-                     tiles_m, k_chunks, cps, pk);
+  hipLaunchKernelGGL((mfma_gemm_bf16_kernel<T, AL, BL, NCHW, PASS>), grid, dim3(T::NT), lds_bytes, stream, ap, bp, ep,
+                     tiles_m, k_chunks, cps);
   return launch_status();
 }
 
-// The direct-to-LDS form for packed operands (ring of four LDS buffers, one pass over the whole contraction).
-template <class T, bool A_LINEAR, bool B_LINEAR, bool NCHW, class PASS, bool PK = false, int R = 4>
+// The direct-to-LDS form for packed operands (one pass over the whole contraction).
+template <class T, bool A_LINEAR, bool B_LINEAR, bool NCHW, class PASS, bool PK = false, int R = 4, int KS = 1>
 inline int launch_mfma_gemm_bf16_dma(const RowV8Params& ap, const RowV8Params& bp, const EpiParams& ep, int K,
                                      hipStream_t stream, const char* tag, int k_algorithmic = 0,
                                      const PackedOut& pk = PackedOut()) {
   const int tiles_m = cdiv(ep.rows, T::BM), tiles_n = cdiv(ep.cols, T::BN);
   if (K <= 0 || K % T::BK != 0) return RH_E_INVALID;
-  constexpr size_t lds_bytes = 16 * R * (T::BK / 8) * (T::BM + T::BN);
-  static_assert(lds_bytes * T::OCC <= 160 * 1024, "the blocks meant to share a CU do not fit its 160 KB of LDS");
+  constexpr size_t lds_bytes = bf16_dma_lds_bytes(T::BM, T::BN, T::BK, R, KS);
+  static_assert(lds_bytes * T::OCC * 4 / (T::NT / kWave * KS) <= 160 * 1024, "the blocks meant to share a CU do not fit its 160 KB of LDS");
   if (lds_bytes > 48 * 1024) {
     static const hipError_t attr = hipFuncSetAttribute(
-        reinterpret_cast<const void*>(&mfma_gemm_bf16_dma_kernel<T, A_LINEAR, B_LINEAR, NCHW, PASS, PK, R>),
+        reinterpret_cast<const void*>(&mfma_gemm_bf16_dma_kernel<T, A_LINEAR, B_LINEAR, NCHW, PASS, PK, R, KS>),
         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_bytes);
     if (attr != hipSuccess) return (int)attr;
   }
   ProfScope prof(tag, 2.0 * (double)ep.rows * (double)ep.cols * (double)(k_algorithmic > 0 ? k_algorithmic : K), stream);
   if (PK && !pk.ptr) return RH_E_INVALID;
-  hipLaunchKernelGGL((mfma_gemm_bf16_dma_kernel<T, A_LINEAR, B_LINEAR, NCHW, PASS, PK, R>), dim3((unsigned)(tiles_m * tiles_n)),
-                     dim3(T::NT), lds_bytes, stream, ap, bp, ep, tiles_m, K / T::BK, pk);
+  hipLaunchKernelGGL((mfma_gemm_bf16_dma_kernel<T, A_LINEAR, B_LINEAR, NCHW, PASS, PK, R, KS>), dim3((unsigned)(tiles_m * tiles_n)),
+                     dim3(T::NT * KS), lds_bytes, stream, ap, bp, ep, tiles_m, K / T::BK, pk);
   return launch_status();
 }
 
@@ -157,6 +155,11 @@ typedef Tile<128, 128, RH_BF16_BK, 2, 2, RH_BF16_OCC> T128x128bf;
 typedef Tile<256, 256, 32, 2, 4, 1> T256x256bf;
 typedef Tile<256, 128, 32, 2, 2, 2> T256x128bf;   // direct-to-LDS form with a ring of three: two blocks of four waves share a CU
 typedef Tile<128, 256, 32, 2, 2, 2> T128x256bf;   // the same for filter counts that would waste rows of a 256-row tile
+// The same loop for grids of few tiles (see bf16_small_form): smaller tiles, and groups of waves that share a tile's K steps.
+typedef Tile<128, 128, 32, 2, 2, 3> T128x128bd;   // ring of three, three blocks per CU
+typedef Tile<128, 128, 32, 2, 2, 2> T128x128bd2;  // two groups, one block per CU
+typedef Tile<64, 128, 32, 2, 2, 4> T64x128bf;     // ring of three, four blocks per CU: up to 64 filters
+typedef Tile<64, 64, 32, 2, 2, 4> T64x64bf;       // ring of four, two groups (two blocks per CU) or four (one)
 typedef Tile<64, 256, 16, 1, 4, 3> T64x256;
 typedef Tile<32, 256, 16, 1, 4, 3> T32x256;
 // few result columns as well (a first layer's filter gradient: 20 x 25, 32 x 75): narrower tiles, fewer dead columns

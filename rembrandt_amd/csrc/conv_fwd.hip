@@ -496,7 +496,7 @@ static int bf16_pack_input(const ConvDims& d, const Bf16FwdPlan& bpn, const floa
 // The contraction on prepared operands: `xb` the image copy, `wprep` the filter stage's result.  The result goes to
 // ep.out as fp32 NCHW, or, with pk.ptr set, as packed bf16 for the next convolution (ep.out unused).  Which kernel
 // runs depends on the geometry only, so both forms of the result come from the same accumulators.
-template <class T, bool DMA, bool PK, int R = 4>
+template <class T, bool PK, int R = 4, int KS = 1>
 static int bf16_gemm_on(const ConvDims& d, const Bf16FwdPlan& bpn, const void* xb, const void* wprep, const EpiParams& ep,
                         const PackedOut& pk, hipStream_t stream, const char* tag) {
   const char* base = static_cast<const char*>(wprep);
@@ -519,12 +519,60 @@ static int bf16_gemm_on(const ConvDims& d, const Bf16FwdPlan& bpn, const void* x
   }
   bp.soff = soff8;
   bp.group_stride = 0;
-  typedef LoadRowV8<T::BM, T::BK, T::NT, true> AL;
-  typedef LoadRowV8<T::BN, T::BK, T::NT, false> BL;
-  if constexpr (DMA)
-    return launch_mfma_gemm_bf16_dma<T, true, false, true, PassConvFwd, PK, R>(ap, bp, ep, bpn.n_k, stream, tag, CRS, pk);
-  else
-    return launch_mfma_gemm_bf16<T, AL, BL, true, PassConvFwd, PK>(ap, bp, ep, bpn.n_k, 1, nullptr, stream, tag, CRS, pk);
+  return launch_mfma_gemm_bf16_dma<T, true, false, true, PassConvFwd, PK, R, KS>(ap, bp, ep, bpn.n_k, stream, tag, CRS, pk);
+}
+
+// Forms for grids of few tiles, where a block's chain of K steps (an L2 round trip each, whatever the tile) is what the
+// launch takes: 384 -> 384 3x3 13x13 took 48-55 us at every batch from 1 to 64 on 256 x 128 / 128 x 256 / 128 x 128
+// (registers) tiles of 108 steps.  Smaller tiles shorten the step, groups of waves shorten the chain, and both cost fill
+// bandwidth per multiply-add once every CU has work: 12 us at batch 1 (64 x 64, four groups), 20 at 16 (two groups), 27
+// at 37 and 34 at 64 (128 x 128, two groups; at 64 all 256 CUs fill from the L2).
+struct Bf16Form {
+  int bm, bn, per_cu, groups;
+  // us: a launch; a K step of the tile with the chip nearly empty; with a block on every CU; per further block on a CU
+  double base, lone, full, next;
+};
+constexpr Bf16Form kBf16Forms[] = {
+    {128, 128, 3, 1, 6.0, 0.245, 0.297, 0.296},
+    {128, 128, 1, 2, 7.0, 0.152, 0.257, 0.0},
+    {64, 64, 2, 2, 6.6, 0.046, 0.093, 0.092},
+    {64, 64, 1, 4, 7.1, 0.032, 0.102, 0.0},
+    {64, 128, 4, 1, 5.6, 0.177, 0.222, 0.149},
+};
+// Index into kBf16Forms with the least expected time (constants fitted to 72 launches, 9 layers at batches 1 to 128: 2 %
+// off the fastest form on average, 12 % at most).  64-row tiles fill twice the bytes per multiply-add: they are taken
+// where they save a fifth, since another stream's launches share the L2 (two AlexNet passes of 37 images side by side),
+// or where there are no more rows.  Contractions of up to 256 are not cut: there the streaming 1x1 kernel gives the same bits.
+static int bf16_small_form(int rows, long long cols, int n_k) {
+  const int steps = n_k / 32;
+  int best = 0;
+  double best_us = 0.0;
+  for (int i = 0; i < 5; ++i) {
+    const Bf16Form& f = kBf16Forms[i];
+    const long long tiles = (long long)cdiv(rows, f.bm) * cdiv<long long>(cols, f.bn), slots = 256ll * f.per_cu;
+    if (f.groups > 1 && (steps <= 4 * f.groups || tiles > 2 * 256)) continue;
+    if ((i == 1 && tiles > 256) || (i == 4 && rows > 64)) continue;
+    auto step_us = [&](double blocks) {
+      const double x = blocks / 256.0;
+      return x <= 1.0 ? f.lone + (f.full - f.lone) * x : f.full + (x - 1.0) * f.next;
+    };
+    double us = f.base + (double)(tiles / slots) * (steps * step_us((double)slots) + 1.5) +
+                (tiles % slots ? steps * step_us((double)(tiles % slots)) : 0.0);
+    if (f.bm == 64 && rows > 64) us *= 1.25;
+    if (i == 0 || us < best_us) { best = i; best_us = us; }
+  }
+  return best;
+}
+template <bool PK>
+static int bf16_gemm_small(const ConvDims& d, const Bf16FwdPlan& bpn, const void* xb, const void* wprep, const EpiParams& ep,
+                           const PackedOut& pk, hipStream_t stream) {
+  switch (bf16_small_form(ep.rows, ep.cols, bpn.n_k)) {
+    case 0: return bf16_gemm_on<T128x128bd, PK, 3>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_128x128");
+    case 1: return bf16_gemm_on<T128x128bd2, PK, 3, 2>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_128x128_k2");
+    case 2: return bf16_gemm_on<T64x64bf, PK, 4, 2>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_64x64_k2");
+    case 3: return bf16_gemm_on<T64x64bf, PK, 4, 4>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_64x64_k4");
+    default: return bf16_gemm_on<T64x128bf, PK, 3>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_64x128");
+  }
 }
 
 static int bf16_gemm(const ConvDims& d, const Bf16FwdPlan& bpn, const void* xb, const void* wprep, const EpiParams& ep,
@@ -533,30 +581,28 @@ static int bf16_gemm(const ConvDims& d, const Bf16FwdPlan& bpn, const void* xb, 
   // streaming kernel (same accumulation order, hence the same bits as the tiles)
   if (pk.ptr && bpn.s_groups == 0 && (conv1x1_bf16_stream_applies(d) || (force_stream && conv1x1_bf16_stream_runs(d))))
     return launch_conv1x1_bf16_stream(d, xb, static_cast<const char*>(wprep) + bpn.tab_bytes, ep.bias, ep.relu, pk, stream);
-  // Filter counts that waste no more rows in 256-row tiles than in 128-row ones take a direct-to-LDS kernel:
+  // Grids of up to one 128 x 128 tile per CU and short contractions take bf16_small_form's choice.  (Up to 1024 tiles its
+  // forms are as fast or faster alone, NIN's 1024-channel 3x3 layer at batch 128, 288 tiles: 56 -> 48 us; but with passes
+  // of several workers side by side the larger tiles' smaller fill wins, NIN 421 us a pass against 429.)  Above, filter
+  // counts that waste no more rows in 256-row tiles than in 128-row ones take
   //  - 256 x 256 (one block of eight waves per CU, ring of four) for long contractions on grids of two rounds of
   //    the 256 CUs and more: 1.19 PFLOP/s on 256 x 96 x 27 x 27 -> 256, 5x5 (729 tiles);
-  //  - 256 x 128 (two blocks of four waves per CU, ring of three) otherwise, from contractions of 256 and grids
-  //    of one round on: a block's first loads and its stores hide behind the other block, and a grid of 365
-  //    256 x 256 tiles (the same layer at batch 128) is no longer two rounds with the second 43 % full.
-  // Short contractions and small grids stay with the 128 x 128 tile (three blocks per CU, through registers).
+  //  - 256 x 128 (two blocks of four waves per CU, ring of three) otherwise: a block's first loads and its stores hide
+  //    behind the other block, and a grid of 365 256 x 256 tiles (the same layer at batch 128) is no longer two rounds
+  //    with the second 43 % full;
+  // other filter counts (384: one and a half 256-row tiles) take the same loop on 128 rows x 256 pixels.
+  if (bpn.n_k < 256 || (long long)cdiv(d.K, 128) * cdiv(ep.cols, 128) <= 256)
+    return pk.ptr ? bf16_gemm_small<true>(d, bpn, xb, wprep, ep, pk, stream) : bf16_gemm_small<false>(d, bpn, xb, wprep, ep, pk, stream);
   const bool rows_ok = cdiv(d.K, 256) * 256 == cdiv(d.K, 128) * 128;
-  const long long t256 = (long long)cdiv(d.K, 256) * cdiv(ep.cols, 256);
-  const long long t128 = (long long)cdiv(d.K, 256) * cdiv(ep.cols, 128);
-  const bool big = rows_ok && bpn.n_k >= 512 && t256 >= 512;
-  const bool mid = rows_ok && !big && bpn.n_k >= 256 && t128 >= 96;
-  // other filter counts (384: one and a half 256-row tiles) take the same loop on 128 rows x 256 pixels
-  const bool mid128 = !rows_ok && bpn.n_k >= 256 && (long long)cdiv(d.K, 128) * cdiv(ep.cols, 256) >= 96;
+  const bool big = rows_ok && bpn.n_k >= 512 && (long long)cdiv(d.K, 256) * cdiv(ep.cols, 256) >= 512;
   if (pk.ptr) {
-    if (big) return bf16_gemm_on<T256x256bf, true, true, 4>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_256x256");
-    if (mid) return bf16_gemm_on<T256x128bf, true, true, 3>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_256x128");
-    if (mid128) return bf16_gemm_on<T128x256bf, true, true, 3>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_128x256");
-    return bf16_gemm_on<T128x128bf, false, true>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_128x128");
+    if (big) return bf16_gemm_on<T256x256bf, true, 4>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_256x256");
+    if (rows_ok) return bf16_gemm_on<T256x128bf, true, 3>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_256x128");
+    return bf16_gemm_on<T128x256bf, true, 3>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_128x256");
   }
-  if (big) return bf16_gemm_on<T256x256bf, true, false, 4>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_256x256");
-  if (mid) return bf16_gemm_on<T256x128bf, true, false, 3>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_256x128");
-  if (mid128) return bf16_gemm_on<T128x256bf, true, false, 3>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_128x256");
-  return bf16_gemm_on<T128x128bf, false, false>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_128x128");
+  if (big) return bf16_gemm_on<T256x256bf, false, 4>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_256x256");
+  if (rows_ok) return bf16_gemm_on<T256x128bf, false, 3>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_256x128");
+  return bf16_gemm_on<T128x256bf, false, 3>(d, bpn, xb, wprep, ep, pk, stream, "conv_fwd_bf16p_128x256");
 }
 
 template <class T>

@@ -427,47 +427,6 @@ struct RowV8Params {
   int group_stride;                    // bytes between consecutive groups (LINEAR)
 };
 
-template <int ROWS, int BK, int NT, bool LINEAR>
-struct LoadRowV8 {
-  static constexpr int KG = BK / 8;
-  static constexpr int CNT = ROWS * KG / NT;  // 16-byte groups per thread and K step
-  static_assert(BK % 8 == 0 && NT % ROWS == 0 && (ROWS * KG) % NT == 0 && ROWS % kWave == 0, "loader shape");
-  typedef RowV8Params Params;
-  typedef uint4 Reg;
-  __amdgpu_buffer_rsrc_t rsrc;
-  const int* tab;
-  uint32_t vbase;
-  int g0, row, gstride;
-  int so[CNT];
-
-  __device__ __forceinline__ void init(const Params& p, int row0, int tid) {
-    rsrc = make_rsrc(p.ptr, p.bytes);
-    row = tid % ROWS;
-    g0 = __builtin_amdgcn_readfirstlane(tid / ROWS) * CNT;
-    tab = p.soff;
-    gstride = p.group_stride;
-    const int m = row0 + row;
-    const bool valid = m < p.M;
-    const int mm = valid ? m : 0;
-    const int n = mm / p.inner;
-    const int rem = mm - n * p.inner;
-    const int a = rem / p.innerW;
-    const int b = rem - a * p.innerW;
-    vbase = valid ? (uint32_t)(n * p.img_stride + a * p.a_stride + b * p.b_stride) : 0x80000000u;
-  }
-  __device__ __forceinline__ void prep(int k0) {
-#pragma unroll
-    for (int i = 0; i < CNT; ++i) so[i] = LINEAR ? ((k0 >> 3) + g0 + i) * gstride : tab[(k0 >> 3) + g0 + i];
-  }
-  __device__ __forceinline__ uint4 load_one(int i) const {
-    return __builtin_bit_cast(uint4, __builtin_amdgcn_raw_buffer_load_b128(rsrc, (int)vbase, so[i], 0));
-  }
-  __device__ __forceinline__ void store_bf16(uint4* s, const uint4 (&v)[CNT]) {
-#pragma unroll
-    for (int i = 0; i < CNT; ++i) s[(g0 + i) * ROWS + row] = v[i];
-  }
-};
-
 // ------------------------------------------------------------------------------------------
 // Backward-filter operands: the contraction index k is an output pixel (n,p,q); lanes run
 // along k because both dy and x are contiguous along q.
@@ -1078,16 +1037,16 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_kernel(typename AL::P
 
 // ------------------------------------------------------------------------------------------
 // bf16-operand form of the same tile engine (RH_MATH_BF16_MFMA_FP32ACC): operands reach LDS as bf16 (rounded by the
-// fp32 loaders as they write, or already packed in memory: LoadRowV8), are multiplied with
+// fp32 loaders as they write), are multiplied with
 // v_mfma_f32_32x32x16_bf16 (8 k per lane per operand) and accumulated in fp32.  LDS slabs are [k/8][row] of
 // 16-byte groups, double buffered: a loader writes one ds_write_b128 per 8 values and an MFMA operand is one
 // ds_read_b128.
 // ------------------------------------------------------------------------------------------
-template <class T, class AL, class BL, bool NCHW, class PASS, bool PK = false>
+template <class T, class AL, class BL, bool NCHW, class PASS>
 __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_bf16_kernel(typename AL::Params ap,
                                                                        typename BL::Params bp, EpiParams ep,
                                                                        int tiles_m, int k_chunks,
-                                                                       int chunks_per_split, PackedOut pk) {
+                                                                       int chunks_per_split) {
   constexpr int BM = T::BM, BN = T::BN, BK = T::BK, TM = T::TM, TN = T::TN;
   static_assert(BK % 16 == 0, "one bf16 MFMA contracts 16 k");
   constexpr int KG = BK / 8;  // 16-byte groups per row and K step
@@ -1183,8 +1142,7 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_bf16_kernel(typename 
   for (int it = 0; it + 1 < nk; ++it) k_step(it, std::true_type());
   if (nk > 0) k_step(nk - 1, std::false_type());
 
-  if constexpr (PK) store_tile_packed<T>(acc, ep, pk, m0, n0, wm, wn, lane);
-  else store_tile<T, NCHW>(acc, ep, m0, n0, wm, wn, lane, ep.split_stride != 0 ? split_idx : -1);
+  store_tile<T, NCHW>(acc, ep, m0, n0, wm, wn, lane, ep.split_stride != 0 ? split_idx : -1);
 }
 
 // ------------------------------------------------------------------------------------------
@@ -1209,7 +1167,7 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_bf16_kernel(typename 
 // and no other vector memory instruction is issued between the prologue and the epilogue.
 // Shapes: 256 x 256 with eight waves and a ring of four (128 KB: one block per CU, so the first loads and the
 // stores of a tile are not hidden behind another block: long contractions on large grids), or 256 x 128 with four
-// waves and a ring of three (72 KB: two blocks per CU).
+// waves and a ring of three (72 KB: two blocks per CU); grids of few tiles take smaller ones (bf16_small_form).
 // ------------------------------------------------------------------------------------------
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
 
@@ -1229,8 +1187,8 @@ __device__ __forceinline__ void wait_vmcnt() {
   asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory");
 }
 
-// RowV8Params operand loaded straight into an LDS slab.  Thread -> (row, groups) as in LoadRowV8; a wave covers 64
-// neighbouring rows of each of its groups.  Two sets of group offsets: the loads of a step use `so` while `so_next`
+// RowV8Params operand loaded straight into an LDS slab.  Thread -> (row, groups): row = tid % ROWS, groups in runs of
+// CNT; a wave covers 64 neighbouring rows of each of its groups.  Two sets of group offsets: the loads of a step use `so` while `so_next`
 // is being fetched for the step after.
 template <int ROWS, int BK, int NT, bool LINEAR>
 struct DmaRowV8 {
@@ -1291,9 +1249,15 @@ struct DmaRowV8 {
   }
 };
 
-template <class T, bool A_LINEAR, bool B_LINEAR, bool NCHW, class PASS, bool PK = false, int R = 4>
-__global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_bf16_dma_kernel(RowV8Params ap, RowV8Params bp, EpiParams ep,
-                                                                           int tiles_m, int k_chunks, PackedOut pk) {
+// KS > 1: KS groups of T::NT threads share a tile, each takes a part of the K steps through a ring of its own, and the
+// first adds the others' results, in order, from LDS.
+constexpr int bf16_dma_lds_bytes(int bm, int bn, int bk, int R, int KS) {
+  const int ring = KS * R * (bk / 8) * (bm + bn) * 16, sums = (KS - 1) * bm * bn * 4;
+  return ring > sums ? ring : sums;
+}
+template <class T, bool A_LINEAR, bool B_LINEAR, bool NCHW, class PASS, bool PK = false, int R = 4, int KS = 1>
+__global__ __launch_bounds__(T::NT * KS, T::OCC) void mfma_gemm_bf16_dma_kernel(RowV8Params ap, RowV8Params bp, EpiParams ep,
+                                                                                int tiles_m, int k_chunks, PackedOut pk) {
   constexpr int BM = T::BM, BN = T::BN, BK = T::BK, TM = T::TM, TN = T::TN;
   static_assert(BK % 32 == 0, "an even number of 16-k groups per step keeps the operand register sets in phase");
   typedef DmaRowV8<BM, BK, T::NT, A_LINEAR> AL;
@@ -1302,12 +1266,13 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_bf16_dma_kernel(RowV8
   static_assert(R >= 3, "the ring holds the step being read, one landed or landing, and one in flight at least");
   constexpr int SA = KG * BM, SB = KG * BN;  // 16-byte groups per buffer
   extern __shared__ float lds_dyn[];
-  uint4* const sA_base = reinterpret_cast<uint4*>(lds_dyn);  // [R][KG][BM]
-  uint4* const sB_base = sA_base + R * SA;                   // [R][KG][BN]
+  const int ks = KS > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / T::NT) : 0;  // this wave's group
+  uint4* const sA_base = reinterpret_cast<uint4*>(lds_dyn) + ks * (R * (SA + SB));  // [R][KG][BM]
+  uint4* const sB_base = sA_base + R * SA;                                           // [R][KG][BN]
   const uint32_t ldsA = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)sA_base;
   const uint32_t ldsB = ldsA + R * SA * 16;
 
-  const int tid = threadIdx.x;
+  const int tid = KS > 1 ? threadIdx.x % T::NT : threadIdx.x;
   const int lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int wm = wave % T::WM, wn = wave / T::WM;
@@ -1315,7 +1280,7 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_bf16_dma_kernel(RowV8
   const int logical = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, gridDim.x));
   const int tile_m = logical % tiles_m, tile_n = logical / tiles_m;
   const int m0 = tile_m * BM, n0 = tile_n * BN;
-  const int nk = k_chunks;
+  const int k_first = ks * k_chunks / KS, nk = (ks + 1) * k_chunks / KS - k_first;  // this group's K steps
 
   AL la;
   BL lb;
@@ -1331,8 +1296,8 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_bf16_dma_kernel(RowV8
       for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
 
   auto prep_step = [&](int s) {
-    la.prep(s * BK);
-    lb.prep(s * BK);
+    la.prep((k_first + s) * BK);
+    lb.prep((k_first + s) * BK);
   };
   auto issue_step = [&](int buf) {
     la.issue(ldsA + (uint32_t)(buf * SA) * 16u);
@@ -1373,7 +1338,7 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_bf16_dma_kernel(RowV8
       __builtin_amdgcn_s_waitcnt(0xc07f);
       if (MORE && g == 0) {
         // the offsets of step it+D+1 (used by the loads the next step issues), fetched first for the same reason
-        const int s4 = it + D + 1 < nk ? it + D + 1 : nk - 1;
+        const int s4 = k_first + (it + D + 1 < nk ? it + D + 1 : nk - 1);
         la.prep_next(s4 * BK);
         lb.prep_next(s4 * BK);
       }
@@ -1415,6 +1380,31 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_bf16_dma_kernel(RowV8
   for (; it + D < nk; ++it) step(it, std::true_type());
   for (; it < nk; ++it) step(it, std::false_type());
 
+  if constexpr (KS > 1) {
+    // A step has one barrier and the groups' step counts differ by one at most: the shorter ones meet one more.
+    if (nk < (k_chunks + KS - 1) / KS) __syncthreads();
+    __syncthreads();  // every ring has been read for the last time
+    float* const sums = lds_dyn + wave * (TM * TN * 16 * kWave) + lane;  // [group - 1][wave][value][lane]
+    if (ks > 0) {
+      float* const mine = sums + (ks - 1) * (BM * BN);
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) mine[((i * TN + j) * 16 + v) * kWave] = acc[i][j][v];
+    }
+    __syncthreads();
+    if (ks > 0) return;
+#pragma unroll
+    for (int g = 0; g < KS - 1; ++g)
+#pragma unroll
+      for (int i = 0; i < TM; ++i)
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+#pragma unroll
+          for (int v = 0; v < 16; ++v) acc[i][j][v] += sums[g * (BM * BN) + ((i * TN + j) * 16 + v) * kWave];
+  }
   if constexpr (PK) store_tile_packed<T>(acc, ep, pk, m0, n0, wm, wn, lane);
   else store_tile<T, NCHW>(acc, ep, m0, n0, wm, wn, lane, -1);
 }

@@ -461,6 +461,16 @@ def test_conv2d_fwd_bf16_packed_chain_forms(dev, case):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("case", [(1, 48, 13, 13, 72, 5, 1, 2, 1), (1, 136, 13, 13, 72, 3, 1, 1, 0), (16, 72, 13, 13, 136, 3, 1, 1, 1),
+                                  (37, 72, 13, 13, 384, 3, 1, 1, 1), (40, 40, 13, 13, 264, 3, 1, 1, 0), (1, 1024, 6, 6, 1000, 1, 1, 0, 0)],
+                         ids=lambda c: str(c))
+def test_conv2d_fwd_bf16_small_grids(dev, case):
+    """The forms for grids of few tiles: 64 x 64 with four groups of waves over the K steps (38 steps: 9, 10, 9, 10; 40),
+    64 x 64 with two, 128 x 128 with two and with one; ragged rows and columns; fp32 and packed results."""
+    test_conv2d_fwd_bf16_packed_chain_forms(dev, case)
+    test_conv2d_fwd_bf16_operands(dev, case[:8])
+
+
 BF16_POOL_CASES = [
     # N, C, H, W, size, stride, pad, rounding, halo of the result
     (3, 16, 13, 13, 3, 2, 0, 0, 1),
