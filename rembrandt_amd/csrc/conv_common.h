@@ -310,10 +310,12 @@ inline SoffPlan plan_soff_fwd(const ConvDims& d) {
 // Winograd F(2x2, 3x3) form of a 3x3 stride-1 layer (conv_wino.hip), written as a forward convolution: an input of
 // (N, Ci, Hi, Wi) with `halo` zeros around it, Ko filters, a result of (N, Ko, P, Q).  Backward-data is the same over dy
 // with halo 2 - pad.  Scratch: [U: transformed filter][V: transformed image patches].
-constexpr int kWinoBM = 128, kWinoBN = 32, kWinoR = 3;
+constexpr int kWinoBM = 128, kWinoBM2 = 64, kWinoBN = 32, kWinoR = 3;
 struct WinoGeom {
   int N, Ci, Hi, Wi, Ko, halo, P, Q, TP, TQ;
   int Cg;                     // groups of four input channels
+  int bm;                     // rows of a tile: kWinoBM (one block per CU) or kWinoBM2 (two)
+  int slots() const { return bm == kWinoBM ? 256 : 512; }
   int rows_p;                 // Ko rounded up to whole row tiles
   long long tiles, tiles_p;   // 2x2 output tiles; rounded up to whole column tiles
   size_t u_bytes, v_bytes;
@@ -334,6 +336,12 @@ struct WinoGeom {
   size_t img_bytes = 0;
   size_t total() const { return u_bytes + v_bytes + img_bytes + part_bytes; }
 };
+// 64-row tiles where 128-row ones would execute an eighth more rows at least (64 filters, 192, 320): row for row they are a
+// tenth slower (384 -> 384 13x13 b256 601 us against 532), with half of the rows empty the larger tile takes 655 us on
+// 64 -> 64 56x56 b256 where the smaller takes 382 and the direct form 572.
+inline int wino_bm(int Ci, int Ko, int blk5) {
+  return Ci % 4 == 0 && !blk5 && round_up(Ko, kWinoBM2) * 9 <= round_up(Ko, kWinoBM) * 8 ? kWinoBM2 : kWinoBM;
+}
 WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int blk5 = 0);
 inline bool wino_shape(const ConvDims& d) { return d.R == 3 && d.S == 3 && d.st == 1 && d.pad <= 2; }
 inline bool wino_shape5(const ConvDims& d) { return d.R == 5 && d.S == 5 && d.st == 1 && d.pad <= 4 && d.P > 0 && d.Q > 0; }
@@ -404,8 +412,12 @@ inline bool wino_fastest(const ConvDims& d, const WinoGeom& g, const LdsConvPlan
 }
 inline bool wino_pays(const ConvDims& d, const WinoGeom& g, const LdsConvPlan& lp) {
   if (!g.ok || g.Ci < 64 || g.Ko < 64) return false;
+  const long long blocks = (long long)(g.rows_p / g.bm) * (g.tiles_p / kWinoBN);
+  // 64-row tiles, two to a CU: from a whole round of blocks on, or from three quarters of the CUs on where it is expected
+  // to be the fastest (64 -> 64 56x56: batch 24, 588 blocks 53 us against 57 direct; 64 98 against 144)
+  if (g.bm == kWinoBM2) return 4 * g.Ko >= 3 * g.rows_p && (blocks >= 512 || (blocks >= 192 && wino_fastest(d, g, lp)));
   // (rows: 128-row tiles at least three quarters full: 64 filters in one would execute as much as the direct form)
-  if (4 * g.Ko >= 3 * g.rows_p && (long long)(g.rows_p / kWinoBM) * (g.tiles_p / kWinoBN) >= 192) return true;
+  if (4 * g.Ko >= 3 * g.rows_p && blocks >= 192) return true;
   return wino_fastest(d, g, lp);
 }
 // The 5x5 forward form executes 64 % of the direct form's multiply-adds (a little more where the 2x2 tiles overhang

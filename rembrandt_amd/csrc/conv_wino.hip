@@ -16,6 +16,7 @@
 //    from memory to LDS (buffer_load_dwordx4 ... lds) into a ring of three stages of four channels each, two stages
 //    ahead of the MFMAs; V is made in the kernel from the image's patches; the one barrier of a stage stands in front
 //    of its last quarter of MFMAs.  (wino_gemm_kernel: the same with V read from memory, for other channel counts.)
+//  * wino_gemm64_kernel: 64 rows x 32 tiles, two blocks to a CU, for filter counts that fill 64-row tiles much better.
 //  * the epilogue: a lane's element e of the 16 accumulators is the whole 4x4 M of one (row, tile): A^T M A is 24
 //    additions in registers, then alpha / beta, bias, ReLU or the mask of a folded ReLU backward, and the 2x2 pixels
 //    go to the NCHW result (odd extents: the tile's pixels past the edge are dropped).
@@ -56,7 +57,8 @@ WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int blk5) {
   g.tiles = (long long)N * g.TP * g.TQ;
   g.tiles_p = (g.tiles + kWinoBN - 1) / kWinoBN * kWinoBN;
   g.Cg = cdiv(Ci, 4);
-  g.rows_p = round_up(Ko, kWinoBM);
+  g.bm = wino_bm(Ci, Ko, blk5);
+  g.rows_p = round_up(Ko, g.bm);
   const unsigned long long ub = 16ull * g.Cg * 2 * (unsigned long long)g.rows_p * 8;
   const unsigned long long vb = 16ull * g.Cg * 2 * (unsigned long long)g.tiles_p * 8;
   g.u_bytes = align256((size_t)ub);
@@ -65,33 +67,40 @@ WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int blk5) {
   g.ok = g.P > 0 && g.Q > 0 && halo >= 0 && halo <= 2 && ub < (1ull << 31) && (Ci % 4 == 0 || vb < (1ull << 31)) &&
          g.tiles_p < (1ll << 30) && (long long)N * Ko * g.P * g.Q < (1ll << 30) && (long long)N * Ci * Hi * Wi < (1ll << 30);
   if (blk5) g.ok = g.ok && g.pad5 <= 4 && g.Hi >= g.H5 + g.pad5 && g.Wi >= g.W5 + g.pad5;
-  // One block per CU at a time: 784 blocks are four rounds of the 256 CUs with the last one 6 % full.  The blocks past
-  // the last whole round are cut into slices of the channel loop (every slice a whole number of stages, four at
-  // least), so that the last round is as short as its share of the work; their partial results are added by
+  // One block per CU at a time (128-row tiles): 784 blocks are four rounds of the 256 CUs with the last one 6 % full.  The
+  // blocks past the last whole round are cut into slices of the channel loop (every slice a whole number of stages, four
+  // at least), so that the last round is as short as its share of the work; their partial results are added by
   // wino_tail_reduce_kernel.  A block costs about eight stages' time before and after its loop (measured: 1176 blocks
   // of 64 stages gain nothing from five slices of 13), and the slabs and that kernel 3 % of a round.
   g.full_tiles = 0; g.tail_S = 1; g.tail_L = g.Cg; g.part_first = 0; g.slab_elems = 0; g.part_bytes = 0;
-  const long long tiles_m = g.rows_p / kWinoBM, T = tiles_m * (g.tiles_p / kWinoBN);
-  const long long full = T / 256 * 256, tail = T - full;
+  const long long tiles_m = g.rows_p / g.bm, T = tiles_m * (g.tiles_p / kWinoBN), slots = g.slots();
+  const long long full = T / slots * slots, tail = T - full;
   const long long out_elems = (long long)N * Ko * g.P * g.Q;
   // Time of a call in microseconds (a fit to 260 timings of nine layers, both passes, batches 1 to 128; rms error 6 %): a
   // stage takes 0.98 us, a block's prologue and epilogue as long as 8.2 of them; the filter transform writes U at 1.6 TB/s,
-  // the slabs pass at 2.8 TB/s through a launch of 2 us; the 5x5 form's copy is a launch more.
+  // the slabs pass at 2.8 TB/s through a launch of 2 us; the 5x5 form's copy is a launch more.  (64-row tiles: 1.03 us for
+  // the two blocks of a CU, 13.6 stages outside the loop; up to one block per CU a round takes 0.57 of that.)
+  const bool two = g.bm == kWinoBM2;
+  const double outside = two ? 13.6 : 8.2, tail_outside = two ? 13.6 : 8.0, stage_us = two ? 1.03 : 0.975;
   const double fixed_us = 7.8 + (double)ub / 1.6e6 + (blk5 ? 4.0 + 2.0 * (double)g.img_bytes / 22.0e6 : 0.0);
-  auto stages_us = [](double rounds, int stages) { return rounds * (stages + 8.2) * 0.975; };
-  g.us = fixed_us + stages_us((double)cdiv<long long>(T, 256), g.Cg);
+  auto rounds = [&](long long blocks) {
+    const long long rem = blocks % slots;
+    return (double)(blocks / slots) + (rem == 0 ? 0.0 : two && rem <= 256 ? 0.57 : 1.0);
+  };
+  auto stages_us = [&](double n, int stages) { return n * (stages + outside) * stage_us; };
+  g.us = fixed_us + stages_us(rounds(T), g.Cg);
   if (g.ok && Ci % 4 == 0 && tail > 0) {
-    double best = (double)cdiv<long long>(T, 256) * 0.97, best_us = g.us;
+    double best = rounds(T) * 0.97, best_us = g.us;
     for (int S = 2; S <= 16; ++S) {
       const int L = cdiv(g.Cg, S);
       if (L < 4 || cdiv(g.Cg, L) != S) continue;
       if (full > 0) {
-        const double cost = (double)(full / 256) + (double)cdiv<long long>(tail * S, 256) * (L + 8.0) / (g.Cg + 8.0) + 0.03;
+        const double cost = (double)(full / slots) + rounds(tail * S) * (L + tail_outside) / (g.Cg + tail_outside) + 0.03;
         if (cost < best) { best = cost; g.tail_S = S; g.tail_L = L; }
       } else {
         // Fewer blocks than CUs: all of them are cut, into as many slices as the whole call is shortest with (384 -> 384 on
         // 13 x 13, batch 8: 39 blocks as 8 slices, 44 us; whole 116; the direct form 58).
-        const double us = fixed_us + stages_us((double)cdiv<long long>(T * S, 256), L) + 2.0 + 4.0 * (double)out_elems * (S + 1) / 2.84e6;
+        const double us = fixed_us + stages_us(rounds(T * S), L) + 2.0 + 4.0 * (double)out_elems * (S + 1) / 2.84e6;
         if (us < best_us) { best_us = us; g.tail_S = S; g.tail_L = L; }
       }
     }
@@ -102,7 +111,7 @@ WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int blk5) {
       g.part_first = n0 * g.Ko * g.P * g.Q;
       g.slab_elems = out_elems - g.part_first;
       g.part_bytes = align256(sizeof(float) * (size_t)g.slab_elems * g.tail_S);
-      g.us = fixed_us + stages_us((double)(full / 256), g.Cg) + stages_us((double)cdiv<long long>(tail * g.tail_S, 256), g.tail_L) +
+      g.us = fixed_us + stages_us((double)(full / slots), g.Cg) + stages_us(rounds(tail * g.tail_S), g.tail_L) +
              2.0 + 4.0 * (double)g.slab_elems * (g.tail_S + 1) / 2.84e6;
     }
   }
@@ -244,9 +253,10 @@ struct WinoEpi {
 // lane: nothing else can run on a CU beside it.  wino_pin_acc says "these are still in accumulation registers here"
 // in front of every block of the epilogue, so that a block's 64 values are fetched when its turn comes and the
 // allocation stays near 360: a bandwidth-bound kernel of another stream finds room on the same CUs.)
-__device__ __forceinline__ void wino_pin_acc(f32x16 (&acc)[16]) {
+template <int NF>
+__device__ __forceinline__ void wino_pin_acc(f32x16 (&acc)[NF]) {
 #pragma unroll
-  for (int f = 0; f < 16; ++f) asm volatile("" : "+a"(acc[f]));
+  for (int f = 0; f < NF; ++f) asm volatile("" : "+a"(acc[f]));
 }
 
 // One accumulator element, fetched where it is used (written as the instruction itself: as an ordinary element access
@@ -257,46 +267,121 @@ __device__ __forceinline__ float wino_acc_elem(const f32x16& v, int e) {
   return r;
 }
 
+// Where a lane's outputs lie: rows row_lane + 8 (e / 4) + e % 4 of accumulator element e, the pixels of rows ai0 .. ai0 + NA - 1
+// of the 2x2 tile n0 + lane % 32.
+template <int NA>
+struct WinoOut {
+  uint32_t voff[NA][2];
+  int row_lane, rows_left, PQ4, srow;
+  __amdgpu_buffer_rsrc_t rout, rmask, rbias;
+  __device__ __forceinline__ void init(const WinoEpi& ep, int row0, unsigned n0, int lane, int ai0) {
+    const int h = lane >> 5, r = lane & 31;
+    const unsigned t = n0 + (unsigned)r;
+    uint32_t q1, tx, n, ty;
+    ep.dTQ.divmod(t, q1, tx);
+    ep.dTP.divmod(q1, n, ty);
+    const int PQ = ep.P * ep.Q;
+    row_lane = row0 + 4 * h;
+    rows_left = ep.Ko - row_lane;
+#pragma unroll
+    for (int ai = 0; ai < NA; ++ai)
+#pragma unroll
+      for (int bi = 0; bi < 2; ++bi) {
+        const int pp = 2 * (int)ty + ai0 + ai, qq = 2 * (int)tx + bi;
+        const bool ok = t < ep.tiles && pp < ep.P && qq < ep.Q;
+        voff[ai][bi] = ok ? ((n * (unsigned)ep.Ko + 4u * (unsigned)h) * (unsigned)PQ + (unsigned)(pp * ep.Q + qq)) * 4u : kInvalidByteOff;
+      }
+    rout = make_rsrc(ep.out, ep.out_bytes);
+    rmask = make_rsrc(ep.mask ? ep.mask : ep.out, ep.out_bytes);
+    rbias = make_rsrc(ep.bias ? ep.bias : ep.out, ep.bias ? 4u * (unsigned)ep.Ko : 0u);
+    PQ4 = PQ * 4;
+    srow = row0 * PQ4;   // wave-uniform byte offset of the wave's first row
+  }
+  static __device__ __forceinline__ constexpr int row_of(int e) { return 8 * (e >> 2) + (e & 3); }
+  __device__ __forceinline__ float bias(int e) const {
+    return __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rbias, (row_lane + row_of(e)) * 4, 0, 0));
+  }
+};
+
+// Blend, bias, ReLU / mask and the stores of elements e0 .. e0 + EB - 1 (loads of a block stand ahead of its stores).
+template <int EB, int NA>
+__device__ __forceinline__ void wino_store_block(const WinoOut<NA>& o, const WinoEpi& ep, int e0, float (&y)[EB][NA][2], const float* bv) {
+  const bool blend = ep.beta != 0.0f, masked = ep.mask != nullptr;
+  uint32_t vo[EB][NA][2];
+  float aux[EB][NA][2];   // mask values, or the old result
+#pragma unroll
+  for (int e4 = 0; e4 < EB; ++e4) {
+    const bool row_ok = WinoOut<NA>::row_of(e0 + e4) < o.rows_left;
+#pragma unroll
+    for (int ai = 0; ai < NA; ++ai)
+#pragma unroll
+      for (int bi = 0; bi < 2; ++bi) {
+        vo[e4][ai][bi] = row_ok ? o.voff[ai][bi] : kInvalidByteOff;
+        y[e4][ai][bi] *= ep.alpha;
+      }
+  }
+  if (masked || blend) {
+    // (both at once: the mask first, then the old values, block by block; neither occurs in a train step's forward pass)
+#pragma unroll
+    for (int e4 = 0; e4 < EB; ++e4)
+#pragma unroll
+      for (int ai = 0; ai < NA; ++ai)
+#pragma unroll
+        for (int bi = 0; bi < 2; ++bi)
+          aux[e4][ai][bi] = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(blend ? o.rout : o.rmask, (int)vo[e4][ai][bi], o.srow + WinoOut<NA>::row_of(e0 + e4) * o.PQ4, 0));
+  }
+#pragma unroll
+  for (int e4 = 0; e4 < EB; ++e4)
+#pragma unroll
+    for (int ai = 0; ai < NA; ++ai)
+#pragma unroll
+      for (int bi = 0; bi < 2; ++bi) {
+        float x = y[e4][ai][bi];
+        if (blend) x = fmaf(ep.beta, aux[e4][ai][bi], x);
+        x += bv[e4];
+        if (ep.relu) x = fmaxf(x, 0.0f);
+        if (masked && !blend) x = aux[e4][ai][bi] > 0.0f ? x : 0.0f;
+        y[e4][ai][bi] = x;
+      }
+  if (masked && blend) {
+#pragma unroll
+    for (int e4 = 0; e4 < EB; ++e4)
+#pragma unroll
+      for (int ai = 0; ai < NA; ++ai)
+#pragma unroll
+        for (int bi = 0; bi < 2; ++bi) {
+          const float mk = __builtin_bit_cast(
+              float, __builtin_amdgcn_raw_buffer_load_b32(o.rmask, (int)vo[e4][ai][bi], o.srow + WinoOut<NA>::row_of(e0 + e4) * o.PQ4, 0));
+          y[e4][ai][bi] = mk > 0.0f ? y[e4][ai][bi] : 0.0f;
+        }
+  }
+  __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+  for (int e4 = 0; e4 < EB; ++e4)
+#pragma unroll
+    for (int ai = 0; ai < NA; ++ai)
+#pragma unroll
+      for (int bi = 0; bi < 2; ++bi)
+        __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y[e4][ai][bi]), o.rout, (int)vo[e4][ai][bi],
+                                              o.srow + WinoOut<NA>::row_of(e0 + e4) * o.PQ4, 0);
+}
+
 __device__ __forceinline__ void wino_epilogue(f32x16 (&acc)[16], const WinoEpi& ep, int m0, unsigned n0, int wave, int lane) {
-  const int h = lane >> 5, r = lane & 31;
-  const unsigned t = n0 + (unsigned)r;
-  uint32_t q1, tx, n, ty;
-  ep.dTQ.divmod(t, q1, tx);
-  ep.dTP.divmod(q1, n, ty);
-  const int PQ = ep.P * ep.Q;
-  const int row_lane = m0 + wave * 32 + 4 * h;     // + 8 (e / 4) + e % 4
-  const int rows_left = ep.Ko - row_lane;
-  uint32_t voff[2][2];
-#pragma unroll
-  for (int ai = 0; ai < 2; ++ai)
-#pragma unroll
-    for (int bi = 0; bi < 2; ++bi) {
-      const bool ok = t < ep.tiles && 2 * (int)ty + ai < ep.P && 2 * (int)tx + bi < ep.Q;
-      voff[ai][bi] = ok ? ((n * (unsigned)ep.Ko + 4u * (unsigned)h) * (unsigned)PQ + (2u * ty + ai) * (unsigned)ep.Q + 2u * tx + bi) * 4u
-                        : kInvalidByteOff;
-    }
-  const __amdgpu_buffer_rsrc_t rout = make_rsrc(ep.out, ep.out_bytes);
-  const __amdgpu_buffer_rsrc_t rmask = make_rsrc(ep.mask ? ep.mask : ep.out, ep.out_bytes);
-  const __amdgpu_buffer_rsrc_t rbias = make_rsrc(ep.bias ? ep.bias : ep.out, ep.bias ? 4u * (unsigned)ep.Ko : 0u);
+  WinoOut<2> o;
+  o.init(ep, m0 + wave * 32, n0, lane, 0);
   float bv[16];
 #pragma unroll
-  for (int e = 0; e < 16; ++e) {
-    const int re = 8 * (e >> 2) + (e & 3);
-    bv[e] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(rbias, (row_lane + re) * 4, 0, 0));
-  }
-  const int srow = (m0 + wave * 32) * PQ * 4;   // wave-uniform byte offset of the wave's first row
-  const bool blend = ep.beta != 0.0f, masked = ep.mask != nullptr;
-  constexpr int EB = 4;   // accumulator elements per block (loads of a block stand ahead of its stores)
+  for (int e = 0; e < 16; ++e) bv[e] = o.bias(e);
+  constexpr int EB = 4;
 #pragma unroll
-  for (int eb = 0; eb < 16 / EB; ++eb) {
+  for (int e0 = 0; e0 < 16; e0 += EB) {
     __builtin_amdgcn_sched_barrier(0);
     wino_pin_acc(acc);
     float y[EB][2][2];
-    uint32_t vo[EB][2][2];
-    float aux[EB][2][2];   // mask values, or the old result
 #pragma unroll
     for (int e4 = 0; e4 < EB; ++e4) {
-      const int e = EB * eb + e4, re = 8 * (e >> 2) + (e & 3);
+      const int e = e0 + e4;
       float s0[4], s1[4];
 #pragma unroll
       for (int j = 0; j < 4; ++j) {
@@ -309,60 +394,8 @@ __device__ __forceinline__ void wino_epilogue(f32x16 (&acc)[16], const WinoEpi& 
       y[e4][0][1] = s0[1] - s0[2] - s0[3];
       y[e4][1][0] = s1[0] + s1[1] + s1[2];
       y[e4][1][1] = s1[1] - s1[2] - s1[3];
-      const bool row_ok = re < rows_left;
-#pragma unroll
-      for (int ai = 0; ai < 2; ++ai)
-#pragma unroll
-        for (int bi = 0; bi < 2; ++bi) {
-          vo[e4][ai][bi] = row_ok ? voff[ai][bi] : kInvalidByteOff;
-          y[e4][ai][bi] *= ep.alpha;
-        }
     }
-    if (masked || blend) {
-      // (both at once: the mask first, then the old values, block by block; neither occurs in a train step's forward pass)
-#pragma unroll
-      for (int e4 = 0; e4 < EB; ++e4)
-#pragma unroll
-        for (int ai = 0; ai < 2; ++ai)
-#pragma unroll
-          for (int bi = 0; bi < 2; ++bi)
-            aux[e4][ai][bi] = __builtin_bit_cast(
-                float, __builtin_amdgcn_raw_buffer_load_b32(blend ? rout : rmask, (int)vo[e4][ai][bi], srow + (8 * ((EB * eb + e4) >> 2) + ((EB * eb + e4) & 3)) * PQ * 4, 0));
-    }
-#pragma unroll
-    for (int e4 = 0; e4 < EB; ++e4)
-#pragma unroll
-      for (int ai = 0; ai < 2; ++ai)
-#pragma unroll
-        for (int bi = 0; bi < 2; ++bi) {
-          float x = y[e4][ai][bi];
-          if (blend) x = fmaf(ep.beta, aux[e4][ai][bi], x);
-          x += bv[EB * eb + e4];
-          if (ep.relu) x = fmaxf(x, 0.0f);
-          if (masked && !blend) x = aux[e4][ai][bi] > 0.0f ? x : 0.0f;
-          y[e4][ai][bi] = x;
-        }
-    if (masked && blend) {
-#pragma unroll
-      for (int e4 = 0; e4 < EB; ++e4)
-#pragma unroll
-        for (int ai = 0; ai < 2; ++ai)
-#pragma unroll
-          for (int bi = 0; bi < 2; ++bi) {
-            const float mk = __builtin_bit_cast(
-                float, __builtin_amdgcn_raw_buffer_load_b32(rmask, (int)vo[e4][ai][bi], srow + (8 * ((EB * eb + e4) >> 2) + ((EB * eb + e4) & 3)) * PQ * 4, 0));
-            y[e4][ai][bi] = mk > 0.0f ? y[e4][ai][bi] : 0.0f;
-          }
-    }
-    __builtin_amdgcn_sched_barrier(0);
-#pragma unroll
-    for (int e4 = 0; e4 < EB; ++e4)
-#pragma unroll
-      for (int ai = 0; ai < 2; ++ai)
-#pragma unroll
-        for (int bi = 0; bi < 2; ++bi)
-          __builtin_amdgcn_raw_buffer_store_b32(__builtin_bit_cast(uint32_t, y[e4][ai][bi]), rout, (int)vo[e4][ai][bi],
-                                                srow + (8 * ((EB * eb + e4) >> 2) + ((EB * eb + e4) & 3)) * PQ * 4, 0);
+    wino_store_block<EB, 2>(o, ep, e0, y, bv + e0);
   }
 }
 
@@ -764,6 +797,253 @@ __global__ __launch_bounds__(256, 1) void wino_gemm_fused_kernel(const float* __
   wino_epilogue(acc, ep, m0, n0, wave, lane);
 }
 
+// ---- the same on 64 rows, two blocks to a CU ---------------------------------------------------------------------------
+// A block of four waves owns 64 rows x 32 tiles: wave = (half of the rows, half of the f), 128 accumulation registers, two
+// waves to a SIMD.  What a block of wino_gemm_fused_kernel leaves idle (its prologue and epilogue, its waits at the stage's
+// barrier, the VALU time of the transforms) the other block's MFMAs fill, and 64 filters are a whole row tile; the image's
+// patches are read and transformed once per 64 rows instead of 128.
+// U goes to LDS two stages deep, the patches' taps to two sets of registers (ordinary loads: nothing of them passes
+// through LDS), three stages ahead.  The two waves that share rows exchange half of A^T M A: each stores one row of the 2x2
+// pixels, with what the other's f contribute to it read from LDS.
+// 64 -> 64 on 56 x 56, batch 256 (16 stages): 382 us, 69 TFLOP/s executed and 155 in the direct form's, where the direct
+// kernels take 570 - 635 with their operand copy; ResNet-18 b256 step 26.3 -> 25.1 ms.  What bounds it: some 6 us a block
+// outside its loop (31 us a pair of blocks on a CU, 16 of them MFMAs).
+constexpr int kWinoSA2 = 16 * 2 * kWinoBM2 * 8, kWinoStage2 = kWinoSA2 + kWinoSB;
+
+__global__ __launch_bounds__(256, 2) void wino_gemm64_kernel(const float* __restrict__ U, WinoImage im, int Cg, int rows_p,
+                                                            int tiles_m, unsigned u_bytes, WinoEpi ep, WinoTail tl) {
+  extern __shared__ float lds_dyn[];   // [2 stages: U | V]
+  const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)lds_dyn;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int rw = wave & 1, fh = wave >> 1;
+  const int h = lane >> 5, r = lane & 31;
+  int tile, cg0 = 0, nk = Cg;   // (tail blocks: as in wino_gemm_fused_kernel)
+  if (tl.S <= 1) {
+    tile = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, gridDim.x));
+  } else if ((int)blockIdx.x < tl.full) {
+    tile = __builtin_amdgcn_readfirstlane(xcd_remap(blockIdx.x, tl.full));
+  } else {
+    const int ti = __builtin_amdgcn_readfirstlane(xcd_remap((int)blockIdx.x - tl.full, (int)gridDim.x - tl.full));
+    const int slice = ti % tl.S;
+    tile = tl.full + ti / tl.S;
+    cg0 = slice * tl.L;
+    nk = Cg - cg0 < tl.L ? Cg - cg0 : tl.L;
+    ep.out = tl.part + (long long)slice * tl.slab_elems - tl.part_first;
+    ep.bias = nullptr; ep.mask = nullptr; ep.alpha = 1.0f; ep.beta = 0.0f; ep.relu = 0;
+  }
+  const int tile_m = tile % tiles_m, tile_n = tile / tiles_m;
+  const int m0 = tile_m * kWinoBM2;
+  const unsigned n0 = (unsigned)tile_n * kWinoBN;
+
+  u32x4 rsU;
+  {
+    const uint64_t pu = reinterpret_cast<uint64_t>(U);
+    rsU.x = __builtin_amdgcn_readfirstlane((uint32_t)pu);
+    rsU.y = __builtin_amdgcn_readfirstlane((uint32_t)(pu >> 32) & 0xffffu);
+    rsU.z = u_bytes; rsU.w = 0x00020000u;
+  }
+  const __amdgpu_buffer_rsrc_t rsX = make_rsrc(im.x, im.x_bytes);
+  // U of one f and stage is 2 x 64 x 8 bytes, one direct load of a wave: half-wave h brings the rows of channels 2 h, 2 h + 1
+  const uint32_t strideA = 2u * (uint32_t)rows_p * 8u, strideF = (uint32_t)Cg * strideA;
+  const uint32_t voffA = (uint32_t)h * ((uint32_t)rows_p * 8u) + (uint32_t)m0 * 8u + (uint32_t)r * 16u;
+  const int HW = im.Hi * im.Wi;
+  uint32_t poff[3][4];   // this thread's twelve patch taps, as in wino_gemm_fused_kernel
+  {
+    const unsigned t = n0 + (unsigned)r;
+    uint32_t q1, tx, n, ty;
+    ep.dTQ.divmod(t, q1, tx);
+    ep.dTP.divmod(q1, n, ty);
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        const int hh = 2 * (int)ty - im.halo + h + a, ww = 2 * (int)tx - im.halo + k;
+        const bool in = t < ep.tiles && (unsigned)hh < (unsigned)im.Hi && (unsigned)ww < (unsigned)im.Wi;
+        poff[a][k] = in ? ((n * (unsigned)im.Ci) * (unsigned)HW + (unsigned)(hh * im.Wi + ww)) * 4u : kInvalidByteOff;
+      }
+  }
+  const uint32_t chan_stride = (uint32_t)HW * 4u;
+  const uint32_t tap_mul = im.blk5 ? chan_stride : 4u * chan_stride;
+  const uint32_t tap_add = im.blk5 ? (uint32_t)(3 * (wave >> 1) * im.Wi + 3 * (wave & 1)) * 4u : (uint32_t)wave * chan_stride;
+  auto issue_u = [&](int i, int cg, int buf) {
+    dma_load16(rsU, lds0 + (uint32_t)buf * kWinoStage2 + (uint32_t)(wave * 4 + i) * 1024u, voffA,
+               (uint32_t)(wave * 4 + i) * strideF + (uint32_t)(cg0 + cg) * strideA);
+  };
+  float taps[2][3][4];
+  auto issue_tap = [&](int i, int cg, float (&d)[3][4]) {
+    d[i >> 2][i & 3] = __builtin_bit_cast(float, __builtin_amdgcn_raw_buffer_load_b32(
+                                                     rsX, (int)poff[i >> 2][i & 3], (int)((uint32_t)(cg0 + cg) * tap_mul + tap_add), 0));
+  };
+  const int fe = h ? 12 : 0, fo = h ? 8 : 4;
+  float* const vdst = lds_dyn + kWinoSA2 / 4 + (wave >> 1) * (kWinoBN * 2) + r * 2 + (wave & 1);
+  float te[4], to[4];
+  auto transform_cols = [&](const float (&d)[3][4]) {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      te[k] = d[0][k] - d[2][k];
+      to[k] = h ? d[1][k] - d[0][k] : d[1][k] + d[2][k];
+    }
+  };
+  auto transform_row = [&](int which, int buf) {
+    float* d = vdst + buf * (kWinoStage2 / 4) + (which ? fo : fe) * 128;
+    const float* t = which ? to : te;
+    d[0 * 128] = t[0] - t[2];
+    d[1 * 128] = t[1] + t[2];
+    d[2 * 128] = t[2] - t[1];
+    d[3 * 128] = t[1] - t[3];
+  };
+
+  f32x16 acc[8];
+#pragma unroll
+  for (int f = 0; f < 8; ++f)
+#pragma unroll
+    for (int v = 0; v < 16; ++v) acc[f][v] = 0.0f;
+
+  // U of stages 0 and 1 and the taps of 0, 1 and 2 on their way, stage 0's image operand made
+#pragma unroll
+  for (int i = 0; i < 4; ++i) issue_u(i, 0, 0);
+#pragma unroll
+  for (int i = 0; i < 12; ++i) issue_tap(i, 0, taps[0]);
+  if (nk > 1) {
+#pragma unroll
+    for (int i = 0; i < 4; ++i) issue_u(i, 1, 1);
+#pragma unroll
+    for (int i = 0; i < 12; ++i) issue_tap(i, 1, taps[1]);
+  }
+  wait_vmcnt<0>();
+  transform_cols(taps[0]);
+  transform_row(0, 0);
+  transform_row(1, 0);
+  if (nk > 2) {
+#pragma unroll
+    for (int i = 0; i < 12; ++i) issue_tap(i, 2, taps[0]);
+  }
+  __syncthreads();
+
+  const int a_rd = fh * (8 * 256) + h * (kWinoBM2 * 2) + (rw * 32 + r) * 2;
+  const int b_rd = fh * (8 * 128) + h * (kWinoBN * 2) + r * 2;
+  auto stage_a = [&](int buf) { return reinterpret_cast<const float2*>(lds_dyn + buf * (kWinoStage2 / 4) + a_rd); };
+  auto stage_b = [&](int buf) { return reinterpret_cast<const float2*>(lds_dyn + buf * (kWinoStage2 / 4) + kWinoSA2 / 4 + b_rd); };
+  float2 a[2][4], b[2][4];
+#pragma unroll
+  for (int q = 0; q < 4; ++q) {
+    a[0][q] = stage_a(0)[q * 128];
+    b[0][q] = stage_b(0)[q * 64];
+  }
+
+  // Stage `it` (parity BUF): MFMAs on buffer BUF; before its last quarter the image operand of stage it + 1 is made from the
+  // taps loaded two stages ago and the stage's one barrier stands; behind it the loads of U of stage it + 2 (into BUF: all
+  // of its operands have been read) and of the taps of stage it + 3, and the first operands of stage it + 1.
+  auto step = [&](int it, auto buf_tag, auto full_tag) {
+    constexpr int BUF = decltype(buf_tag)::value;
+    constexpr bool FULL = decltype(full_tag)::value;   // there is a stage it + 3
+    const bool more1 = FULL || it + 1 < nk, more2 = FULL || it + 2 < nk, more3 = FULL || it + 3 < nk;
+    const float2* pa = stage_a(BUF);
+    const float2* pb = stage_b(BUF);
+    const float2* pna = stage_a(BUF ^ 1);
+    const float2* pnb = stage_b(BUF ^ 1);
+    float (&nt)[3][4] = taps[BUF ^ 1];
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      acc[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[0][q].x, b[0][q].x, acc[q], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      a[1][q] = pa[(4 + q) * 128];
+      b[1][q] = pb[(4 + q) * 64];
+      __builtin_amdgcn_sched_barrier(0);
+    }
+#pragma unroll
+    for (int q = 0; q < 4; ++q) acc[q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[0][q].y, b[0][q].y, acc[q], 0, 0, 0);
+    __builtin_amdgcn_sched_barrier(0);
+    // U of stage it + 1 and its taps are there when only the twelve taps of stage it + 2 are in flight
+    if (FULL || more2) wait_vmcnt<12>();
+    else wait_vmcnt<0>();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      acc[4 + q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[1][q].x, b[1][q].x, acc[4 + q], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      if (more1) {
+        if (q == 0) transform_cols(nt);
+        if (q == 1) transform_row(0, BUF ^ 1);
+        if (q == 2) transform_row(1, BUF ^ 1);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      acc[4 + q] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[1][q].y, b[1][q].y, acc[4 + q], 0, 0, 0);
+      __builtin_amdgcn_sched_barrier(0);
+      a[0][q] = pna[q * 128];
+      b[0][q] = pnb[q * 64];
+      if (more2) {
+        if (q == 0) {
+#pragma unroll
+          for (int i = 0; i < 4; ++i) issue_u(i, it + 2, BUF);
+        }
+      }
+      if (more3 && q > 0) {
+#pragma unroll
+        for (int i = 4 * (q - 1); i < 4 * q; ++i) issue_tap(i, it + 3, nt);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+  };
+  int it = 0;
+  for (; it + 4 < nk; it += 2) {
+    step(it, std::integral_constant<int, 0>(), std::true_type());
+    step(it + 1, std::integral_constant<int, 1>(), std::true_type());
+  }
+  for (; it < nk; it += 2) {
+    step(it, std::integral_constant<int, 0>(), std::false_type());
+    if (it + 1 < nk) step(it + 1, std::integral_constant<int, 1>(), std::false_type());
+  }
+
+  // Wave fh stores row fh of the 2x2 pixels.  With M rows ma, mb of its f (i = 0, 1 or 2, 3) the two rows of A^T M are
+  // (ma + mb, mb) of the lower f plus (ma, -ma - mb) of the upper: a wave keeps +-(ma + mb) and gives the partner (wave ^ 2)
+  // mb or ma, both after the row pass, through LDS.
+  __syncthreads();
+  float2* const xch = reinterpret_cast<float2*>(lds_dyn);   // [wave][element][lane]
+#pragma unroll
+  for (int e = 0; e < 16; ++e) {
+    if (e % 4 == 0) {
+      __builtin_amdgcn_sched_barrier(0);
+      wino_pin_acc(acc);
+    }
+    float g[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const float ma = wino_acc_elem(acc[j], e), mb = wino_acc_elem(acc[4 + j], e);
+      g[j] = fh ? ma : mb;
+    }
+    xch[(wave * 16 + e) * 64 + lane] = make_float2(g[0] + g[1] + g[2], g[1] - g[2] - g[3]);
+  }
+  WinoOut<1> o;
+  o.init(ep, m0 + rw * 32, n0, lane, fh);
+  float bv[16];
+#pragma unroll
+  for (int e = 0; e < 16; ++e) bv[e] = o.bias(e);
+  const float sign = fh ? -1.0f : 1.0f;
+  __syncthreads();
+  constexpr int EB = 4;
+#pragma unroll
+  for (int e0 = 0; e0 < 16; e0 += EB) {
+    __builtin_amdgcn_sched_barrier(0);
+    wino_pin_acc(acc);
+    float y[EB][1][2];
+#pragma unroll
+    for (int e4 = 0; e4 < EB; ++e4) {
+      float t[4];
+#pragma unroll
+      for (int j = 0; j < 4; ++j) t[j] = wino_acc_elem(acc[j], e0 + e4) + wino_acc_elem(acc[4 + j], e0 + e4);
+      const float2 p = xch[((wave ^ 2) * 16 + e0 + e4) * 64 + lane];
+      y[e4][0][0] = fmaf(sign, t[0] + t[1] + t[2], p.x);
+      y[e4][0][1] = fmaf(sign, t[1] - t[2] - t[3], p.y);
+    }
+    wino_store_block<EB, 1>(o, ep, e0, y, bv + e0);
+  }
+}
+
 // ---- filter gradient --------------------------------------------------------------------------------------------------
 //   dg = G^T [ sum over tiles (A dY A^T) o (B^T d B) ] G      A dY A^T: the 2x2 tile of dy -> 4x4,  A = [1 0; 1 1; 1 -1; 0 -1]
 // The same 16 products with the roles turned: rows = filters, columns = input channels, the contraction runs over
@@ -1115,7 +1395,7 @@ __global__ __launch_bounds__(256) void wino_filter_prep_kernel(WinoFilterPrepArg
 struct WinoTailReduce {
   const float* part; float* out; const float* bias; const float* mask;
   float alpha, beta;
-  int relu, S, Ko, P, Q, TP, TQ, tiles_m, full;
+  int relu, S, Ko, P, Q, TP, TQ, tiles_m, bm, full;
   unsigned first, total;       // elements [first, total) of the result
   long long slab_elems;
   FastDiv dPQ, dQ, dKo;
@@ -1129,7 +1409,7 @@ __global__ __launch_bounds__(256) void wino_tail_reduce_kernel(WinoTailReduce a)
   a.dKo.divmod(plane, n, k);
   a.dQ.divmod(pix, pp, qq);
   const unsigned t = (n * (unsigned)a.TP + (pp >> 1)) * (unsigned)a.TQ + (qq >> 1);
-  const unsigned logical = (t / kWinoBN) * (unsigned)a.tiles_m + k / kWinoBM;
+  const unsigned logical = (t / kWinoBN) * (unsigned)a.tiles_m + k / (unsigned)a.bm;
   if (logical < (unsigned)a.full) return;
   float v = 0.0f;
   for (int sl = 0; sl < a.S; ++sl) v += a.part[(long long)sl * a.slab_elems + i];
@@ -1185,7 +1465,7 @@ int launch_conv_wino(const WinoGeom& g, bool bwd, const float* in, const float* 
   ep.Ko = g.Ko; ep.P = g.P; ep.Q = g.Q; ep.tiles = (unsigned)g.tiles;
   ep.out_bytes = (unsigned)(4ull * (unsigned long long)g.N * g.Ko * g.P * g.Q);
   ep.dTQ = a.dTQ; ep.dTP = a.dTP;
-  const int tiles_m_ = g.rows_p / kWinoBM;
+  const int tiles_m_ = g.rows_p / g.bm;
   const long long tiles_n_ = g.tiles_p / kWinoBN;
   if (fused) {
     constexpr size_t lds_f = (size_t)kWinoR * kWinoStage + 2 * (size_t)kWinoRaw;
@@ -1203,13 +1483,18 @@ int launch_conv_wino(const WinoGeom& g, bool bwd, const float* in, const float* 
     tl.slab_elems = g.slab_elems; tl.part_first = g.part_first;
     const long long T = (long long)tiles_m_ * tiles_n_;
     const long long blocks = g.tail_S > 1 ? g.full_tiles + (T - g.full_tiles) * g.tail_S : T;
-    hipLaunchKernelGGL(wino_gemm_fused_kernel, dim3((unsigned)blocks), dim3(256), lds_f, stream, U, im, g.Cg, g.rows_p, tiles_m_,
-                       (unsigned)(16ull * g.Cg * 2 * g.rows_p * 8), ep, tl);
+    const unsigned u_bytes = (unsigned)(16ull * g.Cg * 2 * g.rows_p * 8);
+    if (g.bm == kWinoBM2)
+      hipLaunchKernelGGL(wino_gemm64_kernel, dim3((unsigned)blocks), dim3(256), 2 * (size_t)kWinoStage2, stream, U, im, g.Cg, g.rows_p,
+                         tiles_m_, u_bytes, ep, tl);
+    else
+      hipLaunchKernelGGL(wino_gemm_fused_kernel, dim3((unsigned)blocks), dim3(256), lds_f, stream, U, im, g.Cg, g.rows_p, tiles_m_,
+                         u_bytes, ep, tl);
     if (g.tail_S > 1) {
       if (int e = launch_status()) return e;
       WinoTailReduce r;
       r.part = tl.part; r.out = out; r.bias = bias; r.mask = mask; r.alpha = alpha; r.beta = beta; r.relu = relu;
-      r.S = g.tail_S; r.Ko = g.Ko; r.P = g.P; r.Q = g.Q; r.TP = g.TP; r.TQ = g.TQ; r.tiles_m = tiles_m_; r.full = g.full_tiles;
+      r.S = g.tail_S; r.Ko = g.Ko; r.P = g.P; r.Q = g.Q; r.TP = g.TP; r.TQ = g.TQ; r.tiles_m = tiles_m_; r.bm = g.bm; r.full = g.full_tiles;
       r.first = (unsigned)g.part_first; r.total = (unsigned)((long long)g.N * g.Ko * g.P * g.Q);
       r.slab_elems = g.slab_elems;
       r.dPQ = FastDiv((uint32_t)(g.P * g.Q)); r.dQ = FastDiv((uint32_t)g.Q); r.dKo = FastDiv((uint32_t)g.Ko);

@@ -288,6 +288,36 @@ def test_conv2d_winograd(dev, case):
     torch.cuda.synchronize()
 
 
+@pytest.mark.parametrize("case", [(3, 4, 9, 7, 64, 1), (2, 8, 13, 13, 64, 1), (2, 12, 8, 9, 33, 0), (3, 16, 7, 7, 50, 2), (2, 20, 11, 6, 64, 1),
+                                  (1, 24, 10, 10, 7, 1), (2, 28, 5, 5, 64, 1), (3, 64, 14, 14, 192, 1), (1, 4, 1, 1, 64, 1),
+                                  (9, 64, 56, 56, 64, 1), (24, 64, 56, 55, 64, 1)], ids=str)
+def test_conv2d_winograd_64_rows(dev, case):
+    """The 64-row tiles of up to 64, 192, ... filters: channel loops of one to seven stages (every way the pipeline starts
+    and drains) and of sixteen, ragged rows and tiles, borders of 0, 1, 2, blocks in slices (9 images) and whole rounds;
+    forward with the fused epilogue, the data gradient masked and blended; the library's own choice."""
+    Nn, C, H, W, K, pad = case
+    say("winograd 64-row case", case)
+    WG = _lib.RH_ALGO_WINOGRAD
+    x, w, b = synth.normal(15, 1, (Nn, C, H, W)), synth.normal(15, 2, (K, C, 3, 3)), synth.normal(15, 3, (K,))
+    y_ref = O.conv2d_fwd(x, w, 1, pad)
+    dy, dx0 = synth.normal(15, 4, y_ref.shape), synth.normal(15, 8, x.shape)
+    xd, wd, bd, dyd = T(x, dev), T(w, dev), T(b, dev), T(dy, dev)
+    y = ops.conv2d_fwd(xd, wd, 1, pad, algo=WG)
+    assert_close(N(y), y_ref, "winograd fwd")
+    yf = ops.conv2d_fwd(xd, wd, 1, pad, bias=bd, relu=True, algo=WG)
+    assert torch.equal(torch.clamp_min(y + bd.view(1, -1, 1, 1), 0.0), yf), "fused epilogue == conv, add_bias, rect"
+    assert_close(N(ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=WG)), O.conv2d_bwd_data(w, dy, x.shape, 1, pad), "winograd bwd data")
+    for alpha, beta in ((1.0, 0.0), (0.5, 2.0)):
+        two = ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, alpha=alpha, beta=beta, dx=T(dx0, dev), algo=WG)
+        assert_close(N(two), O.conv2d_bwd_data(w, dy, x.shape, 1, pad, alpha, beta, dx0.copy()), "winograd bwd data alpha/beta")
+        ops.rect_backprop_inplace(xd, two)
+        one = ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, alpha=alpha, beta=beta, dx=T(dx0, dev), algo=WG, relu_of=xd)
+        assert torch.equal(one, two), "masked data gradient alpha=%g beta=%g" % (alpha, beta)
+    assert torch.equal(ops.conv2d_fwd(xd, wd, 1, pad, algo=WG), y), "run to run the same bits"
+    if Nn >= 24:
+        assert torch.equal(ops.conv2d_fwd(xd, wd, 1, pad), y), "library's choice"
+
+
 WINO5_CASES = [
     # N, C, H, W, K, pad
     (2, 3, 9, 9, 8, 2),
