@@ -213,6 +213,9 @@ void rembrandt_kernel_batch_map_rect_inplace(float* y, int32_t frame_len, int32_
                                              rh_stream_t stream);
 void rembrandt_kernel_batch_map_rect_backprop_inplace(const float* y, int32_t frame_len,
                                                       int32_t batch, float* dy, rh_stream_t stream);
+/* The ReLU backward of a residual unit: dy[i] = y[i] > 0 ? dy[i] : 0, and the result in `copy` as well (the gradient of the
+ * unit's input starts from it).  The three tensors of n values do not overlap. */
+int rh_rect_backprop_copy(const float* y, float* dy, float* copy, size_t n, rh_stream_t stream);
 
 /* ---------------------------------------------------------------------------------------------
  * Column-major SGEMM and BLAS-1.  Replaces array_cuda's BlasMatrixExt::matrix_prod
@@ -430,6 +433,15 @@ int rh_bnorm_fwd_train(int N, int C, int plane, float alpha, const float* x, flo
 int rh_bnorm_fwd_infer(int N, int C, int plane, float alpha, const float* x, float beta, float* y, double epsilon,
                        const float* scale, const float* bias, const float* running_mean, const float* running_ivar,
                        void* ws, size_t ws_bytes, int flags, rh_stream_t stream);
+/* The same with the blend's second term from another tensor: y = alpha*(...) + beta*y0, y0 whole and apart from y, or y
+ * itself (a residual unit's input, which the reference copies to y first, src/operator/conv.rs:1627-1665). */
+int rh_bnorm_fwd_train_add(int N, int C, int plane, float alpha, const float* x, float beta, const float* y0, float* y,
+                           double ema_factor, double epsilon, const float* scale, const float* bias, float* running_mean,
+                           float* running_ivar, float* cached_mean, float* cached_ivar, void* ws, size_t ws_bytes, int flags,
+                           rh_stream_t stream);
+int rh_bnorm_fwd_infer_add(int N, int C, int plane, float alpha, const float* x, float beta, const float* y0, float* y,
+                           double epsilon, const float* scale, const float* bias, const float* running_mean,
+                           const float* running_ivar, void* ws, size_t ws_bytes, int flags, rh_stream_t stream);
 int rh_bnorm_bwd(int N, int C, int plane, float alpha_data, float beta_data, const float* x, const float* dy, float* dx,
                  float alpha_param, float beta_param, double epsilon, const float* scale, float* dscale, float* dbias,
                  const float* cached_mean, const float* cached_ivar, void* ws, size_t ws_bytes, rh_stream_t stream);

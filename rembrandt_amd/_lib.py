@@ -73,6 +73,9 @@ PROTOTYPES = {
     "rh_bnorm_workspace_bytes": (_sz, [_int, _int, _int]),
     "rh_bnorm_fwd_train": (_int, [_int, _int, _int, _f, _vp, _f, _vp, C.c_double, C.c_double, _vp, _vp, _vp, _vp, _vp, _vp,
                                   _vp, _sz, _int, _vp]),
+    "rh_bnorm_fwd_train_add": (_int, [_int, _int, _int, _f, _vp, _f, _vp, _vp, C.c_double, C.c_double, _vp, _vp, _vp, _vp, _vp, _vp,
+                                      _vp, _sz, _int, _vp]),
+    "rh_bnorm_fwd_infer_add": (_int, [_int, _int, _int, _f, _vp, _f, _vp, _vp, C.c_double, _vp, _vp, _vp, _vp, _vp, _sz, _int, _vp]),
     "rh_bnorm_fwd_infer": (_int, [_int, _int, _int, _f, _vp, _f, _vp, C.c_double, _vp, _vp, _vp, _vp, _vp, _sz, _int, _vp]),
     "rh_bnorm_bwd": (_int, [_int, _int, _int, _f, _f, _vp, _vp, _vp, _f, _f, C.c_double, _vp, _vp, _vp, _vp, _vp, _vp, _sz,
                             _vp]),
@@ -104,6 +107,7 @@ PROTOTYPES = {
     "rh_conv2d_bwd_data_relu": (_int, [C.POINTER(ConvGeom), _f, _vp, _vp, _f, _vp, _vp, _vp, _sz, _int, _vp]),
     "rh_add_bias_nchw": (_int, [_vp, _vp, _i32, _i32, _i32, _f, _f, _vp]),
     "rembrandt_kernel_batch_map_rect_inplace": (None, [_vp, _i32, _i32, _vp]),
+    "rh_rect_backprop_copy": (_int, [_vp, _vp, _vp, _sz, _vp]),
     "rembrandt_kernel_batch_map_rect_backprop_inplace": (None, [_vp, _i32, _i32, _vp, _vp]),
     "rh_sgemm_workspace_bytes": (_sz, [_i32, _i32, _i32]),
     "rh_sgemm": (_int, [_int, _int, _i32, _i32, _i32, _f, _vp, _i32, _vp, _i32, _f, _vp, _i32, _vp, _sz, _int, _vp]),

@@ -187,8 +187,10 @@ __global__ void bn_finish_kernel(Stats stats, const float* __restrict__ x, const
   coef[c] = bn_finish(stats, c, x[(size_t)c * plane], s0, s1, true);
 }
 
-// Forward:  out = alpha * f((x - mean)*a + b) + beta*out, f = identity or max(., 0) applied after the blend when RELU.
-// Backward: out = alpha * a*(dy - c2 - (x - mean)*c3) + beta*out.
+// Forward:  out = alpha * f((x - mean)*a + b) + beta*old, f = identity or max(., 0) applied after the blend when RELU.
+// (old: out itself, or the tensor a residual unit adds.  Read where it lies, 5 residual units need no copy of their input in
+// front of this pass: 46 us each for 256 x 64 x 56 x 56, 3 to 5 us for a few images.)
+// Backward: out = alpha * a*(dy - c2 - (x - mean)*c3) + beta*old.
 // MASK (backward only): dy is taken as 0 where the forward ReLU clamped, see bn_reduce_kernel; mb = the layer's bias.
 template <bool BWD, bool RELU, bool MASK>
 __device__ __forceinline__ float bn_one(float xv, float gv, float ov, const float4 k, float mb, float alpha, float beta) {
@@ -242,7 +244,7 @@ struct BnUnits {
 // values) 41 -> 24 us.
 // T = float4 (plane % 4 == 0 and 16-byte aligned tensors, so a unit never crosses a plane) or float.
 template <class T, bool BWD, bool RELU, bool MASK, int THREADS, int U, class Stats>
-__global__ __launch_bounds__(THREADS) void bn_channel_kernel(const T* x, const T* dy, T* out, Stats stats, BnUnits un,
+__global__ __launch_bounds__(THREADS) void bn_channel_kernel(const T* x, const T* dy, const T* old, T* out, Stats stats, BnUnits un,
                                                              uint32_t units, float alpha, float beta, const float* mask_bias) {
   const uint32_t c = blockIdx.x, t = threadIdx.x;
   T xv[U], gv[U], ov[U];
@@ -254,7 +256,7 @@ __global__ __launch_bounds__(THREADS) void bn_channel_kernel(const T* x, const T
       const size_t at = un.at(c, i);
       xv[k] = x[at];
       if constexpr (BWD) gv[k] = dy[at];
-      if (beta != 0.0f) ov[k] = out[at];
+      if (beta != 0.0f) ov[k] = old[at];
     }
   }
   float shift, m_si = 0.0f, mb = 0.0f;
@@ -285,7 +287,7 @@ __global__ __launch_bounds__(THREADS) void bn_channel_kernel(const T* x, const T
 // T = float4 or float as above.  (Forming the coefficients here, each wave adding its channel's partials, saved the finish
 // launch of 9 us and cost this kernel 15: 94 -> 109 us backward on 256 x 64 x 56 x 56.)
 template <class T, bool BWD, bool RELU, bool MASK>
-__global__ __launch_bounds__(256) void bn_apply_kernel(const T* x, const T* dy, T* out, const float4* __restrict__ coef,
+__global__ __launch_bounds__(256) void bn_apply_kernel(const T* x, const T* dy, const T* old, T* out, const float4* __restrict__ coef,
                                                        uint32_t groups, FastDiv plane_groups, FastDiv chans, float alpha,
                                                        float beta, const float* __restrict__ mask_bias) {
   const uint32_t i = blockIdx.x * 256 + threadIdx.x;
@@ -298,13 +300,13 @@ __global__ __launch_bounds__(256) void bn_apply_kernel(const T* x, const T* dy, 
   bn_zero(gv); bn_zero(ov);
   const T xv = x[i];
   if constexpr (BWD) gv = dy[i];
-  if (beta != 0.0f) ov = out[i];
+  if (beta != 0.0f) ov = old[i];
   out[i] = bn_one<BWD, RELU, MASK>(xv, gv, ov, k, mb, alpha, beta);
 }
 
 // Inference: the coefficients are a handful of cached loads per thread.
 template <class T, bool RELU>
-__global__ __launch_bounds__(256) void bn_infer_kernel(const T* x, T* out, const float* __restrict__ scale,
+__global__ __launch_bounds__(256) void bn_infer_kernel(const T* x, const T* old, T* out, const float* __restrict__ scale,
                                                        const float* __restrict__ bias, const float* __restrict__ running_mean,
                                                        const float* __restrict__ running_ivar, uint32_t groups, FastDiv plane_groups,
                                                        FastDiv chans, float alpha, float beta) {
@@ -312,7 +314,7 @@ __global__ __launch_bounds__(256) void bn_infer_kernel(const T* x, T* out, const
   if (i >= groups) return;
   T ov;
   bn_zero(ov);
-  if (beta != 0.0f) ov = out[i];
+  if (beta != 0.0f) ov = old[i];
   const T xv = x[i];
   const uint32_t row = plane_groups.quot(i);  // n*C + c
   const uint32_t c = row - chans.quot(row) * chans.div;
@@ -320,15 +322,16 @@ __global__ __launch_bounds__(256) void bn_infer_kernel(const T* x, T* out, const
   out[i] = bn_one<false, RELU, false>(xv, xv, ov, k, 0.0f, alpha, beta);
 }
 
-inline bool bn_vec(int plane, const void* a, const void* b, const void* c) {
-  return plane % 4 == 0 && ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c)) & 15) == 0;
+inline bool bn_vec(int plane, const void* a, const void* b, const void* c, const void* d = nullptr) {
+  return plane % 4 == 0 && ((reinterpret_cast<uintptr_t>(a) | reinterpret_cast<uintptr_t>(b) | reinterpret_cast<uintptr_t>(c) |
+                             reinterpret_cast<uintptr_t>(d)) & 15) == 0;
 }
 
 template <class T, bool BWD, bool RELU, bool MASK, int THREADS, int U, class Stats>
-void launch_bn_channel(const float* x, const float* dy, float* out, const Stats& stats, const BnUnits& un, uint32_t units,
+void launch_bn_channel(const float* x, const float* dy, const float* old, float* out, const Stats& stats, const BnUnits& un, uint32_t units,
                        float alpha, float beta, const float* mask_bias, hipStream_t st) {
   hipLaunchKernelGGL((bn_channel_kernel<T, BWD, RELU, MASK, THREADS, U, Stats>), dim3(un.C), dim3(THREADS), 0, st,
-                     reinterpret_cast<const T*>(x), reinterpret_cast<const T*>(dy), reinterpret_cast<T*>(out), stats, un, units,
+                     reinterpret_cast<const T*>(x), reinterpret_cast<const T*>(dy), reinterpret_cast<const T*>(old), reinterpret_cast<T*>(out), stats, un, units,
                      alpha, beta, mask_bias);
 }
 
@@ -342,53 +345,53 @@ inline bool bn_whole(bool bwd, bool vec, int N, int plane) {
 }
 
 template <bool BWD, bool RELU, bool MASK, class Stats>
-void launch_bn_whole(const float* x, const float* dy, float* out, const Stats& stats, int N, int C, int plane, float alpha,
+void launch_bn_whole(const float* x, const float* dy, const float* old, float* out, const Stats& stats, int N, int C, int plane, float alpha,
                      float beta, const float* mask_bias, hipStream_t st) {
   const long long values = (long long)N * plane;
   BnUnits un;
   un.C = (uint32_t)C;
-  if (bn_vec(plane, x, dy, out)) {
+  if (bn_vec(plane, x, dy, out, old)) {
     un.pu = (uint32_t)(plane / 4);
     un.by_plane = FastDiv(un.pu);
     const uint32_t units = (uint32_t)(values / 4);
-    if (units <= 256 * 2) launch_bn_channel<float4, BWD, RELU, MASK, 256, 2>(x, dy, out, stats, un, units, alpha, beta, mask_bias, st);
-    else if (units <= 512 * 4) launch_bn_channel<float4, BWD, RELU, MASK, 512, 4>(x, dy, out, stats, un, units, alpha, beta, mask_bias, st);
-    else launch_bn_channel<float4, BWD, RELU, MASK, 1024, 5>(x, dy, out, stats, un, units, alpha, beta, mask_bias, st);
+    if (units <= 256 * 2) launch_bn_channel<float4, BWD, RELU, MASK, 256, 2>(x, dy, old, out, stats, un, units, alpha, beta, mask_bias, st);
+    else if (units <= 512 * 4) launch_bn_channel<float4, BWD, RELU, MASK, 512, 4>(x, dy, old, out, stats, un, units, alpha, beta, mask_bias, st);
+    else launch_bn_channel<float4, BWD, RELU, MASK, 1024, 5>(x, dy, old, out, stats, un, units, alpha, beta, mask_bias, st);
   } else {
     un.pu = (uint32_t)plane;
     un.by_plane = FastDiv(un.pu);
     const uint32_t units = (uint32_t)values;
-    if (units <= 256 * 6) launch_bn_channel<float, BWD, RELU, MASK, 256, 6>(x, dy, out, stats, un, units, alpha, beta, mask_bias, st);
-    else if (units <= 1024 * 6) launch_bn_channel<float, BWD, RELU, MASK, 1024, 6>(x, dy, out, stats, un, units, alpha, beta, mask_bias, st);
-    else if constexpr (!BWD) launch_bn_channel<float, BWD, RELU, MASK, 1024, 20>(x, dy, out, stats, un, units, alpha, beta, mask_bias, st);
+    if (units <= 256 * 6) launch_bn_channel<float, BWD, RELU, MASK, 256, 6>(x, dy, old, out, stats, un, units, alpha, beta, mask_bias, st);
+    else if (units <= 1024 * 6) launch_bn_channel<float, BWD, RELU, MASK, 1024, 6>(x, dy, old, out, stats, un, units, alpha, beta, mask_bias, st);
+    else if constexpr (!BWD) launch_bn_channel<float, BWD, RELU, MASK, 1024, 20>(x, dy, old, out, stats, un, units, alpha, beta, mask_bias, st);
   }
 }
 
 template <bool BWD, bool RELU, bool MASK>
-void launch_bn_apply(const float* x, const float* dy, float* out, const float4* coef, int N, int C, int plane, float alpha,
+void launch_bn_apply(const float* x, const float* dy, const float* old, float* out, const float4* coef, int N, int C, int plane, float alpha,
                      float beta, const float* mask_bias, hipStream_t st) {
   auto go = [&](auto zero, int width) {
     using T = decltype(zero);
     const uint32_t groups = (uint32_t)((long long)N * C * plane / width);
     hipLaunchKernelGGL((bn_apply_kernel<T, BWD, RELU, MASK>), dim3(cdiv(groups, 256u)), dim3(256), 0, st,
-                       reinterpret_cast<const T*>(x), reinterpret_cast<const T*>(dy), reinterpret_cast<T*>(out), coef, groups,
+                       reinterpret_cast<const T*>(x), reinterpret_cast<const T*>(dy), reinterpret_cast<const T*>(old), reinterpret_cast<T*>(out), coef, groups,
                        FastDiv((uint32_t)(plane / width)), FastDiv((uint32_t)C), alpha, beta, mask_bias);
   };
-  if (bn_vec(plane, x, dy, out)) go(float4(), 4);
+  if (bn_vec(plane, x, dy, out, old)) go(float4(), 4);
   else go(0.0f, 1);
 }
 
 template <bool RELU>
-void launch_bn_infer(const float* x, float* out, const float* scale, const float* bias, const float* running_mean,
+void launch_bn_infer(const float* x, const float* old, float* out, const float* scale, const float* bias, const float* running_mean,
                      const float* running_ivar, long long total, int C, int plane, float alpha, float beta, hipStream_t st) {
   auto go = [&](auto zero, int width) {
     using T = decltype(zero);
     const uint32_t groups = (uint32_t)(total / width);
     hipLaunchKernelGGL((bn_infer_kernel<T, RELU>), dim3(cdiv(groups, 256u)), dim3(256), 0, st, reinterpret_cast<const T*>(x),
-                       reinterpret_cast<T*>(out), scale, bias, running_mean, running_ivar, groups,
+                       reinterpret_cast<const T*>(old), reinterpret_cast<T*>(out), scale, bias, running_mean, running_ivar, groups,
                        FastDiv((uint32_t)(plane / width)), FastDiv((uint32_t)C), alpha, beta);
   };
-  if (bn_vec(plane, x, out, nullptr)) go(float4(), 4);
+  if (bn_vec(plane, x, out, old)) go(float4(), 4);
   else go(0.0f, 1);
 }
 
@@ -431,12 +434,12 @@ extern "C" size_t rh_bnorm_workspace_bytes_upto(int N, int C, int plane) {
 }
 
 template <bool RELU>
-static void bn_fwd_train(int N, int C, int plane, float alpha, const float* x, float beta, float* y, const BnFwdStats& stats,
+static void bn_fwd_train(int N, int C, int plane, float alpha, const float* x, float beta, const float* y0, float* y, const BnFwdStats& stats,
                          void* ws, hipStream_t st) {
   const double total = (double)N * C * plane;
-  if (bn_whole(false, bn_vec(plane, x, y, nullptr), N, plane)) {
+  if (bn_whole(false, bn_vec(plane, x, y, y0), N, plane)) {
     ProfScope prof("bnorm_fwd", (beta != 0.0f ? 12.0 : 8.0) * total, st);
-    return launch_bn_whole<false, RELU, false>(x, nullptr, y, stats, N, C, plane, alpha, beta, nullptr, st);
+    return launch_bn_whole<false, RELU, false>(x, nullptr, y0, y, stats, N, C, plane, alpha, beta, nullptr, st);
   }
   const BnPlan p = bn_plan(N, C, plane);
   float2* part = static_cast<float2*>(ws);
@@ -447,41 +450,56 @@ static void bn_fwd_train(int N, int C, int plane, float alpha, const float* x, f
     hipLaunchKernelGGL(bn_finish_kernel<BnFwdStats>, dim3(cdiv(C, 64)), dim3(64), 0, st, stats, x, part, p.G, C, plane, coef);
   }
   ProfScope prof("bnorm_fwd_apply", (beta != 0.0f ? 12.0 : 8.0) * total, st);
-  launch_bn_apply<false, RELU, false>(x, nullptr, y, coef, N, C, plane, alpha, beta, nullptr, st);
+  launch_bn_apply<false, RELU, false>(x, nullptr, y0, y, coef, N, C, plane, alpha, beta, nullptr, st);
 }
 
-extern "C" int rh_bnorm_fwd_train(int N, int C, int plane, float alpha, const float* x, float beta, float* y,
+extern "C" int rh_bnorm_fwd_train_add(int N, int C, int plane, float alpha, const float* x, float beta, const float* y0, float* y,
                                   double ema_factor, double epsilon, const float* scale, const float* bias,
                                   float* running_mean, float* running_ivar, float* cached_mean, float* cached_ivar,
                                   void* ws, size_t ws_bytes, int flags, rh_stream_t stream) {
   long long total;
   if (int e = bn_check(N, C, plane, &total)) return e;
   if (total == 0) return 0;
-  if (!x || !y || !scale || !bias || !running_mean || !running_ivar || !cached_mean || !cached_ivar || !ws) return RH_E_INVALID;
+  if (!x || !y0 || !y || !scale || !bias || !running_mean || !running_ivar || !cached_mean || !cached_ivar || !ws) return RH_E_INVALID;
   if (flags & ~RH_FUSE_RELU) return RH_E_UNSUPPORTED;
   if (ws_bytes < rh_bnorm_workspace_bytes(N, C, plane)) return RH_E_WORKSPACE;
   const BnFwdStats stats = {(double)N * (double)plane, ema_factor, epsilon, scale, bias,
                             running_mean, running_ivar, cached_mean, cached_ivar};
-  if (flags & RH_FUSE_RELU) bn_fwd_train<true>(N, C, plane, alpha, x, beta, y, stats, ws, to_stream(stream));
-  else bn_fwd_train<false>(N, C, plane, alpha, x, beta, y, stats, ws, to_stream(stream));
+  if (flags & RH_FUSE_RELU) bn_fwd_train<true>(N, C, plane, alpha, x, beta, y0, y, stats, ws, to_stream(stream));
+  else bn_fwd_train<false>(N, C, plane, alpha, x, beta, y0, y, stats, ws, to_stream(stream));
+  return launch_status();
+}
+
+extern "C" int rh_bnorm_fwd_train(int N, int C, int plane, float alpha, const float* x, float beta, float* y,
+                                  double ema_factor, double epsilon, const float* scale, const float* bias,
+                                  float* running_mean, float* running_ivar, float* cached_mean, float* cached_ivar,
+                                  void* ws, size_t ws_bytes, int flags, rh_stream_t stream) {
+  return rh_bnorm_fwd_train_add(N, C, plane, alpha, x, beta, y, y, ema_factor, epsilon, scale, bias, running_mean, running_ivar,
+                                cached_mean, cached_ivar, ws, ws_bytes, flags, stream);
+}
+
+extern "C" int rh_bnorm_fwd_infer_add(int N, int C, int plane, float alpha, const float* x, float beta, const float* y0, float* y,
+                                  double epsilon, const float* scale, const float* bias, const float* running_mean,
+                                  const float* running_ivar, void* ws, size_t ws_bytes, int flags, rh_stream_t stream) {
+  (void)epsilon;  // already inside the stored inverse standard deviation
+  long long total;
+  if (int e = bn_check(N, C, plane, &total)) return e;
+  if (total == 0) return 0;
+  if (!x || !y0 || !y || !scale || !bias || !running_mean || !running_ivar || !ws) return RH_E_INVALID;
+  if (flags & ~RH_FUSE_RELU) return RH_E_UNSUPPORTED;
+  if (ws_bytes < rh_bnorm_workspace_bytes(N, C, plane)) return RH_E_WORKSPACE;
+  hipStream_t st = to_stream(stream);
+  ProfScope prof("bnorm_fwd_apply", (beta != 0.0f ? 12.0 : 8.0) * (double)total, st);
+  if (flags & RH_FUSE_RELU) launch_bn_infer<true>(x, y0, y, scale, bias, running_mean, running_ivar, total, C, plane, alpha, beta, st);
+  else launch_bn_infer<false>(x, y0, y, scale, bias, running_mean, running_ivar, total, C, plane, alpha, beta, st);
   return launch_status();
 }
 
 extern "C" int rh_bnorm_fwd_infer(int N, int C, int plane, float alpha, const float* x, float beta, float* y, double epsilon,
                                   const float* scale, const float* bias, const float* running_mean,
                                   const float* running_ivar, void* ws, size_t ws_bytes, int flags, rh_stream_t stream) {
-  (void)epsilon;  // already inside the stored inverse standard deviation
-  long long total;
-  if (int e = bn_check(N, C, plane, &total)) return e;
-  if (total == 0) return 0;
-  if (!x || !y || !scale || !bias || !running_mean || !running_ivar || !ws) return RH_E_INVALID;
-  if (flags & ~RH_FUSE_RELU) return RH_E_UNSUPPORTED;
-  if (ws_bytes < rh_bnorm_workspace_bytes(N, C, plane)) return RH_E_WORKSPACE;
-  hipStream_t st = to_stream(stream);
-  ProfScope prof("bnorm_fwd_apply", (beta != 0.0f ? 12.0 : 8.0) * (double)total, st);
-  if (flags & RH_FUSE_RELU) launch_bn_infer<true>(x, y, scale, bias, running_mean, running_ivar, total, C, plane, alpha, beta, st);
-  else launch_bn_infer<false>(x, y, scale, bias, running_mean, running_ivar, total, C, plane, alpha, beta, st);
-  return launch_status();
+  return rh_bnorm_fwd_infer_add(N, C, plane, alpha, x, beta, y, y, epsilon, scale, bias, running_mean, running_ivar, ws, ws_bytes,
+                                flags, stream);
 }
 
 template <bool MASK>
@@ -490,7 +508,7 @@ static void bn_bwd(int N, int C, int plane, float alpha, const float* x, const f
   const double total = (double)N * C * plane;
   if (bn_whole(true, bn_vec(plane, x, dy, dx), N, plane)) {
     ProfScope prof("bnorm_bwd", (beta != 0.0f ? 16.0 : 12.0) * total, st);
-    return launch_bn_whole<true, false, MASK>(x, dy, dx, stats, N, C, plane, alpha, beta, relu_bias, st);
+    return launch_bn_whole<true, false, MASK>(x, dy, dx, dx, stats, N, C, plane, alpha, beta, relu_bias, st);
   }
   const BnPlan p = bn_plan(N, C, plane);
   float2* part = static_cast<float2*>(ws);
@@ -502,7 +520,7 @@ static void bn_bwd(int N, int C, int plane, float alpha, const float* x, const f
     hipLaunchKernelGGL(bn_finish_kernel<BnBwdStats>, dim3(cdiv(C, 64)), dim3(64), 0, st, stats, x, part, p.G, C, plane, coef);
   }
   ProfScope prof("bnorm_bwd_apply", (beta != 0.0f ? 16.0 : 12.0) * total, st);
-  launch_bn_apply<true, false, MASK>(x, dy, dx, coef, N, C, plane, alpha, beta, relu_bias, st);
+  launch_bn_apply<true, false, MASK>(x, dy, dx, dx, coef, N, C, plane, alpha, beta, relu_bias, st);
 }
 
 static int bnorm_bwd(int N, int C, int plane, float alpha_data, float beta_data, const float* x, const float* dy, float* dx,

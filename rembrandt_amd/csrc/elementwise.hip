@@ -56,10 +56,19 @@ __global__ void rect_inplace_kernel(float* __restrict__ y, long long n) {
   }
 }
 
-__global__ void rect_backprop_inplace_kernel(const float* __restrict__ y, float* __restrict__ dy, long long n) {
+// COPY: the result goes to `copy` too, 16 bytes a value where the pass and a copy behind it move 20 in two launches
+// (ResNet-18 template, five residual units).
+template <bool COPY>
+__global__ void rect_backprop_inplace_kernel(const float* __restrict__ y, float* __restrict__ dy, float* __restrict__ copy,
+                                             long long n) {
   const long long stride = (long long)gridDim.x * blockDim.x;
   const long long t = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-  if (((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(dy)) & 15) == 0) {
+  auto one = [&](long long i) {
+    const float v = y[i] > 0.0f ? dy[i] : 0.0f;
+    dy[i] = v;
+    if (COPY) copy[i] = v;
+  };
+  if (((reinterpret_cast<uintptr_t>(y) | reinterpret_cast<uintptr_t>(dy) | reinterpret_cast<uintptr_t>(copy)) & 15) == 0) {
     const long long n4 = n >> 2;
     const float4* y4 = reinterpret_cast<const float4*>(y);
     float4* d4 = reinterpret_cast<float4*>(dy);
@@ -69,10 +78,11 @@ __global__ void rect_backprop_inplace_kernel(const float* __restrict__ y, float*
       d.x = a.x > 0.0f ? d.x : 0.0f; d.y = a.y > 0.0f ? d.y : 0.0f;
       d.z = a.z > 0.0f ? d.z : 0.0f; d.w = a.w > 0.0f ? d.w : 0.0f;
       d4[i] = d;
+      if (COPY) reinterpret_cast<float4*>(copy)[i] = d;
     }
-    for (long long i = (n4 << 2) + t; i < n; i += stride) dy[i] = y[i] > 0.0f ? dy[i] : 0.0f;
+    for (long long i = (n4 << 2) + t; i < n; i += stride) one(i);
   } else {
-    for (long long i = t; i < n; i += stride) dy[i] = y[i] > 0.0f ? dy[i] : 0.0f;
+    for (long long i = t; i < n; i += stride) one(i);
   }
 }
 
@@ -143,9 +153,18 @@ extern "C" void rembrandt_kernel_batch_map_rect_backprop_inplace(const float* y,
   const long long n = (long long)frame_len * batch;
   if (n <= 0 || !y || !dy) { g_last_error = n == 0 ? 0 : RH_E_INVALID; return; }
   ProfScope prof("rect_bwd", 12.0 * (double)n, to_stream(stream));
-  hipLaunchKernelGGL(rect_backprop_inplace_kernel, dim3(stream_grid((size_t)(n + 3) / 4, 256)), dim3(256), 0,
-                     to_stream(stream), y, dy, n);
+  hipLaunchKernelGGL(rect_backprop_inplace_kernel<false>, dim3(stream_grid((size_t)(n + 3) / 4, 256)), dim3(256), 0,
+                     to_stream(stream), y, dy, nullptr, n);
   g_last_error = launch_status();
+}
+
+extern "C" int rh_rect_backprop_copy(const float* y, float* dy, float* copy, size_t n, rh_stream_t stream) {
+  if (n == 0) return 0;
+  if (!y || !dy || !copy) return RH_E_INVALID;
+  ProfScope prof("rect_bwd", 16.0 * (double)n, to_stream(stream));
+  hipLaunchKernelGGL(rect_backprop_inplace_kernel<true>, dim3(stream_grid((n + 3) / 4, 256)), dim3(256), 0, to_stream(stream), y,
+                     dy, copy, (long long)n);
+  return launch_status();
 }
 
 extern "C" int rh_memset_f32(float* d, float value, size_t n, rh_stream_t stream) {

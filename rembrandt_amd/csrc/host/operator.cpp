@@ -1328,21 +1328,22 @@ struct BNormConvUnit {
     fill(*scale, 1.0f); fill(*bias, 0.0f); fill(*running_mean, 0.0f); fill(*running_ivar, 1.0f);
   }
 
-  // out = beta_out*out + BN(conv(in)); `relu` clamps the blended result (the in-place rect that follows in the reference).
+  // out = beta_out*old + BN(conv(in)), old = out or a tensor apart from it; `relu` clamps the blended result (the in-place rect that follows in the reference).
   void forward(size_t batch, const float* in, float* out, float beta_out, OpPhase phase, const BNormMovingAverage& avg,
-               double epsilon, bool relu, DeviceBuffer<uint8_t>& ws, bool bf16) {
+               double epsilon, bool relu, DeviceBuffer<uint8_t>& ws, bool bf16, const float* old = nullptr) {
     const rh_conv_geom g = geom(batch);
+    if (!old) old = out;
     unwrap(rh_conv2d_fwd(&g, 1.0f, in, weights->as_ptr(), 0.0f, pre_act->as_mut_ptr(), nullptr, ws.as_mut_ptr(), ws.len(),
                          (bf16 ? RH_MATH_BF16_MFMA_FP32ACC : 0) | conv_algo, s()), "conv2d forward");
     const int flags = relu ? RH_FUSE_RELU : 0;
     if (phase.training) {
       if (!backward) panic("batch norm training missing backward operator");
-      unwrap(rh_bnorm_fwd_train(g.N, g.K, plane(), 1.0f, pre_act->as_ptr(), beta_out, out, avg.at_iter(phase.t), epsilon,
-                                scale->as_ptr(), bias->as_ptr(), running_mean->as_mut_ptr(), running_ivar->as_mut_ptr(),
+      unwrap(rh_bnorm_fwd_train_add(g.N, g.K, plane(), 1.0f, pre_act->as_ptr(), beta_out, old, out, avg.at_iter(phase.t), epsilon,
+                                    scale->as_ptr(), bias->as_ptr(), running_mean->as_mut_ptr(), running_ivar->as_mut_ptr(),
                                 cached_mean->as_mut_ptr(), cached_ivar->as_mut_ptr(), ws.as_mut_ptr(), ws.len(), flags, s()),
              "batch norm forward training");
     } else {
-      unwrap(rh_bnorm_fwd_infer(g.N, g.K, plane(), 1.0f, pre_act->as_ptr(), beta_out, out, epsilon, scale->as_ptr(),
+      unwrap(rh_bnorm_fwd_infer_add(g.N, g.K, plane(), 1.0f, pre_act->as_ptr(), beta_out, old, out, epsilon, scale->as_ptr(),
                                 bias->as_ptr(), running_mean->as_ptr(), running_ivar->as_ptr(), ws.as_mut_ptr(), ws.len(),
                                 flags, s()), "batch norm forward inference");
     }
@@ -1686,9 +1687,9 @@ class StackResConv2dOperator : public BNormUnitsOperator {
     units_[0].forward(batch_size, in_act_->as_ptr(), mid_act_->as_mut_ptr(), 0.0f, phase, config_.bnorm_mov_avg,
                       config_.bnorm_epsilon, fuse, *workspace_, opts_.bf16_forward);
     rect_after(config_.act_func, *mid_act_, len, batch_size);
-    unwrap(rh_copy_d2d(out_act_->as_mut_ptr(), in_act_->as_ptr(), len * batch_size * 4, context_->stream()), "send");
+    // (out <- in rides in the second unit's batch norm)
     units_[1].forward(batch_size, mid_act_->as_ptr(), out_act_->as_mut_ptr(), 1.0f, phase, config_.bnorm_mov_avg,
-                      config_.bnorm_epsilon, fuse, *workspace_, opts_.bf16_forward);
+                      config_.bnorm_epsilon, fuse, *workspace_, opts_.bf16_forward, in_act_->as_ptr());
     rect_after(config_.act_func, *out_act_, len, batch_size);
   }
   void backward(size_t batch_size) override {
@@ -1696,7 +1697,13 @@ class StackResConv2dOperator : public BNormUnitsOperator {
     RB_ASSERT((bool)mid_delta_);
     const size_t len = config_.in_dims.len();
     rh_stream_t s = context_->stream();
-    apply_rect_backprop(config_.act_func, out_act_->as_ptr(), len, batch_size, out_delta_->as_mut_ptr(), s);
+    // (in_delta <- out_delta rides in the mask's pass)
+    const bool fold_copy = in_delta_ && opts_.fuse_epilogue && config_.act_func == ActivationFunction::Rect;
+    if (fold_copy)
+      unwrap(rh_rect_backprop_copy(out_act_->as_ptr(), out_delta_->as_mut_ptr(), in_delta_->as_mut_ptr(), len * batch_size, s),
+             "rect backprop");
+    else
+      apply_rect_backprop(config_.act_func, out_act_->as_ptr(), len, batch_size, out_delta_->as_mut_ptr(), s);
     units_[1].backward_params(batch_size, mid_act_->as_ptr(), out_delta_->as_ptr(), config_.bnorm_epsilon, *workspace_, aux_ws());
     units_[1].backward_data(batch_size, mid_delta_->as_mut_ptr(), 0.0f, *workspace_);
     // with fused epilogues the ReLU mask of mid is applied inside unit 0's batch-norm backward (mid_delta keeps the
@@ -1706,7 +1713,7 @@ class StackResConv2dOperator : public BNormUnitsOperator {
     units_[0].backward_params(batch_size, in_act_->as_ptr(), mid_delta_->as_ptr(), config_.bnorm_epsilon, *workspace_, aux_ws(),
                               fold_mid);
     if (in_delta_) {
-      unwrap(rh_copy_d2d(in_delta_->as_mut_ptr(), out_delta_->as_ptr(), len * batch_size * 4, s), "send");
+      if (!fold_copy) unwrap(rh_copy_d2d(in_delta_->as_mut_ptr(), out_delta_->as_ptr(), len * batch_size * 4, s), "send");
       units_[0].backward_data(batch_size, in_delta_->as_mut_ptr(), 1.0f, *workspace_);
     }
   }

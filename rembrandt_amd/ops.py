@@ -145,6 +145,12 @@ def rect_inplace(y):
     return y
 
 
+def rect_backprop_copy(y, dy, copy):
+    """rect_backprop_inplace whose result goes to `copy` too."""
+    check(lib().rh_rect_backprop_copy(_p(y), _p(dy), _p(copy), y.numel(), _stream()), "rh_rect_backprop_copy")
+    return dy
+
+
 def rect_backprop_inplace(y, dy):
     lib().rembrandt_kernel_batch_map_rect_backprop_inplace(_p(y), y.numel() // y.shape[0], y.shape[0], _p(dy),
                                                            _stream())
@@ -505,29 +511,36 @@ def _bnorm_ws(x):
     return torch.empty(nbytes, dtype=torch.uint8, device=x.device), nbytes
 
 
-def bnorm_fwd_train(x, scale, bias, running_mean, running_ivar, ema_factor, epsilon, alpha=1.0, beta=0.0, y=None, relu=False):
-    """Spatial batch-norm, training mode: returns (y, cached_mean, cached_ivar); the running pair is updated in place."""
+def bnorm_fwd_train(x, scale, bias, running_mean, running_ivar, ema_factor, epsilon, alpha=1.0, beta=0.0, y=None, relu=False, y0=None):
+    """Spatial batch-norm, training mode: returns (y, cached_mean, cached_ivar); the running pair is updated in place.
+    `y0`: the tensor that beta weighs, where it is not y itself."""
     N, Cc, H, W = x.shape
     if y is None:
-        assert beta == 0.0
+        assert beta == 0.0 or y0 is not None
         y = torch.empty_like(x)
     cm, ci = torch.empty_like(scale), torch.empty_like(scale)
     ws, nbytes = _bnorm_ws(x)
-    check(lib().rh_bnorm_fwd_train(N, Cc, H * W, alpha, _p(x), beta, _p(y), ema_factor, epsilon, _p(scale), _p(bias),
-                                   _p(running_mean), _p(running_ivar), _p(cm), _p(ci), _p(ws), nbytes,
-                                   _lib.RH_FUSE_RELU if relu else 0, _stream()), "rh_bnorm_fwd_train")
+    args = (ema_factor, epsilon, _p(scale), _p(bias), _p(running_mean), _p(running_ivar), _p(cm), _p(ci), _p(ws), nbytes,
+            _lib.RH_FUSE_RELU if relu else 0, _stream())
+    if y0 is not None:
+        check(lib().rh_bnorm_fwd_train_add(N, Cc, H * W, alpha, _p(x), beta, _p(y0), _p(y), *args), "rh_bnorm_fwd_train_add")
+    else:
+        check(lib().rh_bnorm_fwd_train(N, Cc, H * W, alpha, _p(x), beta, _p(y), *args), "rh_bnorm_fwd_train")
     return y, cm, ci
 
 
-def bnorm_fwd_infer(x, scale, bias, running_mean, running_ivar, epsilon, alpha=1.0, beta=0.0, y=None, relu=False):
+def bnorm_fwd_infer(x, scale, bias, running_mean, running_ivar, epsilon, alpha=1.0, beta=0.0, y=None, relu=False, y0=None):
     N, Cc, H, W = x.shape
     if y is None:
-        assert beta == 0.0
+        assert beta == 0.0 or y0 is not None
         y = torch.empty_like(x)
     ws, nbytes = _bnorm_ws(x)
-    check(lib().rh_bnorm_fwd_infer(N, Cc, H * W, alpha, _p(x), beta, _p(y), epsilon, _p(scale), _p(bias), _p(running_mean),
-                                   _p(running_ivar), _p(ws), nbytes, _lib.RH_FUSE_RELU if relu else 0, _stream()),
-          "rh_bnorm_fwd_infer")
+    args = (epsilon, _p(scale), _p(bias), _p(running_mean), _p(running_ivar), _p(ws), nbytes, _lib.RH_FUSE_RELU if relu else 0,
+            _stream())
+    if y0 is not None:
+        check(lib().rh_bnorm_fwd_infer_add(N, Cc, H * W, alpha, _p(x), beta, _p(y0), _p(y), *args), "rh_bnorm_fwd_infer_add")
+    else:
+        check(lib().rh_bnorm_fwd_infer(N, Cc, H * W, alpha, _p(x), beta, _p(y), *args), "rh_bnorm_fwd_infer")
     return y
 
 

@@ -1135,6 +1135,34 @@ def test_bnorm_at_the_bounds_of_its_forms(dev, shape):
     assert np.array_equal(N(dy), dx)
 
 
+@pytest.mark.parametrize("shape", [(3, 2, 4, 5), (2, 3, 3, 3), (4, 2, 32, 65), (3, 2, 83, 83), (5, 2, 64, 66), (1, 1, 1, 1)])
+def test_residual_sum_and_its_gradient(dev, shape):
+    """The batch norm that adds another tensor gives what the blend with a copy of it gives (one launch, three, single values
+    and 16-byte units, a tensor at a 4-byte offset), and the ReLU backward with a second result what the pass and a copy do."""
+    C = shape[1]
+    x, r, dy = synth.normal(19, 1, shape), synth.normal(19, 2, shape), synth.normal(19, 3, shape)
+    scale, bias = T(synth.normal(19, 4, (C,)), dev), T(synth.normal(19, 5, (C,)), dev)
+    off = torch.empty(r.size + 1, device=dev)[1:].view(shape)
+    off.copy_(T(r, dev))
+    for relu in (False, True):
+        for y0, same_units in ((T(r, dev), True), (off, shape[2] * shape[3] % 4 != 0)):
+            stats = [torch.full((C,), 0.5, device=dev) for _ in range(4)]
+            want = ops.bnorm_fwd_train(T(x, dev), scale, bias, stats[0], stats[1], 0.1, 1e-5, alpha=0.5, beta=1.5, y=T(r, dev), relu=relu)
+            got = ops.bnorm_fwd_train(T(x, dev), scale, bias, stats[2], stats[3], 0.1, 1e-5, alpha=0.5, beta=1.5, y0=y0, relu=relu)
+            for a, b in zip(got + (stats[2], stats[3]), want + (stats[0], stats[1])):
+                # (another unit, another order of the sums)
+                assert torch.equal(a, b) if same_units else torch.allclose(a, b, rtol=1e-5, atol=1e-5)
+            assert np.array_equal(N(y0), r), "the added tensor is read only"
+            want = ops.bnorm_fwd_infer(T(x, dev), scale, bias, stats[0], stats[1], 1e-5, beta=1.0, y=T(r, dev), relu=relu)
+            got = ops.bnorm_fwd_infer(T(x, dev), scale, bias, stats[0], stats[1], 1e-5, beta=1.0, y0=y0, relu=relu)
+            assert torch.equal(got, want)
+    for y in (T(r, dev), off):
+        one, two, copy = T(dy, dev), T(dy, dev), torch.full(shape, 7.0, device=dev)
+        ops.rect_backprop_copy(y, one, copy)
+        ops.rect_backprop_inplace(y, two)
+        assert torch.equal(one, two) and torch.equal(copy, two)
+
+
 @pytest.mark.parametrize("case", [(2, 3, 9, 3, 2, 0), (2, 3, 9, 3, 2, 1), (3, 4, 8, 2, 2, 0), (2, 5, 27, 3, 2, 0), (2, 2, 13, 3, 3, 1)])
 @pytest.mark.parametrize("rounding", [_lib.RH_ROUND_FLOOR, _lib.RH_ROUND_CEIL])
 def test_pool2d_bwd_with_folded_relu_mask(dev, case, rounding):
