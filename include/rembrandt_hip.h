@@ -434,7 +434,7 @@ int rh_bnorm_fwd_infer(int N, int C, int plane, float alpha, const float* x, flo
                        const float* scale, const float* bias, const float* running_mean, const float* running_ivar,
                        void* ws, size_t ws_bytes, int flags, rh_stream_t stream);
 /* The same with the blend's second term from another tensor: y = alpha*(...) + beta*y0, y0 whole and apart from y, or y
- * itself (a residual unit's input, which the reference copies to y first, src/operator/conv.rs:1627-1665). */
+ * itself (a residual unit's input, which the reference copies to y first, src/operator/conv.rs:1497-1672). */
 int rh_bnorm_fwd_train_add(int N, int C, int plane, float alpha, const float* x, float beta, const float* y0, float* y,
                            double ema_factor, double epsilon, const float* scale, const float* bias, float* running_mean,
                            float* running_ivar, float* cached_mean, float* cached_ivar, void* ws, size_t ws_bytes, int flags,

@@ -123,6 +123,7 @@ extern "C" {
   pub fn rembrandt_kernel_batch_map_rect_inplace(y: *mut f32, frame_len: i32, batch: i32, stream: rh_stream_t);
   pub fn rembrandt_kernel_batch_map_rect_backprop_inplace(y: *const f32, frame_len: i32, batch: i32,
                                                           dy: *mut f32, stream: rh_stream_t);
+  pub fn rh_rect_backprop_copy(y: *const f32, dy: *mut f32, copy: *mut f32, n: size_t, stream: rh_stream_t) -> c_int;
 
   pub fn rh_sgemm_workspace_bytes(m: i32, n: i32, k: i32) -> size_t;
   pub fn rh_sgemm(trans_a: c_int, trans_b: c_int, m: i32, n: i32, k: i32, alpha: c_float, a: *const f32,
@@ -232,6 +233,15 @@ extern "C" {
                             y: *mut f32, epsilon: f64, scale: *const f32, bias: *const f32,
                             running_mean: *const f32, running_ivar: *const f32, ws: *mut c_void, ws_bytes: size_t,
                             flags: c_int, stream: rh_stream_t) -> c_int;
+  pub fn rh_bnorm_fwd_train_add(n: c_int, c: c_int, plane: c_int, alpha: c_float, x: *const f32, beta: c_float,
+                                y0: *const f32, y: *mut f32, ema_factor: f64, epsilon: f64, scale: *const f32,
+                                bias: *const f32, running_mean: *mut f32, running_ivar: *mut f32,
+                                cached_mean: *mut f32, cached_ivar: *mut f32, ws: *mut c_void, ws_bytes: size_t,
+                                flags: c_int, stream: rh_stream_t) -> c_int;
+  pub fn rh_bnorm_fwd_infer_add(n: c_int, c: c_int, plane: c_int, alpha: c_float, x: *const f32, beta: c_float,
+                                y0: *const f32, y: *mut f32, epsilon: f64, scale: *const f32, bias: *const f32,
+                                running_mean: *const f32, running_ivar: *const f32, ws: *mut c_void,
+                                ws_bytes: size_t, flags: c_int, stream: rh_stream_t) -> c_int;
   pub fn rh_bnorm_bwd(n: c_int, c: c_int, plane: c_int, alpha_data: c_float, beta_data: c_float, x: *const f32,
                       dy: *const f32, dx: *mut f32, alpha_param: c_float, beta_param: c_float, epsilon: f64,
                       scale: *const f32, dscale: *mut f32, dbias: *mut f32, cached_mean: *const f32,
