@@ -18,14 +18,21 @@
 // per two MFMAs: lanes 0-31 take channels 0, 1 of the quad and lanes 32-63 channels 2, 3 of the same position (or row), so
 // the first MFMA contracts channels {0, 2}, the second {1, 3}.  A tap is a displacement r Wp + s of the position: R
 // address registers and constant offsets, no arithmetic between the MFMAs.  Two stages of LDS, one barrier a stage, the next
-// stage in registers while this one is multiplied; two to four blocks a CU.
+// stage in registers while this one is multiplied; two to five blocks a CU.
+//
+// The sums are formed in two levels: chains of 36 (3x3) or 52 and 48 (5x5) terms in the matrix pipes' accumulators, added
+// to a second set of registers.  One chain over a slice's whole contraction loses up to 3.2 times the bits (relative
+// rms error against 64 bits, 20 -> 50 5x5 forward, 3.8e-7 in one chain of 500 terms, 1.4e-7 in ten; 128 -> 128 3x3, 9
+// images, 4.2e-7 and 1.3e-7) and the engine's slices, chains of 60 to 600 terms, 1.4e-7 to 4e-7.  The second set costs
+// a block of four its place on a CU on the widest tile and 0 to 3 % of the time (24 images of 512 -> 512 7x7, whose one
+// slice is the longest: 67.7 -> 72.4 us).
 //
 // Measured, one call (with whatever it launches) against the same call on the engine, fp32, stride 1:
-//   20 -> 50, 5x5, 14x14, batch 64: 15.3 us (29.8);  32 -> 32, 5x5, 16x16, batch 128: 21.1 (35.1);
-//   64 -> 64, 3x3, 56x56, batch 8: 29.6 (60.5), batch 32: 81 (94), batch 128: 256 (273);
-//   384 -> 384, 3x3, 13x13, batch 1: 18.3 (30.5), batch 4: 33.6 (41.8); 96 -> 256, 5x5, 27x27, batch 16: 123 (155).
-// Where the time goes on 64 channels, 56x56, batch 32 (47 us at the matrix peak, 54 with 6.1 blocks of work a CU as 7):
-// MFMAs, barriers, prologues and the epilogue 74, LDS traffic 4, loads 6.
+//   20 -> 50, 5x5, 14x14, batch 64: 14.2 us (28.4);  32 -> 32, 5x5, 16x16, batch 128: 21.4 (34.2);
+//   64 -> 64, 3x3, 56x56, batch 8: 29.4 us (60.9), batch 32: 93 (93), batch 128: 272 (270);
+//   384 -> 384, 3x3, 13x13, batch 1: 19.4 (29.5), batch 4: 33.8 (40.4); 96 -> 256, 5x5, 27x27, batch 16: 124 (153).
+// What bounds it once it fills the GPU: the MFMAs (47 us of the 93 on 64 channels, 56x56, batch 32, at the matrix peak), what
+// barriers, prologues and epilogues leave idle between them, and a last round of blocks.
 #include <string.h>
 
 #include <algorithm>
@@ -55,10 +62,15 @@ constexpr int kLdsMaxPos = 512;   // staged positions per channel and tile: two 
 // taps of seven rows of a 3x3 filter, of two or three rows of a 5x5 one).
 template <int R> constexpr int lds_tap_stride(int bm) { return bm * 4 + (R == 3 ? 14 : 6); }
 
+// Taps of a quad whose products are added in one chain (36 terms; 52 and 48).
+template <int R> constexpr int lds_chain_taps() { return R == 3 ? 9 : 13; }
+
 // R: filter extent.  T: tile (BM x BN over WM x WN waves).  WK: waves that share a tile and split the quads of a stage
 // among them (their sums meet in LDS at the end).  QC: quads per stage.
+// (Bounds of two blocks: with one the accumulators of the matrix pipes and the sums lie in different halves of the
+// register file, and every fold moves them across: 3 to 6 % slower on every shape.)
 template <int R, class T, int WK, int QC>
-__global__ __launch_bounds__(256) void conv_lds_kernel(LdsConvParams p, EpiParams ep) {
+__global__ __launch_bounds__(256, 2) void conv_lds_kernel(LdsConvParams p, EpiParams ep) {
   constexpr int RS = R * R, BM = T::BM, BN = T::BN, TM = T::TM, TN = T::TN;
   static_assert(T::NT * WK == 256 && QC % WK == 0, "four waves");
   constexpr int WSTR = lds_tap_stride<R>(BM);   // floats from a tap's filter slab to the next
@@ -154,13 +166,13 @@ __global__ __launch_bounds__(256) void conv_lds_kernel(LdsConvParams p, EpiParam
   }
   const int wb = (wm * (TM * 32) + l32) * 2 + half * (BM * 2);
 
-  f32x16 acc[TM][TN];
+  f32x16 sum[TM][TN], acc[TM][TN];
 #pragma unroll
   for (int i = 0; i < TM; ++i)
 #pragma unroll
     for (int j = 0; j < TN; ++j)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][j][v] = 0.0f;
+      for (int v = 0; v < 16; ++v) sum[i][j][v] = acc[i][j][v] = 0.0f;
 
   // Operands of tap u of this wave's share of a stage (QC / WK quads of RS taps): read DIST taps ahead of their MFMAs.
   constexpr int NU = QC / WK * RS, DIST = TM * TN == 1 ? 2 : 1;
@@ -174,14 +186,29 @@ __global__ __launch_bounds__(256) void conv_lds_kernel(LdsConvParams p, EpiParam
 #pragma unroll
     for (int j = 0; j < TN; ++j) b[slot][j] = *reinterpret_cast<const f32x2_t*>(xq + xb[j][r] + s * 2);
   };
-  auto mul = [&](int slot) {
+  auto fold = [&] {
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int j = 0; j < TN; ++j)
+#pragma unroll
+        for (int v = 0; v < 16; ++v) sum[i][j][v] += acc[i][j][v];
+  };
+  auto mul = [&](int u) {
+    const int slot = u % (DIST + 1);
+    const bool first = u % RS % lds_chain_taps<R>() == 0;   // of a chain: the one before it goes to the sums
+    if (first) {
+      fold();
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    const f32x16 zero = {};
 #pragma unroll
     for (int e = 0; e < 2; ++e)
 #pragma unroll
       for (int i = 0; i < TM; ++i)
 #pragma unroll
         for (int j = 0; j < TN; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[slot][i][e], b[slot][j][e], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x2f32(a[slot][i][e], b[slot][j][e], first && e == 0 ? zero : acc[i][j], 0, 0, 0);
   };
 
   const int q0 = (int)blockIdx.y * p.qps, q1 = min(q0 + p.qps, p.nq);
@@ -200,7 +227,7 @@ __global__ __launch_bounds__(256) void conv_lds_kernel(LdsConvParams p, EpiParam
     for (int u = 0; u < NU - DIST; ++u) {
       read(u + DIST, (u + DIST) % (DIST + 1), buf);
       __builtin_amdgcn_sched_barrier(0);
-      mul(u % (DIST + 1));
+      mul(u);
       __builtin_amdgcn_sched_barrier(0);
     }
     if (!more) break;
@@ -222,7 +249,7 @@ __global__ __launch_bounds__(256) void conv_lds_kernel(LdsConvParams p, EpiParam
     }
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
-    for (int u = NU - DIST; u < NU; ++u) mul(u % (DIST + 1));
+    for (int u = NU - DIST; u < NU; ++u) mul(u);
     __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
     for (int u = 0; u < DIST; ++u) {
@@ -233,7 +260,8 @@ __global__ __launch_bounds__(256) void conv_lds_kernel(LdsConvParams p, EpiParam
     }
   }
 #pragma unroll
-  for (int u = NU - DIST; u < NU; ++u) mul(u % (DIST + 1));
+  for (int u = NU - DIST; u < NU; ++u) mul(u);
+  fold();
   if constexpr (WK > 1) {
     // the WK waves of a tile add their sums in LDS, in the order of their quads
     static_assert(TM == 1 && TN == 1, "one block a wave");
@@ -241,15 +269,15 @@ __global__ __launch_bounds__(256) void conv_lds_kernel(LdsConvParams p, EpiParam
     float* const red = smem;   // [tile waves][WK - 1][16][64]
     if (wk > 0)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) red[((wmn * (WK - 1) + wk - 1) * 16 + v) * 64 + lane] = acc[0][0][v];
+      for (int v = 0; v < 16; ++v) red[((wmn * (WK - 1) + wk - 1) * 16 + v) * 64 + lane] = sum[0][0][v];
     __syncthreads();
     if (wk > 0) return;
 #pragma unroll
     for (int k = 1; k < WK; ++k)
 #pragma unroll
-      for (int v = 0; v < 16; ++v) acc[0][0][v] += red[((wmn * (WK - 1) + k - 1) * 16 + v) * 64 + lane];
+      for (int v = 0; v < 16; ++v) sum[0][0][v] += red[((wmn * (WK - 1) + k - 1) * 16 + v) * 64 + lane];
   }
-  store_tile<T, true>(acc, ep, m0, n0, wm, wn, lane, ep.split_stride != 0 ? (int)blockIdx.y : -1);
+  store_tile<T, true>(sum, ep, m0, n0, wm, wn, lane, ep.split_stride != 0 ? (int)blockIdx.y : -1);
 }
 
 typedef Tile<64, 128, 2, 1, 4> L64x128;
@@ -258,9 +286,10 @@ typedef Tile<32, 128, 2, 1, 4> L32x128;
 typedef Tile<32, 64, 2, 1, 2> L32x64;    // two waves a column block
 typedef Tile<32, 32, 2, 1, 1> L32x32;    // four
 
-// mfmas: MFMAs of a wave per tap and stage
-struct LdsShape { int bm, bn, qc, mfmas; };
-static const LdsShape kLdsShapes[kLdsShapeCount] = {{64, 128, 1, 4}, {64, 64, 1, 2}, {32, 128, 1, 2}, {32, 64, 2, 2}, {32, 32, 4, 2}, {32, 128, 2, 4}};
+// mfmas: MFMAs of a wave per tap and stage.  held3, held5: blocks whose registers fit a CU, 3x3 and 5x5 filters.
+struct LdsShape { int bm, bn, qc, mfmas, held3, held5; };
+static const LdsShape kLdsShapes[kLdsShapeCount] = {{64, 128, 1, 4, 3, 2}, {64, 64, 1, 2, 4, 3}, {32, 128, 1, 2, 5, 4},
+                                                    {32, 64, 2, 2, 4, 3}, {32, 32, 4, 2, 3, 2}, {32, 128, 2, 4, 3, 2}};
 
 // Staged positions per channel that any tile of `bn` consecutive output pixels can need.
 static int lds_positions(int P, int Q, int R, int bn) {
@@ -279,7 +308,8 @@ static size_t lds_conv_bytes(int R, int shape, int npos) {
 // taking its stages' MFMAs (times `mfma`, what barriers and the other blocks cost) or, with few blocks, its stages' MFMAs
 // one by one with `wait` in between; 1.2 us a round for prologue and epilogue; slices write and read their partial sums at
 // 4 TB/s in a launch of their own.  The constants are a fit to some 4000 timings (14 layers, both passes, batches 1 to 128,
-// all shapes and slice counts; rms error 8 %, the shape it picks is 3 % from the best on average).
+// all shapes and slice counts).  Against 25000 timings of 792 layers (400 of them of random sizes) the shape and slices it
+// picks take 2.4 % longer than the best on average, 10 % at the 95th percentile, and its estimate of them is 11 % off (rms).
 struct LdsCost { double wait, mfma; };
 static const LdsCost kLdsCost3[kLdsShapeCount] = {{0.70, 1.15}, {0.65, 1.47}, {0.55, 1.36}, {0.92, 1.89}, {0.26, 3.78}, {0.97, 1.40}};
 static const LdsCost kLdsCost5[kLdsShapeCount] = {{1.14, 1.15}, {0.87, 1.32}, {0.54, 1.15}, {0.35, 1.60}, {0.23, 2.43}, {0.87, 1.12}};
@@ -302,7 +332,7 @@ static LdsConvPlan make_lds_plan(int N, int Ci, int rows, int P, int Q, int R) {
     const long long tiles = (long long)cdiv(rows, s.bm) * cdiv<long long>(cols, s.bn);
     const LdsCost& c = (R == 3 ? kLdsCost3 : kLdsCost5)[shape];
     const double mfma_us = s.mfmas * R * R * 64.0 / 2300.0;   // one stage of a wave at the clock it gets
-    const int held = min((int)(160 * 1024 / lds), shape == 0 || shape == 4 ? 4 : 6);
+    const int held = min((int)(160 * 1024 / lds), R == 3 ? s.held3 : s.held5);
     for (int want : kSlices) {
       if (want > stages) break;
       const int per = cdiv(stages, want), slices = cdiv(stages, per);

@@ -191,6 +191,29 @@ def test_conv2d_staged_operands(dev, case):
     assert torch.equal(one, two), "masked data gradient"
 
 
+@pytest.mark.parametrize("case", [(64, 20, 14, 14, 50, 5, 2), (37, 32, 16, 16, 32, 5, 2), (5, 96, 27, 27, 256, 5, 2),
+                                  (9, 128, 28, 28, 128, 3, 1), (9, 256, 14, 14, 256, 3, 1)], ids=str)
+def test_conv2d_staged_operands_error(dev, case):
+    """Error of the staged form against 64-bit sums.  A chain of n rounded additions of independent terms has a relative
+    rms error of sqrt(0.09 n) 2^-24 (a rounding's variance is u^2 / 3 of the power of two below the partial sum, 0.54 of its
+    square on average, and the partial sums grow as a random walk: n / 2 of the last one's); chains of F terms added up
+    in a chain of n / F have that of a chain of F + n / F, and the products' and the result's own roundings stand for
+    four more.  A quarter on top for the spread between tensors; a chain over the whole contraction is 2 to 4 times as far off."""
+    Nn, C, H, W, K, R, pad = case
+    say("staged error case", case)
+    x, w = synth.normal(19, 1, (Nn, C, H, W)), synth.normal(19, 2, (K, C, R, R))
+    dy = synth.normal(19, 3, (Nn, K, H, W))
+    xd, wd, dyd = T(x, dev), T(w, dev), T(dy, dev)
+    D = _lib.RH_ALGO_DIRECT
+    (y, dx), tags = profile_tags(lambda: (ops.conv2d_fwd(xd, wd, 1, pad, algo=D), ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=D)))
+    assert any(t.startswith("conv_fwd_lds") for t in tags) and any(t.startswith("conv_bwd_data_lds") for t in tags), tags
+    for got, ref, chans in ((y, O.conv2d_fwd(x, w, 1, pad), C), (dx, O.conv2d_bwd_data(w, dy, x.shape, 1, pad), K)):
+        terms, chain = chans * R * R, 36 if R == 3 else 52
+        bound = 1.25 * 2.0 ** -24 * (0.09 * (chain + terms / chain + 4)) ** 0.5
+        err = np.linalg.norm(N(got).astype(np.float64) - ref) / np.linalg.norm(ref.astype(np.float64))
+        assert err <= bound, (terms, err, bound)
+
+
 # 3x3 stride-1 layers in the Winograd F(2x2, 3x3) form: odd and even extents (tiles that hang over the edge), every
 # padding it takes, channel counts that do not fill a group of four, filter counts around the 128-row tile, tile counts
 # that are no multiple of the 32-tile block, more blocks than CUs, and the sizes the library takes the form for by itself
