@@ -280,6 +280,18 @@ void launch_split_reduce_nchw(const float* part, int splits, long long stride, f
                               long long col0 = 0, const float* mask = nullptr);
 
 
+// Slices that the direct form cuts the contraction of a forward / stride-1 backward-data call into.
+inline int soff_splits_fwd(const ConvDims& d, int n_k) {
+  const long long cols = (long long)d.N * d.P * d.Q;
+  const int s = plan_k_split(d.K, cols, n_k);
+  return pick_bm(d.K) == 128 && s > 1 ? plan_k_split(d.K, cols, n_k, 64) : s;
+}
+inline int soff_splits_bwd_data(const ConvDims& d, int n_k) {
+  const long long cols = (long long)d.N * d.H * d.W;
+  const int s = plan_k_split(d.C, cols, n_k);
+  return pick_bm(d.C) == 128 && s > 1 && plan_k_split(d.C, cols, n_k, 64) == 1 ? 1 : s;
+}
+
 inline SoffPlan plan_soff_fwd(const ConvDims& d) {
   SoffPlan p;
   p.n_k = round_up(d.C * d.R * d.S, kTabPad);
@@ -291,14 +303,13 @@ inline SoffPlan plan_soff_fwd(const ConvDims& d) {
   const size_t img = sizeof(float) * (size_t)d.N * d.C * p.Hp * p.Wp;
   p.img_bytes = d.pad > 0 ? align256(img) : 0;
   p.ok = img <= kMaxBufferBytes && d.P > 0 && d.Q > 0;
-  p.splits = plan_k_split(d.K, (long long)d.N * d.P * d.Q, p.n_k);
+  p.splits = soff_splits_fwd(d, p.n_k);
   p.tail = plan_tail_split(d.K, (long long)d.N * d.P * d.Q, p.n_k);
-  if (pick_bm(d.K) == 128 && p.splits > 1) {
+  if (pick_bm(d.K) == 128 && plan_k_split(d.K, (long long)d.N * d.P * d.Q, p.n_k) > 1) {
     // Few 128 x 128 tiles (small images late in a network): the half-width tile, planned as such.  Twice the tiles often
     // need no slices any more, only a cut of the tiles past the last multiple of 256 (NIN's 1024-channel layers on
     // 6 x 6: 576 tiles = 512 + 64 in eight slices, instead of 288 x 3 with a reduction over the whole result).
     p.narrow128 = true;
-    p.splits = plan_k_split(d.K, (long long)d.N * d.P * d.Q, p.n_k, 64);
     p.tail = plan_tail_split(d.K, (long long)d.N * d.P * d.Q, p.n_k, 64);
   }
   const size_t tail_elems_f = (size_t)(d.y_elems - tail_first_elem(p.tail, (long long)d.P * d.Q, d.K));
@@ -320,11 +331,13 @@ struct WinoGeom {
   long long tiles, tiles_p;   // 2x2 output tiles; rounded up to whole column tiles
   size_t u_bytes, v_bytes;
   bool ok;
+  bool fine;                  // no call of it loses more bits than the direct form's slices would (see wino_stages_at_most)
   double us;                  // what a call is expected to take
   // Tail form (V made in the kernel only): the blocks past the last multiple of 256 (all of them where there are fewer) are cut into tail_S slices of the
   // channel loop, tail_L stages each, whose untransformed-blend partial results go to slabs of scratch that hold the
   // result from element part_first on (the first image a tail block touches); tail_S == 1: not worth it.
   int full_tiles, tail_S, tail_L;
+  int chains;                 // into which the stages of a slice are divided, see wino_gemm_fused_kernel
   long long part_first, slab_elems;
   size_t part_bytes;
   // 5x5 forward (wino_geom_fwd5): the filter, extended with zeros to 6x6, is four 3x3 filters at offsets (3 bi, 3 bj);
@@ -342,12 +355,27 @@ struct WinoGeom {
 inline int wino_bm(int Ci, int Ko, int blk5) {
   return Ci % 4 == 0 && !blk5 && round_up(Ko, kWinoBM2) * 9 <= round_up(Ko, kWinoBM) * 8 ? kWinoBM2 : kWinoBM;
 }
-WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int blk5 = 0);
+// Stages in a chain of which the form's error against 64 bits is the direct form's at `splits` slices.  Its relative rms
+// error, squared, is 1.35 + 0.351 L in units of 1e-14 (L stages of four channels in a chain: 2.6e-7 at 16, 3.5e-7 at 32,
+// 5.9e-7 at 96), the direct form's 0.030 a term (2.8e-7 at 256, 4.2e-7 at 576).  A direct form that is not sliced has the
+// longer chain at any size.
+inline int wino_stages_at_most(int Ci, int splits) {
+  return splits <= 1 ? cdiv(Ci, 4) : (int)((0.030 * 9.0 * Ci / splits - 1.35) / 0.351);
+}
+// max_L: the stages in a chain up to which a call counts as fine; it is made of such chains where that can be.
+WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int max_L, int blk5 = 0);
 inline bool wino_shape(const ConvDims& d) { return d.R == 3 && d.S == 3 && d.st == 1 && d.pad <= 2; }
 inline bool wino_shape5(const ConvDims& d) { return d.R == 5 && d.S == 5 && d.st == 1 && d.pad <= 4 && d.P > 0 && d.Q > 0; }
-inline WinoGeom wino_geom_fwd5(const ConvDims& d) { return wino_geom(d.N, d.C, d.H, d.W, d.K, d.pad, 1); }
-inline WinoGeom wino_geom_fwd(const ConvDims& d) { return wino_geom(d.N, d.C, d.H, d.W, d.K, d.pad); }
-inline WinoGeom wino_geom_bwd_data(const ConvDims& d) { return wino_geom(d.N, d.K, d.P, d.Q, d.C, 2 - d.pad); }
+// (5x5: 5.3e-7 unsliced on 96 channels, 5.0e-7 with a tail of six slices, the unsliced direct form 8.5e-7, three slices 4.9e-7)
+inline WinoGeom wino_geom_fwd5(const ConvDims& d) {
+  return wino_geom(d.N, d.C, d.H, d.W, d.K, d.pad, soff_splits_fwd(d, round_up(d.C * 25, kTabPad)) <= 1 ? 4 * d.C : 0, 1);
+}
+inline WinoGeom wino_geom_fwd(const ConvDims& d) {
+  return wino_geom(d.N, d.C, d.H, d.W, d.K, d.pad, wino_stages_at_most(d.C, soff_splits_fwd(d, round_up(d.C * 9, kTabPad))));
+}
+inline WinoGeom wino_geom_bwd_data(const ConvDims& d) {
+  return wino_geom(d.N, d.K, d.P, d.Q, d.C, 2 - d.pad, wino_stages_at_most(d.K, soff_splits_bwd_data(d, round_up(d.K * 9, kTabPad))));
+}
 // Filter gradient in the same form: zero-bordered copies of x and dy, S slices of the tiles, their partial sums.
 struct WinoFilterPlan {
   bool ok;
@@ -408,14 +436,14 @@ inline bool lds_pays(const ConvDims& d, const LdsConvPlan& p) { return p.ok && p
 // (Against the staged form by an eighth at least: its two or three launches count for more in a chain of layers than timed
 // back to back, ResNet-18 on 9 images 457 us with 1/8, 476 with the plain comparison.)
 inline bool wino_fastest(const ConvDims& d, const WinoGeom& g, const LdsConvPlan& lp) {
-  return g.Ci % 4 == 0 && g.us < conv_engine_us(d) && !(lp.ok && lp.us * 0.875 <= g.us);
+  return g.fine && g.Ci % 4 == 0 && g.us < conv_engine_us(d) && !(lp.ok && lp.us * 0.875 <= g.us);
 }
 inline bool wino_pays(const ConvDims& d, const WinoGeom& g, const LdsConvPlan& lp) {
   if (!g.ok || g.Ci < 64 || g.Ko < 64) return false;
   const long long blocks = (long long)(g.rows_p / g.bm) * (g.tiles_p / kWinoBN);
   // 64-row tiles, two to a CU: from a whole round of blocks on, or from three quarters of the CUs on where it is expected
   // to be the fastest (64 -> 64 56x56: batch 24, 588 blocks 53 us against 57 direct; 64 98 against 144)
-  if (g.bm == kWinoBM2) return 4 * g.Ko >= 3 * g.rows_p && (blocks >= 512 || (blocks >= 192 && wino_fastest(d, g, lp)));
+  if (g.bm == kWinoBM2) return 4 * g.Ko >= 3 * g.rows_p && ((blocks >= 512 && g.fine) || (blocks >= 192 && wino_fastest(d, g, lp)));
   // (rows: 128-row tiles at least three quarters full: 64 filters in one would execute as much as the direct form)
   if (4 * g.Ko >= 3 * g.rows_p && blocks >= 192) return true;
   return wino_fastest(d, g, lp);
@@ -492,13 +520,12 @@ inline SoffPlan plan_soff_bwd_data(const ConvDims& d) {
   const size_t img = p.halo >= 0 ? sizeof(float) * (size_t)d.N * d.K * p.Hp * p.Wp : 0;
   p.img_bytes = (p.halo > 0 || d.st > 1 || p.Hp != d.P || p.Wp != d.Q) ? align256(img) : 0;
   p.ok = p.halo >= 0 && d.R == d.S && img <= kMaxBufferBytes && d.P > 0 && d.Q > 0;
-  p.splits = plan_k_split(d.C, (long long)d.N * d.H * d.W, p.n_k);
+  p.splits = soff_splits_bwd_data(d, p.n_k);
   p.tail = plan_tail_split(d.C, (long long)d.N * d.H * d.W, p.n_k);
-  if (pick_bm(d.C) == 128 && p.splits > 1 && plan_k_split(d.C, (long long)d.N * d.H * d.W, p.n_k, 64) == 1) {
+  if (pick_bm(d.C) == 128 && p.splits == 1 && plan_k_split(d.C, (long long)d.N * d.H * d.W, p.n_k) > 1) {
     // As in the forward pass, where 128 x 64 tiles need no slices (NIN's 1024-channel 1x1 layers: 0.120 -> 0.098 ms).
     // Where they would still be sliced the 128 x 128 tile stays (a 384-channel 3x3 layer on 6 x 6 lost 9 %).
     p.narrow128 = true;
-    p.splits = 1;
     p.tail = plan_tail_split(d.C, (long long)d.N * d.H * d.W, p.n_k, 64);
   }
   if (d.st > 1) p.tail.splits = 1;  // the zero-dilated form is a fallback only

@@ -39,7 +39,7 @@
 
 namespace rh {
 
-WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int blk5) {
+WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int max_L, int blk5) {
   WinoGeom g;
   g.N = N; g.Ci = Ci; g.Hi = Hi; g.Wi = Wi; g.Ko = Ko; g.halo = halo;
   g.P = Hi + 2 * halo - 2; g.Q = Wi + 2 * halo - 2;
@@ -72,7 +72,7 @@ WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int blk5) {
   // at least), so that the last round is as short as its share of the work; their partial results are added by
   // wino_tail_reduce_kernel.  A block costs about eight stages' time before and after its loop (measured: 1176 blocks
   // of 64 stages gain nothing from five slices of 13), and the slabs and that kernel 3 % of a round.
-  g.full_tiles = 0; g.tail_S = 1; g.tail_L = g.Cg; g.part_first = 0; g.slab_elems = 0; g.part_bytes = 0;
+  g.full_tiles = 0; g.tail_S = 1; g.tail_L = g.Cg; g.chains = 1; g.part_first = 0; g.slab_elems = 0; g.part_bytes = 0;
   const long long tiles_m = g.rows_p / g.bm, T = tiles_m * (g.tiles_p / kWinoBN), slots = g.slots();
   const long long full = T / slots * slots, tail = T - full;
   const long long out_elems = (long long)N * Ko * g.P * g.Q;
@@ -88,7 +88,16 @@ WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int blk5) {
     return (double)(blocks / slots) + (rem == 0 ? 0.0 : two && rem <= 256 ? 0.57 : 1.0);
   };
   auto stages_us = [&](double n, int stages) { return n * (stages + outside) * stage_us; };
-  g.us = fixed_us + stages_us(rounds(T), g.Cg);
+  // (192 blocks of 128 rows three quarters full need no slices for the speed they are taken for: 256 -> 384 13x13 batch 64
+  // data gradient 114 us, the direct form 174 in six slices, with 5.9e-7 and 4.2e-7 of error.)
+  if (4 * Ko >= 3 * round_up(Ko, kWinoBM) && (long long)(round_up(Ko, kWinoBM) / kWinoBM) * (g.tiles_p / kWinoBN) >= 192) max_L = g.Cg;
+  // Stages in chains that are fine, with a fold between two of them that takes the time of 1.75.  (64-row blocks, two to a
+  // CU, have no registers for it.)
+  auto chains_of = [&](int L) { return two || blk5 || Ci % 4 != 0 || max_L < 4 || L <= max_L || L / cdiv(L, max_L) < 4 ? 1 : cdiv(L, max_L); };
+  auto folds_us = [&](int L) { return 1.75 * (chains_of(L) - 1) * stage_us; };
+  g.chains = chains_of(g.Cg);
+  g.fine = cdiv(g.Cg, g.chains) <= max_L;
+  g.us = fixed_us + (stages_us(1.0, g.Cg) + folds_us(g.Cg)) * rounds(T);
   if (g.ok && Ci % 4 == 0 && tail > 0) {
     double best = rounds(T) * 0.97, best_us = g.us;
     for (int S = 2; S <= 16; ++S) {
@@ -98,10 +107,10 @@ WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int blk5) {
         const double cost = (double)(full / slots) + rounds(tail * S) * (L + tail_outside) / (g.Cg + tail_outside) + 0.03;
         if (cost < best) { best = cost; g.tail_S = S; g.tail_L = L; }
       } else {
-        // Fewer blocks than CUs: all of them are cut, into as many slices as the whole call is shortest with (384 -> 384 on
-        // 13 x 13, batch 8: 39 blocks as 8 slices, 44 us; whole 116; the direct form 58).
-        const double us = fixed_us + stages_us(rounds(T * S), L) + 2.0 + 4.0 * (double)out_elems * (S + 1) / 2.84e6;
-        if (us < best_us) { best_us = us; g.tail_S = S; g.tail_L = L; }
+        // Fewer blocks than CUs: all of them are cut, into as many slices as the whole call is shortest with.
+        const bool fine = cdiv(L, chains_of(L)) <= max_L;
+        const double us = fixed_us + (stages_us(1.0, L) + folds_us(L)) * rounds(T * S) + 2.0 + 4.0 * (double)out_elems * (S + 1) / 2.84e6;
+        if (fine > g.fine || (fine == g.fine && us < best_us)) { best_us = us; g.fine = fine; g.tail_S = S; g.tail_L = L; g.chains = chains_of(L); }
       }
     }
     if (g.tail_S > 1) {
@@ -111,7 +120,8 @@ WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int blk5) {
       g.part_first = n0 * g.Ko * g.P * g.Q;
       g.slab_elems = out_elems - g.part_first;
       g.part_bytes = align256(sizeof(float) * (size_t)g.slab_elems * g.tail_S);
-      g.us = fixed_us + stages_us((double)(full / slots), g.Cg) + stages_us(rounds(tail * g.tail_S), g.tail_L) +
+      g.us = fixed_us + (stages_us(1.0, g.Cg) + folds_us(g.Cg)) * (double)(full / slots) +
+             (stages_us(1.0, g.tail_L) + 1.75 * (g.chains - 1) * stage_us) * rounds(tail * g.tail_S) +
              2.0 + 4.0 * (double)g.slab_elems * (g.tail_S + 1) / 2.84e6;
     }
   }
@@ -367,7 +377,26 @@ __device__ __forceinline__ void wino_store_block(const WinoOut<NA>& o, const Win
                                               o.srow + WinoOut<NA>::row_of(e0 + e4) * o.PQ4, 0);
 }
 
-__device__ __forceinline__ void wino_epilogue(f32x16 (&acc)[16], const WinoEpi& ep, int m0, unsigned n0, int wave, int lane) {
+// A^T M A of accumulator element e: the 2x2 pixels of its row.
+__device__ __forceinline__ void wino_pixels(f32x16 (&acc)[16], int e, float (&y)[2][2]) {
+  float s0[4], s1[4];
+#pragma unroll
+  for (int j = 0; j < 4; ++j) {
+    const float m0j = wino_acc_elem(acc[j], e), m1j = wino_acc_elem(acc[4 + j], e), m2j = wino_acc_elem(acc[8 + j], e),
+                m3j = wino_acc_elem(acc[12 + j], e);
+    s0[j] = m0j + m1j + m2j;
+    s1[j] = m1j - m2j - m3j;
+  }
+  y[0][0] = s0[0] + s0[1] + s0[2];
+  y[0][1] = s0[1] - s0[2] - s0[3];
+  y[1][0] = s1[0] + s1[1] + s1[2];
+  y[1][1] = s1[1] - s1[2] - s1[3];
+}
+
+// sum: pixels of the chains before the last one (SUM).
+template <bool SUM>
+__device__ __forceinline__ void wino_epilogue(f32x16 (&acc)[16], const f32x16 (&sum)[4], const WinoEpi& ep, int m0, unsigned n0, int wave,
+                                              int lane) {
   WinoOut<2> o;
   o.init(ep, m0 + wave * 32, n0, lane, 0);
   float bv[16];
@@ -381,19 +410,10 @@ __device__ __forceinline__ void wino_epilogue(f32x16 (&acc)[16], const WinoEpi& 
     float y[EB][2][2];
 #pragma unroll
     for (int e4 = 0; e4 < EB; ++e4) {
-      const int e = e0 + e4;
-      float s0[4], s1[4];
+      wino_pixels(acc, e0 + e4, y[e4]);
+      if (SUM)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const float m0j = wino_acc_elem(acc[j], e), m1j = wino_acc_elem(acc[4 + j], e), m2j = wino_acc_elem(acc[8 + j], e),
-                    m3j = wino_acc_elem(acc[12 + j], e);
-        s0[j] = m0j + m1j + m2j;
-        s1[j] = m1j - m2j - m3j;
-      }
-      y[e4][0][0] = s0[0] + s0[1] + s0[2];
-      y[e4][0][1] = s0[1] - s0[2] - s0[3];
-      y[e4][1][0] = s1[0] + s1[1] + s1[2];
-      y[e4][1][1] = s1[1] - s1[2] - s1[3];
+        for (int i = 0; i < 4; ++i) y[e4][i >> 1][i & 1] += sum[i][e0 + e4];
     }
     wino_store_block<EB, 2>(o, ep, e0, y, bv + e0);
   }
@@ -537,7 +557,8 @@ __global__ __launch_bounds__(256, 1) void wino_gemm_kernel(const float* __restri
   for (; it + 2 < nk; ++it) step(it, std::true_type());
   for (; it < nk; ++it) step(it, std::false_type());
 
-  wino_epilogue(acc, ep, m0, n0, wave, lane);
+  const f32x16 none[4] = {};
+  wino_epilogue<false>(acc, none, ep, m0, n0, wave, lane);
 }
 
 // ---- the same product with B^T d B made inside the kernel ------------------------------------------------------------
@@ -568,9 +589,17 @@ __device__ __forceinline__ void dma_load4(u32x4 rsrc, uint32_t lds_addr, uint32_
 
 struct WinoTail {
   int full, S, L;                     // blocks that take a whole tile; slices of a tail tile; stages per slice
+  int chains;                         // into which a block's stages are divided (FOLD)
   float* part; long long slab_elems, part_first;
 };
 
+// FOLD: a block's stages are divided into chains; the products of each go through the output transform and the pixels are
+// added up in registers (64 of them), for a chain's length of error instead of the whole loop's: on grids where the direct
+// form is cut into slices, and loses few bits by it.  A fold is some 950 vector instructions, the time of 1.75 stages, and
+// the sums leave 75 registers a lane free beside a block.  Data gradients, time and error without, with, and the direct
+// form's: 128 -> 128 28x28 batch 24 46.2 us 3.6e-7, 48.1 us 2.7e-7, 75.5 us 3.0e-7; 384 -> 384 13x13 batch 37 116 us
+// 5.9e-7, 119 us 3.5e-7, 170 us 4.2e-7; 512 -> 512 7x7 batch 50 89.8 us 4.9e-7, 90.4 us 3.2e-7, 123 us 3.3e-7.
+template <bool FOLD>
 __global__ __launch_bounds__(256, 1) void wino_gemm_fused_kernel(const float* __restrict__ U, WinoImage im, int Cg, int rows_p,
                                                                 int tiles_m, unsigned u_bytes, WinoEpi ep, WinoTail tl) {
   constexpr int R = kWinoR;
@@ -789,12 +818,42 @@ __global__ __launch_bounds__(256, 1) void wino_gemm_fused_kernel(const float* __
     const int t = rd; rd = nx; nx = wr; wr = t;
     par ^= 1;
   };
+  f32x16 sum[4] = {};
+  auto fold = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    asm volatile("s_nop 15\n\ts_nop 7" ::: "memory");   // the last MFMA's results are read below by instructions the compiler does not know
+    wino_pin_acc(acc);
+#pragma unroll
+    for (int e = 0; e < (FOLD ? 16 : 0); ++e) {
+      float y[2][2];
+      wino_pixels(acc, e, y);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) sum[i][e] += y[i >> 1][i & 1];
+      if (e % 4 == 3) {
+        __builtin_amdgcn_sched_barrier(0);
+        wino_pin_acc(acc);
+      }
+    }
+    // cleared in place (assigned, the compiler makes a second set and copies it): 0 * 0 + 0
+    float zero = 0.0f;
+    asm volatile("s_nop 7" : "+v"(zero));
+#pragma unroll
+    for (int f = 0; f < 16; ++f) asm volatile("v_mfma_f32_32x32x2_f32 %0, %1, %1, 0" : "+a"(acc[f]) : "v"(zero));
+    __builtin_amdgcn_sched_barrier(0);
+  };
   int it = 0;
+  if constexpr (FOLD) {
+    for (int chain = 1; chain < tl.chains; ++chain) {   // (the last chain has four stages at least: wino_geom)
+      const int end = min(chain * nk / tl.chains, nk - 3);
+      for (; it < end; ++it) step(it, std::true_type(), std::true_type());
+      fold();
+    }
+  }
   for (; it + 3 < nk; ++it) step(it, std::true_type(), std::true_type());
   if (it + 2 < nk) { step(it, std::false_type(), std::true_type()); ++it; }
   for (; it < nk; ++it) step(it, std::false_type(), std::false_type());
 
-  wino_epilogue(acc, ep, m0, n0, wave, lane);
+  wino_epilogue<FOLD>(acc, sum, ep, m0, n0, wave, lane);
 }
 
 // ---- the same on 64 rows, two blocks to a CU ---------------------------------------------------------------------------
@@ -1470,15 +1529,19 @@ int launch_conv_wino(const WinoGeom& g, bool bwd, const float* in, const float* 
   if (fused) {
     constexpr size_t lds_f = (size_t)kWinoR * kWinoStage + 2 * (size_t)kWinoRaw;
     static_assert(lds_f <= 160 * 1024, "ring and patch slots do not fit the 160 KB LDS of a CU");
-    static const hipError_t attr_f = hipFuncSetAttribute(reinterpret_cast<const void*>(&wino_gemm_fused_kernel),
-                                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_f);
+    static const hipError_t attr_f = [] {
+      hipError_t e = hipSuccess;
+      for (const void* k : {reinterpret_cast<const void*>(&wino_gemm_fused_kernel<false>), reinterpret_cast<const void*>(&wino_gemm_fused_kernel<true>)})
+        if (e == hipSuccess) e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_f);
+      return e;
+    }();
     if (attr_f != hipSuccess) return (int)attr_f;
     WinoImage im;
     im.x = in; im.x_bytes = a.x_bytes; im.Ci = g.blk5 ? g.C5 : g.Ci; im.Hi = g.Hi; im.Wi = g.Wi; im.halo = g.halo;
     im.blk5 = g.blk5;
     ProfScope prof(tag, 2.0 * 16.0 * (double)g.Ko * g.Ci * (double)g.tiles, stream);
     WinoTail tl;
-    tl.full = g.full_tiles; tl.S = g.tail_S; tl.L = g.tail_L;
+    tl.full = g.full_tiles; tl.S = g.tail_S; tl.L = g.tail_L; tl.chains = g.chains;
     tl.part = reinterpret_cast<float*>(static_cast<char*>(ws) + g.u_bytes + g.v_bytes + g.img_bytes);
     tl.slab_elems = g.slab_elems; tl.part_first = g.part_first;
     const long long T = (long long)tiles_m_ * tiles_n_;
@@ -1488,8 +1551,8 @@ int launch_conv_wino(const WinoGeom& g, bool bwd, const float* in, const float* 
       hipLaunchKernelGGL(wino_gemm64_kernel, dim3((unsigned)blocks), dim3(256), 2 * (size_t)kWinoStage2, stream, U, im, g.Cg, g.rows_p,
                          tiles_m_, u_bytes, ep, tl);
     else
-      hipLaunchKernelGGL(wino_gemm_fused_kernel, dim3((unsigned)blocks), dim3(256), lds_f, stream, U, im, g.Cg, g.rows_p, tiles_m_,
-                         u_bytes, ep, tl);
+      hipLaunchKernelGGL(g.chains > 1 ? wino_gemm_fused_kernel<true> : wino_gemm_fused_kernel<false>, dim3((unsigned)blocks), dim3(256), lds_f,
+                         stream, U, im, g.Cg, g.rows_p, tiles_m_, u_bytes, ep, tl);
     if (g.tail_S > 1) {
       if (int e = launch_status()) return e;
       WinoTailReduce r;

@@ -235,6 +235,7 @@ WINO_CASES = [
     (90, 64, 13, 13, 128, 1),     # 4410 tiles: the filter gradient in the form too, its tiles in several slices
     (1, 260, 7, 9, 130, 1),       # two blocks in sixteen slices of five stages (the last one of none)
     (5, 132, 12, 14, 64, 1),      # seven blocks, half of their rows past the last filter, in eight slices
+    (24, 252, 13, 13, 244, 1),    # 74 blocks in three slices (21, 21, 20 stages of 63) of two chains
 ]
 
 
@@ -300,15 +301,28 @@ def test_conv2d_winograd(dev, case):
     blocks_f = -(-K // 128) * -(-(Nn * -(-y_ref.shape[2] // 2) * -(-y_ref.shape[3] // 2)) // 32)
     if blocks_f <= 256 or C % 4: assert torch.equal(ys, y)
     if blocks_b <= 256 or K % 4: assert torch.equal(dxs, dx)
-    # what the library picks by itself: this form from 64 channels on both sides, 128-row tiles three quarters full and
-    # 192 blocks on, else a direct one
+    # what the library picks by itself is what it says it picks
     auto = ops.conv2d_fwd(xd, wd, 1, pad)
     direct = ops.conv2d_fwd(xd, wd, 1, pad, algo=_lib.RH_ALGO_DIRECT)
     assert_close(N(direct), y_ref, "RH_ALGO_DIRECT fwd")
-    blocks = -(-K // 128) * -(-(Nn * -(-y_ref.shape[2] // 2) * -(-y_ref.shape[3] // 2)) // 32)
-    takes = C >= 64 and K >= 64 and 4 * K >= 3 * (-(-K // 128) * 128) and blocks >= 192
+    takes = ops.conv2d_winograd_flops(x.shape, w.shape, 1, pad) > 0
     assert torch.equal(auto, y if takes else direct), "library's choice"
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("case", [(24, 128, 28, 28, 128, 1), (19, 384, 13, 13, 384, 1), (27, 512, 7, 7, 512, 1)], ids=str)
+def test_conv2d_winograd_error_on_small_grids(dev, case):
+    """Where the direct form's tiles are few it cuts its contraction into slices, whose short chains of sums lose few bits:
+    the Winograd form has no larger an error against 64 bits on such grids (two correct results' errors differ by
+    about the inverse root of their million elements; 3 % for that and for the fit that the chains are chosen by)."""
+    Nn, C, H, W, K, pad = case
+    say("winograd error case", case)
+    x, w, dy = synth.normal(23, 1, (Nn, C, H, W)), synth.normal(23, 2, (K, C, 3, 3)), synth.normal(23, 3, (Nn, K, H, W))
+    xd, wd, dyd = T(x, dev), T(w, dev), T(dy, dev)
+    for ref, run in ((O.conv2d_fwd(x, w, 1, pad), lambda algo: ops.conv2d_fwd(xd, wd, 1, pad, algo=algo)),
+                     (O.conv2d_bwd_data(w, dy, x.shape, 1, pad), lambda algo: ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=algo))):
+        err = [float(np.linalg.norm(N(run(algo)).astype(np.float64) - ref)) for algo in (_lib.RH_ALGO_WINOGRAD, _lib.RH_ALGO_SCALAR_OFFSET)]
+        assert err[0] <= 1.03 * err[1], err
 
 
 @pytest.mark.parametrize("case", [(3, 4, 9, 7, 64, 1), (2, 8, 13, 13, 64, 1), (2, 12, 8, 9, 33, 0), (3, 16, 7, 7, 50, 2), (2, 20, 11, 6, 64, 1),
