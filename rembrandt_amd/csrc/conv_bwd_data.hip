@@ -173,19 +173,19 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
     if (d.x_elems == 0) return 0;
     return launch_conv1x1_stream(d, RH_CONV_BWD_DATA, w, dy, dx, alpha, beta, nullptr, 0, stream, mask);
   }
-  if (wino_shape(d) && !(flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT))) {
-    WinoGeom wg = wino_geom_bwd_data(d);
-    if (flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays(d, wg, plan_lds_bwd_data(d))) {
-      if (d.x_elems == 0) return 0;
-      if ((flags & RH_ALGO_SHARED_GPU) && wg.full_tiles > 0) wg.tail_S = 1;   // (a grid under one round is sliced all the same)
-      return launch_conv_wino(wg, true, dy, w, dx, alpha, beta, nullptr, 0, mask, ws, stream, "conv_bwd_data_wino");
+  if (has_staged_form(d) && !(flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET))) {
+    const DirectForms f = direct_bwd_data(d);
+    if (wino_shape(d) && !(flags & RH_ALGO_DIRECT)) {
+      WinoGeom wg = wino_geom_bwd_data(d);
+      if (flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays(wg, f)) {
+        if (d.x_elems == 0) return 0;
+        if ((flags & RH_ALGO_SHARED_GPU) && wg.full_tiles > 0) wg.tail_S = 1;   // (a grid under one round is sliced all the same)
+        return launch_conv_wino(wg, true, dy, w, dx, alpha, beta, nullptr, 0, mask, ws, stream, "conv_bwd_data_wino");
+      }
+      if (flags & RH_ALGO_WINOGRAD) return RH_E_UNSUPPORTED;
     }
-    if (flags & RH_ALGO_WINOGRAD) return RH_E_UNSUPPORTED;
-  }
-  if (!(flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET)) && d.x_elems > 0) {
-    const LdsConvPlan lp = plan_lds_bwd_data(d);
-    if (lds_pays(d, lp))
-      return launch_conv_lds(lp, true, d.N, d.K, d.P, d.Q, d.C, d.H, d.W, d.R, d.R - 1 - d.pad, dy, w, dx, alpha, beta, nullptr, 0,
+    if (f.staged && d.x_elems > 0)
+      return launch_conv_lds(f.lds, true, d.N, d.K, d.P, d.Q, d.C, d.H, d.W, d.R, d.R - 1 - d.pad, dy, w, dx, alpha, beta, nullptr, 0,
                              mask, ws, stream);
   }
   const int KRS = d.K * d.R * d.S;

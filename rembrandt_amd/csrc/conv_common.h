@@ -318,6 +318,37 @@ inline SoffPlan plan_soff_fwd(const ConvDims& d) {
   return p;
 }
 
+// Backward-data with stride 1: dx[n,c,h,w] = sum dyp[n,ko,h+R-1-r,w+S-1-s] * w[ko,c,r,s] on dy padded
+// by R-1-pad zeros per side.
+// Backward-data as a stride-1 correlation of the flipped filter with dy.  For stride > 1 the padded copy of dy is
+// also dilated (dy[p][q] lands on [halo + st*p][halo + st*q], zeros between): the contraction then multiplies
+// (st^2 - 1)/st^2 zeros, but runs on the scalar-offset loaders; the copy is (H + R - 1) x (W + S - 1) per plane.
+inline SoffPlan plan_soff_bwd_data(const ConvDims& d) {
+  SoffPlan p;
+  p.n_k = round_up(d.K * d.R * d.S, kTabPad);
+  p.halo = d.R - 1 - d.pad;
+  p.Hp = d.H + d.R - 1;   // = P + 2*halo when the stride is 1
+  p.Wp = d.W + d.S - 1;
+  p.tab_bytes = align256(sizeof(int) * (size_t)p.n_k);
+  p.wt_bytes = align256(sizeof(float) * (size_t)p.n_k * d.C);
+  const size_t img = p.halo >= 0 ? sizeof(float) * (size_t)d.N * d.K * p.Hp * p.Wp : 0;
+  p.img_bytes = (p.halo > 0 || d.st > 1 || p.Hp != d.P || p.Wp != d.Q) ? align256(img) : 0;
+  p.ok = p.halo >= 0 && d.R == d.S && img <= kMaxBufferBytes && d.P > 0 && d.Q > 0;
+  p.splits = soff_splits_bwd_data(d, p.n_k);
+  p.tail = plan_tail_split(d.C, (long long)d.N * d.H * d.W, p.n_k);
+  if (pick_bm(d.C) == 128 && p.splits == 1 && plan_k_split(d.C, (long long)d.N * d.H * d.W, p.n_k) > 1) {
+    // As in the forward pass, where 128 x 64 tiles need no slices (NIN's 1024-channel 1x1 layers: 0.120 -> 0.098 ms).
+    // Where they would still be sliced the 128 x 128 tile stays (a 384-channel 3x3 layer on 6 x 6 lost 9 %).
+    p.narrow128 = true;
+    p.tail = plan_tail_split(d.C, (long long)d.N * d.H * d.W, p.n_k, 64);
+  }
+  if (d.st > 1) p.tail.splits = 1;  // the zero-dilated form is a fallback only
+  const size_t tail_elems_b = (size_t)(d.x_elems - tail_first_elem(p.tail, (long long)d.H * d.W, d.C));
+  p.part_bytes = p.splits > 1 ? align256(sizeof(float) * (size_t)p.splits * (size_t)d.x_elems)
+               : p.tail.splits > 1 ? align256(sizeof(float) * (size_t)p.tail.splits * tail_elems_b) : 0;
+  return p;
+}
+
 // Winograd F(2x2, 3x3) form of a 3x3 stride-1 layer (conv_wino.hip), written as a forward convolution: an input of
 // (N, Ci, Hi, Wi) with `halo` zeros around it, Ko filters, a result of (N, Ko, P, Q).  Backward-data is the same over dy
 // with halo 2 - pad.  Scratch: [U: transformed filter][V: transformed image patches].
@@ -412,14 +443,6 @@ struct LdsConvPlan {
   int qps, splits;       // channel quads per slice of the contraction; slices
   double us;             // what a call is expected to take
 };
-// What the engine's forward and backward-data forms take on a stride-1 layer, with their operand copies and reductions, by
-// the direct form's FLOPs: a fit to the same layers (rms error 17 %; 14 us at 50 MFLOP, 34 at 1 GFLOP, 119 at 10, 363 at 50).
-// The staged form is taken where its own estimate is below this: at every batch of a small network's layers, up to
-// some 10 GFLOP on 128 rows and more, beyond 30 on the 64-row tiles the engine is weakest at.
-inline double conv_engine_us(const ConvDims& d) {
-  const double mflop = 2e-6 * (double)d.y_elems * d.C * d.R * d.S;
-  return 9.3 + mflop / 197.0 + 0.59 * sqrt(mflop);
-}
 // N images of Ci channels, `rows` result channels of P x Q.
 LdsConvPlan plan_conv_lds(int N, int Ci, int rows, int P, int Q, int R, int S, int st);
 inline LdsConvPlan plan_lds_fwd(const ConvDims& d) { return plan_conv_lds(d.N, d.C, d.K, d.P, d.Q, d.R, d.S, d.st); }
@@ -428,25 +451,80 @@ inline LdsConvPlan plan_lds_bwd_data(const ConvDims& d) {   // (halo R - 1 - pad
   p.ok = p.ok && d.pad <= d.R - 1;
   return p;
 }
-inline bool lds_pays(const ConvDims& d, const LdsConvPlan& p) { return p.ok && p.us < conv_engine_us(d); }
-// Where the library takes the Winograd form by itself: enough channels on both sides for the 16 products to be worth their
-// transforms, and either a grid that fills the GPU, or (sliced, wino_geom) a call expected to take less time than both
-// direct forms: from batch 5 or so on for 128 channels and more (256 -> 384, 13 x 13: batch 3 33 us against 25 staged,
-// batch 8 36 against 46 on the engine and 41 staged, batch 32 79 against 97 and 111).
-// (Against the staged form by an eighth at least: its two or three launches count for more in a chain of layers than timed
-// back to back, ResNet-18 on 9 images 457 us with 1/8, 476 with the plain comparison.)
-inline bool wino_fastest(const ConvDims& d, const WinoGeom& g, const LdsConvPlan& lp) {
-  return g.fine && g.Ci % 4 == 0 && g.us < conv_engine_us(d) && !(lp.ok && lp.us * 0.875 <= g.us);
+// What the engine's forward and backward-data forms take on a stride-1 layer of `rows` result channels and `cols` pixels, in
+// microseconds: the copies in front (none in the gather form), rounds of the blocks a CU holds at a time, each K step of a
+// block taking its share of the matrix pipes or, with few blocks, its MFMAs and 0.43 us of waiting, and the reduction of
+// the slices.  A fit to 1582 timings of 792 layers (14 of the benchmark networks at 28 batches, 400 of random sizes; rms
+// error 11 %; by FLOPs alone it is 32 % and too short by a third where tiles are mostly empty).
+inline double engine_us(const SoffPlan& p, int rows, long long cols, size_t w_elems, bool gather) {
+  if (!p.ok) return 1e30;
+  const int bm = pick_bm(rows), splits = gather ? 1 : p.splits;
+  const bool k8 = bm == 64 && rows <= 64 && prefer_k8_64(cols);
+  int bn = bm >= 96 ? 128 : splits > 1 && !gather && !k8 ? 128 : 256;
+  if (bm == 128 && p.narrow128 && !gather) bn = 64;
+  if (bm == 96 && gather) bn = 256;
+  const double out_bytes = 4.0 * (double)rows * (double)cols, steps = p.n_k / 16.0;
+  const double step_us = bm * bn * 16 / 128.0 / 2300.0;   // MFMAs of a step of a block, alone on a CU
+  const double busy_us = step_us * (bm == 128 ? 1.09 : bm == 96 ? 1.17 : bm == 64 ? 1.15 : 1.28) * (gather ? 1.1 : 1.0);
+  const long long tiles = (long long)cdiv(rows, bm) * cdiv<long long>(cols, bn), held = bm >= 96 || k8 ? 4 : 3;
+  double us;
+  if (splits == 1 && !gather && p.tail.splits > 1) {
+    us = steps * busy_us * (double)tiles / 256.0;
+  } else {
+    const long long per_cu = cdiv<long long>(tiles * splits, 256), rem = per_cu % held;
+    auto round_us = [&](long long k) { return steps / splits * fmax((double)k * busy_us, step_us + 0.43); };
+    us = (double)(per_cu / held) * round_us(held) + (rem ? round_us(rem) : 0.0);
+  }
+  us = fmax(us, out_bytes / 4.0e6);
+  us += gather ? 5.8 : 6.1 + fmax(2.0 * (double)p.img_bytes / 3.7e6, 8.0 * (double)w_elems / 1.5e6);
+  if (splits > 1) us += 4.1 + out_bytes * (2 * splits + 1) / 6.0e6;
+  else if (!gather && p.tail.splits > 1) us += 4.1 + 2.0 * (double)p.part_bytes / 6.0e6;
+  return us;
 }
-inline bool wino_pays(const ConvDims& d, const WinoGeom& g, const LdsConvPlan& lp) {
+// A contraction that fits two K steps goes to the gather form of the forward pass, which needs no launch in front of it
+// (a 5x5 layer on one channel).
+inline bool fwd_gathers(const ConvDims& d) { return d.C * d.R * d.S <= 32; }
+
+// The direct forms of a 3x3 or 5x5 stride-1 layer and which of them is taken: the staged one where its estimate is below
+// the engine's by a twentieth at least (on those timings the choice is then 0.35 % slower than the better one on average,
+// 0.31 % with the plain comparison, but in 8 instead of 4 of them 8 % slower than the engine or more; by FLOPs alone 4.4 %).
+struct DirectForms {
+  SoffPlan soff;
+  LdsConvPlan lds;
+  bool staged;
+  double us;   // what the one taken is expected to take
+};
+inline bool has_staged_form(const ConvDims& d) { return d.R == d.S && (d.R == 3 || d.R == 5) && d.st == 1; }
+inline DirectForms pick_direct(const SoffPlan& soff, const LdsConvPlan& lds, double engine) {
+  DirectForms f = {soff, lds, lds.ok && lds.us < 0.95 * engine, engine};
+  if (f.staged) f.us = lds.us;
+  return f;
+}
+inline DirectForms direct_fwd(const ConvDims& d) {
+  const SoffPlan p = plan_soff_fwd(d);
+  return pick_direct(p, plan_lds_fwd(d), engine_us(p, d.K, (long long)d.N * d.P * d.Q, d.w_elems, fwd_gathers(d)));
+}
+inline DirectForms direct_bwd_data(const ConvDims& d) {
+  const SoffPlan p = plan_soff_bwd_data(d);
+  return pick_direct(p, plan_lds_bwd_data(d), engine_us(p, d.C, (long long)d.N * d.H * d.W, d.w_elems, false));
+}
+
+// Where the library takes the Winograd form by itself: enough channels on both sides for the 16 products to be worth their
+// transforms, and either a grid that fills the GPU, or a call expected to take less time than the direct form's: from 8 to
+// 18 images on for 128 channels and more (256 -> 384, 13 x 13: 8, 256 -> 256, 14 x 14: 11, 384 -> 1024, 6 x 6: 18).  Rounds
+// of blocks make either form the shorter one again for a batch or two (512 -> 512, 7 x 7: 16, 21 to 24, from 27 on).
+// A plain comparison of the estimates: against the best of the forms, on the timings above, 0.3 % slower on average;
+// asking an eighth of the Winograd form 1.6 % (and ResNet-18 on 9 images takes 436 us with it plain, 442 with the eighth).
+inline bool wino_fastest(const WinoGeom& g, const DirectForms& f) { return g.fine && g.Ci % 4 == 0 && g.us < f.us; }
+inline bool wino_pays(const WinoGeom& g, const DirectForms& f) {
   if (!g.ok || g.Ci < 64 || g.Ko < 64) return false;
   const long long blocks = (long long)(g.rows_p / g.bm) * (g.tiles_p / kWinoBN);
   // 64-row tiles, two to a CU: from a whole round of blocks on, or from three quarters of the CUs on where it is expected
   // to be the fastest (64 -> 64 56x56: batch 24, 588 blocks 53 us against 57 direct; 64 98 against 144)
-  if (g.bm == kWinoBM2) return 4 * g.Ko >= 3 * g.rows_p && ((blocks >= 512 && g.fine) || (blocks >= 192 && wino_fastest(d, g, lp)));
+  if (g.bm == kWinoBM2) return 4 * g.Ko >= 3 * g.rows_p && ((blocks >= 512 && g.fine) || (blocks >= 192 && wino_fastest(g, f)));
   // (rows: 128-row tiles at least three quarters full: 64 filters in one would execute as much as the direct form)
   if (4 * g.Ko >= 3 * g.rows_p && blocks >= 192) return true;
-  return wino_fastest(d, g, lp);
+  return wino_fastest(g, f);
 }
 // The 5x5 forward form executes 64 % of the direct form's multiply-adds (a little more where the 2x2 tiles overhang
 // the result) at a lower rate than the direct kernels reach, 18 % less time on 96 -> 256 channels, 27 x 27, batch 256:
@@ -454,10 +532,10 @@ inline bool wino_pays(const ConvDims& d, const WinoGeom& g, const LdsConvPlan& l
 // for several row tiles (which share the patches a block reads four times over) from one round on where it is expected to be
 // the fastest (the same layer at batch 24: 151 us against 204 on the engine and 200 staged; below one round, at batch
 // 16, 122 against 124 staged: not worth its scratch).
-inline bool wino_pays5(const ConvDims& d, const WinoGeom& g, const LdsConvPlan& lp) {
+inline bool wino_pays5(const WinoGeom& g, const DirectForms& f) {
   if (!g.ok || !g.blk5 || g.C5 < 64 || g.Ko < 64 || 8 * g.Ko < 7 * g.rows_p) return false;
   const long long blocks = (long long)(g.rows_p / kWinoBM) * (g.tiles_p / kWinoBN);
-  return blocks >= 512 || (blocks >= 256 && g.rows_p > kWinoBM && wino_fastest(d, g, lp));
+  return blocks >= 512 || (blocks >= 256 && g.rows_p > kWinoBM && wino_fastest(g, f));
 }
 
 int launch_conv_lds(const LdsConvPlan& pl, bool bwd, int N, int Ci, int H, int W, int rows, int P, int Q, int R, int halo,
@@ -501,37 +579,6 @@ inline Bf16FwdPlan plan_bf16_fwd(const ConvDims& d) {
   p.img_bytes = align256(img);
   p.ok = (d.C % 8 == 0 || d.st % 2 == 0) && img <= kMaxBufferBytes && d.P > 0 && d.Q > 0 &&
          (long long)p.Hp * p.Wp < (1ll << 31) / 64;
-  return p;
-}
-
-// Backward-data with stride 1: dx[n,c,h,w] = sum dyp[n,ko,h+R-1-r,w+S-1-s] * w[ko,c,r,s] on dy padded
-// by R-1-pad zeros per side.
-// Backward-data as a stride-1 correlation of the flipped filter with dy.  For stride > 1 the padded copy of dy is
-// also dilated (dy[p][q] lands on [halo + st*p][halo + st*q], zeros between): the contraction then multiplies
-// (st^2 - 1)/st^2 zeros, but runs on the scalar-offset loaders; the copy is (H + R - 1) x (W + S - 1) per plane.
-inline SoffPlan plan_soff_bwd_data(const ConvDims& d) {
-  SoffPlan p;
-  p.n_k = round_up(d.K * d.R * d.S, kTabPad);
-  p.halo = d.R - 1 - d.pad;
-  p.Hp = d.H + d.R - 1;   // = P + 2*halo when the stride is 1
-  p.Wp = d.W + d.S - 1;
-  p.tab_bytes = align256(sizeof(int) * (size_t)p.n_k);
-  p.wt_bytes = align256(sizeof(float) * (size_t)p.n_k * d.C);
-  const size_t img = p.halo >= 0 ? sizeof(float) * (size_t)d.N * d.K * p.Hp * p.Wp : 0;
-  p.img_bytes = (p.halo > 0 || d.st > 1 || p.Hp != d.P || p.Wp != d.Q) ? align256(img) : 0;
-  p.ok = p.halo >= 0 && d.R == d.S && img <= kMaxBufferBytes && d.P > 0 && d.Q > 0;
-  p.splits = soff_splits_bwd_data(d, p.n_k);
-  p.tail = plan_tail_split(d.C, (long long)d.N * d.H * d.W, p.n_k);
-  if (pick_bm(d.C) == 128 && p.splits == 1 && plan_k_split(d.C, (long long)d.N * d.H * d.W, p.n_k) > 1) {
-    // As in the forward pass, where 128 x 64 tiles need no slices (NIN's 1024-channel 1x1 layers: 0.120 -> 0.098 ms).
-    // Where they would still be sliced the 128 x 128 tile stays (a 384-channel 3x3 layer on 6 x 6 lost 9 %).
-    p.narrow128 = true;
-    p.tail = plan_tail_split(d.C, (long long)d.N * d.H * d.W, p.n_k, 64);
-  }
-  if (d.st > 1) p.tail.splits = 1;  // the zero-dilated form is a fallback only
-  const size_t tail_elems_b = (size_t)(d.x_elems - tail_first_elem(p.tail, (long long)d.H * d.W, d.C));
-  p.part_bytes = p.splits > 1 ? align256(sizeof(float) * (size_t)p.splits * (size_t)d.x_elems)
-               : p.tail.splits > 1 ? align256(sizeof(float) * (size_t)p.tail.splits * tail_elems_b) : 0;
   return p;
 }
 

@@ -640,21 +640,21 @@ extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x,
   if (!(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET)) && conv1x1_stream_applies(d))
     return launch_conv1x1_stream(d, RH_CONV_FWD, w, x, y, alpha, beta, (flags & RH_FUSE_BIAS) ? bias : nullptr,
                                  (flags & RH_FUSE_RELU) ? 1 : 0, stream);
-  if ((wino_shape(d) || wino_shape5(d)) && !(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT))) {
-    const bool five = wino_shape5(d);   // a 5x5 layer as four 3x3 layers, added in the transform domain
-    WinoGeom wg = five ? wino_geom_fwd5(d) : wino_geom_fwd(d);
-    if ((flags & RH_ALGO_SHARED_GPU) && wg.full_tiles > 0) wg.tail_S = 1;
-    const LdsConvPlan lp = plan_lds_fwd(d);
-    if (flags & RH_ALGO_WINOGRAD ? wg.ok : five ? wino_pays5(d, wg, lp) : wino_pays(d, wg, lp))
-      return launch_conv_wino(wg, false, x, w, y, alpha, beta, (flags & RH_FUSE_BIAS) ? bias : nullptr,
-                              (flags & RH_FUSE_RELU) ? 1 : 0, nullptr, ws, stream, "conv_fwd_wino");
-    if (flags & RH_ALGO_WINOGRAD) return RH_E_UNSUPPORTED;
-  }
-  if (!(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET))) {
-    const LdsConvPlan lp = plan_lds_fwd(d);
-    if (lds_pays(d, lp))
-      return launch_conv_lds(lp, false, d.N, d.C, d.H, d.W, d.K, d.P, d.Q, d.R, d.pad, x, w, y, alpha, beta,
-                             (flags & RH_FUSE_BIAS) ? bias : nullptr, (flags & RH_FUSE_RELU) ? 1 : 0, nullptr, ws, stream);
+  const float* const bias_arg = (flags & RH_FUSE_BIAS) ? bias : nullptr;
+  const int relu_arg = (flags & RH_FUSE_RELU) ? 1 : 0;
+  if (has_staged_form(d) && !(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET))) {
+    const DirectForms f = direct_fwd(d);
+    if ((wino_shape(d) || wino_shape5(d)) && !(flags & RH_ALGO_DIRECT)) {
+      const bool five = wino_shape5(d);   // a 5x5 layer as four 3x3 layers, added in the transform domain
+      WinoGeom wg = five ? wino_geom_fwd5(d) : wino_geom_fwd(d);
+      if ((flags & RH_ALGO_SHARED_GPU) && wg.full_tiles > 0) wg.tail_S = 1;
+      if (flags & RH_ALGO_WINOGRAD ? wg.ok : five ? wino_pays5(wg, f) : wino_pays(wg, f))
+        return launch_conv_wino(wg, false, x, w, y, alpha, beta, bias_arg, relu_arg, nullptr, ws, stream, "conv_fwd_wino");
+      if (flags & RH_ALGO_WINOGRAD) return RH_E_UNSUPPORTED;
+    }
+    if (f.staged)
+      return launch_conv_lds(f.lds, false, d.N, d.C, d.H, d.W, d.K, d.P, d.Q, d.R, d.pad, x, w, y, alpha, beta, bias_arg, relu_arg,
+                             nullptr, ws, stream);
   }
   const int CRS = d.C * d.R * d.S;
   if ((flags & RH_MATH_BF16_MFMA_FP32ACC) && !(flags & RH_ALGO_GATHER)) {
@@ -673,8 +673,7 @@ extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x,
   }
   const SoffPlan sp = plan_soff_fwd(d);
   if ((flags & RH_MATH_BF16_MFMA_FP32ACC) && (!sp.ok || (flags & RH_ALGO_GATHER))) return RH_E_UNSUPPORTED;
-  // (fp32, a contraction of up to 32, a 5x5 layer on one channel: the gather form is as fast and needs no launch in front of it)
-  const bool tiny_k = CRS <= 32 && !(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_SCALAR_OFFSET));
+  const bool tiny_k = fwd_gathers(d) && !(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_SCALAR_OFFSET));
   if (sp.ok && !(flags & RH_ALGO_GATHER) && !tiny_k) {
     int* soff = static_cast<int*>(ws);
     float* wT = reinterpret_cast<float*>(static_cast<char*>(ws) + sp.tab_bytes);

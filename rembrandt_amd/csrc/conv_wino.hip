@@ -1665,7 +1665,7 @@ extern "C" double rh_conv2d_winograd_flops(const rh_conv_geom* g, int pass, int 
   if (flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT)) return 0.0;
   if (wino_shape5(d) && pass == RH_CONV_FWD) {
     const WinoGeom wg = wino_geom_fwd5(d);
-    if (!(flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays5(d, wg, plan_lds_fwd(d)))) return 0.0;
+    if (!(flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays5(wg, direct_fwd(d)))) return 0.0;
     return 2.0 * 16.0 * (double)wg.Ko * wg.Ci * (double)wg.tiles;
   }
   if (!wino_shape(d)) return 0.0;
@@ -1676,7 +1676,7 @@ extern "C" double rh_conv2d_winograd_flops(const rh_conv_geom* g, int pass, int 
   }
   if (pass != RH_CONV_FWD && pass != RH_CONV_BWD_DATA) return 0.0;
   const WinoGeom wg = pass == RH_CONV_FWD ? wino_geom_fwd(d) : wino_geom_bwd_data(d);
-  if (!(flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays(d, wg, pass == RH_CONV_FWD ? plan_lds_fwd(d) : plan_lds_bwd_data(d)))) return 0.0;
+  if (!(flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays(wg, pass == RH_CONV_FWD ? direct_fwd(d) : direct_bwd_data(d)))) return 0.0;
   return 2.0 * 16.0 * (double)wg.Ko * wg.Ci * (double)wg.tiles;
 }
 

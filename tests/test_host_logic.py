@@ -31,6 +31,17 @@ def test_library_exports_every_declared_symbol():
     assert b"gfx950" in _lib.lib().rh_version()
 
 
+@pytest.mark.parametrize("layer", [(128, 28, 128), (256, 13, 384), (384, 13, 384), (384, 13, 256), (256, 14, 256)], ids=str)
+def test_winograd_choice_does_not_flip_with_the_batch(layer):
+    """From 16 images on the 3x3 layers of 128 channels and more take the Winograd form at every batch, in both passes: its
+    time and the direct forms' grow by the same rounds of blocks, and it is a fifth to a half shorter."""
+    c, extent, k = layer
+    for pass_ in (_lib.RH_CONV_FWD, _lib.RH_CONV_BWD_DATA):
+        for n in range(16, 257):
+            g = _lib.ConvGeom(n, c, extent, extent, k, 3, 3, 1, 1)
+            assert _lib.lib().rh_conv2d_winograd_flops(C.byref(g), pass_, 0) > 0, (pass_, n)
+
+
 def _c_prototypes(header):
     """name -> argument count of every function include/<header> declares."""
     text = open(os.path.join(ROOT, "include", header)).read()
