@@ -59,7 +59,8 @@ typedef void* rh_stream_t; /* hipStream_t */
                                              Forms that spend compute-unit time to shorten the call's own last round of
                                              blocks (the Winograd kernels' sliced tail blocks) are not taken: beside
                                              other work the idle units of that round are not idle (measured: the
-                                             ResNet-18 template step 26.5 -> 26.1 ms).  Same result up to summation order. */
+                                             ResNet-18 template step 26.5 -> 26.1 ms).  Grids of less than one round
+                                             are sliced with the hint as without.  Same result up to summation order. */
 
 const char* rh_version(void);
 /* Status of the most recent launch made by a void `rembrandt_kernel_*` entry point on this thread. */

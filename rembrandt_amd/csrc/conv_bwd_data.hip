@@ -177,9 +177,9 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
     const DirectForms f = direct_bwd_data(d);
     if (wino_shape(d) && !(flags & RH_ALGO_DIRECT)) {
       WinoGeom wg = wino_geom_bwd_data(d);
+      if (flags & RH_ALGO_SHARED_GPU) wg.beside_others();
       if (flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays(wg, f)) {
         if (d.x_elems == 0) return 0;
-        if ((flags & RH_ALGO_SHARED_GPU) && wg.full_tiles > 0) wg.tail_S = 1;   // (a grid under one round is sliced all the same)
         return launch_conv_wino(wg, true, dy, w, dx, alpha, beta, nullptr, 0, mask, ws, stream, "conv_bwd_data_wino");
       }
       if (flags & RH_ALGO_WINOGRAD) return RH_E_UNSUPPORTED;

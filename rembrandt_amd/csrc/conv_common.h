@@ -364,6 +364,12 @@ struct WinoGeom {
   bool ok;
   bool fine;                  // no call of it loses more bits than the direct form's slices would (see wino_stages_at_most)
   double us;                  // what a call is expected to take
+  double whole_us;            // the same with the tail form left out
+  // (RH_ALGO_SHARED_GPU: other kernels fill the CUs that a last round leaves idle.  A grid under one round stays sliced:
+  // its slices are how long the call is, with or without neighbours.)
+  void beside_others() {
+    if (full_tiles > 0) { tail_S = 1; us = whole_us; }
+  }
   // Tail form (V made in the kernel only): the blocks past the last multiple of 256 (all of them where there are fewer) are cut into tail_S slices of the
   // channel loop, tail_L stages each, whose untransformed-blend partial results go to slabs of scratch that hold the
   // result from element part_first on (the first image a tail block touches); tail_S == 1: not worth it.

@@ -647,7 +647,7 @@ extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x,
     if ((wino_shape(d) || wino_shape5(d)) && !(flags & RH_ALGO_DIRECT)) {
       const bool five = wino_shape5(d);   // a 5x5 layer as four 3x3 layers, added in the transform domain
       WinoGeom wg = five ? wino_geom_fwd5(d) : wino_geom_fwd(d);
-      if ((flags & RH_ALGO_SHARED_GPU) && wg.full_tiles > 0) wg.tail_S = 1;
+      if (flags & RH_ALGO_SHARED_GPU) wg.beside_others();
       if (flags & RH_ALGO_WINOGRAD ? wg.ok : five ? wino_pays5(wg, f) : wino_pays(wg, f))
         return launch_conv_wino(wg, false, x, w, y, alpha, beta, bias_arg, relu_arg, nullptr, ws, stream, "conv_fwd_wino");
       if (flags & RH_ALGO_WINOGRAD) return RH_E_UNSUPPORTED;

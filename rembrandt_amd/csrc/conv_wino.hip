@@ -21,7 +21,8 @@
 //    additions in registers, then alpha / beta, bias, ReLU or the mask of a folded ReLU backward, and the 2x2 pixels
 //    go to the NCHW result (odd extents: the tile's pixels past the edge are dropped).
 //  * blocks past the last whole round of the 256 CUs take slices of the channel loop and wino_tail_reduce_kernel adds
-//    their partial results (wino_geom); not where the caller says that other kernels run beside the call.
+//    their partial results (wino_geom); not where the caller says that other kernels run beside the call.  Grids of
+//    fewer blocks than that are sliced whole, and a slice's stages divided into chains (FOLD).
 //  * the forward pass of a 5x5 stride-1 layer is the same kernel over four times the channels: the filter's zero
 //    extension to 6x6 is four 3x3 filters, the layer the sum of their four 3x3 layers over the input read 3 rows / 3
 //    columns further on, and that sum is taken in the transform domain like the one over the channels
@@ -97,7 +98,7 @@ WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int max_L, i
   auto folds_us = [&](int L) { return 1.75 * (chains_of(L) - 1) * stage_us; };
   g.chains = chains_of(g.Cg);
   g.fine = cdiv(g.Cg, g.chains) <= max_L;
-  g.us = fixed_us + (stages_us(1.0, g.Cg) + folds_us(g.Cg)) * rounds(T);
+  g.us = g.whole_us = fixed_us + (stages_us(1.0, g.Cg) + folds_us(g.Cg)) * rounds(T);
   if (g.ok && Ci % 4 == 0 && tail > 0) {
     double best = rounds(T) * 0.97, best_us = g.us;
     for (int S = 2; S <= 16; ++S) {
@@ -1664,7 +1665,8 @@ extern "C" double rh_conv2d_winograd_flops(const rh_conv_geom* g, int pass, int 
   if (conv_dims(g, &d)) return 0.0;
   if (flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT)) return 0.0;
   if (wino_shape5(d) && pass == RH_CONV_FWD) {
-    const WinoGeom wg = wino_geom_fwd5(d);
+    WinoGeom wg = wino_geom_fwd5(d);
+    if (flags & RH_ALGO_SHARED_GPU) wg.beside_others();
     if (!(flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays5(wg, direct_fwd(d)))) return 0.0;
     return 2.0 * 16.0 * (double)wg.Ko * wg.Ci * (double)wg.tiles;
   }
@@ -1675,7 +1677,8 @@ extern "C" double rh_conv2d_winograd_flops(const rh_conv_geom* g, int pass, int 
     return 2.0 * 16.0 * (double)d.K * d.C * (double)wp.tiles;
   }
   if (pass != RH_CONV_FWD && pass != RH_CONV_BWD_DATA) return 0.0;
-  const WinoGeom wg = pass == RH_CONV_FWD ? wino_geom_fwd(d) : wino_geom_bwd_data(d);
+  WinoGeom wg = pass == RH_CONV_FWD ? wino_geom_fwd(d) : wino_geom_bwd_data(d);
+  if (flags & RH_ALGO_SHARED_GPU) wg.beside_others();
   if (!(flags & RH_ALGO_WINOGRAD ? wg.ok : wino_pays(wg, pass == RH_CONV_FWD ? direct_fwd(d) : direct_bwd_data(d)))) return 0.0;
   return 2.0 * 16.0 * (double)wg.Ko * wg.Ci * (double)wg.tiles;
 }

@@ -300,8 +300,8 @@ def test_conv2d_winograd(dev, case):
     # run to run the same bits
     assert torch.equal(ops.conv2d_fwd(xd, wd, 1, pad, algo=WG), y)
     assert torch.equal(ops.conv2d_bwd_filter(xd, dyd, w.shape, 1, pad, algo=WG), dw)
-    # RH_ALGO_SHARED_GPU (other kernels run beside the call): whole blocks only, no sliced tail; the same result up to
-    # summation order where a tail was sliced, the same bits where none was
+    # RH_ALGO_SHARED_GPU (other kernels run beside the call): no sliced tail behind a whole round of blocks; the same result
+    # up to summation order where a tail was sliced, the same bits where none was or the grid is under one round
     SH = _lib.RH_ALGO_SHARED_GPU
     ys = ops.conv2d_fwd(xd, wd, 1, pad, algo=WG | SH)
     dxs = ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=WG | SH)

@@ -42,6 +42,16 @@ def test_winograd_choice_does_not_flip_with_the_batch(layer):
             assert _lib.lib().rh_conv2d_winograd_flops(C.byref(g), pass_, 0) > 0, (pass_, n)
 
 
+@pytest.mark.parametrize("layer", [(45, 64, 27, 66), (84, 64, 28, 72), (42, 64, 28, 66)], ids=str)
+def test_winograd_choice_beside_other_kernels_is_by_whole_blocks(layer):
+    """RH_ALGO_SHARED_GPU leaves the slices of a call's last round out, so its Winograd form is judged without them: these
+    calls (one round of blocks and a few more, half of their rows empty) are worth it only with a sliced last round."""
+    n, c, extent, k = layer
+    g = _lib.ConvGeom(n, c, extent, extent, k, 3, 3, 1, 1)
+    assert _lib.lib().rh_conv2d_winograd_flops(C.byref(g), _lib.RH_CONV_FWD, 0) > 0
+    assert _lib.lib().rh_conv2d_winograd_flops(C.byref(g), _lib.RH_CONV_FWD, _lib.RH_ALGO_SHARED_GPU) == 0
+
+
 def _c_prototypes(header):
     """name -> argument count of every function include/<header> declares."""
     text = open(os.path.join(ROOT, "include", header)).read()
