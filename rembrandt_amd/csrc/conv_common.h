@@ -265,7 +265,7 @@ inline int plan_k_split(int rows, long long cols, int n_k, int bn_force = 0) {
   const int bm = pick_bm(rows), bn = bn_force ? bn_force : bm >= 96 ? 128 : 256;
   const long long slots = 256 * (bm >= 96 ? 4 : 3);
   const long long tiles = (long long)cdiv(rows, bm) * cdiv<long long>(cols, bn);
-  if (tiles * 2 > slots) return 1;
+  if (tiles == 0 || tiles * 2 > slots) return 1;
   long long want = slots / tiles;
   const long long by_depth = slices_by_depth(n_k / 16, tiles, slots, 16, 4);
   if (want > by_depth) want = by_depth;

@@ -52,6 +52,17 @@ def test_winograd_choice_beside_other_kernels_is_by_whole_blocks(layer):
     assert _lib.lib().rh_conv2d_winograd_flops(C.byref(g), _lib.RH_CONV_FWD, _lib.RH_ALGO_SHARED_GPU) == 0
 
 
+def test_scratch_of_a_convolution_without_output():
+    """A filter larger than the padded image has no output pixels: the scratch queries answer (they divided by the number
+    of tiles) and no form is chosen for it."""
+    for extent, size, pad in ((2, 3, 0), (1, 3, 0), (3, 5, 0), (2, 7, 1)):
+        g = _lib.ConvGeom(2, 4, extent, extent, 4, size, size, 1, pad)
+        for pass_ in (_lib.RH_CONV_FWD, _lib.RH_CONV_BWD_FILTER, _lib.RH_CONV_BWD_DATA):
+            assert _lib.lib().rh_conv2d_workspace_bytes(C.byref(g), pass_) < 1 << 20
+            assert _lib.lib().rh_conv2d_workspace_bytes_upto(C.byref(g), pass_) < 1 << 20
+            assert _lib.lib().rh_conv2d_winograd_flops(C.byref(g), pass_, 0) == 0
+
+
 def _c_prototypes(header):
     """name -> argument count of every function include/<header> declares."""
     text = open(os.path.join(ROOT, "include", header)).read()
