@@ -451,10 +451,18 @@ struct LdsConvPlan {
 };
 // N images of Ci channels, `rows` result channels of P x Q.
 LdsConvPlan plan_conv_lds(int N, int Ci, int rows, int P, int Q, int R, int S, int st);
-inline LdsConvPlan plan_lds_fwd(const ConvDims& d) { return plan_conv_lds(d.N, d.C, d.K, d.P, d.Q, d.R, d.S, d.st); }
+// (Loads of the channels that a last stage has too many, fifteen at most, are out of range by the top bit of their offset:
+// their planes have to lie below it too, or the offset would wrap into the first planes, whose infinities times the zero
+// filter are no zeros.)
+inline bool lds_fits(long long in_elems, int H, int W) { return (in_elems + 15ll * H * W) * 4 < (1ll << 31); }
+inline LdsConvPlan plan_lds_fwd(const ConvDims& d) {
+  LdsConvPlan p = plan_conv_lds(d.N, d.C, d.K, d.P, d.Q, d.R, d.S, d.st);
+  p.ok = p.ok && lds_fits(d.x_elems, d.H, d.W);
+  return p;
+}
 inline LdsConvPlan plan_lds_bwd_data(const ConvDims& d) {   // (halo R - 1 - pad)
   LdsConvPlan p = plan_conv_lds(d.N, d.K, d.C, d.H, d.W, d.R, d.S, d.st);
-  p.ok = p.ok && d.pad <= d.R - 1;
+  p.ok = p.ok && d.pad <= d.R - 1 && lds_fits(d.y_elems, d.P, d.Q);
   return p;
 }
 // What the engine's forward and backward-data forms take on a stride-1 layer of `rows` result channels and `cols` pixels, in
