@@ -287,9 +287,16 @@ typedef Tile<32, 64, 2, 1, 2> L32x64;    // two waves a column block
 typedef Tile<32, 32, 2, 1, 1> L32x32;    // four
 
 // mfmas: MFMAs of a wave per tap and stage.  held3, held5: blocks whose registers fit a CU, 3x3 and 5x5 filters.
-struct LdsShape { int bm, bn, qc, mfmas, held3, held5; };
-static const LdsShape kLdsShapes[kLdsShapeCount] = {{64, 128, 1, 4, 3, 2}, {64, 64, 1, 2, 4, 3}, {32, 128, 1, 2, 5, 4},
-                                                    {32, 64, 2, 2, 4, 3}, {32, 32, 4, 2, 3, 2}, {32, 128, 2, 4, 3, 2}};
+// tag: of the launch records, forward and backward-data.
+struct LdsShape { int bm, bn, qc, mfmas, held3, held5; const char* tag[2]; };
+static const LdsShape kLdsShapes[kLdsShapeCount] = {
+    {64, 128, 1, 4, 3, 2, {"conv_fwd_lds_64x128", "conv_bwd_data_lds_64x128"}},
+    {64, 64, 1, 2, 4, 3, {"conv_fwd_lds_64x64", "conv_bwd_data_lds_64x64"}},
+    {32, 128, 1, 2, 5, 4, {"conv_fwd_lds_32x128", "conv_bwd_data_lds_32x128"}},
+    {32, 64, 2, 2, 4, 3, {"conv_fwd_lds_32x64", "conv_bwd_data_lds_32x64"}},
+    {32, 32, 4, 2, 3, 2, {"conv_fwd_lds_32x32", "conv_bwd_data_lds_32x32"}},
+    {32, 128, 2, 4, 3, 2, {"conv_fwd_lds_32x128_q2", "conv_bwd_data_lds_32x128_q2"}},
+};
 
 // Staged positions per channel that any tile of `bn` consecutive output pixels can need.
 static int lds_positions(int P, int Q, int R, int bn) {
@@ -421,7 +428,7 @@ int launch_conv_lds(const LdsConvPlan& pl, bool bwd, int N, int Ci, int H, int W
     kep.out = static_cast<float*>(ws); kep.split_stride = total; kep.bias = nullptr; kep.relu = 0; kep.mask = nullptr;
   }
   {
-    ProfScope prof(bwd ? "conv_bwd_data_lds" : "conv_fwd_lds", flops, stream);
+    ProfScope prof(kLdsShapes[pl.shape].tag[bwd], flops, stream);
     if (int e = R == 3 ? launch_lds_R<3>(pl.shape, p, kep, pl.splits, stream) : launch_lds_R<5>(pl.shape, p, kep, pl.splits, stream))
       return e;
   }

@@ -8,7 +8,7 @@ import torch
 import oracle as O
 from rembrandt_amd import _lib, ops, synth
 from conftest import assert_close, say
-from test_gpu_step_graph import profile_tags
+from test_gpu_step_graph import profile_records, profile_tags
 
 pytestmark = pytest.mark.gpu
 
@@ -152,23 +152,56 @@ def test_conv2d_all_passes(dev, case, algo):
     torch.cuda.synchronize()
 
 
-# Stride-1 layers with both operands staged in LDS: for each tile shape and filter extent, whole and in slices of the
-# channels, sizes with remainders everywhere (rows, pixels, channels; tiles that span images), the smallest there is, and
-# a 5x5 layer without padding
+# Stride-1 layers with both operands staged in LDS: each tile shape (rows x pixels, "_q2": two channel quads a stage) that
+# either filter extent is chosen with, whole and in slices of the channels where both are, sizes with remainders everywhere
+# (rows, pixels, channels; tiles that span images), the smallest there is, a 5x5 layer without padding, and as many slices
+# as there are.  With each case the shape and the slices of its forward pass and of its data gradient.
 STAGED_CASES = [
     # N, C, H, W, K, R, pad
-    (1, 1, 1, 1, 1, 3, 1), (2, 5, 9, 7, 21, 5, 0), (3, 2, 4, 30, 33, 3, 2),
-    (16, 3, 56, 56, 33, 3, 1), (11, 66, 31, 32, 33, 3, 1), (25, 3, 28, 28, 130, 5, 2), (22, 33, 27, 28, 33, 5, 2),   # 64 x 128
-    (5, 3, 40, 41, 33, 5, 2), (19, 20, 13, 13, 33, 5, 2), (1, 132, 13, 13, 65, 3, 1),                               # 64 x 64
-    (1, 3, 5, 5, 20, 3, 1), (1, 20, 5, 6, 20, 5, 2), (20, 12, 27, 29, 96, 5, 2),                                     # 32 x 128
-    (1, 8, 5, 6, 20, 3, 1), (1, 33, 5, 5, 33, 5, 2), (9, 40, 20, 20, 70, 3, 1),                                      # 32 x 64
-    (1, 66, 5, 5, 20, 3, 1), (1, 13, 5, 5, 20, 5, 2), (32, 32, 16, 16, 32, 5, 2),                                    # 32 x 32
-    (27, 8, 17, 18, 33, 5, 2), (2, 33, 28, 29, 33, 5, 2),                                                            # 32 x 128, two quads
+    ((1, 1, 1, 1, 1, 3, 1), ("32x32", 1), ("32x32", 1)),
+    ((2, 5, 9, 7, 21, 5, 0), ("32x64", 1), ("32x128", 6)),
+    ((3, 2, 4, 30, 33, 3, 2), ("32x128", 1), ("32x64", 5)),
+    ((16, 3, 56, 56, 33, 3, 1), ("64x128", 1), ("32x128", 1)),
+    ((11, 66, 31, 32, 33, 3, 1), ("64x128", 5), ("32x128", 1)),
+    ((25, 3, 28, 28, 130, 5, 2), ("64x128", 1), ("32x128", 3)),
+    ((22, 33, 27, 28, 33, 5, 2), ("64x128", 3), ("64x128", 3)),
+    ((5, 3, 40, 41, 33, 5, 2), ("64x64", 1), ("32x64", 1)),
+    ((19, 20, 13, 13, 33, 5, 2), ("64x64", 5), ("32x64", 5)),
+    ((1, 132, 13, 13, 65, 3, 1), ("32x32", 5), ("32x32", 5)),
+    ((1, 3, 5, 5, 20, 3, 1), ("32x128", 1), ("32x128", 5)),
+    ((1, 20, 5, 6, 20, 5, 2), ("32x128", 5), ("32x128", 5)),
+    ((20, 12, 27, 29, 96, 5, 2), ("32x128", 1), ("32x128", 4)),
+    ((1, 8, 5, 6, 20, 3, 1), ("32x64", 1), ("32x128", 5)),
+    ((1, 33, 5, 5, 33, 5, 2), ("32x64", 5), ("32x64", 5)),
+    ((9, 40, 20, 20, 70, 3, 1), ("32x64", 1), ("32x128", 6)),
+    ((1, 66, 5, 5, 20, 3, 1), ("32x32", 5), ("32x128", 5)),
+    ((1, 13, 5, 5, 20, 5, 2), ("32x32", 1), ("32x128", 5)),
+    ((32, 32, 16, 16, 32, 5, 2), ("32x32", 1), ("32x32", 1)),
+    ((27, 8, 17, 18, 33, 5, 2), ("32x128_q2", 1), ("32x128", 3)),
+    ((2, 33, 28, 29, 33, 5, 2), ("32x128_q2", 5), ("32x128_q2", 5)),
+    ((1, 20, 5, 5, 20, 3, 1), ("32x128", 5), ("32x128", 5)),
+    ((1, 256, 13, 13, 384, 3, 1), ("32x128", 16), ("32x128", 32)),
+    ((1, 33, 5, 5, 20, 3, 1), ("32x64", 5), ("32x128", 5)),
+    ((1, 512, 7, 7, 512, 3, 1), ("32x64", 32), ("32x64", 32)),
+    ((24, 66, 15, 15, 33, 3, 1), ("64x64", 6), ("32x64", 1)),
+    ((1, 384, 13, 13, 384, 3, 1), ("64x64", 24), ("64x64", 24)),
+    ((24, 8, 37, 37, 130, 3, 1), ("32x128_q2", 1), ("32x128", 3)),
+    ((24, 130, 37, 37, 32, 3, 1), ("32x128", 3), ("32x128_q2", 1)),
+    ((1, 70, 5, 5, 20, 5, 2), ("32x32", 5), ("32x128", 5)),
+    ((1, 9, 7, 9, 96, 5, 2), ("32x32", 1), ("32x128", 24)),
 ]
 
 
-@pytest.mark.parametrize("case", STAGED_CASES, ids=str)
-def test_conv2d_staged_operands(dev, case):
+def staged_forms(records, pass_, elems):
+    """Shapes and slices of the staged convolutions among launch records, one result of `elems` values each: the slices from
+    the bytes that the reduction behind a sliced one moves, 4 (slices + 1) a value."""
+    at = [i for i, (tag, _) in enumerate(records) if tag.startswith("conv_%s_lds_" % pass_)]
+    return [(records[i][0][len("conv_%s_lds_" % pass_):],
+             int(records[i + 1][1] / 4.0 / elems) - 1 if records[i + 1:] and records[i + 1][0] == "split_reduce" else 1) for i in at]
+
+
+@pytest.mark.parametrize("case,fwd,bwd", STAGED_CASES, ids=lambda v: str(v) if len(v) > 2 else "%s/%d" % v)
+def test_conv2d_staged_operands(dev, case, fwd, bwd):
     """Forward and backward-data against the oracle at the edges of the staged form's tiles, with its epilogues."""
     Nn, C, H, W, K, R, pad = case
     say("staged case", case)
@@ -177,8 +210,8 @@ def test_conv2d_staged_operands(dev, case):
     dy = synth.normal(17, 4, y_ref.shape)
     y0, dx0 = synth.normal(17, 5, y_ref.shape), synth.normal(17, 6, x.shape)
     xd, wd, bd, dyd = T(x, dev), T(w, dev), T(b, dev), T(dy, dev)
-    (y, dx), tags = profile_tags(lambda: (ops.conv2d_fwd(xd, wd, 1, pad), ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad)))
-    assert "conv_fwd_lds" in tags, tags   # (the data gradient of a few channels may keep the engine)
+    (y, dx), records = profile_records(lambda: (ops.conv2d_fwd(xd, wd, 1, pad), ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad)))
+    assert staged_forms(records, "fwd", y.numel()) == [fwd] and staged_forms(records, "bwd_data", dx.numel()) == [bwd], records
     assert_close(N(y), y_ref, "staged fwd")
     assert_close(N(dx), O.conv2d_bwd_data(w, dy, x.shape, 1, pad), "staged bwd data")
     yf = ops.conv2d_fwd(xd, wd, 1, pad, bias=bd, relu=True)

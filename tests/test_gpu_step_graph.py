@@ -234,8 +234,8 @@ def test_classifier_tail_in_two_launches(dev, name, batch, steps):
             assert_close(u, v, "%s step %d buffer %d" % (name, step, k))
 
 
-def profile_tags(fn):
-    """Runs fn() with the library's per-launch records on; returns (fn's result, list of the tags launched)."""
+def profile_records(fn):
+    """Runs fn() with the library's per-launch records on; returns (fn's result, list of (tag, work) of the launches)."""
     import ctypes as C
     from rembrandt_amd import _lib
     lib = _lib.lib()
@@ -243,14 +243,20 @@ def profile_tags(fn):
     try:
         res = fn()
         tag, work, ms = C.c_char_p(), C.c_double(), C.c_float()
-        tags = []
+        records = []
         for i in range(lib.rh_profile_count()):
             lib.rh_profile_get(i, C.byref(tag), C.byref(work), C.byref(ms))
-            tags.append(tag.value.decode())
+            records.append((tag.value.decode(), work.value))
     finally:
         lib.rh_profile_enable(0)
         lib.rh_profile_reset()
-    return res, tags
+    return res, records
+
+
+def profile_tags(fn):
+    """Runs fn(); returns (fn's result, list of the tags launched)."""
+    res, records = profile_records(fn)
+    return res, [tag for tag, _ in records]
 
 
 WINO_DIMS = (16, 16, 8)
