@@ -276,8 +276,8 @@ WINO_CASES = [
     (70, 384, 13, 13, 64, 1),     # the same in the data gradient
     (16, 128, 28, 28, 64, 1),
     (90, 64, 13, 13, 128, 1),     # 4410 tiles: the filter gradient in the form too, its tiles in several slices
-    (1, 260, 7, 9, 130, 1),       # two blocks in sixteen slices of five stages (the last one of none)
-    (5, 132, 12, 14, 64, 1),      # seven blocks, half of their rows past the last filter, in eight slices
+    (1, 260, 7, 9, 130, 1),       # three blocks of 64 rows in thirteen slices of five stages
+    (5, 132, 12, 14, 64, 1),      # seven blocks of 64 rows in nine slices of four stages (the last one of one)
     (24, 252, 13, 13, 244, 1),    # 74 blocks in three slices (21, 21, 20 stages of 63) of two chains
 ]
 
@@ -373,7 +373,8 @@ def test_conv2d_winograd_error_on_small_grids(dev, case):
                                   (9, 64, 56, 56, 64, 1), (24, 64, 56, 55, 64, 1)], ids=str)
 def test_conv2d_winograd_64_rows(dev, case):
     """The 64-row tiles of up to 64, 192, ... filters: channel loops of one to seven stages (every way the pipeline starts
-    and drains) and of sixteen, ragged rows and tiles, borders of 0, 1, 2, blocks in slices (9 images) and whole rounds;
+    and drains) and of sixteen, ragged rows and tiles, borders of 0, 1, 2, blocks under one round in slices (14 x 14) and
+    whole (9 images), and a whole round with a sliced last one (24);
     forward with the fused epilogue, the data gradient masked and blended; the library's own choice."""
     Nn, C, H, W, K, pad = case
     say("winograd 64-row case", case)
@@ -406,9 +407,9 @@ WINO5_CASES = [
     (2, 8, 7, 6, 20, 4),
     (2, 16, 12, 13, 64, 3),
     (4, 32, 27, 27, 96, 2),
-    (40, 32, 27, 27, 256, 2),      # 504 blocks: whole rounds and sliced tail blocks
+    (40, 32, 27, 27, 256, 2),      # 490 blocks: a whole round and an unsliced last one
     (70, 96, 13, 14, 128, 2),
-    (44, 64, 27, 27, 128, 2),      # 539 blocks: the library takes this form by itself
+    (44, 64, 27, 27, 128, 2),      # 270 blocks: a whole round and 14 blocks in sixteen slices
 ]
 
 
@@ -442,14 +443,43 @@ def test_conv2d_winograd_5x5_forward(dev, case):
     for fn in (lambda: ops.conv2d_bwd_data(wd, dy, x.shape, 1, pad, algo=WG), lambda: ops.conv2d_bwd_filter(xd, dy, w.shape, 1, pad, algo=WG)):
         with pytest.raises(_lib.RembrandtHipError):
             fn()
-    # the library's choice: this form for full row tiles and several rounds of blocks, else the direct one
+    # what the library picks by itself is what it says it picks (which that is: test_conv2d_winograd_by_itself)
     auto = ops.conv2d_fwd(xd, wd, 1, pad)
     direct = ops.conv2d_fwd(xd, wd, 1, pad, algo=_lib.RH_ALGO_DIRECT)
     assert_close(N(direct), y_ref, "RH_ALGO_DIRECT fwd (5x5)")
-    blocks = -(-K // 128) * -(-(Nn * -(-y_ref.shape[2] // 2) * -(-y_ref.shape[3] // 2)) // 32)
-    takes = C >= 64 and K >= 64 and 8 * K >= 7 * (-(-K // 128) * 128) and blocks >= 512
+    takes = ops.conv2d_winograd_flops(x.shape, w.shape, 1, pad) > 0
     assert torch.equal(auto, y if takes else direct), "library's choice (5x5)"
     torch.cuda.synchronize()
+
+
+@pytest.mark.parametrize("case,takes", [
+    ((16, 256, 13, 13, 384, 3, 1), True),    # 75 blocks in three slices, data gradient 50 blocks in five of two chains
+    ((5, 256, 13, 13, 384, 3, 1), False),    # too few images: the staged form
+    ((18, 64, 56, 56, 64, 3, 1), True),      # 441 blocks on 64 rows, under one round of them
+    ((13, 64, 56, 56, 64, 3, 1), False),     # 319 of them: two blocks on some CUs
+    ((70, 128, 13, 13, 128, 3, 1), True),    # 108 blocks on 128 rows
+    ((44, 256, 13, 13, 256, 3, 1), True),    # 136 blocks
+    ((29, 96, 27, 27, 256, 5, 2), True),     # 5x5: 356 blocks of two row tiles, one round and a sliced one
+    ((19, 96, 27, 27, 256, 5, 2), False),    # 234: under one round
+], ids=str)
+def test_conv2d_winograd_by_itself(dev, case, takes):
+    """Where the library takes the Winograd form without being asked, by the estimates of the forms: the calls under one round
+    of blocks and the 5x5 layers under two.  The same bits as with RH_ALGO_WINOGRAD, right against the oracle."""
+    Nn, C, H, W, K, R, pad = case
+    say("winograd by itself", case)
+    x, w = synth.normal(25, 1, (Nn, C, H, W)), synth.normal(25, 2, (K, C, R, R))
+    y_ref = O.conv2d_fwd(x, w, 1, pad)
+    dy = synth.normal(25, 3, y_ref.shape)
+    xd, wd, dyd = T(x, dev), T(w, dev), T(dy, dev)
+    for pass_, ref, run in (("fwd", y_ref, lambda algo: ops.conv2d_fwd(xd, wd, 1, pad, algo=algo)),
+                            ("bwd_data", None, lambda algo: ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=algo))):
+        if R == 5 and pass_ == "bwd_data":
+            continue
+        y, tags = profile_tags(lambda: run(0))
+        assert ("conv_%s_wino" % pass_ in tags) == takes, tags
+        if takes:
+            assert torch.equal(y, run(_lib.RH_ALGO_WINOGRAD)), pass_
+        assert_close(N(y), O.conv2d_bwd_data(w, dy, x.shape, 1, pad) if ref is None else ref, pass_)
 
 
 def test_conv2d_winograd_refused_geometries(dev):
