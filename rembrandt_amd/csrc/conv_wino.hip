@@ -924,8 +924,7 @@ __global__ __launch_bounds__(256, 2) void wino_gemm64_kernel(const float* __rest
       }
   }
   const uint32_t chan_stride = (uint32_t)HW * 4u;
-  const uint32_t tap_mul = im.blk5 ? chan_stride : 4u * chan_stride;
-  const uint32_t tap_add = im.blk5 ? (uint32_t)(3 * (wave >> 1) * im.Wi + 3 * (wave & 1)) * 4u : (uint32_t)wave * chan_stride;
+  const uint32_t tap_mul = 4u * chan_stride, tap_add = (uint32_t)wave * chan_stride;   // (never the 5x5 form, see wino_bm)
   auto issue_u = [&](int i, int cg, int buf) {
     dma_load16(rsU, lds0 + (uint32_t)buf * kWinoStage2 + (uint32_t)(wave * 4 + i) * 1024u, voffA,
                (uint32_t)(wave * 4 + i) * strideF + (uint32_t)(cg0 + cg) * strideA);
