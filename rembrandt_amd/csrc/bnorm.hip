@@ -240,8 +240,8 @@ struct BnUnits {
 
 // A channel's whole pass in one block: the values stay in registers between the sums and the result.  Small tensors are
 // bound by the dependent launches, not by bytes: 24 x 256 x 14 x 14 backward 12 + 6 + 10 us in three, 9 us in this one;
-// a ResNet-18 training step of 24 samples 4.52 -> 4.25 ms.  At the upper bound (256 x 512 x 7 x 7 forward, single
-// values) 41 -> 24 us.
+// a ResNet-18 training step of 24 samples 4.52 -> 4.25 ms.  256 x 512 x 7 x 7 forward (12544 single values
+// a channel; the most are 20480) 41 -> 24 us.
 // T = float4 (plane % 4 == 0 and 16-byte aligned tensors, so a unit never crosses a plane) or float.
 template <class T, bool BWD, bool RELU, bool MASK, int THREADS, int U, class Stats>
 __global__ __launch_bounds__(THREADS) void bn_channel_kernel(const T* x, const T* dy, const T* old, T* out, Stats stats, BnUnits un,

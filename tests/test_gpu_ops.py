@@ -1228,7 +1228,7 @@ def test_bnorm(dev, shape):
                                    (512, 3, 1, 3), (29, 3, 1, 53), (2048, 3, 1, 3), (5, 2, 1, 1229), (4096, 2, 1, 5), (2, 2, 1, 10241)])
 def test_bnorm_at_the_bounds_of_its_forms(dev, shape):
     """Values per channel at and just past what each block size of the one-launch form holds (2048 / 8192 / 20480 in
-    16-byte units, 1536 / 6144 / 20480 single), where the last is the bound to the two-launch form; results written over
+    16-byte units, 1536 / 6144 / 20480 single), where the last is the bound to the form of three launches; results written over
     their own input are those written elsewhere."""
     test_bnorm(dev, shape)
     C = shape[1]
