@@ -540,9 +540,12 @@ constexpr Bf16Form kBf16Forms[] = {
     {64, 128, 4, 1, 5.6, 0.177, 0.222, 0.149},
 };
 // Index into kBf16Forms with the least expected time (constants fitted to 72 launches, 9 layers at batches 1 to 128: 2 %
-// off the fastest form on average, 12 % at most).  64-row tiles fill twice the bytes per multiply-add: they are taken
-// where they save a fifth, since another stream's launches share the L2 (two AlexNet passes of 37 images side by side),
-// or where there are no more rows.  Contractions of up to 256 are not cut: there the streaming 1x1 kernel gives the same bits.
+// off the fastest form on average, 12 % at most).  64-row tiles fill twice the bytes per multiply-add, and passes of other
+// streams share the L2: beside those their K steps count 1.4 times, where there are rows for the larger tiles.  (Whole
+// passes of several workers side by side, AlexNet's and NIN's layers at 30 batches from 1 to 128: without the factor AlexNet
+// at 28 and 45 images 174 and 223 us against 166 and 217, NIN at 32 149 against 143; with 1.25 on the whole launch the
+// 384-channel 1x1 layers kept 128 x 128 tiles, 4 to 6 % of a NIN pass of 12 to 18 images, and AlexNet at 37 took 202 us
+// against 197.)  Contractions of up to 256 are not cut: there the streaming 1x1 kernel gives the same bits.
 static int bf16_small_form(int rows, long long cols, int n_k) {
   const int steps = n_k / 32;
   int best = 0;
@@ -556,9 +559,10 @@ static int bf16_small_form(int rows, long long cols, int n_k) {
       const double x = blocks / 256.0;
       return x <= 1.0 ? f.lone + (f.full - f.lone) * x : f.full + (x - 1.0) * f.next;
     };
-    double us = f.base + (double)(tiles / slots) * (steps * step_us((double)slots) + 1.5) +
+    double us = (double)(tiles / slots) * (steps * step_us((double)slots) + 1.5) +
                 (tiles % slots ? steps * step_us((double)(tiles % slots)) : 0.0);
-    if (f.bm == 64 && rows > 64) us *= 1.25;
+    if (f.bm == 64 && rows > 64) us *= 1.4;
+    us += f.base;
     if (i == 0 || us < best_us) { best = i; best_us = us; }
   }
   return best;
@@ -582,8 +586,9 @@ static int bf16_gemm(const ConvDims& d, const Bf16FwdPlan& bpn, const void* xb, 
   if (pk.ptr && bpn.s_groups == 0 && (conv1x1_bf16_stream_applies(d) || (force_stream && conv1x1_bf16_stream_runs(d))))
     return launch_conv1x1_bf16_stream(d, xb, static_cast<const char*>(wprep) + bpn.tab_bytes, ep.bias, ep.relu, pk, stream);
   // Grids of up to one 128 x 128 tile per CU and short contractions take bf16_small_form's choice.  (Up to 1024 tiles its
-  // forms are as fast or faster alone, NIN's 1024-channel 3x3 layer at batch 128, 288 tiles: 56 -> 48 us; but with passes
-  // of several workers side by side the larger tiles' smaller fill wins, NIN 421 us a pass against 429.)  Above, filter
+  // forms are as fast or faster alone, NIN's 1024-channel 3x3 layer at batch 128, 288 tiles: 56 -> 48 us, whole passes 0 to
+  // 4 %; but with passes of several workers side by side the larger tiles' smaller fill wins: AlexNet at 64, 100 and 128
+  // images 270, 409 and 489 us a pass against 276, 419 and 502, NIN at 40, 64 and 100 1 %.)  Above, filter
   // counts that waste no more rows in 256-row tiles than in 128-row ones take
   //  - 256 x 256 (one block of eight waves per CU, ring of four) for long contractions on grids of two rounds of
   //    the 256 CUs and more: 1.19 PFLOP/s on 256 x 96 x 27 x 27 -> 256, 5x5 (729 tiles);

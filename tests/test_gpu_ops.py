@@ -601,14 +601,17 @@ def test_conv2d_fwd_bf16_packed_chain_forms(dev, case):
     torch.cuda.synchronize()
 
 
-@pytest.mark.parametrize("case", [(1, 48, 13, 13, 72, 5, 1, 2, 1), (1, 136, 13, 13, 72, 3, 1, 1, 0), (16, 72, 13, 13, 136, 3, 1, 1, 1),
-                                  (37, 72, 13, 13, 384, 3, 1, 1, 1), (40, 40, 13, 13, 264, 3, 1, 1, 0), (1, 1024, 6, 6, 1000, 1, 1, 0, 0)],
-                         ids=lambda c: str(c))
-def test_conv2d_fwd_bf16_small_grids(dev, case):
+@pytest.mark.parametrize("case,form", [
+    ((1, 48, 13, 13, 72, 5, 1, 2, 1), "64x64_k4"), ((1, 136, 13, 13, 72, 3, 1, 1, 0), "64x64_k4"),
+    ((16, 72, 13, 13, 136, 3, 1, 1, 1), "64x64_k2"), ((37, 72, 13, 13, 384, 3, 1, 1, 1), "128x128_k2"),
+    ((40, 40, 13, 13, 264, 3, 1, 1, 0), "128x128"), ((1, 1024, 6, 6, 1000, 1, 1, 0, 0), "64x64_k4"),
+    ((16, 384, 13, 13, 384, 1, 1, 0, 0), "64x64_k2"), ((28, 128, 13, 13, 384, 3, 1, 1, 1), "128x128_k2"),
+    ((16, 16, 13, 13, 48, 3, 1, 1, 1), "64x128")], ids=str)
+def test_conv2d_fwd_bf16_small_grids(dev, case, form):
     """The forms for grids of few tiles: 64 x 64 with four groups of waves over the K steps (38 steps: 9, 10, 9, 10; 40),
-    64 x 64 with two, 128 x 128 with two and with one; ragged rows and columns; fp32 and packed results."""
-    test_conv2d_fwd_bf16_packed_chain_forms(dev, case)
-    test_conv2d_fwd_bf16_operands(dev, case[:8])
+    64 x 64 with two, 128 x 128 with two and with one, 64 x 128; ragged rows and columns; fp32 and packed results."""
+    _, tags = profile_tags(lambda: (test_conv2d_fwd_bf16_packed_chain_forms(dev, case), test_conv2d_fwd_bf16_operands(dev, case[:8])))
+    assert {t for t in tags if t.startswith("conv_fwd_bf16p_")} == {"conv_fwd_bf16p_" + form}, tags
 
 
 BF16_POOL_CASES = [
