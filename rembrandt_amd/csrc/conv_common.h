@@ -392,12 +392,19 @@ struct WinoGeom {
 inline int wino_bm(int Ci, int Ko, int blk5) {
   return Ci % 4 == 0 && !blk5 && round_up(Ko, kWinoBM2) * 9 <= round_up(Ko, kWinoBM) * 8 ? kWinoBM2 : kWinoBM;
 }
-// Stages in a chain of which the form's error against 64 bits is the direct form's at `splits` slices.  Its relative rms
-// error, squared, is 1.35 + 0.351 L in units of 1e-14 (L stages of four channels in a chain: 2.6e-7 at 16, 3.5e-7 at 32,
-// 5.9e-7 at 96), the direct form's 0.030 a term (2.8e-7 at 256, 4.2e-7 at 576).  A direct form that is not sliced has the
-// longer chain at any size.
-inline int wino_stages_at_most(int Ci, int splits) {
-  return splits <= 1 ? cdiv(Ci, 4) : (int)((0.030 * 9.0 * Ci / splits - 1.35) / 0.351);
+// Stages in a chain of which the form's error against 64 bits is the direct form's at `splits` slices, for a result of
+// P x Q with `halo` zeros around the input.  The form's relative rms error, squared, is 1.35 + 0.351 L in units of 1e-14 (L
+// stages of four channels in a chain: 2.6e-7 at 16, 3.5e-7 at 32, 5.9e-7 at 96), the direct form's 0.0335 a term that lies on
+// the image (2.8e-7 at 256, 4.2e-7 at 576 on 13 x 13).  A direct form that is not sliced has the longer chain at any size.
+// Terms on the border add nothing to the result nor to the direct form's error, but the transforms mix them in: with even
+// extents, whose tiles end with the result, 0.173 + 0.176 over the share of live terms a stage (0.354 on 28 x 28, 0.392 on
+// 6 x 6).  (Without that share 384 -> 1024 6x6 batch 40 took one chain of 48 stages, 4.50e-7 against 4.34e-7 in the direct
+// form's five slices; in two chains 3.3e-7, for 2 % of its time.)
+inline int wino_stages_at_most(int Ci, int splits, int P, int Q, int halo) {
+  if (splits <= 1 || P <= 0 || Q <= 0) return cdiv(Ci, 4);
+  const double dead = halo * (halo + 1) / 3.0, live = (1.0 - dead / P) * (1.0 - dead / Q);
+  const double stage = P % 2 == 0 || Q % 2 == 0 ? 0.173 + 0.176 / fmax(live, 0.1) : 0.351;
+  return (int)((0.0335 * live * 9.0 * Ci / splits - 1.35) / stage);
 }
 // max_L: the stages in a chain up to which a call counts as fine; it is made of such chains where that can be.
 WinoGeom wino_geom(int N, int Ci, int Hi, int Wi, int Ko, int halo, int max_L, int blk5 = 0);
@@ -408,10 +415,10 @@ inline WinoGeom wino_geom_fwd5(const ConvDims& d) {
   return wino_geom(d.N, d.C, d.H, d.W, d.K, d.pad, soff_splits_fwd(d, round_up(d.C * 25, kTabPad)) <= 1 ? 4 * d.C : 0, 1);
 }
 inline WinoGeom wino_geom_fwd(const ConvDims& d) {
-  return wino_geom(d.N, d.C, d.H, d.W, d.K, d.pad, wino_stages_at_most(d.C, soff_splits_fwd(d, round_up(d.C * 9, kTabPad))));
+  return wino_geom(d.N, d.C, d.H, d.W, d.K, d.pad, wino_stages_at_most(d.C, soff_splits_fwd(d, round_up(d.C * 9, kTabPad)), d.P, d.Q, d.pad));
 }
 inline WinoGeom wino_geom_bwd_data(const ConvDims& d) {
-  return wino_geom(d.N, d.K, d.P, d.Q, d.C, 2 - d.pad, wino_stages_at_most(d.K, soff_splits_bwd_data(d, round_up(d.K * 9, kTabPad))));
+  return wino_geom(d.N, d.K, d.P, d.Q, d.C, 2 - d.pad, wino_stages_at_most(d.K, soff_splits_bwd_data(d, round_up(d.K * 9, kTabPad)), d.H, d.W, 2 - d.pad));
 }
 // Filter gradient in the same form: zero-bordered copies of x and dy, S slices of the tiles, their partial sums.
 struct WinoFilterPlan {
