@@ -532,7 +532,7 @@ inline DirectForms direct_bwd_data(const ConvDims& d) {
 
 // Where the library takes the Winograd form by itself: enough channels on both sides for the 16 products to be worth their
 // transforms, and either a grid that fills the GPU, or a call expected to take less time than the direct form's: from 8 to
-// 18 images on for 128 channels and more (256 -> 384, 13 x 13: 8, 256 -> 256, 14 x 14: 11, 384 -> 1024, 6 x 6: 18).  Rounds
+// 22 images on for 128 channels and more (256 -> 384, 13 x 13: 8, 256 -> 256, 14 x 14: 11, 384 -> 1024, 6 x 6: 22).  Rounds
 // of blocks make either form the shorter one again for a batch or two (512 -> 512, 7 x 7: 16, 21 to 24, from 27 on).
 // A plain comparison of the estimates: against the best of the forms, on the timings above, 0.3 % slower on average;
 // asking an eighth of the Winograd form 1.6 % (and ResNet-18 on 9 images takes 436 us with it plain, 442 with the eighth).
