@@ -475,7 +475,9 @@ inline LdsConvPlan plan_lds_bwd_data(const ConvDims& d) {   // (halo R - 1 - pad
 // What the engine's forward and backward-data forms take on a stride-1 layer of `rows` result channels and `cols` pixels, in
 // microseconds: the copies in front (none in the gather form), rounds of the blocks a CU holds at a time, each K step of a
 // block taking its share of the matrix pipes or, with few blocks, its MFMAs and 0.43 us of waiting, and the reduction of
-// the slices.  A fit to 1582 timings of 792 layers (14 of the benchmark networks at 28 batches, 400 of random sizes; rms
+// the slices.  Where only the tiles past a multiple of 256 are sliced, the others' whole chains are the shortest a call can
+// be: 1.0 to 1.8 tiles a CU took 15 to 19 % longer than their share of the matrix pipes (212 timings of 60 layers, rms error
+// 15 %, 7 % with the chain), and the staged form 6 to 45 % less than they (16 images of 96 -> 256 5x5 27x27 152 us, 123).  A fit to 1582 timings of 792 layers (14 of the benchmark networks at 28 batches, 400 of random sizes; rms
 // error 11 %; by FLOPs alone it is 32 % and too short by a third where tiles are mostly empty).
 inline double engine_us(const SoffPlan& p, int rows, long long cols, size_t w_elems, bool gather) {
   if (!p.ok) return 1e30;
@@ -490,7 +492,7 @@ inline double engine_us(const SoffPlan& p, int rows, long long cols, size_t w_el
   const long long tiles = (long long)cdiv(rows, bm) * cdiv<long long>(cols, bn), held = bm >= 96 || k8 ? 4 : 3;
   double us;
   if (splits == 1 && !gather && p.tail.splits > 1) {
-    us = steps * busy_us * (double)tiles / 256.0;
+    us = steps * fmax(busy_us * (double)tiles / 256.0, step_us + 0.43);
   } else {
     const long long per_cu = cdiv<long long>(tiles * splits, 256), rem = per_cu % held;
     auto round_us = [&](long long k) { return steps / splits * fmax((double)k * busy_us, step_us + 0.43); };

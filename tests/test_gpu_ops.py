@@ -257,6 +257,17 @@ def test_conv2d_few_channels_on_many_pixels_keep_the_engine(dev, case):
     assert not any(t.startswith("conv_fwd_lds") for t in tags), tags
 
 
+@pytest.mark.parametrize("case", [(16, 96, 27, 27, 256, 5, 2), (48, 48, 17, 17, 160, 3, 1), (21, 320, 33, 33, 100, 3, 1), (56, 130, 17, 17, 96, 3, 1)], ids=str)
+def test_conv2d_one_tile_and_a_little_per_cu_is_staged(dev, case):
+    """The engine slices only the tiles past a multiple of 256, and a whole tile's chain of K steps is the shortest that such a
+    call can be: 1.0 to 1.8 tiles a CU take the staged form (123 us against 152, 30 against 39, 170 against 191)."""
+    Nn, C, H, W, K, R, pad = case
+    x, w = synth.normal(29, 1, (Nn, C, H, W)), synth.normal(29, 2, (K, C, R, R))
+    y, tags = profile_tags(lambda: ops.conv2d_fwd(T(x, dev), T(w, dev), 1, pad, algo=_lib.RH_ALGO_DIRECT))
+    assert any(t.startswith("conv_fwd_lds") for t in tags), tags
+    assert_close(N(y), O.conv2d_fwd(x, w, 1, pad), "staged fwd")
+
+
 # 3x3 stride-1 layers in the Winograd F(2x2, 3x3) form: odd and even extents (tiles that hang over the edge), every
 # padding it takes, channel counts that do not fill a group of four, filter counts around the 128-row tile, tile counts
 # that are no multiple of the 32-tile block, more blocks than CUs, and the sizes the library takes the form for by itself
