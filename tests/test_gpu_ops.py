@@ -365,7 +365,7 @@ def test_conv2d_winograd(dev, case):
 
 
 @pytest.mark.parametrize("case", [(24, 128, 28, 28, 128, 1), (19, 384, 13, 13, 384, 1), (27, 512, 7, 7, 512, 1),
-                                  (40, 384, 6, 6, 1024, 1), (9, 128, 30, 30, 256, 0)], ids=str)
+                                  (40, 384, 6, 6, 1024, 1), (9, 128, 30, 30, 256, 0), (29, 256, 13, 13, 384, 1)], ids=str)
 def test_conv2d_winograd_error_on_small_grids(dev, case):
     """Where the direct form's tiles are few it cuts its contraction into slices, whose short chains of sums lose few bits:
     the Winograd form has no larger an error against 64 bits on such grids (two correct results' errors differ by
