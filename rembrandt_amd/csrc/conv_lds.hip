@@ -28,10 +28,10 @@
 // slice is the longest: 67.7 -> 72.4 us).
 //
 // Measured, one call (with whatever it launches) against the same call on the engine, fp32, stride 1:
-//   20 -> 50, 5x5, 14x14, batch 64: 14.2 us (28.4);  32 -> 32, 5x5, 16x16, batch 128: 21.4 (34.2);
-//   64 -> 64, 3x3, 56x56, batch 8: 29.4 us (60.9), batch 32: 93 (93), batch 128: 272 (270);
-//   384 -> 384, 3x3, 13x13, batch 1: 19.4 (29.5), batch 4: 33.8 (40.4); 96 -> 256, 5x5, 27x27, batch 16: 124 (153).
-// What bounds it once it fills the GPU: the MFMAs (47 us of the 93 on 64 channels, 56x56, batch 32, at the matrix peak), what
+//   20 -> 50, 5x5, 14x14, batch 64: 14.0 us (28.3);  32 -> 32, 5x5, 16x16, batch 128: 20.6 (34.2);
+//   64 -> 64, 3x3, 56x56, batch 8: 28.4 us (61.4), batch 32: 79 (93), batch 128: 274 (270);
+//   384 -> 384, 3x3, 13x13, batch 1: 19.4 (29.7), batch 4: 33.4 (39.4); 96 -> 256, 5x5, 27x27, batch 16: 123 (153).
+// What bounds it once it fills the GPU: the MFMAs (47 us of the 79 on 64 channels, 56x56, batch 32, at the matrix peak), what
 // barriers, prologues and epilogues leave idle between them, and a last round of blocks.
 #include <string.h>
 
