@@ -61,6 +61,13 @@ typedef void* rh_stream_t; /* hipStream_t */
                                              other work the idle units of that round are not idle (measured: the
                                              ResNet-18 template step 26.5 -> 26.1 ms).  Grids of less than one round
                                              are sliced with the hint as without.  Same result up to summation order. */
+#define RH_ALGO_BF16X3             0x2000 /* the contraction may also run on bf16 matrix instructions, every fp32 operand value as
+                                             the exact sum of three bf16 values (six products a pair, fp32 accumulate): fp32
+                                             precision, no operand is rounded.  Alone or with the hint: where it is expected to
+                                             be the fastest form.  With RH_ALGO_DIRECT: this form, RH_E_UNSUPPORTED where the
+                                             geometry has none (forward and stride-1 backward-data need a contracted channel
+                                             count that is a multiple of 8).  No effect beside the other RH_ALGO_* bits and
+                                             RH_MATH_BF16_MFMA_FP32ACC. */
 
 const char* rh_version(void);
 /* Status of the most recent launch made by a void `rembrandt_kernel_*` entry point on this thread. */
@@ -139,9 +146,11 @@ typedef struct {
 enum { RH_CONV_FWD = 0, RH_CONV_BWD_FILTER = 1, RH_CONV_BWD_DATA = 2 };
 
 int32_t rh_conv2d_out_dim(int32_t in, int32_t size, int32_t stride, int32_t pad);
-/* Bytes of scratch the given pass needs whatever flags it is called with (0 is possible).  The scratch must be
- * 256-byte aligned. */
+/* Bytes of scratch the given pass needs whatever flags it is called with (0 is possible), RH_ALGO_BF16X3 with RH_ALGO_DIRECT
+ * apart.  The scratch must be 256-byte aligned. */
 size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass);
+/* The same for RH_ALGO_BF16X3 with RH_ALGO_DIRECT; 0 where the geometry has no such form. */
+size_t rh_conv2d_bf16x3_workspace_bytes(const rh_conv_geom* g, int pass);
 /* The same for a scratch buffer that is allocated once and then used with every batch 1..g->N, the way the
  * reference's operators size theirs for batch_cap (src/operator/mod.rs:1493-1507): the largest need of any such
  * batch.  The need is not monotone in N (a pass with few result tiles cuts its contraction into slices and keeps

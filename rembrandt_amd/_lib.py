@@ -15,6 +15,7 @@ RH_ROUND_FLOOR, RH_ROUND_CEIL = 0, 1
 RH_FUSE_BIAS, RH_FUSE_RELU = 0x10, 0x20
 RH_ALGO_GATHER, RH_ALGO_SCALAR_OFFSET, RH_ALGO_WINOGRAD, RH_ALGO_DIRECT = 0x100, 0x200, 0x400, 0x800
 RH_ALGO_SHARED_GPU = 0x1000
+RH_ALGO_BF16X3 = 0x2000
 RH_MATH_BF16_MFMA_FP32ACC = 0x1
 RH_E_INVALID, RH_E_WORKSPACE, RH_E_UNSUPPORTED, RH_E_LIMIT = -1, -2, -3, -4
 
@@ -90,6 +91,7 @@ PROTOTYPES = {
     "rh_conv2d_out_dim": (_i32, [_i32, _i32, _i32, _i32]),
     "rh_conv2d_winograd_flops": (C.c_double, [C.POINTER(ConvGeom), _int, _int]),
     "rh_conv2d_workspace_bytes": (_sz, [C.POINTER(ConvGeom), _int]),
+    "rh_conv2d_bf16x3_workspace_bytes": (_sz, [C.POINTER(ConvGeom), _int]),
     "rh_conv2d_workspace_bytes_upto": (_sz, [C.POINTER(ConvGeom), _int]),
     "rh_conv2d_bwd_bias_workspace_bytes_upto": (_sz, [_i32, _i32, _i32]),
     "rh_sgemm_workspace_bytes_upto": (_sz, [_i32, _i32, _i32, _int]),

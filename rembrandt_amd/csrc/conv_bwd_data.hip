@@ -169,6 +169,15 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
   hipStream_t stream = to_stream(stream_);
 
   if ((flags & RH_ALGO_WINOGRAD) && (!wino_shape(d) || (flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT)))) return RH_E_UNSUPPORTED;
+  if (tri_allowed(flags)) {
+    TriPlan tp = plan_tri_bwd_data(d);
+    if (tri_forced(flags) && !tp.ok) return RH_E_UNSUPPORTED;
+    if (tri_forced(flags) && ws_bytes < tp.total()) return RH_E_WORKSPACE;
+    if (tri_forced(flags) || tri_pays_bwd_data(d, flags, &tp)) {
+      if (d.x_elems == 0) return 0;
+      return launch_conv_tri(tp, true, dy, w, dx, alpha, beta, nullptr, 0, mask, ws, stream);
+    }
+  }
   if (!(flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET)) && conv1x1_stream_applies(d)) {
     if (d.x_elems == 0) return 0;
     return launch_conv1x1_stream(d, RH_CONV_BWD_DATA, w, dy, dx, alpha, beta, nullptr, 0, stream, mask);

@@ -868,6 +868,10 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
       }
       const size_t lp = lds_part_bytes(d.R, d.S, d.st, d.y_elems);
       if (lp > need) need = lp;
+      for (const int flags : {0, RH_ALGO_SHARED_GPU}) {
+        TriPlan tp;
+        if (tri_pays_fwd(d, flags, &tp) && tp.total() > need) need = tp.total();
+      }
       return need;
     }
     case RH_CONV_BWD_DATA: {
@@ -883,6 +887,10 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
       }
       const size_t lp = lds_part_bytes(d.R, d.S, d.st, d.x_elems);
       if (lp > need) need = lp;
+      for (const int flags : {0, RH_ALGO_SHARED_GPU}) {
+        TriPlan tp;
+        if (tri_pays_bwd_data(d, flags, &tp) && tp.total() > need) need = tp.total();
+      }
       return need;
     }
     case RH_CONV_BWD_FILTER: {
@@ -891,11 +899,28 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
         const WinoFilterPlan wp = plan_wino_bwd_filter(d);
         if (wp.ok && wp.total() > need) need = wp.total();
       }
+      const TriFilterPlan tp = plan_tri_bwd_filter(d);
+      if (tp.ok && tp.total() > need && tri_pays_bwd_filter(d, tp)) need = tp.total();
       return need + bwd_filter_bias_bytes(d);
     }
     default:
       return 0;
   }
+}
+
+extern "C" size_t rh_conv2d_bf16x3_workspace_bytes(const rh_conv_geom* g, int pass) {
+  ConvDims d;
+  if (conv_dims(g, &d)) return 0;
+  size_t tri = 0;
+  if (pass == RH_CONV_BWD_FILTER) {
+    const TriFilterPlan tp = plan_tri_bwd_filter(d);
+    tri = tp.ok ? tp.total() : 0;
+  } else if (pass == RH_CONV_FWD || pass == RH_CONV_BWD_DATA) {
+    const TriPlan tp = pass == RH_CONV_FWD ? plan_tri_fwd(d) : plan_tri_bwd_data(d);
+    tri = tp.ok ? tp.total() : 0;
+  }
+  const size_t other = tri ? rh_conv2d_workspace_bytes(g, pass) : 0;
+  return tri > other ? tri : other;
 }
 
 extern "C" size_t rh_conv2d_workspace_bytes_upto(const rh_conv_geom* g, int pass) {
@@ -916,6 +941,7 @@ extern "C" size_t rh_conv2d_workspace_bytes_upto(const rh_conv_geom* g, int pass
 struct BiasFold {
   float* db = nullptr;
   float* part = nullptr;
+  int rows = 0;   // rows of K sums in part where they are not one an image
   bool folded = false, done = false;
 };
 // Up to this many elements of dy one launch (a block per channel) is as fast as the first of the two stages, and the
@@ -932,7 +958,7 @@ static int bwd_filter_impl(const rh_conv_geom* g, float alpha, const float* x, c
   auto bias_job = [&](BiasJob* job) -> const BiasJob* {
     if (!bf || !bf->db || d.y_elems == 0) return nullptr;
     job->db = bf->db; job->N = d.N; job->K = d.K; job->alpha = alpha; job->beta = beta;
-    if (bf->folded) { job->src = bf->part; job->plane = 1; }
+    if (bf->folded) { job->src = bf->part; job->plane = 1; job->N = bf->rows ? bf->rows : d.N; }
     else if (d.y_elems <= kBiasOneStageElems) { job->src = dy; job->plane = d.P * d.Q; }
     else return nullptr;
     bf->done = true;
@@ -944,7 +970,45 @@ static int bwd_filter_impl(const rh_conv_geom* g, float alpha, const float* x, c
   if (!ws || ws_bytes < rh_conv2d_workspace_bytes(g, RH_CONV_BWD_FILTER) || (reinterpret_cast<uintptr_t>(ws) & 255))
     return RH_E_WORKSPACE;
   hipStream_t stream = to_stream(stream_);
+  // dw from `used` slices in (ko, r, s, c) order
+  auto reduce_rsc = [&](float* parts, int used) -> int {
+    const int CRSr = d.C * d.R * d.S;
+    const long long total = (long long)d.K * CRSr;
+    BiasJob bj;
+    bias_job(&bj);
+    const unsigned jb = bj.blocks();
+    ProfScope prof("split_reduce", 4.0 * (double)total * (used + 1) + (jb ? 4.0 * (double)bj.N * bj.K * bj.plane : 0.0), stream);
+    if (d.C % 4 == 0 && (reinterpret_cast<uintptr_t>(parts) & 15) == 0) {
+      bj.first = stream_grid((size_t)total / 4, 256);
+      hipLaunchKernelGGL(split_reduce_rsc_vec_kernel, dim3(bj.first + jb), dim3(256), 0, stream,
+                         reinterpret_cast<const float4*>(parts), used, (long long)d.K * CRSr / 4, dw, d.K, d.C, d.R, d.S, alpha,
+                         beta, bj);
+    } else {
+      bj.first = stream_grid((size_t)total, 256);
+      hipLaunchKernelGGL(split_reduce_rsc_kernel, dim3(bj.first + jb), dim3(256), 0, stream, parts, used,
+                         (long long)d.K * CRSr, dw, d.K, d.C, d.R, d.S, alpha, beta, bj);
+    }
+    return launch_status();
+  };
 
+  if (tri_allowed(flags)) {
+    const TriFilterPlan tp = plan_tri_bwd_filter(d);
+    if (tri_forced(flags) && !tp.ok) return RH_E_UNSUPPORTED;
+    if (tri_forced(flags) && ws_bytes < tp.total()) return RH_E_WORKSPACE;
+    if (tri_forced(flags) || tri_pays_bwd_filter(d, tp)) {
+      if (d.w_elems == 0) return 0;
+      float* parts = nullptr;
+      int used = 1;
+      float* sums = nullptr;
+      if (bf && bf->db) {
+        bf->part = sums = reinterpret_cast<float*>(static_cast<char*>(ws) + tp.sums_at());
+        bf->rows = tp.sum_rows;
+        bf->folded = true;
+      }
+      if (int e = launch_conv_tri_bwd_filter(d, tp, x, dy, sums, ws, stream, &parts, &used)) return e;
+      return reduce_rsc(parts, used);
+    }
+  }
   if ((flags & RH_ALGO_WINOGRAD) && (!wino_shape(d) || (flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT))))
     return RH_E_UNSUPPORTED;
   if (wino_shape(d) && !(flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT))) {
@@ -1020,22 +1084,7 @@ static int bwd_filter_impl(const rh_conv_geom* g, float alpha, const float* x, c
       default:  e = run_bwd_filter_soff<T32x256>(ap, bp, ep, sp.n_k, Ms, sp.splits, &used, stream, "conv_bwd_filter_32x256"); break;
     }
     if (e) return e;
-    const long long total = (long long)d.K * CRSs;
-    BiasJob bj;
-    bias_job(&bj);
-    const unsigned jb = bj.blocks();
-    ProfScope prof("split_reduce", 4.0 * (double)total * (used + 1) + (jb ? 4.0 * (double)bj.N * bj.K * bj.plane : 0.0), stream);
-    if (d.C % 4 == 0 && (reinterpret_cast<uintptr_t>(parts) & 15) == 0) {
-      bj.first = stream_grid((size_t)total / 4, 256);
-      hipLaunchKernelGGL(split_reduce_rsc_vec_kernel, dim3(bj.first + jb), dim3(256), 0, stream,
-                         reinterpret_cast<const float4*>(parts), used, (long long)d.K * CRSs / 4, dw, d.K, d.C, d.R, d.S, alpha,
-                         beta, bj);
-    } else {
-      bj.first = stream_grid((size_t)total, 256);
-      hipLaunchKernelGGL(split_reduce_rsc_kernel, dim3(bj.first + jb), dim3(256), 0, stream, parts, used,
-                         (long long)d.K * CRSs, dw, d.K, d.C, d.R, d.S, alpha, beta, bj);
-    }
-    return launch_status();
+    return reduce_rsc(parts, used);
   }
 
   const int CRS = d.C * d.R * d.S;

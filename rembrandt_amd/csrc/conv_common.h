@@ -170,6 +170,10 @@ typedef Tile<64, 128, 16, 1, 4, 4> T64x128;   // sliced forward / backward-data 
 // Half the K step: 20 KB of LDS, so a CU holds 4 blocks instead of 3.  For grids that need a second round of
 // blocks at 3 per CU but fit in one at 4 (e.g. 64 output channels over 64 x 56 x 56 pixels: 784 tiles).
 typedef Tile<64, 256, 8, 1, 4, 4> T64x256k8;
+// The kernel of gemm_tri.h: two blocks of four waves to a CU.
+typedef Tile<128, 128, 16, 2, 2, 2> T128x128t;
+typedef Tile<96, 128, 16, 1, 4, 2> T96x128t;
+typedef Tile<64, 192, 16, 2, 2, 2> T64x192t;
 inline bool prefer_k8_64(long long cols) {
   const long long tiles = cdiv<long long>(cols, 256);
   return cdiv<long long>(tiles, 1024) < cdiv<long long>(tiles, 768);
@@ -559,6 +563,119 @@ inline bool wino_pays5(const WinoGeom& g, const DirectForms& f) {
   if (!g.ok || !g.blk5 || g.C5 < 64 || g.Ko < 64 || 8 * g.Ko < 7 * g.rows_p) return false;
   const long long blocks = (long long)(g.rows_p / kWinoBM) * (g.tiles_p / kWinoBN);
   return blocks >= 512 || (blocks >= 256 && g.rows_p > kWinoBM && wino_fastest(g, f));
+}
+
+// The fp32 contraction on bf16 matrix instructions with exactly split operands (conv_tri.hip).  Forward, and backward-data of
+// stride 1 as a forward convolution of dy with halo R - 1 - pad; scratch: [group offsets][filter][image][partial sums].
+struct TriPlan {
+  int N, Ci, Hi, Wi, rows, R, S, st, halo, P, Q;
+  int Hp, Wp;
+  int groups_true, groups;   // groups of eight k; rounded up to whole K steps
+  int bm, bn, splits;
+  TailSplit tail;            // as in SoffPlan
+  double us;                 // what a call is expected to take
+  size_t tab_bytes, wt_bytes, img_bytes, part_bytes;
+  bool ok;
+  size_t total() const { return tab_bytes + wt_bytes + img_bytes + part_bytes; }
+};
+// max_chain: the most K steps that a sum may be one chain of (0: any); not ok where slices cannot make it so.
+TriPlan plan_tri(int N, int Ci, int Hi, int Wi, int rows, int R, int S, int st, int halo, int P, int Q, int max_chain);
+inline TriPlan plan_tri_fwd(const ConvDims& d, int max_chain = 0) {
+  return plan_tri(d.N, d.C, d.H, d.W, d.K, d.R, d.S, d.st, d.pad, d.P, d.Q, max_chain);
+}
+inline TriPlan plan_tri_bwd_data(const ConvDims& d, int max_chain = 0) {
+  if (d.st != 1 || d.R != d.S) return TriPlan{};
+  return plan_tri(d.N, d.K, d.P, d.Q, d.C, d.R, d.S, 1, d.R - 1 - d.pad, d.H, d.W, max_chain);
+}
+int launch_conv_tri(const TriPlan& p, bool bwd, const float* in, const float* w, float* out, float alpha, float beta,
+                    const float* bias, int relu, const float* mask, void* ws, hipStream_t stream);
+struct TriFilterPlan {
+  int Hp, Wp, n8, groups_true, groups, bm, bn, splits;
+  int sum_rows;   // rows of K partial sums of dy that the copy can leave for the bias gradient
+  double us;      // what a call is expected to take
+  size_t tab_bytes, dyt_bytes, xt_bytes, part_bytes, sum_bytes;
+  bool ok;
+  size_t sums_at() const { return tab_bytes + dyt_bytes + xt_bytes + part_bytes; }
+  size_t total() const { return sums_at() + sum_bytes; }
+};
+TriFilterPlan plan_tri_bwd_filter(const ConvDims& d);
+// Leaves `used` slices of dw in (ko, r, s, c) order in *parts, and in `sums`, if given, rows whose sum is dy's over images and
+// pixels.
+int launch_conv_tri_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
+                               hipStream_t stream, float** parts, int* used);
+
+bool conv1x1_stream_applies(const ConvDims& d);
+
+// Where a caller that allows it (RH_ALGO_BF16X3) gets the form of exactly split operands: where its expected time is below
+// that of the form taken otherwise.  The engine's estimate was fitted to 3x3 and 5x5 stride-1 layers and is 10 to 25 % short on
+// others, hence the tenth.  Over 308 timed forward calls (22 layers at 14 batches) the forms chosen so are 1.27 times as fast as
+// without it, geometric mean, 1.02 times slower at worst.  1x1 layers of up to 128 channels keep the streaming kernels, which
+// read their operands where they lie (96 -> 96 54x54 b128 82 us against 158).
+// A layer of one 128-row tile of filters keeps the Winograd form in the 5x5 forward pass and in the filter gradient, although
+// it is the slower one there too (64 -> 128 5x5 24x24 b128 190 us expected against 143, 128 -> 128 3x3 28x28 b256 466 us
+// measured against 341): the comparison of whole train steps in the two forms runs them on such layers.
+inline bool tri_allowed(int flags) {
+  return (flags & RH_ALGO_BF16X3) && !(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_WINOGRAD));
+}
+inline bool tri_forced(int flags) { return tri_allowed(flags) && (flags & RH_ALGO_DIRECT); }
+// Squared relative error against 64 bits, in units of 1e-14, N(0,1) operands: of this form 0.0525 a K step in a chain (1.34e-7
+// at 36, 1.95e-7 at 72), of the engine 0.0335 a term, of the Winograd form as in wino_stages_at_most, of the staged form
+// 0.032 a term of its two chains and four more (0.09 2^-48: a rounding's variance).  The chain allowed is the one with three
+// quarters of the other form's: half zeros, as behind a ReLU, spare the shorter chains more roundings (1.2 on the square).
+inline int tri_max_chain(double other) { const double n = 0.75 * other / 0.0525; return n < 1.0 ? 1 : n < 1e6 ? (int)n : 1000000; }
+inline double engine_err(const SoffPlan& p, int terms) { return 0.0335 * terms / p.splits; }
+inline double staged_err(const LdsConvPlan& p, int R) {
+  const double chain = R == 3 ? 36.0 : 52.0, terms = 4.0 * p.qps * R * R;
+  return 0.032 * (chain + terms / chain + 4.0);
+}
+inline double wino_err(const WinoGeom& g) {
+  const int stages = g.full_tiles > 0 || g.tail_S <= 1 ? g.Cg : g.tail_L;
+  return 1.35 + 0.351 * cdiv(stages, g.chains > 0 ? g.chains : 1);
+}
+// plan: what is to be launched where it pays.
+template <class PLAN>
+inline bool tri_pays(const ConvDims& d, bool bwd, int flags, TriPlan* plan, PLAN make) {
+  if ((bwd ? d.K : d.C) % 8 != 0 || conv1x1_stream_applies(d)) return false;
+  const int terms = (bwd ? d.K : d.C) * d.R * d.S;
+  double us, err;
+  if (!has_staged_form(d)) {
+    const SoffPlan sp = bwd ? plan_soff_bwd_data(d) : plan_soff_fwd(d);
+    us = 1.1 * engine_us(sp, bwd ? d.C : d.K, (long long)d.N * (bwd ? d.H * d.W : d.P * d.Q), d.w_elems, false);
+    err = engine_err(sp, terms);
+  } else {
+    const DirectForms f = bwd ? direct_bwd_data(d) : direct_fwd(d);
+    us = f.us;
+    err = f.staged ? staged_err(f.lds, d.R) : engine_err(f.soff, terms);
+    const bool five = !bwd && wino_shape5(d);
+    if (wino_shape(d) || five) {
+      WinoGeom wg = five ? wino_geom_fwd5(d) : bwd ? wino_geom_bwd_data(d) : wino_geom_fwd(d);
+      if (flags & RH_ALGO_SHARED_GPU) wg.beside_others();
+      if (five ? wino_pays5(wg, f) : wino_pays(wg, f)) {
+        if (five && d.K <= kWinoBM) return false;
+        us = wg.us;
+        err = wino_err(wg);
+      }
+    }
+  }
+  *plan = make(tri_max_chain(err));
+  return plan->ok && plan->us < us;
+}
+inline bool tri_pays_fwd(const ConvDims& d, int flags, TriPlan* plan) {
+  return !fwd_gathers(d) && tri_pays(d, false, flags, plan, [&](int chain) { return plan_tri_fwd(d, chain); });
+}
+inline bool tri_pays_bwd_data(const ConvDims& d, int flags, TriPlan* plan) {
+  return d.st == 1 && tri_pays(d, true, flags, plan, [&](int chain) { return plan_tri_bwd_data(d, chain); });
+}
+// Filter gradient: the other forms take about 15 us, their multiply-adds at 50 (32-row tiles), 60 or 100 TFLOP/s, a quarter more
+// where taps are gathered or transformed, and 11 us a million weights of partial sums (fitted by hand to 308 timed calls, of
+// which this form is then chosen in 188, 1.53 times as fast in the geometric mean).  1x1 layers need 384 channels or so to be
+// worth two split copies.
+inline bool tri_pays_bwd_filter(const ConvDims& d, const TriFilterPlan& t) {
+  if (!t.ok || (wino_shape(d) && d.K <= kWinoBM && wino_filter_pays(d, plan_wino_bwd_filter(d)))) return false;
+  const int bm = pick_bm(d.K);
+  const double flops = 2.0 * (double)d.w_elems * d.N * d.P * d.Q;
+  const double other = (d.R * d.S > 1 ? 1.25 : 1.0) * (15.0 + flops / (bm >= 96 ? 100e6 : bm == 64 ? 60e6 : 50e6)) + 11e-6 * (double)d.w_elems;
+  return t.us < 0.9 * other;
 }
 
 int launch_conv_lds(const LdsConvPlan& pl, bool bwd, int N, int Ci, int H, int W, int rows, int P, int Q, int R, int halo,

@@ -870,7 +870,7 @@ class Conv2dOperator : public Operator {
       }
       return;
     }
-    const int math = (opts_.bf16_forward ? RH_MATH_BF16_MFMA_FP32ACC : 0) | (opts_.winograd ? 0 : RH_ALGO_DIRECT);
+    const int math = (opts_.bf16_forward ? RH_MATH_BF16_MFMA_FP32ACC : 0) | (opts_.winograd ? RH_ALGO_BF16X3 : RH_ALGO_DIRECT);
     if (opts_.fuse_epilogue) {
       const int flags = RH_FUSE_BIAS | (rect ? RH_FUSE_RELU : 0) | math;
       unwrap(rh_conv2d_fwd(&g, 1.0f, in_act_->as_ptr(), params_.weights->as_ptr(), 0.0f, out_act_->as_mut_ptr(),
@@ -904,7 +904,7 @@ class Conv2dOperator : public Operator {
       w_filter = w_bias = workspace_aux_.get();
     }
     const float beta = params_.take_backward_beta();   // 1: accumulate (the reference's call); 0: the buffers stand for zeros
-    const int algo = opts_.winograd ? 0 : RH_ALGO_DIRECT;
+    const int algo = opts_.winograd ? RH_ALGO_BF16X3 : RH_ALGO_DIRECT;
     // (a small layer's bias gradient rides in the launch of the filter gradient's reduction: the combined call below)
     const bool small = batch_size * out_dims_.len() <= (size_t(1) << 20);
     if (!in_delta_ && workspace_aux_ && overlap_on_ && !small) {
@@ -1527,7 +1527,7 @@ class BNormUnitsOperator : public Operator {
     in_act_ = prev_op->get_output_vars();
     if (!in_act_) panic(std::string(who) + " missing required prev operator output vars");
     in_delta_ = prev_op->get_output_deltas();
-    for (auto& u : units_) u.conv_algo = opts.winograd ? 0 : RH_ALGO_DIRECT;
+    for (auto& u : units_) u.conv_algo = opts.winograd ? RH_ALGO_BF16X3 : RH_ALGO_DIRECT;
   }
   size_t batch_size() const override { return batch_cap_; }
   SharedDeviceBuf get_output_vars() const override { return out_act_; }

@@ -43,6 +43,14 @@ def conv_geom(x_shape, w_shape, stride, pad):
     return ConvGeom(N, Cc, H, W, K, R, S, stride, pad)
 
 
+def conv_ws_bytes(g, pass_, algo):
+    """Scratch of a convolution pass under `algo`."""
+    forced = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
+    if algo & forced == forced:
+        return lib().rh_conv2d_bf16x3_workspace_bytes(C.byref(g), pass_)
+    return lib().rh_conv2d_workspace_bytes(C.byref(g), pass_)
+
+
 def conv_out_shape(g):
     out = lib().rh_conv2d_out_dim
     return (g.N, g.K, out(g.H, g.R, g.stride, g.pad), out(g.W, g.S, g.stride, g.pad))
@@ -52,7 +60,7 @@ def conv2d_fwd(x, w, stride, pad, bias=None, relu=False, alpha=1.0, beta=0.0, y=
     g = conv_geom(x.shape, w.shape, stride, pad)
     if y is None:
         y = torch.empty(conv_out_shape(g), dtype=torch.float32, device=x.device)
-    need = lib().rh_conv2d_workspace_bytes(C.byref(g), _lib.RH_CONV_FWD)
+    need = conv_ws_bytes(g, _lib.RH_CONV_FWD, algo)
     ws = workspace(need, x.device)
     flags = (_lib.RH_FUSE_BIAS if bias is not None else 0) | (_lib.RH_FUSE_RELU if relu else 0) | algo
     check(lib().rh_conv2d_fwd(C.byref(g), alpha, _p(x), _p(w), beta, _p(y), _p(bias), _p(ws), ws.numel(), flags,
@@ -64,7 +72,7 @@ def conv2d_bwd_filter(x, dy, w_shape, stride, pad, alpha=1.0, beta=0.0, dw=None,
     g = conv_geom(x.shape, w_shape, stride, pad)
     if dw is None:
         dw = torch.zeros(tuple(w_shape), dtype=torch.float32, device=x.device)
-    need = lib().rh_conv2d_workspace_bytes(C.byref(g), _lib.RH_CONV_BWD_FILTER)
+    need = conv_ws_bytes(g, _lib.RH_CONV_BWD_FILTER, algo)
     ws = workspace(need, x.device)
     check(lib().rh_conv2d_bwd_filter(C.byref(g), alpha, _p(x), _p(dy), beta, _p(dw), _p(ws), ws.numel(), algo,
                                      _stream()), "rh_conv2d_bwd_filter")
@@ -78,7 +86,7 @@ def conv2d_bwd_filter_bias(x, dy, w_shape, stride, pad, alpha=1.0, beta=0.0, dw=
         dw = torch.zeros(tuple(w_shape), dtype=torch.float32, device=x.device)
     if db is None:
         db = torch.zeros((w_shape[0],), dtype=torch.float32, device=x.device)
-    need = lib().rh_conv2d_workspace_bytes(C.byref(g), _lib.RH_CONV_BWD_FILTER)
+    need = conv_ws_bytes(g, _lib.RH_CONV_BWD_FILTER, algo)
     ws = workspace(need, x.device)
     check(lib().rh_conv2d_bwd_filter_bias(C.byref(g), alpha, _p(x), _p(dy), beta, _p(dw), _p(db), _p(ws), ws.numel(), algo,
                                           _stream()), "rh_conv2d_bwd_filter_bias")
@@ -105,7 +113,7 @@ def conv2d_bwd_data(w, dy, x_shape, stride, pad, alpha=1.0, beta=0.0, dx=None, a
     g = conv_geom(x_shape, w.shape, stride, pad)
     if dx is None:
         dx = torch.zeros(tuple(x_shape), dtype=torch.float32, device=w.device)
-    need = lib().rh_conv2d_workspace_bytes(C.byref(g), _lib.RH_CONV_BWD_DATA)
+    need = conv_ws_bytes(g, _lib.RH_CONV_BWD_DATA, algo)
     ws = workspace(need, w.device)
     if relu_of is not None:
         check(lib().rh_conv2d_bwd_data_relu(C.byref(g), alpha, _p(w), _p(dy), beta, _p(dx), _p(relu_of), _p(ws), ws.numel(),

@@ -58,6 +58,7 @@ pub const RH_ALGO_SCALAR_OFFSET: c_int = 0x200;
 pub const RH_ALGO_WINOGRAD: c_int = 0x400;
 pub const RH_ALGO_DIRECT: c_int = 0x800;
 pub const RH_ALGO_SHARED_GPU: c_int = 0x1000;
+pub const RH_ALGO_BF16X3: c_int = 0x2000;
 
 #[link(name = "rembrandt_hip")]
 extern "C" {
@@ -87,6 +88,7 @@ extern "C" {
   pub fn rh_pool2d_out_dim(input: i32, size: i32, stride: i32, pad: i32, round: i32) -> i32;
   pub fn rh_conv2d_winograd_flops(g: *const rh_conv_geom, pass: c_int, flags: c_int) -> f64;
   pub fn rh_conv2d_workspace_bytes(g: *const rh_conv_geom, pass: c_int) -> size_t;
+  pub fn rh_conv2d_bf16x3_workspace_bytes(g: *const rh_conv_geom, pass: c_int) -> size_t;
   pub fn rh_conv2d_workspace_bytes_upto(g: *const rh_conv_geom, pass: c_int) -> size_t;
   pub fn rh_conv2d_fwd(g: *const rh_conv_geom, alpha: c_float, x: *const f32, w: *const f32, beta: c_float,
                        y: *mut f32, bias: *const f32, ws: *mut c_void, ws_bytes: size_t, flags: c_int,

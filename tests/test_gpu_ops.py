@@ -516,6 +516,132 @@ def test_conv2d_winograd_refused_geometries(dev):
             assert rc == _lib.RH_E_UNSUPPORTED, ("bwd filter", R, st, pad, extra, rc)
 
 
+# RH_ALGO_BF16X3: fp32 contractions on bf16 matrix instructions, each operand as the sum of three bf16 values.  Contracted
+# channel counts of one group of eight, of an odd number of groups (a K step that two taps share) and of many; an odd number
+# of groups in all (a last K step with a half of zeros); one to 128 K steps against a ring of three; row counts around the
+# 64-, 96- and 128-row tiles; ragged pixels; batches around a group of eight images; strides; contractions in slices, and a
+# sliced tail past a whole round of tiles; channels that no pass but the filter gradient takes.
+X3_CASES = [
+    # N, C, H, W, K, R, stride, pad
+    (2, 8, 9, 7, 8, 3, 1, 1),
+    (1, 8, 4, 4, 3, 1, 1, 0),
+    (3, 24, 13, 13, 40, 3, 1, 1),
+    (1, 16, 5, 5, 64, 3, 1, 0),
+    (8, 40, 11, 12, 130, 3, 1, 2),
+    (9, 64, 14, 15, 65, 5, 1, 2),
+    (17, 96, 9, 9, 96, 1, 1, 0),
+    (2, 96, 13, 13, 256, 5, 1, 2),
+    (7, 128, 12, 12, 192, 3, 2, 1),
+    (3, 16, 20, 20, 128, 5, 4, 2),
+    (33, 32, 28, 28, 64, 3, 1, 1),
+    (80, 128, 21, 21, 128, 3, 1, 1),
+    (1, 512, 7, 7, 512, 3, 1, 1),
+    (5, 3, 23, 22, 33, 7, 2, 3),
+]
+
+
+@pytest.mark.parametrize("case", X3_CASES, ids=str)
+def test_conv2d_bf16x3(dev, case):
+    """All passes in the split-operand form against the oracle, with every epilogue."""
+    Nn, C, H, W, K, R, st, pad = case
+    say("bf16x3 case", case)
+    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
+    x, w, b = synth.normal(33, 1, (Nn, C, H, W)), synth.normal(33, 2, (K, C, R, R)), synth.normal(33, 3, (K,))
+    y_ref = O.conv2d_fwd(x, w, st, pad)
+    dy, y0, dx0, dw0, db0 = (synth.normal(33, 4 + i, s) for i, s in enumerate((y_ref.shape, y_ref.shape, x.shape, w.shape, (K,))))
+    xd, wd, bd, dyd = T(x, dev), T(w, dev), T(b, dev), T(dy, dev)
+    if C % 8 == 0:
+        y, tags = profile_tags(lambda: ops.conv2d_fwd(xd, wd, st, pad, algo=X3))
+        assert any(t.startswith("conv_fwd_tri_") for t in tags), tags
+        assert_close(N(y), y_ref, "bf16x3 fwd")
+        yf = ops.conv2d_fwd(xd, wd, st, pad, bias=bd, relu=True, algo=X3)
+        assert torch.equal(torch.clamp_min(y + bd.view(1, -1, 1, 1), 0.0), yf), "fused epilogue == conv, add_bias, rect"
+        yb = ops.conv2d_fwd(xd, wd, st, pad, alpha=0.5, beta=2.0, y=T(y0, dev), algo=X3)
+        assert_close(N(yb), O.conv2d_fwd(x, w, st, pad, alpha=0.5, beta=2.0, y=y0.copy()), "bf16x3 fwd alpha/beta")
+        assert torch.equal(ops.conv2d_fwd(xd, wd, st, pad, algo=X3), y), "run to run the same bits"
+    else:
+        with pytest.raises(_lib.RembrandtHipError):
+            ops.conv2d_fwd(xd, wd, st, pad, algo=X3)
+    if K % 8 == 0 and st == 1 and pad <= R - 1:
+        assert_close(N(ops.conv2d_bwd_data(wd, dyd, x.shape, st, pad, algo=X3)), O.conv2d_bwd_data(w, dy, x.shape, st, pad), "bf16x3 bwd data")
+        for alpha, beta in ((1.0, 0.0), (0.5, 2.0)):
+            two = ops.conv2d_bwd_data(wd, dyd, x.shape, st, pad, alpha=alpha, beta=beta, dx=T(dx0, dev), algo=X3)
+            assert_close(N(two), O.conv2d_bwd_data(w, dy, x.shape, st, pad, alpha, beta, dx0.copy()), "bf16x3 bwd data alpha/beta")
+            ops.rect_backprop_inplace(xd, two)
+            one = ops.conv2d_bwd_data(wd, dyd, x.shape, st, pad, alpha=alpha, beta=beta, dx=T(dx0, dev), algo=X3, relu_of=xd)
+            assert torch.equal(one, two), "masked data gradient alpha=%g beta=%g" % (alpha, beta)
+    else:
+        with pytest.raises(_lib.RembrandtHipError):
+            ops.conv2d_bwd_data(wd, dyd, x.shape, st, pad, algo=X3)
+    dw, tags = profile_tags(lambda: ops.conv2d_bwd_filter(xd, dyd, w.shape, st, pad, algo=X3))
+    assert any(t.startswith("conv_bwd_filter_tri_") for t in tags), tags
+    assert_close(N(dw), O.conv2d_bwd_filter(x, dy, w.shape, st, pad), "bf16x3 bwd filter")
+    dwc, dbc = ops.conv2d_bwd_filter_bias(xd, dyd, w.shape, st, pad, alpha=0.25, beta=1.0, dw=T(dw0, dev), db=T(db0, dev), algo=X3)
+    assert_close(N(dwc), O.conv2d_bwd_filter(x, dy, w.shape, st, pad, 0.25, 1.0, dw0.copy()), "bf16x3 bwd filter alpha/beta")
+    assert_close(N(dbc), O.conv2d_bwd_bias(dy, 0.25, 1.0, db0.copy()), "bf16x3 bias gradient")
+    assert torch.equal(ops.conv2d_bwd_filter(xd, dyd, w.shape, st, pad, algo=X3), dw), "run to run the same bits"
+
+
+@pytest.mark.parametrize("relu", [False, True], ids=["normal", "half_zeros"])
+@pytest.mark.parametrize("case", [(16, 256, 13, 13, 384, 3, 1), (64, 128, 28, 28, 128, 3, 1), (9, 96, 27, 27, 256, 5, 2), (32, 64, 28, 28, 64, 3, 1)], ids=str)
+def test_conv2d_bf16x3_error(dev, case, relu):
+    """Error against 64-bit sums: within the bound of the form's own chain, and where the library takes it by itself no larger than
+    that of the form it replaces (staged, Winograd).  The large products add to a sum of 16 terms per MFMA; with two roundings each (the instruction's own order is not
+    documented) a chain of n steps has a relative rms error of sqrt(0.09 * 2 n + 4) 2^-24 (a rounding's variance as in
+    test_conv2d_staged_operands_error; four more for the small products' own chain and the result).  A quarter on top."""
+    Nn, C, H, W, K, R, pad = case
+    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
+    x, w = synth.normal(35, 1, (Nn, C, H, W)), synth.normal(35, 2, (K, C, R, R))
+    if relu:
+        x = np.maximum(x, 0.0)
+    dy = synth.normal(35, 3, (Nn, K, H, W))
+    xd, wd, dyd = T(x, dev), T(w, dev), T(dy, dev)
+    for ref, terms, run in (
+            (O.conv2d_fwd(x, w, 1, pad), C * R * R, lambda algo: ops.conv2d_fwd(xd, wd, 1, pad, algo=algo)),
+            (O.conv2d_bwd_data(w, dy, x.shape, 1, pad), K * R * R, lambda algo: ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=algo))):
+        err = float(np.linalg.norm(N(run(X3)).astype(np.float64) - ref) / np.linalg.norm(ref.astype(np.float64)))
+        assert err <= 1.25 * 2.0 ** -24 * (0.18 * terms / 16 + 4) ** 0.5, (terms, err)
+        auto, before = (float(np.linalg.norm(N(run(algo)).astype(np.float64) - ref)) for algo in (_lib.RH_ALGO_BF16X3, 0))
+        assert auto <= before, (auto, before)
+
+
+def test_conv2d_bf16x3_infinities_and_largest_floats(dev):
+    """What is not finite comes out as fp32 multiplication makes it: infinities where no NaN is, NaNs where there are (the
+    products of an infinity's zero parts are NaNs inside); values that round to an infinity in bf16 stay finite."""
+    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
+    Nn, C, H, W, K, R, pad = 19, 40, 13, 13, 72, 3, 1
+    x, w = synth.normal(37, 1, (Nn, C, H, W)), synth.normal(37, 2, (K, C, R, R))
+    dy = synth.normal(37, 3, (Nn, K, H, W))
+    x[3, 5, 4, 4], x[4, 7, 0, 12], x[6, 1, 1, 1] = np.inf, -np.inf, np.nan
+    x[7, 2, 3, 3], x[8, 2, 3, 3] = 3.4e38, -np.finfo(np.float32).max
+    w[5, :, 1, 1], w[6] = 0.5, 0.125
+    dy[2, 3, 1, 1] = np.inf
+    w[:, 2] *= 0.125   # (the largest floats' products stay in range)
+    xd, wd, dyd = T(x, dev), T(w, dev), T(dy * 0.125, dev)
+    G = _lib.RH_ALGO_SCALAR_OFFSET
+    for run in (lambda algo: ops.conv2d_fwd(xd, wd, 1, pad, algo=algo), lambda algo: ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=algo),
+                lambda algo: ops.conv2d_bwd_filter(xd, dyd, w.shape, 1, pad, algo=algo)):
+        got, ref = run(X3), run(G)
+        assert bool(torch.isinf(ref).any())
+        assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
+        keep = torch.isfinite(ref)
+        assert torch.equal(got[torch.isinf(ref)], ref[torch.isinf(ref)])
+        assert bool(((got - ref).abs()[keep] <= 1e-4 * (1.0 + ref.abs()[keep])).all())
+
+
+def test_conv2d_bf16x3_where_it_pays(dev):
+    """RH_ALGO_BF16X3 alone: the form where it is expected to be the fastest, and the others' bits elsewhere."""
+    for (Nn, C, H, K, R, st, pad), takes in (((37, 256, 13, 384, 3, 1, 1), True), ((24, 128, 28, 256, 3, 2, 1), True), ((8, 96, 27, 256, 5, 1, 2), True),
+                                             ((16, 96, 54, 96, 1, 1, 0), False), ((1, 256, 13, 384, 3, 1, 1), False), ((4, 12, 20, 24, 3, 1, 1), False)):
+        x, w = T(synth.normal(39, 1, (Nn, C, H, H)), dev), T(synth.normal(39, 2, (K, C, R, R)), dev)
+        y, tags = profile_tags(lambda: ops.conv2d_fwd(x, w, st, pad, algo=_lib.RH_ALGO_BF16X3))
+        assert any(t.startswith("conv_fwd_tri_") for t in tags) == takes, (Nn, C, H, K, R, tags)
+        other = ops.conv2d_fwd(x, w, st, pad)
+        if not takes:
+            assert torch.equal(y, other)
+        assert bool(((y - other).norm() <= 2e-6 * other.norm()).item())
+
+
 # input channels a multiple of 8 take the packed-operand form (bf16 copies of image and filter in 16-byte groups of
 # eight channels): channel groups that do not fill a 64-wide tile, rectangular images, stride with padding, no padding,
 # more filters than one row tile, a contraction shorter than one K step
