@@ -237,6 +237,10 @@ int rh_rect_backprop_copy(const float* y, float* dy, float* copy, size_t n, rh_s
  * GPU split the contraction across blocks and reduce in a fixed order; without it (ws == NULL)
  * the same result is computed unsplit. */
 size_t rh_sgemm_workspace_bytes(int32_t m, int32_t n, int32_t k);
+/* The same for RH_ALGO_BF16X3 with RH_ALGO_DIRECT; 0 where the product has no such form: it needs A or B untransposed, m a
+ * multiple of 4, and with A transposed k a multiple of 16 (unless B is transposed also lda a multiple of 4 and A 16-byte
+ * aligned).  RH_ALGO_BF16X3 alone takes that form where it is expected to be faster and the scratch holds it. */
+size_t rh_sgemm_bf16x3_workspace_bytes(int transA, int transB, int32_t m, int32_t n, int32_t k);
 /* Largest need when one extent varies from 1 up to the value given (which: 0 = m, 1 = n, 2 = k): the affine
  * operators call with the batch as n (forward, data gradient) or k (weight gradient) and any batch <= batch_cap. */
 size_t rh_sgemm_workspace_bytes_upto(int32_t m, int32_t n, int32_t k, int which);

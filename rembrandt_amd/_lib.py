@@ -112,6 +112,7 @@ PROTOTYPES = {
     "rh_rect_backprop_copy": (_int, [_vp, _vp, _vp, _sz, _vp]),
     "rembrandt_kernel_batch_map_rect_backprop_inplace": (None, [_vp, _i32, _i32, _vp, _vp]),
     "rh_sgemm_workspace_bytes": (_sz, [_i32, _i32, _i32]),
+    "rh_sgemm_bf16x3_workspace_bytes": (_sz, [_int, _int, _i32, _i32, _i32]),
     "rh_sgemm": (_int, [_int, _int, _i32, _i32, _i32, _f, _vp, _i32, _vp, _i32, _f, _vp, _i32, _vp, _sz, _int, _vp]),
     "rh_sgemm_bias_act": (_int, [_int, _int, _i32, _i32, _i32, _f, _vp, _i32, _vp, _i32, _f, _vp, _i32, _vp, _vp, _sz, _int, _vp]),
     "rh_saxpy": (_int, [_i64, _f, _vp, _vp, _vp]),

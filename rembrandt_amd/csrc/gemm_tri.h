@@ -26,12 +26,11 @@ struct TriParams {
   int plane;
 };
 
-// Eight values (one group) into the three parts' groups.
-__device__ __forceinline__ void tri_pack8(const float (&v)[8], uint4 (&o)[3]) {
+// Eight values (one group) into the three parts' groups: pair() for each of the four pairs, then fix().
+struct TriPack8 {
   uint32_t w[3][4];
   float rest = 0.0f;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
+  __device__ __forceinline__ void pair(const float (&v)[8], int e) {
     float x = v[2 * e], y = v[2 * e + 1];
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
@@ -41,7 +40,8 @@ __device__ __forceinline__ void tri_pack8(const float (&v)[8], uint4 (&o)[3]) {
     }
     rest += x + y;   // zeros, or a NaN where a first part is no number
   }
-  if (!(rest == 0.0f)) {
+  __device__ __forceinline__ void fix(const float (&v)[8]) {
+    if (rest == 0.0f) return;
     // infinities and NaNs have no further parts; the largest floats, which round to an infinity, are cut off instead
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
@@ -64,8 +64,15 @@ __device__ __forceinline__ void tri_pack8(const float (&v)[8], uint4 (&o)[3]) {
       }
     }
   }
+  __device__ __forceinline__ uint4 part(int i) const { return make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]); }
+};
+__device__ __forceinline__ void tri_pack8(const float (&v)[8], uint4 (&o)[3]) {
+  TriPack8 t;
 #pragma unroll
-  for (int i = 0; i < 3; ++i) o[i] = make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]);
+  for (int e = 0; e < 4; ++e) t.pair(v, e);
+  t.fix(v);
+#pragma unroll
+  for (int i = 0; i < 3; ++i) o[i] = t.part(i);
 }
 
 // Brings one K step (16 k = two groups, three parts) of both operands to LDS with direct loads.  A tile has four blocks of

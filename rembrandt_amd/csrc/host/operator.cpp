@@ -668,6 +668,7 @@ class AffineOperator : public Operator {
   AffineOperator(size_t batch_size, OpCapability capability, const AffineOperatorConfig& config, const Operator* prev_op,
                  Ctx context, const ExecOptions& opts)
       : batch_cap_(batch_size), config_(config), context_(context), fuse_epilogue_(opts.fuse_epilogue),
+        algo_(opts.winograd ? RH_ALGO_BF16X3 : 0),
         overlap_built_(opts.overlap_backward && backward_enabled(capability)), overlap_on_(overlap_built_) {
     RB_ASSERT(prev_op != nullptr);
     in_act_ = prev_op->get_output_vars();
@@ -705,11 +706,11 @@ class AffineOperator : public Operator {
       // bias and activation in the product's epilogue: one kernel for the reference's three
       unwrap(rh_sgemm_bias_act(1, 0, o, b, i, 1.0f, params_.weights->as_ptr(), i, in_act_->as_ptr(), i, 0.0f,
                                out_act_->as_mut_ptr(), o, params_.bias->as_ptr(), ws_ptr(), ws_len(),
-                               RH_FUSE_BIAS | (rect ? RH_FUSE_RELU : 0), s), "matrix_prod");
+                               RH_FUSE_BIAS | (rect ? RH_FUSE_RELU : 0) | algo_, s), "matrix_prod");
       return;
     }
     unwrap(rh_sgemm(1, 0, o, b, i, 1.0f, params_.weights->as_ptr(), i, in_act_->as_ptr(), i, 0.0f,
-                    out_act_->as_mut_ptr(), o, ws_ptr(), ws_len(), 0, s), "matrix_prod");
+                    out_act_->as_mut_ptr(), o, ws_ptr(), ws_len(), algo_, s), "matrix_prod");
     unwrap(rh_add_bias_nchw(params_.bias->as_ptr(), out_act_->as_mut_ptr(), 1, o, b, 1.0f, 1.0f, s), "add_bias");
     apply_rect(config_.act_func, out_act_->as_mut_ptr(), config_.out_channels, batch_size, s);
   }
@@ -735,7 +736,7 @@ class AffineOperator : public Operator {
     const float beta = params_.take_backward_beta();   // 1: accumulate (the reference's call); 0: the buffers stand for zeros
     // grad_weights(in, out) += in_act(in, B) * out_delta(out, B)^T
     unwrap(rh_sgemm(0, 1, i, o, b, 1.0f, in_act_->as_ptr(), i, out_delta_->as_ptr(), o, beta,
-                    params_.grad_weights->as_mut_ptr(), i, wg, wg_len, 0, sg), "matrix_prod");
+                    params_.grad_weights->as_mut_ptr(), i, wg, wg_len, algo_, sg), "matrix_prod");
     // grad_bias(1, out) += 1(1, B) * out_delta^T: the column sums of out_delta, without the ones vector
     if (!bias_grad_done_)
       unwrap(rh_conv2d_bwd_bias(b, o, 1, 1.0f, out_delta_->as_ptr(), beta, params_.grad_bias->as_mut_ptr(), sg), "matrix_prod");
@@ -743,7 +744,7 @@ class AffineOperator : public Operator {
     if (in_delta_) {
       // in_delta(in, B) = weights(in, out) * out_delta(out, B)
       unwrap(rh_sgemm(0, 0, i, b, o, 1.0f, params_.weights->as_ptr(), i, out_delta_->as_ptr(), o, 0.0f,
-                      in_delta_->as_mut_ptr(), i, ws_ptr(), ws_len(), 0, s), "matrix_prod");
+                      in_delta_->as_mut_ptr(), i, ws_ptr(), ws_len(), algo_, s), "matrix_prod");
     }
   }
   void regularize(Regularization reg) override { params_.regularize(reg); }
@@ -784,6 +785,7 @@ class AffineOperator : public Operator {
   AffineOperatorConfig config_;
   Ctx context_;
   bool fuse_epilogue_;               // bias and activation inside the forward product
+  int algo_;                         // forms that the three products may take
   SharedDeviceBuf in_act_, in_delta_, out_act_, out_delta_;
   ParamTensors params_;
   std::unique_ptr<DeviceBuffer<uint8_t>> workspace_, workspace_aux_;

@@ -9,6 +9,7 @@
 #include <type_traits>
 
 #include "conv_common.h"
+#include "sgemm_tri.h"
 
 namespace rh {
 
@@ -195,6 +196,26 @@ static int skinny_mode(int m, int n, int k) {
   return 0;
 }
 
+// Where a caller that allows it (RH_ALGO_BF16X3) gets the form of exactly split operands: where it was faster, or as fast, in 77
+// layers and batches timed in all three products with the weights in turn from four buffers, and where its chains of sums are no
+// longer than the engine's error allows (tri_max_chain).  Engine -> this form, us, 9216 -> 4096 at 8, 37, 64, 128, 256 images:
+// forward 40 -> 33, 63 -> 38, 66 -> 42, 94 -> 65, 164 -> 112, data gradient the same within 5 %, filter gradient 31 -> 33,
+// 46 -> 46, 56 -> 56, 94 -> 68, 155 -> 114.  The split copy is a launch of its own, 3 to 6 us: 1024 -> 512 is slower in both
+// passes at every batch (37 images 14.0 -> 14.9), 2048 -> 1024 faster up to 128 (17.3 -> 15.1) and slower at 200 (22.6 -> 24.6).
+// A block of 32 rows is bound by the weights' bytes in either form, and only many of them cover the copy.  Filter gradients
+// of up to 64 images are bound by the result's bytes; those of 65 to 96 gain where the result is large.
+static bool sgemm_tri_pays(bool a_trans, bool b_trans, int m, int n, int k, SgemmTriPlan* plan) {
+  const long long mk = (long long)m * k, mn = (long long)m * n;
+  *plan = SgemmTriPlan{};
+  if (b_trans) {
+    if (a_trans || k <= 32 || mn < (k <= 96 ? 16ll << 20 : k <= 256 ? 1ll << 19 : 4ll << 20)) return false;
+  } else if (n > 512 || mk < (n <= 32 ? 16ll << 20 : n <= 128 ? 3ll << 19 : 4000000ll)) {
+    return false;
+  }
+  *plan = plan_sgemm_tri(a_trans, b_trans, m, n, k);
+  return plan->ok && cdiv(plan->groups / 2, plan->splits) <= tri_max_chain(0.0335 * k / plan_sgemm(m, n, k).splits);
+}
+
 // y[i] += alpha * x[i]
 __global__ void saxpy_kernel(long long n, float alpha, const float* __restrict__ x, float* __restrict__ y) {
   const long long stride = (long long)gridDim.x * blockDim.x;
@@ -242,8 +263,17 @@ using namespace rh;
 extern "C" size_t rh_sgemm_workspace_bytes(int32_t m, int32_t n, int32_t k) {
   if (m <= 0 || n <= 0 || k <= 0) return 0;
   const SgemmPlan p = plan_sgemm(m, n, k);
-  if (p.splits <= 1) return 0;
-  return align256(sizeof(float) * (size_t)p.splits * m * n);
+  size_t need = p.splits > 1 ? align256(sizeof(float) * (size_t)p.splits * m * n) : 0;
+  for (int form = 0; form < 3; ++form) {
+    SgemmTriPlan tp;
+    if (sgemm_tri_pays(form == 1, form == 2, m, n, k, &tp) && tp.total() > need) need = tp.total();
+  }
+  return need;
+}
+
+extern "C" size_t rh_sgemm_bf16x3_workspace_bytes(int transA, int transB, int32_t m, int32_t n, int32_t k) {
+  const SgemmTriPlan p = plan_sgemm_tri(transA, transB, m, n, k);
+  return p.ok ? p.total() : 0;
 }
 
 extern "C" size_t rh_sgemm_workspace_bytes_upto(int32_t m, int32_t n, int32_t k, int which) {
@@ -282,7 +312,8 @@ extern "C" int rh_sgemm_bias_act(int transA, int transB, int32_t m, int32_t n, i
       ((size_t)ldc * (n - 1) + m) * 4 > kMaxBufferBytes)
     return RH_E_LIMIT;
 
-  if (!(flags & RH_ALGO_GATHER)) {
+  const bool tri_forced = tri_allowed(flags) && (flags & RH_ALGO_DIRECT);
+  if (!(flags & RH_ALGO_GATHER) && !tri_forced) {
     if (const int mode = skinny_mode(m, n, k)) {
       SkinnyArgs a;
       a.A = A; a.B = B; a.C = C; a.bias_col = bias_col;
@@ -302,31 +333,41 @@ extern "C" int rh_sgemm_bias_act(int transA, int transB, int32_t m, int32_t n, i
   DenseParams bp;  // engine B operand = opA, rows = m
   bp.ptr = A; bp.bytes = (uint32_t)(a_elems * 4); bp.rows = m; bp.K = k; bp.ld = lda; bp.ktab = nullptr;
 
+  EpiParams ep;
+  ep.bias = nullptr; ep.alpha = alpha; ep.beta = beta; ep.rows = n; ep.cols = m; ep.inner = 0;
+  ep.relu = relu; ep.bias_col = bias_col;   // (ignored by blocks that write partial sums)
+  auto set_out = [&](float* part) {
+    ep.out = part ? part : C; ep.ld = part ? m : ldc; ep.split_stride = part ? (long long)m * n : 0;
+  };
+  auto reduce = [&](int used) -> int {
+    launch_split_reduce(ep.out, used, (long long)m * n, C, n, m, ldc, alpha, beta, stream, bias_col, relu);
+    return launch_status();
+  };
+  int used = 1, e;
+  if (tri_allowed(flags)) {
+    SgemmTriPlan tp;
+    const bool pays = sgemm_tri_pays(transA, transB, m, n, k, &tp);
+    if (tri_forced) tp = plan_sgemm_tri(transA, transB, m, n, k);
+    const bool form = tp.ok && (transB || (lda % 4 == 0 && (reinterpret_cast<uintptr_t>(A) & 15) == 0));
+    const bool room = ws && ws_bytes >= tp.total() && (reinterpret_cast<uintptr_t>(ws) & 255) == 0;
+    if (tri_forced && !form) return RH_E_UNSUPPORTED;
+    if (tri_forced && !room) return RH_E_WORKSPACE;
+    if (form && room && (tri_forced || pays)) {
+      set_out(tp.splits > 1 ? reinterpret_cast<float*>(static_cast<char*>(ws) + tp.part_at()) : nullptr);
+      e = launch_sgemm_tri(tp, transA, transB, ap, bp, ep, ws, stream, &used);
+      return e || tp.splits <= 1 ? e : reduce(used);
+    }
+  }
   SgemmPlan plan = plan_sgemm(m, n, k);
   const size_t need = plan.splits > 1 ? align256(sizeof(float) * (size_t)plan.splits * m * n) : 0;
   if (plan.splits > 1 && (!ws || ws_bytes < need || (reinterpret_cast<uintptr_t>(ws) & 255))) plan.splits = 1;
 
-  EpiParams ep;
-  ep.bias = nullptr; ep.alpha = alpha; ep.beta = beta; ep.rows = n; ep.cols = m; ep.inner = 0;
-  ep.relu = relu; ep.bias_col = bias_col;   // (ignored by blocks that write partial sums)
-  if (plan.splits > 1) {
-    ep.out = static_cast<float*>(ws); ep.ld = m; ep.split_stride = (long long)m * n;
-  } else {
-    ep.out = C; ep.ld = ldc; ep.split_stride = 0;
-  }
-
-  int used = 1, e;
+  set_out(plan.splits > 1 ? static_cast<float*>(ws) : nullptr);
   if (!transB && !transA)      e = dispatch_tile<false, false>(plan.bm, ap, bp, ep, k, plan.splits, &used, stream);
   else if (!transB && transA)  e = dispatch_tile<false, true>(plan.bm, ap, bp, ep, k, plan.splits, &used, stream);
   else if (transB && !transA)  e = dispatch_tile<true, false>(plan.bm, ap, bp, ep, k, plan.splits, &used, stream);
   else                         e = dispatch_tile<true, true>(plan.bm, ap, bp, ep, k, plan.splits, &used, stream);
-  if (e) return e;
-  if (plan.splits > 1) {
-    launch_split_reduce(static_cast<const float*>(ws), used, (long long)m * n, C, n, m, ldc, alpha, beta, stream, bias_col,
-                        relu);
-    return launch_status();
-  }
-  return 0;
+  return e || plan.splits <= 1 ? e : reduce(used);
 }
 
 extern "C" int rh_saxpy(int64_t n, float alpha, const float* x, float* y, rh_stream_t stream) {

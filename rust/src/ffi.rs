@@ -128,6 +128,7 @@ extern "C" {
   pub fn rh_rect_backprop_copy(y: *const f32, dy: *mut f32, copy: *mut f32, n: size_t, stream: rh_stream_t) -> c_int;
 
   pub fn rh_sgemm_workspace_bytes(m: i32, n: i32, k: i32) -> size_t;
+  pub fn rh_sgemm_bf16x3_workspace_bytes(trans_a: c_int, trans_b: c_int, m: i32, n: i32, k: i32) -> size_t;
   pub fn rh_sgemm(trans_a: c_int, trans_b: c_int, m: i32, n: i32, k: i32, alpha: c_float, a: *const f32,
                   lda: i32, b: *const f32, ldb: i32, beta: c_float, c: *mut f32, ldc: i32, ws: *mut c_void,
                   ws_bytes: size_t, flags: c_int, stream: rh_stream_t) -> c_int;

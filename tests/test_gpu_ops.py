@@ -855,6 +855,98 @@ def test_sgemm_bias_act(dev, case):
             assert np.array_equal(N(Cs), got), "fused and separate calls differ"
 
 
+# The products of affine layers with RH_ALGO_BF16X3.  Rows (n) around the 32-, 64- and 128-row blocks and two of them; columns
+# (m) that do not fill a block of 128, a wave's 32 or a group of 8; contractions of one K step, of fewer than a block's ring of
+# steps (4, 5 and 7), of an odd number, in slices whose last one is shorter, and with a last step that is not full (where k is no
+# contiguous extent of A).  Padded lda, ldb, ldc.
+SGEMM_X3_CASES = [
+    # tA, tB, m, n, k
+    (1, 0, 4, 1, 16), (1, 0, 132, 31, 48), (1, 0, 260, 33, 80), (1, 0, 96, 64, 112), (1, 0, 100, 65, 64), (1, 0, 516, 129, 496),
+    (1, 0, 1000, 37, 4096), (1, 0, 2052, 256, 2064),
+    (0, 0, 4, 1, 3), (0, 0, 132, 32, 50), (0, 0, 260, 40, 77), (0, 0, 36, 63, 129), (0, 0, 100, 100, 16), (0, 0, 516, 130, 1000),
+    (0, 0, 4096, 50, 1000),
+    (0, 1, 4, 1, 1), (0, 1, 132, 129, 9), (0, 1, 500, 1000, 50), (0, 1, 1028, 260, 256),
+]
+
+
+@pytest.mark.parametrize("case", SGEMM_X3_CASES, ids=str)
+def test_sgemm_bf16x3(dev, case):
+    """The split-operand form against the oracle, its error against 64-bit sums, and what is not finite.  Bound of the error: as
+    in test_conv2d_bf16x3_error, a chain of n steps of 16 terms has sqrt(0.18 n + 4) 2^-24, a quarter on top."""
+    tA, tB, m, n, k = case
+    say("sgemm bf16x3", case)
+    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
+    a_shape, b_shape = ((m, k) if tA else (k, m)), ((k, n) if tB else (n, k))
+    lda, ldb, ldc = (a_shape[1] + 7) // 4 * 4, b_shape[1] + 1, m + 2
+    A, B, C0 = synth.normal(16, 1, (a_shape[0], lda)), synth.normal(16, 2, (b_shape[0], ldb)), synth.normal(16, 3, (n, ldc))
+    bias = synth.normal(16, 4, (m,))
+    Ad, Bd = T(A, dev), T(B, dev)
+    opA = (A[:, :k].T if tA else A[:, :m]).astype(np.float64)     # [k][m]
+    opB = (B[:, :n].T if tB else B[:, :k]).astype(np.float64)     # [n][k]
+    exact = opB @ opA
+    for alpha, beta, relu in ((1.0, 0.0, False), (0.5, 1.0, False), (1.0, 0.0, True)):
+        Cd = T(C0, dev)
+        ops.sgemm(tA, tB, m, n, k, alpha, Ad, lda, Bd, ldb, beta, Cd, ldc, bias=T(bias, dev) if relu else None, relu=relu, algo=X3)
+        got, ref = N(Cd), alpha * exact + beta * C0[:, :m]
+        if relu:
+            ref = np.maximum(ref + bias, 0.0)
+        assert_close(got[:, :m], ref.astype(np.float32), "sgemm bf16x3 alpha=%g beta=%g" % (alpha, beta))
+        assert np.array_equal(got[:, m:], C0[:, m:]), "wrote outside ldc padding"
+        if alpha == 1.0 and not relu:
+            err = np.linalg.norm(got[:, :m] - exact) / np.linalg.norm(exact)
+            assert err <= 1.25 * 2.0 ** -24 * (0.18 * k / 16 + 4) ** 0.5, err
+    # an infinity, a NaN and values that round to an infinity in bf16, in either operand
+    A[0, 0], B[n // 2 if not tB else 0, 0] = np.inf, -3.4e38
+    A[-1, (k if tA else m) - 1] = -np.inf
+    B[-1, (n if tB else k) - 1] = np.nan if n > 2 and not tB else 2.0
+    A[:, :] *= np.float32(0.125)
+    out = []
+    for algo in (X3, _lib.RH_ALGO_GATHER):
+        Cd = T(C0, dev)
+        ops.sgemm(tA, tB, m, n, k, 1.0, T(A, dev), lda, T(B, dev), ldb, 0.0, Cd, ldc, algo=algo)
+        out.append(N(Cd)[:, :m])
+    assert np.array_equal(np.isnan(out[0]), np.isnan(out[1])) and np.array_equal(np.isinf(out[0]), np.isinf(out[1]))
+    keep = np.isfinite(out[1])
+    assert np.array_equal(out[0][np.isinf(out[1])], out[1][np.isinf(out[1])])
+    assert np.all(np.abs(out[0][keep].astype(np.float64) - out[1][keep]) <= 1e-4 * (1.0 + np.abs(out[1][keep].astype(np.float64))))
+
+
+def test_sgemm_bf16x3_where_it_pays(dev):
+    """RH_ALGO_BF16X3 alone: the form on large affine products, with no larger error against 64-bit sums than the form that it
+    replaces, half of the activations zeros; the other forms' bits elsewhere and where the scratch does not hold it."""
+    for tA, tB, m, n, k, takes in ((1, 0, 4096, 32, 4096, True), (1, 0, 4096, 31, 4080, False), (1, 0, 1000, 33, 4096, True), (1, 0, 512, 64, 1024, False),
+                                   (1, 0, 1000, 129, 4096, True), (1, 0, 1024, 200, 2048, False), (0, 0, 4096, 37, 1000, True), (0, 0, 4096, 256, 4096, True),
+                                   (0, 1, 4096, 4096, 50, True), (0, 1, 4096, 1000, 96, False), (0, 1, 4096, 1000, 97, True), (0, 1, 4096, 4096, 256, True),
+                                   (0, 1, 800, 500, 128, False)):
+        say("sgemm bf16x3 pays", (tA, tB, m, n, k))
+        A, B = synth.normal(17, 1, (m, k) if tA else (k, m)), synth.normal(17, 2, (k, n) if tB else (n, k))
+        B = np.maximum(B, 0.0)
+        Ad, Bd, C = T(A, dev), T(B, dev), torch.empty(n, m, device=dev)
+        run = lambda algo, ws=True: N(ops.sgemm(tA, tB, m, n, k, 1.0, Ad, A.shape[1], Bd, B.shape[1], 0.0, C, m, use_workspace=ws, algo=algo)).copy()
+        got, tags = profile_tags(lambda: run(_lib.RH_ALGO_BF16X3))
+        assert any(t.startswith("sgemm_tri_") for t in tags) == takes, ((tA, tB, m, n, k), tags)
+        before = run(0)
+        exact = (B.T if tB else B).astype(np.float64) @ (A.T if tA else A).astype(np.float64)
+        assert np.linalg.norm(got - exact) <= np.linalg.norm(before - exact), (tA, tB, m, n, k)
+        if not takes:
+            assert np.array_equal(got, before)
+        assert np.array_equal(run(_lib.RH_ALGO_BF16X3, False), run(0, False))
+
+
+def test_sgemm_bf16x3_refused(dev):
+    """No such form: both operands transposed, m no multiple of 4, k no multiple of 16 with A transposed, A or lda not aligned."""
+    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
+    buf = torch.zeros(1 << 16, device=dev)
+    ws = torch.empty(1 << 20, dtype=torch.uint8, device=dev)
+    for tA, tB, m, n, k, lda, shift in ((1, 1, 64, 64, 64, 64, 0), (0, 0, 66, 8, 16, 68, 0), (1, 0, 64, 8, 24, 24, 0), (1, 0, 64, 8, 32, 33, 0), (0, 0, 64, 8, 16, 64, 1)):
+        C = torch.full((n, m), 7.0, device=dev)
+        rc = _lib.lib().rh_sgemm(tA, tB, m, n, k, 1.0, buf.data_ptr() + 4 * shift, lda, buf.data_ptr(), max(n, k), 0.0, C.data_ptr(), m,
+                                 ws.data_ptr(), ws.numel(), X3, None)
+        assert rc == _lib.RH_E_UNSUPPORTED, (tA, tB, m, n, k, rc)
+        torch.cuda.synchronize()
+        assert bool((C == 7.0).all())
+
+
 def test_bias_relu(dev):
     for shape in [(3, 7, 5, 9), (2, 96, 27, 27), (64, 500), (5, 3, 16, 20)]:
         say("bias/relu", shape)
