@@ -144,7 +144,7 @@ __device__ __forceinline__ float tri_dot(const TriParams& a, const TriParams& b,
     const uint16_t* qb = reinterpret_cast<const uint16_t*>(pb + (B_LINEAR ? g * b.v.group_stride : b.v.soff[g]));
     auto value = [](const uint16_t* q, int plane, int e) {
       auto part = [&](int i) { return __builtin_bit_cast(float, (uint32_t)q[(size_t)i * (plane / 2) + e] << 16); };
-      return (part(0) + part(1)) + part(2);
+      return part(0) + (part(1) + part(2));   // (exact; the largest floats' first two parts add up to 2^128)
     };
     for (int e = 0; e < 8; ++e) sum = fmaf(value(qa, a.plane, e), value(qb, b.plane, e), sum);
   }

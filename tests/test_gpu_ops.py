@@ -629,6 +629,15 @@ def test_conv2d_bf16x3_infinities_and_largest_floats(dev):
         assert bool(((got - ref).abs()[keep] <= 1e-4 * (1.0 + ref.abs()[keep])).all())
 
 
+def test_conv2d_bf16x3_largest_floats_beside_an_infinity(dev):
+    """A result that is formed again in fp32 because of an infinity takes the largest floats as they are: their first two parts add
+    up to 2^128, and an infinity of the other sign would make a NaN of the result."""
+    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
+    x, w = torch.full((1, 8, 4, 4), -0.125, device=dev), torch.full((16, 8, 1, 1), 0.5, device=dev)
+    x[0, 0], w[:, 1] = float("inf"), torch.finfo(torch.float32).max
+    assert bool((ops.conv2d_fwd(x, w, 1, 0, algo=X3) == float("inf")).all())
+
+
 def test_conv2d_bf16x3_where_it_pays(dev):
     """RH_ALGO_BF16X3 alone: the form where it is expected to be the fastest, and the others' bits elsewhere."""
     for (Nn, C, H, K, R, st, pad), takes in (((37, 256, 13, 384, 3, 1, 1), True), ((24, 128, 28, 256, 3, 2, 1), True), ((8, 96, 27, 256, 5, 1, 2), True),
