@@ -202,6 +202,28 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
   if (pp.ok && !(flags & RH_ALGO_GATHER)) {
     if (mask) return RH_E_UNSUPPORTED;
     if (d.x_elems == 0) return 0;
+    PhaseTable tab;
+    for (int i = 0; i < d.st * d.st; ++i) {
+      const PhaseGeom& g = pp.ph[i];
+      tab.u0[i] = g.u0; tab.U[i] = g.U; tab.v0[i] = g.v0; tab.V[i] = g.V;
+      tab.off[i] = g.Ra > 0 && g.Sb > 0 && g.U > 0 && g.V > 0 ? g.sub_off : -1;
+    }
+    auto interleave = [&](const float* sub) -> int {
+      ProfScope prof("phase_interleave", 8.0 * (double)d.x_elems, stream);
+      hipLaunchKernelGGL(phase_interleave_kernel, dim3(stream_grid((size_t)(d.x_elems + 3) / 4, 256)), dim3(256), 0, stream, sub, dx,
+                         (unsigned)d.x_elems, FastDiv((uint32_t)d.W), FastDiv((uint32_t)d.H), FastDiv((uint32_t)d.st), d.st, d.pad,
+                         tab, alpha, beta);
+      return launch_status();
+    };
+    if (tri_allowed(flags)) {
+      const TriPhasePlan tp = plan_tri_phases(d, pp);
+      if (tp.ok) {
+        if (ws_bytes < tp.total()) return RH_E_WORKSPACE;
+        float* sub;
+        const int e = launch_conv_tri_phases(d, pp, tp, w, dy, ws, stream, &sub);
+        return e ? e : interleave(sub);
+      }
+    }
     char* base = static_cast<char*>(ws);
     int* soff = reinterpret_cast<int*>(base);
     float* wT = reinterpret_cast<float*>(base + pp.tab_bytes);
@@ -215,14 +237,11 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
       img = dyp;
     }
     const size_t img_floats = (size_t)d.N * d.K * pp.Hp * pp.Wp;
-    PhaseTable tab;
     for (int a = 0; a < d.st; ++a)
       for (int b = 0; b < d.st; ++b) {
         const int i = a * d.st + b;
         const PhaseGeom& g = pp.ph[i];
-        const bool live = g.Ra > 0 && g.Sb > 0 && g.U > 0 && g.V > 0;
-        tab.u0[i] = g.u0; tab.U[i] = g.U; tab.v0[i] = g.v0; tab.V[i] = g.V; tab.off[i] = live ? g.sub_off : -1;
-        if (!live) continue;
+        if (tab.off[i] < 0) continue;
         const int k_true = d.K * g.Ra * g.Sb, n_k = round_up(k_true, kTabPad);
         hipLaunchKernelGGL(prep_bwd_data_phase_kernel, dim3(stream_grid((size_t)n_k * d.C, 256)), dim3(256), 0, stream, w, wT,
                            soff, n_k, k_true, d.C, d.R, d.S, d.st, a, b, g.Ra, g.Sb, pp.Hp * pp.Wp, pp.Wp);
@@ -250,11 +269,7 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
         }
         if (e) return e;
       }
-    ProfScope prof("phase_interleave", 8.0 * (double)d.x_elems, stream);
-    hipLaunchKernelGGL(phase_interleave_kernel, dim3(stream_grid((size_t)(d.x_elems + 3) / 4, 256)), dim3(256), 0, stream, sub, dx,
-                       (unsigned)d.x_elems, FastDiv((uint32_t)d.W), FastDiv((uint32_t)d.H), FastDiv((uint32_t)d.st), d.st, d.pad,
-                       tab, alpha, beta);
-    return launch_status();
+    return interleave(sub);
   }
   const SoffPlan sp = plan_soff_bwd_data(d);
   if (sp.ok && !(flags & RH_ALGO_GATHER)) {

@@ -878,7 +878,11 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
       const size_t legacy = align256(sizeof(int4) * (size_t)round_up(KRS, kTabPad)) +
                             align256(sizeof(int) * (size_t)round_up(KRS, kTabPad));
       const PhasePlan pp = plan_phase_bwd_data(d);
-      if (pp.ok) return pp.total() > legacy ? pp.total() : legacy;
+      if (pp.ok) {
+        const TriPhasePlan xp = plan_tri_phases(d, pp);
+        const size_t most = xp.ok && xp.total() > pp.total() ? xp.total() : pp.total();
+        return most > legacy ? most : legacy;
+      }
       const SoffPlan sp = plan_soff_bwd_data(d);
       size_t need = sp.ok && sp.total() > legacy ? sp.total() : legacy;
       if (wino_shape(d)) {

@@ -792,6 +792,54 @@ inline PhasePlan plan_phase_bwd_data(const ConvDims& d) {
   return p;
 }
 
+// The residue classes with exactly split operands (conv_tri.hip): one copy of dy, the sub-filters of all classes, one launch for
+// all contractions.  ok where it is expected to pay and where no class has a longer chain of sums than tri_max_chain allows.
+struct TriPhasePlan {
+  bool ok;
+  int bm, groups;   // groups of eight k of all classes, each a whole number of K steps
+  size_t tab_bytes, wt_bytes, img_bytes, sub_bytes;
+  size_t total() const { return tab_bytes + wt_bytes + img_bytes + sub_bytes; }
+};
+// The other form is a preparation, a product and mostly a reduction for each class, about 10 us and its multiply-adds at 100 TFLOP/s;
+// this one copies once and launches once, so it gains most on few pixels.  3x3, stride 2, us: 64 -> 128 56x56 at 8, 24, 64, 128,
+// 256 images 93 -> 39, 124 -> 50, 176 -> 99, 274 -> 181, 521 -> 355; 128 -> 256 28x28 at 64, 128, 256 images 176 -> 78, 272 -> 121,
+// 405 -> 230; 256 -> 512 14x14 at 256 403 -> 194.  Below those batches the other form's many slices have the smaller error.
+inline TriPhasePlan plan_tri_phases(const ConvDims& d, const PhasePlan& pp) {
+  TriPhasePlan p = {};
+  if (!pp.ok || d.K % 8 != 0 || d.x_elems == 0 || d.R * d.S == 1) return p;
+  p.bm = pick_bm(d.C);
+  if (p.bm == 32) return p;
+  const int bn = p.bm == 64 ? 192 : 128;
+  double other = 30.0, us = 20.0, steps_all = 0.0, longest = 0.0;
+  for (int i = 0; i < d.st * d.st; ++i) {
+    const PhaseGeom& g = pp.ph[i];
+    const long long cols = (long long)d.N * g.U * g.V;
+    if (g.Ra * g.Sb == 0 || cols == 0) continue;
+    const int k_true = d.K * g.Ra * g.Sb, n = round_up(k_true / 8, 2) / 2;
+    // (the engine's slices, and a rounding for each slice added to those before)
+    if (n > tri_max_chain(0.0335 * k_true / g.splits + (g.splits > 1 ? 0.016 * g.splits : 0.0))) return p;
+    p.groups += 2 * n;
+    steps_all += (double)n * cdiv(d.C, p.bm) * (double)cdiv<long long>(cols, bn);
+    if (n > longest) longest = n;
+    other += 10.0 + 2.0 * (double)d.C * (double)cols * k_true / 100e6;
+  }
+  const size_t img = 6 * (size_t)d.N * d.K * pp.Hp * pp.Wp, wt = 48 * (size_t)p.groups * d.C;
+  if (p.groups == 0 || img > kMaxBufferBytes || wt > kMaxBufferBytes) return p;
+  const double step_us = p.bm == 128 ? 0.456 : 0.377;
+  us += fmax(longest * step_us, steps_all / 256.0 * step_us) + (4.0 * (double)d.y_elems + (double)img) / 5.3e6 + 12.0 * (double)d.x_elems / 5.3e6 +
+        10.0 * (double)d.w_elems / 2.2e6;
+  if (us >= other) return p;
+  p.tab_bytes = align256(sizeof(int) * (size_t)p.groups);
+  p.wt_bytes = align256(wt);
+  p.img_bytes = align256(img);
+  p.sub_bytes = pp.sub_bytes;
+  p.ok = true;
+  return p;
+}
+// Leaves the classes' results at *sub, PhaseGeom::sub_off apart.
+int launch_conv_tri_phases(const ConvDims& d, const PhasePlan& pp, const TriPhasePlan& p, const float* w, const float* dy, void* ws,
+                           hipStream_t stream, float** sub);
+
 // 1x1 / stride 1 / no padding layers with at most this many channels on both sides run on the register-resident
 // streaming kernel (conv1x1.hip) in forward and backward-data.
 constexpr int kConv1x1MaxChannels = 128;

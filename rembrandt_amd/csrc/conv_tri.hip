@@ -55,6 +55,42 @@ __device__ __forceinline__ void tri_filter_body(const TriFilterArgs& a, long lon
   }
 }
 
+// The sub-filters of all residue classes one behind the other, [class][k/8][c][8] in three parts each, and their tables; k order and
+// taps as above, a class's taps (i, j) being the filter's (a + st i, b + st j).
+struct TriClassFilter { int first, groups, groups_true, a, b, Ra, Sb; };   // groups of all classes before; of this one
+struct TriClassFilterArgs {
+  const float* w; uint4* wt; int* soff;
+  int groups, C, K, R, S, st, Wp, count;
+  TriClassFilter c[16];
+};
+__device__ __forceinline__ void tri_class_filter_body(const TriClassFilterArgs& f, long long i) {
+  if (i >= (long long)f.groups * f.C) return;
+  const int all = (int)(i / f.C), row = (int)(i - (long long)all * f.C);
+  int q = 0;
+  while (q + 1 < f.count && all >= f.c[q + 1].first) ++q;
+  const TriClassFilter c = f.c[q];
+  const int g = all - c.first, taps = c.Ra * c.Sb, pairs = f.K / 16 * taps, step = g >> 1;
+  int t, k0;
+  if (step < pairs) {
+    t = step % taps;
+    k0 = step / taps * 16 + (g & 1) * 8;
+  } else {
+    t = g - 2 * pairs;
+    k0 = f.K - 8;
+  }
+  const bool live = g < c.groups_true;
+  const int ti = live ? t / c.Sb : 0, tj = live ? t - ti * c.Sb : 0;
+  float v[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e)
+    v[e] = live ? f.w[(((size_t)(k0 + e) * f.C + row) * f.R + (c.a + f.st * ti)) * f.S + (c.b + f.st * tj)] : 0.0f;
+  tri_store(f.wt + (size_t)c.first * 3 * f.C, (size_t)g * f.C + row, (size_t)c.groups * f.C, v);
+  if (row == 0) f.soff[all] = live ? (((c.Ra - 1 - ti) * (f.K / 8) + k0 / 8) * f.Wp + (c.Sb - 1 - tj)) * 16 : 0;
+}
+__global__ __launch_bounds__(256) void tri_class_filter_kernel(TriClassFilterArgs f) {
+  tri_class_filter_body(f, (long long)blockIdx.x * 256 + threadIdx.x);
+}
+
 // x [n][C][H][W] -> [n][Hp][C/8][Wp][8], a thread per group, and behind it the filter copy, which is independent of it: one
 // launch less in front of the contraction.  Blocks that follow one another stay on an XCD: their reads share cache lines.
 __global__ __launch_bounds__(256) void tri_image_kernel(const float* __restrict__ x, uint4* __restrict__ xt, unsigned total, int H,
@@ -309,6 +345,83 @@ int launch_conv_tri(const TriPlan& p, bool bwd, const float* in, const float* w,
     launch_split_reduce_nchw(part, used, total - first, fin.out, total, fin.inner, fin.rows, fin.alpha, fin.beta, fin.bias, fin.relu,
                              stream, p.splits > 1 ? 0 : p.tail.col0, fin.mask);
   return launch_status();
+}
+
+int launch_conv_tri_phases(const ConvDims& d, const PhasePlan& pp, const TriPhasePlan& p, const float* w, const float* dy, void* ws,
+                           hipStream_t stream, float** sub) {
+  char* base = static_cast<char*>(ws);
+  int* soff = reinterpret_cast<int*>(base);
+  uint4* wt = reinterpret_cast<uint4*>(base + p.tab_bytes);
+  uint4* xt = reinterpret_cast<uint4*>(base + p.tab_bytes + p.wt_bytes);
+  *sub = reinterpret_cast<float*>(base + p.tab_bytes + p.wt_bytes + p.img_bytes);
+  const int order_max = d.st * d.st;
+  int order[16], count = 0;
+  for (int i = 0; i < order_max; ++i) {
+    const PhaseGeom& g = pp.ph[i];
+    if (g.Ra * g.Sb == 0 || g.U <= 0 || g.V <= 0) continue;
+    int at = count++;   // longest first
+    for (; at > 0 && pp.ph[order[at - 1]].Ra * pp.ph[order[at - 1]].Sb < g.Ra * g.Sb; --at) order[at] = order[at - 1];
+    order[at] = i;
+  }
+  const int tm = p.bm, tn = p.bm == 64 ? 192 : 128;
+  TriClassFilterArgs f;
+  TriClasses t;
+  f.w = w; f.wt = wt; f.soff = soff; f.groups = p.groups; f.C = d.C; f.K = d.K; f.R = d.R; f.S = d.S; f.st = d.st; f.Wp = pp.Wp; f.count = count;
+  t.count = count; t.tiles_m = cdiv(d.C, tm);
+  int groups = 0, tiles = 0;
+  double flops = 0.0;
+  for (int q = 0; q < count; ++q) {
+    const PhaseGeom& g = pp.ph[order[q]];
+    TriClassFilter& c = f.c[q];
+    c.first = groups; c.groups_true = d.K / 8 * g.Ra * g.Sb; c.groups = round_up(c.groups_true, 2);
+    c.a = order[q] / d.st; c.b = order[q] % d.st; c.Ra = g.Ra; c.Sb = g.Sb;
+    TriClass& k = t.c[q];
+    k.first_tile = tiles; k.steps = c.groups / 2; k.groups_true = c.groups_true;
+    k.inner = g.U * g.V; k.innerW = g.V; k.cols = d.N * k.inner;
+    k.wt_at = (uint32_t)(48 * (size_t)groups * d.C);
+    k.img_at = (uint32_t)(16 * ((size_t)(g.u0 + pp.L - (g.Ra - 1)) * (d.K / 8) * pp.Wp + (size_t)(g.v0 + pp.L - (g.Sb - 1))));
+    k.soff_at = groups;
+    k.out_at = g.sub_off;
+    groups += c.groups;
+    tiles += t.tiles_m * cdiv(k.cols, tn);
+    flops += 12.0 * (double)d.C * k.cols * d.K * g.Ra * g.Sb;
+  }
+  if (groups != p.groups) return RH_E_INVALID;
+  const size_t img_groups = (size_t)d.N * (d.K / 8) * pp.Hp * pp.Wp;
+  {
+    const unsigned img_blocks = (unsigned)cdiv<size_t>(img_groups, 256);
+    ProfScope prof("tri_image", 4.0 * (double)d.y_elems + 48.0 * (double)img_groups, stream);
+    hipLaunchKernelGGL(tri_image_kernel, dim3(img_blocks), dim3(256), 0, stream, dy, xt, (unsigned)img_groups, d.P, d.Q,
+                       FastDiv((uint32_t)pp.Wp), FastDiv((uint32_t)(d.K / 8)), FastDiv((uint32_t)pp.Hp), pp.L, (int)img_blocks, TriFilterArgs{});
+  }
+  if (int e = launch_status()) return e;
+  hipLaunchKernelGGL(tri_class_filter_kernel, dim3((unsigned)cdiv<long long>((long long)groups * d.C, 256)), dim3(256), 0, stream, f);
+  if (int e = launch_status()) return e;
+  TriParams ap, bp;
+  ap.v.ptr = wt; ap.plane = 0; ap.v.bytes = 0;   // (a class's)
+  ap.v.M = d.C; ap.v.inner = 1; ap.v.innerW = 1; ap.v.img_stride = 16; ap.v.a_stride = 0; ap.v.b_stride = 0;
+  ap.v.soff = nullptr; ap.v.group_stride = d.C * 16;
+  bp.v.ptr = xt; bp.plane = (int)(16 * img_groups); bp.v.bytes = (uint32_t)(48 * img_groups);
+  bp.v.M = 0; bp.v.inner = 1; bp.v.innerW = 1;
+  bp.v.img_stride = pp.Hp * pp.Wp * d.K * 2; bp.v.a_stride = (d.K / 8) * pp.Wp * 16; bp.v.b_stride = 16;
+  bp.v.soff = soff; bp.v.group_stride = 0;
+  EpiParams ep;
+  ep.out = *sub; ep.bias = nullptr; ep.alpha = 1.0f; ep.beta = 0.0f;
+  ep.rows = d.C; ep.cols = 0; ep.inner = 1; ep.ld = 0; ep.relu = 0; ep.split_stride = 0;
+  auto launch = [&](auto* tag, auto tile) -> int {
+    typedef decltype(tile) T;
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm_tri_classes_kernel<T>),
+                                                       hipFuncAttributeMaxDynamicSharedMemorySize, kTriLdsBytes);
+    if (attr != hipSuccess) return (int)attr;
+    ProfScope prof(tag, flops, stream);
+    hipLaunchKernelGGL((mfma_gemm_tri_classes_kernel<T>), dim3((unsigned)tiles), dim3(T::NT), kTriLdsBytes, stream, ap, bp, ep, t);
+    return launch_status();
+  };
+  switch (p.bm) {
+    case 128: return launch("conv_bwd_data_tri_128x128", T128x128t());
+    case 96: return launch("conv_bwd_data_tri_96x128", T96x128t());
+    default: return launch("conv_bwd_data_tri_64x192", T64x192t());
+  }
 }
 
 TriFilterPlan plan_tri_bwd_filter(const ConvDims& d) {

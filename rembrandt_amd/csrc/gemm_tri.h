@@ -160,9 +160,10 @@ __device__ __forceinline__ float tri_dot(const TriParams& a, const TriParams& b,
 constexpr int kTriRing = 3;
 constexpr int kTriLdsBytes = kTriRing * 6 * 16 * 256;
 
-template <class T, bool B_LINEAR, bool NCHW, class PASS>
-__global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_kernel(TriParams ap, TriParams bp, EpiParams ep, int tiles_m,
-                                                                      int k_steps, int steps_per_split, int groups) {
+// K steps [s_begin, s_end) of the tile at (m0, n0).
+template <class T, bool B_LINEAR, bool NCHW>
+__device__ __forceinline__ void tri_block(const TriParams& ap, const TriParams& bp, const EpiParams& ep, int m0, int n0, int s_begin,
+                                          int s_end, int groups, int dst_split) {
   constexpr int TM = T::TM, TN = T::TN, R = kTriRing, RA = (T::BM + 63) / 64 * 64, RBn = (T::BN + 63) / 64 * 64;
   static_assert(T::NT == 4 * kWave && T::BK == 16, "four waves, 16 k a step");
   static_assert(kTriLdsBytes >= TN * 16 * 4 * kWave * 4, "a row of blocks fits the ring");
@@ -176,35 +177,6 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_kernel(TriParams 
   const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
   const int wm = wave % T::WM, wn = wave / T::WM;
 
-  int slice, logical, dst_split;   // as in mfma_gemm_kernel
-  if (ep.tail_tiles > 0) {
-    const int b = blockIdx.x;
-    if (b < ep.full_tiles) {
-      logical = xcd_remap(b, ep.full_tiles);
-      slice = 0;
-      dst_split = -1;
-    } else {
-      const int r = xcd_remap(b - ep.full_tiles, ep.tail_tiles * ep.tail_splits);
-      slice = r / ep.tail_tiles;
-      logical = ep.full_tiles + (r - slice * ep.tail_tiles);
-      dst_split = slice;
-    }
-  } else {
-    const int tiles = gridDim.x;
-    const int linear = xcd_remap(blockIdx.y * tiles + blockIdx.x, tiles * gridDim.y);
-    slice = linear / tiles;
-    logical = linear - slice * tiles;
-    dst_split = ep.split_stride != 0 ? slice : -1;
-  }
-  slice = __builtin_amdgcn_readfirstlane(slice);
-  logical = __builtin_amdgcn_readfirstlane(logical);
-  dst_split = __builtin_amdgcn_readfirstlane(dst_split);
-  const int tile_m = logical % tiles_m, tile_n = logical / tiles_m;
-  const int m0 = tile_m * T::BM, n0 = tile_n * T::BN;
-  const bool whole = ep.tail_tiles > 0 && dst_split < 0;
-  const int s_begin = whole ? 0 : slice * steps_per_split;
-  int s_end = whole ? k_steps : s_begin + steps_per_split;
-  if (s_end > k_steps) s_end = k_steps;
   const int nk = s_end - s_begin;
 
   Loader ld;
@@ -336,6 +308,73 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_kernel(TriParams 
     }
   }
   store_tile<T, NCHW>(acc, ep, m0, n0, wm, wn, lane, dst_split);
+}
+
+template <class T, bool B_LINEAR, bool NCHW, class PASS>
+__global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_kernel(TriParams ap, TriParams bp, EpiParams ep, int tiles_m,
+                                                                      int k_steps, int steps_per_split, int groups) {
+  int slice, logical, dst_split;   // as in mfma_gemm_kernel
+  if (ep.tail_tiles > 0) {
+    const int b = blockIdx.x;
+    if (b < ep.full_tiles) {
+      logical = xcd_remap(b, ep.full_tiles);
+      slice = 0;
+      dst_split = -1;
+    } else {
+      const int r = xcd_remap(b - ep.full_tiles, ep.tail_tiles * ep.tail_splits);
+      slice = r / ep.tail_tiles;
+      logical = ep.full_tiles + (r - slice * ep.tail_tiles);
+      dst_split = slice;
+    }
+  } else {
+    const int tiles = gridDim.x;
+    const int linear = xcd_remap(blockIdx.y * tiles + blockIdx.x, tiles * gridDim.y);
+    slice = linear / tiles;
+    logical = linear - slice * tiles;
+    dst_split = ep.split_stride != 0 ? slice : -1;
+  }
+  slice = __builtin_amdgcn_readfirstlane(slice);
+  logical = __builtin_amdgcn_readfirstlane(logical);
+  dst_split = __builtin_amdgcn_readfirstlane(dst_split);
+  const int tile_m = logical % tiles_m, tile_n = logical / tiles_m;
+  const int m0 = tile_m * T::BM, n0 = tile_n * T::BN;
+  const bool whole = ep.tail_tiles > 0 && dst_split < 0;
+  const int s_begin = whole ? 0 : slice * steps_per_split;
+  int s_end = whole ? k_steps : s_begin + steps_per_split;
+  if (s_end > k_steps) s_end = k_steps;
+  tri_block<T, B_LINEAR, NCHW>(ap, bp, ep, m0, n0, s_begin, s_end, groups, dst_split);
+}
+
+// Backward-data of stride 2 to 4 (conv_common.h: residue classes): the classes' contractions in one launch, the longest first, so that
+// the short ones fill the last round (launched one by one the classes of 64 -> 128 56x56 b24 are 98 tiles each on 256 CUs).  Bound by
+// the MFMAs as above and by the classes' results, which a second pass interleaves.
+struct TriClass {
+  int first_tile, steps, groups_true;
+  int cols, inner, innerW;   // n U V, U V, V
+  uint32_t wt_at, img_at;    // bytes into the operand copies: the class's filter, its first pixel at its first tap
+  int soff_at;
+  long long out_at;          // floats
+};
+struct TriClasses { int count, tiles_m; TriClass c[16]; };
+template <class T>
+__global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_classes_kernel(TriParams ap, TriParams bp, EpiParams ep, TriClasses t) {
+  const int block = blockIdx.x;
+  int i = 0;
+  while (i + 1 < t.count && block >= t.c[i + 1].first_tile) ++i;
+  i = __builtin_amdgcn_readfirstlane(i);
+  const TriClass c = t.c[i];
+  const int tiles = (i + 1 < t.count ? t.c[i + 1].first_tile : (int)gridDim.x) - c.first_tile;
+  const int logical = __builtin_amdgcn_readfirstlane(xcd_remap(block - c.first_tile, tiles));
+  ap.v.ptr = static_cast<const char*>(ap.v.ptr) + c.wt_at;
+  ap.plane = c.steps * 2 * ap.v.M * 16;
+  ap.v.bytes = (uint32_t)(3 * ap.plane);
+  bp.v.ptr = static_cast<const char*>(bp.v.ptr) + c.img_at;
+  bp.v.bytes -= c.img_at;
+  bp.v.M = c.cols; bp.v.inner = c.inner; bp.v.innerW = c.innerW;
+  bp.v.soff += c.soff_at;
+  ep.out += c.out_at;
+  ep.cols = c.cols; ep.inner = c.inner;
+  tri_block<T, false, true>(ap, bp, ep, logical % t.tiles_m * T::BM, logical / t.tiles_m * T::BN, 0, c.steps, c.groups_true, -1);
 }
 
 }  // namespace rh

@@ -582,6 +582,50 @@ def test_conv2d_bf16x3(dev, case):
     assert torch.equal(ops.conv2d_bwd_filter(xd, dyd, w.shape, st, pad, algo=X3), dw), "run to run the same bits"
 
 
+# Backward-data of stride 2 to 4 by residue classes in the split-operand form: odd extents (classes of different sizes), classes
+# without taps (a filter smaller than the stride) and without pixels, an odd number of groups (8, 24, 40 filters), rows past the
+# 64-, 96- and 128-row tiles, one to many tiles a class, no padding and more than the filter needs.
+X3_STRIDED_CASES = [
+    # N, C, H, W, K, R, stride, pad
+    (3, 64, 9, 7, 40, 3, 2, 1),
+    (1, 65, 1, 5, 8, 3, 2, 1),
+    (2, 96, 13, 12, 24, 5, 2, 2),
+    (1, 128, 11, 11, 8, 7, 3, 3),
+    (5, 70, 10, 9, 16, 3, 2, 0),
+    (2, 64, 17, 16, 64, 2, 4, 0),
+    (9, 250, 14, 15, 72, 5, 4, 1),
+    (4, 64, 8, 8, 64, 3, 2, 3),
+    (24, 64, 56, 56, 128, 3, 2, 1),
+]
+
+
+@pytest.mark.parametrize("case", X3_STRIDED_CASES, ids=str)
+def test_conv2d_bf16x3_strided_bwd_data(dev, case):
+    """Against the oracle and no further from its sums than the form it replaces; the alpha / beta blend; infinities."""
+    Nn, C, H, W, K, R, st, pad = case
+    say("bf16x3 strided bwd data", case)
+    X3 = _lib.RH_ALGO_BF16X3
+    P, Q = (H + 2 * pad - R) // st + 1, (W + 2 * pad - R) // st + 1
+    w, dy, dx0 = synth.normal(41, 1, (K, C, R, R)), synth.normal(41, 2, (Nn, K, P, Q)), synth.normal(41, 3, (Nn, C, H, W))
+    wd, dyd = T(w, dev), T(dy, dev)
+    got, tags = profile_tags(lambda: ops.conv2d_bwd_data(wd, dyd, dx0.shape, st, pad, algo=X3))
+    assert any(t.startswith("conv_bwd_data_tri_") for t in tags), tags
+    ref = O.conv2d_bwd_data(w, dy, dx0.shape, st, pad)
+    assert_close(N(got), ref, "strided bf16x3")
+    before = ops.conv2d_bwd_data(wd, dyd, dx0.shape, st, pad)
+    # (of the oracle's sums, which are in 64 bits and then rounded; 1e-8: what that rounding moves, at most half an ulp)
+    err, old = (float(np.linalg.norm(N(t).astype(np.float64) - ref) / np.linalg.norm(ref.astype(np.float64))) for t in (got, before))
+    assert err <= old + 1e-8, (err, old)
+    blend = ops.conv2d_bwd_data(wd, dyd, dx0.shape, st, pad, alpha=0.5, beta=2.0, dx=T(dx0, dev), algo=X3)
+    assert_close(N(blend), O.conv2d_bwd_data(w, dy, dx0.shape, st, pad, 0.5, 2.0, dx0.copy()), "strided bf16x3 alpha/beta")
+    # (products with the largest float stay in range, |dy| < 8 / 8: a finite overflow beside an infinity of the other sign is -inf, inf
+    # or NaN by the order of the additions)
+    dy *= np.float32(0.125)
+    dy[0, 0, 0, 0], w[-1, -1, 0, 0] = np.inf, np.finfo(np.float32).max
+    a, b = (ops.conv2d_bwd_data(T(w, dev), T(dy, dev), dx0.shape, st, pad, algo=f) for f in (X3, _lib.RH_ALGO_GATHER))
+    assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isinf(a), torch.isinf(b))
+
+
 @pytest.mark.parametrize("relu", [False, True], ids=["normal", "half_zeros"])
 @pytest.mark.parametrize("case", [(16, 256, 13, 13, 384, 3, 1), (64, 128, 28, 28, 128, 3, 1), (9, 96, 27, 27, 256, 5, 2), (32, 64, 28, 28, 64, 3, 1)], ids=str)
 def test_conv2d_bf16x3_error(dev, case, relu):
