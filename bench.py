@@ -101,7 +101,9 @@ def collect_profile(lib, steps):
             continue
         if mfma:
             achieved, unit = work / ms / 1e9, "TFLOP/s"
-            peak = PEAK_BF16_MFMA_TFLOPS if name.startswith("conv_fwd_bf16") else PEAK_FP32_MFMA_TFLOPS
+            # (the split-operand kernels execute six bf16 products for an fp32 one, and report those)
+            bf16 = name.startswith("conv_fwd_bf16") or "_tri_" in name
+            peak = PEAK_BF16_MFMA_TFLOPS if bf16 else PEAK_FP32_MFMA_TFLOPS
         else:
             achieved, peak, unit = work / ms / 1e6, PEAK_HBM_GBS, "GB/s"
         out.append({"kernel": name, "bound": "mfma" if mfma else "hbm", "launches_per_step": count / steps,
@@ -291,7 +293,7 @@ def short_train_leg(lib, name, steps, warmup):
             "launches_per_step": sum(k["launches_per_step"] for k in kernels),
             "gemm_gflop_per_step": flops / 1e9,
             "step_frac_of_mfma_peak": flops / (dt / steps) / 1e12 / PEAK_FP32_MFMA_TFLOPS,
-            "all_mfma": {"ms_per_step": mfma_ms, "frac": executed / mfma_ms / 1e9 / PEAK_FP32_MFMA_TFLOPS if mfma_ms else None},
+            "all_mfma": {"ms_per_step": mfma_ms, "executed_gflop_per_step": executed / 1e9, "frac": _mfma_frac(kernels)},
             "roofline": _roof(_dominant(kernels))}
 
 
@@ -388,6 +390,13 @@ def _executed_flops(kernels):
     """FLOPs per step that the contraction kernels execute: what the kernels report as their work (the Winograd
     kernels 16 multiply-adds per 2x2 tile, filter and channel, where the direct form's count has 36)."""
     return sum(k["achieved"] * 1e9 * k["ms_per_step"] for k in kernels if k["bound"] == "mfma")
+
+
+def _mfma_frac(kernels):
+    """Share of the matrix peak, each contraction kernel's own, over the time of all of them."""
+    mfma = [k for k in kernels if k["bound"] == "mfma"]
+    ms = sum(k["ms_per_step"] for k in mfma)
+    return sum(k["frac"] * k["ms_per_step"] for k in mfma) / ms if ms else None
 
 
 def conv_sweep_leg(iters, warmup):
@@ -613,11 +622,12 @@ def main():
                      "traffic": traffic,
                      "traffic_unit": "bytes per launch (L2<->fabric, FETCH_SIZE + WRITE_SIZE counters)",
                      "traffic_source": traffic_source, **_wino_note(net, batch, dom)},
-        # all contraction kernels together: executed FLOPs (the Winograd kernels' own count) against the matrix peak;
+        # all contraction kernels together: executed FLOPs (the Winograd and split-operand kernels' own count); each kernel's
+        # against the peak of its instruction, fp32 or bf16;
         # `direct_form_tflops` prices the same time in the direct form's multiply-adds (config.gemm_gflop_per_step)
         "all_mfma": {"ms_per_step": gemm_ms, "executed_gflop_per_step": _executed_flops(mfma) / 1e9,
                      "achieved": _executed_flops(mfma) / gemm_ms / 1e9 if gemm_ms else None,
-                     "unit": "TFLOP/s", "frac": _executed_flops(mfma) / gemm_ms / 1e9 / PEAK_FP32_MFMA_TFLOPS if gemm_ms else None,
+                     "unit": "TFLOP/s", "frac": _mfma_frac(mfma),
                      "direct_form_tflops": gemm_flops / gemm_ms / 1e9 if gemm_ms else None},
         "calibration": calibration,
         "kernels_note": "per-kernel table from an untimed pass of %d steps with HIP events on every launch and the "
