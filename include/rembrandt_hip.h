@@ -63,7 +63,10 @@ typedef void* rh_stream_t; /* hipStream_t */
                                              are sliced with the hint as without.  Same result up to summation order. */
 #define RH_ALGO_BF16X3             0x2000 /* the contraction may also run on bf16 matrix instructions, every fp32 operand value as
                                              the exact sum of three bf16 values (six products a pair, fp32 accumulate): fp32
-                                             precision, no operand is rounded.  Alone or with the hint: where it is expected to
+                                             precision, no operand is rounded.  Results with an operand that has no such sum
+                                             (an infinity, a NaN, a float that rounds to an infinity in bf16, one below 2^-110
+                                             with bits under bf16's smallest value, 2^-133) are formed on fp32 instructions, at
+                                             4 to 8 times the time where all are.  Alone or with the hint: where it is expected to
                                              be the fastest form.  With RH_ALGO_DIRECT: this form, RH_E_UNSUPPORTED where the
                                              geometry has none (forward and stride-1 backward-data need a contracted channel
                                              count that is a multiple of 8).  No effect beside the other RH_ALGO_* bits and

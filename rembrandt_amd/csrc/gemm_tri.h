@@ -1,8 +1,8 @@
 // fp32 contractions on the bf16 matrix instructions: every operand value is the sum of three bf16 values.
 //
 // v_mfma_f32_32x32x2_f32 executes 256 FLOP per cycle and SIMD, v_mfma_f32_32x32x16_bf16 sixteen times that.  An fp32
-// value a is exactly a1 + a2 + a3 with a1 = bf16(a), a2 = bf16(a - a1), a3 = a - a1 - a2 (8 + 8 + 8 significand bits;
-// bf16 has the exponent range of fp32, so nothing is scaled), the product of two bf16 values is exact in fp32, and of the
+// value a is exactly a1 + a2 + a3 with a1 = bf16(a), a2 = bf16(a - a1), a3 = a - a1 - a2 (8 + 8 + 8 significand bits; for
+// all values but those below), the product of two bf16 values is exact in fp32, and of the
 // nine products of a pair the three below 2^-24 of it (a2 b3, a3 b2, a3 b3) are left out: six MFMAs do the work of
 // eight times 16 / 2 fp32 ones in 6/16 of their time.  Registers only, six products on random data: 302 TFLOP/s of fp32
 // multiply-adds (1.81 PFLOP/s of bf16 at the clock it settles at) where the fp32 instruction reaches 154.
@@ -12,8 +12,10 @@
 // 3456 terms against 64 bits, N(0,1) data: 0.9e-7, 2.0e-7 and 3.6e-7, the fp32 instruction 2.9e-7, 6.1e-7 and 10.4e-7 (with
 // one set of accumulators 2.4e-7, 5.2e-7 and 9.2e-7, and above the fp32 instruction where half of one operand is zero).
 //
-// Infinities.  The parts of an infinity are (inf, 0, 0), and inf * 0 makes a NaN where fp32 multiplication has none.  So a
-// result that is not finite is computed again from the parts (whose sum is the operand), term by term in fp32.
+// Values without such a sum: infinities and NaNs, the floats that round to an infinity in bf16, and below 2^-110 those whose
+// last bits lie under bf16's smallest value, 2^-133 (their parts would lose 2^-14 of them at 2^-120, all of them under 2^-134).
+// Their first part is a NaN and the other two hold their bits, so every result that has one among its operands comes out as
+// a NaN, and a result that is not finite is formed again from the operands' values on the fp32 instruction (tri_redo).
 #pragma once
 #include "gemm_core.h"
 
@@ -27,9 +29,10 @@ struct TriParams {
 };
 
 // Eight values (one group) into the three parts' groups: pair() for each of the four pairs, then fix().
+constexpr uint32_t kTriNoSum = 0x7fc0u;   // first part of a value that is no sum of three
 struct TriPack8 {
   uint32_t w[3][4];
-  float rest = 0.0f;
+  uint32_t rest = 0;
   __device__ __forceinline__ void pair(const float (&v)[8], int e) {
     float x = v[2 * e], y = v[2 * e + 1];
 #pragma unroll
@@ -38,34 +41,33 @@ struct TriPack8 {
       x -= __builtin_bit_cast(float, w[i][e] << 16);
       y -= __builtin_bit_cast(float, w[i][e] & 0xffff0000u);
     }
-    rest += x + y;   // zeros, or a NaN where a first part is no number
+    rest |= __builtin_bit_cast(uint32_t, x) | __builtin_bit_cast(uint32_t, y);   // (+0 where the parts add up to the value)
   }
   __device__ __forceinline__ void fix(const float (&v)[8]) {
-    if (rest == 0.0f) return;
-    // infinities and NaNs have no further parts; the largest floats, which round to an infinity, are cut off instead
+    if (rest == 0) return;
 #pragma unroll
     for (int e = 0; e < 4; ++e) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
-        const float x = v[2 * e + h];
-        const uint32_t bits = __builtin_bit_cast(uint32_t, x), mag = bits & 0x7fffffffu;
-        if (mag <= 0x7f7f7fffu) continue;
-        uint32_t p = bits >> 16, q = 0, r = 0;
-        if (mag > 0x7f800000u) p |= 0x40u;
-        if (mag < 0x7f800000u) {
-          const float t = x - __builtin_bit_cast(float, p << 16);
-          q = pack_bf16(t, 0.0f) & 0xffffu;
-          r = pack_bf16(t - __builtin_bit_cast(float, q << 16), 0.0f) & 0xffffu;
-        }
+        const uint32_t bits = __builtin_bit_cast(uint32_t, v[2 * e + h]);
         const uint32_t keep = h ? 0xffffu : 0xffff0000u, sh = 16 * h;
-        w[0][e] = (w[0][e] & keep) | (p << sh);
-        w[1][e] = (w[1][e] & keep) | (q << sh);
-        w[2][e] = (w[2][e] & keep) | (r << sh);
+        float x = v[2 * e + h];
+#pragma unroll
+        for (int i = 0; i < 3; ++i) x -= __builtin_bit_cast(float, h ? w[i][e] & 0xffff0000u : w[i][e] << 16);
+        if (__builtin_bit_cast(uint32_t, x) == 0) continue;
+        w[0][e] = (w[0][e] & keep) | (kTriNoSum << sh);
+        w[1][e] = (w[1][e] & keep) | ((bits >> 16) << sh);
+        w[2][e] = (w[2][e] & keep) | ((bits & 0xffffu) << sh);
       }
     }
   }
   __device__ __forceinline__ uint4 part(int i) const { return make_uint4(w[i][0], w[i][1], w[i][2], w[i][3]); }
 };
+// The value again: p, q, r its parts.
+__device__ __forceinline__ float tri_value(uint32_t p, uint32_t q, uint32_t r) {
+  const float sum = __builtin_bit_cast(float, p << 16) + (__builtin_bit_cast(float, q << 16) + __builtin_bit_cast(float, r << 16));
+  return p == kTriNoSum ? __builtin_bit_cast(float, q << 16 | r) : sum;
+}
 __device__ __forceinline__ void tri_pack8(const float (&v)[8], uint4 (&o)[3]) {
   TriPack8 t;
 #pragma unroll
@@ -129,27 +131,73 @@ struct DmaTri {
   }
 };
 
-// Element (row, col) over groups [g0, g1), from the operands' parts, in fp32.
-template <bool B_LINEAR>
-__device__ __forceinline__ float tri_dot(const TriParams& a, const TriParams& b, int row, int col, int g0, int g1) {
-  auto base = [](const RowV8Params& p, int m) {
-    const int n = m / p.inner, rem = m - n * p.inner, a2 = rem / p.innerW, b2 = rem - a2 * p.innerW;
-    return static_cast<const char*>(p.ptr) + (uint32_t)(n * p.img_stride + a2 * p.a_stride + b2 * p.b_stride);
-  };
-  const char* pa = base(a.v, row);
-  const char* pb = base(b.v, col);
-  float sum = 0.0f;
-  for (int g = g0; g < g1 && sum == sum; ++g) {   // (a NaN stays one)
-    const uint16_t* qa = reinterpret_cast<const uint16_t*>(pa + g * a.v.group_stride);
-    const uint16_t* qb = reinterpret_cast<const uint16_t*>(pb + (B_LINEAR ? g * b.v.group_stride : b.v.soff[g]));
-    auto value = [](const uint16_t* q, int plane, int e) {
-      auto part = [&](int i) { return __builtin_bit_cast(float, (uint32_t)q[(size_t)i * (plane / 2) + e] << 16); };
-      return part(0) + (part(1) + part(2));   // (exact; the largest floats' first two parts add up to 2^128)
-    };
-    for (int e = 0; e < 8; ++e) sum = fmaf(value(qa, a.plane, e), value(qb, b.plane, e), sum);
+// The block d of 32 x 32 results with its elements that are not finite and lie in the result formed again over groups
+// [g0, g1) on the fp32 instruction: load_a(g, v) and load_b(g, v) give this lane's row (lane % 32) and column their eight values of
+// group g.  Two levels of sums, 128 terms each, as the chains of K steps may be longer than fp32's rounding allows.  The whole wave
+// takes part whether one element or all of them are formed.  Bound by the latency of its own loads: 2 us for 16 k of a block, so a call
+// with one such value takes 80 to 470 us longer, one with nothing else 4 to 8 times as long (96 -> 256 5x5 27x27 b256 forward 967 us,
+// with one such value 1197, with nothing else 5150).
+template <class LA, class LB>
+__device__ __forceinline__ void tri_redo(f32x16& d, int rows_left, int cols_left, int lane, int g0, int g1, LA load_a, LB load_b) {
+  bool any = false;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) {
+    const bool in = (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3) < rows_left && (lane & 31) < cols_left;
+    any |= in && !(fabsf(d[v]) < INFINITY);
   }
-  return sum;
+  if (!__any(any)) return;
+  f32x16 sum;
+#pragma unroll
+  for (int v = 0; v < 16; ++v) sum[v] = 0.0f;
+#pragma unroll 1
+  for (int top = g0; top < g1; top += 16) {
+    f32x16 part;
+#pragma unroll
+    for (int v = 0; v < 16; ++v) part[v] = 0.0f;
+#pragma unroll 1
+    for (int g = top; g < top + 16 && g < g1; g += 2) {
+      const int mine = g + (lane >> 5);   // k 0 and 1 of an MFMA: of this group and of the next
+      float a[8], b[8];
+#pragma unroll
+      for (int e = 0; e < 8; ++e) a[e] = b[e] = 0.0f;
+      if (mine < g1) {
+        load_a(mine, a);
+        load_b(mine, b);
+      }
+#pragma unroll
+      for (int e = 0; e < 8; ++e) part = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], part, 0, 0, 0);
+    }
+    sum += part;
+  }
+#pragma unroll
+  for (int v = 0; v < 16; ++v)
+    if (!(fabsf(d[v]) < INFINITY)) d[v] = sum[v];
 }
+
+// Row (or column) m of an operand of three parts: its eight values of the group `at` bytes into it.
+struct TriRow {
+  const char* base;
+  int plane;
+  __device__ __forceinline__ TriRow(const TriParams& t, int m) : plane(t.plane) {
+    const RowV8Params& p = t.v;
+    const int mm = m < p.M ? m : 0;
+    const int n = mm / p.inner, rem = mm - n * p.inner, a2 = rem / p.innerW, b2 = rem - a2 * p.innerW;
+    base = static_cast<const char*>(p.ptr) + (uint32_t)(n * p.img_stride + a2 * p.a_stride + b2 * p.b_stride);
+  }
+  __device__ __forceinline__ void load(size_t at, float (&v)[8]) const {
+    uint32_t w[3][4];
+#pragma unroll
+    for (int i = 0; i < 3; ++i) {
+      const uint4 p = *reinterpret_cast<const uint4*>(base + at + (size_t)i * plane);
+      w[i][0] = p.x; w[i][1] = p.y; w[i][2] = p.z; w[i][3] = p.w;
+    }
+#pragma unroll
+    for (int e = 0; e < 4; ++e) {
+      v[2 * e] = tri_value(w[0][e] & 0xffffu, w[1][e] & 0xffffu, w[2][e] & 0xffffu);
+      v[2 * e + 1] = tri_value(w[0][e] >> 16, w[1][e] >> 16, w[2][e] >> 16);
+    }
+  }
+};
 
 // A block's tile in a ring of R buffers of one K step each.  Step `it` of a wave: its operands are in registers (read a step
 // ago); once all waves are there, buffer `it` is free and buffer it+1 complete; between its MFMAs, one to a slot, it reads
@@ -166,7 +214,6 @@ __device__ __forceinline__ void tri_block(const TriParams& ap, const TriParams& 
                                           int s_end, int groups, int dst_split) {
   constexpr int TM = T::TM, TN = T::TN, R = kTriRing, RA = (T::BM + 63) / 64 * 64, RBn = (T::BN + 63) / 64 * 64;
   static_assert(T::NT == 4 * kWave && T::BK == 16, "four waves, 16 k a step");
-  static_assert(kTriLdsBytes >= TN * 16 * 4 * kWave * 4, "a row of blocks fits the ring");
   typedef DmaTri<RA, RBn, B_LINEAR> Loader;
   constexpr int SA = 6 * RA, SB = 6 * RBn;   // 16-byte pieces of a step
   extern __shared__ float lds_dyn[];
@@ -283,28 +330,22 @@ __device__ __forceinline__ void tri_block(const TriParams& ap, const TriParams& 
 #pragma unroll
       for (int v = 0; v < 16; ++v) finite = fmaf(acc[i][j][v], 0.0f, finite);
     }
-  __syncthreads();   // the ring has been read for the last time
   if (__any(!(finite == 0.0f))) {
-    float* const mine = lds_dyn + wave * (TN * 16 * kWave) + lane;   // [value][lane]
     const int g0 = 2 * s_begin, g1 = 2 * s_end < groups ? 2 * s_end : groups;
-#pragma unroll
-    for (int i = 0; i < TM; ++i) {
-#pragma unroll
-      for (int j = 0; j < TN; ++j)
-#pragma unroll
-        for (int v = 0; v < 16; ++v) mine[(j * 16 + v) * kWave] = acc[i][j][v];
 #pragma unroll 1
-      for (int e = 0; e < TN * 16; ++e) {
-        const int v = e & 15, j = e >> 4;
-        const int row = m0 + wm * (TM * 32) + i * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3);
-        const int col = n0 + wn * (TN * 32) + j * 32 + (lane & 31);
-        if (!(fabsf(mine[e * kWave]) < INFINITY) && row < ep.rows && col < ep.cols)
-          mine[e * kWave] = tri_dot<B_LINEAR>(ap, bp, row, col, g0, g1);
-      }
+    for (int t = 0; t < TM * TN; ++t) {
+      f32x16 d = acc[0][0];
 #pragma unroll
-      for (int j = 0; j < TN; ++j)
+      for (int u = 1; u < TM * TN; ++u)
+        if (t == u) d = acc[u / TN][u % TN];
+      const int row0 = m0 + wm * (TM * 32) + t / TN * 32, col0 = n0 + wn * (TN * 32) + t % TN * 32;
+      const TriRow ra(ap, row0 + (lane & 31)), rb(bp, col0 + (lane & 31));
+      tri_redo(d, ep.rows - row0, ep.cols - col0, lane, g0, g1,
+               [&](int g, float (&v)[8]) { ra.load((size_t)g * ap.v.group_stride, v); },
+               [&](int g, float (&v)[8]) { rb.load(B_LINEAR ? (size_t)g * bp.v.group_stride : (size_t)bp.v.soff[g], v); });
 #pragma unroll
-        for (int v = 0; v < 16; ++v) acc[i][j][v] = mine[(j * 16 + v) * kWave];
+      for (int u = 0; u < TM * TN; ++u)
+        if (t == u) acc[u / TN][u % TN] = d;
     }
   }
   store_tile<T, NCHW>(acc, ep, m0, n0, wm, wn, lane, dst_split);

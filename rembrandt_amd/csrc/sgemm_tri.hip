@@ -63,7 +63,6 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_stream_kernel(Tri
   typedef TriStream<T> S;
   constexpr int TM = T::TM, RA = S::RA, R = S::R, CNT = S::CNT;
   static_assert(T::TN == 1 && T::WM == 1 && T::WN == 4 && T::BK == 16 && R >= 4 && (TM == 1 || TM % 2 == 0), "block shape");
-  static_assert(S::LDS >= 4 * 16 * kWave * 4, "a block of results a wave fits the ring");
   extern __shared__ float lds_dyn[];
   uint4* const sm = reinterpret_cast<uint4*>(lds_dyn);
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)sm;
@@ -220,27 +219,22 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_stream_kernel(Tri
 #pragma unroll
     for (int v = 0; v < 16; ++v) finite = fmaf(acc[i][0][v], 0.0f, finite);
   }
-  __syncthreads();   // the ring has been read for the last time
-  if (__any(!(finite == 0.0f))) {   // as in mfma_gemm_tri_kernel, from the operands themselves
-    float* const mine = lds_dyn + wave * (16 * kWave) + lane;
-    const int k0 = s_begin * 16, k1 = s_end * 16 < bp.K ? s_end * 16 : bp.K;
+  if (__any(!(finite == 0.0f))) {   // as in tri_block, from the operands themselves
+    const int col0 = n0 + wave * 32, col = col0 + (lane & 31) < bp.rows ? col0 + (lane & 31) : 0;
+    const float* const pb = bp.ptr + (K_CONTIG ? (size_t)col * bp.ld : (size_t)col);
+    const int k1 = s_end * 16 < bp.K ? s_end * 16 : bp.K;
 #pragma unroll
     for (int i = 0; i < TM; ++i) {
+      const int row0 = m0 + i * 32, row = row0 + (lane & 31) < rows32.rows ? row0 + (lane & 31) : 0;
+      const float* const pa = rows32.ptr + (size_t)row * rows32.ld;
+      auto load = [&](const float* p, size_t step, int g, float (&v)[8]) {
 #pragma unroll
-      for (int v = 0; v < 16; ++v) mine[v * kWave] = acc[i][0][v];
-#pragma unroll 1
-      for (int v = 0; v < 16; ++v) {
-        const int row = m0 + i * 32 + (v >> 2) * 8 + (lane >> 5) * 4 + (v & 3), col = n0 + wave * 32 + (lane & 31);
-        if (!(fabsf(mine[v * kWave]) < INFINITY) && row < ep.rows && col < ep.cols) {
-          const float* pa = rows32.ptr + (size_t)row * rows32.ld;
-          const float* pb = bp.ptr + (K_CONTIG ? (size_t)col * bp.ld : (size_t)col);
-          float sum = 0.0f;
-          for (int k = k0; k < k1 && sum == sum; ++k) sum = fmaf(pa[k], pb[K_CONTIG ? (size_t)k : (size_t)k * bp.ld], sum);
-          mine[v * kWave] = sum;
-        }
-      }
-#pragma unroll
-      for (int v = 0; v < 16; ++v) acc[i][0][v] = mine[v * kWave];
+        for (int e = 0; e < 8; ++e)
+          if (g * 8 + e < k1) v[e] = p[(size_t)(g * 8 + e) * step];
+      };
+      tri_redo(acc[i][0], ep.rows - row0, ep.cols - col0, lane, s_begin * 2, (k1 + 7) / 8,
+               [&](int g, float (&v)[8]) { load(pa, 1, g, v); },
+               [&](int g, float (&v)[8]) { load(pb, K_CONTIG ? 1 : (size_t)bp.ld, g, v); });
     }
   }
   store_tile<T, false>(acc, ep, m0, n0, 0, wave, lane, ep.split_stride != 0 ? slice : -1);

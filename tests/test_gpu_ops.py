@@ -682,6 +682,66 @@ def test_conv2d_bf16x3_largest_floats_beside_an_infinity(dev):
     assert bool((ops.conv2d_fwd(x, w, 1, 0, algo=X3) == float("inf")).all())
 
 
+def _redo_bound(terms):
+    """Relative error of sums on the fp32 instruction in two levels, chains of 128 terms and the sum of them: a rounding's variance
+    as in test_conv2d_staged_operands_error, a quarter on top."""
+    return 1.25 * 2.0 ** -24 * (0.09 * (128 + terms / 128) + 4) ** 0.5
+
+
+@pytest.mark.parametrize("exponent", [-112, -120, -126, -140])
+def test_conv2d_bf16x3_small_operands(dev, exponent):
+    """Operands whose last bits lie under bf16's smallest value, 2^-133, beside large ones: no bit of them is lost.  Both of a
+    pass's operands in turn, all of a tensor or one value in a hundred (of which the others' results must not suffer)."""
+    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
+    Nn, C, H, W, K, R, pad = 9, 40, 12, 11, 72, 3, 1
+    shapes = (Nn, C, H, W), (K, C, R, R), (Nn, K, H, W)
+    big = np.float32(2.0 ** 100)
+    for tiny in range(3):
+        for share in (1.0, 0.01):
+            say("bf16x3 small operands", exponent, tiny, share)
+            t = [synth.normal(43, 1 + i, s) for i, s in enumerate(shapes)]
+            small = (t[tiny].astype(np.float64) * 2.0 ** exponent).astype(np.float32)
+            assert np.any(small != 0)
+            t = [a * big for a in t]
+            t[tiny] = small if share == 1.0 else np.where(synth.uniform(43, 9, t[tiny].shape) < share, small, t[tiny] / big)
+            x, w, dy = t
+            xd, wd, dyd = T(x, dev), T(w, dev), T(dy, dev)
+            for name, operands, terms, ref, run in (
+                    ("fwd", (0, 1), C * R * R, lambda: O.conv2d_fwd(x, w, 1, pad), lambda: ops.conv2d_fwd(xd, wd, 1, pad, algo=X3)),
+                    ("bwd_data", (1, 2), K * R * R, lambda: O.conv2d_bwd_data(w, dy, x.shape, 1, pad), lambda: ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=X3)),
+                    ("bwd_filter", (0, 2), Nn * H * W, lambda: O.conv2d_bwd_filter(x, dy, w.shape, 1, pad), lambda: ops.conv2d_bwd_filter(xd, dyd, w.shape, 1, pad, algo=X3))):
+                if tiny not in operands:
+                    continue
+                want = ref().astype(np.float64)
+                err = np.linalg.norm(N(run()).astype(np.float64) - want) / np.linalg.norm(want)
+                assert err <= _redo_bound(terms), (name, err)
+
+
+@pytest.mark.parametrize("exponent", [-112, -126, -140])
+def test_conv2d_bf16x3_strided_small_operands(dev, exponent):
+    """As above, the data gradient by residue classes."""
+    Nn, C, H, W, K, R, st, pad = X3_STRIDED_CASES[0]
+    P, Q = (H + 2 * pad - R) // st + 1, (W + 2 * pad - R) // st + 1
+    w, dy = synth.normal(45, 1, (K, C, R, R)), synth.normal(45, 2, (Nn, K, P, Q))
+    for a, b in ((exponent, 100), (100, exponent)):
+        ws, dys = ((t.astype(np.float64) * 2.0 ** e).astype(np.float32) for t, e in ((w, a), (dy, b)))
+        got, tags = profile_tags(lambda: ops.conv2d_bwd_data(T(ws, dev), T(dys, dev), (Nn, C, H, W), st, pad, algo=_lib.RH_ALGO_BF16X3))
+        assert any(t.startswith("conv_bwd_data_tri_") for t in tags), tags
+        want = O.conv2d_bwd_data(ws, dys, (Nn, C, H, W), st, pad).astype(np.float64)
+        err = np.linalg.norm(N(got).astype(np.float64) - want) / np.linalg.norm(want)
+        assert err <= _redo_bound(K * R * R), err
+
+
+def test_conv2d_bf16x3_what_the_parts_leave_cancels(dev):
+    """Two values of a group of eight of which nothing fits the parts, of opposite signs: each counts by itself."""
+    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
+    x, w = torch.zeros((1, 8, 4, 4), device=dev), torch.zeros((16, 8, 1, 1), device=dev)
+    x[0, 0], x[0, 1] = 2.0 ** -149, -2.0 ** -149
+    w[:, 0], w[:8, 1] = 2.0 ** 100, -2.0 ** 101
+    y = ops.conv2d_fwd(x, w, 1, 0, algo=X3)
+    assert bool((y[:, :8] == 3 * 2.0 ** -49).all()) and bool((y[:, 8:] == 2.0 ** -49).all())
+
+
 def test_conv2d_bf16x3_where_it_pays(dev):
     """RH_ALGO_BF16X3 alone: the form where it is expected to be the fastest, and the others' bits elsewhere."""
     for (Nn, C, H, K, R, st, pad), takes in (((37, 256, 13, 384, 3, 1, 1), True), ((24, 128, 28, 256, 3, 2, 1), True), ((8, 96, 27, 256, 5, 1, 2), True),
@@ -962,6 +1022,27 @@ def test_sgemm_bf16x3(dev, case):
     keep = np.isfinite(out[1])
     assert np.array_equal(out[0][np.isinf(out[1])], out[1][np.isinf(out[1])])
     assert np.all(np.abs(out[0][keep].astype(np.float64) - out[1][keep]) <= 1e-4 * (1.0 + np.abs(out[1][keep].astype(np.float64))))
+
+
+@pytest.mark.parametrize("exponent", [-112, -126, -140])
+@pytest.mark.parametrize("case", [(1, 0, 132, 31, 48), (1, 0, 516, 129, 496), (0, 0, 260, 40, 77), (0, 0, 516, 130, 1000), (0, 1, 500, 1000, 50)], ids=str)
+def test_sgemm_bf16x3_small_operands(dev, case, exponent):
+    """As test_conv2d_bf16x3_small_operands: either operand all below bf16's parts, or one value in a hundred."""
+    tA, tB, m, n, k = case
+    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
+    base = synth.normal(18, 1, (m, k) if tA else (k, m)), synth.normal(18, 2, (k, n) if tB else (n, k))
+    for tiny in (0, 1):
+        for share in (1.0, 0.01):
+            say("sgemm bf16x3 small operands", case, exponent, tiny, share)
+            t = [a * np.float32(2.0 ** 100) for a in base]
+            small = (base[tiny].astype(np.float64) * 2.0 ** exponent).astype(np.float32)
+            t[tiny] = small if share == 1.0 else np.where(synth.uniform(18, 9, small.shape) < share, small, base[tiny])
+            A, B = t
+            C = torch.empty(n, m, device=dev)
+            ops.sgemm(tA, tB, m, n, k, 1.0, T(A, dev), A.shape[1], T(B, dev), B.shape[1], 0.0, C, m, algo=X3)
+            exact = (B.T if tB else B).astype(np.float64) @ (A.T if tA else A).astype(np.float64)
+            err = np.linalg.norm(N(C).astype(np.float64) - exact) / np.linalg.norm(exact)
+            assert err <= _redo_bound(k), err
 
 
 def test_sgemm_bf16x3_where_it_pays(dev):
