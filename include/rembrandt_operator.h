@@ -123,6 +123,9 @@ int rho_config_from_model_file(const char* path, rho_config** out);
  *                           sums in another order, same tolerance against the oracle.  The flag keeps the direct form on
  *                           fp32 instructions for convolutions and affine products of every size. */
 #define RHO_EXEC_DIRECT_CONV 0x20
+/*   RHO_EXEC_FP32_INSTRUCTIONS  convolutions and affine products keep the fp32 matrix instructions (no RH_ALGO_BF16X3): the
+ *                           Winograd form where the library takes it, the direct form elsewhere. */
+#define RHO_EXEC_FP32_INSTRUCTIONS 0x40
 int rho_worker_new(const rho_config* cfg, int32_t batch_size, int capability, uint64_t seed0, uint64_t seed1,
                    int device, int exec_flags, rho_worker** out);
 int rho_worker_free(rho_worker* w);

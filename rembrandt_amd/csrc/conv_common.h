@@ -610,10 +610,8 @@ bool conv1x1_stream_applies(const ConvDims& d);
 // that of the form taken otherwise.  The engine's estimate was fitted to 3x3 and 5x5 stride-1 layers and is 10 to 25 % short on
 // others, hence the tenth.  Over 308 timed forward calls (22 layers at 14 batches) the forms chosen so are 1.27 times as fast as
 // without it, geometric mean, 1.02 times slower at worst.  1x1 layers of up to 128 channels keep the streaming kernels, which
-// read their operands where they lie (96 -> 96 54x54 b128 82 us against 158).
-// A layer of one 128-row tile of filters keeps the Winograd form in the 5x5 forward pass and in the filter gradient, although
-// it is the slower one there too (64 -> 128 5x5 24x24 b128 190 us expected against 143, 128 -> 128 3x3 28x28 b256 466 us
-// measured against 341): the comparison of whole train steps in the two forms runs them on such layers.
+// read their operands where they lie (96 -> 96 54x54 b128 82 us against 158).  Winograd -> this form on one row tile of filters:
+// 64 -> 128 5x5 24x24 b128 forward 198 -> 141 us, 128 -> 128 3x3 28x28 filter gradient b37, 64, 256 98 -> 64, 139 -> 92, 466 -> 349.
 inline bool tri_allowed(int flags) {
   return (flags & RH_ALGO_BF16X3) && !(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_WINOGRAD));
 }
@@ -651,7 +649,6 @@ inline bool tri_pays(const ConvDims& d, bool bwd, int flags, TriPlan* plan, PLAN
       WinoGeom wg = five ? wino_geom_fwd5(d) : bwd ? wino_geom_bwd_data(d) : wino_geom_fwd(d);
       if (flags & RH_ALGO_SHARED_GPU) wg.beside_others();
       if (five ? wino_pays5(wg, f) : wino_pays(wg, f)) {
-        if (five && d.K <= kWinoBM) return false;
         us = wg.us;
         err = wino_err(wg);
       }
@@ -671,7 +668,7 @@ inline bool tri_pays_bwd_data(const ConvDims& d, int flags, TriPlan* plan) {
 // which this form is then chosen in 188, 1.53 times as fast in the geometric mean).  1x1 layers need 384 channels or so to be
 // worth two split copies.
 inline bool tri_pays_bwd_filter(const ConvDims& d, const TriFilterPlan& t) {
-  if (!t.ok || (wino_shape(d) && d.K <= kWinoBM && wino_filter_pays(d, plan_wino_bwd_filter(d)))) return false;
+  if (!t.ok) return false;
   const int bm = pick_bm(d.K);
   const double flops = 2.0 * (double)d.w_elems * d.N * d.P * d.Q;
   const double other = (d.R * d.S > 1 ? 1.25 : 1.0) * (15.0 + flops / (bm >= 96 ? 100e6 : bm == 64 ? 60e6 : 50e6)) + 11e-6 * (double)d.w_elems;

@@ -211,6 +211,9 @@ namespace {
 
 typedef std::shared_ptr<DeviceContext> Ctx;
 
+// The forms that a worker's options allow its convolutions.
+int product_algo(const ExecOptions& o) { return !o.winograd ? RH_ALGO_DIRECT : o.split_operands ? RH_ALGO_BF16X3 : 0; }
+
 // Scratch is allocated once for batch_cap, but a pass may be called with any batch <= batch_cap and the library's
 // plans are not monotone in the batch (fewer result tiles make it cut the contraction into more slices, whose partial
 // sums can need more room than the full batch does): every scratch buffer is sized with the *_upto functions.
@@ -668,7 +671,7 @@ class AffineOperator : public Operator {
   AffineOperator(size_t batch_size, OpCapability capability, const AffineOperatorConfig& config, const Operator* prev_op,
                  Ctx context, const ExecOptions& opts)
       : batch_cap_(batch_size), config_(config), context_(context), fuse_epilogue_(opts.fuse_epilogue),
-        algo_(opts.winograd ? RH_ALGO_BF16X3 : 0),
+        algo_(product_algo(opts) & RH_ALGO_BF16X3),
         overlap_built_(opts.overlap_backward && backward_enabled(capability)), overlap_on_(overlap_built_) {
     RB_ASSERT(prev_op != nullptr);
     in_act_ = prev_op->get_output_vars();
@@ -872,7 +875,7 @@ class Conv2dOperator : public Operator {
       }
       return;
     }
-    const int math = (opts_.bf16_forward ? RH_MATH_BF16_MFMA_FP32ACC : 0) | (opts_.winograd ? RH_ALGO_BF16X3 : RH_ALGO_DIRECT);
+    const int math = (opts_.bf16_forward ? RH_MATH_BF16_MFMA_FP32ACC : 0) | product_algo(opts_);
     if (opts_.fuse_epilogue) {
       const int flags = RH_FUSE_BIAS | (rect ? RH_FUSE_RELU : 0) | math;
       unwrap(rh_conv2d_fwd(&g, 1.0f, in_act_->as_ptr(), params_.weights->as_ptr(), 0.0f, out_act_->as_mut_ptr(),
@@ -906,7 +909,7 @@ class Conv2dOperator : public Operator {
       w_filter = w_bias = workspace_aux_.get();
     }
     const float beta = params_.take_backward_beta();   // 1: accumulate (the reference's call); 0: the buffers stand for zeros
-    const int algo = opts_.winograd ? RH_ALGO_BF16X3 : RH_ALGO_DIRECT;
+    const int algo = product_algo(opts_);
     // (a small layer's bias gradient rides in the launch of the filter gradient's reduction: the combined call below)
     const bool small = batch_size * out_dims_.len() <= (size_t(1) << 20);
     if (!in_delta_ && workspace_aux_ && overlap_on_ && !small) {
@@ -1529,7 +1532,7 @@ class BNormUnitsOperator : public Operator {
     in_act_ = prev_op->get_output_vars();
     if (!in_act_) panic(std::string(who) + " missing required prev operator output vars");
     in_delta_ = prev_op->get_output_deltas();
-    for (auto& u : units_) u.conv_algo = opts.winograd ? RH_ALGO_BF16X3 : RH_ALGO_DIRECT;
+    for (auto& u : units_) u.conv_algo = product_algo(opts);
   }
   size_t batch_size() const override { return batch_cap_; }
   SharedDeviceBuf get_output_vars() const override { return out_act_; }

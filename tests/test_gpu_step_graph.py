@@ -25,10 +25,10 @@ def param_buffers(net, read_grads=True):
 
 
 def run(net, batch, steps, graph, seed, sgd_kwargs, fused=True, toggle_at=None, read_grads=True, fuse_tail=True, extra=(),
-        winograd=True):
+        winograd=True, split_operands=True):
     dims, layers, ncat = net
     w = SequentialOperatorWorker(configs.build_config(net), batch, "Backward", shared_seed=(seed, seed + 1), graph_steps=graph,
-                                 fuse_tail=fuse_tail, winograd=winograd)
+                                 fuse_tail=fuse_tail, winograd=winograd, split_operands=split_operands)
     w.init_params()
     sgd = SgdOpt(batch, **sgd_kwargs)
     sgd.begin(w)
@@ -279,7 +279,7 @@ def wino_net(kind):
 @pytest.mark.parametrize("kind", ["plain", "bnorm", "five"])
 def test_winograd_steps_match_direct_steps(dev, kind):
     """Train steps whose 3x3 layers of 128 channels run in the Winograd form (all three passes, what the library picks
-    by itself at this size; "five": the forward pass of a 5x5 layer) against the same steps with RHO_EXEC_DIRECT_CONV: same losses, counts,
+    by itself at this size on fp32 instructions; "five": the forward pass of a 5x5 layer) against the same steps with RHO_EXEC_DIRECT_CONV: same losses, counts,
     parameters and momentum to rounding; the Winograd kernels did run in the first and not in the second.
     Two fp32 paths that add in different orders are compared here, through ReLU masks (an activation within rounding
     of zero changes side) and bias gradients (sums of 32768 deltas that largely cancel): relative L2 distance 4.5e-3 after the first step, 1e-2 after
@@ -297,7 +297,7 @@ def test_winograd_steps_match_direct_steps(dev, kind):
     batch, steps = 128, 3
     kw = dict(step_size=0.01, momentum=("Update", 0.9), l2_reg_coef=5e-4)
     say("winograd steps", kind)
-    (a, _), tags_a = profile_tags(lambda: run(net, batch, steps, False, 0x3141, kw, read_grads=False))
+    (a, _), tags_a = profile_tags(lambda: run(net, batch, steps, False, 0x3141, kw, read_grads=False, split_operands=False))
     (b, _), tags_b = profile_tags(lambda: run(net, batch, steps, False, 0x3141, kw, read_grads=False, winograd=False))
     assert "conv_fwd_wino" in tags_a and "wino_transform" in tags_a
     if kind == "five":   # forward only: the backward passes of a 5x5 layer stay direct
@@ -322,7 +322,8 @@ def test_recorded_steps_of_winograd_networks(dev, kind):
     say("step graph, winograd", kind)
     net = wino_net(kind)
     kw = dict(step_size=0.01, momentum=("Update", 0.9), l2_reg_coef=5e-4)
-    eager, n0 = run(net, 128, 5, False, 0x6A11, kw)
-    graph, n1 = run(net, 128, 5, True, 0x6A11, kw)
-    assert n0 == 0 and n1 == 3
-    same(eager, graph, "winograd " + kind)
+    for split in (False, True):   # (and the same networks' steps in the split-operand form)
+        eager, n0 = run(net, 128, 5, False, 0x6A11, kw, split_operands=split)
+        graph, n1 = run(net, 128, 5, True, 0x6A11, kw, split_operands=split)
+        assert n0 == 0 and n1 == 3
+        same(eager, graph, "winograd " + kind)
