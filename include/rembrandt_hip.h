@@ -152,13 +152,17 @@ int32_t rh_conv2d_out_dim(int32_t in, int32_t size, int32_t stride, int32_t pad)
 /* Bytes of scratch the given pass needs whatever flags it is called with (0 is possible), RH_ALGO_BF16X3 with RH_ALGO_DIRECT
  * apart.  The scratch must be 256-byte aligned. */
 size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass);
-/* The same for RH_ALGO_BF16X3 with RH_ALGO_DIRECT; 0 where the geometry has no such form. */
+/* The same with room for the form of RH_ALGO_BF16X3 where `flags` allow it and it is expected to be the fastest, with the hint
+ * RH_ALGO_SHARED_GPU or without: with less a call takes another form. */
+size_t rh_conv2d_workspace_bytes_for(const rh_conv_geom* g, int pass, int flags);
+/* The same for RH_ALGO_BF16X3 with RH_ALGO_DIRECT, which needs it; 0 where the geometry has no such form. */
 size_t rh_conv2d_bf16x3_workspace_bytes(const rh_conv_geom* g, int pass);
 /* The same for a scratch buffer that is allocated once and then used with every batch 1..g->N, the way the
  * reference's operators size theirs for batch_cap (src/operator/mod.rs:1493-1507): the largest need of any such
  * batch.  The need is not monotone in N (a pass with few result tiles cuts its contraction into slices and keeps
  * their partial sums in the scratch), so this can exceed rh_conv2d_workspace_bytes of g itself. */
 size_t rh_conv2d_workspace_bytes_upto(const rh_conv_geom* g, int pass);
+size_t rh_conv2d_workspace_bytes_for_upto(const rh_conv_geom* g, int pass, int flags);
 /* FLOPs (2 per multiply-add) that a pass (RH_CONV_FWD, RH_CONV_BWD_DATA, RH_CONV_BWD_FILTER) executes on this geometry when the library takes
  * the Winograd F(2x2, 3x3) form for it under `flags` (16 multiply-adds per 2x2 output tile, filter and channel; tiles
  * that hang over an odd extent count whole), 0 when it takes a direct form.  The direct form's count is

@@ -93,6 +93,8 @@ PROTOTYPES = {
     "rh_conv2d_workspace_bytes": (_sz, [C.POINTER(ConvGeom), _int]),
     "rh_conv2d_bf16x3_workspace_bytes": (_sz, [C.POINTER(ConvGeom), _int]),
     "rh_conv2d_workspace_bytes_upto": (_sz, [C.POINTER(ConvGeom), _int]),
+    "rh_conv2d_workspace_bytes_for": (_sz, [C.POINTER(ConvGeom), _int, _int]),
+    "rh_conv2d_workspace_bytes_for_upto": (_sz, [C.POINTER(ConvGeom), _int, _int]),
     "rh_conv2d_bwd_bias_workspace_bytes_upto": (_sz, [_i32, _i32, _i32]),
     "rh_sgemm_workspace_bytes_upto": (_sz, [_i32, _i32, _i32, _int]),
     "rh_bnorm_workspace_bytes_upto": (_sz, [_int, _int, _int]),

@@ -170,10 +170,13 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
 
   if ((flags & RH_ALGO_WINOGRAD) && (!wino_shape(d) || (flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT)))) return RH_E_UNSUPPORTED;
   if (tri_allowed(flags)) {
-    TriPlan tp = plan_tri_bwd_data(d);
-    if (tri_forced(flags) && !tp.ok) return RH_E_UNSUPPORTED;
-    if (tri_forced(flags) && ws_bytes < tp.total()) return RH_E_WORKSPACE;
-    if (tri_forced(flags) || tri_pays_bwd_data(d, flags, &tp)) {
+    TriPlan tp = {};
+    if (tri_forced(flags)) {
+      tp = plan_tri_bwd_data(d);
+      if (!tp.ok) return RH_E_UNSUPPORTED;
+      if (ws_bytes < tp.total()) return RH_E_WORKSPACE;
+    }
+    if (tri_forced(flags) || (tri_pays(d, true, flags, &tp) && ws_bytes >= tp.total())) {
       if (d.x_elems == 0) return 0;
       return launch_conv_tri(tp, true, dy, w, dx, alpha, beta, nullptr, 0, mask, ws, stream);
     }
@@ -217,8 +220,7 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
     };
     if (tri_allowed(flags)) {
       const TriPhasePlan tp = plan_tri_phases(d, pp);
-      if (tp.ok) {
-        if (ws_bytes < tp.total()) return RH_E_WORKSPACE;
+      if (tp.ok && ws_bytes >= tp.total()) {
         float* sub;
         const int e = launch_conv_tri_phases(d, pp, tp, w, dy, ws, stream, &sub);
         return e ? e : interleave(sub);

@@ -868,21 +868,13 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
       }
       const size_t lp = lds_part_bytes(d.R, d.S, d.st, d.y_elems);
       if (lp > need) need = lp;
-      for (const int flags : {0, RH_ALGO_SHARED_GPU}) {
-        TriPlan tp;
-        if (tri_pays_fwd(d, flags, &tp) && tp.total() > need) need = tp.total();
-      }
       return need;
     }
     case RH_CONV_BWD_DATA: {
       const size_t legacy = align256(sizeof(int4) * (size_t)round_up(KRS, kTabPad)) +
                             align256(sizeof(int) * (size_t)round_up(KRS, kTabPad));
       const PhasePlan pp = plan_phase_bwd_data(d);
-      if (pp.ok) {
-        const TriPhasePlan xp = plan_tri_phases(d, pp);
-        const size_t most = xp.ok && xp.total() > pp.total() ? xp.total() : pp.total();
-        return most > legacy ? most : legacy;
-      }
+      if (pp.ok) return pp.total() > legacy ? pp.total() : legacy;
       const SoffPlan sp = plan_soff_bwd_data(d);
       size_t need = sp.ok && sp.total() > legacy ? sp.total() : legacy;
       if (wino_shape(d)) {
@@ -891,10 +883,6 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
       }
       const size_t lp = lds_part_bytes(d.R, d.S, d.st, d.x_elems);
       if (lp > need) need = lp;
-      for (const int flags : {0, RH_ALGO_SHARED_GPU}) {
-        TriPlan tp;
-        if (tri_pays_bwd_data(d, flags, &tp) && tp.total() > need) need = tp.total();
-      }
       return need;
     }
     case RH_CONV_BWD_FILTER: {
@@ -903,8 +891,6 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
         const WinoFilterPlan wp = plan_wino_bwd_filter(d);
         if (wp.ok && wp.total() > need) need = wp.total();
       }
-      const TriFilterPlan tp = plan_tri_bwd_filter(d);
-      if (tp.ok && tp.total() > need && tri_pays_bwd_filter(d, tp)) need = tp.total();
       return need + bwd_filter_bias_bytes(d);
     }
     default:
@@ -912,22 +898,46 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
   }
 }
 
+// Scratch of the split-operand form where `flags` (with RH_ALGO_BF16X3) take it; 0 where they do not, and where it cannot be
+// more than `floor` (the filter gradient's copies, and slices of up to 1024 tiles or 256 MB in all).
+static size_t bf16x3_bytes(const ConvDims& d, int pass, int flags, size_t floor) {
+  if (pass == RH_CONV_BWD_FILTER) {
+    const double copies = 6.0 * round_up(d.N, 8) * ((double)d.K * (d.P * d.Q + 1) + (double)d.C * (d.H + 2 * d.pad) * (d.W + 2 * d.pad));
+    const double slices = fmin(256e6, fmax(4.0 * (double)d.w_elems, 1024.0 * 4 * 128 * 192));
+    const double rest = (double)cdiv(d.N, 8) * 4.0 * (d.P * d.Q + (double)d.K * (d.P * d.Q / 32 + 1)) + 4096.0;
+    if (copies + slices + rest < (double)floor) return 0;
+    const TriFilterPlan tp = plan_tri_bwd_filter(d);
+    return tp.ok && (tri_forced(flags) || tri_pays_bwd_filter(d, tp)) ? tp.total() : 0;
+  }
+  if (pass != RH_CONV_FWD && pass != RH_CONV_BWD_DATA) return 0;
+  const bool bwd = pass == RH_CONV_BWD_DATA;
+  if (tri_forced(flags)) {
+    const TriPlan tp = plan_tri_pass(d, bwd, 0);
+    return tp.ok ? tp.total() : 0;
+  }
+  if (bwd && d.st > 1) {
+    const PhasePlan pp = plan_phase_bwd_data(d);
+    const TriPhasePlan tp = plan_tri_phases(d, pp);
+    return tp.ok ? tp.total() : 0;
+  }
+  return tri_bytes(d, bwd, floor);
+}
+
+extern "C" size_t rh_conv2d_workspace_bytes_for(const rh_conv_geom* g, int pass, int flags) {
+  ConvDims d;
+  if (conv_dims(g, &d)) return 0;
+  const size_t need = rh_conv2d_workspace_bytes(g, pass), tri = tri_allowed(flags) ? bf16x3_bytes(d, pass, flags, need) : 0;
+  return tri > need ? tri : need;
+}
+
 extern "C" size_t rh_conv2d_bf16x3_workspace_bytes(const rh_conv_geom* g, int pass) {
   ConvDims d;
   if (conv_dims(g, &d)) return 0;
-  size_t tri = 0;
-  if (pass == RH_CONV_BWD_FILTER) {
-    const TriFilterPlan tp = plan_tri_bwd_filter(d);
-    tri = tp.ok ? tp.total() : 0;
-  } else if (pass == RH_CONV_FWD || pass == RH_CONV_BWD_DATA) {
-    const TriPlan tp = pass == RH_CONV_FWD ? plan_tri_fwd(d) : plan_tri_bwd_data(d);
-    tri = tp.ok ? tp.total() : 0;
-  }
-  const size_t other = tri ? rh_conv2d_workspace_bytes(g, pass) : 0;
-  return tri > other ? tri : other;
+  const int forced = RH_ALGO_BF16X3 | RH_ALGO_DIRECT;
+  return bf16x3_bytes(d, pass, forced, 0) ? rh_conv2d_workspace_bytes_for(g, pass, forced) : 0;
 }
 
-extern "C" size_t rh_conv2d_workspace_bytes_upto(const rh_conv_geom* g, int pass) {
+extern "C" size_t rh_conv2d_workspace_bytes_for_upto(const rh_conv_geom* g, int pass, int flags) {
   if (!g) return 0;
   rh_conv_geom h = *g;
   size_t need = 0;
@@ -935,8 +945,16 @@ extern "C" size_t rh_conv2d_workspace_bytes_upto(const rh_conv_geom* g, int pass
     h.N = n;
     const size_t b = rh_conv2d_workspace_bytes(&h, pass);
     if (b > need) need = b;
+    ConvDims d;
+    if (!tri_allowed(flags) || conv_dims(&h, &d)) continue;
+    const size_t tri = bf16x3_bytes(d, pass, flags, need);
+    if (tri > need) need = tri;
   }
   return need;
+}
+
+extern "C" size_t rh_conv2d_workspace_bytes_upto(const rh_conv_geom* g, int pass) {
+  return rh_conv2d_workspace_bytes_for_upto(g, pass, 0);
 }
 
 // The bias gradient beside the filter gradient (rh_conv2d_bwd_filter_bias).  part: where the pass over dy may leave the
@@ -999,7 +1017,7 @@ static int bwd_filter_impl(const rh_conv_geom* g, float alpha, const float* x, c
     const TriFilterPlan tp = plan_tri_bwd_filter(d);
     if (tri_forced(flags) && !tp.ok) return RH_E_UNSUPPORTED;
     if (tri_forced(flags) && ws_bytes < tp.total()) return RH_E_WORKSPACE;
-    if (tri_forced(flags) || tri_pays_bwd_filter(d, tp)) {
+    if (tri_forced(flags) || (tri_pays_bwd_filter(d, tp) && ws_bytes >= tp.total())) {
       if (d.w_elems == 0) return 0;
       float* parts = nullptr;
       int used = 1;

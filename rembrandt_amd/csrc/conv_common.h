@@ -630,38 +630,66 @@ inline double wino_err(const WinoGeom& g) {
   const int stages = g.full_tiles > 0 || g.tail_S <= 1 ? g.Cg : g.tail_L;
   return 1.35 + 0.351 * cdiv(stages, g.chains > 0 ? g.chains : 1);
 }
-// plan: what is to be launched where it pays.
-template <class PLAN>
-inline bool tri_pays(const ConvDims& d, bool bwd, int flags, TriPlan* plan, PLAN make) {
-  if ((bwd ? d.K : d.C) % 8 != 0 || conv1x1_stream_applies(d)) return false;
+// The form that a call takes without the bit, [1] with RH_ALGO_SHARED_GPU beside it: its expected time and its error.
+struct TriRival { double us, err; };
+inline void tri_rivals(const ConvDims& d, bool bwd, TriRival (&r)[2]) {
   const int terms = (bwd ? d.K : d.C) * d.R * d.S;
-  double us, err;
   if (!has_staged_form(d)) {
     const SoffPlan sp = bwd ? plan_soff_bwd_data(d) : plan_soff_fwd(d);
-    us = 1.1 * engine_us(sp, bwd ? d.C : d.K, (long long)d.N * (bwd ? d.H * d.W : d.P * d.Q), d.w_elems, false);
-    err = engine_err(sp, terms);
-  } else {
-    const DirectForms f = bwd ? direct_bwd_data(d) : direct_fwd(d);
-    us = f.us;
-    err = f.staged ? staged_err(f.lds, d.R) : engine_err(f.soff, terms);
-    const bool five = !bwd && wino_shape5(d);
-    if (wino_shape(d) || five) {
-      WinoGeom wg = five ? wino_geom_fwd5(d) : bwd ? wino_geom_bwd_data(d) : wino_geom_fwd(d);
-      if (flags & RH_ALGO_SHARED_GPU) wg.beside_others();
-      if (five ? wino_pays5(wg, f) : wino_pays(wg, f)) {
-        us = wg.us;
-        err = wino_err(wg);
-      }
-    }
+    r[0].us = 1.1 * engine_us(sp, bwd ? d.C : d.K, (long long)d.N * (bwd ? d.H * d.W : d.P * d.Q), d.w_elems, false);
+    r[0].err = engine_err(sp, terms);
+    r[1] = r[0];
+    return;
   }
-  *plan = make(tri_max_chain(err));
-  return plan->ok && plan->us < us;
+  const DirectForms f = bwd ? direct_bwd_data(d) : direct_fwd(d);
+  r[0].us = f.us;
+  r[0].err = f.staged ? staged_err(f.lds, d.R) : engine_err(f.soff, terms);
+  r[1] = r[0];
+  const bool five = !bwd && wino_shape5(d);
+  if (!wino_shape(d) && !five) return;
+  WinoGeom wg = five ? wino_geom_fwd5(d) : bwd ? wino_geom_bwd_data(d) : wino_geom_fwd(d);
+  for (int shared = 0; shared < 2; ++shared) {
+    if (shared) wg.beside_others();
+    if (five ? wino_pays5(wg, f) : wino_pays(wg, f)) r[shared] = TriRival{wg.us, wino_err(wg)};
+  }
 }
-inline bool tri_pays_fwd(const ConvDims& d, int flags, TriPlan* plan) {
-  return !fwd_gathers(d) && tri_pays(d, false, flags, plan, [&](int chain) { return plan_tri_fwd(d, chain); });
+inline bool tri_shape(const ConvDims& d, bool bwd) {
+  return (bwd ? d.st == 1 && d.K % 8 == 0 : d.C % 8 == 0 && !fwd_gathers(d)) && !conv1x1_stream_applies(d);
 }
-inline bool tri_pays_bwd_data(const ConvDims& d, int flags, TriPlan* plan) {
-  return d.st == 1 && tri_pays(d, true, flags, plan, [&](int chain) { return plan_tri_bwd_data(d, chain); });
+inline TriPlan plan_tri_pass(const ConvDims& d, bool bwd, int max_chain) {
+  return bwd ? plan_tri_bwd_data(d, max_chain) : plan_tri_fwd(d, max_chain);
+}
+// plan: what is to be launched where it pays.
+inline bool tri_pays(const ConvDims& d, bool bwd, int flags, TriPlan* plan) {
+  if (!tri_shape(d, bwd)) return false;
+  TriRival r[2];
+  tri_rivals(d, bwd, r);
+  const TriRival& other = r[flags & RH_ALGO_SHARED_GPU ? 1 : 0];
+  *plan = plan_tri_pass(d, bwd, tri_max_chain(other.err));
+  return plan->ok && plan->us < other.us;
+}
+// Scratch of the form where it pays, with the hint or without; 0 also where it cannot be more than `floor`: sized for every
+// batch up to a capacity from the largest down, many batches end there.
+inline size_t tri_bytes(const ConvDims& d, bool bwd, size_t floor) {
+  if (!tri_shape(d, bwd)) return 0;
+  // (plan_tri's copies, and 24 slices of all tiles, of 256 MB together, or 12 of up to 255 tiles and of an image that they share)
+  const int halo = bwd ? d.R - 1 - d.pad : d.pad, rows = bwd ? d.C : d.K, Ci = bwd ? d.K : d.C;
+  const double img = 6.0 * d.N * Ci * ((bwd ? d.P : d.H) + 2 * halo) * ((bwd ? d.Q : d.W) + 2 * halo);
+  const double out = 4.0 * (double)(bwd ? d.x_elems : d.y_elems);
+  const double parts = fmin(24.0 * out, 12.0 * ((256.0 + rows / 64) * 128 * 192 * 4 + out / d.N));
+  if (img + (6.5 * Ci * d.R * d.S + 48.0) * rows + parts + 4096.0 < (double)floor) return 0;
+  TriRival r[2];
+  tri_rivals(d, bwd, r);
+  size_t need = 0;
+  TriPlan p = {};
+  int chain = 0;
+  for (const TriRival& other : r) {
+    const int c = tri_max_chain(other.err);
+    if (c != chain) p = plan_tri_pass(d, bwd, c);
+    chain = c;
+    if (p.ok && p.us < other.us && p.total() > need) need = p.total();
+  }
+  return need;
 }
 // Filter gradient: the other forms take about 15 us, their multiply-adds at 50 (32-row tiles), 60 or 100 TFLOP/s, a quarter more
 // where taps are gathered or transformed, and 11 us a million weights of partial sums (fitted by hand to 308 timed calls, of

@@ -643,10 +643,13 @@ extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x,
                                      (flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT))))
     return RH_E_UNSUPPORTED;
   if (tri_allowed(flags)) {
-    TriPlan tp = plan_tri_fwd(d);
-    if (tri_forced(flags) && !tp.ok) return RH_E_UNSUPPORTED;
-    if (tri_forced(flags) && ws_bytes < tp.total()) return RH_E_WORKSPACE;
-    if (tri_forced(flags) || tri_pays_fwd(d, flags, &tp))
+    TriPlan tp = {};
+    if (tri_forced(flags)) {
+      tp = plan_tri_fwd(d);
+      if (!tp.ok) return RH_E_UNSUPPORTED;
+      if (ws_bytes < tp.total()) return RH_E_WORKSPACE;
+    }
+    if (tri_forced(flags) || (tri_pays(d, false, flags, &tp) && ws_bytes >= tp.total()))
       return launch_conv_tri(tp, false, x, w, y, alpha, beta, (flags & RH_FUSE_BIAS) ? bias : nullptr, (flags & RH_FUSE_RELU) ? 1 : 0,
                              nullptr, ws, stream);
   }

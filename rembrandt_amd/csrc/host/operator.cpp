@@ -217,7 +217,7 @@ int product_algo(const ExecOptions& o) { return !o.winograd ? RH_ALGO_DIRECT : o
 // Scratch is allocated once for batch_cap, but a pass may be called with any batch <= batch_cap and the library's
 // plans are not monotone in the batch (fewer result tiles make it cut the contraction into more slices, whose partial
 // sums can need more room than the full batch does): every scratch buffer is sized with the *_upto functions.
-size_t conv_ws_upto(const rh_conv_geom& g, int pass) { return rh_conv2d_workspace_bytes_upto(&g, pass); }
+size_t conv_ws_upto(const rh_conv_geom& g, int pass, int algo) { return rh_conv2d_workspace_bytes_for_upto(&g, pass, algo); }
 size_t bias_ws_upto(int batch, int K, int plane) { return rh_conv2d_bwd_bias_workspace_bytes_upto(batch, K, plane); }
 size_t bnorm_ws_upto(int batch, int C, int plane) { return rh_bnorm_workspace_bytes_upto(batch, C, plane); }
 // The affine GEMMs of a layer (out, B, in), (in, out, B), (in, B, out): B is the batch.
@@ -815,17 +815,15 @@ class Conv2dOperator : public Operator {
                   backward_enabled(capability), context);
     // one scratch buffer sized for the largest of the three passes (src/operator/mod.rs:1493-1507)
     const rh_conv_geom g = geom(batch_size);
-    size_t ws = conv_ws_upto(g, RH_CONV_FWD);
+    const int algo = product_algo(opts);
+    size_t ws = conv_ws_upto(g, RH_CONV_FWD, (opts.bf16_forward ? RH_MATH_BF16_MFMA_FP32ACC : 0) | algo), wa = 0;
     if (backward_enabled(capability)) {
-      ws = std::max(ws, conv_ws_upto(g, RH_CONV_BWD_FILTER));
-      ws = std::max(ws, conv_ws_upto(g, RH_CONV_BWD_DATA));
-      ws = std::max(ws, bias_ws_upto(g.N, g.K, (int)(out_dims_.w * out_dims_.h)));
+      wa = std::max(conv_ws_upto(g, RH_CONV_BWD_FILTER, algo), bias_ws_upto(g.N, g.K, (int)(out_dims_.w * out_dims_.h)));
+      ws = std::max(std::max(ws, wa), conv_ws_upto(g, RH_CONV_BWD_DATA, algo));
     }
     workspace_.reset(new DeviceBuffer<uint8_t>(std::max<size_t>(ws, 256), context));
     if (backward_enabled(capability) && opts.overlap_backward) {
       // the filter / bias gradients run on the second stream with scratch of their own
-      size_t wa = conv_ws_upto(g, RH_CONV_BWD_FILTER);
-      wa = std::max(wa, bias_ws_upto(g.N, g.K, (int)(out_dims_.w * out_dims_.h)));
       workspace_aux_.reset(new DeviceBuffer<uint8_t>(std::max<size_t>(wa, 256), context));
     }
     // the data gradient can zero what the ReLU below would have masked in a pass of its own
@@ -1272,6 +1270,7 @@ struct BNormConvUnit {
   Buf pre_act, pre_delta;  // the conv output the batch norm reads, and the gradient w.r.t. it
   bool backward = false;
   int conv_algo = 0;       // RH_ALGO_* bits of the unit's convolution calls
+  size_t aux_bytes = 0;    // scratch of the filter gradient
   bool beside = false;     // the last backward_params put the filter gradient on the second stream: the data gradient runs beside it
 
   void alloc(size_t batch, Dims3 in, size_t size, size_t stride, size_t pad, size_t out_channels, bool bwd, Ctx c) {
@@ -1300,11 +1299,8 @@ struct BNormConvUnit {
   int plane() const { return (int)(out_dims.w * out_dims.h); }
   size_t workspace_bytes() const {
     const rh_conv_geom g = geom(batch_cap);
-    size_t ws = std::max(conv_ws_upto(g, RH_CONV_FWD), bnorm_ws_upto(g.N, g.K, plane()));
-    if (backward) {
-      ws = std::max(ws, conv_ws_upto(g, RH_CONV_BWD_FILTER));
-      ws = std::max(ws, conv_ws_upto(g, RH_CONV_BWD_DATA));
-    }
+    size_t ws = std::max(conv_ws_upto(g, RH_CONV_FWD, conv_algo), bnorm_ws_upto(g.N, g.K, plane()));
+    if (backward) ws = std::max(std::max(ws, aux_bytes), conv_ws_upto(g, RH_CONV_BWD_DATA, conv_algo));
     return ws;
   }
   rh_stream_t s() const { return ctx->stream(); }
@@ -1381,10 +1377,6 @@ struct BNormConvUnit {
     }
     unwrap(rh_conv2d_bwd_filter(&g, 1.0f, in, pre_delta->as_ptr(), 1.0f, grad_weights->as_mut_ptr(), wg->as_mut_ptr(),
                                 wg->len(), conv_algo, sg), "conv2d backward filter");
-  }
-  size_t aux_workspace_bytes() const {
-    const rh_conv_geom g = geom(batch_cap);
-    return conv_ws_upto(g, RH_CONV_BWD_FILTER);
   }
   // in_delta = beta*in_delta + dconv^T(weights, pre_delta)
   void backward_data(size_t batch, float* in_delta, float beta, DeviceBuffer<uint8_t>& ws) {
@@ -1588,11 +1580,13 @@ class BNormUnitsOperator : public Operator {
     out_act_.reset(new DeviceBuffer<float>(out_dims.len() * batch_cap_, context_));
     out_delta_.reset(new DeviceBuffer<float>(out_dims.len() * batch_cap_, context_));
     size_t ws = 256;
+    if (bwd)
+      for (auto& u : units_) u.aux_bytes = conv_ws_upto(u.geom(batch_cap_), RH_CONV_BWD_FILTER, u.conv_algo);
     for (auto& u : units_) ws = std::max(ws, u.workspace_bytes());
     workspace_.reset(new DeviceBuffer<uint8_t>(ws, context_));
     if (bwd && opts_.overlap_backward) {
       size_t wa = 256;
-      for (auto& u : units_) wa = std::max(wa, u.aux_workspace_bytes());
+      for (auto& u : units_) wa = std::max(wa, u.aux_bytes);
       workspace_aux_.reset(new DeviceBuffer<uint8_t>(wa, context_));
     }
   }

@@ -45,10 +45,7 @@ def conv_geom(x_shape, w_shape, stride, pad):
 
 def conv_ws_bytes(g, pass_, algo):
     """Scratch of a convolution pass under `algo`."""
-    forced = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
-    if algo & forced == forced:
-        return lib().rh_conv2d_bf16x3_workspace_bytes(C.byref(g), pass_)
-    return lib().rh_conv2d_workspace_bytes(C.byref(g), pass_)
+    return lib().rh_conv2d_workspace_bytes_for(C.byref(g), pass_, algo)
 
 
 def conv_out_shape(g):

@@ -90,6 +90,8 @@ extern "C" {
   pub fn rh_conv2d_workspace_bytes(g: *const rh_conv_geom, pass: c_int) -> size_t;
   pub fn rh_conv2d_bf16x3_workspace_bytes(g: *const rh_conv_geom, pass: c_int) -> size_t;
   pub fn rh_conv2d_workspace_bytes_upto(g: *const rh_conv_geom, pass: c_int) -> size_t;
+  pub fn rh_conv2d_workspace_bytes_for(g: *const rh_conv_geom, pass: c_int, flags: c_int) -> size_t;
+  pub fn rh_conv2d_workspace_bytes_for_upto(g: *const rh_conv_geom, pass: c_int, flags: c_int) -> size_t;
   pub fn rh_conv2d_fwd(g: *const rh_conv_geom, alpha: c_float, x: *const f32, w: *const f32, beta: c_float,
                        y: *mut f32, bias: *const f32, ws: *mut c_void, ws_bytes: size_t, flags: c_int,
                        stream: rh_stream_t) -> c_int;

@@ -755,6 +755,45 @@ def test_conv2d_bf16x3_where_it_pays(dev):
         assert bool(((y - other).norm() <= 2e-6 * other.norm()).item())
 
 
+def test_conv2d_bf16x3_without_room_for_it(dev):
+    """RH_ALGO_BF16X3 alone with the scratch of a caller that does not know the bit, in all passes and with a stride: taken, in the
+    form that runs without it; with room for the form, that form.  With RH_ALGO_DIRECT, which leaves no other, refused."""
+    import ctypes as C
+    lib, X3 = _lib.lib(), _lib.RH_ALGO_BF16X3
+    for Nn, Cc, H, K, R, st, pad in ((37, 256, 13, 384, 3, 1, 1), (24, 64, 56, 128, 3, 2, 1)):
+        say("bf16x3 without room", (Nn, Cc, H, K, R, st))
+        g = _lib.ConvGeom(Nn, Cc, H, H, K, R, R, st, pad)
+        P = (H + 2 * pad - R) // st + 1
+        x, w, dy = (T(synth.normal(49, 1 + i, s), dev) for i, s in enumerate(((Nn, Cc, H, H), (K, Cc, R, R), (Nn, K, P, P))))
+        for pass_, name in ((_lib.RH_CONV_FWD, "fwd"), (_lib.RH_CONV_BWD_DATA, "bwd_data"), (_lib.RH_CONV_BWD_FILTER, "bwd_filter")):
+            plain, need = lib.rh_conv2d_workspace_bytes(C.byref(g), pass_), lib.rh_conv2d_workspace_bytes_for(C.byref(g), pass_, X3)
+            ws = torch.empty(max(plain, need) + 256, dtype=torch.uint8, device=dev)
+            at = (ws.data_ptr() + 255) // 256 * 256
+
+            def call(flags, room):
+                out = torch.zeros_like({"fwd": dy, "bwd_data": x, "bwd_filter": w}[name])
+                o = out.data_ptr()
+                if name == "fwd":
+                    rc = lib.rh_conv2d_fwd(C.byref(g), 1.0, x.data_ptr(), w.data_ptr(), 0.0, o, None, at, room, flags, None)
+                elif name == "bwd_data":
+                    rc = lib.rh_conv2d_bwd_data(C.byref(g), 1.0, w.data_ptr(), dy.data_ptr(), 0.0, o, at, room, flags, None)
+                else:
+                    rc = lib.rh_conv2d_bwd_filter(C.byref(g), 1.0, x.data_ptr(), dy.data_ptr(), 0.0, o, at, room, flags, None)
+                torch.cuda.synchronize()
+                return rc, out
+            (rc0, without), (rc1, small) = call(0, plain), call(X3, plain)
+            assert rc0 == 0 and rc1 == 0, (name, rc0, rc1)
+            (rc2, _), tags = profile_tags(lambda: call(X3, need))
+            took = any(t.startswith("conv_%s_tri_" % name) for t in tags)
+            assert rc2 == 0 and (took or name == "bwd_filter" and st == 2), (name, tags)
+            if need > plain or not took:
+                assert torch.equal(without, small), name
+            if st == 1:
+                forced = lib.rh_conv2d_bf16x3_workspace_bytes(C.byref(g), pass_)
+                if forced > plain:
+                    assert call(X3 | _lib.RH_ALGO_DIRECT, plain)[0] == _lib.RH_E_WORKSPACE, name
+
+
 def test_conv2d_bf16x3_on_one_row_tile_of_filters(dev):
     """Layers of up to 128 filters take the form where it is the faster one as others do: the filter gradient (98 -> 64, 139 -> 92
     us) and the 5x5 forward pass (198 -> 141 us), no further from 64-bit sums than the Winograd form."""

@@ -187,6 +187,46 @@ def test_scratch_sized_once_covers_every_smaller_batch():
         assert all(lib.rh_bnorm_workspace_bytes(n, C_, plane) <= room for n in range(1, 257))
 
 
+BF16X3_GEOMS = [   # N, C, H, K, R, stride, pad: of the benchmark networks, then small and odd ones
+    (256, 64, 56, 64, 3, 1, 1), (256, 64, 56, 128, 3, 2, 1), (256, 64, 56, 128, 1, 2, 0), (256, 128, 28, 128, 3, 1, 1),
+    (256, 512, 7, 512, 3, 1, 1), (256, 96, 27, 256, 5, 1, 2), (256, 384, 13, 256, 3, 1, 1), (128, 1024, 6, 1024, 1, 1, 0),
+    (128, 32, 16, 32, 5, 1, 2), (64, 32, 8, 64, 5, 1, 2), (100, 8, 5, 9, 1, 1, 0), (40, 24, 9, 40, 3, 4, 1), (70, 72, 1, 1000, 1, 1, 0),
+]
+
+
+@pytest.mark.parametrize("geom", BF16X3_GEOMS, ids=str)
+def test_bf16x3_scratch_is_for_callers_that_allow_the_form(geom):
+    """rh_conv2d_workspace_bytes does not know of the split-operand form; rh_conv2d_workspace_bytes_for does where the flags allow
+    it.  The *_upto form, which leaves out batches whose need cannot be the largest, is the largest of all batches'."""
+    lib = _lib.lib()
+    cap, c, extent, k, size, st, pad = geom
+    X3 = _lib.RH_ALGO_BF16X3
+    for pass_ in (_lib.RH_CONV_FWD, _lib.RH_CONV_BWD_FILTER, _lib.RH_CONV_BWD_DATA):
+        for flags in (0, X3, X3 | _lib.RH_ALGO_DIRECT):
+            most = 0
+            for n in range(1, cap + 1):
+                g = _lib.ConvGeom(n, c, extent, extent, k, size, size, st, pad)
+                plain, need = lib.rh_conv2d_workspace_bytes(C.byref(g), pass_), lib.rh_conv2d_workspace_bytes_for(C.byref(g), pass_, flags)
+                assert need >= plain and (flags or need == plain)
+                assert need == lib.rh_conv2d_workspace_bytes_for(C.byref(g), pass_, flags | _lib.RH_ALGO_SHARED_GPU)
+                most = max(most, need)
+            g = _lib.ConvGeom(cap, c, extent, extent, k, size, size, st, pad)
+            assert lib.rh_conv2d_workspace_bytes_for_upto(C.byref(g), pass_, flags) == most, (pass_, flags)
+            if not flags:
+                assert lib.rh_conv2d_workspace_bytes_upto(C.byref(g), pass_) == most
+
+
+def test_conv_scratch_without_the_bf16x3_bit():
+    """What a caller without the bit needs is what the other forms need: 13 MB where the split copies take 52, 131 where they take
+    159, 355 where they take 483."""
+    lib = _lib.lib()
+    for (n, c, extent, k, size, pad), pass_, mb in (((128, 1024, 6, 1024, 1, 0), _lib.RH_CONV_FWD, 14), ((256, 96, 27, 256, 5, 2), _lib.RH_CONV_FWD, 132),
+                                                    ((256, 96, 27, 256, 5, 2), _lib.RH_CONV_BWD_FILTER, 356)):
+        g = _lib.ConvGeom(n, c, extent, extent, k, size, size, 1, pad)
+        assert lib.rh_conv2d_workspace_bytes(C.byref(g), pass_) < mb * 1e6
+        assert lib.rh_conv2d_workspace_bytes_for(C.byref(g), pass_, _lib.RH_ALGO_BF16X3) > 1.15 * mb * 1e6
+
+
 def test_rng_is_a_pure_function_of_seed_stream_index():
     a = synth.normal(5, 7, (1000,))
     assert np.array_equal(a, synth.normal(5, 7, (1000,)))
