@@ -378,6 +378,25 @@ static BwdFilterSoffPlan plan_bwd_filter_soff(const ConvDims& d) {
   return p;
 }
 
+// (The error of the form otherwise taken, in the units of tri_max_chain: the engine's and the gathering kernels' as engine_err; the
+// Winograd form's 0.35 a tile group of its slices at least, 0.35 to 0.53 in 16 calls measured.)
+bool tri_pays_bwd_filter(const ConvDims& d, const TriFilterPlan& t) {
+  if (!t.ok) return false;
+  const int bm = pick_bm(d.K);
+  const double terms = (double)d.N * d.P * d.Q, flops = 2.0 * (double)d.w_elems * terms;
+  const double other = (d.R * d.S > 1 ? 1.25 : 1.0) * (15.0 + flops / (bm >= 96 ? 100e6 : bm == 64 ? 60e6 : 50e6)) + 11e-6 * (double)d.w_elems;
+  if (t.us >= 0.9 * other) return false;
+  double err;
+  const WinoFilterPlan wp = wino_shape(d) ? plan_wino_bwd_filter(d) : WinoFilterPlan{};
+  if (wino_filter_pays(d, wp)) {
+    err = 0.35 * wp.stages;
+  } else {
+    const BwdFilterSoffPlan sp = plan_bwd_filter_soff(d);
+    err = 0.0335 * terms / (sp.ok && use_soff_bwd_filter(d) ? sp.splits : plan_bwd_filter(d).splits);
+  }
+  return cdiv(t.groups / 2, t.splits) <= tri_max_chain(err);
+}
+
 // dst[n][pix][c] (pix over Hp x Wp, zero halo) = src[n][c][h][w]: 32 x 32 tiles through LDS so that both
 // the reads (along w) and the writes (along c) are contiguous.
 __device__ __forceinline__ void nchw_to_nhwc_body(float* __restrict__ lds, int bx, int by, int bz,

@@ -620,6 +620,10 @@ inline bool tri_forced(int flags) { return tri_allowed(flags) && (flags & RH_ALG
 // at 36, 1.95e-7 at 72), of the engine 0.0335 a term, of the Winograd form as in wino_stages_at_most, of the staged form
 // 0.032 a term of its two chains and four more (0.09 2^-48: a rounding's variance).  The chain allowed is the one with three
 // quarters of the other form's: half zeros, as behind a ReLU, spare the shorter chains more roundings (1.2 on the square).
+// Measured where the form is taken, relative to the other form's error: activations, filters and deltas of AlexNet, NIN and CIFAR-10
+// steps 0.62, 0.53 and 0.49 in the geometric mean (forward, data and filter gradient, 64 calls), 0.97 at most.  Sums of operands of
+// one sign on both sides are another matter, slices make them more exact than their chains alone: uniform [0, 1) on all sides
+// 0.8 to 0.9 in the geometric mean of 137 calls, but up to 1.9 beside a form of many slices, 3e-7 and less in all.
 inline int tri_max_chain(double other) { const double n = 0.75 * other / 0.0525; return n < 1.0 ? 1 : n < 1e6 ? (int)n : 1000000; }
 inline double engine_err(const SoffPlan& p, int terms) { return 0.0335 * terms / p.splits; }
 inline double staged_err(const LdsConvPlan& p, int R) {
@@ -694,14 +698,9 @@ inline size_t tri_bytes(const ConvDims& d, bool bwd, size_t floor) {
 // Filter gradient: the other forms take about 15 us, their multiply-adds at 50 (32-row tiles), 60 or 100 TFLOP/s, a quarter more
 // where taps are gathered or transformed, and 11 us a million weights of partial sums (fitted by hand to 308 timed calls, of
 // which this form is then chosen in 188, 1.53 times as fast in the geometric mean).  1x1 layers need 384 channels or so to be
-// worth two split copies.
-inline bool tri_pays_bwd_filter(const ConvDims& d, const TriFilterPlan& t) {
-  if (!t.ok) return false;
-  const int bm = pick_bm(d.K);
-  const double flops = 2.0 * (double)d.w_elems * d.N * d.P * d.Q;
-  const double other = (d.R * d.S > 1 ? 1.25 : 1.0) * (15.0 + flops / (bm >= 96 ? 100e6 : bm == 64 ? 60e6 : 50e6)) + 11e-6 * (double)d.w_elems;
-  return t.us < 0.9 * other;
-}
+// worth two split copies.  Its slices are short enough for the chain limit almost everywhere: it turns down 4 of 5493 calls (30
+// layers at every batch up to 256), of one to four images.
+bool tri_pays_bwd_filter(const ConvDims& d, const TriFilterPlan& t);
 
 int launch_conv_lds(const LdsConvPlan& pl, bool bwd, int N, int Ci, int H, int W, int rows, int P, int Q, int R, int halo,
                     const float* in, const float* w, float* out, float alpha, float beta, const float* bias, int relu,

@@ -626,27 +626,109 @@ def test_conv2d_bf16x3_strided_bwd_data(dev, case):
     assert torch.equal(torch.isnan(a), torch.isnan(b)) and torch.equal(torch.isinf(a), torch.isinf(b))
 
 
-@pytest.mark.parametrize("relu", [False, True], ids=["normal", "half_zeros"])
-@pytest.mark.parametrize("case", [(16, 256, 13, 13, 384, 3, 1), (64, 128, 28, 28, 128, 3, 1), (9, 96, 27, 27, 256, 5, 2), (32, 64, 28, 28, 64, 3, 1)], ids=str)
-def test_conv2d_bf16x3_error(dev, case, relu):
-    """Error against 64-bit sums: within the bound of the form's own chain, and where the library takes it by itself no larger than
-    that of the form it replaces (staged, Winograd).  The large products add to a sum of 16 terms per MFMA; with two roundings each (the instruction's own order is not
-    documented) a chain of n steps has a relative rms error of sqrt(0.09 * 2 n + 4) 2^-24 (a rounding's variance as in
+# Layers with the passes that the library takes in this form by itself: under a chain limit that asks for slices, against the staged,
+# the engine's and the Winograd form, with stride, with one image and with nine (a group of eight and one more in the filter gradient)
+X3_ERROR_CASES = [
+    # N, C, H, K, R, stride, pad, passes
+    (16, 256, 13, 384, 3, 1, 1, "fdw"),
+    (9, 96, 27, 256, 5, 1, 2, "fdw"),
+    (24, 256, 14, 256, 3, 1, 1, "fdw"),
+    (64, 512, 7, 512, 3, 1, 1, "fdw"),
+    (24, 128, 28, 128, 3, 1, 1, "fdw"),
+    (64, 128, 28, 128, 3, 1, 1, "w"),
+    (32, 64, 28, 64, 3, 1, 1, "w"),
+    (50, 1024, 6, 1024, 1, 1, 0, "fdw"),
+    (50, 128, 28, 256, 3, 2, 1, "fdw"),
+    (50, 64, 56, 128, 3, 2, 1, "fdw"),
+    (1, 384, 13, 384, 3, 1, 1, ""),
+    (1, 512, 7, 512, 3, 1, 1, ""),     # filter gradient: faster by the estimates, but one chain of 25 steps where the engine's is of 49 terms
+]
+
+
+def _conv_sums64(x, w, dy, st, pad):
+    """Forward, data gradient and filter gradient of device tensors as plain matrix products in 64 bits."""
+    import torch.nn.functional as F
+    (Nn, C, H, W), (K, _, R, S), (P, Q) = x.shape, w.shape, dy.shape[2:]
+    w2, y, dx = w.double().reshape(K, -1), torch.empty(dy.shape, dtype=torch.float64, device=x.device), torch.empty(x.shape, dtype=torch.float64, device=x.device)
+    wt, dw = w2.t().contiguous(), torch.zeros_like(w2)
+    step = max(1, 10 ** 8 // (C * R * S * P * Q))
+    for i in range(0, Nn, step):
+        n = min(step, Nn - i)
+        col = F.unfold(x[i:i + n].double(), (R, S), padding=pad, stride=st).permute(1, 0, 2).reshape(C * R * S, -1).contiguous()
+        rows = dy[i:i + n].double().reshape(n, K, -1).permute(1, 0, 2).reshape(K, -1).contiguous()
+        y[i:i + n] = (w2 @ col).reshape(K, n, P * Q).permute(1, 0, 2).reshape(n, K, P, Q)
+        dx[i:i + n] = F.fold((wt @ rows).reshape(C * R * S, n, P * Q).permute(1, 0, 2).contiguous(), (H, W), (R, S), padding=pad, stride=st)
+        dw += rows @ col.t().contiguous()
+    return y, dx, dw.reshape(w.shape)
+
+
+def _chain_bound(terms):
+    """The large products add to a sum of 16 terms per MFMA; with two roundings each at the size of the sum (the instruction's own
+    order is not documented) a chain of n steps has a relative rms error of sqrt(0.09 * 2 n + 4) 2^-24 (a rounding's variance as in
     test_conv2d_staged_operands_error; four more for the small products' own chain and the result).  A quarter on top."""
-    Nn, C, H, W, K, R, pad = case
-    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT
-    x, w = synth.normal(35, 1, (Nn, C, H, W)), synth.normal(35, 2, (K, C, R, R))
-    if relu:
-        x = np.maximum(x, 0.0)
-    dy = synth.normal(35, 3, (Nn, K, H, W))
-    xd, wd, dyd = T(x, dev), T(w, dev), T(dy, dev)
-    for ref, terms, run in (
-            (O.conv2d_fwd(x, w, 1, pad), C * R * R, lambda algo: ops.conv2d_fwd(xd, wd, 1, pad, algo=algo)),
-            (O.conv2d_bwd_data(w, dy, x.shape, 1, pad), K * R * R, lambda algo: ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=algo))):
-        err = float(np.linalg.norm(N(run(X3)).astype(np.float64) - ref) / np.linalg.norm(ref.astype(np.float64)))
-        assert err <= 1.25 * 2.0 ** -24 * (0.18 * terms / 16 + 4) ** 0.5, (terms, err)
-        auto, before = (float(np.linalg.norm(N(run(algo)).astype(np.float64) - ref)) for algo in (_lib.RH_ALGO_BF16X3, 0))
-        assert auto <= before, (auto, before)
+    return 1.25 * 2.0 ** -24 * (0.18 * terms / 16 + 4) ** 0.5
+
+
+@pytest.mark.parametrize("data", ["normal", "half_zeros", "positive"])
+@pytest.mark.parametrize("case", X3_ERROR_CASES, ids=str)
+def test_conv2d_bf16x3_error(dev, case, data):
+    """Error against 64-bit sums, all passes: within the bound of the form's own chain, and where the library takes it by itself (it
+    does in the passes named) no larger than that of the form it replaces.  positive: all three tensors of one sign, whose sums grow
+    with every term; such operands are held to the bound only (tri_max_chain is made for others)."""
+    Nn, C, H, K, R, st, pad, takes = case
+    say("bf16x3 error", case, data)
+    P = (H + 2 * pad - R) // st + 1
+    make = synth.uniform if data == "positive" else synth.normal
+    x, w, dy = (T(make(35, 1 + i, s), dev) for i, s in enumerate(((Nn, C, H, H), (K, C, R, R), (Nn, K, P, P))))
+    if data == "half_zeros":
+        x = x.clamp_min(0.0)
+    refs = _conv_sums64(x, w, dy, st, pad)
+    for key, name, terms, ref, run in (("f", "fwd", C * R * R, refs[0], lambda algo: ops.conv2d_fwd(x, w, st, pad, algo=algo)),
+                                       ("d", "bwd_data", K * R * R, refs[1], lambda algo: ops.conv2d_bwd_data(w, dy, x.shape, st, pad, algo=algo)),
+                                       ("w", "bwd_filter", Nn * P * P, refs[2], lambda algo: ops.conv2d_bwd_filter(x, dy, w.shape, st, pad, algo=algo))):
+        auto, tags = profile_tags(lambda: run(_lib.RH_ALGO_BF16X3))
+        assert any(t.startswith("conv_%s_tri_" % name) for t in tags) == (key in takes), (name, tags)
+        form = auto if key in takes else None if key == "d" and st > 1 else run(_lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT)
+        if form is None:
+            continue
+        err = float((form.double() - ref).norm() / ref.norm())
+        assert err <= _chain_bound(terms), (name, terms, err)
+        if key in takes and data != "positive":
+            before = float((run(0).double() - ref).norm() / ref.norm())
+            assert err <= before, (name, err, before)
+
+
+@pytest.mark.parametrize("case", [(9, 16, 14, 11, 40, 3, 5, 1, 2), (3, 24, 9, 12, 72, 1, 4, 1, 0), (8, 40, 12, 9, 64, 5, 1, 1, 1),
+                                  (5, 16, 13, 10, 33, 2, 3, 2, 1), (24, 64, 30, 28, 128, 2, 3, 2, 1)], ids=str)
+def test_conv2d_bf16x3_filters_that_are_not_square(dev, case):
+    """R != S through the C interface: forward and filter gradient have the form; the data gradient has it by residue classes, with a
+    stride, and with RH_ALGO_DIRECT is RH_E_UNSUPPORTED."""
+    import ctypes as C
+    Nn, Cc, H, W, K, R, S, st, pad = case
+    say("bf16x3 not square", case)
+    lib, X3 = _lib.lib(), _lib.RH_ALGO_BF16X3
+    forced = X3 | _lib.RH_ALGO_DIRECT
+    g = _lib.ConvGeom(Nn, Cc, H, W, K, R, S, st, pad)
+    P, Q = (H + 2 * pad - R) // st + 1, (W + 2 * pad - S) // st + 1
+    x, w, dy = (T(synth.normal(51, 1 + i, s), dev) for i, s in enumerate(((Nn, Cc, H, W), (K, Cc, R, S), (Nn, K, P, Q))))
+    y_ref, dx_ref, dw_ref = _conv_sums64(x, w, dy, st, pad)
+    size = max(lib.rh_conv2d_workspace_bytes_for(C.byref(g), p, f) for p in range(3) for f in (X3, forced))
+    ws = torch.empty(size + 256, dtype=torch.uint8, device=dev)
+    at = (ws.data_ptr() + 255) // 256 * 256
+    y, dw, dx, dx0 = torch.empty_like(dy), torch.empty_like(w), torch.zeros_like(x), torch.zeros_like(x)
+    assert lib.rh_conv2d_fwd(C.byref(g), 1.0, x.data_ptr(), w.data_ptr(), 0.0, y.data_ptr(), None, at, size, forced, None) == 0
+    assert lib.rh_conv2d_bwd_filter(C.byref(g), 1.0, x.data_ptr(), dy.data_ptr(), 0.0, dw.data_ptr(), at, size, forced, None) == 0
+    bwd_data = lambda out, flags: lib.rh_conv2d_bwd_data(C.byref(g), 1.0, w.data_ptr(), dy.data_ptr(), 0.0, out.data_ptr(), at, size, flags, None)
+    assert bwd_data(dx, forced) == _lib.RH_E_UNSUPPORTED
+    rc, tags = profile_tags(lambda: bwd_data(dx, X3))
+    classes = any(t.startswith("conv_bwd_data_tri_") for t in tags)
+    assert rc == 0 and classes == (case[0] == 24), tags
+    assert bwd_data(dx0, 0) == 0
+    torch.cuda.synchronize()
+    for got, ref, terms in ((y, y_ref, Cc * R * S), (dw, dw_ref, Nn * P * Q)) + (((dx, dx_ref, K * R * S),) if classes else ()):
+        err = float((got.double() - ref).norm() / ref.norm())
+        assert err <= _chain_bound(terms), (err, terms)
+    assert classes or torch.equal(dx, dx0)
 
 
 def test_conv2d_bf16x3_infinities_and_largest_floats(dev):
