@@ -202,8 +202,17 @@ static int skinny_mode(int m, int n, int k) {
 // forward 40 -> 33, 63 -> 38, 66 -> 42, 94 -> 65, 164 -> 112, data gradient the same within 5 %, filter gradient 31 -> 33,
 // 46 -> 46, 56 -> 56, 94 -> 68, 155 -> 114.  The split copy is a launch of its own, 3 to 6 us: 1024 -> 512 is slower in both
 // passes at every batch (37 images 14.0 -> 14.9), 2048 -> 1024 faster up to 128 (17.3 -> 15.1) and slower at 200 (22.6 -> 24.6).
-// A block of 32 rows is bound by the weights' bytes in either form, and only many of them cover the copy.  Filter gradients
-// of up to 64 images are bound by the result's bytes; those of 65 to 96 gain where the result is large.
+// Where the lines lie, this form's time over the engine's, forward and data gradient:
+//   33 to 128 rows  1.6 million weights (3136 -> 512) 0.90 to 1.03, from 2 million on 0.63 to 0.96
+//   more            1.6 to 2.4 million 0.79 to 1.23 at 160 and 200 rows, from 4.1 million on 0.48 to 0.95
+//   up to 32        6 to 12.6 million 0.95 to 1.19, 16.8 million (4096 -> 4096) 0.88 to 1.01
+// A block of up to 32 rows is bound by the weights' bytes in either form: only many of them cover the copy, and not where a few blocks
+// are left to a round of their own (two to a CU; data gradient of 4096 columns in 512 blocks 0.88 to 0.96, 9216 in 576 0.97 to 0.99,
+// 12544 in 588 1.02 to 1.10, 6144 in 528 1.06 to 1.10, 5120 -> 5120 in 520 1.07 to 1.19); forward, a result of few columns in many slices does not (8192 -> 2048 in 32
+// 1.03 to 1.06, 8192 -> 4096 in 16 0.79 to 0.83).  AlexNet's bf16 forward pass with its affine layers in this form: 8, 16, 32, 64 images
+// 175 -> 168, 203 -> 197, 276 -> 270, 374 -> 354 us.
+// Filter gradients of up to 64 images are bound by the result's bytes (4096 x 4096: 32 images 1.08, 48 1.02, 64 0.94); those of 65 to 96
+// gain where the result is large (0.82 to 0.88 from 16.8 million on, 0.85 to 1.05 below).
 static bool sgemm_tri_pays(bool a_trans, bool b_trans, int m, int n, int k, SgemmTriPlan* plan) {
   const long long mk = (long long)m * k, mn = (long long)m * n;
   *plan = SgemmTriPlan{};
@@ -213,6 +222,10 @@ static bool sgemm_tri_pays(bool a_trans, bool b_trans, int m, int n, int k, Sgem
     return false;
   }
   *plan = plan_sgemm_tri(a_trans, b_trans, m, n, k);
+  if (!b_trans && n <= 32) {
+    const int last = cdiv(m, 128) * plan->splits % 512;
+    if ((a_trans && m < 4096) || (last > 0 && last < 64)) return false;
+  }
   return plan->ok && cdiv(plan->groups / 2, plan->splits) <= tri_max_chain(0.0335 * k / plan_sgemm(m, n, k).splits);
 }
 

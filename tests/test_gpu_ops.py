@@ -1187,7 +1187,8 @@ def test_sgemm_bf16x3_small_operands(dev, case, exponent):
 def test_sgemm_bf16x3_where_it_pays(dev):
     """RH_ALGO_BF16X3 alone: the form on large affine products, with no larger error against 64-bit sums than the form that it
     replaces, half of the activations zeros; the other forms' bits elsewhere and where the scratch does not hold it."""
-    for tA, tB, m, n, k, takes in ((1, 0, 4096, 32, 4096, True), (1, 0, 4096, 31, 4080, False), (1, 0, 1000, 33, 4096, True), (1, 0, 512, 64, 1024, False),
+    for tA, tB, m, n, k, takes in ((1, 0, 4096, 32, 4096, True), (1, 0, 2048, 16, 8192, False), (0, 0, 4096, 24, 4096, True), (0, 0, 6144, 8, 4096, False),
+                                   (0, 0, 9216, 32, 4096, True), (0, 0, 9216, 33, 4096, True), (1, 0, 4096, 31, 4080, False), (1, 0, 1000, 33, 4096, True), (1, 0, 512, 64, 1024, False),
                                    (1, 0, 1000, 129, 4096, True), (1, 0, 1024, 200, 2048, False), (0, 0, 4096, 37, 1000, True), (0, 0, 4096, 256, 4096, True),
                                    (0, 1, 4096, 4096, 50, True), (0, 1, 4096, 1000, 96, False), (0, 1, 4096, 1000, 97, True), (0, 1, 4096, 4096, 256, True),
                                    (0, 1, 800, 500, 128, False)):
