@@ -60,17 +60,21 @@ typedef void* rh_stream_t; /* hipStream_t */
                                              blocks (the Winograd kernels' sliced tail blocks) are not taken: beside
                                              other work the idle units of that round are not idle (measured: the
                                              ResNet-18 template step 26.5 -> 26.1 ms).  Grids of less than one round
-                                             are sliced with the hint as without.  Same result up to summation order. */
+                                             are sliced with the hint as without, and so is the last round of the form of
+                                             RH_ALGO_BF16X3 (whole blocks there: the same step 22.4 -> 22.6 ms, AlexNet's and
+                                             NIN's as before).  Same result up to summation order. */
 #define RH_ALGO_BF16X3             0x2000 /* the contraction may also run on bf16 matrix instructions, every fp32 operand value as
                                              the exact sum of three bf16 values (six products a pair, fp32 accumulate): fp32
                                              precision, no operand is rounded.  Results with an operand that has no such sum
                                              (an infinity, a NaN, a float that rounds to an infinity in bf16, one below 2^-110
                                              with bits under bf16's smallest value, 2^-133) are formed on fp32 instructions, at
                                              4 to 8 times the time where all are.  Alone or with the hint: where it is expected to
-                                             be the fastest form.  With RH_ALGO_DIRECT: this form, RH_E_UNSUPPORTED where the
-                                             geometry has none (forward and stride-1 backward-data need a contracted channel
-                                             count that is a multiple of 8).  No effect beside the other RH_ALGO_* bits and
-                                             RH_MATH_BF16_MFMA_FP32ACC. */
+                                             be the fastest form and the scratch holds it (rh_conv2d_workspace_bytes_for).
+                                             With RH_ALGO_DIRECT: this form, RH_E_UNSUPPORTED where the geometry has none:
+                                             forward and backward-data need a contracted channel count that is a multiple of
+                                             8, and backward-data stride 1 and R = S (of stride 2 to 4, any R and S, it has
+                                             the form without RH_ALGO_DIRECT only).  No effect beside the other RH_ALGO_* bits
+                                             and RH_MATH_BF16_MFMA_FP32ACC. */
 
 const char* rh_version(void);
 /* Status of the most recent launch made by a void `rembrandt_kernel_*` entry point on this thread. */
