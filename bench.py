@@ -402,9 +402,25 @@ def _mfma_frac(kernels):
 def conv_sweep_leg(iters, warmup):
     """Forward, backward-data and backward-filter of the three sweep shapes, each call timed alone (HIP events on the
     stream the kernels run on; a call includes the operand copies it makes): ms, TFLOP/s against the fp32 matrix peak and
-    algorithmic bytes (x, w, y once) per second against the HBM peak: the 1x1 shape sits on the ridge of both roofs."""
+    algorithmic bytes (x, w, y once) per second against the HBM peak: the 1x1 shape sits on the ridge of both roofs.  The figures
+    are of calls on fp32 instructions; `as_operators_call` is the same call with RH_ALGO_BF16X3, the operators' default, and where
+    that takes the split-operand form `frac_mfma` is its six bf16 products for an fp32 one against the bf16 peak."""
     import torch
-    from rembrandt_amd import ops
+    from rembrandt_amd import _lib, ops
+    from rembrandt_amd.kernel_bench import launched_tags
+
+    def time_call(fn):
+        for _ in range(warmup):
+            fn()
+        torch.cuda.synchronize()
+        s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
+        s.record()
+        for _ in range(iters):
+            fn()
+        e.record()
+        torch.cuda.synchronize()
+        return s.elapsed_time(e) / iters
+
     dev = torch.device("cuda:0")
     out = {}
     for name, (N, C, H, W, K, R, st, pad) in SWEEP.items():
@@ -417,21 +433,12 @@ def conv_sweep_leg(iters, warmup):
         dw, dx = torch.zeros_like(w), torch.zeros_like(x)
         flops = 2.0 * y.numel() * C * R * R
         byts = 4.0 * (x.numel() + w.numel() + y.numel())
-        calls = {"fwd": lambda: ops.conv2d_fwd(x, w, st, pad, y=y),
-                 "bwd_data": lambda: ops.conv2d_bwd_data(w, dy, x.shape, st, pad, dx=dx),
-                 "bwd_filter": lambda: ops.conv2d_bwd_filter(x, dy, w.shape, st, pad, dw=dw)}
+        calls = {"fwd": lambda algo: ops.conv2d_fwd(x, w, st, pad, y=y, algo=algo),
+                 "bwd_data": lambda algo: ops.conv2d_bwd_data(w, dy, x.shape, st, pad, dx=dx, algo=algo),
+                 "bwd_filter": lambda algo: ops.conv2d_bwd_filter(x, dy, w.shape, st, pad, dw=dw, algo=algo)}
         row = {"gflop": flops / 1e9, "algorithmic_mb": byts / 1e6}
         for pname, fn in calls.items():
-            for _ in range(warmup):
-                fn()
-            torch.cuda.synchronize()
-            s, e = torch.cuda.Event(enable_timing=True), torch.cuda.Event(enable_timing=True)
-            s.record()
-            for _ in range(iters):
-                fn()
-            e.record()
-            torch.cuda.synchronize()
-            ms = s.elapsed_time(e) / iters
+            ms = time_call(lambda: fn(0))
             # `tflops` counts the direct form's multiply-adds (the sweep's metric); where the library takes the Winograd
             # form, `frac_mfma` is what its kernel executes against the matrix peak
             wino = ops.conv2d_winograd_flops(x.shape, w.shape, st, pad, pname)
@@ -440,6 +447,13 @@ def conv_sweep_leg(iters, warmup):
                           "gbs": byts / ms / 1e6, "frac_hbm": byts / ms / 1e6 / PEAK_HBM_GBS}
             if wino:
                 row[pname].update({"form": "winograd F(2x2,3x3)", "executed_tflops": wino / ms / 1e9})
+            call = lambda: fn(_lib.RH_ALGO_BF16X3)
+            split = any("_tri_" in t for t in launched_tags(call))
+            ms = time_call(call)
+            row[pname]["as_operators_call"] = {"ms": ms, "tflops": flops / ms / 1e9, "form": "split operands" if split else "as above"}
+            if split:
+                row[pname]["as_operators_call"].update({"executed_tflops": 6.0 * flops / ms / 1e9,
+                                                        "frac_mfma": 6.0 * flops / ms / 1e9 / PEAK_BF16_MFMA_TFLOPS})
         out[name] = row
         del x, w, y, dy, dw, dx
     return out

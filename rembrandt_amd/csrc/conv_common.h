@@ -609,7 +609,8 @@ bool conv1x1_stream_applies(const ConvDims& d);
 // Where a caller that allows it (RH_ALGO_BF16X3) gets the form of exactly split operands: where its expected time is below
 // that of the form taken otherwise.  The engine's estimate was fitted to 3x3 and 5x5 stride-1 layers and is 10 to 25 % short on
 // others, hence the tenth.  Over 308 timed forward calls (22 layers at 14 batches) the forms chosen so are 1.27 times as fast as
-// without it, geometric mean, 1.02 times slower at worst.  1x1 layers of up to 128 channels keep the streaming kernels, which
+// without it, geometric mean; of 900 calls of all passes the slowest beside the form replaced are 384 -> 1024 3x3 6x6 data gradients
+// (batch 24 56 -> 60 us, 90 129 -> 137) and 256 -> 384 13x13 b256 (355 -> 370).  1x1 layers of up to 128 channels keep the streaming kernels, which
 // read their operands where they lie (96 -> 96 54x54 b128 82 us against 158).  Winograd -> this form on one row tile of filters:
 // 64 -> 128 5x5 24x24 b128 forward 198 -> 141 us, 128 -> 128 3x3 28x28 filter gradient b37, 64, 256 98 -> 64, 139 -> 92, 466 -> 349.
 inline bool tri_allowed(int flags) {

@@ -10,7 +10,8 @@
 // Precision.  The five small products of a pair have accumulators of their own, added to the large product's behind the
 // loop: one rounding at the size of the sum per 16 terms instead of one per two.  Relative error of chains of 256, 1152 and
 // 3456 terms against 64 bits, N(0,1) data: 0.9e-7, 2.0e-7 and 3.6e-7, the fp32 instruction 2.9e-7, 6.1e-7 and 10.4e-7 (with
-// one set of accumulators 2.4e-7, 5.2e-7 and 9.2e-7, and above the fp32 instruction where half of one operand is zero).
+// one set of accumulators 2.4e-7, 5.2e-7 and 9.2e-7, and above the fp32 instruction where half of one operand is zero).  Operands of
+// one sign, uniform [0, 1), chains of 576, 1152, 2304 and 6400 terms: 1.2e-7, 1.7e-7, 2.3e-7 and 4.2e-7, the fp32 instruction at 6400 11e-7.
 //
 // Values without such a sum: infinities and NaNs, the floats that round to an infinity in bf16, and below 2^-110 those whose
 // last bits lie under bf16's smallest value, 2^-133 (their parts would lose 2^-14 of them at 2^-120, all of them under 2^-134).

@@ -8,6 +8,8 @@ bandwidth-bound kernels at AlexNet sizes.
 Times are HIP-event averages over --iters launches after --warmup launches; `frac` is measured against the
 datasheet peaks (fp32 MFMA 157.3 TFLOP/s, bf16 MFMA 2500 TFLOP/s, HBM 8000 GB/s).  A conv "call" includes the
 operand copies the scalar-offset loaders make (padded image, transposed filter), i.e. what an operator pays.
+--split-operands times the fp32 calls as the operators make them, with RH_ALGO_BF16X3: where the library takes that form,
+`executed` counts its six bf16 products for an fp32 one and `frac` is against the bf16 peak.
 """
 import argparse
 import json
@@ -50,6 +52,27 @@ CONV_LAYERS = {
 FC_LAYERS = {"alexnet_fc6": (256, 9216, 4096), "alexnet_fc7": (256, 4096, 4096), "alexnet_fc8": (256, 4096, 1000)}
 
 
+def launched_tags(fn):
+    """The tags of the launches that fn() makes."""
+    import ctypes as C
+    from . import _lib
+    lib = _lib.lib()
+    lib.rh_profile_reset()
+    lib.rh_profile_filter(None)
+    lib.rh_profile_enable(1)
+    try:
+        fn()
+        tag, work, ms = C.c_char_p(), C.c_double(), C.c_float()
+        tags = set()
+        for i in range(lib.rh_profile_count()):
+            _lib.check(lib.rh_profile_get(i, C.byref(tag), C.byref(work), C.byref(ms)), "rh_profile_get")
+            tags.add(tag.value.decode())
+    finally:
+        lib.rh_profile_enable(0)
+        lib.rh_profile_reset()
+    return tags
+
+
 def main(argv=None):
     ap = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
     ap.add_argument("what", nargs="*", default=["conv", "fc", "mem"], help="conv | fc | mem")
@@ -58,6 +81,7 @@ def main(argv=None):
     ap.add_argument("--iters", type=int, default=5)
     ap.add_argument("--warmup", type=int, default=2)
     ap.add_argument("--relu-data", action="store_true", help="x = max(N(0,1), 0): the sparsity real activations have")
+    ap.add_argument("--split-operands", action="store_true", help="fp32 calls with RH_ALGO_BF16X3, as the operators make them")
     args = ap.parse_args(argv)
 
     import torch
@@ -67,6 +91,7 @@ def main(argv=None):
     from . import _lib, ops
     dev = torch.device("cuda:0")
     passes = set(args.passes.split(","))
+    algo = _lib.RH_ALGO_BF16X3 if args.split_operands else 0
 
     def timeit(fn):
         for _ in range(args.warmup):
@@ -91,6 +116,15 @@ def main(argv=None):
             rec.update({"form": "winograd F(2x2,3x3)", "executed": round(executed / ms / 1e9, 1)})
         print(json.dumps(rec), flush=True)
 
+    def report_product(kernel, layer, fn, work, winograd=0.0):
+        ms = timeit(fn)
+        if algo and any("_tri_" in t for t in launched_tags(fn)):
+            print(json.dumps({"kernel": kernel, "layer": layer, "ms": round(ms, 4), "achieved": round(work / ms / 1e9, 1), "unit": "TFLOP/s",
+                              "peak": PEAK["bf16"], "frac": round(6.0 * work / ms / 1e9 / PEAK["bf16"], 4), "form": "split operands",
+                              "executed": round(6.0 * work / ms / 1e9, 1)}), flush=True)
+        else:
+            report(kernel, layer, ms, work, "fp32", winograd)
+
     if "conv" in args.what:
         for name, (N, C, H, W, K, R, st, pad) in CONV_LAYERS.items():
             if args.layer and not name.startswith(args.layer):
@@ -103,16 +137,16 @@ def main(argv=None):
             dy = torch.randn_like(y)
             flops = 2.0 * y.numel() * C * R * R
             if "fwd" in passes:
-                report("conv_fwd", name, timeit(lambda: ops.conv2d_fwd(x, w, st, pad, y=y)), flops, "fp32",
-                       ops.conv2d_winograd_flops(x.shape, w.shape, st, pad, "fwd"))
+                report_product("conv_fwd", name, lambda: ops.conv2d_fwd(x, w, st, pad, y=y, algo=algo), flops,
+                               ops.conv2d_winograd_flops(x.shape, w.shape, st, pad, "fwd", algo))
             if "bwd_filter" in passes:
                 dw = torch.zeros_like(w)
-                report("conv_bwd_filter", name, timeit(lambda: ops.conv2d_bwd_filter(x, dy, w.shape, st, pad, dw=dw)), flops, "fp32",
-                       ops.conv2d_winograd_flops(x.shape, w.shape, st, pad, "bwd_filter"))
+                report_product("conv_bwd_filter", name, lambda: ops.conv2d_bwd_filter(x, dy, w.shape, st, pad, dw=dw, algo=algo), flops,
+                               ops.conv2d_winograd_flops(x.shape, w.shape, st, pad, "bwd_filter", algo))
             if "bwd_data" in passes:
                 dx = torch.zeros_like(x)
-                report("conv_bwd_data", name, timeit(lambda: ops.conv2d_bwd_data(w, dy, x.shape, st, pad, dx=dx)), flops, "fp32",
-                       ops.conv2d_winograd_flops(x.shape, w.shape, st, pad, "bwd_data"))
+                report_product("conv_bwd_data", name, lambda: ops.conv2d_bwd_data(w, dy, x.shape, st, pad, dx=dx, algo=algo), flops,
+                               ops.conv2d_winograd_flops(x.shape, w.shape, st, pad, "bwd_data", algo))
             if "fwd_bf16" in passes:
                 report("conv_fwd_bf16", name,
                        timeit(lambda: ops.conv2d_fwd(x, w, st, pad, y=y, algo=_lib.RH_MATH_BF16_MFMA_FP32ACC)), flops, "bf16")
@@ -124,9 +158,9 @@ def main(argv=None):
             X, Wt, dY = torch.randn(B, i, device=dev), torch.randn(o, i, device=dev), torch.randn(B, o, device=dev)
             Y, dW, dX = torch.empty(B, o, device=dev), torch.zeros(o, i, device=dev), torch.empty(B, i, device=dev)
             flops = 2.0 * B * i * o
-            report("sgemm_fwd", name, timeit(lambda: ops.sgemm(1, 0, o, B, i, 1.0, Wt, i, X, i, 0.0, Y, o)), flops, "fp32")
-            report("sgemm_bwd_w", name, timeit(lambda: ops.sgemm(0, 1, i, o, B, 1.0, X, i, dY, o, 1.0, dW, i)), flops, "fp32")
-            report("sgemm_bwd_x", name, timeit(lambda: ops.sgemm(0, 0, i, B, o, 1.0, Wt, i, dY, o, 0.0, dX, i)), flops, "fp32")
+            report_product("sgemm_fwd", name, lambda: ops.sgemm(1, 0, o, B, i, 1.0, Wt, i, X, i, 0.0, Y, o, algo=algo), flops)
+            report_product("sgemm_bwd_w", name, lambda: ops.sgemm(0, 1, i, o, B, 1.0, X, i, dY, o, 1.0, dW, i, algo=algo), flops)
+            report_product("sgemm_bwd_x", name, lambda: ops.sgemm(0, 0, i, B, o, 1.0, Wt, i, dY, o, 0.0, dX, i, algo=algo), flops)
     if "mem" in args.what and not args.layer:
         y = torch.randn(256, 96, 55, 55, device=dev)
         dy, b = torch.randn_like(y), torch.randn(96, device=dev)
