@@ -925,7 +925,7 @@ static size_t bf16x3_bytes(const ConvDims& d, int pass, int flags, size_t floor)
     const double slices = fmin(256e6, fmax(4.0 * (double)d.w_elems, 1024.0 * 4 * 128 * 192));
     const double rest = (double)cdiv(d.N, 8) * 4.0 * (d.P * d.Q + (double)d.K * (d.P * d.Q / 32 + 1)) + 4096.0;
     if (copies + slices + rest < (double)floor) return 0;
-    const TriFilterPlan tp = plan_tri_bwd_filter(d);
+    const TriFilterPlan tp = plan_tri_bwd_filter(d, tri_wide(flags));
     return tp.ok && (tri_forced(flags) || tri_pays_bwd_filter(d, tp)) ? tp.total() : 0;
   }
   if (pass != RH_CONV_FWD && pass != RH_CONV_BWD_DATA) return 0;
@@ -1033,7 +1033,7 @@ static int bwd_filter_impl(const rh_conv_geom* g, float alpha, const float* x, c
   };
 
   if (tri_allowed(flags)) {
-    const TriFilterPlan tp = plan_tri_bwd_filter(d);
+    const TriFilterPlan tp = plan_tri_bwd_filter(d, tri_wide(flags));
     if (tri_forced(flags) && !tp.ok) return RH_E_UNSUPPORTED;
     if (tri_forced(flags) && ws_bytes < tp.total()) return RH_E_WORKSPACE;
     if (tri_forced(flags) || (tri_pays_bwd_filter(d, tp) && ws_bytes >= tp.total())) {

@@ -593,12 +593,13 @@ struct TriFilterPlan {
   int Hp, Wp, n8, groups_true, groups, bm, bn, splits;
   int sum_rows;   // rows of K partial sums of dy that the copy can leave for the bias gradient
   double us;      // what a call is expected to take
+  bool wide;      // the wide form (gemm_tri.h)
   size_t tab_bytes, dyt_bytes, xt_bytes, part_bytes, sum_bytes;
   bool ok;
   size_t sums_at() const { return tab_bytes + dyt_bytes + xt_bytes + part_bytes; }
   size_t total() const { return sums_at() + sum_bytes; }
 };
-TriFilterPlan plan_tri_bwd_filter(const ConvDims& d);
+TriFilterPlan plan_tri_bwd_filter(const ConvDims& d, bool wide);
 // Leaves `used` slices of dw in (ko, r, s, c) order in *parts, and in `sums`, if given, rows whose sum is dy's over images and
 // pixels.
 int launch_conv_tri_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
@@ -616,13 +617,15 @@ bool conv1x1_stream_applies(const ConvDims& d);
 inline bool tri_allowed(int flags) {
   return (flags & RH_ALGO_BF16X3) && !(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_WINOGRAD));
 }
+inline bool tri_wide(int flags) { return (flags & RH_ALGO_BF16X3_WIDE) != 0; }
 inline bool tri_forced(int flags) { return tri_allowed(flags) && (flags & RH_ALGO_DIRECT); }
 // Squared relative error against 64 bits, in units of 1e-14, N(0,1) operands: of this form 0.0525 a K step in a chain (1.34e-7
 // at 36, 1.95e-7 at 72), of the engine 0.0335 a term, of the Winograd form as in wino_stages_at_most, of the staged form
 // 0.032 a term of its two chains and four more (0.09 2^-48: a rounding's variance).  The chain allowed is the one with three
 // quarters of the other form's: half zeros, as behind a ReLU, spare the shorter chains more roundings (1.2 on the square).
-// Measured where the form is taken, relative to the other form's error: activations, filters and deltas of AlexNet, NIN and CIFAR-10
-// steps 0.62, 0.53 and 0.49 in the geometric mean (forward, data and filter gradient, 64 calls), 0.97 at most.  Sums of operands of
+// Measured where the form is taken, relative to the other form's error, on the networks' own activations, filters and deltas (forward,
+// data and filter gradient; geometric mean and largest): AlexNet 0.77, 0.53, 0.47 and 0.98, NIN 0.54, 0.58, 0.51 and 1.01, ResNet-18 0.49,
+// 0.69, 0.43 and 1.00 (its filter gradients in the wide form), CIFAR-10's and LeNet's filter gradients 0.44 and 0.65 (882 calls).  Sums of operands of
 // one sign on both sides are another matter, slices make them more exact than their chains alone: uniform [0, 1) on all sides
 // 0.8 to 0.9 in the geometric mean of 137 calls, but up to 1.9 beside a form of many slices, 3e-7 and less in all.
 inline int tri_max_chain(double other) { const double n = 0.75 * other / 0.0525; return n < 1.0 ? 1 : n < 1e6 ? (int)n : 1000000; }

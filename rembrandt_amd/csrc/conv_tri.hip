@@ -13,9 +13,9 @@
 namespace rh {
 
 // part i of the group at `at` (16-byte pieces), parts `plane` pieces apart
-__device__ __forceinline__ void tri_store(uint4* dst, size_t at, size_t plane, const float (&v)[8]) {
+__device__ __forceinline__ void tri_store(uint4* dst, size_t at, size_t plane, const float (&v)[8], bool wide = false) {
   uint4 o[3];
-  tri_pack8(v, o);
+  tri_pack8(v, o, wide);
 #pragma unroll
   for (int i = 0; i < 3; ++i) dst[at + i * plane] = o[i];
 }
@@ -130,6 +130,7 @@ struct TriBatchArgs {
   size_t plane;         // 16-byte pieces of a part
   int px, cx, blocks;   // blocks along the pixels and the channels; all of them
   float* sums;          // [n/8][pixel block][C], or nullptr
+  bool wide;            // mark for the wide form
 };
 __device__ __forceinline__ void tri_batch_body(const TriBatchArgs& a, int b, float (&tile)[8][kTriCh][kTriPix + 1]) {
   const int bx = b % a.px, t = b / a.px, by = t % a.cx, bz = t / a.cx;
@@ -166,7 +167,7 @@ __device__ __forceinline__ void tri_batch_body(const TriBatchArgs& a, int b, flo
 #pragma unroll
     for (int n = 0; n < 8; ++n) v[n] = tile[n][cl][pl];
     if (a.sums) sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-    if (pix < a.HpWp && c < a.C) tri_store(a.xt, ((size_t)bz * a.HpWp + pix) * a.C + c, a.plane, v);
+    if (pix < a.HpWp && c < a.C) tri_store(a.xt, ((size_t)bz * a.HpWp + pix) * a.C + c, a.plane, v, a.wide);
   }
   if (a.sums) {
     __syncthreads();
@@ -205,7 +206,7 @@ __global__ __launch_bounds__(256) void tri_batch_kernel(TriBatchArgs dy, TriBatc
   soff[g] = off;
 }
 
-template <class T, bool B_LINEAR, bool NCHW, class PASS>
+template <class T, bool B_LINEAR, bool NCHW, class PASS, bool WIDE = false>
 static int launch_tri(const TriParams& ap, const TriParams& bp, const EpiParams& ep, int k_steps, int groups, int splits, int* used,
                       double flops, hipStream_t stream, const char* tag) {
   const int tiles_m = cdiv(ep.rows, T::BM), tiles_n = cdiv(ep.cols, T::BN);
@@ -221,10 +222,10 @@ static int launch_tri(const TriParams& ap, const TriParams& bp, const EpiParams&
   constexpr size_t lds = kTriLdsBytes;
   static_assert(2 * lds <= 160 * 1024, "two blocks share a CU");
   static const hipError_t attr = hipFuncSetAttribute(
-      reinterpret_cast<const void*>(&mfma_gemm_tri_kernel<T, B_LINEAR, NCHW, PASS>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
+      reinterpret_cast<const void*>(&mfma_gemm_tri_kernel<T, B_LINEAR, NCHW, PASS, WIDE>), hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return (int)attr;
   ProfScope prof(tag, flops, stream);
-  hipLaunchKernelGGL((mfma_gemm_tri_kernel<T, B_LINEAR, NCHW, PASS>), grid, dim3(T::NT), lds, stream, ap, bp, ep, tiles_m,
+  hipLaunchKernelGGL((mfma_gemm_tri_kernel<T, B_LINEAR, NCHW, PASS, WIDE>), grid, dim3(T::NT), lds, stream, ap, bp, ep, tiles_m,
                      k_steps, sps, groups);
   return launch_status();
 }
@@ -424,8 +425,9 @@ int launch_conv_tri_phases(const ConvDims& d, const PhasePlan& pp, const TriPhas
   }
 }
 
-TriFilterPlan plan_tri_bwd_filter(const ConvDims& d) {
+TriFilterPlan plan_tri_bwd_filter(const ConvDims& d, bool wide) {
   TriFilterPlan p = {};
+  p.wide = wide;
   if (d.P <= 0 || d.Q <= 0) return p;
   p.Hp = d.H + 2 * d.pad; p.Wp = d.W + 2 * d.pad;
   p.n8 = cdiv(d.N, 8);
@@ -443,6 +445,10 @@ TriFilterPlan plan_tri_bwd_filter(const ConvDims& d) {
   const int CRS = d.C * d.R * d.S, tiles = cdiv(d.K, p.bm) * cdiv(CRS, p.bn), steps = p.groups / 2;
   // slices: two blocks to a CU where there are (0.445 us a K step of 128 x 128), their partial sums written and read (a fit to
   // 1859 timed calls; 11664 steps of 38 tiles: 13 slices 1031 us, 6, which leave 28 CUs idle, 1171)
+  // (the wide form's K steps take 1.07 and 1.14 times as long, 64-row and other tiles; priced as plain ones, since with those factors
+  // 64 -> 128 56x56 stride 2 at batch 32 and 50 go to a form of 76 and 109 us where this one takes 57 and 81; of 83 calls of
+  // ResNet-18's layers that come here four are slower than the form replaced: 256 -> 256 14x14 at 90, 128 and 256 images by 0 to 6 %,
+  // 256 -> 512 at one image 34 -> 36 us)
   p.us = 1e30;
   for (int want = 1; want <= 256 && (want == 1 || (want * 8 <= steps && (long long)tiles * want <= 1024)); ++want) {
     const int n = cdiv(steps, want), S = cdiv(steps, n);
@@ -471,9 +477,9 @@ int launch_conv_tri_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const 
   {
     TriBatchArgs a, b;
     a.x = dy; a.xt = dyt; a.N = d.N; a.C = d.K; a.H = d.P; a.W = d.Q; a.halo = 0; a.HpWp = d.P * d.Q; a.dWp = FastDiv((uint32_t)d.Q);
-    a.plane = dy_plane; a.px = cdiv(a.HpWp, kTriPix); a.cx = cdiv(a.C, kTriCh); a.blocks = a.px * a.cx * p.n8; a.sums = sums;
+    a.plane = dy_plane; a.px = cdiv(a.HpWp, kTriPix); a.cx = cdiv(a.C, kTriCh); a.blocks = a.px * a.cx * p.n8; a.sums = sums; a.wide = p.wide;
     b.x = x; b.xt = xt; b.N = d.N; b.C = d.C; b.H = d.H; b.W = d.W; b.halo = d.pad; b.HpWp = p.Hp * p.Wp; b.dWp = FastDiv((uint32_t)p.Wp);
-    b.plane = x_plane; b.px = cdiv(b.HpWp, kTriPix); b.cx = cdiv(b.C, kTriCh); b.blocks = b.px * b.cx * p.n8; b.sums = nullptr;
+    b.plane = x_plane; b.px = cdiv(b.HpWp, kTriPix); b.cx = cdiv(b.C, kTriCh); b.blocks = b.px * b.cx * p.n8; b.sums = nullptr; b.wide = false;
     ProfScope prof("tri_batch", 4.0 * (double)(d.y_elems + d.x_elems) + 48.0 * (double)(dy_plane + x_plane), stream);
     hipLaunchKernelGGL(tri_batch_kernel, dim3((unsigned)(a.blocks + b.blocks + cdiv(p.groups, 256))), dim3(256), 0, stream, a, b, soff,
                        p.groups, p.groups_true, d.P * d.Q, d.Q, d.st, p.Wp);
@@ -491,13 +497,19 @@ int launch_conv_tri_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const 
   EpiParams ep;
   ep.out = *parts; ep.bias = nullptr; ep.alpha = 1.0f; ep.beta = 0.0f;
   ep.rows = d.K; ep.cols = CRS; ep.inner = 0; ep.ld = CRS; ep.relu = 0; ep.split_stride = (long long)d.K * CRS;
-  const double flops = 12.0 * (double)d.w_elems * d.N * d.P * d.Q;
+  const double flops = (p.wide ? 14.0 : 12.0) * (double)d.w_elems * d.N * d.P * d.Q;
   const int steps = p.groups / 2;
+#define RH_TRI(TILE, TAG)                                                                                              \
+  (p.wide ? launch_tri<TILE, false, false, PassConvBwdFilter, true>(ap, bp, ep, steps, p.groups_true, p.splits, used, flops, stream, \
+                                                                    "conv_bwd_filter_tri_wide_" TAG)                                 \
+          : launch_tri<TILE, false, false, PassConvBwdFilter>(ap, bp, ep, steps, p.groups_true, p.splits, used, flops, stream,       \
+                                                              "conv_bwd_filter_tri_" TAG))
   switch (p.bm) {
-    case 128: return launch_tri<T128x128t, false, false, PassConvBwdFilter>(ap, bp, ep, steps, p.groups_true, p.splits, used, flops, stream, "conv_bwd_filter_tri_128x128");
-    case 96: return launch_tri<T96x128t, false, false, PassConvBwdFilter>(ap, bp, ep, steps, p.groups_true, p.splits, used, flops, stream, "conv_bwd_filter_tri_96x128");
-    default: return launch_tri<T64x192t, false, false, PassConvBwdFilter>(ap, bp, ep, steps, p.groups_true, p.splits, used, flops, stream, "conv_bwd_filter_tri_64x192");
+    case 128: return RH_TRI(T128x128t, "128x128");
+    case 96: return RH_TRI(T96x128t, "96x128");
+    default: return RH_TRI(T64x192t, "64x192");
   }
+#undef RH_TRI
 }
 
 }  // namespace rh

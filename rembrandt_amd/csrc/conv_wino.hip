@@ -1666,7 +1666,7 @@ extern "C" double rh_conv2d_winograd_flops(const rh_conv_geom* g, int pass, int 
   if (conv_dims(g, &d)) return 0.0;
   if (flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT)) return 0.0;
   TriPlan tp;
-  if (tri_allowed(flags) && (tri_forced(flags) || (pass == RH_CONV_BWD_FILTER ? tri_pays_bwd_filter(d, plan_tri_bwd_filter(d))
+  if (tri_allowed(flags) && (tri_forced(flags) || (pass == RH_CONV_BWD_FILTER ? tri_pays_bwd_filter(d, plan_tri_bwd_filter(d, tri_wide(flags)))
                                                                   : tri_pays(d, pass == RH_CONV_BWD_DATA, flags, &tp))))
     return 0.0;
   if (wino_shape5(d) && pass == RH_CONV_FWD) {

@@ -6,6 +6,7 @@ import struct
 
 import numpy as np
 import pytest
+import torch
 
 import oracle as O
 from oracle import graph as OG
@@ -153,6 +154,45 @@ def check_step(w, ref, sgd, rsgd, x, labels, fused_sgd, tag, teacher=False):
                 assert_close(w.read(i, "u%d.%s" % (k, gname)), getattr(u, rname).ravel(), "%s unit %d %s" % (what, k, gname))
             for gname, _ in UNIT_GRADS:
                 assert not w.read(i, "u%d.%s" % (k, gname)).any(), "reset() zeroes the gradients"
+
+
+def _filter_gradient64(x, dy, size):
+    """The filter gradient of a stride-1 layer that keeps the extent, as a plain matrix product in 64 bits."""
+    (n, c, _, _), (k, p, q) = x.shape, dy.shape[1:]
+    dw, step = 0.0, max(1, 10 ** 8 // (c * size * size * p * q))
+    for i in range(0, n, step):
+        m = min(step, n - i)
+        col = torch.nn.functional.unfold(x[i:i + m].double(), size, padding=size // 2).permute(0, 2, 1).reshape(m * p * q, -1).contiguous()
+        dw = dw + dy[i:i + m].double().reshape(m, k, p * q).permute(1, 0, 2).reshape(k, -1).contiguous() @ col
+    return dw.reshape(-1)
+
+
+def test_filter_gradients_behind_a_batch_norm_are_as_exact_as_on_fp32_instructions(dev):
+    """Units of ResNet-18's first residual operators, a train step's forward and backward: each filter gradient against 64-bit sums of
+    the unit's own input and deltas (a small value of one sign almost everywhere), no further off than with split_operands=False."""
+    dims, layers, ncat = net = configs.resnet18()
+    batch, size = 24, 56
+    say("bnorm filter gradients")
+    errs = []
+    for split in (True, False):
+        w = SequentialOperatorWorker(configs.build_config(net), batch, "Backward", shared_seed=(0xB4002, 0xB4003), split_operands=split)
+        w.init_params()
+        w.load_frames_f32(synth.normal(0xB4002, 100, (batch,) + tuple(dims[::-1])))
+        w.stage_batch(synth.integers(0xB4002, 200, (batch,), ncat), 1.0 / batch)
+        w.forward(batch, training=True)
+        w.store_loss(batch)
+        w.backward(batch)
+        read = lambda i, which, *shape: torch.from_numpy(w.read(i, which)).to(dev)[:int(np.prod(shape))].reshape(shape)
+        errs.append({})
+        for i, unit, c in ((2, 0, 64), (2, 1, 64), (3, 0, 64), (3, 1, 64), (4, 1, 128)):
+            h = size if i < 4 else size // 2
+            x = read(i, "mid_act", batch, c, h, h) if unit else read(i - 1, "out_act", batch, c, h, h)
+            ref = _filter_gradient64(x, read(i, "u%d.pre_delta" % unit, batch, c, h, h), 3)
+            got = torch.from_numpy(w.read(i, "u%d.grad_weights" % unit)).to(dev).double()
+            errs[-1][i, unit] = float((got - ref).norm() / ref.norm())
+        w.close()
+    for unit, err in errs[0].items():
+        assert err <= errs[1][unit], (unit, err, errs[1][unit])
 
 
 @pytest.mark.parametrize("fuse,fused_sgd,flavour", [(True, True, "Update"), (False, False, "Update"), (True, False, "GradientNesterov")])

@@ -580,6 +580,14 @@ def test_conv2d_bf16x3(dev, case):
     assert_close(N(dwc), O.conv2d_bwd_filter(x, dy, w.shape, st, pad, 0.25, 1.0, dw0.copy()), "bf16x3 bwd filter alpha/beta")
     assert_close(N(dbc), O.conv2d_bwd_bias(dy, 0.25, 1.0, db0.copy()), "bf16x3 bias gradient")
     assert torch.equal(ops.conv2d_bwd_filter(xd, dyd, w.shape, st, pad, algo=X3), dw), "run to run the same bits"
+    X3 |= _lib.RH_ALGO_BF16X3_WIDE
+    wide, tags = profile_tags(lambda: ops.conv2d_bwd_filter(xd, dyd, w.shape, st, pad, algo=X3))
+    assert any(t.startswith("conv_bwd_filter_tri_wide_") for t in tags), tags
+    assert_close(N(wide), O.conv2d_bwd_filter(x, dy, w.shape, st, pad), "bf16x3 wide bwd filter")
+    dwc, dbc = ops.conv2d_bwd_filter_bias(xd, dyd, w.shape, st, pad, alpha=0.25, beta=1.0, dw=T(dw0, dev), db=T(db0, dev), algo=X3)
+    assert_close(N(dwc), O.conv2d_bwd_filter(x, dy, w.shape, st, pad, 0.25, 1.0, dw0.copy()), "bf16x3 wide bwd filter alpha/beta")
+    assert_close(N(dbc), O.conv2d_bwd_bias(dy, 0.25, 1.0, db0.copy()), "bf16x3 wide bias gradient")
+    assert torch.equal(ops.conv2d_bwd_filter(xd, dyd, w.shape, st, pad, algo=X3), wide), "run to run the same bits"
 
 
 # Backward-data of stride 2 to 4 by residue classes in the split-operand form: odd extents (classes of different sizes), classes
@@ -698,6 +706,51 @@ def test_conv2d_bf16x3_error(dev, case, data):
             assert err <= before, (name, err, before)
 
 
+@pytest.mark.parametrize("case", [(48, 64, 56, 64, 3, 1), (24, 64, 56, 128, 3, 2), (64, 96, 28, 96, 3, 1), (64, 128, 28, 256, 3, 2), (24, 256, 14, 256, 3, 1)], ids=str)
+def test_conv2d_bf16x3_deltas_behind_a_batch_norm(dev, case):
+    """Filter gradients of positive inputs and deltas with a small value of one sign almost everywhere: one value in ten is large and each
+    channel's mean is taken off.  No larger an error against 64-bit sums than the fp32 instruction's, and infinities, NaNs and the
+    values that have no sum of three stay where they are."""
+    Nn, C, H, K, R, st = case
+    say("bf16x3 wide", case)
+    P = (H + 2 - R) // st + 1
+    x = (1.5 + 0.6 * T(synth.normal(51, 1, (Nn, C, H, H)), dev)).clamp_min(0.01)
+    dy = T(synth.normal(51, 2, (Nn, K, P, P)) * (synth.uniform(51, 3, (Nn, K, P, P)) < 0.1), dev)
+    dy = dy - dy.mean((0, 2, 3), keepdim=True)
+    shape = (K, C, R, R)
+    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_BF16X3_WIDE
+    ref = _conv_sums64(x, torch.zeros(shape, device=dev), dy, st, 1)[2]
+    got, before = (ops.conv2d_bwd_filter(x, dy, shape, st, 1, algo=algo).double() for algo in (X3 | _lib.RH_ALGO_DIRECT, _lib.RH_ALGO_SCALAR_OFFSET))
+    err, err0 = (float((t - ref).norm() / ref.norm()) for t in (got, before))
+    assert err <= err0, (err, err0)
+
+
+def test_conv2d_bf16x3_wide_marks(dev):
+    """The wide form's marks in the last bit of a part: powers of two over the whole range beside a large value, exact products, so that
+    every result is known; with an infinity of dy, or a value whose parts need that bit, in the group of eight images."""
+    X3 = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_BF16X3_WIDE | _lib.RH_ALGO_DIRECT
+    say("bf16x3 wide marks")
+    Nn, C, K = 8, 8, 64
+    exps = np.linspace(-149, 100, K).astype(int)
+    odd = np.float64(1.0 + 2.0 ** -23)    # 24 significant bits where the exponent has them
+    for image in range(Nn):
+        for extra in (0.0, 2.0 ** 101, -(2.0 ** 127), np.inf):
+            dy = np.zeros((Nn, K, 1, 1), np.float32)
+            dy[image, :, 0, 0] = (odd * 2.0 ** exps).astype(np.float32)
+            other = (image + 3) % Nn
+            dy[other, :, 0, 0] = extra
+            x = np.zeros((Nn, C, 1, 1), np.float32)
+            x[image], x[other, 4:] = 1.0, 1.0
+            got = N(ops.conv2d_bwd_filter(T(x, dev), T(dy, dev), (K, C, 1, 1), 1, 0, algo=X3))[:, :, 0, 0]
+            alone = dy[image, :, 0, 0].astype(np.float64)
+            if extra == np.inf:
+                assert np.all(got[:, 4:] == np.inf) and np.all(np.isnan(got[:, :4]))   # (0 x inf)
+                continue
+            want = np.stack([alone] * 4 + [alone + extra] * 4, 1).astype(np.float32)
+            assert np.all(np.abs(got - want) <= np.spacing(np.abs(want))), (image, extra)
+            assert np.array_equal(got[:, :4], want[:, :4]), (image, extra)
+
+
 @pytest.mark.parametrize("case", [(9, 16, 14, 11, 40, 3, 5, 1, 2), (3, 24, 9, 12, 72, 1, 4, 1, 0), (8, 40, 12, 9, 64, 5, 1, 1, 1),
                                   (5, 16, 13, 10, 33, 2, 3, 2, 1), (24, 64, 30, 28, 128, 2, 3, 2, 1)], ids=str)
 def test_conv2d_bf16x3_filters_that_are_not_square(dev, case):
@@ -745,9 +798,11 @@ def test_conv2d_bf16x3_infinities_and_largest_floats(dev):
     w[:, 2] *= 0.125   # (the largest floats' products stay in range)
     xd, wd, dyd = T(x, dev), T(w, dev), T(dy * 0.125, dev)
     G = _lib.RH_ALGO_SCALAR_OFFSET
-    for run in (lambda algo: ops.conv2d_fwd(xd, wd, 1, pad, algo=algo), lambda algo: ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=algo),
-                lambda algo: ops.conv2d_bwd_filter(xd, dyd, w.shape, 1, pad, algo=algo)):
-        got, ref = run(X3), run(G)
+    wide = X3 | _lib.RH_ALGO_BF16X3_WIDE
+    for form, run in ((X3, lambda algo: ops.conv2d_fwd(xd, wd, 1, pad, algo=algo)), (X3, lambda algo: ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=algo)),
+                      (X3, lambda algo: ops.conv2d_bwd_filter(xd, dyd, w.shape, 1, pad, algo=algo)),
+                      (wide, lambda algo: ops.conv2d_bwd_filter(xd, dyd, w.shape, 1, pad, algo=algo))):
+        got, ref = run(form), run(G)
         assert bool(torch.isinf(ref).any())
         assert torch.equal(torch.isnan(got), torch.isnan(ref)) and torch.equal(torch.isinf(got), torch.isinf(ref))
         keep = torch.isfinite(ref)
@@ -791,7 +846,9 @@ def test_conv2d_bf16x3_small_operands(dev, exponent):
             for name, operands, terms, ref, run in (
                     ("fwd", (0, 1), C * R * R, lambda: O.conv2d_fwd(x, w, 1, pad), lambda: ops.conv2d_fwd(xd, wd, 1, pad, algo=X3)),
                     ("bwd_data", (1, 2), K * R * R, lambda: O.conv2d_bwd_data(w, dy, x.shape, 1, pad), lambda: ops.conv2d_bwd_data(wd, dyd, x.shape, 1, pad, algo=X3)),
-                    ("bwd_filter", (0, 2), Nn * H * W, lambda: O.conv2d_bwd_filter(x, dy, w.shape, 1, pad), lambda: ops.conv2d_bwd_filter(xd, dyd, w.shape, 1, pad, algo=X3))):
+                    ("bwd_filter", (0, 2), Nn * H * W, lambda: O.conv2d_bwd_filter(x, dy, w.shape, 1, pad), lambda: ops.conv2d_bwd_filter(xd, dyd, w.shape, 1, pad, algo=X3)),
+                    ("bwd_filter wide", (0, 2), Nn * H * W, lambda: O.conv2d_bwd_filter(x, dy, w.shape, 1, pad),
+                     lambda: ops.conv2d_bwd_filter(xd, dyd, w.shape, 1, pad, algo=X3 | _lib.RH_ALGO_BF16X3_WIDE))):
                 if tiny not in operands:
                     continue
                 want = ref().astype(np.float64)
