@@ -101,8 +101,8 @@ def collect_profile(lib, steps):
             continue
         if mfma:
             achieved, unit = work / ms / 1e9, "TFLOP/s"
-            # (the split-operand kernels execute six bf16 products for an fp32 one, and report those)
-            bf16 = name.startswith("conv_fwd_bf16") or "_tri_" in name
+            # (the split-operand kernels execute six bf16 or three fp16 products, of one rate, for an fp32 one, and report those)
+            bf16 = name.startswith("conv_fwd_bf16") or "_tri_" in name or "_duo_" in name
             peak = PEAK_BF16_MFMA_TFLOPS if bf16 else PEAK_FP32_MFMA_TFLOPS
         else:
             achieved, peak, unit = work / ms / 1e6, PEAK_HBM_GBS, "GB/s"
@@ -403,11 +403,12 @@ def conv_sweep_leg(iters, warmup):
     """Forward, backward-data and backward-filter of the three sweep shapes, each call timed alone (HIP events on the
     stream the kernels run on; a call includes the operand copies it makes): ms, TFLOP/s against the fp32 matrix peak and
     algorithmic bytes (x, w, y once) per second against the HBM peak: the 1x1 shape sits on the ridge of both roofs.  The figures
-    are of calls on fp32 instructions; `as_operators_call` is the same call with RH_ALGO_BF16X3, the operators' default, and where
-    that takes the split-operand form `frac_mfma` is its six bf16 products for an fp32 one against the bf16 peak."""
+    are of calls on fp32 instructions; `as_operators_call` is the same call with RH_ALGO_BF16X3 and RH_ALGO_F16X2, the operators'
+    default, and where that takes a split-operand form `frac_mfma` is its six bf16 or three fp16 products for an fp32 one against
+    the peak of those instructions."""
     import torch
     from rembrandt_amd import _lib, ops
-    from rembrandt_amd.kernel_bench import launched_tags
+    from rembrandt_amd.kernel_bench import launched_tags, split_products
 
     def time_call(fn):
         for _ in range(warmup):
@@ -447,13 +448,13 @@ def conv_sweep_leg(iters, warmup):
                           "gbs": byts / ms / 1e6, "frac_hbm": byts / ms / 1e6 / PEAK_HBM_GBS}
             if wino:
                 row[pname].update({"form": "winograd F(2x2,3x3)", "executed_tflops": wino / ms / 1e9})
-            call = lambda: fn(_lib.RH_ALGO_BF16X3)
-            split = any("_tri_" in t for t in launched_tags(call))
+            call = lambda: fn(_lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_F16X2)
+            split = split_products(launched_tags(call))
             ms = time_call(call)
-            row[pname]["as_operators_call"] = {"ms": ms, "tflops": flops / ms / 1e9, "form": "split operands" if split else "as above"}
+            row[pname]["as_operators_call"] = {"ms": ms, "tflops": flops / ms / 1e9, "form": "split operands, %d products" % split if split else "as above"}
             if split:
-                row[pname]["as_operators_call"].update({"executed_tflops": 6.0 * flops / ms / 1e9,
-                                                        "frac_mfma": 6.0 * flops / ms / 1e9 / PEAK_BF16_MFMA_TFLOPS})
+                row[pname]["as_operators_call"].update({"executed_tflops": split * flops / ms / 1e9,
+                                                        "frac_mfma": split * flops / ms / 1e9 / PEAK_BF16_MFMA_TFLOPS})
         out[name] = row
         del x, w, y, dy, dw, dx
     return out

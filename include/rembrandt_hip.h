@@ -83,6 +83,20 @@ typedef void* rh_stream_t; /* hipStream_t */
                                              are multiplied apart (seven products a pair, 4 to 12 % more time) and the
                                              error is below the fp32 instruction's again.  The operators set it for their
                                              batch-normalised convolutions. */
+#define RH_ALGO_F16X2              0x8000 /* convolutions: the contraction may also run on fp16 matrix instructions, every fp32 operand
+                                             value, times a power of two, as the sum of two fp16 values (three products a pair,
+                                             fp32 accumulate in short chains).  The power is one for a filter and one for an
+                                             image, in the filter gradient one for a channel of either operand.  Two parts
+                                             hold a value to 2^-23 of itself down to 2^-29 of the largest of its filter, image
+                                             or channel, and to 2^-51 of that largest value below; results with an operand
+                                             that has no larger one beside it in a group of eight (2^-49 for filters and in the
+                                             filter gradient), an infinity or a NaN are formed on fp32 instructions, as with
+                                             RH_ALGO_BF16X3.  With or without that bit, with the hint or without: where it is
+                                             expected to be the fastest form, its error against 64-bit sums no larger than that
+                                             of the form it replaces, and the scratch holds it.  With RH_ALGO_DIRECT and without
+                                             RH_ALGO_BF16X3: this form, RH_E_UNSUPPORTED where the geometry has none (as there;
+                                             a stride in backward-data has none).  rh_conv2d_workspace_bytes_for says what it
+                                             needs.  No effect beside the other RH_ALGO_* bits and RH_MATH_BF16_MFMA_FP32ACC. */
 
 const char* rh_version(void);
 /* Status of the most recent launch made by a void `rembrandt_kernel_*` entry point on this thread. */
@@ -164,8 +178,8 @@ int32_t rh_conv2d_out_dim(int32_t in, int32_t size, int32_t stride, int32_t pad)
 /* Bytes of scratch the given pass needs whatever flags it is called with (0 is possible), RH_ALGO_BF16X3 with RH_ALGO_DIRECT
  * apart.  The scratch must be 256-byte aligned. */
 size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass);
-/* The same with room for the form of RH_ALGO_BF16X3 where `flags` allow it and it is expected to be the fastest, with the hint
- * RH_ALGO_SHARED_GPU or without: with less a call takes another form. */
+/* The same with room for the forms of RH_ALGO_BF16X3 and RH_ALGO_F16X2 where `flags` allow them and they are expected to be the
+ * fastest, with the hint RH_ALGO_SHARED_GPU or without: with less a call takes another form. */
 size_t rh_conv2d_workspace_bytes_for(const rh_conv_geom* g, int pass, int flags);
 /* The same for RH_ALGO_BF16X3 with RH_ALGO_DIRECT, which needs it; 0 where the geometry has no such form. */
 size_t rh_conv2d_bf16x3_workspace_bytes(const rh_conv_geom* g, int pass);

@@ -17,6 +17,7 @@ RH_ALGO_GATHER, RH_ALGO_SCALAR_OFFSET, RH_ALGO_WINOGRAD, RH_ALGO_DIRECT = 0x100,
 RH_ALGO_SHARED_GPU = 0x1000
 RH_ALGO_BF16X3 = 0x2000
 RH_ALGO_BF16X3_WIDE = 0x4000
+RH_ALGO_F16X2 = 0x8000
 RH_MATH_BF16_MFMA_FP32ACC = 0x1
 RH_E_INVALID, RH_E_WORKSPACE, RH_E_UNSUPPORTED, RH_E_LIMIT = -1, -2, -3, -4
 

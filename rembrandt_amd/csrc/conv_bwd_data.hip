@@ -169,17 +169,12 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
   hipStream_t stream = to_stream(stream_);
 
   if ((flags & RH_ALGO_WINOGRAD) && (!wino_shape(d) || (flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT)))) return RH_E_UNSUPPORTED;
-  if (tri_allowed(flags)) {
-    TriPlan tp = {};
-    if (tri_forced(flags)) {
-      tp = plan_tri_bwd_data(d);
-      if (!tp.ok) return RH_E_UNSUPPORTED;
-      if (ws_bytes < tp.total()) return RH_E_WORKSPACE;
-    }
-    if (tri_forced(flags) || (tri_pays(d, true, flags, &tp) && ws_bytes >= tp.total())) {
-      if (d.x_elems == 0) return 0;
-      return launch_conv_tri(tp, true, dy, w, dx, alpha, beta, nullptr, 0, mask, ws, stream);
-    }
+  const SplitPick split = pick_split(d, true, flags, ws_bytes);
+  if (split.parts) {
+    if (!split.plan.ok) return RH_E_UNSUPPORTED;
+    if (ws_bytes < split.plan.total()) return RH_E_WORKSPACE;
+    if (d.x_elems == 0) return 0;
+    return (split.parts == 3 ? launch_conv_tri : launch_conv_duo)(split.plan, true, dy, w, dx, alpha, beta, nullptr, 0, mask, ws, stream);
   }
   if (!(flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET)) && conv1x1_stream_applies(d)) {
     if (d.x_elems == 0) return 0;

@@ -380,21 +380,52 @@ static BwdFilterSoffPlan plan_bwd_filter_soff(const ConvDims& d) {
 
 // (The error of the form otherwise taken, in the units of tri_max_chain: the engine's and the gathering kernels' as engine_err; the
 // Winograd form's 0.35 a tile group of its slices at least, 0.35 to 0.53 in 16 calls measured.)
-bool tri_pays_bwd_filter(const ConvDims& d, const TriFilterPlan& t) {
-  if (!t.ok) return false;
+static TriRival filter_rival(const ConvDims& d) {
   const int bm = pick_bm(d.K);
   const double terms = (double)d.N * d.P * d.Q, flops = 2.0 * (double)d.w_elems * terms;
-  const double other = (d.R * d.S > 1 ? 1.25 : 1.0) * (15.0 + flops / (bm >= 96 ? 100e6 : bm == 64 ? 60e6 : 50e6)) + 11e-6 * (double)d.w_elems;
-  if (t.us >= 0.9 * other) return false;
-  double err;
+  const double us = (d.R * d.S > 1 ? 1.25 : 1.0) * (15.0 + flops / (bm >= 96 ? 100e6 : bm == 64 ? 60e6 : 50e6)) + 11e-6 * (double)d.w_elems;
   const WinoFilterPlan wp = wino_shape(d) ? plan_wino_bwd_filter(d) : WinoFilterPlan{};
-  if (wino_filter_pays(d, wp)) {
-    err = 0.35 * wp.stages;
-  } else {
-    const BwdFilterSoffPlan sp = plan_bwd_filter_soff(d);
-    err = 0.0335 * terms / (sp.ok && use_soff_bwd_filter(d) ? sp.splits : plan_bwd_filter(d).splits);
+  if (wino_filter_pays(d, wp)) return TriRival{0.9 * us, 0.35 * wp.stages};
+  const BwdFilterSoffPlan sp = plan_bwd_filter_soff(d);
+  return TriRival{0.9 * us, 0.0335 * terms / (sp.ok && use_soff_bwd_filter(d) ? sp.splits : plan_bwd_filter(d).splits)};
+}
+// Two parts beside the form of time `other_us` and error `err`; both errors with a twentieth of the products not zero, as behind a
+// max-pool, where two parts are the least ahead (1e-14 on the square): three parts 0.005 a K step of a slice and 0.016 a slice; two 1.0
+// and 0.016 a slice (of AlexNet's conv5 at 128 images 0.92e-7 and 1.08e-7, at 256 1.30 and 1.15, of its conv2 at 50 1.28 and 1.26).
+static bool duo_filter_pays(const TriFilterPlan& p, double other_us, double err) {
+  return p.ok && p.us < 0.96 * other_us && 1.0 + 0.016 * p.splits <= err;
+}
+// need: the scratch of the forms that may be taken with less
+SplitFilterPick pick_split_bwd_filter(const ConvDims& d, int flags, size_t ws_bytes, size_t* need) {
+  SplitFilterPick s = {};
+  if (tri_forced(flags) || duo_forced(flags)) {
+    s.parts = tri_forced(flags) ? 3 : 2;
+    s.plan = s.parts == 3 ? plan_tri_bwd_filter(d, tri_wide(flags)) : plan_duo_bwd_filter(d);
+    if (need && s.plan.ok) *need = s.plan.total();
+    return s;
   }
-  return cdiv(t.groups / 2, t.splits) <= tri_max_chain(err);
+  const bool duo = duo_allowed(flags) && !(tri_allowed(flags) && tri_wide(flags));
+  if (!tri_allowed(flags) && !duo) return s;
+  const TriRival other = filter_rival(d);
+  double us = other.us, err = 0.2 * other.err;
+  if (tri_allowed(flags)) {
+    const TriFilterPlan p = plan_tri_bwd_filter(d, tri_wide(flags));
+    const int chain = p.ok ? cdiv(p.groups / 2, p.splits) : 0;
+    if (p.ok && p.us < other.us && chain <= tri_max_chain(other.err) && p.total() <= ws_bytes) {
+      s = SplitFilterPick{3, p};
+      us = p.us;
+      err = 0.005 * chain + 0.016 * p.splits;
+      if (need && p.total() > *need) *need = p.total();
+    }
+  }
+  if (duo) {
+    const TriFilterPlan p = plan_duo_bwd_filter(d);
+    if (p.total() <= ws_bytes && duo_filter_pays(p, us, err)) {
+      s = SplitFilterPick{2, p};
+      if (need && p.total() > *need) *need = p.total();
+    }
+  }
+  return s;
 }
 
 // dst[n][pix][c] (pix over Hp x Wp, zero halo) = src[n][c][h][w]: 32 x 32 tiles through LDS so that both
@@ -917,35 +948,36 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
   }
 }
 
-// Scratch of the split-operand form where `flags` (with RH_ALGO_BF16X3) take it; 0 where they do not, and where it cannot be
-// more than `floor` (the filter gradient's copies, and slices of up to 1024 tiles or 256 MB in all).
-static size_t bf16x3_bytes(const ConvDims& d, int pass, int flags, size_t floor) {
+// Scratch of the split-operand forms where `flags` take them; 0 where they do not, and where it cannot be
+// more than `floor` (the filter gradient's copies, exponents and maxima, and slices of up to 2048 tiles or 256 MB in all).
+static size_t split_scratch(const ConvDims& d, int pass, int flags, size_t floor) {
   if (pass == RH_CONV_BWD_FILTER) {
     const double copies = 6.0 * round_up(d.N, 8) * ((double)d.K * (d.P * d.Q + 1) + (double)d.C * (d.H + 2 * d.pad) * (d.W + 2 * d.pad));
-    const double slices = fmin(256e6, fmax(4.0 * (double)d.w_elems, 1024.0 * 4 * 128 * 192));
-    const double rest = (double)cdiv(d.N, 8) * 4.0 * (d.P * d.Q + (double)d.K * (d.P * d.Q / 32 + 1)) + 4096.0;
+    const double slices = fmin(256e6, fmax(4.0 * (double)d.w_elems, 2048.0 * 4 * 128 * 128));
+    const double rest = (double)cdiv(d.N, 8) * 4.0 * (d.P * d.Q + (double)d.K * (d.P * d.Q / 32 + 1)) + 64.0 * (d.K + d.C) + 65536.0;
     if (copies + slices + rest < (double)floor) return 0;
-    const TriFilterPlan tp = plan_tri_bwd_filter(d, tri_wide(flags));
-    return tp.ok && (tri_forced(flags) || tri_pays_bwd_filter(d, tp)) ? tp.total() : 0;
+    size_t need = 0;
+    pick_split_bwd_filter(d, flags, ~size_t(0), &need);
+    return need;
   }
   if (pass != RH_CONV_FWD && pass != RH_CONV_BWD_DATA) return 0;
   const bool bwd = pass == RH_CONV_BWD_DATA;
-  if (tri_forced(flags)) {
-    const TriPlan tp = plan_tri_pass(d, bwd, 0);
-    return tp.ok ? tp.total() : 0;
+  if (tri_forced(flags) || duo_forced(flags)) {
+    const SplitPick s = pick_split(d, bwd, flags, 0);
+    return s.plan.ok ? s.plan.total() : 0;
   }
   if (bwd && d.st > 1) {
     const PhasePlan pp = plan_phase_bwd_data(d);
     const TriPhasePlan tp = plan_tri_phases(d, pp);
     return tp.ok ? tp.total() : 0;
   }
-  return tri_bytes(d, bwd, floor);
+  return split_bytes(d, bwd, flags, floor);
 }
 
 extern "C" size_t rh_conv2d_workspace_bytes_for(const rh_conv_geom* g, int pass, int flags) {
   ConvDims d;
   if (conv_dims(g, &d)) return 0;
-  const size_t need = rh_conv2d_workspace_bytes(g, pass), tri = tri_allowed(flags) ? bf16x3_bytes(d, pass, flags, need) : 0;
+  const size_t need = rh_conv2d_workspace_bytes(g, pass), tri = tri_allowed(flags) || duo_allowed(flags) ? split_scratch(d, pass, flags, need) : 0;
   return tri > need ? tri : need;
 }
 
@@ -953,7 +985,7 @@ extern "C" size_t rh_conv2d_bf16x3_workspace_bytes(const rh_conv_geom* g, int pa
   ConvDims d;
   if (conv_dims(g, &d)) return 0;
   const int forced = RH_ALGO_BF16X3 | RH_ALGO_DIRECT;
-  return bf16x3_bytes(d, pass, forced, 0) ? rh_conv2d_workspace_bytes_for(g, pass, forced) : 0;
+  return split_scratch(d, pass, forced, 0) ? rh_conv2d_workspace_bytes_for(g, pass, forced) : 0;
 }
 
 extern "C" size_t rh_conv2d_workspace_bytes_for_upto(const rh_conv_geom* g, int pass, int flags) {
@@ -965,8 +997,8 @@ extern "C" size_t rh_conv2d_workspace_bytes_for_upto(const rh_conv_geom* g, int 
     const size_t b = rh_conv2d_workspace_bytes(&h, pass);
     if (b > need) need = b;
     ConvDims d;
-    if (!tri_allowed(flags) || conv_dims(&h, &d)) continue;
-    const size_t tri = bf16x3_bytes(d, pass, flags, need);
+    if ((!tri_allowed(flags) && !duo_allowed(flags)) || conv_dims(&h, &d)) continue;
+    const size_t tri = split_scratch(d, pass, flags, need);
     if (tri > need) need = tri;
   }
   return need;
@@ -1032,23 +1064,22 @@ static int bwd_filter_impl(const rh_conv_geom* g, float alpha, const float* x, c
     return launch_status();
   };
 
-  if (tri_allowed(flags)) {
-    const TriFilterPlan tp = plan_tri_bwd_filter(d, tri_wide(flags));
-    if (tri_forced(flags) && !tp.ok) return RH_E_UNSUPPORTED;
-    if (tri_forced(flags) && ws_bytes < tp.total()) return RH_E_WORKSPACE;
-    if (tri_forced(flags) || (tri_pays_bwd_filter(d, tp) && ws_bytes >= tp.total())) {
-      if (d.w_elems == 0) return 0;
-      float* parts = nullptr;
-      int used = 1;
-      float* sums = nullptr;
-      if (bf && bf->db) {
-        bf->part = sums = reinterpret_cast<float*>(static_cast<char*>(ws) + tp.sums_at());
-        bf->rows = tp.sum_rows;
-        bf->folded = true;
-      }
-      if (int e = launch_conv_tri_bwd_filter(d, tp, x, dy, sums, ws, stream, &parts, &used)) return e;
-      return reduce_rsc(parts, used);
+  const SplitFilterPick split = pick_split_bwd_filter(d, flags, ws_bytes);
+  if (split.parts) {
+    const TriFilterPlan& tp = split.plan;
+    if (!tp.ok) return RH_E_UNSUPPORTED;
+    if (ws_bytes < tp.total()) return RH_E_WORKSPACE;
+    if (d.w_elems == 0) return 0;
+    float* parts = nullptr;
+    int used = 1;
+    float* sums = nullptr;
+    if (bf && bf->db) {
+      bf->part = sums = reinterpret_cast<float*>(static_cast<char*>(ws) + tp.sums_at());
+      bf->rows = tp.sum_rows;
+      bf->folded = true;
     }
+    if (int e = (split.parts == 3 ? launch_conv_tri_bwd_filter : launch_conv_duo_bwd_filter)(d, tp, x, dy, sums, ws, stream, &parts, &used)) return e;
+    return reduce_rsc(parts, used);
   }
   if ((flags & RH_ALGO_WINOGRAD) && (!wino_shape(d) || (flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT))))
     return RH_E_UNSUPPORTED;

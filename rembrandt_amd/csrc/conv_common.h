@@ -174,6 +174,7 @@ typedef Tile<64, 256, 8, 1, 4, 4> T64x256k8;
 typedef Tile<128, 128, 16, 2, 2, 2> T128x128t;
 typedef Tile<96, 128, 16, 1, 4, 2> T96x128t;
 typedef Tile<64, 192, 16, 2, 2, 2> T64x192t;
+typedef Tile<64, 256, 16, 1, 4, 2> T64x256t;   // gemm_duo.h
 inline bool prefer_k8_64(long long cols) {
   const long long tiles = cdiv<long long>(cols, 256);
   return cdiv<long long>(tiles, 1024) < cdiv<long long>(tiles, 768);
@@ -589,6 +590,15 @@ inline TriPlan plan_tri_bwd_data(const ConvDims& d, int max_chain = 0) {
 }
 int launch_conv_tri(const TriPlan& p, bool bwd, const float* in, const float* w, float* out, float alpha, float beta,
                     const float* bias, int relu, const float* mask, void* ws, hipStream_t stream);
+// The same with operands of two scaled fp16 parts (conv_duo.hip): scratch [group offsets, exponents, maxima][filter][image][partial sums].
+TriPlan plan_duo(int N, int Ci, int Hi, int Wi, int rows, int R, int S, int st, int halo, int P, int Q);
+inline TriPlan plan_duo_pass(const ConvDims& d, bool bwd) {
+  if (!bwd) return plan_duo(d.N, d.C, d.H, d.W, d.K, d.R, d.S, d.st, d.pad, d.P, d.Q);
+  if (d.st != 1 || d.R != d.S) return TriPlan{};
+  return plan_duo(d.N, d.K, d.P, d.Q, d.C, d.R, d.S, 1, d.R - 1 - d.pad, d.H, d.W);
+}
+int launch_conv_duo(const TriPlan& p, bool bwd, const float* in, const float* w, float* out, float alpha, float beta,
+                    const float* bias, int relu, const float* mask, void* ws, hipStream_t stream);
 struct TriFilterPlan {
   int Hp, Wp, n8, groups_true, groups, bm, bn, splits;
   int sum_rows;   // rows of K partial sums of dy that the copy can leave for the bias gradient
@@ -603,6 +613,9 @@ TriFilterPlan plan_tri_bwd_filter(const ConvDims& d, bool wide);
 // Leaves `used` slices of dw in (ko, r, s, c) order in *parts, and in `sums`, if given, rows whose sum is dy's over images and
 // pixels.
 int launch_conv_tri_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
+                               hipStream_t stream, float** parts, int* used);
+TriFilterPlan plan_duo_bwd_filter(const ConvDims& d);
+int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
                                hipStream_t stream, float** parts, int* used);
 
 bool conv1x1_stream_applies(const ConvDims& d);
@@ -619,6 +632,10 @@ inline bool tri_allowed(int flags) {
 }
 inline bool tri_wide(int flags) { return (flags & RH_ALGO_BF16X3_WIDE) != 0; }
 inline bool tri_forced(int flags) { return tri_allowed(flags) && (flags & RH_ALGO_DIRECT); }
+inline bool duo_allowed(int flags) {
+  return (flags & RH_ALGO_F16X2) && !(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_WINOGRAD));
+}
+inline bool duo_forced(int flags) { return duo_allowed(flags) && (flags & RH_ALGO_DIRECT) && !tri_allowed(flags); }
 // Squared relative error against 64 bits, in units of 1e-14, N(0,1) operands: of this form 0.0525 a K step in a chain (1.34e-7
 // at 36, 1.95e-7 at 72), of the engine 0.0335 a term, of the Winograd form as in wino_stages_at_most, of the staged form
 // 0.032 a term of its two chains and four more (0.09 2^-48: a rounding's variance).  The chain allowed is the one with three
@@ -667,35 +684,81 @@ inline bool tri_shape(const ConvDims& d, bool bwd) {
 inline TriPlan plan_tri_pass(const ConvDims& d, bool bwd, int max_chain) {
   return bwd ? plan_tri_bwd_data(d, max_chain) : plan_tri_fwd(d, max_chain);
 }
-// plan: what is to be launched where it pays.
-inline bool tri_pays(const ConvDims& d, bool bwd, int flags, TriPlan* plan) {
-  if (!tri_shape(d, bwd)) return false;
+// The form of split operands that a call takes, if any: 3 or 2 parts.  Two parts where they are expected to be faster than what the
+// call takes otherwise, and no further from 64 bits.
+// What two parts lose that three do not, 2^-23 of a value, is the same at every length, and deltas behind a max-pool are zeros for the most
+// part, so the chains that three parts round are short: of AlexNet's conv5 (384 filters in 256) the data gradient has an error of
+// 1.04e-7 with three parts at 144 K steps in a chain and 0.79e-7 at 72, with two parts 0.94 and 1.03e-7.  In the forward pass, half
+// zeros: 1.04 and 1.16e-7 at 36 steps, 1.55 and 1.2 at 72, 2.3 and 1.3 at 144 (three and two parts).  So two parts replace three from
+// about 55 K steps in a chain on, in backward-data from 130.
+inline bool duo_replaces_tri(bool bwd, const TriPlan& tri, int duo_steps) {
+  const int chain = cdiv(tri.groups / 2, tri.splits);
+  return bwd ? chain >= 130 : 0.0525 * chain >= 2.5 + 0.008 * duo_steps;
+}
+// The others' errors are in tri_max_chain's units, N(0,1).  Over 539 timed calls (18 layers at 11 batches, all passes, half zeros) two parts
+// are taken in 137, 1.34 times as fast in the geometric mean, none slower, with 0.50 of the error of the form replaced, 0.87 at most; on
+// the networks' own activations, filters and deltas (forward, data and filter gradient; geometric mean and largest) AlexNet 0.59, 0.54,
+// 0.50 and 0.92, NIN 0.62, 0.50, 0.26 and 0.94, ResNet-18 0.52, 0.34 and 0.81 (131 calls).
+inline bool duo_replaces(double err, int duo_steps) { return 2.5 + 0.008 * duo_steps <= err; }
+struct SplitPick {
+  int parts;
+  TriPlan plan;
+};
+// (the estimates of three and two parts have an error of 6 % each; a twenty-fifth keeps the choice from changing for nothing)
+inline bool duo_pays(const TriPlan& p, bool bwd, const TriPlan* tri, const TriRival& other) {
+  const int steps = p.ok ? cdiv(p.groups / 2, p.splits) : 0;
+  if (!p.ok || p.us >= 0.96 * (tri ? tri->us : other.us)) return false;
+  return tri ? duo_replaces_tri(bwd, *tri, steps) : duo_replaces(other.err, steps);
+}
+inline SplitPick pick_split(const ConvDims& d, bool bwd, int flags, size_t ws_bytes) {
+  SplitPick s = {};
+  if (tri_forced(flags) || duo_forced(flags)) {
+    s.parts = tri_forced(flags) ? 3 : 2;
+    s.plan = s.parts == 3 ? plan_tri_pass(d, bwd, 0) : plan_duo_pass(d, bwd);
+    return s;
+  }
+  if ((!tri_allowed(flags) && !duo_allowed(flags)) || !tri_shape(d, bwd)) return s;
   TriRival r[2];
   tri_rivals(d, bwd, r);
   const TriRival& other = r[flags & RH_ALGO_SHARED_GPU ? 1 : 0];
-  *plan = plan_tri_pass(d, bwd, tri_max_chain(other.err));
-  return plan->ok && plan->us < other.us;
+  if (tri_allowed(flags)) {
+    const TriPlan p = plan_tri_pass(d, bwd, tri_max_chain(other.err));
+    if (p.ok && p.us < other.us && p.total() <= ws_bytes) s = SplitPick{3, p};
+  }
+  if (duo_allowed(flags)) {
+    const TriPlan p = plan_duo_pass(d, bwd);
+    if (p.total() <= ws_bytes && duo_pays(p, bwd, s.parts ? &s.plan : nullptr, other)) s = SplitPick{2, p};
+  }
+  return s;
 }
-// Scratch of the form where it pays, with the hint or without; 0 also where it cannot be more than `floor`: sized for every
-// batch up to a capacity from the largest down, many batches end there.
-inline size_t tri_bytes(const ConvDims& d, bool bwd, size_t floor) {
+// Scratch of these forms where they pay, with the hint or without (three parts' also where two are taken: with less scratch a call
+// takes those); 0 also where it cannot be more than `floor`: sized for every batch up to a capacity from the largest down, many
+// batches end there.
+inline size_t split_bytes(const ConvDims& d, bool bwd, int flags, size_t floor) {
   if (!tri_shape(d, bwd)) return 0;
-  // (plan_tri's copies, and 24 slices of all tiles, of 256 MB together, or 12 of up to 255 tiles and of an image that they share)
+  // (the copies of three parts, and 24 slices of all tiles, of 256 MB together, or 12 of up to 255 tiles and of an image that they share;
+  // exponents and maxima)
   const int halo = bwd ? d.R - 1 - d.pad : d.pad, rows = bwd ? d.C : d.K, Ci = bwd ? d.K : d.C;
   const double img = 6.0 * d.N * Ci * ((bwd ? d.P : d.H) + 2 * halo) * ((bwd ? d.Q : d.W) + 2 * halo);
   const double out = 4.0 * (double)(bwd ? d.x_elems : d.y_elems);
   const double parts = fmin(24.0 * out, 12.0 * ((256.0 + rows / 64) * 128 * 192 * 4 + out / d.N));
-  if (img + (6.5 * Ci * d.R * d.S + 48.0) * rows + parts + 4096.0 < (double)floor) return 0;
+  if (img + (6.5 * Ci * d.R * d.S + 64.0) * rows + parts + 160.0 * d.N + 8192.0 < (double)floor) return 0;
   TriRival r[2];
   tri_rivals(d, bwd, r);
   size_t need = 0;
-  TriPlan p = {};
+  TriPlan p = {}, q = {};
+  if (duo_allowed(flags)) q = plan_duo_pass(d, bwd);
   int chain = 0;
   for (const TriRival& other : r) {
-    const int c = tri_max_chain(other.err);
-    if (c != chain) p = plan_tri_pass(d, bwd, c);
-    chain = c;
-    if (p.ok && p.us < other.us && p.total() > need) need = p.total();
+    bool tri = false;
+    if (tri_allowed(flags)) {
+      const int c = tri_max_chain(other.err);
+      if (c != chain) p = plan_tri_pass(d, bwd, c);
+      chain = c;
+      tri = p.ok && p.us < other.us;
+      if (tri && p.total() > need) need = p.total();
+    }
+    if (duo_pays(q, bwd, tri ? &p : nullptr, other) && q.total() > need) need = q.total();
   }
   return need;
 }
@@ -704,7 +767,11 @@ inline size_t tri_bytes(const ConvDims& d, bool bwd, size_t floor) {
 // which this form is then chosen in 188, 1.53 times as fast in the geometric mean).  1x1 layers need 384 channels or so to be
 // worth two split copies.  Its slices are short enough for the chain limit almost everywhere: it turns down 4 of 5493 calls (30
 // layers at every batch up to 256), of one to four images.
-bool tri_pays_bwd_filter(const ConvDims& d, const TriFilterPlan& t);
+struct SplitFilterPick {
+  int parts;
+  TriFilterPlan plan;
+};
+SplitFilterPick pick_split_bwd_filter(const ConvDims& d, int flags, size_t ws_bytes, size_t* need = nullptr);
 
 int launch_conv_lds(const LdsConvPlan& pl, bool bwd, int N, int Ci, int H, int W, int rows, int P, int Q, int R, int halo,
                     const float* in, const float* w, float* out, float alpha, float beta, const float* bias, int relu,

@@ -642,16 +642,12 @@ extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x,
   if ((flags & RH_ALGO_WINOGRAD) && (!(wino_shape(d) || wino_shape5(d)) ||
                                      (flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT))))
     return RH_E_UNSUPPORTED;
-  if (tri_allowed(flags)) {
-    TriPlan tp = {};
-    if (tri_forced(flags)) {
-      tp = plan_tri_fwd(d);
-      if (!tp.ok) return RH_E_UNSUPPORTED;
-      if (ws_bytes < tp.total()) return RH_E_WORKSPACE;
-    }
-    if (tri_forced(flags) || (tri_pays(d, false, flags, &tp) && ws_bytes >= tp.total()))
-      return launch_conv_tri(tp, false, x, w, y, alpha, beta, (flags & RH_FUSE_BIAS) ? bias : nullptr, (flags & RH_FUSE_RELU) ? 1 : 0,
-                             nullptr, ws, stream);
+  const SplitPick split = pick_split(d, false, flags, ws_bytes);
+  if (split.parts) {
+    if (!split.plan.ok) return RH_E_UNSUPPORTED;
+    if (ws_bytes < split.plan.total()) return RH_E_WORKSPACE;
+    return (split.parts == 3 ? launch_conv_tri : launch_conv_duo)(split.plan, false, x, w, y, alpha, beta, (flags & RH_FUSE_BIAS) ? bias : nullptr,
+                                                                (flags & RH_FUSE_RELU) ? 1 : 0, nullptr, ws, stream);
   }
   if (!(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET)) && conv1x1_stream_applies(d))
     return launch_conv1x1_stream(d, RH_CONV_FWD, w, x, y, alpha, beta, (flags & RH_FUSE_BIAS) ? bias : nullptr,

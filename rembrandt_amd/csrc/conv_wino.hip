@@ -1665,9 +1665,7 @@ extern "C" double rh_conv2d_winograd_flops(const rh_conv_geom* g, int pass, int 
   ConvDims d;
   if (conv_dims(g, &d)) return 0.0;
   if (flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT)) return 0.0;
-  TriPlan tp;
-  if (tri_allowed(flags) && (tri_forced(flags) || (pass == RH_CONV_BWD_FILTER ? tri_pays_bwd_filter(d, plan_tri_bwd_filter(d, tri_wide(flags)))
-                                                                  : tri_pays(d, pass == RH_CONV_BWD_DATA, flags, &tp))))
+  if (pass == RH_CONV_BWD_FILTER ? pick_split_bwd_filter(d, flags, ~size_t(0)).parts : pick_split(d, pass == RH_CONV_BWD_DATA, flags, ~size_t(0)).parts)
     return 0.0;
   if (wino_shape5(d) && pass == RH_CONV_FWD) {
     WinoGeom wg = wino_geom_fwd5(d);

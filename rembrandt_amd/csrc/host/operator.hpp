@@ -291,8 +291,8 @@ struct ExecOptions {
   // 3x3 stride-1 convolutions of 64 channels and more (all three passes) by Winograd F(2x2, 3x3), where the library
   // takes that form by itself; false keeps the direct form everywhere (RH_ALGO_DIRECT).
   bool winograd = true;
-  // Convolutions and affine products on bf16 matrix instructions with exactly split operands (RH_ALGO_BF16X3), where the
-  // library takes that form by itself; not without `winograd`.
+  // Convolutions and affine products on bf16 or fp16 matrix instructions with split operands (RH_ALGO_BF16X3, RH_ALGO_F16X2), where the
+  // library takes those forms by itself; not without `winograd`.
   bool split_operands = true;
 };
 

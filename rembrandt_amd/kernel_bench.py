@@ -73,6 +73,11 @@ def launched_tags(fn):
     return tags
 
 
+def split_products(tags):
+    """Products that the split-operand kernel among `tags` executes for an fp32 one; 0 without one."""
+    return 3.0 if any("_duo_" in t for t in tags) else 6.0 if any("_tri_" in t for t in tags) else 0.0
+
+
 def main(argv=None):
     ap = argparse.ArgumentParser(description=__doc__, formatter_class=argparse.RawDescriptionHelpFormatter)
     ap.add_argument("what", nargs="*", default=["conv", "fc", "mem"], help="conv | fc | mem")
@@ -81,7 +86,7 @@ def main(argv=None):
     ap.add_argument("--iters", type=int, default=5)
     ap.add_argument("--warmup", type=int, default=2)
     ap.add_argument("--relu-data", action="store_true", help="x = max(N(0,1), 0): the sparsity real activations have")
-    ap.add_argument("--split-operands", action="store_true", help="fp32 calls with RH_ALGO_BF16X3, as the operators make them")
+    ap.add_argument("--split-operands", action="store_true", help="fp32 calls with RH_ALGO_BF16X3 and RH_ALGO_F16X2, as the operators make them")
     args = ap.parse_args(argv)
 
     import torch
@@ -91,7 +96,7 @@ def main(argv=None):
     from . import _lib, ops
     dev = torch.device("cuda:0")
     passes = set(args.passes.split(","))
-    algo = _lib.RH_ALGO_BF16X3 if args.split_operands else 0
+    algo = _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_F16X2 if args.split_operands else 0
 
     def timeit(fn):
         for _ in range(args.warmup):
@@ -118,10 +123,11 @@ def main(argv=None):
 
     def report_product(kernel, layer, fn, work, winograd=0.0):
         ms = timeit(fn)
-        if algo and any("_tri_" in t for t in launched_tags(fn)):
+        split = split_products(launched_tags(fn)) if algo else 0
+        if split:
             print(json.dumps({"kernel": kernel, "layer": layer, "ms": round(ms, 4), "achieved": round(work / ms / 1e9, 1), "unit": "TFLOP/s",
-                              "peak": PEAK["bf16"], "frac": round(6.0 * work / ms / 1e9 / PEAK["bf16"], 4), "form": "split operands",
-                              "executed": round(6.0 * work / ms / 1e9, 1)}), flush=True)
+                              "peak": PEAK["bf16"], "frac": round(split * work / ms / 1e9 / PEAK["bf16"], 4), "form": "split operands",
+                              "executed": round(split * work / ms / 1e9, 1)}), flush=True)
         else:
             report(kernel, layer, ms, work, "fp32", winograd)
 

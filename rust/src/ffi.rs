@@ -60,6 +60,7 @@ pub const RH_ALGO_DIRECT: c_int = 0x800;
 pub const RH_ALGO_SHARED_GPU: c_int = 0x1000;
 pub const RH_ALGO_BF16X3: c_int = 0x2000;
 pub const RH_ALGO_BF16X3_WIDE: c_int = 0x4000;
+pub const RH_ALGO_F16X2: c_int = 0x8000;
 
 #[link(name = "rembrandt_hip")]
 extern "C" {

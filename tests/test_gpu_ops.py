@@ -751,6 +751,137 @@ def test_conv2d_bf16x3_wide_marks(dev):
             assert np.array_equal(got[:, :4], want[:, :4]), (image, extra)
 
 
+# RH_ALGO_F16X2: every operand value as the sum of two scaled fp16 values.  X3_CASES are at its edges too (64 rows to a block of a tile;
+# 64 x 256, 96 x 128 and 128 x 128 tiles); then K steps around a chain's end and the ring's (8 K steps and 4 or 5 buffers).
+F16X2_CASES = X3_CASES + [(1, 16 * n, 3, 3, 70, 1, 1, 0) for n in (4, 5, 11, 12, 13, 20, 21)] + [(1, 16 * n, 2, 2, 128, 1, 1, 0) for n in (11, 12, 29)] + \
+    [(8, 8, 1, 2 * n, 128, 1, 1, 0) for n in (3, 13, 27)]
+
+
+@pytest.mark.parametrize("case", F16X2_CASES, ids=str)
+def test_conv2d_f16x2(dev, case):
+    """All passes with operands of two parts against the oracle, with every epilogue; images, filters and channels far apart in size."""
+    Nn, C, H, W, K, R, st, pad = case
+    say("f16x2 case", case)
+    F2 = _lib.RH_ALGO_F16X2 | _lib.RH_ALGO_DIRECT
+    x, w, b = synth.normal(37, 1, (Nn, C, H, W)), synth.normal(37, 2, (K, C, R, R)), synth.normal(37, 3, (K,))
+    y_ref = O.conv2d_fwd(x, w, st, pad)
+    dy, y0, dx0, dw0, db0 = (synth.normal(37, 4 + i, s) for i, s in enumerate((y_ref.shape, y_ref.shape, x.shape, w.shape, (K,))))
+    xd, wd, bd, dyd = T(x, dev), T(w, dev), T(b, dev), T(dy, dev)
+    image, row = ((2.0 ** (10 * synth.normal(38, i, (n,))).astype(int)[:, None, None, None]).astype(np.float32) for i, n in ((0, Nn), (1, K)))
+    if C % 8 == 0:
+        y, tags = profile_tags(lambda: ops.conv2d_fwd(xd, wd, st, pad, algo=F2))
+        assert any(t.startswith("conv_fwd_duo_") for t in tags), tags
+        assert_close(N(y), y_ref, "f16x2 fwd")
+        yf = ops.conv2d_fwd(xd, wd, st, pad, bias=bd, relu=True, algo=F2)
+        assert torch.equal(torch.clamp_min(y + bd.view(1, -1, 1, 1), 0.0), yf), "fused epilogue == conv, add_bias, rect"
+        yb = ops.conv2d_fwd(xd, wd, st, pad, alpha=0.5, beta=2.0, y=T(y0, dev), algo=F2)
+        assert_close(N(yb), O.conv2d_fwd(x, w, st, pad, alpha=0.5, beta=2.0, y=y0.copy()), "f16x2 fwd alpha/beta")
+        assert torch.equal(ops.conv2d_fwd(xd, wd, st, pad, algo=F2), y), "run to run the same bits"
+        scaled = ops.conv2d_fwd(T(x * image, dev), T(w * row, dev), st, pad, algo=F2)
+        assert np.array_equal(N(scaled), N(y) * image * row.reshape(1, -1, 1, 1)), "powers of two of an image and a filter"
+    else:
+        with pytest.raises(_lib.RembrandtHipError):
+            ops.conv2d_fwd(xd, wd, st, pad, algo=F2)
+    if K % 8 == 0 and st == 1 and pad <= R - 1:
+        dx, tags = profile_tags(lambda: ops.conv2d_bwd_data(wd, dyd, x.shape, st, pad, algo=F2))
+        assert any(t.startswith("conv_bwd_data_duo_") for t in tags), tags
+        assert_close(N(dx), O.conv2d_bwd_data(w, dy, x.shape, st, pad), "f16x2 bwd data")
+        two = ops.conv2d_bwd_data(wd, dyd, x.shape, st, pad, alpha=0.5, beta=2.0, dx=T(dx0, dev), algo=F2)
+        assert_close(N(two), O.conv2d_bwd_data(w, dy, x.shape, st, pad, 0.5, 2.0, dx0.copy()), "f16x2 bwd data alpha/beta")
+        ops.rect_backprop_inplace(xd, two)
+        one = ops.conv2d_bwd_data(wd, dyd, x.shape, st, pad, alpha=0.5, beta=2.0, dx=T(dx0, dev), algo=F2, relu_of=xd)
+        assert torch.equal(one, two), "masked data gradient"
+        assert np.array_equal(N(ops.conv2d_bwd_data(wd, T(dy * image, dev), x.shape, st, pad, algo=F2)), N(dx) * image), "powers of two of an image"
+    else:
+        with pytest.raises(_lib.RembrandtHipError):
+            ops.conv2d_bwd_data(wd, dyd, x.shape, st, pad, algo=F2)
+    dw, tags = profile_tags(lambda: ops.conv2d_bwd_filter(xd, dyd, w.shape, st, pad, algo=F2))
+    assert any(t.startswith("conv_bwd_filter_duo_") for t in tags), tags
+    assert_close(N(dw), O.conv2d_bwd_filter(x, dy, w.shape, st, pad), "f16x2 bwd filter")
+    dwc, dbc = ops.conv2d_bwd_filter_bias(xd, dyd, w.shape, st, pad, alpha=0.25, beta=1.0, dw=T(dw0, dev), db=T(db0, dev), algo=F2)
+    assert_close(N(dwc), O.conv2d_bwd_filter(x, dy, w.shape, st, pad, 0.25, 1.0, dw0.copy()), "f16x2 bwd filter alpha/beta")
+    assert_close(N(dbc), O.conv2d_bwd_bias(dy, 0.25, 1.0, db0.copy()), "f16x2 bias gradient")
+    assert torch.equal(ops.conv2d_bwd_filter(xd, dyd, w.shape, st, pad, algo=F2), dw), "run to run the same bits"
+    scaled = ops.conv2d_bwd_filter(xd, T(dy * row.reshape(1, -1, 1, 1), dev), w.shape, st, pad, algo=F2)
+    assert np.array_equal(N(scaled), N(dw) * row), "powers of two of a channel"
+
+
+def test_conv2d_f16x2_values_out_of_range(dev):
+    """What two parts cannot hold is formed again from the operands: values far below the largest of their image or channel where no larger
+    one is beside them, infinities, NaNs, the largest and the smallest floats."""
+    say("f16x2 values")
+    F2, big = _lib.RH_ALGO_F16X2 | _lib.RH_ALGO_DIRECT, np.finfo(np.float32).max
+    Nn, C, H, K, R = 9, 24, 12, 72, 3
+    x, w = synth.normal(39, 1, (Nn, C, H, H)), 0.01 * synth.normal(39, 2, (K, C, R, R))
+    dy = synth.normal(39, 3, (Nn, K, H, H))
+    x[0, :, 2, 2], x[1] = 1e25, x[1] * 1e-30             # one pixel beside which the others of its image have no bits; a small image
+    x[2, 3, 5, 5], x[3, 4, 1, 1], x[4, 0, 0, 0] = np.inf, np.nan, -np.inf
+    x[5] *= np.float32(1e-42)                            # denormal
+    w[7] *= np.float32(1e-38)
+    dy[:, 5, 0, 0] = 0.0
+    dy[8, 5, 3, 3] = 1e28
+    for name, run, ref in (("fwd", lambda a: ops.conv2d_fwd(T(x, dev), T(w, dev), 1, 1, algo=a), O.conv2d_fwd(x, w, 1, 1)),
+                           ("bwd filter", lambda a: ops.conv2d_bwd_filter(T(x[6:], dev), T(dy[6:], dev), w.shape, 1, 1, algo=a),
+                            O.conv2d_bwd_filter(x[6:], dy[6:], w.shape, 1, 1)),
+                           ("bwd data", lambda a: ops.conv2d_bwd_data(T(w, dev), T(dy, dev), x.shape, 1, 1, algo=a), O.conv2d_bwd_data(w, dy, x.shape, 1, 1))):
+        got, other = N(run(F2)), N(run(_lib.RH_ALGO_GATHER))
+        assert np.array_equal(np.isnan(got), np.isnan(other)) and np.array_equal(np.isinf(got), np.isinf(other)), name
+        ok = np.isfinite(ref) & (np.abs(ref) >= 2.0 ** -126)
+        # of each result plane, whose sums are of one size; 24 x 9 terms of relative error 2^-22 at most each, in quadrature below 2^-21
+        for g, r, m in zip(got.reshape(-1, got.shape[-1] ** 2).astype(np.float64), ref.reshape(-1, got.shape[-1] ** 2).astype(np.float64), ok.reshape(-1, got.shape[-1] ** 2)):
+            if not m.any() or np.abs(r[m]).max() > 1e3 * np.median(np.abs(r[m])):   # (a plane with the large pixel: its far results below)
+                continue
+            assert np.linalg.norm(g[m] - r[m]) <= 2.0 ** -21 * np.linalg.norm(r[m]), name
+        if name == "fwd":   # away from the large pixel of image 0
+            far = np.s_[0, :, 5:, 5:]
+            assert np.linalg.norm((got[far] - ref[far]).astype(np.float64)) <= 2.0 ** -21 * np.linalg.norm(ref[far].astype(np.float64))
+    x = np.zeros((1, 8, 1, 8), np.float32)
+    x[0, 3] = [big, -big, 1.0, 2.0 ** -149, 2.0 ** -126, 0.0, -0.0, 3.0]
+    w = np.zeros((64, 8, 1, 1), np.float32)
+    w[:, 3, 0, 0] = 1.0
+    got = N(ops.conv2d_fwd(T(x, dev), T(w, dev), 1, 0, algo=F2))
+    assert np.array_equal(got[0], np.broadcast_to(x[0, 3], (64, 1, 8)))
+
+
+# Layers with the passes that the library takes in this form by itself beside RH_ALGO_BF16X3: whole contractions, slices, a sliced
+# tail, 64- and 96-row tiles
+F16X2_ERROR_CASES = [
+    # N, C, H, K, R, stride, pad, passes
+    (50, 384, 13, 384, 3, 1, 1, "fd"),
+    (24, 96, 27, 256, 5, 1, 2, "f"),
+    (128, 96, 27, 256, 5, 1, 2, "fw"),
+    (64, 128, 28, 128, 3, 1, 1, "fd"),
+    (200, 64, 56, 64, 3, 1, 1, "fd"),
+    (128, 512, 7, 512, 3, 1, 1, "fd"),
+    (16, 96, 27, 256, 1, 1, 0, ""),
+]
+
+
+@pytest.mark.parametrize("data", ["normal", "half_zeros"])
+@pytest.mark.parametrize("case", F16X2_ERROR_CASES, ids=str)
+def test_conv2d_f16x2_error(dev, case, data):
+    """Error against 64-bit sums where the library takes the form by itself: no larger than that of the form it replaces."""
+    Nn, C, H, K, R, st, pad, takes = case
+    say("f16x2 error", case, data)
+    P = (H + 2 * pad - R) // st + 1
+    x, w, dy = (T(synth.normal(36, 1 + i, s), dev) for i, s in enumerate(((Nn, C, H, H), (K, C, R, R), (Nn, K, P, P))))
+    if data == "half_zeros":
+        x, dy = x.clamp_min(0.0), dy * (T(synth.uniform(36, 4, dy.shape), dev) < 0.5)
+    X3 = _lib.RH_ALGO_BF16X3
+    refs = _conv_sums64(x, w, dy, st, pad)
+    for key, name, ref, run in (("f", "fwd", refs[0], lambda algo: ops.conv2d_fwd(x, w, st, pad, algo=algo)),
+                                ("d", "bwd_data", refs[1], lambda algo: ops.conv2d_bwd_data(w, dy, x.shape, st, pad, algo=algo)),
+                                ("w", "bwd_filter", refs[2], lambda algo: ops.conv2d_bwd_filter(x, dy, w.shape, st, pad, algo=algo))):
+        got, tags = profile_tags(lambda: run(X3 | _lib.RH_ALGO_F16X2))
+        assert any(t.startswith("conv_%s_duo_" % name) for t in tags) == (key in takes), (name, tags)
+        before = run(X3)
+        if key in takes:
+            err, err0 = (float((t.double() - ref).norm() / ref.norm()) for t in (got, before))
+            assert err <= err0, (name, err, err0)
+        else:
+            assert torch.equal(got, before), name
+
+
 @pytest.mark.parametrize("case", [(9, 16, 14, 11, 40, 3, 5, 1, 2), (3, 24, 9, 12, 72, 1, 4, 1, 0), (8, 40, 12, 9, 64, 5, 1, 1, 1),
                                   (5, 16, 13, 10, 33, 2, 3, 2, 1), (24, 64, 30, 28, 128, 2, 3, 2, 1)], ids=str)
 def test_conv2d_bf16x3_filters_that_are_not_square(dev, case):

@@ -216,6 +216,25 @@ def test_bf16x3_scratch_is_for_callers_that_allow_the_form(geom):
                 assert lib.rh_conv2d_workspace_bytes_upto(C.byref(g), pass_) == most
 
 
+@pytest.mark.parametrize("geom", BF16X3_GEOMS, ids=str)
+def test_f16x2_scratch_is_for_callers_that_allow_the_form(geom):
+    """The same for RH_ALGO_F16X2, beside RH_ALGO_BF16X3 and forced; beside it a call with the other form's scratch alone stays valid."""
+    lib = _lib.lib()
+    cap, c, extent, k, size, st, pad = geom
+    X3, F2 = _lib.RH_ALGO_BF16X3, _lib.RH_ALGO_F16X2
+    for pass_ in (_lib.RH_CONV_FWD, _lib.RH_CONV_BWD_FILTER, _lib.RH_CONV_BWD_DATA):
+        for flags in (X3 | F2, F2, F2 | _lib.RH_ALGO_DIRECT):
+            most = 0
+            for n in range(1, cap + 1):
+                g = _lib.ConvGeom(n, c, extent, extent, k, size, size, st, pad)
+                need = lib.rh_conv2d_workspace_bytes_for(C.byref(g), pass_, flags)
+                assert need >= lib.rh_conv2d_workspace_bytes_for(C.byref(g), pass_, flags & X3)
+                assert need == lib.rh_conv2d_workspace_bytes_for(C.byref(g), pass_, flags | _lib.RH_ALGO_SHARED_GPU)
+                most = max(most, need)
+            g = _lib.ConvGeom(cap, c, extent, extent, k, size, size, st, pad)
+            assert lib.rh_conv2d_workspace_bytes_for_upto(C.byref(g), pass_, flags) == most, (pass_, flags)
+
+
 def test_conv_scratch_without_the_bf16x3_bit():
     """What a caller without the bit needs is what the other forms need: 13 MB where the split copies take 52, 131 where they take
     159, 355 where they take 483."""
