@@ -223,12 +223,12 @@ def test_f16x2_scratch_is_for_callers_that_allow_the_form(geom):
     cap, c, extent, k, size, st, pad = geom
     X3, F2 = _lib.RH_ALGO_BF16X3, _lib.RH_ALGO_F16X2
     for pass_ in (_lib.RH_CONV_FWD, _lib.RH_CONV_BWD_FILTER, _lib.RH_CONV_BWD_DATA):
-        for flags in (X3 | F2, F2, F2 | _lib.RH_ALGO_DIRECT):
+        for flags in (X3 | F2, F2, F2 | _lib.RH_ALGO_DIRECT, X3 | F2 | _lib.RH_ALGO_BF16X3_WIDE, F2 | _lib.RH_ALGO_DIRECT | _lib.RH_ALGO_BF16X3_WIDE):
             most = 0
             for n in range(1, cap + 1):
                 g = _lib.ConvGeom(n, c, extent, extent, k, size, size, st, pad)
                 need = lib.rh_conv2d_workspace_bytes_for(C.byref(g), pass_, flags)
-                assert need >= lib.rh_conv2d_workspace_bytes_for(C.byref(g), pass_, flags & X3)
+                assert need >= lib.rh_conv2d_workspace_bytes_for(C.byref(g), pass_, flags & (X3 | _lib.RH_ALGO_BF16X3_WIDE))
                 assert need == lib.rh_conv2d_workspace_bytes_for(C.byref(g), pass_, flags | _lib.RH_ALGO_SHARED_GPU)
                 most = max(most, need)
             g = _lib.ConvGeom(cap, c, extent, extent, k, size, size, st, pad)
