@@ -86,30 +86,31 @@ __device__ __forceinline__ float sum_splits(const float* __restrict__ part, int 
   return (a0 + a1) + (a2 + a3);
 }
 
-// Column sums of an [N][K] matrix (dy of an affine layer, or per-image plane sums) for the 64 columns from 64 b on by
-// one block of 256 threads: its 4 waves take every fourth row and are combined through LDS in a fixed order.
+// Column sums of an [N][K] matrix (dy of an affine layer, or per-image plane sums) for bias_rows_cols(N) columns by one block of 256
+// threads.  Bound by the chain of a thread's reads, eight at a time: with 64 columns to a block the 3040 rows that the copies of a
+// 96-channel 55 x 55 layer leave at 256 images were 95 round trips, 56 us for the launch, now 12 and 15.  A fixed order.
 __device__ __forceinline__ void bwd_bias_rows_block(const float* __restrict__ dy, int N, int K, float alpha, float beta,
                                                     float* __restrict__ db, unsigned b) {
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int k = (int)b * 64 + lane;
-  // eight independent partial sums per thread (rows wave, wave + 4, ... in turn): the loop is a chain of memory round
-  // trips, so its length is what the kernel takes
+  const int cols = bias_rows_cols(N), rows = 256 / cols;
+  const int cl = threadIdx.x & (cols - 1), k = (int)b * cols + cl;
   float a[8] = {0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f, 0.0f};
   if (k < K) {
-    int n = wave;
-    for (; n + 28 < N; n += 32) {
+    int n = threadIdx.x / cols;
+    for (; n + 7 * rows < N; n += 8 * rows) {
 #pragma unroll
-      for (int j = 0; j < 8; ++j) a[j] += dy[(size_t)(n + 4 * j) * K + k];
+      for (int j = 0; j < 8; ++j) a[j] += dy[(size_t)(n + rows * j) * K + k];
     }
 #pragma unroll
     for (int j = 0; j < 8; ++j)
-      if (n + 4 * j < N) a[j] += dy[(size_t)(n + 4 * j) * K + k];
+      if (n + rows * j < N) a[j] += dy[(size_t)(n + rows * j) * K + k];
   }
-  __shared__ float sm[4][64];
-  sm[wave][lane] = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+  float v = ((a[0] + a[1]) + (a[2] + a[3])) + ((a[4] + a[5]) + (a[6] + a[7]));
+  for (int o = cols; o < 64; o <<= 1) v += __shfl_xor(v, o, 64);
+  __shared__ float sm[4][16];
+  if ((int)(threadIdx.x & 63) < cols) sm[threadIdx.x >> 6][cl] = v;
   __syncthreads();
-  if (wave == 0 && k < K) {
-    float v = alpha * ((sm[0][lane] + sm[1][lane]) + (sm[2][lane] + sm[3][lane]));
+  if ((int)threadIdx.x < cols && k < K) {
+    v = alpha * ((sm[0][cl] + sm[1][cl]) + (sm[2][cl] + sm[3][cl]));
     if (beta != 0.0f) v += beta * db[k];
     db[k] = v;
   }
@@ -659,57 +660,101 @@ __global__ __launch_bounds__(256) void bwd_filter_prep_kernel(NhwcCopyArgs dy, f
                             x.Wp, x.C, Kout);
 }
 
-// dw[ko][c][r][s] = alpha * sum_s part[s][ko][(r,s,c)] + beta * dw
-__global__ void split_reduce_rsc_kernel(const float* __restrict__ part, int splits, long long split_stride,
-                                        float* __restrict__ dw, int K, int C, int R, int S, float alpha, float beta, BiasJob bj) {
+// dw[ko][c][r][s] = alpha * sum_s part[s][ko][(r,s,c)] + beta * dw.  A block forms TS taps of CH channels of one filter: G groups of
+// its threads read every G-th slab along c, and the sums go through LDS to dw's order, so that a block's writes are runs of whole lines.
+// (Written from the slabs' order, a 36-byte stride, dw's lines were assembled from nine blocks on different XCDs.)  Bound by the
+// slabs' bytes where there are few and by the chain of reads of a thread where there are many, hence the groups.
+// From the slabs' order and now, us: 512 x 512 3x3 of 3 slices 49 and 11.9, 64 x 64 3x3 of 85 slices 10.5 and 6.5, 64 x 3 7x7 of 85
+// slices 26 and 10.4; of 16 layers that come here 13.7 and 7.6 in the geometric mean, none slower.
+struct TapsArgs {
+  const float* part; float* dw;
+  int splits, K, C, RS, CH, TS, G;
+  int c_chunks, chunks;      // of a filter: along c, in all
+  unsigned units, work;      // of a block: reads of a slab, of all groups
+  FastDiv d_units, d_row, d_ts;
+  float alpha, beta;
+};
+constexpr int kTapsLds = 8192;   // floats: G TS (CH + 1)
+template <class V>
+__global__ __launch_bounds__(256) void split_reduce_taps_kernel(TapsArgs a, BiasJob bj) {
   if (bj.db && blockIdx.x >= bj.first) { bias_job_block(bj, blockIdx.x - bj.first); return; }
-  const unsigned nb = bj.db ? bj.first : gridDim.x;
-  const int CRS = C * R * S;
-  const unsigned total = (unsigned)K * (unsigned)CRS;
-  for (unsigned idx = blockIdx.x * blockDim.x + threadIdx.x; idx < total; idx += nb * blockDim.x) {
-    const float acc = sum_splits(part, splits, split_stride, idx);
-    const int ko = (int)(idx / (unsigned)CRS), j = (int)(idx - (unsigned)ko * (unsigned)CRS);
-    const int r = j / (S * C), rem = j - r * (S * C), s2 = rem / C, c = rem - s2 * C;
-    float* dst = dw + (((size_t)ko * C + c) * R + r) * S + s2;
-    float val = alpha * acc;
-    if (beta != 0.0f) val += beta * *dst;
+  constexpr int E = sizeof(V) / 4;
+  extern __shared__ float lds[];   // [group][tap][CH + 1]
+  const int ko = (int)blockIdx.x / a.chunks, chunk = (int)blockIdx.x - ko * a.chunks;
+  const int rs0 = chunk / a.c_chunks * a.TS, c0 = chunk % a.c_chunks * a.CH;
+  const int taps = min(a.TS, a.RS - rs0), chans = min(a.CH, a.C - c0);
+  const size_t CRS = (size_t)a.C * a.RS, stride = CRS * a.K;
+  const float* const src = a.part + (size_t)ko * CRS + (size_t)rs0 * a.C + c0;
+  for (unsigned w = threadIdx.x; w < a.work; w += 256) {
+    uint32_t g, u, t, c;
+    a.d_units.divmod(w, g, u);
+    a.d_row.divmod(u, t, c);
+    if ((int)t >= taps || (int)c * E >= chans) continue;
+    const float* p = src + (size_t)t * a.C + c * E;
+    float x[4][E];
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+#pragma unroll
+      for (int e = 0; e < E; ++e) x[i][e] = 0.0f;
+    auto add = [&](float (&d)[E], int sp) {
+      const V v = *reinterpret_cast<const V*>(p + (size_t)sp * stride);
+#pragma unroll
+      for (int e = 0; e < E; ++e) d[e] += reinterpret_cast<const float*>(&v)[e];
+    };
+    int sp = (int)g;
+    for (; sp + 3 * a.G < a.splits; sp += 4 * a.G) {
+#pragma unroll
+      for (int i = 0; i < 4; ++i) add(x[i], sp + i * a.G);
+    }
+    for (; sp < a.splits; sp += a.G) add(x[0], sp);
+    float* const d = lds + ((int)g * a.TS + (int)t) * (a.CH + 1) + (int)c * E;
+#pragma unroll
+    for (int e = 0; e < E; ++e) d[e] = (x[0][e] + x[1][e]) + (x[2][e] + x[3][e]);
+  }
+  __syncthreads();
+  float* const out = a.dw + (size_t)ko * CRS + (size_t)c0 * a.RS + rs0;
+  for (unsigned o = threadIdx.x; o < (unsigned)(chans * a.TS); o += 256) {
+    uint32_t c, t;
+    a.d_ts.divmod(o, c, t);
+    if ((int)t >= taps) continue;
+    const float* const s = lds + (int)t * (a.CH + 1) + (int)c;
+    float v = s[0];
+    for (int g = 1; g < a.G; ++g) v += s[g * a.TS * (a.CH + 1)];
+    float* const dst = out + (size_t)c * a.RS + t;
+    float val = a.alpha * v;
+    if (a.beta != 0.0f) val += a.beta * *dst;
     *dst = val;
   }
 }
 
-// The same for C % 4 == 0: a thread takes four consecutive channels of one (ko, r, s), read as 16-byte groups from
-// every slab (4-byte reads top out well below what 16-byte reads reach); sums in the order of sum_splits.
-__global__ __launch_bounds__(256) void split_reduce_rsc_vec_kernel(const float4* __restrict__ part, int splits, long long stride4,
-                                                                   float* __restrict__ dw, int K, int C, int R, int S,
-                                                                   float alpha, float beta, BiasJob bj) {
-  if (bj.db && blockIdx.x >= bj.first) { bias_job_block(bj, blockIdx.x - bj.first); return; }
-  const int CRS4 = (C * R * S) >> 2;
-  const unsigned total4 = (unsigned)K * (unsigned)CRS4;
-  const unsigned idx = blockIdx.x * blockDim.x + threadIdx.x;
-  if (idx >= total4) return;
-  const float4 z = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
-  float4 a0 = z, a1 = z, a2 = z, a3 = z;
-  auto add = [](float4& a, const float4 v) { a.x += v.x; a.y += v.y; a.z += v.z; a.w += v.w; };
-  const float4* p = part + idx;
-  int sp = 0;
-  for (; sp + 3 < splits; sp += 4) {
-    add(a0, p[(long long)sp * stride4]);
-    add(a1, p[(long long)(sp + 1) * stride4]);
-    add(a2, p[(long long)(sp + 2) * stride4]);
-    add(a3, p[(long long)(sp + 3) * stride4]);
+// 1024 values to a block, or fewer where that leaves CUs idle, down to 64 bytes a read of a slab.
+static void launch_split_reduce_taps(const float* part, int splits, float* dw, int K, int C, int RS, float alpha, float beta, BiasJob bj,
+                                     hipStream_t stream) {
+  const bool vec = C % 4 == 0 && (reinterpret_cast<uintptr_t>(part) & 15) == 0;
+  TapsArgs a;
+  a.part = part; a.dw = dw; a.splits = splits; a.K = K; a.C = C; a.RS = RS; a.alpha = alpha; a.beta = beta;
+  int want = cdiv(C * RS, 1024);
+  if (want < cdiv(512, K)) want = cdiv(512, K);
+  a.CH = min(C, max(16, round_up(cdiv(C, want), 4)));
+  a.c_chunks = cdiv(C, a.CH);
+  a.TS = max(cdiv(RS, cdiv(want, a.c_chunks)), min(RS, 16));
+  while (a.TS * (a.CH + 1) > kTapsLds / 2) a.TS = cdiv(a.TS, 2);
+  a.chunks = a.c_chunks * cdiv(RS, a.TS);
+  const int row = vec ? a.CH / 4 : a.CH;
+  a.units = (unsigned)(a.TS * row);
+  a.G = 1;
+  double least = 1e30;   // reads of a thread, and of LDS
+  for (int g = 1; g <= 16 && g <= splits && g * a.TS * (a.CH + 1) <= kTapsLds; ++g) {
+    const double reads = cdiv(a.units * (unsigned)g, 256u) * cdiv(splits, g) + 0.5 * g;
+    if (reads < least) { least = reads; a.G = g; }
   }
-  for (; sp < splits; ++sp) add(a0, p[(long long)sp * stride4]);
-  const float v[4] = {(a0.x + a1.x) + (a2.x + a3.x), (a0.y + a1.y) + (a2.y + a3.y), (a0.z + a1.z) + (a2.z + a3.z),
-                      (a0.w + a1.w) + (a2.w + a3.w)};
-  const int ko = (int)(idx / (unsigned)CRS4), j = 4 * (int)(idx - (unsigned)ko * (unsigned)CRS4);
-  const int r = j / (S * C), rem = j - r * (S * C), s2 = rem / C, c = rem - s2 * C;
-  float* dst = dw + (((size_t)ko * C + c) * R + r) * S + s2;
-#pragma unroll
-  for (int e = 0; e < 4; ++e) {
-    float val = alpha * v[e];
-    if (beta != 0.0f) val += beta * dst[(size_t)e * R * S];
-    dst[(size_t)e * R * S] = val;
-  }
+  a.work = a.units * (unsigned)a.G;
+  a.d_units = FastDiv(a.units); a.d_row = FastDiv((uint32_t)row); a.d_ts = FastDiv((uint32_t)a.TS);
+  bj.first = (unsigned)K * (unsigned)a.chunks;
+  const dim3 grid(bj.first + bj.blocks());
+  const size_t lds = sizeof(float) * (size_t)a.G * a.TS * (a.CH + 1);
+  if (vec) hipLaunchKernelGGL(split_reduce_taps_kernel<float4>, grid, dim3(256), lds, stream, a, bj);
+  else hipLaunchKernelGGL(split_reduce_taps_kernel<float>, grid, dim3(256), lds, stream, a, bj);
 }
 
 template <class T>
@@ -1049,22 +1094,12 @@ static int bwd_filter_impl(const rh_conv_geom* g, float alpha, const float* x, c
   hipStream_t stream = to_stream(stream_);
   // dw from `used` slices in (ko, r, s, c) order
   auto reduce_rsc = [&](float* parts, int used) -> int {
-    const int CRSr = d.C * d.R * d.S;
-    const long long total = (long long)d.K * CRSr;
+    const long long total = (long long)d.K * d.C * d.R * d.S;
     BiasJob bj;
     bias_job(&bj);
     const unsigned jb = bj.blocks();
     ProfScope prof("split_reduce", 4.0 * (double)total * (used + 1) + (jb ? 4.0 * (double)bj.N * bj.K * bj.plane : 0.0), stream);
-    if (d.C % 4 == 0 && (reinterpret_cast<uintptr_t>(parts) & 15) == 0) {
-      bj.first = stream_grid((size_t)total / 4, 256);
-      hipLaunchKernelGGL(split_reduce_rsc_vec_kernel, dim3(bj.first + jb), dim3(256), 0, stream,
-                         reinterpret_cast<const float4*>(parts), used, (long long)d.K * CRSr / 4, dw, d.K, d.C, d.R, d.S, alpha,
-                         beta, bj);
-    } else {
-      bj.first = stream_grid((size_t)total, 256);
-      hipLaunchKernelGGL(split_reduce_rsc_kernel, dim3(bj.first + jb), dim3(256), 0, stream, parts, used,
-                         (long long)d.K * CRSr, dw, d.K, d.C, d.R, d.S, alpha, beta, bj);
-    }
+    launch_split_reduce_taps(parts, used, dw, d.K, d.C, d.R * d.S, alpha, beta, bj, stream);
     return launch_status();
   };
 
@@ -1247,7 +1282,7 @@ extern "C" int rh_conv2d_bwd_filter_bias(const rh_conv_geom* g, float alpha, con
   const int plane = d.P * d.Q;
   if (bf.folded) {   // the sums over the images of what the pass over dy left
     ProfScope prof("bwd_bias_finish", 4.0 * (double)d.N * d.K, stream);
-    hipLaunchKernelGGL(bwd_bias_rows_kernel, dim3(cdiv(d.K, 64)), dim3(256), 0, stream, bias_ws, d.N, d.K, alpha, beta, db);
+    hipLaunchKernelGGL(bwd_bias_rows_kernel, dim3(cdiv(d.K, bias_rows_cols(d.N))), dim3(256), 0, stream, bias_ws, d.N, d.K, alpha, beta, db);
     return launch_status();
   }
   ProfScope prof("bwd_bias", 4.0 * (double)d.y_elems, stream);
@@ -1292,14 +1327,14 @@ static int bwd_bias_two_stage(int N, int K, int plane, float alpha, const float*
   hipLaunchKernelGGL(bwd_bias_rowsum_kernel, dim3((unsigned)(blocks > 65536 ? 65536 : blocks)), dim3(256), 0, stream, dy,
                      rows, plane, rowsum);
   if (int e = launch_status()) return e;
-  hipLaunchKernelGGL(bwd_bias_rows_kernel, dim3(cdiv(K, 64)), dim3(256), 0, stream, rowsum, N, K, alpha, beta, db);
+  hipLaunchKernelGGL(bwd_bias_rows_kernel, dim3(cdiv(K, bias_rows_cols(N))), dim3(256), 0, stream, rowsum, N, K, alpha, beta, db);
   return launch_status();
 }
 
 static int bwd_bias_one_stage(int N, int K, int plane, float alpha, const float* dy, float beta, float* db,
                               hipStream_t stream) {
   if (plane == 1) {
-    hipLaunchKernelGGL(bwd_bias_rows_kernel, dim3(cdiv(K, 64)), dim3(256), 0, stream, dy, N, K, alpha, beta,
+    hipLaunchKernelGGL(bwd_bias_rows_kernel, dim3(cdiv(K, bias_rows_cols(N))), dim3(256), 0, stream, dy, N, K, alpha, beta,
                        db);
   } else {
     hipLaunchKernelGGL(bwd_bias_kernel, dim3(K), dim3(1024), 0, stream, dy, N, K, plane, alpha, beta, db);

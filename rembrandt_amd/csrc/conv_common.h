@@ -180,6 +180,9 @@ inline bool prefer_k8_64(long long cols) {
   return cdiv<long long>(tiles, 1024) < cdiv<long long>(tiles, 768);
 }
 
+// Columns of a block that adds up the rows of an [N][K] matrix: 64-byte reads, or of 32 where the rows are many.
+__host__ __device__ constexpr int bias_rows_cols(int N) { return N > 512 ? 8 : 16; }
+
 // Second pass of a split contraction: out[i*ld + j] = alpha * sum_s part[s][i*cols + j] + beta*out.
 // A bias gradient that rides in a reduction's launch, in blocks of its own behind the reduction's (small layers are
 // bound by the number of dependent launches): db[k] = alpha * sum over n and the plane of src[(n K + k) plane + i] +
@@ -190,7 +193,7 @@ struct BiasJob {
   int N = 0, K = 0, plane = 0;
   float alpha = 1.0f, beta = 0.0f;
   unsigned first = 0;            // the job's first block (filled in by the launcher)
-  unsigned blocks() const { return !db ? 0u : plane == 1 ? (unsigned)((K + 63) / 64) : (unsigned)K; }
+  unsigned blocks() const { return !db ? 0u : plane == 1 ? (unsigned)cdiv(K, bias_rows_cols(N)) : (unsigned)K; }
 };
 void launch_split_reduce(const float* part, int splits, long long split_stride, float* out, int rows, int cols,
                          int ld, float alpha, float beta, hipStream_t stream, const float* bias_col = nullptr, int relu = 0,

@@ -590,6 +590,27 @@ def test_conv2d_bf16x3(dev, case):
     assert torch.equal(ops.conv2d_bwd_filter(xd, dyd, w.shape, st, pad, algo=X3), wide), "run to run the same bits"
 
 
+# The reduction of a filter gradient's slices: channels that end in a chunk of their own (4 of 20, 8 of 136, 2 of 18), no multiple of
+# four, one channel; taps in chunks and a chunk of fewer; one tap; one slice and many; chunks of the widest result of a block.
+@pytest.mark.parametrize("case", [(16, 20, 14, 14, 50, 5, 1, 0), (2, 136, 9, 9, 8, 3, 1, 1), (40, 18, 21, 20, 70, 3, 1, 1), (9, 3, 60, 59, 33, 11, 4, 2),
+                                  (24, 5, 17, 17, 300, 3, 1, 1), (31, 1, 24, 24, 20, 5, 1, 0), (6, 72, 25, 25, 520, 1, 1, 0), (1, 8, 3, 3, 3, 3, 1, 0),
+                                  (8, 516, 6, 6, 513, 3, 1, 1)], ids=str)
+def test_conv2d_bwd_filter_slices(dev, case):
+    Nn, C, H, W, K, R, st, pad = case
+    say("filter slices case", case)
+    x = synth.normal(71, 1, (Nn, C, H, W))
+    w_shape = (K, C, R, R)
+    dy = synth.normal(71, 2, (Nn, K, (H + 2 * pad - R) // st + 1, (W + 2 * pad - R) // st + 1))
+    dw0, db0 = synth.normal(71, 3, w_shape), synth.normal(71, 4, (K,))
+    xd, dyd = T(x, dev), T(dy, dev)
+    for algo in (_lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_DIRECT, _lib.RH_ALGO_F16X2 | _lib.RH_ALGO_DIRECT):
+        for alpha, beta in ((1.0, 0.0), (0.25, 1.0)):
+            dw, db = ops.conv2d_bwd_filter_bias(xd, dyd, w_shape, st, pad, alpha=alpha, beta=beta, dw=T(dw0, dev), db=T(db0, dev), algo=algo)
+            assert_close(N(dw), O.conv2d_bwd_filter(x, dy, w_shape, st, pad, alpha, beta, dw0.copy()), "filter gradient from slices")
+            assert_close(N(db), O.conv2d_bwd_bias(dy, alpha, beta, db0.copy()), "bias gradient beside it")
+        assert torch.equal(ops.conv2d_bwd_filter_bias(xd, dyd, w_shape, st, pad, alpha=0.25, beta=1.0, dw=T(dw0, dev), db=T(db0, dev), algo=algo)[0], dw)
+
+
 # Backward-data of stride 2 to 4 by residue classes in the split-operand form: odd extents (classes of different sizes), classes
 # without taps (a filter smaller than the stride) and without pixels, an odd number of groups (8, 24, 40 filters), rows past the
 # 64-, 96- and 128-row tiles, one to many tiles a class, no padding and more than the filter needs.
