@@ -489,6 +489,12 @@ int rh_bnorm_fwd_train_add(int N, int C, int plane, float alpha, const float* x,
 int rh_bnorm_fwd_infer_add(int N, int C, int plane, float alpha, const float* x, float beta, const float* y0, float* y,
                            double epsilon, const float* scale, const float* bias, const float* running_mean,
                            const float* running_ivar, void* ws, size_t ws_bytes, int flags, rh_stream_t stream);
+/* rh_conv2d_fwd (alpha 1, beta 0) to `pre`, then rh_bnorm_fwd_infer_add from it: the same bits in both tensors.  Where the convolution's
+ * result comes out of a reduction of slices the batch norm is formed in it.  flags: the convolution's algorithm bits, RH_FUSE_RELU for
+ * the batch norm; ws: as large as the larger of the two calls asks for. */
+int rh_conv2d_fwd_bnorm_infer(const rh_conv_geom* g, const float* x, const float* w, float* pre, float beta, const float* y0, float* y,
+                              double epsilon, const float* scale, const float* bias, const float* running_mean,
+                              const float* running_ivar, void* ws, size_t ws_bytes, int flags, rh_stream_t stream);
 int rh_bnorm_bwd(int N, int C, int plane, float alpha_data, float beta_data, const float* x, const float* dy, float* dx,
                  float alpha_param, float beta_param, double epsilon, const float* scale, float* dscale, float* dbias,
                  const float* cached_mean, const float* cached_ivar, void* ws, size_t ws_bytes, rh_stream_t stream);

@@ -79,6 +79,7 @@ PROTOTYPES = {
     "rh_bnorm_fwd_train_add": (_int, [_int, _int, _int, _f, _vp, _f, _vp, _vp, C.c_double, C.c_double, _vp, _vp, _vp, _vp, _vp, _vp,
                                       _vp, _sz, _int, _vp]),
     "rh_bnorm_fwd_infer_add": (_int, [_int, _int, _int, _f, _vp, _f, _vp, _vp, C.c_double, _vp, _vp, _vp, _vp, _vp, _sz, _int, _vp]),
+    "rh_conv2d_fwd_bnorm_infer": (_int, [C.POINTER(ConvGeom), _vp, _vp, _vp, _f, _vp, _vp, C.c_double, _vp, _vp, _vp, _vp, _vp, _sz, _int, _vp]),
     "rh_bnorm_fwd_infer": (_int, [_int, _int, _int, _f, _vp, _f, _vp, C.c_double, _vp, _vp, _vp, _vp, _vp, _sz, _int, _vp]),
     "rh_bnorm_bwd": (_int, [_int, _int, _int, _f, _f, _vp, _vp, _vp, _f, _f, C.c_double, _vp, _vp, _vp, _vp, _vp, _vp, _sz,
                             _vp]),

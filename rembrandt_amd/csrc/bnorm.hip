@@ -46,7 +46,6 @@ __device__ __forceinline__ float wave_sum(float v) {
 // VEC (plane % 4 == 0, 16-byte aligned tensors): a lane reads 16 bytes at a time, two such loads in flight per operand.
 // MASK (MODE 1): dy counts only where the forward pass's ReLU let the value through, i.e. where
 // bn_affine(x, mean, scale*ivar, bias) > 0, recomputed here exactly as the forward pass computed it.
-__device__ __forceinline__ float bn_affine(float x, float mean, float si, float bias) { return fmaf(x - mean, si, bias); }
 
 struct BnMask { const float* scale; const float* ivar; const float* bias; };
 

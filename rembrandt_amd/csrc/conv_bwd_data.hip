@@ -174,7 +174,7 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
     if (!split.plan.ok) return RH_E_UNSUPPORTED;
     if (ws_bytes < split.plan.total()) return RH_E_WORKSPACE;
     if (d.x_elems == 0) return 0;
-    return (split.parts == 3 ? launch_conv_tri : launch_conv_duo)(split.plan, true, dy, w, dx, alpha, beta, nullptr, 0, mask, ws, stream);
+    return (split.parts == 3 ? launch_conv_tri : launch_conv_duo)(split.plan, true, dy, w, dx, alpha, beta, nullptr, 0, mask, ws, stream, nullptr);
   }
   if (!(flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET)) && conv1x1_stream_applies(d)) {
     if (d.x_elems == 0) return 0;

@@ -281,11 +281,22 @@ inline int plan_k_split(int rows, long long cols, int n_k, int bn_force = 0) {
   return want < 3 ? 1 : (int)want;   // two slices only trade one round of blocks for the partial-sum traffic
 }
 
+// A batch norm at inference behind a forward pass: y = relu?((x - mean[k]) scale[k] ivar[k] + bias[k] + beta old), by the expressions of
+// bn_infer_kernel.  A pass whose whole result comes out of the reduction of slices has it formed there and says so in `done`: the
+// result x is written as without it.
+struct BnInfer {
+  const float *mean, *ivar, *scale, *bias, *old;
+  float* y;
+  float alpha, beta;
+  int relu;
+};
+struct BnInferJob { BnInfer bn; bool done; };
+
 // out[i] = alpha * sum_s part[s*stride + i] + beta*out[i] (+ bias[channel], ReLU) over an NCHW tensor of `total`
 // elements, channel = (i / inner) % rows; only elements whose column (image * inner + pixel) is >= col0.
 void launch_split_reduce_nchw(const float* part, int splits, long long stride, float* out, long long total, int inner,
                               int rows, float alpha, float beta, const float* bias, int relu, hipStream_t stream,
-                              long long col0 = 0, const float* mask = nullptr);
+                              long long col0 = 0, const float* mask = nullptr, BnInferJob* bn = nullptr);
 
 
 // Slices that the direct form cuts the contraction of a forward / stride-1 backward-data call into.
@@ -592,7 +603,7 @@ inline TriPlan plan_tri_bwd_data(const ConvDims& d, int max_chain = 0) {
   return plan_tri(d.N, d.K, d.P, d.Q, d.C, d.R, d.S, 1, d.R - 1 - d.pad, d.H, d.W, max_chain);
 }
 int launch_conv_tri(const TriPlan& p, bool bwd, const float* in, const float* w, float* out, float alpha, float beta,
-                    const float* bias, int relu, const float* mask, void* ws, hipStream_t stream);
+                    const float* bias, int relu, const float* mask, void* ws, hipStream_t stream, BnInferJob* bn = nullptr);
 // The same with operands of two scaled fp16 parts (conv_duo.hip): scratch [group offsets, exponents, maxima][filter][image][partial sums].
 TriPlan plan_duo(int N, int Ci, int Hi, int Wi, int rows, int R, int S, int st, int halo, int P, int Q);
 inline TriPlan plan_duo_pass(const ConvDims& d, bool bwd) {
@@ -601,7 +612,7 @@ inline TriPlan plan_duo_pass(const ConvDims& d, bool bwd) {
   return plan_duo(d.N, d.K, d.P, d.Q, d.C, d.R, d.S, 1, d.R - 1 - d.pad, d.H, d.W);
 }
 int launch_conv_duo(const TriPlan& p, bool bwd, const float* in, const float* w, float* out, float alpha, float beta,
-                    const float* bias, int relu, const float* mask, void* ws, hipStream_t stream);
+                    const float* bias, int relu, const float* mask, void* ws, hipStream_t stream, BnInferJob* bn = nullptr);
 struct TriFilterPlan {
   int Hp, Wp, n8, groups_true, groups, bm, bn, splits;
   int sum_rows;   // rows of K partial sums of dy that the copy can leave for the bias gradient
@@ -778,7 +789,7 @@ SplitFilterPick pick_split_bwd_filter(const ConvDims& d, int flags, size_t ws_by
 
 int launch_conv_lds(const LdsConvPlan& pl, bool bwd, int N, int Ci, int H, int W, int rows, int P, int Q, int R, int halo,
                     const float* in, const float* w, float* out, float alpha, float beta, const float* bias, int relu,
-                    const float* mask, void* ws, hipStream_t stream);
+                    const float* mask, void* ws, hipStream_t stream, BnInferJob* bn = nullptr);
 
 // Forward with packed bf16 operands (RH_MATH_BF16_MFMA_FP32ACC, input channels a multiple of 8): the contraction runs
 // over k = (r, s, c) with c fastest, the image is copied once to bf16 as [n][hp][c/8][wp][8] with its zero border,

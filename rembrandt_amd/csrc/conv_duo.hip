@@ -342,7 +342,7 @@ TriPlan plan_duo(int N, int Ci, int Hi, int Wi, int rows, int R, int S, int st, 
 }
 
 int launch_conv_duo(const TriPlan& p, bool bwd, const float* in, const float* w, float* out, float alpha, float beta,
-                    const float* bias, int relu, const float* mask, void* ws, hipStream_t stream) {
+                    const float* bias, int relu, const float* mask, void* ws, hipStream_t stream, BnInferJob* bn) {
   char* base = static_cast<char*>(ws);
   int* soff = reinterpret_cast<int*>(base);
   int* exps_a = reinterpret_cast<int*>(base + align256(sizeof(int) * (size_t)p.groups));
@@ -414,7 +414,7 @@ int launch_conv_duo(const TriPlan& p, bool bwd, const float* in, const float* w,
   if (e) return e;
   if (p.splits > 1 || p.tail.splits > 1)
     launch_split_reduce_nchw(part, used, total - first, fin.out, total, fin.inner, fin.rows, fin.alpha, fin.beta, fin.bias, fin.relu,
-                             stream, p.splits > 1 ? 0 : p.tail.col0, fin.mask);
+                             stream, p.splits > 1 ? 0 : p.tail.col0, fin.mask, bn);
   return launch_status();
 }
 

@@ -197,14 +197,16 @@ void launch_pad_image_prep_soff(const float* src, float* dst, long long planes, 
                      H, W, FastDiv((uint32_t)Hp), FastDiv((uint32_t)Wp), halo, vec, pad_blocks, a, (unsigned)(planes * H * W));
 }
 
+// BN: the batch norm behind the pass as well (BnInfer; `first` and col0 are 0), its result to bn.y: a launch and a read of the result less.
+// ResNet-18 on 9 images, 13 of its 20 batch norms: 378 -> 371 us a pass with passes of other workers beside it.
 // VEC: four consecutive elements per thread through 16-byte loads and stores (slab stride, first element and all
 // pointers multiples of four floats); otherwise one element per thread.
-template <bool VEC>
+template <bool VEC, bool BN>
 __global__ __launch_bounds__(256) void split_reduce_nchw_kernel(const float* __restrict__ part, int splits, long long stride,
                                                                 float* __restrict__ out, unsigned first, unsigned total,
                                                                 FastDiv inner, FastDiv rows, float alpha, float beta,
                                                                 const float* __restrict__ bias, int relu,
-                                                                unsigned col0, const float* __restrict__ mask) {
+                                                                unsigned col0, const float* __restrict__ mask, BnInfer bn) {
   constexpr int E = VEC ? 4 : 1;
   const unsigned i0 = first + (blockIdx.x * blockDim.x + threadIdx.x) * (unsigned)E;
   if (i0 >= total) return;
@@ -237,8 +239,20 @@ __global__ __launch_bounds__(256) void split_reduce_nchw_kernel(const float* __r
       old[0] = out[i0];
     }
   }
-  float res[E];
+  float res[E], norm[E], add_to[E];
   bool keep[E];
+  if (BN) {
+#pragma unroll
+    for (int e = 0; e < E; ++e) add_to[e] = 0.0f;
+    if (bn.beta != 0.0f) {
+      if (VEC) {
+        const float4 o = *reinterpret_cast<const float4*>(bn.old + i0);
+        add_to[0] = o.x; add_to[E > 1 ? 1 : 0] = o.y; add_to[E > 2 ? 2 : 0] = o.z; add_to[E > 3 ? 3 : 0] = o.w;
+      } else {
+        add_to[0] = bn.old[i0];
+      }
+    }
+  }
 #pragma unroll
   for (int e = 0; e < E; ++e) {
     const unsigned i = i0 + e;
@@ -251,6 +265,17 @@ __global__ __launch_bounds__(256) void split_reduce_nchw_kernel(const float* __r
     if (relu) v = v > 0.0f ? v : 0.0f;
     if (mask && !(mask[i < total ? i : i0] > 0.0f)) v = 0.0f;
     res[e] = v;
+    if (BN) {   // (as bn_one)
+      const uint32_t c = plane - img * rows.div;
+      float u = bn_affine(v, bn.mean[c], bn.scale[c] * bn.ivar[c], bn.bias[c]);
+      u *= bn.alpha;
+      if (bn.beta != 0.0f) u = fmaf(bn.beta, add_to[e], u);
+      norm[e] = bn.relu ? (u > 0.0f ? u : 0.0f) : u;
+    }
+  }
+  if (BN) {
+    if (VEC) *reinterpret_cast<float4*>(bn.y + i0) = make_float4(norm[0], norm[E > 1 ? 1 : 0], norm[E > 2 ? 2 : 0], norm[E > 3 ? 3 : 0]);
+    else bn.y[i0] = norm[0];
   }
   if (VEC) {
     if (keep[0] && keep[E - 1]) {
@@ -265,20 +290,28 @@ __global__ __launch_bounds__(256) void split_reduce_nchw_kernel(const float* __r
 
 void launch_split_reduce_nchw(const float* part, int splits, long long stride, float* out, long long total, int inner,
                               int rows, float alpha, float beta, const float* bias, int relu, hipStream_t stream,
-                              long long col0, const float* mask) {
+                              long long col0, const float* mask, BnInferJob* bn) {
   // elements before the image that holds column col0 are not part of the reduction
   const long long first = col0 > 0 ? (col0 / inner) * (long long)rows * inner : 0;
   ProfScope prof("split_reduce", 4.0 * (double)(total - first) * (splits + 1), stream);
+  const bool norm = bn && col0 == 0;
+  const BnInfer b = norm ? bn->bn : BnInfer{};
   const bool vec = stride % 4 == 0 && first % 4 == 0 && total % 4 == 0 &&
-                   ((reinterpret_cast<uintptr_t>(part) | reinterpret_cast<uintptr_t>(out)) & 15) == 0;
-  if (vec)
-    hipLaunchKernelGGL((split_reduce_nchw_kernel<true>), dim3(stream_grid((size_t)(total - first) / 4, 256)), dim3(256), 0, stream,
-                       part, splits, stride, out, (unsigned)first, (unsigned)total, FastDiv((uint32_t)inner),
-                       FastDiv((uint32_t)rows), alpha, beta, bias, relu, (unsigned)col0, mask);
-  else
-    hipLaunchKernelGGL((split_reduce_nchw_kernel<false>), dim3(stream_grid((size_t)(total - first), 256)), dim3(256), 0, stream,
-                       part, splits, stride, out, (unsigned)first, (unsigned)total, FastDiv((uint32_t)inner),
-                       FastDiv((uint32_t)rows), alpha, beta, bias, relu, (unsigned)col0, mask);
+                   ((reinterpret_cast<uintptr_t>(part) | reinterpret_cast<uintptr_t>(out) | reinterpret_cast<uintptr_t>(b.y) |
+                     reinterpret_cast<uintptr_t>(b.old)) & 15) == 0;
+  auto go = [&](auto kernel, int width) {
+    hipLaunchKernelGGL(kernel, dim3(stream_grid((size_t)(total - first) / width, 256)), dim3(256), 0, stream, part, splits, stride, out,
+                       (unsigned)first, (unsigned)total, FastDiv((uint32_t)inner), FastDiv((uint32_t)rows), alpha, beta, bias, relu,
+                       (unsigned)col0, mask, b);
+  };
+  if (norm) {
+    if (vec) go(split_reduce_nchw_kernel<true, true>, 4);
+    else go(split_reduce_nchw_kernel<false, true>, 1);
+    bn->done = true;
+  } else {
+    if (vec) go(split_reduce_nchw_kernel<true, false>, 4);
+    else go(split_reduce_nchw_kernel<false, false>, 1);
+  }
 }
 
 // `splits` > 1: slices of the contraction write unblended partial results to `part`, then one reduction applies the
@@ -286,7 +319,7 @@ void launch_split_reduce_nchw(const float* part, int splits, long long stride, f
 template <class T>
 static int run_fwd_soff(const RowSParams& ap, const RowSParams& bp, EpiParams ep, int n_k, int k_true,
                         hipStream_t stream, const char* tag, int splits = 1, float* part = nullptr,
-                        const TailSplit* tail = nullptr) {
+                        const TailSplit* tail = nullptr, BnInferJob* bn = nullptr) {
   constexpr int AROWS = T::BM % 64 == 0 ? T::BM : (T::BM + 63) / 64 * 64;  // loader rows: a multiple of the wave
   // The transposed filter is read four rows per lane where the tile's shape allows (forward kernel 1-5 % faster alone).
   // The backward passes keep the one-row loader: there the same change made the two-stream step 0.2 ms slower,
@@ -315,7 +348,7 @@ static int run_fwd_soff(const RowSParams& ap, const RowSParams& bp, EpiParams ep
   int used = 1;
   if (int e = launch_mfma_gemm<T, AL, BL, true, PassConvFwd>(ap, bp, ep, n_k, splits, &used, stream, tag, k_true)) return e;
   launch_split_reduce_nchw(part, used, total, fin.out, total, fin.inner, fin.rows, fin.alpha, fin.beta, fin.bias, fin.relu,
-                           stream);
+                           stream, 0, nullptr, bn);
   return launch_status();
 }
 
@@ -627,9 +660,8 @@ extern "C" int32_t rh_conv2d_out_dim(int32_t in, int32_t size, int32_t stride, i
   return conv_out_dim(in, size, stride, pad);
 }
 
-extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x, const float* w,
-                             float beta, float* y, const float* bias, void* ws, size_t ws_bytes,
-                             int flags, rh_stream_t stream_) {
+static int conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x, const float* w, float beta, float* y, const float* bias,
+                      void* ws, size_t ws_bytes, int flags, rh_stream_t stream_, BnInferJob* bn) {
   ConvDims d;
   if (int e = conv_dims(g, &d)) return e;
   if (!x || !w || !y) return RH_E_INVALID;
@@ -647,7 +679,7 @@ extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x,
     if (!split.plan.ok) return RH_E_UNSUPPORTED;
     if (ws_bytes < split.plan.total()) return RH_E_WORKSPACE;
     return (split.parts == 3 ? launch_conv_tri : launch_conv_duo)(split.plan, false, x, w, y, alpha, beta, (flags & RH_FUSE_BIAS) ? bias : nullptr,
-                                                                (flags & RH_FUSE_RELU) ? 1 : 0, nullptr, ws, stream);
+                                                                (flags & RH_FUSE_RELU) ? 1 : 0, nullptr, ws, stream, bn);
   }
   if (!(flags & (RH_MATH_BF16_MFMA_FP32ACC | RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET)) && conv1x1_stream_applies(d))
     return launch_conv1x1_stream(d, RH_CONV_FWD, w, x, y, alpha, beta, (flags & RH_FUSE_BIAS) ? bias : nullptr,
@@ -666,7 +698,7 @@ extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x,
     }
     if (f.staged)
       return launch_conv_lds(f.lds, false, d.N, d.C, d.H, d.W, d.K, d.P, d.Q, d.R, d.pad, x, w, y, alpha, beta, bias_arg, relu_arg,
-                             nullptr, ws, stream);
+                             nullptr, ws, stream, bn);
   }
   const int CRS = d.C * d.R * d.S;
   if ((flags & RH_MATH_BF16_MFMA_FP32ACC) && !(flags & RH_ALGO_GATHER)) {
@@ -717,19 +749,19 @@ extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x,
     switch (pick_bm(d.K)) {
       case 128:
         // (sliced contractions on the half-width tile, as below: NIN's 6 x 6 layers 4-7 % faster)
-        if (sp.narrow128) return run_fwd_soff<T128x64>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_128x64", sp.splits, part, &sp.tail);
-        return run_fwd_soff<T128x128>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_128x128", sp.splits, part, &sp.tail);
-      case 96:  return run_fwd_soff<T96x128>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_96x128", sp.splits, part, &sp.tail);
+        if (sp.narrow128) return run_fwd_soff<T128x64>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_128x64", sp.splits, part, &sp.tail, bn);
+        return run_fwd_soff<T128x128>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_128x128", sp.splits, part, &sp.tail, bn);
+      case 96:  return run_fwd_soff<T96x128>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_96x128", sp.splits, part, &sp.tail, bn);
       case 64:
         if (cdiv(d.K, 64) == 1 && prefer_k8_64(ep.cols))
-          return run_fwd_soff<T64x256k8>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_64x256k8", sp.splits, part, &sp.tail);
+          return run_fwd_soff<T64x256k8>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_64x256k8", sp.splits, part, &sp.tail, bn);
         // a sliced contraction (a small layer) on the half-width tile: twice the blocks over the same slices, so that a
         // CU has others to run while one waits for its next K step's loads
-        if (sp.splits > 1) return run_fwd_soff<T64x128>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_64x128", sp.splits, part, &sp.tail);
-        return run_fwd_soff<T64x256>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_64x256", sp.splits, part, &sp.tail);
+        if (sp.splits > 1) return run_fwd_soff<T64x128>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_64x128", sp.splits, part, &sp.tail, bn);
+        return run_fwd_soff<T64x256>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_64x256", sp.splits, part, &sp.tail, bn);
       default:
-        if (sp.splits > 1) return run_fwd_soff<T32x128>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_32x128", sp.splits, part, &sp.tail);
-        return run_fwd_soff<T32x256>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_32x256", sp.splits, part, &sp.tail);
+        if (sp.splits > 1) return run_fwd_soff<T32x128>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_32x128", sp.splits, part, &sp.tail, bn);
+        return run_fwd_soff<T32x256>(ap, bp, ep, sp.n_k, CRS, stream, "conv_fwd_32x256", sp.splits, part, &sp.tail, bn);
     }
   }
   const int n_tab = round_up(CRS, kTabPad);
@@ -755,6 +787,28 @@ extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x,
     case 64:  return run_fwd<T64x256>(d, ap, bp, ep, stream, "conv_fwd_64x256");
     default:  return run_fwd<T32x256>(d, ap, bp, ep, stream, "conv_fwd_32x256");
   }
+}
+
+extern "C" int rh_conv2d_fwd(const rh_conv_geom* g, float alpha, const float* x, const float* w,
+                             float beta, float* y, const float* bias, void* ws, size_t ws_bytes,
+                             int flags, rh_stream_t stream) {
+  return conv2d_fwd(g, alpha, x, w, beta, y, bias, ws, ws_bytes, flags, stream, nullptr);
+}
+
+extern "C" int rh_conv2d_fwd_bnorm_infer(const rh_conv_geom* g, const float* x, const float* w, float* pre, float beta, const float* y0,
+                                         float* y, double epsilon, const float* scale, const float* bias, const float* running_mean,
+                                         const float* running_ivar, void* ws, size_t ws_bytes, int flags, rh_stream_t stream) {
+  ConvDims d;
+  if (int e = conv_dims(g, &d)) return e;
+  if (d.y_elems != 0 && (!y || !y0 || !scale || !bias || !running_mean || !running_ivar)) return RH_E_INVALID;
+  if ((flags & RH_FUSE_BIAS) || pre == y || (y0 == pre && beta != 0.0f)) return RH_E_INVALID;
+  const int norm_flags = flags & RH_FUSE_RELU;
+  if (d.y_elems != 0 && ws_bytes < rh_bnorm_workspace_bytes(d.N, d.K, d.P * d.Q)) return RH_E_WORKSPACE;
+  BnInferJob job = {{running_mean, running_ivar, scale, bias, y0, y, 1.0f, beta, norm_flags ? 1 : 0}, false};
+  if (int e = conv2d_fwd(g, 1.0f, x, w, 0.0f, pre, nullptr, ws, ws_bytes, flags & ~RH_FUSE_RELU, stream, &job)) return e;
+  if (job.done) return 0;
+  return rh_bnorm_fwd_infer_add(d.N, d.K, d.P * d.Q, 1.0f, pre, beta, y0, y, epsilon, scale, bias, running_mean, running_ivar, ws, ws_bytes,
+                                norm_flags, stream);
 }
 
 // ---------------------------------------------------------------------------------------------------------------

@@ -405,7 +405,7 @@ static int launch_lds_R(int shape, const LdsConvParams& p, const EpiParams& ep, 
 
 int launch_conv_lds(const LdsConvPlan& pl, bool bwd, int N, int Ci, int H, int W, int rows, int P, int Q, int R, int halo,
                     const float* in, const float* w, float* out, float alpha, float beta, const float* bias, int relu,
-                    const float* mask, void* ws, hipStream_t stream) {
+                    const float* mask, void* ws, hipStream_t stream, BnInferJob* bn) {
   LdsConvParams p;
   p.in = in; p.w = w;
   p.in_bytes = (uint32_t)(sizeof(float) * (size_t)N * Ci * H * W);
@@ -435,7 +435,7 @@ int launch_conv_lds(const LdsConvPlan& pl, bool bwd, int N, int Ci, int H, int W
   }
   if (pl.splits <= 1) return 0;
   launch_split_reduce_nchw(static_cast<float*>(ws), pl.splits, total, out, total, ep.inner, rows, alpha, beta, bias, relu, stream, 0,
-                           mask);
+                           mask, bn);
   return launch_status();
 }
 

@@ -289,7 +289,7 @@ TriPlan plan_tri(int N, int Ci, int Hi, int Wi, int rows, int R, int S, int st, 
 }
 
 int launch_conv_tri(const TriPlan& p, bool bwd, const float* in, const float* w, float* out, float alpha, float beta,
-                    const float* bias, int relu, const float* mask, void* ws, hipStream_t stream) {
+                    const float* bias, int relu, const float* mask, void* ws, hipStream_t stream, BnInferJob* bn) {
   char* base = static_cast<char*>(ws);
   int* soff = reinterpret_cast<int*>(base);
   uint4* wt = reinterpret_cast<uint4*>(base + p.tab_bytes);
@@ -344,7 +344,7 @@ int launch_conv_tri(const TriPlan& p, bool bwd, const float* in, const float* w,
   if (e) return e;
   if (p.splits > 1 || p.tail.splits > 1)
     launch_split_reduce_nchw(part, used, total - first, fin.out, total, fin.inner, fin.rows, fin.alpha, fin.beta, fin.bias, fin.relu,
-                             stream, p.splits > 1 ? 0 : p.tail.col0, fin.mask);
+                             stream, p.splits > 1 ? 0 : p.tail.col0, fin.mask, bn);
   return launch_status();
 }
 

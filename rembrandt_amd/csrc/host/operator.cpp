@@ -1341,19 +1341,19 @@ struct BNormConvUnit {
                double epsilon, bool relu, DeviceBuffer<uint8_t>& ws, bool bf16, const float* old = nullptr) {
     const rh_conv_geom g = geom(batch);
     if (!old) old = out;
-    unwrap(rh_conv2d_fwd(&g, 1.0f, in, weights->as_ptr(), 0.0f, pre_act->as_mut_ptr(), nullptr, ws.as_mut_ptr(), ws.len(),
-                         (bf16 ? RH_MATH_BF16_MFMA_FP32ACC : 0) | conv_algo, s()), "conv2d forward");
-    const int flags = relu ? RH_FUSE_RELU : 0;
+    const int algo = (bf16 ? RH_MATH_BF16_MFMA_FP32ACC : 0) | conv_algo, flags = relu ? RH_FUSE_RELU : 0;
     if (phase.training) {
+      unwrap(rh_conv2d_fwd(&g, 1.0f, in, weights->as_ptr(), 0.0f, pre_act->as_mut_ptr(), nullptr, ws.as_mut_ptr(), ws.len(), algo, s()),
+             "conv2d forward");
       if (!backward) panic("batch norm training missing backward operator");
       unwrap(rh_bnorm_fwd_train_add(g.N, g.K, plane(), 1.0f, pre_act->as_ptr(), beta_out, old, out, avg.at_iter(phase.t), epsilon,
                                     scale->as_ptr(), bias->as_ptr(), running_mean->as_mut_ptr(), running_ivar->as_mut_ptr(),
                                 cached_mean->as_mut_ptr(), cached_ivar->as_mut_ptr(), ws.as_mut_ptr(), ws.len(), flags, s()),
              "batch norm forward training");
     } else {
-      unwrap(rh_bnorm_fwd_infer_add(g.N, g.K, plane(), 1.0f, pre_act->as_ptr(), beta_out, old, out, epsilon, scale->as_ptr(),
-                                bias->as_ptr(), running_mean->as_ptr(), running_ivar->as_ptr(), ws.as_mut_ptr(), ws.len(),
-                                flags, s()), "batch norm forward inference");
+      unwrap(rh_conv2d_fwd_bnorm_infer(&g, in, weights->as_ptr(), pre_act->as_mut_ptr(), beta_out, old, out, epsilon, scale->as_ptr(),
+                                       bias->as_ptr(), running_mean->as_ptr(), running_ivar->as_ptr(), ws.as_mut_ptr(), ws.len(),
+                                       algo | flags, s()), "conv2d and batch norm forward inference");
     }
   }
   // pre_delta = dBN(out_delta) with the scale / bias gradients accumulated, then grad_weights += dconv(in, pre_delta).

@@ -551,6 +551,19 @@ def bnorm_fwd_infer(x, scale, bias, running_mean, running_ivar, epsilon, alpha=1
     return y
 
 
+def conv2d_fwd_bnorm_infer(x, w, stride, pad, scale, bias, running_mean, running_ivar, epsilon, beta=0.0, y0=None, relu=False, algo=0):
+    """Returns (the convolution's result, the batch norm's): conv2d_fwd, then bnorm_fwd_infer (rh_conv2d_fwd_bnorm_infer)."""
+    g = conv_geom(x.shape, w.shape, stride, pad)
+    shape = conv_out_shape(g)
+    pre, y = (torch.empty(shape, dtype=torch.float32, device=x.device) for _ in range(2))
+    need = max(conv_ws_bytes(g, _lib.RH_CONV_FWD, algo), lib().rh_bnorm_workspace_bytes(g.N, g.K, shape[2] * shape[3]))
+    ws = workspace(need, x.device)
+    check(lib().rh_conv2d_fwd_bnorm_infer(C.byref(g), _p(x), _p(w), _p(pre), beta, _p(y if y0 is None else y0), _p(y), epsilon, _p(scale),
+                                          _p(bias), _p(running_mean), _p(running_ivar), _p(ws), ws.numel(),
+                                          algo | (_lib.RH_FUSE_RELU if relu else 0), _stream()), "rh_conv2d_fwd_bnorm_infer")
+    return pre, y
+
+
 def bnorm_bwd(x, dy, scale, cached_mean, cached_ivar, epsilon, dscale=None, dbias=None, alpha_data=1.0, beta_data=0.0,
               dx=None, alpha_param=1.0, beta_param=0.0, relu_bias=None):
     """Returns (dx, dscale, dbias); with beta_param = 1 the parameter gradients accumulate as in the reference.

@@ -249,6 +249,10 @@ extern "C" {
                                 y0: *const f32, y: *mut f32, epsilon: f64, scale: *const f32, bias: *const f32,
                                 running_mean: *const f32, running_ivar: *const f32, ws: *mut c_void,
                                 ws_bytes: size_t, flags: c_int, stream: rh_stream_t) -> c_int;
+  pub fn rh_conv2d_fwd_bnorm_infer(g: *const rh_conv_geom, x: *const f32, w: *const f32, pre: *mut f32, beta: c_float,
+                                   y0: *const f32, y: *mut f32, epsilon: f64, scale: *const f32, bias: *const f32,
+                                   running_mean: *const f32, running_ivar: *const f32, ws: *mut c_void,
+                                   ws_bytes: size_t, flags: c_int, stream: rh_stream_t) -> c_int;
   pub fn rh_bnorm_bwd(n: c_int, c: c_int, plane: c_int, alpha_data: c_float, beta_data: c_float, x: *const f32,
                       dy: *const f32, dx: *mut f32, alpha_param: c_float, beta_param: c_float, epsilon: f64,
                       scale: *const f32, dscale: *mut f32, dbias: *mut f32, cached_mean: *const f32,

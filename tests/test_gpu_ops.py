@@ -2019,6 +2019,33 @@ def test_residual_sum_and_its_gradient(dev, shape):
         assert torch.equal(one, two) and torch.equal(copy, two)
 
 
+# A batch norm behind a forward pass at inference: whole results and a sliced tail (the batch norm in a launch of its own), contractions in
+# slices of each form (split operands, the engine, staged), planes and channels that are no multiple of four.
+@pytest.mark.parametrize("case", [(9, 64, 56, 56, 64, 3, 1, 1), (9, 128, 28, 28, 128, 3, 1, 1), (9, 512, 7, 7, 512, 3, 1, 1), (9, 256, 14, 14, 512, 1, 2, 0),
+                                  (5, 256, 13, 11, 70, 3, 2, 1), (1, 24, 5, 7, 40, 3, 1, 1), (33, 96, 27, 27, 250, 5, 1, 2), (2, 3, 30, 30, 33, 7, 2, 3),
+                                  (60, 256, 14, 14, 256, 3, 1, 1)], ids=str)
+def test_conv2d_fwd_bnorm_infer(dev, case):
+    """rh_conv2d_fwd_bnorm_infer against the two calls that it stands for: the same bits in both results."""
+    Nn, C, H, W, K, R, st, pad = case
+    say("conv bnorm infer case", case)
+    x, w = T(synth.normal(73, 1, (Nn, C, H, W)), dev), T(synth.normal(73, 2, (K, C, R, R)), dev)
+    scale, bias, mean = (T(synth.normal(73, 3 + i, (K,)), dev) for i in range(3))
+    ivar = T(np.abs(synth.normal(73, 6, (K,))) + 0.1, dev)
+    fused = set()
+    for algo in (0, _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_F16X2, _lib.RH_ALGO_DIRECT, _lib.RH_ALGO_SCALAR_OFFSET):
+        pre = ops.conv2d_fwd(x, w, st, pad, algo=algo)
+        y0 = T(synth.normal(73, 7, tuple(pre.shape)), dev)
+        for beta, old, relu in ((0.0, None, True), (1.0, y0, True), (0.5, y0, False)):
+            want = ops.bnorm_fwd_infer(pre, scale, bias, mean, ivar, 1e-5, beta=beta, y0=old, relu=relu)
+            (got_pre, got), tags = profile_tags(lambda: ops.conv2d_fwd_bnorm_infer(x, w, st, pad, scale, bias, mean, ivar, 1e-5, beta=beta,
+                                                                                  y0=old, relu=relu, algo=algo))
+            assert torch.equal(got_pre, pre) and torch.equal(got, want), (algo, beta, relu)
+            fused.add("bnorm_fwd_apply" not in tags)
+    if case[:2] in ((9, 128), (9, 512)):
+        assert True in fused, "the batch norm in the reduction of slices"
+
+
+
 @pytest.mark.parametrize("case", [(2, 3, 9, 3, 2, 0), (2, 3, 9, 3, 2, 1), (3, 4, 8, 2, 2, 0), (2, 5, 27, 3, 2, 0), (2, 2, 13, 3, 3, 1)])
 @pytest.mark.parametrize("rounding", [_lib.RH_ROUND_FLOOR, _lib.RH_ROUND_CEIL])
 def test_pool2d_bwd_with_folded_relu_mask(dev, case, rounding):
