@@ -386,8 +386,8 @@ struct PoolColors {
   FastDiv dCnt[4], dQb[2];
 };
 
-template <int J, class MT>
-__global__ __launch_bounds__(256) void pool_bwd_mask_color_kernel(PoolDims d, PoolColors pc, int PB, long long planes,
+template <int J, int NT, class MT>
+__global__ __launch_bounds__(NT) void pool_bwd_mask_color_kernel(PoolDims d, PoolColors pc, int PB, long long planes,
                                                                   const float* __restrict__ dy, const MT* __restrict__ argmax,
                                                                   const float* __restrict__ y, float* __restrict__ dx) {
   extern __shared__ float lds_pool[];
@@ -415,7 +415,7 @@ __global__ __launch_bounds__(256) void pool_bwd_mask_color_kernel(PoolDims d, Po
       const int n_c = np * pc.cnt[c];
 #pragma unroll
       for (int j = 0; j < J; ++j) {
-        const int t = (int)threadIdx.x + 256 * j;
+        const int t = (int)threadIdx.x + NT * j;
         if (t < n_c) {
           uint32_t pl, rem, i, jj;
           pc.dCnt[c].divmod((uint32_t)t, pl, rem);
@@ -433,7 +433,7 @@ __global__ __launch_bounds__(256) void pool_bwd_mask_color_kernel(PoolDims d, Po
   {
     float4* z4 = reinterpret_cast<float4*>(lds_pool);
     const int nz = (n_in + 4 + 3) >> 2;
-    for (int i = threadIdx.x; i < nz; i += 256) z4[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+    for (int i = threadIdx.x; i < nz; i += NT) z4[i] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
   }
   __syncthreads();
 #pragma unroll
@@ -450,8 +450,8 @@ __global__ __launch_bounds__(256) void pool_bwd_mask_color_kernel(PoolDims d, Po
   const int n4 = (n_in - head) >> 2;
   float4* g4 = reinterpret_cast<float4*>(gdx + head);
   const float4* s4 = reinterpret_cast<const float4*>(sdx + head);
-  for (int g = threadIdx.x; g < n4; g += 256) g4[g] = s4[g];
-  for (int e = head + (n4 << 2) + threadIdx.x; e < n_in; e += 256) gdx[e] = sdx[e];
+  for (int g = threadIdx.x; g < n4; g += NT) g4[g] = s4[g];
+  for (int e = head + (n4 << 2) + threadIdx.x; e < n_in; e += NT) gdx[e] = sdx[e];
 }
 
 // Launches one instantiation of the LDS forward; RH_E_UNSUPPORTED when the block's LDS cannot be had.
@@ -574,16 +574,16 @@ static bool lds_bwd_ok(const PoolDims& d) { return d.P * d.Q <= 4096 && d.H * d.
 
 // The colour form: one or two colours per axis, a plane's dx within 60 KB of LDS, at most 8 windows per thread and
 // colour.  Returns RH_E_UNSUPPORTED when the geometry is outside that.
-template <int J, class MT>
+template <int J, int NT, class MT>
 static int launch_pool_bwd_color_j(const PoolDims& d, const PoolColors& pc, int PB, long long planes, long long blocks,
                                    size_t lds_bytes, const float* dy, const MT* argmax, const float* relu_y, float* dx,
                                    rh_stream_t stream) {
   if (lds_bytes > 48 * 1024) {
-    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&pool_bwd_mask_color_kernel<J, MT>),
+    static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&pool_bwd_mask_color_kernel<J, NT, MT>),
                                                        hipFuncAttributeMaxDynamicSharedMemorySize, 64 * 1024);
     if (attr != hipSuccess) return RH_E_UNSUPPORTED;
   }
-  hipLaunchKernelGGL((pool_bwd_mask_color_kernel<J, MT>), dim3((unsigned)blocks), dim3(256), lds_bytes, to_stream(stream), d, pc, PB,
+  hipLaunchKernelGGL((pool_bwd_mask_color_kernel<J, NT, MT>), dim3((unsigned)blocks), dim3(NT), lds_bytes, to_stream(stream), d, pc, PB,
                      planes, dy, argmax, relu_y, dx);
   return launch_status();
 }
@@ -625,10 +625,12 @@ static int launch_pool_bwd_color(const PoolDims& d, const float* dy, const MT* a
   if (blocks >= (1ll << 31)) return RH_E_LIMIT;
   const size_t lds_bytes = ((size_t)PB * HW + 8) * sizeof(float);
   if (dry_run) return 0;
-  if (per_thread <= 1) return launch_pool_bwd_color_j<1, MT>(d, pc, PB, planes, blocks, lds_bytes, dy, argmax, relu_y, dx, stream);
-  if (per_thread <= 2) return launch_pool_bwd_color_j<2, MT>(d, pc, PB, planes, blocks, lds_bytes, dy, argmax, relu_y, dx, stream);
-  if (per_thread <= 4) return launch_pool_bwd_color_j<4, MT>(d, pc, PB, planes, blocks, lds_bytes, dy, argmax, relu_y, dx, stream);
-  return launch_pool_bwd_color_j<8, MT>(d, pc, PB, planes, blocks, lds_bytes, dy, argmax, relu_y, dx, stream);
+  if (per_thread <= 1) return launch_pool_bwd_color_j<1, 256, MT>(d, pc, PB, planes, blocks, lds_bytes, dy, argmax, relu_y, dx, stream);
+  if (per_thread <= 2) return launch_pool_bwd_color_j<2, 256, MT>(d, pc, PB, planes, blocks, lds_bytes, dy, argmax, relu_y, dx, stream);
+  // (such a plane has 8 to 60 KB of dx in LDS: with 512 threads the CU's few blocks have twice the loads in flight.  256 x 64 x 112 x 112
+  // 3x3 stride 2: 348 us with 256 threads, 289 with 512, 280 with 1024; 9 images 13.2, 10.7 and 12.0)
+  if (per_thread <= 4) return launch_pool_bwd_color_j<2, 512, MT>(d, pc, PB, planes, blocks, lds_bytes, dy, argmax, relu_y, dx, stream);
+  return launch_pool_bwd_color_j<4, 512, MT>(d, pc, PB, planes, blocks, lds_bytes, dy, argmax, relu_y, dx, stream);
 }
 
 static int launch_pool_bwd_lds(const PoolDims& d, const float* dy, const int32_t* argmax, const float* relu_y, float* dx,
