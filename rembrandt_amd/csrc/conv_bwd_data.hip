@@ -48,6 +48,9 @@ struct PhaseTable {
   int u0[kMaxPhaseStride * kMaxPhaseStride], U[kMaxPhaseStride * kMaxPhaseStride];
   int v0[kMaxPhaseStride * kMaxPhaseStride], V[kMaxPhaseStride * kMaxPhaseStride];
   long long off[kMaxPhaseStride * kMaxPhaseStride];  // < 0: no taps
+  int slices[kMaxPhaseStride * kMaxPhaseStride];     // whose sum a result is, `slab` floats apart
+  long long slab;
+  bool sliced;   // any class
 };
 __global__ __launch_bounds__(256) void phase_interleave_kernel(const float* __restrict__ sub, float* __restrict__ dx,
                                                                unsigned total, FastDiv dW, FastDiv dH, FastDiv dSt, int st,
@@ -55,13 +58,14 @@ __global__ __launch_bounds__(256) void phase_interleave_kernel(const float* __re
   // per class: {offset of its result minus the offset of its first pixel, row length V, plane size U*V}; the table is
   // indexed per element, so it lives in LDS rather than in the kernel arguments
   __shared__ long long s_base[kMaxPhaseStride * kMaxPhaseStride];
-  __shared__ int s_V[kMaxPhaseStride * kMaxPhaseStride], s_UV[kMaxPhaseStride * kMaxPhaseStride];
+  __shared__ int s_V[kMaxPhaseStride * kMaxPhaseStride], s_UV[kMaxPhaseStride * kMaxPhaseStride], s_S[kMaxPhaseStride * kMaxPhaseStride];
   if (threadIdx.x < kMaxPhaseStride * kMaxPhaseStride) {
     const int i = threadIdx.x;
     const bool live = i < st * st && t.off[i] >= 0;
     s_base[i] = live ? t.off[i] - ((long long)t.u0[i] * t.V[i] + t.v0[i]) : -1;
     s_V[i] = live ? t.V[i] : 0;
     s_UV[i] = live ? t.U[i] * t.V[i] : 0;
+    s_S[i] = live ? t.slices[i] : 0;
   }
   __syncthreads();
   // four consecutive elements of dx per thread, one 16-byte store (and load, when blending) if dx is aligned
@@ -91,7 +95,12 @@ __global__ __launch_bounds__(256) void phase_interleave_kernel(const float* __re
     const int ph = (int)(a * st + b);
     const int V = s_V[ph];
     float x = 0.0f;
-    if (V > 0 && i0 + e < total) x = sub[s_base[ph] + (long long)plane * s_UV[ph] + (long long)u * V + v];
+    if (V > 0 && i0 + e < total) {
+      const float* const p = sub + s_base[ph] + (long long)plane * s_UV[ph] + (long long)u * V + v;
+      x = p[0];
+      if (t.sliced)
+        for (int s = 1; s < s_S[ph]; ++s) x += p[s * t.slab];
+    }
     x *= alpha;
     if (beta != 0.0f) x = fmaf(beta, old[e], x);
     val[e] = x;
@@ -201,9 +210,12 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
     if (mask) return RH_E_UNSUPPORTED;
     if (d.x_elems == 0) return 0;
     PhaseTable tab;
+    tab.slab = (long long)(pp.sub_bytes / sizeof(float));
+    tab.sliced = false;
     for (int i = 0; i < d.st * d.st; ++i) {
       const PhaseGeom& g = pp.ph[i];
       tab.u0[i] = g.u0; tab.U[i] = g.U; tab.v0[i] = g.v0; tab.V[i] = g.V;
+      tab.slices[i] = 1;
       tab.off[i] = g.Ra > 0 && g.Sb > 0 && g.U > 0 && g.V > 0 ? g.sub_off : -1;
     }
     auto interleave = [&](const float* sub) -> int {
@@ -216,6 +228,8 @@ static int bwd_data_impl(const rh_conv_geom* g, float alpha, const float* w, con
     if (tri_allowed(flags)) {
       const TriPhasePlan tp = plan_tri_phases(d, pp);
       if (tp.ok && ws_bytes >= tp.total()) {
+        tab.sliced = tp.most > 1;
+        for (int i = 0; i < d.st * d.st; ++i) tab.slices[i] = tp.slices[i];
         float* sub;
         const int e = launch_conv_tri_phases(d, pp, tp, w, dy, ws, stream, &sub);
         return e ? e : interleave(sub);

@@ -906,42 +906,74 @@ inline PhasePlan plan_phase_bwd_data(const ConvDims& d) {
 struct TriPhasePlan {
   bool ok;
   int bm, groups;   // groups of eight k of all classes, each a whole number of K steps
+  int slices[kMaxPhaseStride * kMaxPhaseStride], most;   // of a class's contraction; the largest count: slabs of all classes' results
   size_t tab_bytes, wt_bytes, img_bytes, sub_bytes;
   size_t total() const { return tab_bytes + wt_bytes + img_bytes + sub_bytes; }
 };
 // The other form is a preparation, a product and mostly a reduction for each class, about 10 us and its multiply-adds at 100 TFLOP/s;
 // this one copies once and launches once, so it gains most on few pixels.  3x3, stride 2, us: 64 -> 128 56x56 at 8, 24, 64, 128,
 // 256 images 93 -> 39, 124 -> 50, 176 -> 99, 274 -> 181, 521 -> 355; 128 -> 256 28x28 at 64, 128, 256 images 176 -> 78, 272 -> 121,
-// 405 -> 230; 256 -> 512 14x14 at 256 403 -> 194.  Below those batches the other form's many slices have the smaller error.
+// 405 -> 230; 256 -> 512 14x14 at 256 403 -> 194.
+// Below those batches the other form's slices had the smaller error, so here the long classes go in slices too, as many as the error asks
+// for or the time: the pass that interleaves the classes adds them up.  128 -> 256 28x28 at 1, 8, 24, 36 images 83 -> 33, 88 -> 39, 125 -> 50,
+// 134 -> 58, 256 -> 512 14x14 at 8, 24, 64, 128 94 -> 40, 129 -> 50, 184 -> 79, 253 -> 113, 96 -> 64 5x5 27x27 at 8 and 64 75 -> 32, 133 -> 56;
+// 44 layers and batches have 0.45 to 0.83 of the other form's error against 64 bits.
 inline TriPhasePlan plan_tri_phases(const ConvDims& d, const PhasePlan& pp) {
   TriPhasePlan p = {};
   if (!pp.ok || d.K % 8 != 0 || d.x_elems == 0 || d.R * d.S == 1) return p;
   p.bm = pick_bm(d.C);
   if (p.bm == 32) return p;
   const int bn = p.bm == 64 ? 192 : 128;
-  double other = 30.0, us = 20.0, steps_all = 0.0, longest = 0.0;
+  double other = 30.0;
+  int steps[kMaxPhaseStride * kMaxPhaseStride] = {}, least[kMaxPhaseStride * kMaxPhaseStride] = {}, longest = 0;
   for (int i = 0; i < d.st * d.st; ++i) {
     const PhaseGeom& g = pp.ph[i];
     const long long cols = (long long)d.N * g.U * g.V;
     if (g.Ra * g.Sb == 0 || cols == 0) continue;
     const int k_true = d.K * g.Ra * g.Sb, n = round_up(k_true / 8, 2) / 2;
     // (the engine's slices, and a rounding for each slice added to those before)
-    if (n > tri_max_chain(0.0335 * k_true / g.splits + (g.splits > 1 ? 0.016 * g.splits : 0.0))) return p;
+    const double err = 0.0335 * k_true / g.splits + (g.splits > 1 ? 0.016 * g.splits : 0.0);
+    int S = 1;
+    while (S <= 8 && cdiv(n, S) > tri_max_chain(err - (S > 1 ? 0.021 * S : 0.0))) ++S;
+    if (S > 8) return p;
+    steps[i] = n; least[i] = S;
     p.groups += 2 * n;
-    steps_all += (double)n * cdiv(d.C, p.bm) * (double)cdiv<long long>(cols, bn);
     if (n > longest) longest = n;
     other += 10.0 + 2.0 * (double)d.C * (double)cols * k_true / 100e6;
   }
   const size_t img = 6 * (size_t)d.N * d.K * pp.Hp * pp.Wp, wt = 48 * (size_t)p.groups * d.C;
   if (p.groups == 0 || img > kMaxBufferBytes || wt > kMaxBufferBytes) return p;
   const double step_us = p.bm == 128 ? 0.456 : 0.377;
-  us += fmax(longest * step_us, steps_all / 256.0 * step_us) + (4.0 * (double)d.y_elems + (double)img) / 5.3e6 + 12.0 * (double)d.x_elems / 5.3e6 +
+  double run = 1e30;
+  for (int want = 1; want <= 8; ++want) {
+    const int cap = cdiv(longest, want);
+    double all = 0.0, slabs = 0.0;
+    int chain = 0, most = 1, slices[kMaxPhaseStride * kMaxPhaseStride] = {};
+    for (int i = 0; i < d.st * d.st; ++i) {
+      if (steps[i] == 0) continue;
+      const int S = max(least[i], cdiv(steps[i], cap)), n = cdiv(steps[i], S);
+      const long long cols = (long long)d.N * pp.ph[i].U * pp.ph[i].V;
+      slices[i] = cdiv(steps[i], n);
+      all += (double)steps[i] * cdiv(d.C, p.bm) * (double)cdiv<long long>(cols, bn);
+      slabs += 8.0 * (slices[i] - 1) * (double)d.C * (double)cols / 3e6;
+      chain = max(chain, n);
+      most = max(most, slices[i]);
+    }
+    if (most > 8) continue;
+    const double t = fmax(chain * step_us, all / 256.0 * step_us) + slabs;
+    if (t >= 0.95 * run) continue;
+    run = t;
+    p.most = most;
+    for (int i = 0; i < d.st * d.st; ++i) p.slices[i] = slices[i];
+  }
+  const double us = 20.0 + run + (4.0 * (double)d.y_elems + (double)img) / 5.3e6 + 12.0 * (double)d.x_elems / 5.3e6 +
         10.0 * (double)d.w_elems / 2.2e6;
   if (us >= other) return p;
   p.tab_bytes = align256(sizeof(int) * (size_t)p.groups);
   p.wt_bytes = align256(wt);
   p.img_bytes = align256(img);
-  p.sub_bytes = pp.sub_bytes;
+  p.sub_bytes = pp.sub_bytes * (size_t)p.most;
+  if (p.sub_bytes > kMaxBufferBytes) return p;
   p.ok = true;
   return p;
 }

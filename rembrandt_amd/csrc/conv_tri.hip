@@ -368,7 +368,7 @@ int launch_conv_tri_phases(const ConvDims& d, const PhasePlan& pp, const TriPhas
   TriClassFilterArgs f;
   TriClasses t;
   f.w = w; f.wt = wt; f.soff = soff; f.groups = p.groups; f.C = d.C; f.K = d.K; f.R = d.R; f.S = d.S; f.st = d.st; f.Wp = pp.Wp; f.count = count;
-  t.count = count; t.tiles_m = cdiv(d.C, tm);
+  t.count = count; t.tiles_m = cdiv(d.C, tm); t.slab = (long long)(pp.sub_bytes / sizeof(float));
   int groups = 0, tiles = 0;
   double flops = 0.0;
   for (int q = 0; q < count; ++q) {
@@ -384,7 +384,9 @@ int launch_conv_tri_phases(const ConvDims& d, const PhasePlan& pp, const TriPhas
     k.soff_at = groups;
     k.out_at = g.sub_off;
     groups += c.groups;
-    tiles += t.tiles_m * cdiv(k.cols, tn);
+    k.tiles = t.tiles_m * cdiv(k.cols, tn);
+    k.slice_steps = cdiv(k.steps, p.slices[order[q]]);
+    tiles += k.tiles * cdiv(k.steps, k.slice_steps);
     flops += 12.0 * (double)d.C * k.cols * d.K * g.Ra * g.Sb;
   }
   if (groups != p.groups) return RH_E_INVALID;

@@ -456,12 +456,13 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_kernel(TriParams 
 // the MFMAs as above and by the classes' results, which a second pass interleaves.
 struct TriClass {
   int first_tile, steps, groups_true;
+  int tiles, slice_steps;    // of a slice: its tiles, and K steps at most
   int cols, inner, innerW;   // n U V, U V, V
   uint32_t wt_at, img_at;    // bytes into the operand copies: the class's filter, its first pixel at its first tap
   int soff_at;
   long long out_at;          // floats
 };
-struct TriClasses { int count, tiles_m; TriClass c[16]; };
+struct TriClasses { int count, tiles_m; long long slab; TriClass c[16]; };   // slab: floats from a slice's results to the next's
 template <class T>
 __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_classes_kernel(TriParams ap, TriParams bp, EpiParams ep, TriClasses t) {
   const int block = blockIdx.x;
@@ -469,8 +470,10 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_classes_kernel(Tr
   while (i + 1 < t.count && block >= t.c[i + 1].first_tile) ++i;
   i = __builtin_amdgcn_readfirstlane(i);
   const TriClass c = t.c[i];
-  const int tiles = (i + 1 < t.count ? t.c[i + 1].first_tile : (int)gridDim.x) - c.first_tile;
-  const int logical = __builtin_amdgcn_readfirstlane(xcd_remap(block - c.first_tile, tiles));
+  const int blocks = (i + 1 < t.count ? t.c[i + 1].first_tile : (int)gridDim.x) - c.first_tile;
+  const int linear = __builtin_amdgcn_readfirstlane(xcd_remap(block - c.first_tile, blocks));
+  const int slice = linear / c.tiles, logical = linear - slice * c.tiles;
+  const int s0 = slice * c.slice_steps, s1 = s0 + c.slice_steps < c.steps ? s0 + c.slice_steps : c.steps;
   ap.v.ptr = static_cast<const char*>(ap.v.ptr) + c.wt_at;
   ap.plane = c.steps * 2 * ap.v.M * 16;
   ap.v.bytes = (uint32_t)(3 * ap.plane);
@@ -478,9 +481,9 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_classes_kernel(Tr
   bp.v.bytes -= c.img_at;
   bp.v.M = c.cols; bp.v.inner = c.inner; bp.v.innerW = c.innerW;
   bp.v.soff += c.soff_at;
-  ep.out += c.out_at;
+  ep.out += c.out_at + slice * t.slab;
   ep.cols = c.cols; ep.inner = c.inner;
-  tri_block<T, false, true, false>(ap, bp, ep, logical % t.tiles_m * T::BM, logical / t.tiles_m * T::BN, 0, c.steps, c.groups_true, -1);
+  tri_block<T, false, true, false>(ap, bp, ep, logical % t.tiles_m * T::BM, logical / t.tiles_m * T::BN, s0, s1, c.groups_true, -1);
 }
 
 }  // namespace rh

@@ -625,6 +625,9 @@ X3_STRIDED_CASES = [
     (9, 250, 14, 15, 72, 5, 4, 1),
     (4, 64, 8, 8, 64, 3, 2, 3),
     (24, 64, 56, 56, 128, 3, 2, 1),
+    (2, 256, 14, 13, 512, 3, 2, 1),      # the long classes in slices, of unequal numbers
+    (1, 128, 9, 11, 200, 5, 3, 2),
+    (8, 64, 28, 28, 264, 4, 2, 1),
 ]
 
 
