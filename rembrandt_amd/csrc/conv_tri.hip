@@ -183,6 +183,29 @@ __device__ __forceinline__ void tri_batch_body(const TriBatchArgs& a, int b, flo
   }
 }
 
+// The same for x of a first layer, up to kTriFew channels, where 29 of the 32 channels above would be none: a thread a pixel, all its
+// channels and images, past LDS.  Bound by its bytes.  Copies of both operands, 3 channels, us: 96 filters 11x11 stride 4 at 50 and 256 images 80 -> 51
+// and 343 -> 238, 64 filters 7x7 stride 2 at 24 and 256 50 -> 41 and 608 -> 487.
+constexpr int kTriFew = 4, kTriFewPix = 256;
+__device__ __forceinline__ void tri_few_body(const TriBatchArgs& a, int b) {
+  const int bx = b % a.px, bz = b / a.px, pix = bx * kTriFewPix + (int)threadIdx.x, n0 = bz * 8;
+  if (pix >= a.HpWp) return;
+  uint32_t hp, wp;
+  a.dWp.divmod((uint32_t)pix, hp, wp);
+  const int h = (int)hp - a.halo, w = (int)wp - a.halo;
+  const bool in = (unsigned)h < (unsigned)a.H && (unsigned)w < (unsigned)a.W;
+  const size_t hw = (size_t)a.H * a.W;
+  const float* const src = a.x + (size_t)(in ? h * a.W + w : 0);
+  float v[kTriFew][8];
+#pragma unroll
+  for (int c = 0; c < kTriFew; ++c)
+#pragma unroll
+    for (int n = 0; n < 8; ++n) v[c][n] = in && c < a.C && n0 + n < a.N ? src[((size_t)(n0 + n) * a.C + c) * hw] : 0.0f;
+#pragma unroll
+  for (int c = 0; c < kTriFew; ++c)
+    if (c < a.C) tri_store(a.xt, ((size_t)bz * a.HpWp + pix) * a.C + c, a.plane, v[c], false);
+}
+
 // Both operands of a filter gradient and soff[g], the place of group g = (n/8, p, q) in x's copy; the groups past the last
 // are zeros of dy.
 __global__ __launch_bounds__(256) void tri_batch_kernel(TriBatchArgs dy, TriBatchArgs x, int* __restrict__ soff, int groups,
@@ -191,7 +214,11 @@ __global__ __launch_bounds__(256) void tri_batch_kernel(TriBatchArgs dy, TriBatc
   int b = blockIdx.x;
   if (b < dy.blocks) { tri_batch_body(dy, xcd_remap(b, dy.blocks), tile); return; }
   b -= dy.blocks;
-  if (b < x.blocks) { tri_batch_body(x, xcd_remap(b, x.blocks), tile); return; }
+  if (b < x.blocks) {
+    if (x.C <= kTriFew) tri_few_body(x, xcd_remap(b, x.blocks));
+    else tri_batch_body(x, xcd_remap(b, x.blocks), tile);
+    return;
+  }
   b -= x.blocks;
   if (groups > groups_true)   // (one group: every block of the table writes a share)
     for (int i = b * 256 + threadIdx.x; i < 3 * dy.C; i += (int)(gridDim.x - dy.blocks - x.blocks) * 256)
@@ -481,7 +508,7 @@ int launch_conv_tri_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const 
     a.x = dy; a.xt = dyt; a.N = d.N; a.C = d.K; a.H = d.P; a.W = d.Q; a.halo = 0; a.HpWp = d.P * d.Q; a.dWp = FastDiv((uint32_t)d.Q);
     a.plane = dy_plane; a.px = cdiv(a.HpWp, kTriPix); a.cx = cdiv(a.C, kTriCh); a.blocks = a.px * a.cx * p.n8; a.sums = sums; a.wide = p.wide;
     b.x = x; b.xt = xt; b.N = d.N; b.C = d.C; b.H = d.H; b.W = d.W; b.halo = d.pad; b.HpWp = p.Hp * p.Wp; b.dWp = FastDiv((uint32_t)p.Wp);
-    b.plane = x_plane; b.px = cdiv(b.HpWp, kTriPix); b.cx = cdiv(b.C, kTriCh); b.blocks = b.px * b.cx * p.n8; b.sums = nullptr; b.wide = false;
+    b.plane = x_plane; b.px = cdiv(b.HpWp, d.C <= kTriFew ? kTriFewPix : kTriPix); b.cx = cdiv(b.C, kTriCh); b.blocks = b.px * b.cx * p.n8; b.sums = nullptr; b.wide = false;
     ProfScope prof("tri_batch", 4.0 * (double)(d.y_elems + d.x_elems) + 48.0 * (double)(dy_plane + x_plane), stream);
     hipLaunchKernelGGL(tri_batch_kernel, dim3((unsigned)(a.blocks + b.blocks + cdiv(p.groups, 256))), dim3(256), 0, stream, a, b, soff,
                        p.groups, p.groups_true, d.P * d.Q, d.Q, d.st, p.Wp);
