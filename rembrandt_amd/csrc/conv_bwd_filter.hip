@@ -998,11 +998,11 @@ extern "C" size_t rh_conv2d_workspace_bytes(const rh_conv_geom* g, int pass) {
 }
 
 // Scratch of the split-operand forms where `flags` take them; 0 where they do not, and where it cannot be
-// more than `floor` (the filter gradient's copies, exponents and maxima, and slices of up to 2048 tiles or 256 MB in all).
+// more than `floor` (the filter gradient's copies, exponents and maxima, and one slab or slices of up to 2048 tiles and 256 MB in all).
 static size_t split_scratch(const ConvDims& d, int pass, int flags, size_t floor) {
   if (pass == RH_CONV_BWD_FILTER) {
     const double copies = 6.0 * round_up(d.N, 8) * ((double)d.K * (d.P * d.Q + 1) + (double)d.C * (d.H + 2 * d.pad) * (d.W + 2 * d.pad));
-    const double slices = fmin(256e6, fmax(4.0 * (double)d.w_elems, 2048.0 * 4 * 128 * 128));
+    const double slices = fmax(4.0 * (double)d.w_elems, fmin(256e6, 2048.0 * 4 * 128 * 128));
     const double rest = (double)cdiv(d.N, 8) * 4.0 * (d.P * d.Q + (double)d.K * (d.P * d.Q / 32 + 1)) + 64.0 * (d.K + d.C) + 65536.0;
     if (copies + slices + rest < (double)floor) return 0;
     size_t need = 0;

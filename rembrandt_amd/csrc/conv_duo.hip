@@ -449,6 +449,7 @@ TriFilterPlan plan_duo_bwd_filter(const ConvDims& d, bool wide) {
     const double us = duo_run_us(rate, (long long)tiles * S, n) + 0.45 * S + 1.6e-6 * (double)d.w_elems * (S + 1);
     if (us < p.us) { p.us = us; p.splits = S; }
   }
+  if (p.splits == 0) p.splits = 1;   // (as plan_tri_bwd_filter)
   p.us += 22.8 + 2e-6 * (double)(d.x_elems + d.y_elems);
   p.part_bytes = align256(sizeof(float) * (size_t)p.splits * (size_t)d.w_elems);
   p.sum_rows = p.n8 * cdiv(d.P * d.Q, kDuoPix);

@@ -487,6 +487,7 @@ TriFilterPlan plan_tri_bwd_filter(const ConvDims& d, bool wide) {
                       4.0 * (double)d.w_elems * (S + 1) / 2.2e6;
     if (us < p.us) { p.us = us; p.splits = S; }
   }
+  if (p.splits == 0) p.splits = 1;   // (one slab is past the limit: not taken by itself, but whole where the flags ask for it)
   p.us += 15.0 + (4.0 * (double)(d.x_elems + d.y_elems) + 3.0 * (double)(dy_part + x_part)) / 5.3e6;
   p.part_bytes = align256(sizeof(float) * (size_t)p.splits * (size_t)d.w_elems);
   p.sum_rows = p.n8 * cdiv(d.P * d.Q, kTriPix);

@@ -235,6 +235,22 @@ def test_f16x2_scratch_is_for_callers_that_allow_the_form(geom):
             assert lib.rh_conv2d_workspace_bytes_for_upto(C.byref(g), pass_, flags) == most, (pass_, flags)
 
 
+@pytest.mark.parametrize("geom", [(1, 9216, 13, 8192, 1, 1, 0), (1, 8200, 9, 8200, 1, 1, 0)], ids=str)
+def test_split_filter_gradient_scratch_of_the_largest_filters(geom):
+    """Filters of more than 64e6 weights, whose one slab is past the planners' limit on slices: the scratch asked for holds both operand
+    copies, that slab and the rows of the bias gradient's sums behind it."""
+    lib = _lib.lib()
+    n, c, extent, k, size, st, pad = geom
+    g = _lib.ConvGeom(n, c, extent, extent, k, size, size, st, pad)
+    out, n8 = (extent + 2 * pad - size) // st + 1, (n + 7) // 8
+    groups = n8 * out * out
+    values = 8 * (groups * k + n8 * (extent + 2 * pad) ** 2 * c)
+    slab, sums = 4 * k * c * size * size, 4 * n8 * ((out * out + 31) // 32) * k
+    for flags, part_bytes in ((_lib.RH_ALGO_BF16X3, 6), (_lib.RH_ALGO_F16X2, 4), (_lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_BF16X3_WIDE, 6)):
+        need = lib.rh_conv2d_workspace_bytes_for(C.byref(g), _lib.RH_CONV_BWD_FILTER, flags | _lib.RH_ALGO_DIRECT)
+        assert need >= part_bytes * values + slab + sums, (flags, need)
+
+
 def test_conv_scratch_without_the_bf16x3_bit():
     """What a caller without the bit needs is what the other forms need: 13 MB where the split copies take 52, 131 where they take
     159, 355 where they take 483."""
