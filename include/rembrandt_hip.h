@@ -75,12 +75,12 @@ typedef void* rh_stream_t; /* hipStream_t */
                                              8, and backward-data stride 1 and R = S (of stride 2 to 4, any R and S, it has
                                              the form without RH_ALGO_DIRECT only).  No effect beside the other RH_ALGO_* bits
                                              and RH_MATH_BF16_MFMA_FP32ACC. */
-#define RH_ALGO_BF16X3_WIDE        0x4000 /* with RH_ALGO_BF16X3 or RH_ALGO_F16X2, on the filter gradient (no effect elsewhere): dy holds small
+#define RH_ALGO_BF16X3_WIDE        0x4000 /* with RH_ALGO_BF16X3, on the filter gradient (no effect elsewhere): dy holds small
                                              values of one sign almost everywhere beside a few large ones, as the deltas
                                              that a batch norm's backward leaves behind a ReLU.  The bf16 instruction cuts
                                              products at 2^-24 of the largest of eight, which against a positive x adds up
                                              to several times the fp32 instruction's error; with this bit the small values
-                                             are multiplied apart (seven products a pair, 4 to 12 % more time; four of fp16) and the
+                                             are multiplied apart (seven products a pair, 4 to 12 % more time) and the
                                              error is below the fp32 instruction's again.  The operators set it for their
                                              batch-normalised convolutions. */
 #define RH_ALGO_F16X2              0x8000 /* convolutions: the contraction may also run on fp16 matrix instructions, every fp32 operand

@@ -628,7 +628,7 @@ TriFilterPlan plan_tri_bwd_filter(const ConvDims& d, bool wide);
 // pixels.
 int launch_conv_tri_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
                                hipStream_t stream, float** parts, int* used);
-TriFilterPlan plan_duo_bwd_filter(const ConvDims& d, bool wide);
+TriFilterPlan plan_duo_bwd_filter(const ConvDims& d);
 int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
                                hipStream_t stream, float** parts, int* used);
 

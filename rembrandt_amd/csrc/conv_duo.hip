@@ -73,12 +73,11 @@ __global__ __launch_bounds__(256) void duo_max_kernel(DuoMaxJob a, DuoMaxJob b) 
   else duo_max_body(b, blockIdx.x - a.blocks, wave_top);
 }
 
-template <bool WIDE = false>
 __device__ __forceinline__ void duo_store(uint4* dst, size_t at, size_t plane, const float (&v)[8], int e, float least) {
-  uint4 o[WIDE ? 3 : 2];
-  duo_pack8<WIDE>(v, e, least, o);
-#pragma unroll
-  for (int p = 0; p < (WIDE ? 3 : 2); ++p) dst[at + p * plane] = o[p];
+  uint4 o[2];
+  duo_pack8(v, e, least, o);
+  dst[at] = o[0];
+  dst[at + plane] = o[1];
 }
 
 // Filter copy, its rows' exponents and the table of the image's group offsets; tri_filter_body's items and order.
@@ -167,7 +166,6 @@ struct DuoBatchArgs {
   int px, cx, blocks;
   float* sums;
 };
-template <bool WIDE>
 __device__ __forceinline__ void duo_batch_body(const DuoBatchArgs& a, int b, float (&tile)[8][kDuoCh][kDuoPix + 1], float (&tops)[8][kDuoCh]) {
   const int bx = b % a.px, t = b / a.px, by = t % a.cx, bz = t / a.cx;
   const int pix0 = bx * kDuoPix, c0 = by * kDuoCh, n0 = bz * 8;
@@ -213,7 +211,7 @@ __device__ __forceinline__ void duo_batch_body(const DuoBatchArgs& a, int b, flo
 #pragma unroll
     for (int n = 0; n < 8; ++n) v[n] = tile[n][cl][pl];
     if (a.sums) sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-    if (pix < a.HpWp && c < a.C) duo_store<WIDE>(a.xt, ((size_t)bz * a.HpWp + pix) * a.C + c, a.plane, v, ex, kDuoLeastSum);
+    if (pix < a.HpWp && c < a.C) duo_store(a.xt, ((size_t)bz * a.HpWp + pix) * a.C + c, a.plane, v, ex, kDuoLeastSum);
   }
   if (a.sums) {
     __syncthreads();
@@ -231,18 +229,17 @@ __device__ __forceinline__ void duo_batch_body(const DuoBatchArgs& a, int b, flo
 
 // Both operands of a filter gradient and soff[g], the place of group g = (n/8, p, q) in x's copy; the groups past the last
 // are zeros of dy.
-template <bool WIDE>
 __global__ __launch_bounds__(256) void duo_batch_kernel(DuoBatchArgs dy, DuoBatchArgs x, int* __restrict__ soff, int groups,
                                                         int groups_true, int PQ, int Q, int st, int Wp) {
   __shared__ float tile[8][kDuoCh][kDuoPix + 1];
   __shared__ float tops[8][kDuoCh];
   int b = blockIdx.x;
-  if (b < dy.blocks) { duo_batch_body<WIDE>(dy, xcd_remap(b, dy.blocks), tile, tops); return; }
+  if (b < dy.blocks) { duo_batch_body(dy, xcd_remap(b, dy.blocks), tile, tops); return; }
   b -= dy.blocks;
-  if (b < x.blocks) { duo_batch_body<false>(x, xcd_remap(b, x.blocks), tile, tops); return; }
+  if (b < x.blocks) { duo_batch_body(x, xcd_remap(b, x.blocks), tile, tops); return; }
   b -= x.blocks;
   if (groups > groups_true)   // (one group: every block of the table writes a share)
-    for (int i = b * 256 + threadIdx.x; i < (WIDE ? 3 : 2) * dy.C; i += (int)(gridDim.x - dy.blocks - x.blocks) * 256)
+    for (int i = b * 256 + threadIdx.x; i < 2 * dy.C; i += (int)(gridDim.x - dy.blocks - x.blocks) * 256)
       dy.xt[(size_t)(i / dy.C) * dy.plane + (size_t)groups_true * dy.C + i % dy.C] = make_uint4(0, 0, 0, 0);
   const int g = b * 256 + threadIdx.x;
   if (g >= groups) return;
@@ -254,7 +251,7 @@ __global__ __launch_bounds__(256) void duo_batch_kernel(DuoBatchArgs dy, DuoBatc
   soff[g] = off;
 }
 
-template <class T, bool NCHW, class PASS, bool WIDE = false>
+template <class T, bool NCHW, class PASS>
 static int launch_duo(const DuoParams& ap, const DuoParams& bp, const DuoSource& src, const EpiParams& ep, int k_steps, int groups,
                       int splits, int* used, double flops, hipStream_t stream, const char* tag) {
   const int tiles_m = cdiv(ep.rows, T::BM), tiles_n = cdiv(ep.cols, T::BN);
@@ -267,13 +264,13 @@ static int launch_duo(const DuoParams& ap, const DuoParams& bp, const DuoSource&
     if (n_split != ep.tail_splits || ep.full_tiles + ep.tail_tiles != tiles_m * tiles_n) return RH_E_INVALID;
     grid = dim3((unsigned)(ep.full_tiles + ep.tail_tiles * ep.tail_splits), 1u);
   }
-  constexpr size_t lds = DuoShape<T, WIDE>::LDS;
+  constexpr size_t lds = DuoShape<T>::LDS;
   static_assert(2 * lds <= 160 * 1024, "two blocks share a CU");
-  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm_duo_kernel<T, NCHW, PASS, WIDE>),
+  static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm_duo_kernel<T, NCHW, PASS>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return (int)attr;
   ProfScope prof(tag, flops, stream);
-  hipLaunchKernelGGL((mfma_gemm_duo_kernel<T, NCHW, PASS, WIDE>), grid, dim3(T::NT), lds, stream, ap, bp, src, ep, tiles_m, k_steps, sps, groups);
+  hipLaunchKernelGGL((mfma_gemm_duo_kernel<T, NCHW, PASS>), grid, dim3(T::NT), lds, stream, ap, bp, src, ep, tiles_m, k_steps, sps, groups);
   return launch_status();
 }
 
@@ -420,10 +417,8 @@ int launch_conv_duo(const TriPlan& p, bool bwd, const float* in, const float* w,
 
 // (1355 timed calls of 13 layers, slices of 1 to 128: rms error 9 %, the slices chosen 0.6 % slower than the best of them.)
 static const DuoRates kDuoFilter128 = {0.279, 2.9, 0.233, 0.0}, kDuoFilter96 = {0.267, 9.4, 0.482, 0.0}, kDuoFilter64 = {0.282, 0.8, 0.24, 1.9};
-TriFilterPlan plan_duo_bwd_filter(const ConvDims& d, bool wide) {
+TriFilterPlan plan_duo_bwd_filter(const ConvDims& d) {
   TriFilterPlan p = {};
-  p.wide = wide;
-  const int parts_a = wide ? 3 : 2;
   if (d.P <= 0 || d.Q <= 0) return p;
   p.Hp = d.H + 2 * d.pad; p.Wp = d.W + 2 * d.pad;
   p.n8 = cdiv(d.N, 8);
@@ -431,18 +426,17 @@ TriFilterPlan plan_duo_bwd_filter(const ConvDims& d, bool wide) {
   p.groups_true = (int)groups;
   p.groups = round_up(p.groups_true, 2);
   const size_t dy_part = 16 * (size_t)p.groups * d.K, x_part = 16 * (size_t)p.n8 * p.Hp * p.Wp * d.C;
-  if (parts_a * dy_part > kMaxBufferBytes || 2 * x_part > kMaxBufferBytes) return p;
+  if (2 * dy_part > kMaxBufferBytes || 2 * x_part > kMaxBufferBytes) return p;
   p.tab_bytes = align256(sizeof(int) * (size_t)p.groups) + align256(sizeof(int) * ((size_t)round_up(d.K, 128) + d.C)) +
                 align256(sizeof(float) * ((size_t)d.K * duo_channel_parts(d.K) + (size_t)d.C * duo_channel_parts(d.C)));
-  p.dyt_bytes = align256(parts_a * dy_part);
+  p.dyt_bytes = align256(2 * dy_part);
   p.xt_bytes = align256(2 * x_part);
   p.bm = pick_bm(d.K);
   if (p.bm == 32) p.bm = 64;
-  p.bn = p.bm > 64 ? 128 : wide ? 192 : 256;
+  p.bn = p.bm == 64 ? 256 : 128;
   const int CRS = d.C * d.R * d.S, tiles = cdiv(d.K, p.bm) * cdiv(CRS, p.bn), steps = p.groups / 2;
   p.us = 1e30;
-  DuoRates rate = p.bm == 128 ? kDuoFilter128 : p.bm == 96 ? kDuoFilter96 : kDuoFilter64;
-  if (wide) { rate.one *= 4.0 / 3; rate.two *= 4.0 / 3; }   // (by its products)
+  const DuoRates& rate = p.bm == 128 ? kDuoFilter128 : p.bm == 96 ? kDuoFilter96 : kDuoFilter64;
   for (int want = 1; want <= 256 && (want == 1 || (want * 6 <= steps && (long long)tiles * want <= 2048)); ++want) {
     const int n = cdiv(steps, want), S = cdiv(steps, n);
     if (S != want || 4.0 * (double)S * (double)d.w_elems > 256e6) continue;
@@ -485,17 +479,14 @@ int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const 
     b.x = x; b.xt = xt; b.top = top_b; b.parts = parts_b; b.exps = exps_b; b.N = d.N; b.C = d.C; b.H = d.H; b.W = d.W; b.halo = d.pad;
     b.HpWp = p.Hp * p.Wp; b.dWp = FastDiv((uint32_t)p.Wp); b.plane = x_plane; b.px = cdiv(b.HpWp, kDuoPix); b.cx = cdiv(b.C, kDuoCh);
     b.blocks = b.px * b.cx * p.n8; b.sums = nullptr;
-    ProfScope prof("duo_batch", 4.0 * (double)(d.y_elems + d.x_elems) + 16.0 * (double)((p.wide ? 3 : 2) * dy_plane + 2 * x_plane), stream);
-    const dim3 grid((unsigned)(a.blocks + b.blocks + cdiv(p.groups, 256)));
-    if (p.wide)
-      hipLaunchKernelGGL(duo_batch_kernel<true>, grid, dim3(256), 0, stream, a, b, soff, p.groups, p.groups_true, d.P * d.Q, d.Q, d.st, p.Wp);
-    else
-      hipLaunchKernelGGL(duo_batch_kernel<false>, grid, dim3(256), 0, stream, a, b, soff, p.groups, p.groups_true, d.P * d.Q, d.Q, d.st, p.Wp);
+    ProfScope prof("duo_batch", 4.0 * (double)(d.y_elems + d.x_elems) + 32.0 * (double)(dy_plane + x_plane), stream);
+    hipLaunchKernelGGL(duo_batch_kernel, dim3((unsigned)(a.blocks + b.blocks + cdiv(p.groups, 256))), dim3(256), 0, stream, a, b, soff,
+                       p.groups, p.groups_true, d.P * d.Q, d.Q, d.st, p.Wp);
   }
   if (int e = launch_status()) return e;
   const int CRS = d.C * d.R * d.S;
   DuoParams ap, bp;
-  ap.t.v.ptr = dyt; ap.t.plane = (int)(16 * dy_plane); ap.t.v.bytes = (uint32_t)((p.wide ? 48 : 32) * dy_plane);
+  ap.t.v.ptr = dyt; ap.t.plane = (int)(16 * dy_plane); ap.t.v.bytes = (uint32_t)(32 * dy_plane);
   ap.t.v.M = d.K; ap.t.v.inner = 1; ap.t.v.innerW = 1; ap.t.v.img_stride = 16; ap.t.v.a_stride = 0; ap.t.v.b_stride = 0;
   ap.t.v.soff = nullptr; ap.t.v.group_stride = d.K * 16;
   ap.exps = exps_a; ap.ediv = 1; ap.emod = d.K;
@@ -510,22 +501,14 @@ int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const 
   EpiParams ep;
   ep.out = *parts; ep.bias = nullptr; ep.alpha = 1.0f; ep.beta = 0.0f;
   ep.rows = d.K; ep.cols = CRS; ep.inner = 0; ep.ld = CRS; ep.relu = 0; ep.split_stride = (long long)d.K * CRS;
-  const double flops = (p.wide ? 8.0 : 6.0) * (double)d.w_elems * d.N * d.P * d.Q;
+  const double flops = 6.0 * (double)d.w_elems * d.N * d.P * d.Q;
   const int steps = p.groups / 2;
-#define RH_DUO(TILE, WIDE, TAG)                                                                                                        \
-  launch_duo<TILE, false, PassConvBwdFilter, WIDE>(ap, bp, src, ep, steps, p.groups_true, p.splits, used, flops, stream, \
-                                                   "conv_bwd_filter_duo_" TAG)
-  if (p.wide) {
-    switch (p.bm) {
-      case 128: return RH_DUO(T128x128t, true, "wide_128x128");
-      case 96: return RH_DUO(T96x128t, true, "wide_96x128");
-      default: return RH_DUO(T64x192t, true, "wide_64x192");
-    }
-  }
+#define RH_DUO(TILE, TAG) \
+  launch_duo<TILE, false, PassConvBwdFilter>(ap, bp, src, ep, steps, p.groups_true, p.splits, used, flops, stream, "conv_bwd_filter_duo_" TAG)
   switch (p.bm) {
-    case 128: return RH_DUO(T128x128t, false, "128x128");
-    case 96: return RH_DUO(T96x128t, false, "96x128");
-    default: return RH_DUO(T64x256t, false, "64x256");
+    case 128: return RH_DUO(T128x128t, "128x128");
+    case 96: return RH_DUO(T96x128t, "96x128");
+    default: return RH_DUO(T64x256t, "64x256");
   }
 #undef RH_DUO
 }

@@ -37,9 +37,8 @@ __device__ __forceinline__ int duo_exponent(float top) {
 // Eight values (one group) of a row with exponent e.  A group whose largest scaled value is under `least` is marked.
 constexpr float kDuoLeast = 6.103515625e-5f;        // 2^-14: from here on the two parts hold 22 bits
 constexpr float kDuoLeastSum = 5.820766091e-11f;    // 2^-34: from here on they hold two
-template <bool WIDE>
-__device__ __forceinline__ void duo_pack8(const float (&v)[8], int e, float least, uint4 (&o)[WIDE ? 3 : 2]) {
-  uint32_t w[3][4];
+__device__ __forceinline__ void duo_pack8(const float (&v)[8], int e, float least, uint4 (&o)[2]) {
+  uint32_t w[2][4];
   uint32_t top = 0, any = 0;
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
@@ -68,20 +67,8 @@ __device__ __forceinline__ void duo_pack8(const float (&v)[8], int e, float leas
       }
     }
   }
-  if (WIDE) {   // the first parts of the values under 2^-kTriWide of the group's largest, as a third part
-    const uint32_t limit = top > ((uint32_t)kTriWide << 23) ? top - ((uint32_t)kTriWide << 23) : 0u;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      uint32_t small = 0;
-#pragma unroll
-      for (int h = 0; h < 2; ++h)
-        if ((__builtin_bit_cast(uint32_t, __builtin_amdgcn_ldexpf(v[2 * i + h], e)) & 0x7fffffffu) < limit) small |= 0xffffu << (16 * h);
-      w[2][i] = w[0][i] & small;
-      w[0][i] ^= w[2][i];
-    }
-  }
-#pragma unroll
-  for (int p = 0; p < (WIDE ? 3 : 2); ++p) o[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
+  for (int p = 0; p < 2; ++p) o[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
 }
 
 // An operand of this form: TriParams with two parts, and the exponents of its rows: row m has exps[m / ediv % emod].
@@ -145,14 +132,12 @@ struct DuoSource {
 };
 
 // Brings one K step (16 k = two groups, two parts) of both operands to LDS with direct loads: four a block of 64 rows.  Each wave
-// brings one block, and its share of what is left: of a fifth block (the last of B) one (part, group), of A's third part in the wide
-// form one group of one of its two blocks, or of its one block (by two waves each).
-template <int RA, int RB, bool WIDE>
+// brings one block; of a fifth block (the last of B) each wave brings one (part, group).
+template <int RA, int RB>
 struct DmaDuo {
-  static constexpr int NB = (RA + RB) / 64, PA = WIDE ? 3 : 2;
-  static_assert(RA % 64 == 0 && RB % 64 == 0 && (NB == 4 || (NB == 5 && !WIDE)), "a block of rows for every wave");
-  static constexpr bool EXTRA = NB == 5 || WIDE;
-  static constexpr int CNT = EXTRA ? 5 : 4;
+  static constexpr int NB = (RA + RB) / 64;
+  static_assert(RA % 64 == 0 && RB % 64 == 0 && (NB == 4 || NB == 5), "a block of rows for every wave");
+  static constexpr int CNT = NB;
   typedef const __attribute__((address_space(4))) int* ctab_t;
   u32x4 rsrc, xrsrc;
   const int* tab;
@@ -181,20 +166,13 @@ struct DmaDuo {
     rsrc = resource(t.v);
     tab = bp.t.v.soff;
     plane = __builtin_amdgcn_readfirstlane(t.plane);
-    gstride = __builtin_amdgcn_readfirstlane(WIDE ? ap.t.v.group_stride : t.v.group_stride);
+    gstride = __builtin_amdgcn_readfirstlane(t.v.group_stride);
     linear = is_a;
     const int rb = is_a ? wave : wave - RA / 64;
-    lds = (uint32_t)(((is_a ? 0 : 2 * PA * RA) + rb * 64) * 16);
+    lds = (uint32_t)(((is_a ? 0 : 4 * RA) + rb * 64) * 16);
     lds_slab = (uint32_t)((is_a ? RA : RB) * 16);
     vbase = row_offset(t.v, (is_a ? m0 : n0) + rb * 64 + lane);
-    if (WIDE) {
-      const int xb = RA == 128 ? wave & 1 : 0;
-      xhalf = RA == 128 ? wave >> 1 : wave & 1;
-      xrsrc = resource(ap.t.v);
-      xplane = __builtin_amdgcn_readfirstlane(2 * ap.t.plane);
-      xlds = (uint32_t)(((4 + xhalf) * RA + xb * 64) * 16);
-      xvbase = row_offset(ap.t.v, m0 + xb * 64 + lane);
-    } else if (NB == 5) {
+    if (NB == 5) {
       xrsrc = resource(bp.t.v);
       xhalf = wave >> 1;
       xplane = __builtin_amdgcn_readfirstlane((wave & 1) * bp.t.plane);
@@ -209,31 +187,22 @@ struct DmaDuo {
       const int g = 2 * step + h;
       const int t = ((ctab_t)(uintptr_t)tab)[g];
       so[h] = linear ? g * gstride : t;
-      if (EXTRA && h == xhalf) xso = WIDE ? g * gstride : t;
+      if (NB == 5 && h == xhalf) xso = t;
     }
   }
-  __device__ __forceinline__ void issue(uint32_t base, int i) const {   // i = part + 2 group; 4: the share of what is left
+  __device__ __forceinline__ void issue(uint32_t base, int i) const {   // i = part + 2 group; 4: the share of the fifth block
     if (i < 4) dma_load16(rsrc, base + lds + (uint32_t)((i & 1) * 2 + i / 2) * lds_slab, vbase, (uint32_t)(so[i / 2] + (i & 1) * plane));
     else dma_load16(xrsrc, base + xlds, xvbase, (uint32_t)(xso + xplane));
   }
 };
 
-// The ring: a step of four blocks of 64 rows is 16 KB, of five 20 KB, A's third part 1 KB a block and group; two blocks share a CU's
-// 160 KB.
-template <class T, bool WIDE>
+// The ring: a step of four blocks of 64 rows is 16 KB, of five 20 KB; two blocks share a CU's 160 KB.
+template <class T>
 struct DuoShape {
-  static constexpr int RA = (T::BM + 63) / 64 * 64, RB = (T::BN + 63) / 64 * 64;
-  static constexpr int SA = (WIDE ? 6 : 4) * RA, SB = 4 * RB, R = 80 * 1024 / (16 * (SA + SB)), LDS = R * (SA + SB) * 16;
+  static constexpr int RA = (T::BM + 63) / 64 * 64, RB = (T::BN + 63) / 64 * 64, STEP = 4 * (RA + RB), R = 80 * 1024 / (16 * STEP), LDS = R * STEP * 16;
   static_assert(T::NT == 4 * kWave && T::BK == 16 && R >= 4, "four waves, 16 k a step");
 };
 
-// The wide form, for what gemm_tri.h's is for: the fp16 instruction cuts the eight products that it adds at a time toward zero at 2^-24
-// of the largest of them as the bf16 one does, so the first parts of A's small values are a part of their own and multiplied apart
-// (a1 = large | small): four MFMAs a block and step.  A's first part then has no second set of registers: this step's large first parts
-// are read behind the step's barrier and wanted at its second product.  (No KEEP: with it a dozen registers go to scratch, and the
-// wait for a scratch load is a wait for the direct loads issued before it; the kernel takes twice as long.)  256 -> 256 3x3 14x14
-// b256 364 us with three parts -> 270, 512 -> 512 7x7 340 -> 273, with 0.56 to 0.82 of the error.
-//
 // K steps [s_begin, s_end) of the tile at (m0, n0).  Three MFMAs for each 32 x 32 block of a wave and step: a2 b1, a1 b2 (accumulators
 // of their own, 2^11 times as large) and a1 b1.  a2 and b2 of the next step are read over this step's once their product has been
 // issued, a1 and b1 into a second set: 64 x 64 of a 128 x 128 tile are 192 accumulators in three sets and 48 registers of operands, two
@@ -241,13 +210,13 @@ struct DuoShape {
 // have R - 2 steps to land.  Bound by the power that the MFMAs draw: 384 -> 384 3x3 13x13 b256 forward takes 270 us = 425 TFLOP/s of fp32
 // multiply-adds, the matrix pipes busy 69 % of the time at 1.77 GHz (three bf16 parts 470 us; from registers alone three products would
 // reach 600 TFLOP/s); a barrier every second step, or a raised wave priority, changes nothing.
-template <class T, bool NCHW, bool KEEP, bool WIDE>
+template <class T, bool NCHW, bool KEEP>
 __device__ __forceinline__ void duo_block(const DuoParams& ap, const DuoParams& bp, const DuoSource& src, const EpiParams& ep, int m0,
                                           int n0, int s_begin, int s_end, int groups, int dst_split) {
-  typedef DuoShape<T, WIDE> D;
+  typedef DuoShape<T> D;
   constexpr int TM = T::TM, TN = T::TN, Q = TM * TN, R = D::R, RA = D::RA, RBn = D::RB;
-  typedef DmaDuo<RA, RBn, WIDE> Loader;
-  constexpr int SA = D::SA, SB = D::SB;   // 16-byte pieces of a step
+  typedef DmaDuo<RA, RBn> Loader;
+  constexpr int SA = 4 * RA, SB = 4 * RBn;   // 16-byte pieces of a step
   extern __shared__ float lds_dyn[];
   uint4* const sm = reinterpret_cast<uint4*>(lds_dyn);   // [R][A: part, group, row; B]
   const uint32_t lds0 = (uint32_t)(uintptr_t)(__attribute__((address_space(3))) void*)sm;
@@ -282,9 +251,9 @@ __device__ __forceinline__ void duo_block(const DuoParams& ap, const DuoParams& 
 
   const uint4* const pa0 = sm + (lane >> 5) * RA + wm * (TM * 32) + (lane & 31);
   const uint4* const pb0 = sm + SA + (lane >> 5) * RBn + wn * (TN * 32) + (lane & 31);
-  uint4 a1[2][TM], b1[2][TN], a2[TM], b2[TN];   // (wide: a1[0] the large first parts, a1[1] the small ones, or both)
+  uint4 a1[2][TM], b1[2][TN], a2[TM], b2[TN];
 #pragma unroll
-  for (int i = 0; i < TM; ++i) { a1[WIDE][i] = pa0[(WIDE ? 4 : 0) * RA + i * 32]; a2[i] = pa0[2 * RA + i * 32]; }
+  for (int i = 0; i < TM; ++i) { a1[0][i] = pa0[i * 32]; a2[i] = pa0[2 * RA + i * 32]; }
 #pragma unroll
   for (int j = 0; j < TN; ++j) { b1[0][j] = pb0[j * 32]; b2[j] = pb0[2 * RBn + j * 32]; }
 
@@ -347,82 +316,19 @@ __device__ __forceinline__ void duo_block(const DuoParams& ap, const DuoParams& 
       __builtin_amdgcn_sched_barrier(0);
     }
   };
-  auto wide_step = [&](int it, auto c_tag, auto more_tag, auto first_tag) {
-    constexpr int c = decltype(c_tag)::value, n = c ^ 1;
-    constexpr bool MORE = decltype(more_tag)::value, FIRST = decltype(first_tag)::value;
-    __builtin_amdgcn_sched_barrier(0);
-    if (MORE) wait_vmcnt<(R - 3) * Loader::CNT>();
-    else wait_vmcnt<0>();
-    __syncthreads();
-    const int nx = rd + 1 == R ? 0 : rd + 1, past = rd == 0 ? R - 1 : rd - 1;
-    const uint4* const pc = pa0 + rd * (SA + SB);
-    const uint4* const pa = pa0 + nx * (SA + SB);
-    const uint4* const pb = pb0 + nx * (SA + SB);
-    const uint32_t base = lds0 + (uint32_t)(past * (SA + SB)) * 16u;
-    rd = nx;
-    // this step's large first parts, then of the next one b1, a2 behind the first product, b2 behind the second, the small first parts
-    // behind the third
-    constexpr int kL = TM, kB1 = kL + TN, kA2 = kB1 + TM, kB2 = kA2 + TN, kS = kB2 + TM;
-    auto read = [&](int s) {
-      if (s < kL) a1[0][s] = pc[s * 32];
-      else if (s < kB1) b1[n][s - kL] = pb[(s - kL) * 32];
-      else if (s < kA2) a2[s - kB1] = pa[2 * RA + (s - kB1) * 32];
-      else if (s < kB2) b2[s - kA2] = pb[2 * RBn + (s - kA2) * 32];
-      else if (s < kS) a1[1][s - kB2] = pa[4 * RA + (s - kB2) * 32];
-    };
-    auto toggle = [&] {   // the small first parts to both and back: no value has both
-#pragma unroll
-      for (int i = 0; i < TM; ++i) {
-        a1[1][i].x ^= a1[0][i].x; a1[1][i].y ^= a1[0][i].y; a1[1][i].z ^= a1[0][i].z; a1[1][i].w ^= a1[0][i].w;
-      }
-    };
-    int slot = 0, load = 0, moved = 0;
-#pragma unroll
-    for (; slot < kL; ++slot) read(slot);
-#pragma unroll
-    for (int m = 0; m < 4 * Q; ++m) {
-      const int p = m / Q, t = m % Q, i = t / TN, j = t % TN;
-      if (p < 2)
-        low[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, p ? a1[1][i] : a2[i]),
-                                                           __builtin_bit_cast(f16x8_t, p ? b2[j] : b1[c][j]), low[i][j], 0, 0, 0);
-      else
-        acc[i][j] = __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(f16x8_t, a1[p == 2][i]), __builtin_bit_cast(f16x8_t, b1[c][j]),
-                                                           FIRST && !KEEP && p == 2 ? zero : acc[i][j], 0, 0, 0);
-      __builtin_amdgcn_sched_barrier(0);
-      if (FIRST) {
-#pragma unroll
-        for (; moved < 16 * Q && moved < (m + 1) * 8; ++moved) end_chain(moved);
-      }
-      const int upto = m < Q ? kL + (m + 1) * TN / Q : m < 2 * Q ? kB1 + (m + 1 - Q) * TM / Q : m < 3 * Q ? kA2 + (m + 1 - 2 * Q) * TN / Q
-                       : m + 1 - 3 * Q < TM ? kB2 + m + 1 - 3 * Q : kS;
-#pragma unroll
-      for (; slot < upto; ++slot) read(slot);
-      if (m == Q - 1 || m == 2 * Q - 1) toggle();
-      if (MORE) {
-#pragma unroll
-        for (; load < Loader::CNT && load < (m + 1) * Loader::CNT / (4 * Q - 2); ++load) ld.issue(base, load);
-        if (m == 4 * Q - 1) ld.prep(s_begin + (it + R < nk ? it + R : nk - 1));
-      }
-      __builtin_amdgcn_sched_barrier(0);
-    }
-  };
   const std::integral_constant<int, 0> c0;
   const std::integral_constant<int, 1> c1;
   const std::true_type yes;
   const std::false_type no;
-  auto go = [&](int it, auto c_tag, auto more_tag, auto first_tag) {
-    if constexpr (WIDE) wide_step(it, c_tag, more_tag, first_tag);
-    else step(it, c_tag, more_tag, first_tag);
-  };
   int it = 0;
   for (; it + kDuoChain + R - 2 < nk; it += kDuoChain) {
-    go(it, c0, yes, yes);
+    step(it, c0, yes, yes);
 #pragma unroll 1
     for (int u = 1; u + 1 < kDuoChain; u += 2) {
-      go(it + u, c1, yes, no);
-      go(it + u + 1, c0, yes, no);
+      step(it + u, c1, yes, no);
+      step(it + u + 1, c0, yes, no);
     }
-    go(it + kDuoChain - 1, c1, yes, no);
+    step(it + kDuoChain - 1, c1, yes, no);
   }
   if (it > 0) {
 #pragma unroll
@@ -432,18 +338,18 @@ __device__ __forceinline__ void duo_block(const DuoParams& ap, const DuoParams& 
     }
   }
   for (; it + R < nk; it += 2) {
-    go(it, c0, yes, no);
-    go(it + 1, c1, yes, no);
+    step(it, c0, yes, no);
+    step(it + 1, c1, yes, no);
   }
   if (it + R - 1 < nk) {
-    go(it, c0, yes, no);
-    go(it + 1, c1, no, no);
+    step(it, c0, yes, no);
+    step(it + 1, c1, no, no);
     it += 2;
   }
   while (it < nk) {
-    go(it++, c0, no, no);
+    step(it++, c0, no, no);
     if (it >= nk) break;
-    go(it++, c1, no, no);
+    step(it++, c1, no, no);
   }
 
   // the sums, scaled back by the row's and the column's exponent
@@ -491,7 +397,7 @@ __device__ __forceinline__ void duo_block(const DuoParams& ap, const DuoParams& 
   store_tile<T, NCHW>(acc, ep, m0, n0, wm, wn, lane, dst_split);
 }
 
-template <class T, bool NCHW, class PASS, bool WIDE = false>
+template <class T, bool NCHW, class PASS>
 __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_duo_kernel(DuoParams ap, DuoParams bp, DuoSource src, EpiParams ep,
                                                                       int tiles_m, int k_steps, int steps_per_split, int groups) {
   int slice, logical, dst_split;   // as in mfma_gemm_kernel
@@ -522,7 +428,7 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_duo_kernel(DuoParams 
   const int s_begin = whole ? 0 : slice * steps_per_split;
   int s_end = whole ? k_steps : s_begin + steps_per_split;
   if (s_end > k_steps) s_end = k_steps;
-  duo_block<T, NCHW, !WIDE && !std::is_same<PASS, PassConvFwd>::value, WIDE>(ap, bp, src, ep, tile_m * T::BM, tile_n * T::BN, s_begin, s_end, groups, dst_split);
+  duo_block<T, NCHW, !std::is_same<PASS, PassConvFwd>::value>(ap, bp, src, ep, tile_m * T::BM, tile_n * T::BN, s_begin, s_end, groups, dst_split);
 }
 
 }  // namespace rh

@@ -828,15 +828,6 @@ def test_conv2d_f16x2(dev, case):
     assert torch.equal(ops.conv2d_bwd_filter(xd, dyd, w.shape, st, pad, algo=F2), dw), "run to run the same bits"
     scaled = ops.conv2d_bwd_filter(xd, T(dy * row.reshape(1, -1, 1, 1), dev), w.shape, st, pad, algo=F2)
     assert np.array_equal(N(scaled), N(dw) * row), "powers of two of a channel"
-    F2 |= _lib.RH_ALGO_BF16X3_WIDE
-    mixed = dy * np.where(synth.uniform(37, 9, dy.shape) < 0.5, np.float32(1.0), np.float32(0.01))   # small values to multiply apart
-    dw, tags = profile_tags(lambda: ops.conv2d_bwd_filter(xd, T(mixed, dev), w.shape, st, pad, algo=F2))
-    assert any(t.startswith("conv_bwd_filter_duo_wide_") for t in tags), tags
-    assert_close(N(dw), O.conv2d_bwd_filter(x, mixed, w.shape, st, pad), "f16x2 wide bwd filter")
-    dwc, dbc = ops.conv2d_bwd_filter_bias(xd, T(mixed, dev), w.shape, st, pad, alpha=0.25, beta=1.0, dw=T(dw0, dev), db=T(db0, dev), algo=F2)
-    assert_close(N(dwc), O.conv2d_bwd_filter(x, mixed, w.shape, st, pad, 0.25, 1.0, dw0.copy()), "f16x2 wide bwd filter alpha/beta")
-    assert_close(N(dbc), O.conv2d_bwd_bias(mixed, 0.25, 1.0, db0.copy()), "f16x2 wide bias gradient")
-    assert torch.equal(ops.conv2d_bwd_filter(xd, T(mixed, dev), w.shape, st, pad, algo=F2), dw), "run to run the same bits"
 
 
 def test_conv2d_f16x2_values_out_of_range(dev):
@@ -876,9 +867,9 @@ def test_conv2d_f16x2_values_out_of_range(dev):
     assert np.array_equal(got[0], np.broadcast_to(x[0, 3], (64, 1, 8)))
 
 
-@pytest.mark.parametrize("case", [(90, 256, 14, 256, 3, 1), (90, 512, 7, 512, 3, 1), (24, 256, 14, 256, 3, 1)], ids=str)
+@pytest.mark.parametrize("case", [(90, 256, 14, 256, 3, 1), (24, 512, 7, 512, 3, 1)], ids=str)
 def test_conv2d_f16x2_deltas_behind_a_batch_norm(dev, case):
-    """As test_conv2d_bf16x3_deltas_behind_a_batch_norm: where the wide form is taken, no larger an error than that of the one it replaces."""
+    """A filter gradient whose caller sets RH_ALGO_BF16X3_WIDE stays with three parts."""
     Nn, C, H, K, R, st = case
     say("f16x2 wide", case)
     P = (H + 2 - R) // st + 1
@@ -887,14 +878,8 @@ def test_conv2d_f16x2_deltas_behind_a_batch_norm(dev, case):
     dy = dy - dy.mean((0, 2, 3), keepdim=True)
     shape, X3 = (K, C, R, R), _lib.RH_ALGO_BF16X3 | _lib.RH_ALGO_BF16X3_WIDE
     got, tags = profile_tags(lambda: ops.conv2d_bwd_filter(x, dy, shape, st, 1, algo=X3 | _lib.RH_ALGO_F16X2))
-    before = ops.conv2d_bwd_filter(x, dy, shape, st, 1, algo=X3)
-    assert any(t.startswith("conv_bwd_filter_duo_wide_") for t in tags) == (Nn >= 90), tags
-    if Nn < 90:
-        assert torch.equal(got, before)
-        return
-    ref = _conv_sums64(x, torch.zeros(shape, device=dev), dy, st, 1)[2]
-    err, err0 = (float((t.double() - ref).norm() / ref.norm()) for t in (got, before))
-    assert err <= err0, (err, err0)
+    assert any(t.startswith("conv_bwd_filter_tri_wide_") for t in tags), tags
+    assert torch.equal(got, ops.conv2d_bwd_filter(x, dy, shape, st, 1, algo=X3))
 
 
 # Layers with the passes that the library takes in this form by itself beside RH_ALGO_BF16X3: whole contractions, slices, a sliced
