@@ -751,12 +751,12 @@ inline SplitPick pick_split(const ConvDims& d, bool bwd, int flags, size_t ws_by
 inline size_t split_bytes(const ConvDims& d, bool bwd, int flags, size_t floor) {
   if (!tri_shape(d, bwd)) return 0;
   // (the copies of three parts, and 24 slices of all tiles, of 256 MB together, or 12 of up to 255 tiles and of an image that they share;
-  // exponents and maxima)
+  // exponents, maxima and ratios)
   const int halo = bwd ? d.R - 1 - d.pad : d.pad, rows = bwd ? d.C : d.K, Ci = bwd ? d.K : d.C;
   const double img = 6.0 * d.N * Ci * ((bwd ? d.P : d.H) + 2 * halo) * ((bwd ? d.Q : d.W) + 2 * halo);
   const double out = 4.0 * (double)(bwd ? d.x_elems : d.y_elems);
   const double parts = fmin(24.0 * out, 12.0 * ((256.0 + rows / 64) * 128 * 192 * 4 + out / d.N));
-  if (img + (6.5 * Ci * d.R * d.S + 64.0) * rows + parts + 160.0 * d.N + 8192.0 < (double)floor) return 0;
+  if (img + (6.5 * Ci * d.R * d.S + 64.0) * rows + parts + 160.0 * d.N + 4.0 * Ci + 8192.0 < (double)floor) return 0;
   TriRival r[2];
   tri_rivals(d, bwd, r);
   size_t need = 0;

@@ -1,7 +1,7 @@
 // fp32 convolutions on the fp16 matrix instructions with operands of two scaled parts (gemm_duo.h): forward, stride-1
 // backward-data and backward-filter.
 //
-// Three launches in front of the reduction of slices: the largest magnitudes, the operand copies in two fp16 parts (4 bytes a value,
+// Three launches in front of the reduction of slices: the largest magnitudes (and the filters' ratios), the operand copies in two fp16 parts (4 bytes a value,
 // in the orders of conv_tri.hip), the contraction.  The exponents are the filter's by row and the image's by image, and in the filter
 // gradient both operands' by channel.
 #include "conv_common.h"
@@ -13,12 +13,14 @@ namespace rh {
 // its reads: a block has eight loads a thread in flight.
 struct DuoMaxJob {
   const float* src; float* part;
+  int* zero; int zeros;        // with the first block: counts to begin with
   int R, parts, blocks, vec;   // vec: by four values, I a multiple of 4 and src 16-byte aligned
   unsigned I, total, len;      // of a row, in units of four values where vec: I, O I and those of a part
   FastDiv dI;
 };
-static DuoMaxJob duo_max_job(const float* src, float* part, int O, int R, int I, int parts) {
+static DuoMaxJob duo_max_job(const float* src, float* part, int O, int R, int I, int parts, int* zero = nullptr, int zeros = 0) {
   DuoMaxJob j;
+  j.zero = zero; j.zeros = zeros;
   j.src = src; j.part = part; j.R = R; j.parts = parts; j.blocks = R * parts;
   j.vec = I % 4 == 0 && (reinterpret_cast<uintptr_t>(src) & 15) == 0;
   j.I = (unsigned)(j.vec ? I / 4 : I);
@@ -52,6 +54,8 @@ __device__ __forceinline__ uint32_t duo_max_range(const DuoMaxJob& j, int r, uns
 }
 __device__ __forceinline__ void duo_max_body(const DuoMaxJob& j, int b, uint32_t (&wave_top)[4]) {
   const int r = b / j.parts, q = b - r * j.parts;
+  if (b == 0)
+    for (int i = threadIdx.x; i < j.zeros; i += 256) j.zero[i] = 0;
   const unsigned f0 = (unsigned)q * j.len, f1 = f0 + j.len < j.total ? f0 + j.len : j.total;
   uint32_t top = j.vec ? duo_max_range<float4>(j, r, f0, f1) : duo_max_range<float>(j, r, f0, f1);
 #pragma unroll
@@ -67,23 +71,61 @@ __device__ __forceinline__ void duo_max_body(const DuoMaxJob& j, int b, uint32_t
     j.part[b] = __builtin_bit_cast(float, top);
   }
 }
-__global__ __launch_bounds__(256) void duo_max_kernel(DuoMaxJob a, DuoMaxJob b) {
+// For each group of eight channels of a filter tensor (Ck / 8 of them) the least ratio, over rows and taps, of a value to the largest of
+// its eight (0: a zero beside others), in kDuoRatioParts parts.
+constexpr int kDuoRatioParts = 8;
+struct DuoRatioJob {
+  const float* w; float* part;
+  int rows, Ck, RS, bwd;
+  FastDiv dRS;
+};
+__device__ __forceinline__ void duo_ratio_body(const DuoRatioJob& j, int b, uint32_t (&wave_least)[4]) {
+  const int cg = b / kDuoRatioParts, q = b - cg * kDuoRatioParts;
+  float least = 1.0f;
+  for (unsigned i = (unsigned)q * 256 + threadIdx.x; i < (unsigned)j.rows * (unsigned)j.RS; i += kDuoRatioParts * 256) {
+    uint32_t row, rs;
+    j.dRS.divmod(i, row, rs);
+    const float* const w = j.bwd ? j.w + ((size_t)cg * 8 * j.rows + row) * j.RS + rs : j.w + ((size_t)row * j.Ck + cg * 8) * j.RS + rs;
+    const size_t stride = j.bwd ? (size_t)j.rows * j.RS : (size_t)j.RS;
+    float v[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) v[e] = fabsf(w[e * stride]);
+    float lo = v[0], hi = v[0];
+#pragma unroll
+    for (int e = 1; e < 8; ++e) { lo = fminf(lo, v[e]); hi = fmaxf(hi, v[e]); }
+    if (hi > 0.0f) least = fminf(least, lo / hi);
+  }
+#pragma unroll
+  for (int d = 32; d > 0; d >>= 1) least = fminf(least, __shfl_xor(least, d));
+  if ((threadIdx.x & 63) == 0) wave_least[threadIdx.x >> 6] = __builtin_bit_cast(uint32_t, least);
+  __syncthreads();
+  if (threadIdx.x == 0) {
+#pragma unroll
+    for (int w = 1; w < 4; ++w) least = fminf(least, __builtin_bit_cast(float, wave_least[w]));
+    j.part[b] = least;
+  }
+}
+__global__ __launch_bounds__(256) void duo_max_kernel(DuoMaxJob a, DuoMaxJob b, DuoRatioJob c) {
   __shared__ uint32_t wave_top[4];
-  if ((int)blockIdx.x < a.blocks) duo_max_body(a, blockIdx.x, wave_top);
-  else duo_max_body(b, blockIdx.x - a.blocks, wave_top);
+  const int at = (int)blockIdx.x - a.blocks;
+  if (at < 0) duo_max_body(a, blockIdx.x, wave_top);
+  else if (at < b.blocks) duo_max_body(b, at, wave_top);
+  else duo_ratio_body(c, at - b.blocks, wave_top);
 }
 
-__device__ __forceinline__ void duo_store(uint4* dst, size_t at, size_t plane, const float (&v)[8], int e, float least) {
+template <class MARK>
+__device__ __forceinline__ int duo_store(uint4* dst, size_t at, size_t plane, const float (&v)[8], int e, MARK mark) {
   uint4 o[2];
-  duo_pack8(v, e, least, o);
-  dst[at] = o[0];
-  dst[at + plane] = o[1];
+  const int lost = duo_pack8(v, e, mark, o);
+#pragma unroll
+  for (int p = 0; p < 2; ++p) dst[at + p * plane] = o[p];
+  return lost;
 }
 
 // Filter copy, its rows' exponents and the table of the image's group offsets; tri_filter_body's items and order.
 struct DuoFilterArgs {
   const float* w; uint4* wt; int* soff;
-  const float* top; int* exps;   // of a row
+  const float* top; int *exps, *lost;   // of a row
   int groups, groups_true, rows, Ck, RS, S, Wp, bwd;
 };
 __device__ __forceinline__ void duo_filter_body(const DuoFilterArgs& a, long long i) {
@@ -107,7 +149,8 @@ __device__ __forceinline__ void duo_filter_body(const DuoFilterArgs& a, long lon
       v[e] = a.bwd ? a.w[((size_t)(c0 + e) * a.rows + row) * a.RS + (a.RS - 1 - rs)] : a.w[((size_t)row * a.Ck + c0 + e) * a.RS + rs];
   }
   const int e = duo_exponent(a.top[row]);
-  duo_store(a.wt, (size_t)i, (size_t)total, v, e, kDuoLeastSum);
+  const int lost = duo_store(a.wt, (size_t)i, (size_t)total, v, e, [](float, int) { return false; });
+  if (lost > 0) atomicAdd(a.lost + row, lost);
   if (g == 0) a.exps[row] = e;
   if (row == 0) {
     const int r = rs / a.S, s2 = rs - r * a.S;
@@ -120,7 +163,7 @@ __device__ __forceinline__ void duo_filter_body(const DuoFilterArgs& a, long lon
 __global__ __launch_bounds__(256) void duo_image_kernel(const float* __restrict__ x, uint4* __restrict__ xt, unsigned total, int H,
                                                         int W, FastDiv dWp, FastDiv dCg, FastDiv dHp, int halo, int img_blocks,
                                                         const float4* __restrict__ top, int parts, int* __restrict__ exps,
-                                                        DuoFilterArgs f) {
+                                                        const float4* __restrict__ ratio, DuoFilterArgs f) {
   if ((int)blockIdx.x >= img_blocks) {
     duo_filter_body(f, (long long)(blockIdx.x - img_blocks) * 256 + threadIdx.x);
     return;
@@ -149,7 +192,13 @@ __global__ __launch_bounds__(256) void duo_image_kernel(const float* __restrict_
     m = fmaxf(m, fmaxf(fmaxf(p.x, p.y), fmaxf(p.z, p.w)));
   }
   const int e = duo_exponent(m);
-  duo_store(xt, i, total, v, e, kDuoLeast);
+  duo_store(xt, i, total, v, e, [&](float most, int n) {
+    const float4* const r = ratio + (size_t)cg * (kDuoRatioParts / 4);
+    float least = 1.0f;
+#pragma unroll
+    for (int q = 0; q < kDuoRatioParts / 4; ++q) least = fminf(least, fminf(fminf(r[q].x, r[q].y), fminf(r[q].z, r[q].w)));
+    return !(most * least >= (float)n * kDuoBeside);
+  });
   if (wp == 0 && cg == 0 && hp == 0) exps[n] = e;
 }
 
@@ -211,7 +260,7 @@ __device__ __forceinline__ void duo_batch_body(const DuoBatchArgs& a, int b, flo
 #pragma unroll
     for (int n = 0; n < 8; ++n) v[n] = tile[n][cl][pl];
     if (a.sums) sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-    if (pix < a.HpWp && c < a.C) duo_store(a.xt, ((size_t)bz * a.HpWp + pix) * a.C + c, a.plane, v, ex, kDuoLeastSum);
+    if (pix < a.HpWp && c < a.C) duo_store(a.xt, ((size_t)bz * a.HpWp + pix) * a.C + c, a.plane, v, ex, [](float most, int) { return most < 5.820766091e-11f; });   // 2^-34
   }
   if (a.sums) {
     __syncthreads();
@@ -285,6 +334,9 @@ static double duo_run_us(const DuoRates& r, long long blocks, int steps) {
 static int duo_image_parts(int N) { return N >= 128 ? 8 : N >= 32 ? 16 : 32; }
 static int duo_channel_parts(int C) { const int p = round_up(cdiv(2048, C), 8); return p < 64 ? p : 64; }
 
+// Rows of a table that the tiles read whole.
+static int duo_rows(int rows) { return round_up(rows, 128); }
+
 // The constants are a fit to 1561 timed calls (12 layers at 10 batches, slices of 1 to 24 and tails of 2 to 6; rms error 6 %); the
 // slices chosen by it are 0.5 % slower than the best of them on average.
 static const DuoRates kDuo128 = {0.285, 2.4, 0.262, 0.7}, kDuo96 = {0.22, 10.2, 0.224, 0.9}, kDuo64 = {0.107, 6.9, 0.269, 0.6};
@@ -295,8 +347,8 @@ TriPlan plan_duo(int N, int Ci, int Hi, int Wi, int rows, int R, int S, int st, 
   p.Hp = Hi + 2 * halo; p.Wp = Wi + 2 * halo;
   p.groups_true = Ci / 8 * R * S;
   p.groups = round_up(p.groups_true, 2);
-  p.tab_bytes = align256(sizeof(int) * (size_t)p.groups) + align256(sizeof(int) * ((size_t)round_up(rows, 128) + N)) +
-                align256(sizeof(float) * ((size_t)N * duo_image_parts(N) + rows));
+  p.tab_bytes = align256(sizeof(int) * (size_t)p.groups) + align256(sizeof(int) * (2 * (size_t)duo_rows(rows) + N)) +
+                align256(sizeof(float) * ((size_t)N * duo_image_parts(N) + round_up(rows, 4) + Ci / 8 * kDuoRatioParts));
   const size_t w_part = 16 * (size_t)p.groups * rows, img_part = 2 * (size_t)N * Ci * p.Hp * p.Wp;
   if (2 * w_part > kMaxBufferBytes || 2 * img_part > kMaxBufferBytes) return p;
   p.wt_bytes = align256(2 * w_part);
@@ -343,10 +395,12 @@ int launch_conv_duo(const TriPlan& p, bool bwd, const float* in, const float* w,
   char* base = static_cast<char*>(ws);
   int* soff = reinterpret_cast<int*>(base);
   int* exps_a = reinterpret_cast<int*>(base + align256(sizeof(int) * (size_t)p.groups));
-  int* exps_b = exps_a + round_up(p.rows, 128);
-  float* top_b = reinterpret_cast<float*>(reinterpret_cast<char*>(exps_a) + align256(sizeof(int) * ((size_t)round_up(p.rows, 128) + p.N)));
+  int* lost = exps_a + duo_rows(p.rows);
+  int* exps_b = lost + duo_rows(p.rows);
+  float* top_b = reinterpret_cast<float*>(reinterpret_cast<char*>(exps_a) + align256(sizeof(int) * (2 * (size_t)duo_rows(p.rows) + p.N)));
   const int parts = duo_image_parts(p.N);
   float* top_a = top_b + (size_t)p.N * parts;
+  float* ratio = top_a + round_up(p.rows, 4);
   uint4* wt = reinterpret_cast<uint4*>(base + p.tab_bytes);
   uint4* xt = reinterpret_cast<uint4*>(base + p.tab_bytes + p.wt_bytes);
   float* part = reinterpret_cast<float*>(base + p.tab_bytes + p.wt_bytes + p.img_bytes);
@@ -354,32 +408,35 @@ int launch_conv_duo(const TriPlan& p, bool bwd, const float* in, const float* w,
   const int RS = p.R * p.S;
   {
     const DuoMaxJob ji = duo_max_job(in, top_b, 1, p.N, p.Ci * p.Hi * p.Wi, parts);
-    const DuoMaxJob jw = bwd ? duo_max_job(w, top_a, p.Ci, p.rows, RS, 1) : duo_max_job(w, top_a, 1, p.rows, p.Ci * RS, 1);
-    ProfScope prof("duo_max", 4.0 * ((double)p.N * p.Ci * p.Hi * p.Wi + (double)p.rows * p.Ci * RS), stream);
-    hipLaunchKernelGGL(duo_max_kernel, dim3((unsigned)(ji.blocks + jw.blocks)), dim3(256), 0, stream, ji, jw);
+    const DuoMaxJob jw = bwd ? duo_max_job(w, top_a, p.Ci, p.rows, RS, 1, lost, duo_rows(p.rows)) : duo_max_job(w, top_a, 1, p.rows, p.Ci * RS, 1, lost, duo_rows(p.rows));
+    DuoRatioJob jr;
+    jr.w = w; jr.part = ratio; jr.rows = p.rows; jr.Ck = p.Ci; jr.RS = RS; jr.bwd = bwd ? 1 : 0; jr.dRS = FastDiv((uint32_t)RS);
+    ProfScope prof("duo_max", 4.0 * ((double)p.N * p.Ci * p.Hi * p.Wi + 2.0 * p.rows * p.Ci * RS), stream);
+    hipLaunchKernelGGL(duo_max_kernel, dim3((unsigned)(ji.blocks + jw.blocks + p.Ci / 8 * kDuoRatioParts)), dim3(256), 0, stream, ji, jw, jr);
   }
   if (int e = launch_status()) return e;
   {
     DuoFilterArgs f;
-    f.w = w; f.wt = wt; f.soff = soff; f.top = top_a; f.exps = exps_a; f.groups = p.groups; f.groups_true = p.groups_true; f.rows = p.rows;
+    f.w = w; f.wt = wt; f.soff = soff; f.top = top_a; f.exps = exps_a; f.lost = lost; f.groups = p.groups; f.groups_true = p.groups_true; f.rows = p.rows;
     f.Ck = p.Ci; f.RS = RS; f.S = p.S; f.Wp = p.Wp; f.bwd = bwd ? 1 : 0;
     const unsigned img_blocks = (unsigned)cdiv<size_t>(img_groups, 256);
     ProfScope prof("duo_image", 4.0 * (double)p.N * p.Ci * p.Hi * p.Wi + 32.0 * (double)img_groups + 64.0 * (double)w_plane, stream);
     hipLaunchKernelGGL(duo_image_kernel, dim3(img_blocks + (unsigned)cdiv<size_t>(w_plane, 256)), dim3(256), 0, stream, in, xt,
                        (unsigned)img_groups, p.Hi, p.Wi, FastDiv((uint32_t)p.Wp), FastDiv((uint32_t)(p.Ci / 8)), FastDiv((uint32_t)p.Hp),
-                       p.halo, (int)img_blocks, reinterpret_cast<const float4*>(top_b), parts, exps_b, f);
+                       p.halo, (int)img_blocks, reinterpret_cast<const float4*>(top_b), parts, exps_b,
+                       reinterpret_cast<const float4*>(ratio), f);
   }
   if (int e = launch_status()) return e;
   DuoParams ap, bp;
   ap.t.v.ptr = wt; ap.t.plane = (int)(16 * w_plane); ap.t.v.bytes = (uint32_t)(32 * w_plane);
   ap.t.v.M = p.rows; ap.t.v.inner = 1; ap.t.v.innerW = 1; ap.t.v.img_stride = 16; ap.t.v.a_stride = 0; ap.t.v.b_stride = 0;
   ap.t.v.soff = nullptr; ap.t.v.group_stride = p.rows * 16;
-  ap.exps = exps_a; ap.ediv = 1; ap.emod = p.rows;
+  ap.exps = exps_a; ap.lost = lost; ap.ediv = 1; ap.emod = p.rows;
   bp.t.v.ptr = xt; bp.t.plane = (int)(16 * img_groups); bp.t.v.bytes = (uint32_t)(32 * img_groups);
   bp.t.v.M = p.N * p.P * p.Q; bp.t.v.inner = p.P * p.Q; bp.t.v.innerW = p.Q;
   bp.t.v.img_stride = p.Hp * p.Wp * p.Ci * 2; bp.t.v.a_stride = p.st * (p.Ci / 8) * p.Wp * 16; bp.t.v.b_stride = p.st * 16;
   bp.t.v.soff = soff; bp.t.v.group_stride = 0;
-  bp.exps = exps_b; bp.ediv = p.P * p.Q; bp.emod = p.N;
+  bp.exps = exps_b; bp.lost = nullptr; bp.ediv = p.P * p.Q; bp.emod = p.N;
   DuoSource src;
   src.pass = bwd ? RH_CONV_BWD_DATA : RH_CONV_FWD; src.a = w; src.b = in; src.N = p.N; src.C = p.Ci; src.H = p.Hi; src.W = p.Wi;
   src.rows = p.rows; src.R = p.R; src.S = p.S; src.st = p.st; src.halo = p.halo; src.P = p.P; src.Q = p.Q;
@@ -427,7 +484,7 @@ TriFilterPlan plan_duo_bwd_filter(const ConvDims& d) {
   p.groups = round_up(p.groups_true, 2);
   const size_t dy_part = 16 * (size_t)p.groups * d.K, x_part = 16 * (size_t)p.n8 * p.Hp * p.Wp * d.C;
   if (2 * dy_part > kMaxBufferBytes || 2 * x_part > kMaxBufferBytes) return p;
-  p.tab_bytes = align256(sizeof(int) * (size_t)p.groups) + align256(sizeof(int) * ((size_t)round_up(d.K, 128) + d.C)) +
+  p.tab_bytes = align256(sizeof(int) * (size_t)p.groups) + align256(sizeof(int) * (2 * (size_t)duo_rows(d.K) + d.C)) +
                 align256(sizeof(float) * ((size_t)d.K * duo_channel_parts(d.K) + (size_t)d.C * duo_channel_parts(d.C)));
   p.dyt_bytes = align256(2 * dy_part);
   p.xt_bytes = align256(2 * x_part);
@@ -457,8 +514,9 @@ int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const 
   char* base = static_cast<char*>(ws);
   int* soff = reinterpret_cast<int*>(base);
   int* exps_a = reinterpret_cast<int*>(base + align256(sizeof(int) * (size_t)p.groups));
-  int* exps_b = exps_a + round_up(d.K, 128);
-  float* top_a = reinterpret_cast<float*>(reinterpret_cast<char*>(exps_a) + align256(sizeof(int) * ((size_t)round_up(d.K, 128) + d.C)));
+  int* lost = exps_a + duo_rows(d.K);
+  int* exps_b = lost + duo_rows(d.K);
+  float* top_a = reinterpret_cast<float*>(reinterpret_cast<char*>(exps_a) + align256(sizeof(int) * (2 * (size_t)duo_rows(d.K) + d.C)));
   const int parts_a = duo_channel_parts(d.K), parts_b = duo_channel_parts(d.C);
   float* top_b = top_a + (size_t)d.K * parts_a;
   uint4* dyt = reinterpret_cast<uint4*>(base + p.tab_bytes);
@@ -466,9 +524,9 @@ int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const 
   *parts = reinterpret_cast<float*>(base + p.tab_bytes + p.dyt_bytes + p.xt_bytes);
   const size_t dy_plane = (size_t)p.groups * d.K, x_plane = (size_t)p.n8 * p.Hp * p.Wp * d.C;
   {
-    const DuoMaxJob ja = duo_max_job(dy, top_a, d.N, d.K, d.P * d.Q, parts_a), jb = duo_max_job(x, top_b, d.N, d.C, d.H * d.W, parts_b);
+    const DuoMaxJob ja = duo_max_job(dy, top_a, d.N, d.K, d.P * d.Q, parts_a, lost, duo_rows(d.K)), jb = duo_max_job(x, top_b, d.N, d.C, d.H * d.W, parts_b);
     ProfScope prof("duo_max", 4.0 * (double)(d.y_elems + d.x_elems), stream);
-    hipLaunchKernelGGL(duo_max_kernel, dim3((unsigned)(ja.blocks + jb.blocks)), dim3(256), 0, stream, ja, jb);
+    hipLaunchKernelGGL(duo_max_kernel, dim3((unsigned)(ja.blocks + jb.blocks)), dim3(256), 0, stream, ja, jb, DuoRatioJob{});
   }
   if (int e = launch_status()) return e;
   {
@@ -489,12 +547,12 @@ int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const 
   ap.t.v.ptr = dyt; ap.t.plane = (int)(16 * dy_plane); ap.t.v.bytes = (uint32_t)(32 * dy_plane);
   ap.t.v.M = d.K; ap.t.v.inner = 1; ap.t.v.innerW = 1; ap.t.v.img_stride = 16; ap.t.v.a_stride = 0; ap.t.v.b_stride = 0;
   ap.t.v.soff = nullptr; ap.t.v.group_stride = d.K * 16;
-  ap.exps = exps_a; ap.ediv = 1; ap.emod = d.K;
+  ap.exps = exps_a; ap.lost = lost; ap.ediv = 1; ap.emod = d.K;
   bp.t.v.ptr = xt; bp.t.plane = (int)(16 * x_plane); bp.t.v.bytes = (uint32_t)(32 * x_plane);
   bp.t.v.M = CRS; bp.t.v.inner = d.S * d.C; bp.t.v.innerW = d.C;   // columns j = (r, s, c)
   bp.t.v.img_stride = p.Wp * d.C * 16; bp.t.v.a_stride = d.C * 16; bp.t.v.b_stride = 16;
   bp.t.v.soff = soff; bp.t.v.group_stride = 0;
-  bp.exps = exps_b; bp.ediv = 1; bp.emod = d.C;
+  bp.exps = exps_b; bp.lost = nullptr; bp.ediv = 1; bp.emod = d.C;
   DuoSource src;
   src.pass = RH_CONV_BWD_FILTER; src.a = dy; src.b = x; src.N = d.N; src.C = d.C; src.H = d.H; src.W = d.W;
   src.rows = d.K; src.R = d.R; src.S = d.S; src.st = d.st; src.halo = d.pad; src.P = d.P; src.Q = d.Q;

@@ -14,9 +14,17 @@
 // 3.5e-7.  So it is for long contractions (duo_replaces, conv_common.h).  KEEP costs 5 % of the kernel's time and takes the data
 // gradient of AlexNet's conv5, whose deltas are zeros for the most part, from 1.21 to 0.94e-7 (three parts 1.04).
 //
-// Range.  A value keeps its 22 bits down to 2^-29 of the largest of its row; below that its error is 2^-51 of that largest value.  A
-// group of eight values without a larger one, and values that are no finite numbers, are marked by a NaN in the first part, and a
-// result that is not finite is formed again from the operands themselves on the fp32 instruction (tri_redo).
+// Range.  A value keeps its 22 bits down to 2^-29 of the largest of its row; below that a product with b loses up to 2^-35 b (scaled).  A
+// result in which that could be seen is not finite and formed again from the operands themselves on the fp32 instruction (tri_redo), as
+// is one with an operand that is no finite number.
+// * An image's small value is marked by a NaN in the first part, unless the other seven of its group (eight channels of a pixel, which
+//   every result with one of them has, met by eight channels of one tap of a filter) make up for it: ratio is the least one, over the
+//   filters, of a value to the largest of its group, so if the group's largest, times it, is n 2^-14 at least, there is a product of
+//   n 2^-14 b beside the n 2^-35 b that n small values lose.  Of AlexNet's, NIN's and ResNet-18's activations none was marked, nor of
+//   AlexNet's and NIN's deltas.  Behind a batch norm all deltas are small beside the few that a ReLU let through: in ResNet-18 up to 1250 of a
+//   tensor are under 2^-29 and of four tensors of 13 some are marked; there the operators ask for three parts.
+// * A filter's small values (one in 1e8 of normal weights) are counted.  They cost a result 2^-20 each at most, so its sum, before it is
+//   scaled back, has to be four times their number: 2^27 is usual.  (A mark would have the filter's whole plane formed again.)
 #pragma once
 #include "gemm_tri.h"
 
@@ -27,6 +35,7 @@ typedef __attribute__((ext_vector_type(2))) _Float16 f16x2_t;
 
 constexpr int kDuoChain = 8;         // K steps in a chain of large products (even)
 constexpr float kDuoLow = 2048.0f;   // the second part is held 2^11 times as large
+constexpr float kDuoBeside = 6.103515625e-5f;   // 2^-14
 
 // The exponent for a row whose largest finite magnitude is `top`.
 __device__ __forceinline__ int duo_exponent(float top) {
@@ -34,32 +43,44 @@ __device__ __forceinline__ int duo_exponent(float top) {
   return 141 - (e > 0 ? e : 1);
 }
 
-// Eight values (one group) of a row with exponent e.  A group whose largest scaled value is under `least` is marked.
-constexpr float kDuoLeast = 6.103515625e-5f;        // 2^-14: from here on the two parts hold 22 bits
-constexpr float kDuoLeastSum = 5.820766091e-11f;    // 2^-34: from here on they hold two
-__device__ __forceinline__ void duo_pack8(const float (&v)[8], int e, float least, uint4 (&o)[2]) {
+// The bits of the smallest magnitude, in a row with exponent e, of which two parts hold 22 bits: 2^-14 scaled.
+__device__ __forceinline__ uint32_t duo_least(int e) {
+  const int b = 113 - e;
+  return b > 0 ? (uint32_t)b << 23 : b > -23 ? 1u << (22 + b) : 0u;
+}
+
+// Eight values (one group) of a row with exponent e; returns how many of them, not 0, are under duo_least.  mark(most, n) says whether
+// those n are marked, most being the group's largest scaled value.
+template <class MARK>
+__device__ __forceinline__ int duo_pack8(const float (&v)[8], int e, MARK mark, uint4 (&o)[2]) {
   uint32_t w[2][4];
-  uint32_t top = 0, any = 0;
+  uint32_t top = 0, low = 0xffffffffu;   // the largest magnitude, and one under the smallest that is not 0
 #pragma unroll
   for (int i = 0; i < 4; ++i) {
-    any |= (__builtin_bit_cast(uint32_t, v[2 * i]) | __builtin_bit_cast(uint32_t, v[2 * i + 1])) << 1;   // (scaled, a value may be 0)
     const float x = __builtin_amdgcn_ldexpf(v[2 * i], e), y = __builtin_amdgcn_ldexpf(v[2 * i + 1], e);
     const f16x2_t h = {(_Float16)x, (_Float16)y};
     const f16x2_t l = {(_Float16)((x - (float)h.x) * kDuoLow), (_Float16)((y - (float)h.y) * kDuoLow)};
     w[0][i] = __builtin_bit_cast(uint32_t, h);
     w[1][i] = __builtin_bit_cast(uint32_t, l);
-    const uint32_t mx = __builtin_bit_cast(uint32_t, x) & 0x7fffffffu, my = __builtin_bit_cast(uint32_t, y) & 0x7fffffffu;
-    top = mx > top ? mx : top;
-    top = my > top ? my : top;
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+      const uint32_t bits = __builtin_bit_cast(uint32_t, v[2 * i + k]) & 0x7fffffffu;
+      top = bits > top ? bits : top;
+      low = bits - 1u < low ? bits - 1u : low;
+    }
   }
-  const bool tiny = any != 0 && top < __builtin_bit_cast(uint32_t, least);
-  if (tiny || top >= 0x7f800000u) {
+  const uint32_t least = duo_least(e), under = least > 0 ? least - 1u : 0u;
+  int lost = 0;
+  if ((low < under) | (top >= 0x7f800000u)) {
+#pragma unroll
+    for (int i = 0; i < 8; ++i) lost += (__builtin_bit_cast(uint32_t, v[i]) & 0x7fffffffu) - 1u < under;
+    const bool small = mark(__builtin_amdgcn_ldexpf(__builtin_bit_cast(float, top), e), lost);
 #pragma unroll
     for (int i = 0; i < 4; ++i) {
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const uint32_t bits = __builtin_bit_cast(uint32_t, v[2 * i + h]) & 0x7fffffffu;
-        if (bits >= 0x7f800000u || (tiny && bits != 0)) {
+        if (bits >= 0x7f800000u || (small && bits - 1u < under)) {
           const uint32_t keep = h ? 0xffffu : 0xffff0000u;
           w[0][i] = (w[0][i] & keep) | (0x7e00u << (16 * h));
           w[1][i] &= keep;
@@ -69,12 +90,14 @@ __device__ __forceinline__ void duo_pack8(const float (&v)[8], int e, float leas
   }
 #pragma unroll
   for (int p = 0; p < 2; ++p) o[p] = make_uint4(w[p][0], w[p][1], w[p][2], w[p][3]);
+  return lost;
 }
 
-// An operand of this form: TriParams with two parts, and the exponents of its rows: row m has exps[m / ediv % emod].
+// An operand of this form: TriParams with two parts, the exponents of its rows: row m has exps[m / ediv % emod], and the counts of their
+// small values (of A).
 struct DuoParams {
   TriParams t;
-  const int* exps;
+  const int *exps, *lost;
   int ediv, emod;
 };
 
@@ -245,9 +268,14 @@ __device__ __forceinline__ void duo_block(const DuoParams& ap, const DuoParams& 
 #pragma unroll
       for (int i = 0; i < Loader::CNT; ++i) ld.issue(lds0 + (uint32_t)(s * (SA + SB)) * 16u, i);
     }
+  int lost_here = 0;   // small values in a row of the wave's (looked at once the first steps have landed)
+#pragma unroll
+  for (int r = 0; r < TM * 32; r += 64)
+    if (r + lane < TM * 32) lost_here |= ap.lost[m0 + wm * (TM * 32) + r + lane];
   ld.prep(s_begin + (R - 1 < nk ? R - 1 : nk - 1));
   wait_vmcnt<0>();
   __syncthreads();
+  const bool any_lost = __any(lost_here != 0);
 
   const uint4* const pa0 = sm + (lane >> 5) * RA + wm * (TM * 32) + (lane & 31);
   const uint4* const pb0 = sm + SA + (lane >> 5) * RBn + wn * (TN * 32) + (lane & 31);
@@ -350,6 +378,18 @@ __device__ __forceinline__ void duo_block(const DuoParams& ap, const DuoParams& 
     step(it++, c0, no, no);
     if (it >= nk) break;
     step(it++, c1, no, no);
+  }
+
+  if (any_lost) {   // (sums in which small values could be seen)
+#pragma unroll
+    for (int i = 0; i < TM; ++i)
+#pragma unroll
+      for (int v = 0; v < 16; ++v) {
+        const float least = 4.0f * (float)ap.lost[m0 + wm * (TM * 32) + i * 32 + (lane >> 5) * 4 + (v >> 2) * 8 + (v & 3)];
+#pragma unroll
+        for (int j = 0; j < TN; ++j)
+          if (fabsf(sum[i][j][v] + fmaf(low[i][j][v], 1.0f / kDuoLow, acc[i][j][v])) < least) sum[i][j][v] = __builtin_nanf("");
+      }
   }
 
   // the sums, scaled back by the row's and the column's exponent

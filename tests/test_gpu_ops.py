@@ -867,6 +867,46 @@ def test_conv2d_f16x2_values_out_of_range(dev):
     assert np.array_equal(got[0], np.broadcast_to(x[0, 3], (64, 1, 8)))
 
 
+def _f16x2_range_passes(dev, algo):
+    """name, run(filter, input), the same by the oracle, for the two passes whose operands share groups of eight channels: stride 1, extents kept."""
+    pad = lambda w: w.shape[2] // 2
+    yield "fwd", lambda w, x: N(ops.conv2d_fwd(T(x, dev), T(w, dev), 1, pad(w), algo=algo)), lambda w, x: O.conv2d_fwd(x, w, 1, pad(w))
+    flip = lambda w: np.ascontiguousarray(w.transpose(1, 0, 2, 3))   # contracted: the filters
+    shape = lambda w, x: (len(x), len(w)) + x.shape[2:]
+    yield ("bwd data", lambda w, x: N(ops.conv2d_bwd_data(T(flip(w), dev), T(x, dev), shape(w, x), 1, pad(w), algo=algo)),
+           lambda w, x: O.conv2d_bwd_data(flip(w), x, shape(w, x), 1, pad(w)))
+
+
+@pytest.mark.parametrize("k", [20, 29, 31, 36, 45, 52, 80, 120])
+def test_conv2d_f16x2_small_values_beside_large_ones(dev, k):
+    """Every channel but the eighth of each group 2^-k as large, in the input where the eighth's weight is 0 and in the filter where the
+    eighth's input is: the result is of the small values alone, and has the bits of any other.  16 x 9 products of relative error 2^-21 at
+    most each, and sums of a hundred roundings of 2^-24 at most: 2^-18 of the sum of magnitudes."""
+    say("f16x2 small beside large", k)
+    x0, w0 = synth.normal(40, 1, (3, 16, 7, 6)), 0.1 * synth.normal(40, 2, (70, 16, 3, 3))
+    eighth = np.arange(16) % 8 == 7
+    for small, other in ((0, 1), (1, 0)):
+        pair = [x0.copy(), w0.copy()]
+        pair[small][:, ~eighth] *= np.float32(2.0) ** -k
+        pair[other][:, eighth] = 0.0
+        x, w = pair
+        for name, run, ref in _f16x2_range_passes(dev, _lib.RH_ALGO_F16X2 | _lib.RH_ALGO_DIRECT):
+            got, want, size = run(w, x), ref(w, x), ref(np.abs(w), np.abs(x))
+            assert np.all(np.abs(got.astype(np.float64) - want) <= 2.0 ** -18 * size), (name, small)
+
+
+def test_conv2d_f16x2_values_of_all_sizes(dev):
+    """Values of every size beside one another, zeros among them: each result as exact against the sum of its products' magnitudes."""
+    say("f16x2 all sizes")
+    x, w = synth.normal(41, 1, (5, 8, 17, 16)), synth.normal(41, 2, (136, 8, 1, 1))
+    x *= np.float32(2.0) ** -np.floor(50 * synth.uniform(41, 3, x.shape)) * (synth.uniform(41, 4, x.shape) < 0.7)
+    for spread, zeros in ((0, 0.0), (12, 0.0), (12, 0.6), (50, 0.6)):
+        ww = w * np.float32(2.0) ** -np.floor(spread * synth.uniform(41, 5, w.shape)) * (synth.uniform(41, 6, w.shape) >= zeros)
+        for name, run, ref in _f16x2_range_passes(dev, _lib.RH_ALGO_F16X2 | _lib.RH_ALGO_DIRECT):
+            got, want, size = run(ww, x), ref(ww, x), ref(np.abs(ww), np.abs(x))
+            assert np.all(np.abs(got.astype(np.float64) - want) <= 2.0 ** -20 * size), (name, spread, zeros)
+
+
 @pytest.mark.parametrize("case", [(90, 256, 14, 256, 3, 1), (24, 512, 7, 512, 3, 1)], ids=str)
 def test_conv2d_f16x2_deltas_behind_a_batch_norm(dev, case):
     """A filter gradient whose caller sets RH_ALGO_BF16X3_WIDE stays with three parts."""
