@@ -25,6 +25,10 @@
 //   tensor are under 2^-29 and of four tensors of 13 some are marked; there the operators ask for three parts.
 // * A filter's small values (one in 1e8 of normal weights) are counted.  They cost a result 2^-20 each at most, so its sum, before it is
 //   scaled back, has to be four times their number: 2^27 is usual.  (A mark would have the filter's whole plane formed again.)
+//   Formed again, a block of 32 x 32 results is bound by the latency of its loads, 32 of them in flight (one by one 384 -> 384 3x3 13x13
+//   b256 forward took 3.0 ms longer for one value): 330 us, with one value in x 930, with one in every group 3.9 ms (three parts 550 us,
+//   1.4 and 2.9 ms); 5x5 of 96 channels 0.6, 0.9 and 12 ms, 1x1 at 128 images 54, 93 and 260 us.  In the filter gradient, whose loads are
+//   of 32 channels a plane apart, 350 us, 3.9 and 9.3 ms.
 #pragma once
 #include "gemm_tri.h"
 
@@ -107,39 +111,39 @@ struct DuoSource {
   const float *a, *b;       // forward: filter, image; backward-data: filter, dy; backward-filter: dy, image
   int N, C, H, W;           // of the tensor b
   int rows, R, S, st, halo, P, Q;
+  // eight values `stride` floats apart, the first n of them there
+  static __device__ __forceinline__ void load8(const float* p, size_t stride, int n, float (&v)[8]) {
+#pragma unroll
+    for (int e = 0; e < 8; ++e) {
+      const float x = p[e < n ? e * stride : 0];
+      v[e] = e < n ? x : 0.0f;
+    }
+  }
   // row, or column, m of the operand; its eight values of group g
   __device__ __forceinline__ void load_a(int m, int g, float (&v)[8]) const {
     if (pass == RH_CONV_BWD_FILTER) {
       const int PQ = P * Q, n8 = g / PQ, pq = g - n8 * PQ;
-#pragma unroll 1
-      for (int e = 0; e < 8; ++e)
-        if (n8 * 8 + e < N) v[e] = a[((size_t)(n8 * 8 + e) * rows + m) * PQ + pq];
-      return;
+      return load8(a + ((size_t)n8 * 8 * rows + m) * PQ + pq, (size_t)rows * PQ, N - n8 * 8, v);
     }
     int rs, c0;
     tap(g, rs, c0);
     const int RS = R * S;
-#pragma unroll 1
-    for (int e = 0; e < 8; ++e)
-      v[e] = pass == RH_CONV_BWD_DATA ? a[((size_t)(c0 + e) * rows + m) * RS + (RS - 1 - rs)] : a[((size_t)m * C + c0 + e) * RS + rs];
+    if (pass == RH_CONV_BWD_DATA) load8(a + ((size_t)c0 * rows + m) * RS + (RS - 1 - rs), (size_t)rows * RS, 8, v);
+    else load8(a + ((size_t)m * C + c0) * RS + rs, RS, 8, v);
   }
   __device__ __forceinline__ void load_b(int m, int g, float (&v)[8]) const {
     if (pass == RH_CONV_BWD_FILTER) {   // m = (r, s, c)
       const int PQ = P * Q, n8 = g / PQ, pq = g - n8 * PQ, p = pq / Q, q = pq - p * Q;
       const int rs = m / C, c = m - rs * C, r = rs / S, h = p * st + r - halo, w = q * st + (rs - r * S) - halo;
       if ((unsigned)h >= (unsigned)H || (unsigned)w >= (unsigned)W) return;
-#pragma unroll 1
-      for (int e = 0; e < 8; ++e)
-        if (n8 * 8 + e < N) v[e] = b[((size_t)((n8 * 8 + e) * C + c) * H + h) * W + w];
-      return;
+      return load8(b + (((size_t)n8 * 8 * C + c) * H + h) * W + w, (size_t)C * H * W, N - n8 * 8, v);
     }
     int rs, c0;
     tap(g, rs, c0);
     const int PQ = P * Q, n = m / PQ, pq = m - n * PQ, p = pq / Q, q = pq - p * Q, r = rs / S;
     const int h = p * st + r - halo, w = q * st + (rs - r * S) - halo;
     if (n >= N || (unsigned)h >= (unsigned)H || (unsigned)w >= (unsigned)W) return;
-#pragma unroll 1
-    for (int e = 0; e < 8; ++e) v[e] = b[((size_t)(n * C + c0 + e) * H + h) * W + w];
+    load8(b + (((size_t)n * C + c0) * H + h) * W + w, (size_t)H * W, 8, v);
   }
   // the tap and the first channel of group g (tri_filter_body's order)
   __device__ __forceinline__ void tap(int g, int& rs, int& c0) const {

@@ -167,9 +167,9 @@ struct DmaTri {
 // The block d of 32 x 32 results with its elements that are not finite and lie in the result formed again over groups
 // [g0, g1) on the fp32 instruction: load_a(g, v) and load_b(g, v) give this lane's row (lane % 32) and column their eight values of
 // group g.  Two levels of sums, 128 terms each, as the chains of K steps may be longer than fp32's rounding allows.  The whole wave
-// takes part whether one element or all of them are formed.  Bound by the latency of its own loads: 2 us for 16 k of a block, so a call
-// with one such value takes 80 to 470 us longer, one with nothing else 4 to 8 times as long (96 -> 256 5x5 27x27 b256 forward 967 us,
-// with one such value 1197, with nothing else 5150).
+// takes part whether one element or all of them are formed.  Bound by the latency of its own loads, so a call with one such value takes
+// 50 to 1100 us longer, one with one in every group 3 to 8 times as long (96 -> 256 5x5 27x27 b256 forward 1000 us, with one such value
+// 1180, with one in every group 5190).
 template <class LA, class LB>
 __device__ __forceinline__ void tri_redo(f32x16& d, int rows_left, int cols_left, int lane, int g0, int g1, LA load_a, LB load_b) {
   bool any = false;
@@ -188,17 +188,22 @@ __device__ __forceinline__ void tri_redo(f32x16& d, int rows_left, int cols_left
 #pragma unroll
     for (int v = 0; v < 16; ++v) part[v] = 0.0f;
 #pragma unroll 1
-    for (int g = top; g < top + 16 && g < g1; g += 2) {
-      const int mine = g + (lane >> 5);   // k 0 and 1 of an MFMA: of this group and of the next
-      float a[8], b[8];
+    for (int g = top; g < top + 16 && g < g1; g += 4) {   // (the loads of four groups in flight)
+      float a[2][8], b[2][8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e) a[e] = b[e] = 0.0f;
-      if (mine < g1) {
-        load_a(mine, a);
-        load_b(mine, b);
+      for (int u = 0; u < 2; ++u) {
+        const int mine = g + 2 * u + (lane >> 5);   // k 0 and 1 of an MFMA: of this group and of the next
+#pragma unroll
+        for (int e = 0; e < 8; ++e) a[u][e] = b[u][e] = 0.0f;
+        if (mine < g1) {
+          load_a(mine, a[u]);
+          load_b(mine, b[u]);
+        }
       }
 #pragma unroll
-      for (int e = 0; e < 8; ++e) part = __builtin_amdgcn_mfma_f32_32x32x2f32(a[e], b[e], part, 0, 0, 0);
+      for (int u = 0; u < 2; ++u)
+#pragma unroll
+        for (int e = 0; e < 8; ++e) part = __builtin_amdgcn_mfma_f32_32x32x2f32(a[u][e], b[u][e], part, 0, 0, 0);
     }
     sum += part;
   }
