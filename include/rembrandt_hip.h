@@ -88,12 +88,15 @@ typedef void* rh_stream_t; /* hipStream_t */
                                              fp32 accumulate in short chains).  The power is one for a filter and one for an
                                              image, in the filter gradient one for a channel of either operand.  Two parts
                                              hold a value to 2^-23 of itself down to 2^-29 of the largest of its filter, image
-                                             or channel, and to 2^-51 of that largest value below; results with an operand
-                                             that has no larger one beside it in a group of eight (2^-49 for filters and in the
-                                             filter gradient), an infinity or a NaN are formed on fp32 instructions, as with
-                                             RH_ALGO_BF16X3.  With or without that bit, with the hint or without: where it is
-                                             expected to be the fastest form, its error against 64-bit sums no larger than that
-                                             of the form it replaces, and the scratch holds it.  With RH_ALGO_DIRECT and without
+                                             or channel, and to 2^-51 of that largest value below.  A result to which that could
+                                             matter (2^-21 of the sum of its products' magnitudes), or with an infinity or a NaN
+                                             among its operands, is formed on fp32 instructions, as with RH_ALGO_BF16X3; with
+                                             that bit too, a filter gradient with such values is formed in three parts.  With or
+                                             without that bit, with the hint or without: where it is expected to be the fastest
+                                             form and, for N(0,1) operands with up to 19 in 20 of them zeros, no further from
+                                             64-bit sums than the form it replaces, and the scratch holds it.  (Sums of few
+                                             products, of operands that are zeros almost everywhere, have up to 1.2e-7 where
+                                             three parts have 0.3e-7.)  With RH_ALGO_DIRECT and without
                                              RH_ALGO_BF16X3: this form, RH_E_UNSUPPORTED where the geometry has none (as there;
                                              a stride in backward-data has none).  rh_conv2d_workspace_bytes_for says what it
                                              needs.  No effect beside the other RH_ALGO_* bits and RH_MATH_BF16_MFMA_FP32ACC. */

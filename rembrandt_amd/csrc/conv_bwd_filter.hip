@@ -411,20 +411,31 @@ SplitFilterPick pick_split_bwd_filter(const ConvDims& d, int flags, size_t ws_by
   if (!tri_allowed(flags) && !duo) return s;
   const TriRival other = filter_rival(d);
   double us = other.us, err = 0.2 * other.err;
+  TriFilterPlan three = {};
   if (tri_allowed(flags)) {
     const TriFilterPlan p = plan_tri_bwd_filter(d, tri_wide(flags));
     const int chain = p.ok ? cdiv(p.groups / 2, p.splits) : 0;
-    if (p.ok && p.us < other.us && chain <= tri_max_chain(other.err) && p.total() <= ws_bytes) {
-      s = SplitFilterPick{3, p};
+    if (p.ok && chain <= tri_max_chain(other.err)) three = p;
+    if (three.ok && p.us < other.us && p.total() <= ws_bytes) {
+      s = SplitFilterPick{3, p, {}};
       us = p.us;
       err = 0.005 * chain + 0.016 * p.splits;
       if (need && p.total() > *need) *need = p.total();
     }
   }
   if (duo) {
-    const TriFilterPlan p = plan_duo_bwd_filter(d);
-    if (p.total() <= ws_bytes && duo_filter_pays(p, us, err)) {
-      s = SplitFilterPick{2, p};
+    // (two parts and, in the same scratch, three, for the calls whose values two cannot hold: deltas of samples that the network is sure of
+    // may be 1e-9 of the others, and where those meet zeros the gradient is of the small ones alone.  Which it is the blocks look
+    // up on the device)
+    TriFilterPlan p = plan_duo_bwd_filter(d);
+    if (p.ok && three.ok) {
+      const size_t copies = std::max(p.dyt_bytes + p.xt_bytes, three.tab_bytes + three.dyt_bytes + three.xt_bytes);
+      p.xt_bytes = copies - p.dyt_bytes;
+      three.xt_bytes = copies - three.tab_bytes - three.dyt_bytes;
+      p.part_bytes = std::max(p.part_bytes, three.part_bytes);
+    }
+    if ((three.ok || !tri_allowed(flags)) && p.total() <= ws_bytes && duo_filter_pays(p, us, err)) {
+      s = SplitFilterPick{2, p, three};
       if (need && p.total() > *need) *need = p.total();
     }
   }
@@ -666,6 +677,7 @@ __global__ __launch_bounds__(256) void bwd_filter_prep_kernel(NhwcCopyArgs dy, f
 // slices 26 and 10.4; of 16 layers that come here 13.7 and 7.6 in the geometric mean, none slower.
 struct TapsArgs {
   const float* part; float* dw;
+  OrThree or_three;
   int splits, K, C, RS, CH, TS, G;
   int c_chunks, chunks;      // of a filter: along c, in all
   unsigned units, work;      // of a block: reads of a slab, of all groups
@@ -678,6 +690,7 @@ __global__ __launch_bounds__(256) void split_reduce_taps_kernel(TapsArgs a, Bias
   if (bj.db && blockIdx.x >= bj.first) { bias_job_block(bj, blockIdx.x - bj.first); return; }
   constexpr int E = sizeof(V) / 4;
   extern __shared__ float lds[];   // [group][tap][CH + 1]
+  const int splits = a.or_three.any && *a.or_three.any != 0 ? a.or_three.splits : a.splits;
   const int ko = (int)blockIdx.x / a.chunks, chunk = (int)blockIdx.x - ko * a.chunks;
   const int rs0 = chunk / a.c_chunks * a.TS, c0 = chunk % a.c_chunks * a.CH;
   const int taps = min(a.TS, a.RS - rs0), chans = min(a.CH, a.C - c0);
@@ -700,11 +713,11 @@ __global__ __launch_bounds__(256) void split_reduce_taps_kernel(TapsArgs a, Bias
       for (int e = 0; e < E; ++e) d[e] += reinterpret_cast<const float*>(&v)[e];
     };
     int sp = (int)g;
-    for (; sp + 3 * a.G < a.splits; sp += 4 * a.G) {
+    for (; sp + 3 * a.G < splits; sp += 4 * a.G) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) add(x[i], sp + i * a.G);
     }
-    for (; sp < a.splits; sp += a.G) add(x[0], sp);
+    for (; sp < splits; sp += a.G) add(x[0], sp);
     float* const d = lds + ((int)g * a.TS + (int)t) * (a.CH + 1) + (int)c * E;
 #pragma unroll
     for (int e = 0; e < E; ++e) d[e] = (x[0][e] + x[1][e]) + (x[2][e] + x[3][e]);
@@ -727,10 +740,10 @@ __global__ __launch_bounds__(256) void split_reduce_taps_kernel(TapsArgs a, Bias
 
 // 1024 values to a block, or fewer where that leaves CUs idle, down to 64 bytes a read of a slab.
 static void launch_split_reduce_taps(const float* part, int splits, float* dw, int K, int C, int RS, float alpha, float beta, BiasJob bj,
-                                     hipStream_t stream) {
+                                     hipStream_t stream, const OrThree& or_three) {
   const bool vec = C % 4 == 0 && (reinterpret_cast<uintptr_t>(part) & 15) == 0;
   TapsArgs a;
-  a.part = part; a.dw = dw; a.splits = splits; a.K = K; a.C = C; a.RS = RS; a.alpha = alpha; a.beta = beta;
+  a.part = part; a.dw = dw; a.or_three = or_three; a.splits = splits; a.K = K; a.C = C; a.RS = RS; a.alpha = alpha; a.beta = beta;
   int want = cdiv(C * RS, 1024);
   if (want < cdiv(512, K)) want = cdiv(512, K);
   a.CH = min(C, max(16, round_up(cdiv(C, want), 4)));
@@ -1001,7 +1014,7 @@ static size_t split_scratch(const ConvDims& d, int pass, int flags, size_t floor
   if (pass == RH_CONV_BWD_FILTER) {
     const double copies = 6.0 * round_up(d.N, 8) * ((double)d.K * (d.P * d.Q + 1) + (double)d.C * (d.H + 2 * d.pad) * (d.W + 2 * d.pad));
     const double slices = fmax(4.0 * (double)d.w_elems, fmin(256e6, 2048.0 * 4 * 128 * 128));
-    const double rest = (double)cdiv(d.N, 8) * 4.0 * (d.P * d.Q + (double)d.K * (d.P * d.Q / 32 + 1)) + 64.0 * (d.K + d.C) + 65536.0;
+    const double rest = (double)cdiv(d.N, 8) * 4.0 * (2.0 * d.P * d.Q + (double)d.K * (d.P * d.Q / 32 + 1)) + 64.0 * (d.K + d.C) + 65536.0;
     if (copies + slices + rest < (double)floor) return 0;
     size_t need = 0;
     pick_split_bwd_filter(d, flags, ~size_t(0), &need);
@@ -1091,13 +1104,13 @@ static int bwd_filter_impl(const rh_conv_geom* g, float alpha, const float* x, c
     return RH_E_WORKSPACE;
   hipStream_t stream = to_stream(stream_);
   // dw from `used` slices in (ko, r, s, c) order
-  auto reduce_rsc = [&](float* parts, int used) -> int {
+  auto reduce_rsc = [&](float* parts, int used, const OrThree& or_three = OrThree{}) -> int {
     const long long total = (long long)d.K * d.C * d.R * d.S;
     BiasJob bj;
     bias_job(&bj);
     const unsigned jb = bj.blocks();
     ProfScope prof("split_reduce", 4.0 * (double)total * (used + 1) + (jb ? 4.0 * (double)bj.N * bj.K * bj.plane : 0.0), stream);
-    launch_split_reduce_taps(parts, used, dw, d.K, d.C, d.R * d.S, alpha, beta, bj, stream);
+    launch_split_reduce_taps(parts, used, dw, d.K, d.C, d.R * d.S, alpha, beta, bj, stream, or_three);
     return launch_status();
   };
 
@@ -1115,8 +1128,11 @@ static int bwd_filter_impl(const rh_conv_geom* g, float alpha, const float* x, c
       bf->rows = tp.sum_rows;
       bf->folded = true;
     }
-    if (int e = (split.parts == 3 ? launch_conv_tri_bwd_filter : launch_conv_duo_bwd_filter)(d, tp, x, dy, sums, ws, stream, &parts, &used)) return e;
-    return reduce_rsc(parts, used);
+    OrThree or_three = {};
+    const int e = split.parts == 3 ? launch_conv_tri_bwd_filter(d, tp, x, dy, sums, ws, stream, &parts, &used)
+                                   : launch_conv_duo_bwd_filter(d, tp, x, dy, sums, ws, stream, &parts, &used,
+                                                                split.or_three.ok ? &split.or_three : nullptr, &or_three);
+    return e ? e : reduce_rsc(parts, used, or_three);
   }
   if ((flags & RH_ALGO_WINOGRAD) && (!wino_shape(d) || (flags & (RH_ALGO_GATHER | RH_ALGO_SCALAR_OFFSET | RH_ALGO_DIRECT))))
     return RH_E_UNSUPPORTED;

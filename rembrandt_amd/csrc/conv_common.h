@@ -629,8 +629,11 @@ TriFilterPlan plan_tri_bwd_filter(const ConvDims& d, bool wide);
 int launch_conv_tri_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
                                hipStream_t stream, float** parts, int* used);
 TriFilterPlan plan_duo_bwd_filter(const ConvDims& d);
+// three: the plan of three parts for operands that two cannot hold (SplitFilterPick); then there are or_three->splits slices where
+// *or_three->any, on the device, is set.
+struct OrThree { const int* any; int splits; };
 int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
-                               hipStream_t stream, float** parts, int* used);
+                               hipStream_t stream, float** parts, int* used, const TriFilterPlan* three, OrThree* or_three);
 
 bool conv1x1_stream_applies(const ConvDims& d);
 
@@ -781,9 +784,11 @@ inline size_t split_bytes(const ConvDims& d, bool bwd, int flags, size_t floor) 
 // which this form is then chosen in 188, 1.53 times as fast in the geometric mean).  1x1 layers need 384 channels or so to be
 // worth two split copies.  Its slices are short enough for the chain limit almost everywhere: it turns down 4 of 5493 calls (30
 // layers at every batch up to 256), of one to four images.
+// (or_three: beside a plan of two parts, the one for operands that two cannot hold; at plan.tab_bytes of its scratch, its slabs in the
+// same place)
 struct SplitFilterPick {
   int parts;
-  TriFilterPlan plan;
+  TriFilterPlan plan, or_three;
 };
 SplitFilterPick pick_split_bwd_filter(const ConvDims& d, int flags, size_t ws_bytes, size_t* need = nullptr);
 

@@ -209,6 +209,7 @@ struct DuoBatchArgs {
   const float* x; uint4* xt;
   const float* top; int parts;   // [C][parts]
   int* exps;
+  int* any;                      // set where a value has too few bits: it is marked, and TriRest's form may take over
   int N, C, H, W, halo, HpWp;
   FastDiv dWp;
   size_t plane;
@@ -253,6 +254,7 @@ __device__ __forceinline__ void duo_batch_body(const DuoBatchArgs& a, int b, flo
   const int ex = duo_exponent(m);
   if (bx == 0 && bz == 0 && threadIdx.x < kDuoCh && c < a.C) a.exps[c] = ex;
   float sum = 0.0f;
+  int lost = 0;
 #pragma unroll
   for (int i = 0; i < kDuoPix / 8; ++i) {
     const int pl = (threadIdx.x >> 5) + 8 * i, pix = pix0 + pl;
@@ -260,8 +262,9 @@ __device__ __forceinline__ void duo_batch_body(const DuoBatchArgs& a, int b, flo
 #pragma unroll
     for (int n = 0; n < 8; ++n) v[n] = tile[n][cl][pl];
     if (a.sums) sum += ((v[0] + v[1]) + (v[2] + v[3])) + ((v[4] + v[5]) + (v[6] + v[7]));
-    if (pix < a.HpWp && c < a.C) duo_store(a.xt, ((size_t)bz * a.HpWp + pix) * a.C + c, a.plane, v, ex, [](float most, int) { return most < 5.820766091e-11f; });   // 2^-34
+    if (pix < a.HpWp && c < a.C) lost |= duo_store(a.xt, ((size_t)bz * a.HpWp + pix) * a.C + c, a.plane, v, ex, [](float, int) { return true; });
   }
+  if (lost != 0) *a.any = 1;
   if (a.sums) {
     __syncthreads();
     float* const part = &tile[0][0][0];
@@ -302,7 +305,7 @@ __global__ __launch_bounds__(256) void duo_batch_kernel(DuoBatchArgs dy, DuoBatc
 
 template <class T, bool NCHW, class PASS>
 static int launch_duo(const DuoParams& ap, const DuoParams& bp, const DuoSource& src, const EpiParams& ep, int k_steps, int groups,
-                      int splits, int* used, double flops, hipStream_t stream, const char* tag) {
+                      int splits, int* used, double flops, hipStream_t stream, const char* tag, const TriRest& rest = TriRest{}) {
   const int tiles_m = cdiv(ep.rows, T::BM), tiles_n = cdiv(ep.cols, T::BN);
   if (ep.tail_tiles > 0) splits = ep.tail_splits;
   const int sps = cdiv(k_steps, splits < 1 ? 1 : splits);
@@ -314,12 +317,12 @@ static int launch_duo(const DuoParams& ap, const DuoParams& bp, const DuoSource&
     grid = dim3((unsigned)(ep.full_tiles + ep.tail_tiles * ep.tail_splits), 1u);
   }
   constexpr size_t lds = DuoShape<T>::LDS;
-  static_assert(2 * lds <= 160 * 1024, "two blocks share a CU");
+  static_assert(2 * lds <= 160 * 1024 && lds >= kTriLdsBytes, "two blocks share a CU");
   static const hipError_t attr = hipFuncSetAttribute(reinterpret_cast<const void*>(&mfma_gemm_duo_kernel<T, NCHW, PASS>),
                                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds);
   if (attr != hipSuccess) return (int)attr;
   ProfScope prof(tag, flops, stream);
-  hipLaunchKernelGGL((mfma_gemm_duo_kernel<T, NCHW, PASS>), grid, dim3(T::NT), lds, stream, ap, bp, src, ep, tiles_m, k_steps, sps, groups);
+  hipLaunchKernelGGL((mfma_gemm_duo_kernel<T, NCHW, PASS>), grid, dim3(T::NT), lds, stream, ap, bp, src, ep, tiles_m, k_steps, sps, groups, rest);
   return launch_status();
 }
 
@@ -484,7 +487,7 @@ TriFilterPlan plan_duo_bwd_filter(const ConvDims& d) {
   p.groups = round_up(p.groups_true, 2);
   const size_t dy_part = 16 * (size_t)p.groups * d.K, x_part = 16 * (size_t)p.n8 * p.Hp * p.Wp * d.C;
   if (2 * dy_part > kMaxBufferBytes || 2 * x_part > kMaxBufferBytes) return p;
-  p.tab_bytes = align256(sizeof(int) * (size_t)p.groups) + align256(sizeof(int) * (2 * (size_t)duo_rows(d.K) + d.C)) +
+  p.tab_bytes = align256(sizeof(int) * (size_t)p.groups) + align256(sizeof(int) * ((size_t)duo_rows(d.K) + d.C + 1)) +
                 align256(sizeof(float) * ((size_t)d.K * duo_channel_parts(d.K) + (size_t)d.C * duo_channel_parts(d.C)));
   p.dyt_bytes = align256(2 * dy_part);
   p.xt_bytes = align256(2 * x_part);
@@ -510,13 +513,12 @@ TriFilterPlan plan_duo_bwd_filter(const ConvDims& d) {
 }
 
 int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
-                               hipStream_t stream, float** parts, int* used) {
+                               hipStream_t stream, float** parts, int* used, const TriFilterPlan* three, OrThree* or_three) {
   char* base = static_cast<char*>(ws);
   int* soff = reinterpret_cast<int*>(base);
   int* exps_a = reinterpret_cast<int*>(base + align256(sizeof(int) * (size_t)p.groups));
-  int* lost = exps_a + duo_rows(d.K);
-  int* exps_b = lost + duo_rows(d.K);
-  float* top_a = reinterpret_cast<float*>(reinterpret_cast<char*>(exps_a) + align256(sizeof(int) * (2 * (size_t)duo_rows(d.K) + d.C)));
+  int *exps_b = exps_a + duo_rows(d.K), *any = exps_b + d.C;
+  float* top_a = reinterpret_cast<float*>(reinterpret_cast<char*>(exps_a) + align256(sizeof(int) * ((size_t)duo_rows(d.K) + d.C + 1)));
   const int parts_a = duo_channel_parts(d.K), parts_b = duo_channel_parts(d.C);
   float* top_b = top_a + (size_t)d.K * parts_a;
   uint4* dyt = reinterpret_cast<uint4*>(base + p.tab_bytes);
@@ -524,17 +526,17 @@ int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const 
   *parts = reinterpret_cast<float*>(base + p.tab_bytes + p.dyt_bytes + p.xt_bytes);
   const size_t dy_plane = (size_t)p.groups * d.K, x_plane = (size_t)p.n8 * p.Hp * p.Wp * d.C;
   {
-    const DuoMaxJob ja = duo_max_job(dy, top_a, d.N, d.K, d.P * d.Q, parts_a, lost, duo_rows(d.K)), jb = duo_max_job(x, top_b, d.N, d.C, d.H * d.W, parts_b);
+    const DuoMaxJob ja = duo_max_job(dy, top_a, d.N, d.K, d.P * d.Q, parts_a, any, 1), jb = duo_max_job(x, top_b, d.N, d.C, d.H * d.W, parts_b);
     ProfScope prof("duo_max", 4.0 * (double)(d.y_elems + d.x_elems), stream);
     hipLaunchKernelGGL(duo_max_kernel, dim3((unsigned)(ja.blocks + jb.blocks)), dim3(256), 0, stream, ja, jb, DuoRatioJob{});
   }
   if (int e = launch_status()) return e;
   {
     DuoBatchArgs a, b;
-    a.x = dy; a.xt = dyt; a.top = top_a; a.parts = parts_a; a.exps = exps_a; a.N = d.N; a.C = d.K; a.H = d.P; a.W = d.Q; a.halo = 0;
+    a.x = dy; a.xt = dyt; a.top = top_a; a.parts = parts_a; a.exps = exps_a; a.any = any; a.N = d.N; a.C = d.K; a.H = d.P; a.W = d.Q; a.halo = 0;
     a.HpWp = d.P * d.Q; a.dWp = FastDiv((uint32_t)d.Q); a.plane = dy_plane; a.px = cdiv(a.HpWp, kDuoPix); a.cx = cdiv(a.C, kDuoCh);
     a.blocks = a.px * a.cx * p.n8; a.sums = sums;
-    b.x = x; b.xt = xt; b.top = top_b; b.parts = parts_b; b.exps = exps_b; b.N = d.N; b.C = d.C; b.H = d.H; b.W = d.W; b.halo = d.pad;
+    b.x = x; b.xt = xt; b.top = top_b; b.parts = parts_b; b.exps = exps_b; b.any = any; b.N = d.N; b.C = d.C; b.H = d.H; b.W = d.W; b.halo = d.pad;
     b.HpWp = p.Hp * p.Wp; b.dWp = FastDiv((uint32_t)p.Wp); b.plane = x_plane; b.px = cdiv(b.HpWp, kDuoPix); b.cx = cdiv(b.C, kDuoCh);
     b.blocks = b.px * b.cx * p.n8; b.sums = nullptr;
     ProfScope prof("duo_batch", 4.0 * (double)(d.y_elems + d.x_elems) + 32.0 * (double)(dy_plane + x_plane), stream);
@@ -542,12 +544,17 @@ int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const 
                        p.groups, p.groups_true, d.P * d.Q, d.Q, d.st, p.Wp);
   }
   if (int e = launch_status()) return e;
+  TriRest rest = {};
+  if (three) {
+    if (int e = launch_tri_rest_copies(d, *three, x, dy, base + p.tab_bytes, any, stream, &rest)) return e;
+    or_three->any = any; or_three->splits = rest.splits;
+  }
   const int CRS = d.C * d.R * d.S;
   DuoParams ap, bp;
   ap.t.v.ptr = dyt; ap.t.plane = (int)(16 * dy_plane); ap.t.v.bytes = (uint32_t)(32 * dy_plane);
   ap.t.v.M = d.K; ap.t.v.inner = 1; ap.t.v.innerW = 1; ap.t.v.img_stride = 16; ap.t.v.a_stride = 0; ap.t.v.b_stride = 0;
   ap.t.v.soff = nullptr; ap.t.v.group_stride = d.K * 16;
-  ap.exps = exps_a; ap.lost = lost; ap.ediv = 1; ap.emod = d.K;
+  ap.exps = exps_a; ap.lost = nullptr; ap.ediv = 1; ap.emod = d.K;
   bp.t.v.ptr = xt; bp.t.plane = (int)(16 * x_plane); bp.t.v.bytes = (uint32_t)(32 * x_plane);
   bp.t.v.M = CRS; bp.t.v.inner = d.S * d.C; bp.t.v.innerW = d.C;   // columns j = (r, s, c)
   bp.t.v.img_stride = p.Wp * d.C * 16; bp.t.v.a_stride = d.C * 16; bp.t.v.b_stride = 16;
@@ -562,7 +569,7 @@ int launch_conv_duo_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const 
   const double flops = 6.0 * (double)d.w_elems * d.N * d.P * d.Q;
   const int steps = p.groups / 2;
 #define RH_DUO(TILE, TAG) \
-  launch_duo<TILE, false, PassConvBwdFilter>(ap, bp, src, ep, steps, p.groups_true, p.splits, used, flops, stream, "conv_bwd_filter_duo_" TAG)
+  launch_duo<TILE, false, PassConvBwdFilter>(ap, bp, src, ep, steps, p.groups_true, p.splits, used, flops, stream, "conv_bwd_filter_duo_" TAG, rest)
   switch (p.bm) {
     case 128: return RH_DUO(T128x128t, "128x128");
     case 96: return RH_DUO(T96x128t, "96x128");

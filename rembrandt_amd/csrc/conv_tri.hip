@@ -208,10 +208,9 @@ __device__ __forceinline__ void tri_few_body(const TriBatchArgs& a, int b) {
 
 // Both operands of a filter gradient and soff[g], the place of group g = (n/8, p, q) in x's copy; the groups past the last
 // are zeros of dy.
-__global__ __launch_bounds__(256) void tri_batch_kernel(TriBatchArgs dy, TriBatchArgs x, int* __restrict__ soff, int groups,
-                                                        int groups_true, int PQ, int Q, int st, int Wp) {
-  __shared__ float tile[8][kTriCh][kTriPix + 1];
-  int b = blockIdx.x;
+struct TriTableArgs { int* soff; int groups, groups_true, PQ, Q, st, Wp, blocks; };
+__device__ __forceinline__ void tri_batch_block(const TriBatchArgs& dy, const TriBatchArgs& x, const TriTableArgs& t, int b,
+                                                float (&tile)[8][kTriCh][kTriPix + 1]) {
   if (b < dy.blocks) { tri_batch_body(dy, xcd_remap(b, dy.blocks), tile); return; }
   b -= dy.blocks;
   if (b < x.blocks) {
@@ -220,17 +219,31 @@ __global__ __launch_bounds__(256) void tri_batch_kernel(TriBatchArgs dy, TriBatc
     return;
   }
   b -= x.blocks;
-  if (groups > groups_true)   // (one group: every block of the table writes a share)
-    for (int i = b * 256 + threadIdx.x; i < 3 * dy.C; i += (int)(gridDim.x - dy.blocks - x.blocks) * 256)
-      dy.xt[(size_t)(i / dy.C) * dy.plane + (size_t)groups_true * dy.C + i % dy.C] = make_uint4(0, 0, 0, 0);
+  if (t.groups > t.groups_true)   // (one group: every block of the table writes a share)
+    for (int i = b * 256 + threadIdx.x; i < 3 * dy.C; i += t.blocks * 256)
+      dy.xt[(size_t)(i / dy.C) * dy.plane + (size_t)t.groups_true * dy.C + i % dy.C] = make_uint4(0, 0, 0, 0);
   const int g = b * 256 + threadIdx.x;
-  if (g >= groups) return;
+  if (g >= t.groups) return;
   int off = 0;
-  if (g < groups_true) {
-    const int n8 = g / PQ, pq = g - n8 * PQ, p = pq / Q, q = pq - p * Q;
-    off = (n8 * x.HpWp + p * st * Wp + q * st) * x.C * 16;
+  if (g < t.groups_true) {
+    const int n8 = g / t.PQ, pq = g - n8 * t.PQ, p = pq / t.Q, q = pq - p * t.Q;
+    off = (n8 * x.HpWp + p * t.st * t.Wp + q * t.st) * x.C * 16;
   }
-  soff[g] = off;
+  t.soff[g] = off;
+}
+__global__ __launch_bounds__(256) void tri_batch_kernel(TriBatchArgs dy, TriBatchArgs x, TriTableArgs t) {
+  __shared__ float tile[8][kTriCh][kTriPix + 1];
+  tri_batch_block(dy, x, t, blockIdx.x, tile);
+}
+// The same by a few blocks, and only where it is wanted (TriRest): a launch of as many blocks as there is work for would wait, beside
+// another stream's, for a place for each of them before it could end (AlexNet b256: 77 us on average, 12 so).
+__global__ __launch_bounds__(256) void tri_rest_batch_kernel(TriBatchArgs dy, TriBatchArgs x, TriTableArgs t, const int* __restrict__ any) {
+  __shared__ float tile[8][kTriCh][kTriPix + 1];
+  if (*any == 0) return;
+  for (int b = blockIdx.x; b < dy.blocks + x.blocks + t.blocks; b += (int)gridDim.x) {
+    tri_batch_block(dy, x, t, b, tile);
+    __syncthreads();   // (the tile is the next block's)
+  }
 }
 
 template <class T, bool B_LINEAR, bool NCHW, class PASS, bool WIDE = false>
@@ -496,34 +509,64 @@ TriFilterPlan plan_tri_bwd_filter(const ConvDims& d, bool wide) {
   return p;
 }
 
-int launch_conv_tri_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
-                               hipStream_t stream, float** parts, int* used) {
+// What the copies of a filter gradient's operands are made from, and the operands that they are.
+struct TriFilterSetup {
+  TriBatchArgs dy, x;
+  TriTableArgs table;
+  TriParams ap, bp;
+  float* parts;
+};
+static TriFilterSetup tri_filter_setup(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws) {
+  TriFilterSetup s;
   char* base = static_cast<char*>(ws);
-  int* soff = reinterpret_cast<int*>(base);
   uint4* dyt = reinterpret_cast<uint4*>(base + p.tab_bytes);
   uint4* xt = reinterpret_cast<uint4*>(base + p.tab_bytes + p.dyt_bytes);
-  *parts = reinterpret_cast<float*>(base + p.tab_bytes + p.dyt_bytes + p.xt_bytes);
+  s.parts = reinterpret_cast<float*>(base + p.tab_bytes + p.dyt_bytes + p.xt_bytes);
   const size_t dy_plane = (size_t)p.groups * d.K, x_plane = (size_t)p.n8 * p.Hp * p.Wp * d.C;
-  {
-    TriBatchArgs a, b;
-    a.x = dy; a.xt = dyt; a.N = d.N; a.C = d.K; a.H = d.P; a.W = d.Q; a.halo = 0; a.HpWp = d.P * d.Q; a.dWp = FastDiv((uint32_t)d.Q);
-    a.plane = dy_plane; a.px = cdiv(a.HpWp, kTriPix); a.cx = cdiv(a.C, kTriCh); a.blocks = a.px * a.cx * p.n8; a.sums = sums; a.wide = p.wide;
-    b.x = x; b.xt = xt; b.N = d.N; b.C = d.C; b.H = d.H; b.W = d.W; b.halo = d.pad; b.HpWp = p.Hp * p.Wp; b.dWp = FastDiv((uint32_t)p.Wp);
-    b.plane = x_plane; b.px = cdiv(b.HpWp, d.C <= kTriFew ? kTriFewPix : kTriPix); b.cx = cdiv(b.C, kTriCh); b.blocks = b.px * b.cx * p.n8; b.sums = nullptr; b.wide = false;
-    ProfScope prof("tri_batch", 4.0 * (double)(d.y_elems + d.x_elems) + 48.0 * (double)(dy_plane + x_plane), stream);
-    hipLaunchKernelGGL(tri_batch_kernel, dim3((unsigned)(a.blocks + b.blocks + cdiv(p.groups, 256))), dim3(256), 0, stream, a, b, soff,
-                       p.groups, p.groups_true, d.P * d.Q, d.Q, d.st, p.Wp);
-  }
-  if (int e = launch_status()) return e;
-  const int CRS = d.C * d.R * d.S;
-  TriParams ap, bp;
+  TriBatchArgs &a = s.dy, &b = s.x;
+  a.x = dy; a.xt = dyt; a.N = d.N; a.C = d.K; a.H = d.P; a.W = d.Q; a.halo = 0; a.HpWp = d.P * d.Q; a.dWp = FastDiv((uint32_t)d.Q);
+  a.plane = dy_plane; a.px = cdiv(a.HpWp, kTriPix); a.cx = cdiv(a.C, kTriCh); a.blocks = a.px * a.cx * p.n8; a.sums = sums; a.wide = p.wide;
+  b.x = x; b.xt = xt; b.N = d.N; b.C = d.C; b.H = d.H; b.W = d.W; b.halo = d.pad; b.HpWp = p.Hp * p.Wp; b.dWp = FastDiv((uint32_t)p.Wp);
+  b.plane = x_plane; b.px = cdiv(b.HpWp, d.C <= kTriFew ? kTriFewPix : kTriPix); b.cx = cdiv(b.C, kTriCh); b.blocks = b.px * b.cx * p.n8; b.sums = nullptr; b.wide = false;
+  s.table = TriTableArgs{reinterpret_cast<int*>(base), p.groups, p.groups_true, d.P * d.Q, d.Q, d.st, p.Wp, cdiv(p.groups, 256)};
+  TriParams &ap = s.ap, &bp = s.bp;
   ap.v.ptr = dyt; ap.plane = (int)(16 * dy_plane); ap.v.bytes = (uint32_t)(48 * dy_plane);
   ap.v.M = d.K; ap.v.inner = 1; ap.v.innerW = 1; ap.v.img_stride = 16; ap.v.a_stride = 0; ap.v.b_stride = 0;
   ap.v.soff = nullptr; ap.v.group_stride = d.K * 16;
   bp.v.ptr = xt; bp.plane = (int)(16 * x_plane); bp.v.bytes = (uint32_t)(48 * x_plane);
-  bp.v.M = CRS; bp.v.inner = d.S * d.C; bp.v.innerW = d.C;   // rows j = (r, s, c)
+  bp.v.M = d.C * d.R * d.S; bp.v.inner = d.S * d.C; bp.v.innerW = d.C;   // rows j = (r, s, c)
   bp.v.img_stride = p.Wp * d.C * 16; bp.v.a_stride = d.C * 16; bp.v.b_stride = 16;
-  bp.v.soff = soff; bp.v.group_stride = 0;
+  bp.v.soff = s.table.soff; bp.v.group_stride = 0;
+  return s;
+}
+
+int launch_tri_rest_copies(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, void* ws, const int* any,
+                           hipStream_t stream, TriRest* rest) {
+  const TriFilterSetup s = tri_filter_setup(d, p, x, dy, nullptr, ws);
+  const int bm = p.bm == 128 ? 128 : p.bm == 96 ? 96 : 64, bn = bm == 64 ? 192 : 128, blocks = s.dy.blocks + s.x.blocks + s.table.blocks;
+  rest->any = any; rest->ap = s.ap; rest->bp = s.bp;
+  rest->tiles_m = cdiv(d.K, bm);
+  rest->tiles = rest->tiles_m * cdiv(d.C * d.R * d.S, bn);
+  rest->k_steps = p.groups / 2;
+  rest->steps_per_split = cdiv(rest->k_steps, p.splits);
+  rest->splits = cdiv(rest->k_steps, rest->steps_per_split);
+  rest->groups = p.groups_true;
+  ProfScope prof("tri_rest", 0.0, stream);
+  hipLaunchKernelGGL(tri_rest_batch_kernel, dim3((unsigned)(blocks < 512 ? blocks : 512)), dim3(256), 0, stream, s.dy, s.x, s.table, any);
+  return launch_status();
+}
+
+int launch_conv_tri_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
+                               hipStream_t stream, float** parts, int* used) {
+  const TriFilterSetup s = tri_filter_setup(d, p, x, dy, sums, ws);
+  *parts = s.parts;
+  {
+    ProfScope prof("tri_batch", 4.0 * (double)(d.y_elems + d.x_elems) + 48.0 * (double)(s.dy.plane + s.x.plane), stream);
+    hipLaunchKernelGGL(tri_batch_kernel, dim3((unsigned)(s.dy.blocks + s.x.blocks + s.table.blocks)), dim3(256), 0, stream, s.dy, s.x, s.table);
+  }
+  if (int e = launch_status()) return e;
+  const TriParams &ap = s.ap, &bp = s.bp;
+  const int CRS = d.C * d.R * d.S;
   EpiParams ep;
   ep.out = *parts; ep.bias = nullptr; ep.alpha = 1.0f; ep.beta = 0.0f;
   ep.rows = d.K; ep.cols = CRS; ep.inner = 0; ep.ld = CRS; ep.relu = 0; ep.split_stride = (long long)d.K * CRS;

@@ -25,6 +25,8 @@
 //   tensor are under 2^-29 and of four tensors of 13 some are marked; there the operators ask for three parts.
 // * A filter's small values (one in 1e8 of normal weights) are counted.  They cost a result 2^-20 each at most, so its sum, before it is
 //   scaled back, has to be four times their number: 2^27 is usual.  (A mark would have the filter's whole plane formed again.)
+// * In the filter gradient, where the eight of a group are images and zeros of the other operand say nothing of the sum, every small value
+//   is marked, and one such value makes it a call in three parts (TriRest; AlexNet b256 one call in 48, in NIN b128 the 5x5 layer's).
 //   Formed again, a block of 32 x 32 results is bound by the latency of its loads, 32 of them in flight (one by one 384 -> 384 3x3 13x13
 //   b256 forward took 3.0 ms longer for one value): 330 us, with one value in x 930, with one in every group 3.9 ms (three parts 550 us,
 //   1.4 and 2.9 ms); 5x5 of 96 channels 0.6, 0.9 and 12 ms, 1x1 at 128 images 54, 93 and 260 us.  In the filter gradient, whose loads are
@@ -53,8 +55,8 @@ __device__ __forceinline__ uint32_t duo_least(int e) {
   return b > 0 ? (uint32_t)b << 23 : b > -23 ? 1u << (22 + b) : 0u;
 }
 
-// Eight values (one group) of a row with exponent e; returns how many of them, not 0, are under duo_least.  mark(most, n) says whether
-// those n are marked, most being the group's largest scaled value.
+// Eight values (one group) of a row with exponent e; returns how many of them are, but not 0, under duo_least or no finite numbers.
+// mark(most, n) says whether the n small ones are marked, most being the group's largest scaled value.
 template <class MARK>
 __device__ __forceinline__ int duo_pack8(const float (&v)[8], int e, MARK mark, uint4 (&o)[2]) {
   uint32_t w[2][4];
@@ -84,6 +86,7 @@ __device__ __forceinline__ int duo_pack8(const float (&v)[8], int e, MARK mark, 
 #pragma unroll
       for (int h = 0; h < 2; ++h) {
         const uint32_t bits = __builtin_bit_cast(uint32_t, v[2 * i + h]) & 0x7fffffffu;
+        lost += bits >= 0x7f800000u;
         if (bits >= 0x7f800000u || (small && bits - 1u < under)) {
           const uint32_t keep = h ? 0xffffu : 0xffff0000u;
           w[0][i] = (w[0][i] & keep) | (0x7e00u << (16 * h));
@@ -98,7 +101,7 @@ __device__ __forceinline__ int duo_pack8(const float (&v)[8], int e, MARK mark, 
 }
 
 // An operand of this form: TriParams with two parts, the exponents of its rows: row m has exps[m / ediv % emod], and the counts of their
-// small values (of A).
+// small values (of A, nullptr in the filter gradient).
 struct DuoParams {
   TriParams t;
   const int *exps, *lost;
@@ -272,10 +275,11 @@ __device__ __forceinline__ void duo_block(const DuoParams& ap, const DuoParams& 
 #pragma unroll
       for (int i = 0; i < Loader::CNT; ++i) ld.issue(lds0 + (uint32_t)(s * (SA + SB)) * 16u, i);
     }
-  int lost_here = 0;   // small values in a row of the wave's (looked at once the first steps have landed)
+  int lost_here = 0;   // small values in the wave's rows (looked at once the first steps have landed)
+  if (ap.lost)
 #pragma unroll
-  for (int r = 0; r < TM * 32; r += 64)
-    if (r + lane < TM * 32) lost_here |= ap.lost[m0 + wm * (TM * 32) + r + lane];
+    for (int r = 0; r < TM * 32; r += 64)
+      if (r + lane < TM * 32) lost_here |= ap.lost[m0 + wm * (TM * 32) + r + lane];
   ld.prep(s_begin + (R - 1 < nk ? R - 1 : nk - 1));
   wait_vmcnt<0>();
   __syncthreads();
@@ -443,7 +447,13 @@ __device__ __forceinline__ void duo_block(const DuoParams& ap, const DuoParams& 
 
 template <class T, bool NCHW, class PASS>
 __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_duo_kernel(DuoParams ap, DuoParams bp, DuoSource src, EpiParams ep,
-                                                                      int tiles_m, int k_steps, int steps_per_split, int groups) {
+                                                                      int tiles_m, int k_steps, int steps_per_split, int groups, TriRest rest) {
+  if constexpr (std::is_same<PASS, PassConvBwdFilter>::value) {
+    if (rest.any && *rest.any != 0) {
+      tri_rest_blocks<typename std::conditional<T::BM == 64, T64x192t, T>::type>(rest, ep);
+      return;
+    }
+  }
   int slice, logical, dst_split;   // as in mfma_gemm_kernel
   if (ep.tail_tiles > 0) {
     const int b = blockIdx.x;

@@ -456,6 +456,28 @@ __global__ __launch_bounds__(T::NT, T::OCC) void mfma_gemm_tri_kernel(TriParams 
   tri_block<T, B_LINEAR, NCHW, WIDE>(ap, bp, ep, m0, n0, s_begin, s_end, groups, dst_split);
 }
 
+// A filter gradient in three parts for operands that two fp16 parts cannot hold: *any is set where their copies met a value with too few
+// bits there.  Its copies are a launch of a few blocks, its contraction the work of the blocks of the one in two parts (gemm_duo.h),
+// so that where it is not wanted it costs one short launch.
+struct TriRest {
+  const int* any;   // nullptr: no such form
+  TriParams ap, bp;
+  int tiles_m, tiles, splits, k_steps, steps_per_split, groups;
+};
+int launch_tri_rest_copies(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, void* ws, const int* any,
+                           hipStream_t stream, TriRest* rest);
+template <class T>
+__device__ __forceinline__ void tri_rest_blocks(const TriRest& r, const EpiParams& ep) {
+  const int blocks = (int)(gridDim.x * gridDim.y), total = r.tiles * r.splits;
+  for (int b = (int)(blockIdx.y * gridDim.x + blockIdx.x); b < total; b += blocks) {
+    const int slice = __builtin_amdgcn_readfirstlane(b / r.tiles), logical = __builtin_amdgcn_readfirstlane(b - slice * r.tiles);
+    const int s0 = slice * r.steps_per_split, s1 = s0 + r.steps_per_split < r.k_steps ? s0 + r.steps_per_split : r.k_steps;
+    tri_block<T, false, false, false>(r.ap, r.bp, ep, logical % r.tiles_m * T::BM, logical / r.tiles_m * T::BN, s0, s1, r.groups,
+                                      ep.split_stride != 0 ? slice : -1);
+    __syncthreads();   // (the ring is the next tile's)
+  }
+}
+
 // Backward-data of stride 2 to 4 (conv_common.h: residue classes): the classes' contractions in one launch, the longest first, so that
 // the short ones fill the last round (launched one by one the classes of 64 -> 128 56x56 b24 are 98 tiles each on 256 CUs).  Bound by
 // the MFMAs as above and by the classes' results, which a second pass interleaves.

@@ -907,6 +907,55 @@ def test_conv2d_f16x2_values_of_all_sizes(dev):
             assert np.all(np.abs(got.astype(np.float64) - want) <= 2.0 ** -20 * size), (name, spread, zeros)
 
 
+@pytest.mark.parametrize("k", [20, 29, 31, 36, 45, 52, 80, 120])
+def test_conv2d_f16x2_filter_gradient_of_small_values(dev, k):
+    """The same for the filter gradient: one sample's values large where the other operand's are 0, the others' 2^-k as large, a few of
+    them or all.  18 x 56 products at most: 2^-18 of the sum of magnitudes."""
+    say("f16x2 small in a batch", k)
+    x0, dy0, shape = synth.normal(42, 1, (18, 10, 8, 7)), synth.normal(42, 2, (18, 70, 8, 7)), (70, 10, 3, 3)
+    few = synth.uniform(42, 3, (18, 1, 8, 7)) < 0.01
+    for small, other in ((0, 1), (1, 0)):
+        for some in (few, np.ones_like(few)):
+            pair = [x0.copy(), dy0.copy()]
+            pair[small][1:] *= np.float32(2.0) ** -k * some[1:]
+            pair[other][0] = 0.0
+            x, dy = pair
+            got = N(ops.conv2d_bwd_filter(T(x, dev), T(dy, dev), shape, 1, 1, algo=_lib.RH_ALGO_F16X2 | _lib.RH_ALGO_DIRECT))
+            want, size = O.conv2d_bwd_filter(x, dy, shape, 1, 1), O.conv2d_bwd_filter(np.abs(x), np.abs(dy), shape, 1, 1)
+            assert np.all(np.abs(got.astype(np.float64) - want) <= 2.0 ** -18 * size), (small, some.all())
+
+
+@pytest.mark.parametrize("kind", ["none", "one", "many", "x", "nan"])
+def test_conv2d_f16x2_filter_gradient_in_three_parts(dev, kind):
+    """Where the library takes two parts by itself, beside RH_ALGO_BF16X3: a value that two parts cannot hold, or that is no finite number,
+    makes it the call with RH_ALGO_BF16X3 alone."""
+    say("f16x2 or three parts", kind)
+    Nn, C, H, K, R, pad = 128, 96, 27, 96, 5, 2
+    x, dy = T(synth.normal(43, 1, (Nn, C, H, H)), dev).clamp_min(0.0), T(synth.normal(43, 2, (Nn, K, H, H)), dev)
+    x, dy = (torch.where(t.abs() < 1e-4, torch.zeros_like(t), t) for t in (x, dy))   # (none by chance)
+    X3, F2, shape = _lib.RH_ALGO_BF16X3, _lib.RH_ALGO_F16X2, (K, C, R, R)
+    x[0], x[:, 5] = 0.0, 0.0
+    if kind == "one":
+        dy[77, 11, 26, 26] = 2.0 ** -41
+    elif kind == "many":
+        dy[1:] *= 2.0 ** -40
+    elif kind == "x":
+        x[127, 95, 0, 0] = 2.0 ** -45
+    elif kind == "nan":
+        dy[3, 2], x[40, 3, 3, 3], x[41, 17, 0, 0] = float("nan"), float("inf"), float("nan")
+    call = lambda algo: ops.conv2d_bwd_filter_bias(x, dy, shape, 1, pad, alpha=0.5, algo=algo)
+    (got, db), tags = profile_tags(lambda: call(X3 | F2))
+    assert any(t.startswith("conv_bwd_filter_duo_") for t in tags) and "tri_rest" in tags, tags
+    (three, db3), tags = profile_tags(lambda: call(X3))
+    assert any(t.startswith("conv_bwd_filter_tri_") for t in tags), tags
+    same = torch.equal(torch.isnan(got), torch.isnan(three)) and torch.equal(got.nan_to_num(), three.nan_to_num())
+    assert same == (kind != "none")
+    assert torch.allclose(got, three, rtol=1e-5, atol=1e-5 * float(three.nan_to_num().abs().max()), equal_nan=True)
+    assert torch.allclose(db, db3, rtol=1e-5, atol=1e-5 * float(db3.nan_to_num().abs().max()), equal_nan=True)
+    again = call(X3 | F2)
+    assert torch.equal(again[0].nan_to_num(), got.nan_to_num()) and torch.equal(again[1].nan_to_num(), db.nan_to_num()), "run to run the same bits"
+
+
 @pytest.mark.parametrize("case", [(90, 256, 14, 256, 3, 1), (24, 512, 7, 512, 3, 1)], ids=str)
 def test_conv2d_f16x2_deltas_behind_a_batch_norm(dev, case):
     """A filter gradient whose caller sets RH_ALGO_BF16X3_WIDE stays with three parts."""
