@@ -1303,13 +1303,11 @@ struct BNormConvUnit {
   // against 64 bits, relative to the other forms', 8 to 200 images: 64 -> 64 56x56 1.2 to 5.1 in the units whose input is
   // positive, 64 -> 128 1.4 to 3.1, 128 -> 128 28x28 0.7 to 1.4, 128 -> 256 0.5 to 1.2; 256 and 512 channels on 14x14 and 7x7 0.2 to 0.9.
   // Its deltas are a batch norm's: a small value almost everywhere beside the large ones that a ReLU let through.
-  // (behind the batch norm's backward: small deltas everywhere, of which some are more than 2^29 under the largest of their image)
-  int data_algo() const { return conv_algo & ~RH_ALGO_F16X2; }
   int filter_algo() const { return conv_algo | (conv_algo & RH_ALGO_BF16X3 ? RH_ALGO_BF16X3_WIDE : 0); }
   size_t workspace_bytes() const {
     const rh_conv_geom g = geom(batch_cap);
     size_t ws = std::max(conv_ws_upto(g, RH_CONV_FWD, conv_algo), bnorm_ws_upto(g.N, g.K, plane()));
-    if (backward) ws = std::max(std::max(ws, aux_bytes), conv_ws_upto(g, RH_CONV_BWD_DATA, data_algo()));
+    if (backward) ws = std::max(std::max(ws, aux_bytes), conv_ws_upto(g, RH_CONV_BWD_DATA, conv_algo));
     return ws;
   }
   rh_stream_t s() const { return ctx->stream(); }
@@ -1391,7 +1389,7 @@ struct BNormConvUnit {
   void backward_data(size_t batch, float* in_delta, float beta, DeviceBuffer<uint8_t>& ws) {
     const rh_conv_geom g = geom(batch);
     unwrap(rh_conv2d_bwd_data(&g, 1.0f, weights->as_ptr(), pre_delta->as_ptr(), beta, in_delta, ws.as_mut_ptr(), ws.len(),
-                              data_algo() | (beside ? RH_ALGO_SHARED_GPU : 0), s()), "conv2d backward data");
+                              conv_algo | (beside ? RH_ALGO_SHARED_GPU : 0), s()), "conv2d backward data");
   }
 
   void axpy(float a, const DeviceBuffer<float>& x, DeviceBuffer<float>& y) {
