@@ -393,8 +393,8 @@ static TriRival filter_rival(const ConvDims& d) {
 // Two parts beside the form of time `other_us` and error `err`; both errors with a twentieth of the products not zero, as behind a
 // max-pool, where two parts are the least ahead (1e-14 on the square): three parts 0.005 a K step of a slice and 0.016 a slice; two 1.0
 // and 0.016 a slice (of AlexNet's conv5 at 128 images 0.92e-7 and 1.08e-7, at 256 1.30 and 1.15, of its conv2 at 50 1.28 and 1.26).
-static bool duo_filter_pays(const TriFilterPlan& p, double other_us, double err) {
-  return p.ok && p.us < 0.96 * other_us && 1.0 + 0.016 * p.splits <= err;
+static bool duo_filter_pays(int splits, double us, double other_us, double err) {
+  return us < 0.96 * other_us && 1.0 + 0.016 * splits <= err;
 }
 // need: the scratch of the forms that may be taken with less
 SplitFilterPick pick_split_bwd_filter(const ConvDims& d, int flags, size_t ws_bytes, size_t* need) {
@@ -423,7 +423,8 @@ SplitFilterPick pick_split_bwd_filter(const ConvDims& d, int flags, size_t ws_by
       if (need && p.total() > *need) *need = p.total();
     }
   }
-  if (duo) {
+  // (planned only where its copies leave time for a product and its error a slice: a call's plans are made anew each time)
+  if (duo && duo_filter_pays(1, kDuoFilterCopies + 2e-6 * (double)(d.x_elems + d.y_elems), us, err)) {
     // (two parts and, in the same scratch, three, for the calls whose values two cannot hold: deltas of samples that the network is sure of
     // may be 1e-9 of the others, and where those meet zeros the gradient is of the small ones alone.  Which it is the blocks look
     // up on the device)
@@ -434,7 +435,7 @@ SplitFilterPick pick_split_bwd_filter(const ConvDims& d, int flags, size_t ws_by
       three.xt_bytes = copies - three.tab_bytes - three.dyt_bytes;
       p.part_bytes = std::max(p.part_bytes, three.part_bytes);
     }
-    if ((three.ok || !tri_allowed(flags)) && p.total() <= ws_bytes && duo_filter_pays(p, us, err)) {
+    if ((three.ok || !tri_allowed(flags)) && p.ok && p.total() <= ws_bytes && duo_filter_pays(p.splits, p.us, us, err)) {
       s = SplitFilterPick{2, p, three};
       if (need && p.total() > *need) *need = p.total();
     }

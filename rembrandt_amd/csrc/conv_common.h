@@ -628,6 +628,7 @@ TriFilterPlan plan_tri_bwd_filter(const ConvDims& d, bool wide);
 // pixels.
 int launch_conv_tri_bwd_filter(const ConvDims& d, const TriFilterPlan& p, const float* x, const float* dy, float* sums, void* ws,
                                hipStream_t stream, float** parts, int* used);
+constexpr double kDuoFilterCopies = 22.8;   // us of a call besides its bytes, slices and product
 TriFilterPlan plan_duo_bwd_filter(const ConvDims& d);
 // three: the plan of three parts for operands that two cannot hold (SplitFilterPick); then there are or_three->splits slices where
 // *or_three->any, on the device, is set.

@@ -497,14 +497,15 @@ TriFilterPlan plan_duo_bwd_filter(const ConvDims& d) {
   const int CRS = d.C * d.R * d.S, tiles = cdiv(d.K, p.bm) * cdiv(CRS, p.bn), steps = p.groups / 2;
   p.us = 1e30;
   const DuoRates& rate = p.bm == 128 ? kDuoFilter128 : p.bm == 96 ? kDuoFilter96 : kDuoFilter64;
-  for (int want = 1; want <= 256 && (want == 1 || (want * 6 <= steps && (long long)tiles * want <= 2048)); ++want) {
+  // (more slices take 0.45 us each at least)
+  for (int want = 1; want <= 256 && 0.45 * want < p.us && (want == 1 || (want * 6 <= steps && (long long)tiles * want <= 2048)); ++want) {
     const int n = cdiv(steps, want), S = cdiv(steps, n);
     if (S != want || 4.0 * (double)S * (double)d.w_elems > 256e6) continue;
     const double us = duo_run_us(rate, (long long)tiles * S, n) + 0.45 * S + 1.6e-6 * (double)d.w_elems * (S + 1);
     if (us < p.us) { p.us = us; p.splits = S; }
   }
   if (p.splits == 0) p.splits = 1;   // (as plan_tri_bwd_filter)
-  p.us += 22.8 + 2e-6 * (double)(d.x_elems + d.y_elems);
+  p.us += kDuoFilterCopies + 2e-6 * (double)(d.x_elems + d.y_elems);
   p.part_bytes = align256(sizeof(float) * (size_t)p.splits * (size_t)d.w_elems);
   p.sum_rows = p.n8 * cdiv(d.P * d.Q, kDuoPix);
   p.sum_bytes = align256(sizeof(float) * (size_t)p.sum_rows * d.K);
