@@ -704,14 +704,26 @@ inline TriPlan plan_tri_pass(const ConvDims& d, bool bwd, int max_chain) {
 }
 // The form of split operands that a call takes, if any: 3 or 2 parts.  Two parts where they are expected to be faster than what the
 // call takes otherwise, and no further from 64 bits.
-// What two parts lose that three do not, 2^-23 of a value, is the same at every length, and deltas behind a max-pool are zeros for the most
-// part, so the chains that three parts round are short: of AlexNet's conv5 (384 filters in 256) the data gradient has an error of
-// 1.04e-7 with three parts at 144 K steps in a chain and 0.79e-7 at 72, with two parts 0.94 and 1.03e-7.  In the forward pass, half
-// zeros: 1.04 and 1.16e-7 at 36 steps, 1.55 and 1.2 at 72, 2.3 and 1.3 at 144 (three and two parts).  So two parts replace three from
-// about 55 K steps in a chain on, in backward-data from 130.
-inline bool duo_replaces_tri(bool bwd, const TriPlan& tri, int duo_steps) {
-  const int chain = cdiv(tri.groups / 2, tri.splits);
-  return bwd ? chain >= 130 : 0.0525 * chain >= 2.5 + 0.008 * duo_steps;
+// What a result is summed from, over all tiles: K steps in a chain, and slices beyond the first (a sliced tail has short chains).
+struct MeanChain { double steps, slices; };
+inline MeanChain mean_chain(const TriPlan& p) {
+  const double n = cdiv(p.groups / 2, p.splits);
+  if (p.tail.splits <= 1) return MeanChain{n, p.splits - 1.0};
+  const double tail = (double)p.tail.tail_tiles / (p.tail.full_tiles + p.tail.tail_tiles);
+  return MeanChain{(1.0 - tail) * n + tail * cdiv(p.groups / 2, p.tail.splits), tail * (p.tail.splits - 1)};
+}
+// What two parts lose that three do not, 2^-23 of a value, is the same at every length; what three round grows with the chain, and with the
+// deltas that are not zeros, of which few are left behind a max-pool.  Squared error in units of 1e-14, a fit to 118 layers and batches of
+// N(0,1) operands (0.87 to 1.16 of its square root measured): forward, half of the image zeros, three parts 0.0327 a step and
+// 0.012 a slice, two 1.25, 0.004 and 0.027; data gradient, nine deltas in ten zeros, 0.06, 0.0066 and 0.028, two 1.0 and 0.035 a slice.  So
+// taken, the error is 0.59 of three parts' forward (geometric mean; 0.93 at most) and 0.78 backward (0.96, and 1.02 at the line); with half
+// of the deltas 0.38, with one in twenty 1.04 (1.3 at most).  dense: the caller says that there are deltas almost everywhere (RH_ALGO_BF16X3_WIDE), where three parts have
+// 0.0526 a step: 0.33 over 311 data gradients of ResNet-18 (0.45 at most).
+inline bool duo_replaces_tri(bool bwd, bool dense, const TriPlan& tri, const TriPlan& duo) {
+  const MeanChain a = mean_chain(tri), b = mean_chain(duo);
+  if (bwd && dense) return cdiv(tri.groups / 2, tri.splits) >= 130;
+  return bwd ? 0.0066 * a.steps + 0.028 * a.slices >= 0.92 + 0.035 * b.slices
+             : 0.0327 * a.steps + 0.012 * a.slices >= 1.56 + 0.005 * b.steps + 0.034 * b.slices;
 }
 // The others' errors are in tri_max_chain's units, N(0,1).  Over 539 timed calls (18 layers at 11 batches, all passes, half zeros) two parts
 // are taken in 137, 1.34 times as fast in the geometric mean, none slower, with 0.50 of the error of the form replaced, 0.87 at most; on
@@ -723,10 +735,9 @@ struct SplitPick {
   TriPlan plan;
 };
 // (the estimates of three and two parts have an error of 6 % each; a twenty-fifth keeps the choice from changing for nothing)
-inline bool duo_pays(const TriPlan& p, bool bwd, const TriPlan* tri, const TriRival& other) {
-  const int steps = p.ok ? cdiv(p.groups / 2, p.splits) : 0;
+inline bool duo_pays(const TriPlan& p, bool bwd, int flags, const TriPlan* tri, const TriRival& other) {
   if (!p.ok || p.us >= 0.96 * (tri ? tri->us : other.us)) return false;
-  return tri ? duo_replaces_tri(bwd, *tri, steps) : duo_replaces(other.err, steps);
+  return tri ? duo_replaces_tri(bwd, tri_wide(flags), *tri, p) : duo_replaces(other.err, cdiv(p.groups / 2, p.splits));
 }
 inline SplitPick pick_split(const ConvDims& d, bool bwd, int flags, size_t ws_bytes) {
   SplitPick s = {};
@@ -745,7 +756,7 @@ inline SplitPick pick_split(const ConvDims& d, bool bwd, int flags, size_t ws_by
   }
   if (duo_allowed(flags)) {
     const TriPlan p = plan_duo_pass(d, bwd);
-    if (p.total() <= ws_bytes && duo_pays(p, bwd, s.parts ? &s.plan : nullptr, other)) s = SplitPick{2, p};
+    if (p.total() <= ws_bytes && duo_pays(p, bwd, flags, s.parts ? &s.plan : nullptr, other)) s = SplitPick{2, p};
   }
   return s;
 }
@@ -776,7 +787,7 @@ inline size_t split_bytes(const ConvDims& d, bool bwd, int flags, size_t floor) 
       tri = p.ok && p.us < other.us;
       if (tri && p.total() > need) need = p.total();
     }
-    if (duo_pays(q, bwd, tri ? &p : nullptr, other) && q.total() > need) need = q.total();
+    if (duo_pays(q, bwd, flags, tri ? &p : nullptr, other) && q.total() > need) need = q.total();
   }
   return need;
 }

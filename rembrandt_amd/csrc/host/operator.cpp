@@ -1302,12 +1302,12 @@ struct BNormConvUnit {
   // eight that it adds at once: where the inputs are of one sign that adds up over the pixels.  Error of ResNet-18's filter gradients
   // against 64 bits, relative to the other forms', 8 to 200 images: 64 -> 64 56x56 1.2 to 5.1 in the units whose input is
   // positive, 64 -> 128 1.4 to 3.1, 128 -> 128 28x28 0.7 to 1.4, 128 -> 256 0.5 to 1.2; 256 and 512 channels on 14x14 and 7x7 0.2 to 0.9.
-  // Its deltas are a batch norm's: a small value almost everywhere beside the large ones that a ReLU let through.
-  int filter_algo() const { return conv_algo | (conv_algo & RH_ALGO_BF16X3 ? RH_ALGO_BF16X3_WIDE : 0); }
+  // The gradients': deltas are a batch norm's, a small value almost everywhere beside the large ones that a ReLU let through.
+  int grad_algo() const { return conv_algo | (conv_algo & RH_ALGO_BF16X3 ? RH_ALGO_BF16X3_WIDE : 0); }
   size_t workspace_bytes() const {
     const rh_conv_geom g = geom(batch_cap);
     size_t ws = std::max(conv_ws_upto(g, RH_CONV_FWD, conv_algo), bnorm_ws_upto(g.N, g.K, plane()));
-    if (backward) ws = std::max(std::max(ws, aux_bytes), conv_ws_upto(g, RH_CONV_BWD_DATA, conv_algo));
+    if (backward) ws = std::max(std::max(ws, aux_bytes), conv_ws_upto(g, RH_CONV_BWD_DATA, grad_algo()));
     return ws;
   }
   rh_stream_t s() const { return ctx->stream(); }
@@ -1383,13 +1383,13 @@ struct BNormConvUnit {
       wg = ws_aux;
     }
     unwrap(rh_conv2d_bwd_filter(&g, 1.0f, in, pre_delta->as_ptr(), 1.0f, grad_weights->as_mut_ptr(), wg->as_mut_ptr(),
-                                wg->len(), filter_algo(), sg), "conv2d backward filter");
+                                wg->len(), grad_algo(), sg), "conv2d backward filter");
   }
   // in_delta = beta*in_delta + dconv^T(weights, pre_delta)
   void backward_data(size_t batch, float* in_delta, float beta, DeviceBuffer<uint8_t>& ws) {
     const rh_conv_geom g = geom(batch);
     unwrap(rh_conv2d_bwd_data(&g, 1.0f, weights->as_ptr(), pre_delta->as_ptr(), beta, in_delta, ws.as_mut_ptr(), ws.len(),
-                              conv_algo | (beside ? RH_ALGO_SHARED_GPU : 0), s()), "conv2d backward data");
+                              grad_algo() | (beside ? RH_ALGO_SHARED_GPU : 0), s()), "conv2d backward data");
   }
 
   void axpy(float a, const DeviceBuffer<float>& x, DeviceBuffer<float>& y) {
@@ -1588,7 +1588,7 @@ class BNormUnitsOperator : public Operator {
     out_delta_.reset(new DeviceBuffer<float>(out_dims.len() * batch_cap_, context_));
     size_t ws = 256;
     if (bwd)
-      for (auto& u : units_) u.aux_bytes = conv_ws_upto(u.geom(batch_cap_), RH_CONV_BWD_FILTER, u.filter_algo());
+      for (auto& u : units_) u.aux_bytes = conv_ws_upto(u.geom(batch_cap_), RH_CONV_BWD_FILTER, u.grad_algo());
     for (auto& u : units_) ws = std::max(ws, u.workspace_bytes());
     workspace_.reset(new DeviceBuffer<uint8_t>(ws, context_));
     if (bwd && opts_.overlap_backward) {

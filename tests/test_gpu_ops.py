@@ -2096,6 +2096,27 @@ def test_residual_sum_and_its_gradient(dev, shape):
         assert torch.equal(one, two) and torch.equal(copy, two)
 
 
+# Data gradients of deltas that are zeros for nine in ten, as behind a max-pool, where what three parts round is less; whether two are taken:
+# tiles that three parts sum in shorter chains (a tail in slices), whole contractions in slices, one long chain.
+@pytest.mark.parametrize("case", [(105, 384, 13, 256, 3, False), (97, 384, 13, 256, 3, False), (105, 256, 14, 256, 3, False), (64, 512, 7, 512, 3, False),
+                                  (24, 1024, 6, 1024, 3, False), (200, 384, 13, 384, 3, True), (105, 96, 27, 256, 5, True)], ids=str)
+def test_conv2d_f16x2_error_of_sparse_deltas(dev, case):
+    """As test_conv2d_f16x2_error; with RH_ALGO_BF16X3_WIDE (few deltas are zeros) the choice is another, on such operands."""
+    Nn, C, H, K, R, takes = case
+    say("f16x2 sparse deltas", case)
+    X3, F2, WIDE = _lib.RH_ALGO_BF16X3, _lib.RH_ALGO_F16X2, _lib.RH_ALGO_BF16X3_WIDE
+    x, w = torch.zeros((Nn, C, H, H), device=dev), T(synth.normal(45, 1, (K, C, R, R)), dev)
+    dense = T(synth.normal(45, 2, (Nn, K, H, H)), dev)
+    sparse = dense * (T(synth.uniform(45, 3, (Nn, K, H, H)), dev) < 0.1)
+    for dy, flags, taken in ((sparse, X3, takes), (dense, X3 | WIDE, None)):
+        run = lambda algo: ops.conv2d_bwd_data(w, dy, x.shape, 1, R // 2, algo=algo)
+        got, tags = profile_tags(lambda: run(flags | F2))
+        assert taken is None or any(t.startswith("conv_bwd_data_duo_") for t in tags) == taken, tags
+        ref = _conv_sums64(x, w, dy, 1, R // 2)[1]
+        err, err0 = (float((t.double() - ref).norm() / ref.norm()) for t in (got, run(flags)))
+        assert err <= err0, (flags, err, err0)
+
+
 # A batch norm behind a forward pass at inference: whole results and a sliced tail (the batch norm in a launch of its own), contractions in
 # slices of each form (split operands, the engine, staged), planes and channels that are no multiple of four.
 @pytest.mark.parametrize("case", [(9, 64, 56, 56, 64, 3, 1, 1), (9, 128, 28, 28, 128, 3, 1, 1), (9, 512, 7, 7, 512, 3, 1, 1), (9, 256, 14, 14, 512, 1, 2, 0),
