@@ -119,13 +119,16 @@ int rho_config_from_model_file(const char* path, rho_config** out);
  *                           Without it the library takes Winograd's F(2x2, 3x3) for 3x3 layers of 64 channels and more
  *                           (2.25x fewer multiply-adds) and for the forward pass of such 5x5 layers (1.56x fewer), and
  *                           any convolution or affine product on bf16 or fp16 matrix instructions with split fp32
- *                           operands (RH_ALGO_BF16X3, RH_ALGO_F16X2), each where it is expected to be the fastest form:
- *                           sums in another order, same tolerance against the oracle.  The flag keeps the direct form on
- *                           fp32 instructions for convolutions and affine products of every size. */
+ *                           operands (RH_ALGO_BF16X3, RH_ALGO_F16X2), each where it is expected to be the fastest form.
+ *                           Same tolerance against the oracle: sums in another order, and with RH_ALGO_F16X2 operands of 22 to
+ *                           24 of their 24 bits (which values keep how many stands at that flag).  The flag keeps the direct
+ *                           form on fp32 instructions for convolutions and affine products of every size. */
 #define RHO_EXEC_DIRECT_CONV 0x20
 /*   RHO_EXEC_FP32_INSTRUCTIONS  convolutions and affine products keep the fp32 matrix instructions (no RH_ALGO_BF16X3, no RH_ALGO_F16X2): the
  *                           Winograd form where the library takes it, the direct form elsewhere. */
 #define RHO_EXEC_FP32_INSTRUCTIONS 0x40
+/*   RHO_EXEC_EXACT_OPERANDS  of the forms with split operands only the one that holds every fp32 value exactly (no RH_ALGO_F16X2). */
+#define RHO_EXEC_EXACT_OPERANDS 0x80
 int rho_worker_new(const rho_config* cfg, int32_t batch_size, int capability, uint64_t seed0, uint64_t seed1,
                    int device, int exec_flags, rho_worker** out);
 int rho_worker_free(rho_worker* w);

@@ -278,6 +278,7 @@ int rho_worker_new(const rho_config* cfg, int32_t batch_size, int capability, ui
     opts.fuse_tail = (exec_flags & RHO_EXEC_SEPARATE_TAIL) == 0;
     opts.winograd = (exec_flags & RHO_EXEC_DIRECT_CONV) == 0;
     opts.split_operands = (exec_flags & RHO_EXEC_FP32_INSTRUCTIONS) == 0;
+    opts.scaled_parts = (exec_flags & RHO_EXEC_EXACT_OPERANDS) == 0;
     w->graph_steps = opts.graph_steps;
     w->fuse_epilogue = opts.fuse_epilogue;
     w->worker.reset(new SequentialOperatorWorker(cfg->cfg, (size_t)batch_size,

@@ -212,7 +212,9 @@ namespace {
 typedef std::shared_ptr<DeviceContext> Ctx;
 
 // The forms that a worker's options allow its convolutions.
-int product_algo(const ExecOptions& o) { return !o.winograd ? RH_ALGO_DIRECT : o.split_operands ? RH_ALGO_BF16X3 | RH_ALGO_F16X2 : 0; }
+int product_algo(const ExecOptions& o) {
+  return !o.winograd ? RH_ALGO_DIRECT : o.split_operands ? RH_ALGO_BF16X3 | (o.scaled_parts ? RH_ALGO_F16X2 : 0) : 0;
+}
 
 // Scratch is allocated once for batch_cap, but a pass may be called with any batch <= batch_cap and the library's
 // plans are not monotone in the batch (fewer result tiles make it cut the contraction into more slices, whose partial

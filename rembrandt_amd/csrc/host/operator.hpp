@@ -294,6 +294,9 @@ struct ExecOptions {
   // Convolutions and affine products on bf16 or fp16 matrix instructions with split operands (RH_ALGO_BF16X3, RH_ALGO_F16X2), where the
   // library takes those forms by itself; not without `winograd`.
   bool split_operands = true;
+  // Of these, the form whose two scaled fp16 parts hold 22 to 24 of a value's 24 bits (RH_ALGO_F16X2); false leaves the one of three bf16 parts,
+  // which are the value exactly.
+  bool scaled_parts = true;
 };
 
 // ---- Operator trait -------------------------------------------------------------------------------

@@ -25,10 +25,10 @@ def param_buffers(net, read_grads=True):
 
 
 def run(net, batch, steps, graph, seed, sgd_kwargs, fused=True, toggle_at=None, read_grads=True, fuse_tail=True, extra=(),
-        winograd=True, split_operands=True):
+        winograd=True, split_operands=True, scaled_parts=True):
     dims, layers, ncat = net
     w = SequentialOperatorWorker(configs.build_config(net), batch, "Backward", shared_seed=(seed, seed + 1), graph_steps=graph,
-                                 fuse_tail=fuse_tail, winograd=winograd, split_operands=split_operands)
+                                 fuse_tail=fuse_tail, winograd=winograd, split_operands=split_operands, scaled_parts=scaled_parts)
     w.init_params()
     sgd = SgdOpt(batch, **sgd_kwargs)
     sgd.begin(w)
@@ -313,6 +313,17 @@ def test_winograd_steps_match_direct_steps(dev, kind):
             dist = np.sqrt(((u - v) ** 2).sum()) / max(np.sqrt((v ** 2).sum()), 1e-30)
             bound = 4.5e-3 if step == 0 else {"plain": 1e-2, "five": 5e-2, "bnorm": (4.5e-2, 0.18)[step - 1]}[kind]
             assert dist <= bound, "%s step %d buffer %d: relative L2 distance %.3g" % (kind, step, k, dist)
+
+
+def test_exact_operands_only(dev):
+    """scaled_parts=False: a layer whose passes take two fp16 parts takes three bf16 parts instead, and has the same results to rounding."""
+    net = ((27, 27, 96),) + configs._chain((27, 27, 96), [("conv", 5, 1, 2, 256, "Rect"), ("conv", 5, 1, 2, 96, "Rect"), ("fc", 10, "Identity")])
+    say("exact operands")
+    kw = dict(step_size=0.01, momentum=("Update", 0.9), l2_reg_coef=5e-4)
+    (a, _), tags_a = profile_tags(lambda: run(net, 64, 1, False, 0x51, kw))
+    (b, _), tags_b = profile_tags(lambda: run(net, 64, 1, False, 0x51, kw, scaled_parts=False))
+    assert any("_duo_" in t for t in tags_a) and any("_tri_" in t for t in tags_b) and not any("duo" in t for t in tags_b), (tags_a, tags_b)
+    assert abs(a[0][0] - b[0][0]) <= 1e-5 * abs(b[0][0])
 
 
 @pytest.mark.parametrize("kind", ["plain", "five"])
