@@ -623,6 +623,9 @@ def main():
         "scaling": "weak",
         "vs_baseline": None,
         "dtype": "f32",
+        "products": "operands, results and sums in f32; large convolutions and affine products multiply on 16-bit matrix instructions, each "
+                    "f32 operand as the exact sum of three bf16 values or (convolutions) of two scaled fp16 values, 22 to 24 of its 24 bits: "
+                    "which one is chosen so that the error against 64-bit sums is no larger than that of the form it replaces",
         "data": "synthetic",
         "config": {"workload": "%s-shaped train step (fwd+bwd+SGD momentum 0.9), batch %d, fp32, input %dx%dx%d N(0,1), "
                                "weights N(0,0.01), %s%s" % (args.workload, batch, dims[2], dims[1], dims[0],

@@ -41,14 +41,13 @@ __device__ __forceinline__ float wave_sum(float v) {
   return v;
 }
 
+struct BnMask { const float* scale; const float* ivar; const float* bias; };
+
 // MODE 0: (sum d, sum d*d) with d = x - x[first value of the channel].
 // MODE 1: (sum dy, sum dy*(x - mean[c])).
 // VEC (plane % 4 == 0, 16-byte aligned tensors): a lane reads 16 bytes at a time, two such loads in flight per operand.
 // MASK (MODE 1): dy counts only where the forward pass's ReLU let the value through, i.e. where
 // bn_affine(x, mean, scale*ivar, bias) > 0, recomputed here exactly as the forward pass computed it.
-
-struct BnMask { const float* scale; const float* ivar; const float* bias; };
-
 template <int MODE, bool VEC, bool MASK = false>
 __global__ __launch_bounds__(256) void bn_reduce_kernel(const float* __restrict__ x, const float* __restrict__ dy,
                                                         const float* __restrict__ mean, int C, int plane, int chunks,

@@ -35,13 +35,13 @@ inline int stream_grid(size_t work_items, int block) {
   return static_cast<int>(want);
 }
 
+// A batch norm of one value, si = scale * inverse deviation: one expression wherever it is formed or formed again.
+__device__ __forceinline__ float bn_affine(float x, float mean, float si, float bias) { return fmaf(x - mean, si, bias); }
+
 // Division of a non-negative 32-bit index (< 2^31) by a runtime constant as multiply-high + add + shift
 // (Granlund-Montgomery round-up method); the divisor's constants are computed once on the host.  The
 // bandwidth-bound kernels decompose a flat index per element: hardware integer division there costs
 // more instructions than everything else in the kernel.
-// A batch norm of one value, si = scale * inverse deviation: one expression wherever it is formed or formed again.
-__device__ __forceinline__ float bn_affine(float x, float mean, float si, float bias) { return fmaf(x - mean, si, bias); }
-
 struct FastDiv {
   uint32_t mul, shift, div;
   __host__ __device__ FastDiv() : mul(1), shift(0), div(1) {}

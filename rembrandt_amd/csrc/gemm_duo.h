@@ -3,7 +3,10 @@
 // a 2^e = a1 + a2 2^-11 with a1 = fp16(a 2^e) and a2 = fp16((a 2^e - a1) 2^11); e is one exponent for a row of the operand (for
 // the image of a convolution: for all pixels of an image) and takes its largest value to [2^14, 2^15).  The product of two fp16
 // values is exact in fp32, and of the four products of a pair the one of two second parts (2^-22 of it) is left out: three
-// v_mfma_f32_32x32x16_f16 do the work for which the exact sum of three bf16 values (gemm_tri.h) needs six.
+// v_mfma_f32_32x32x16_f16 do the work for which the exact sum of three bf16 values (gemm_tri.h) needs six.  (Two halves, the second held
+// 2^11 times as large, three products and sums kept outside the matrix unit are a published scheme: Ootomo and Yokota, "Recovering single
+// precision accuracy from Tensor Cores while surpassing the FP32 theoretical peak performance", 2022.  The exponents by row and what is
+// done about values out of range are this library's.)
 //
 // Precision.  Two parts hold 22 to 24 of a value's 24 bits: three values of four exactly, the fourth is off by its last bit
 // (relative error 4.3e-8, rms; with the product left out 7.5e-8 a product, N(0,1) data).  What a sum of many products loses, the
@@ -26,7 +29,8 @@
 // * A filter's small values (one in 1e8 of normal weights) are counted.  They cost a result 2^-20 each at most, so its sum, before it is
 //   scaled back, has to be four times their number: 2^27 is usual.  (A mark would have the filter's whole plane formed again.)
 // * In the filter gradient, where the eight of a group are images and zeros of the other operand say nothing of the sum, every small value
-//   is marked, and one such value makes it a call in three parts (TriRest; AlexNet b256 one call in 48, in NIN b128 the 5x5 layer's).
+//   is marked, and one such value makes it a call in three parts (TriRest; AlexNet's at 26 batches one call in 39, of
+//   NIN's the 5x5 layer's 16 of 17, of its 3x3 layers' 7 of 15).
 //   Formed again, a block of 32 x 32 results is bound by the latency of its loads, 32 of them in flight (one by one 384 -> 384 3x3 13x13
 //   b256 forward took 3.0 ms longer for one value): 330 us, with one value in x 930, with one in every group 3.9 ms (three parts 550 us,
 //   1.4 and 2.9 ms); 5x5 of 96 channels 0.6, 0.9 and 12 ms, 1x1 at 128 images 54, 93 and 260 us.  In the filter gradient, whose loads are
