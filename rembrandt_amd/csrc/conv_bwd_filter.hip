@@ -390,9 +390,11 @@ static TriRival filter_rival(const ConvDims& d) {
   const BwdFilterSoffPlan sp = plan_bwd_filter_soff(d);
   return TriRival{0.9 * us, 0.0335 * terms / (sp.ok && use_soff_bwd_filter(d) ? sp.splits : plan_bwd_filter(d).splits)};
 }
-// Two parts beside the form of time `other_us` and error `err`; both errors with a twentieth of the products not zero, as behind a
-// max-pool, where two parts are the least ahead (1e-14 on the square): three parts 0.005 a K step of a slice and 0.016 a slice; two 1.0
-// and 0.016 a slice (of AlexNet's conv5 at 128 images 0.92e-7 and 1.08e-7, at 256 1.30 and 1.15, of its conv2 at 50 1.28 and 1.26).
+// Two parts beside the form of time `other_us` and error `err` (1e-14 on the square, fitted to the networks' layers behind a max-pool, where
+// two parts are the least ahead): three parts 0.005 a K step of a slice and 0.016 a slice; two 1.0 and 0.016 a slice (of AlexNet's conv5 at
+// 128 images 0.92e-7 and 1.08e-7, at 256 1.30 and 1.15, of its conv2 at 50 1.28 and 1.26).  Over 92 layers and batches of N(0,1) operands, half of
+// x zeros, the error of those taken is 0.32 of three parts' (geometric mean), with half of the deltas zeros 0.42, with nine in ten 0.85 (1.2 at
+// most).
 static bool duo_filter_pays(int splits, double us, double other_us, double err) {
   return us < 0.96 * other_us && 1.0 + 0.016 * splits <= err;
 }

@@ -726,9 +726,10 @@ inline bool duo_replaces_tri(bool bwd, bool dense, const TriPlan& tri, const Tri
              : 0.0327 * a.steps + 0.012 * a.slices >= 1.56 + 0.005 * b.steps + 0.034 * b.slices;
 }
 // The others' errors are in tri_max_chain's units, N(0,1).  Over 539 timed calls (18 layers at 11 batches, all passes, half zeros) two parts
-// are taken in 137, 1.34 times as fast in the geometric mean, none slower, with 0.50 of the error of the form replaced, 0.87 at most; on
-// the networks' own activations, filters and deltas (forward, data and filter gradient; geometric mean and largest) AlexNet 0.59, 0.54,
-// 0.50 and 0.92, NIN 0.62, 0.50, 0.26 and 0.94, ResNet-18 0.52, 0.34 and 0.81 (131 calls).
+// are taken in a quarter, 1.34 times as fast in the geometric mean, none slower, with 0.50 of the error of the form replaced, 0.87 at most; on
+// the networks' own activations, filters and deltas at 26 batches (906 calls; forward, data gradient, filter gradient) AlexNet 0.58, 0.47 and
+// 0.57, NIN 0.59, 0.41 and 0.74 (20 of its 26 filter gradients end in three parts), ResNet-18 0.51 and 0.33; 0.89, 0.94
+// and 0.96 at most.
 inline bool duo_replaces(double err, int duo_steps) { return 2.5 + 0.008 * duo_steps <= err; }
 struct SplitPick {
   int parts;
