@@ -242,10 +242,10 @@ struct DuoShape {
 // issued, a1 and b1 into a second set: 64 x 64 of a 128 x 128 tile are 192 accumulators in three sets and 48 registers of operands, two
 // waves to a SIMD.  Step `it` of a wave issues the loads of step it + R - 1 into the buffer that step it - 1 left, so they
 // have R - 2 steps to land.  Bound by the power that the MFMAs draw: 384 -> 384 3x3 13x13 b256 forward takes 270 us = 425 TFLOP/s of fp32
-// multiply-adds (three bf16 parts 470 us; from registers alone three products reach 545 to 573 TFLOP/s with N(0,1) operands, 600 to 622 where
-// half of one are zeros, from box to box).  In AlexNet's step at 256 images the matrix pipes are busy 66 to 69 % of the time forward, at 1.65 to 1.87 GHz, and 58 to 63 % in the
-// gradients, at 1.86 to 2.06 GHz, where the ends of chains (KEEP) and their sums are 4.0 to 4.5 VALU instructions an MFMA for 2.5.  A barrier every
-// second step, or a raised wave priority, changes nothing.
+// multiply-adds (three bf16 parts 470 us; from registers alone three products reach 530 to 573 TFLOP/s with N(0,1) operands, 580 to 622 where
+// half of one are zeros, from box to box).  In AlexNet's step at 256 images the matrix pipes are busy 64 to 69 % of the time forward, at
+// 1.6 to 1.9 GHz, and 58 to 63 % in the gradients, at 1.8 to 2.1 GHz, where the ends of chains (KEEP) and their sums are 4.0 to 4.5 VALU
+// instructions an MFMA for 2.5.  A barrier every second step, or a raised wave priority, changes nothing.
 template <class T, bool NCHW, bool KEEP>
 __device__ __forceinline__ void duo_block(const DuoParams& ap, const DuoParams& bp, const DuoSource& src, const EpiParams& ep, int m0,
                                           int n0, int s_begin, int s_end, int groups, int dst_split) {
