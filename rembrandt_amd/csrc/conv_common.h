@@ -727,9 +727,8 @@ inline bool duo_replaces_tri(bool bwd, bool dense, const TriPlan& tri, const Tri
 }
 // The others' errors are in tri_max_chain's units, N(0,1).  Over 539 timed calls (18 layers at 11 batches, all passes, half zeros) two parts
 // are taken in a quarter, 1.34 times as fast in the geometric mean, none slower, with 0.50 of the error of the form replaced, 0.87 at most; on
-// the networks' own activations, filters and deltas at 26 batches (906 calls; forward, data gradient, filter gradient) AlexNet 0.58, 0.47 and
-// 0.57, NIN 0.59, 0.41 and 0.74 (20 of its 26 filter gradients end in three parts), ResNet-18 0.51 and 0.33; 0.89, 0.94
-// and 0.96 at most.
+// the networks' own activations, filters and deltas at 67 batches (2423 calls; forward, data gradient, filter gradient) AlexNet 0.55, 0.46 and
+// 0.55, NIN 0.59, 0.39 and 0.73 (most of its filter gradients end in three parts), ResNet-18 0.52 and 0.33; 0.89, 0.94 and 0.98 at most.
 inline bool duo_replaces(double err, int duo_steps) { return 2.5 + 0.008 * duo_steps <= err; }
 struct SplitPick {
   int parts;

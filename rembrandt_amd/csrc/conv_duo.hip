@@ -1,8 +1,9 @@
 // fp32 convolutions on the fp16 matrix instructions with operands of two scaled parts (gemm_duo.h): forward, stride-1
 // backward-data and backward-filter.
 //
-// Three launches in front of the reduction of slices: the largest magnitudes (and the filters' ratios), the operand copies in two fp16 parts (4 bytes a value,
-// in the orders of conv_tri.hip), the contraction.  The exponents are the filter's by row and the image's by image, and in the filter
+// Three launches in front of the reduction of slices: the largest magnitudes (and the filters' ratios), the operand copies in two fp16 parts (4
+// bytes a value, in the orders of conv_tri.hip), the contraction; in the filter gradient a fourth before the contraction, which copies in
+// three parts where a value asks for them (TriRest).  The exponents are the filter's by row and the image's by image, and in the filter
 // gradient both operands' by channel.
 #include "conv_common.h"
 #include "gemm_duo.h"

@@ -1299,12 +1299,11 @@ struct BNormConvUnit {
     return g;
   }
   int plane() const { return (int)(out_dims.w * out_dims.h); }
-  // The filter gradient's: split operands on short sums only.  A batch norm's backward leaves a small value everywhere beside the few
+  // The gradients' (RH_ALGO_BF16X3_WIDE): a batch norm's backward leaves a small value everywhere beside the few
   // large ones that a ReLU let through, and RH_ALGO_BF16X3's instruction cuts products toward zero at 2^-24 of the largest of the
   // eight that it adds at once: where the inputs are of one sign that adds up over the pixels.  Error of ResNet-18's filter gradients
-  // against 64 bits, relative to the other forms', 8 to 200 images: 64 -> 64 56x56 1.2 to 5.1 in the units whose input is
+  // against 64 bits without that bit, relative to the other forms', 8 to 200 images: 64 -> 64 56x56 1.2 to 5.1 in the units whose input is
   // positive, 64 -> 128 1.4 to 3.1, 128 -> 128 28x28 0.7 to 1.4, 128 -> 256 0.5 to 1.2; 256 and 512 channels on 14x14 and 7x7 0.2 to 0.9.
-  // The gradients': deltas are a batch norm's, a small value almost everywhere beside the large ones that a ReLU let through.
   int grad_algo() const { return conv_algo | (conv_algo & RH_ALGO_BF16X3 ? RH_ALGO_BF16X3_WIDE : 0); }
   size_t workspace_bytes() const {
     const rh_conv_geom g = geom(batch_cap);
